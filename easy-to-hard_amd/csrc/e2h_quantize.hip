@@ -23,15 +23,64 @@ __device__ __forceinline__ float load_w(const void *w, size_t i) {
   }
 }
 
-template <bool BF16>
+// One code: rintf(w / scale), clamped.  The quotient from the reciprocal is a few units in the last place off, which matters only
+// next to a rounding boundary n + 1/2; there (and for anything not finite) the true division decides.
+__device__ __forceinline__ int int8_code(float w, float scale, float rcp) {
+  float v = w * rcp;
+  const float near = v - floorf(v) - 0.5f;
+  if (!(fabsf(near) > 1e-3f)) v = w / scale;   // :66  true division
+  return static_cast<int>(fminf(fmaxf(rintf(v), -128.f), 127.f));  // :67 half to even, :69
+}
+
+// One row per workgroup, bound by HBM.  VEC: eight values per load and lane (rows a multiple of eight values, 16-byte aligned); rows
+// up to kHeld * 2048 values stay in registers between the two passes, which otherwise read the row again.
+template <bool BF16, bool VEC>
 __global__ __launch_bounds__(256) void int8_quantize_rows_kernel(const void *__restrict__ w, int8_t *__restrict__ q,
                                                                  float *__restrict__ scales_f32,
                                                                  uint16_t *__restrict__ scales_bf16, int64_t K) {
+  constexpr int kHeld = 6;
   const int64_t row = blockIdx.x;
   const size_t base = static_cast<size_t>(row) * K;
+  const auto load8 = [&](int64_t k, float (&v)[8]) {
+    if constexpr (BF16) {
+      const u32x4_t raw = *reinterpret_cast<const u32x4_t *>(static_cast<const uint16_t *>(w) + base + k);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[2 * i] = __builtin_bit_cast(float, raw[i] << 16);
+        v[2 * i + 1] = __builtin_bit_cast(float, raw[i] & 0xFFFF0000u);
+      }
+    } else {
+      const f32x4_t *p = reinterpret_cast<const f32x4_t *>(static_cast<const float *>(w) + base + k);
+      const f32x4_t lo = p[0], hi = p[1];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[i] = lo[i];
+        v[4 + i] = hi[i];
+      }
+    }
+  };
   // max(-min(min_val, 0), max(max_val, 0)) == max |x| over the row  (:49-58)
-  float amax = 0.f;
-  for (int64_t k = threadIdx.x; k < K; k += blockDim.x) amax = fmaxf(amax, fabsf(load_w<BF16>(w, base + k)));
+  float amax = 0.f, held[kHeld][8];
+  if constexpr (VEC) {
+#pragma unroll
+    for (int i = 0; i < kHeld; ++i) {
+      const int64_t k = (i * 256 + threadIdx.x) * int64_t{8};
+      if (k < K) load8(k, held[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < kHeld; ++i)
+      if ((i * 256 + threadIdx.x) * int64_t{8} < K)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(held[i][j]));
+    for (int64_t k = (kHeld * 256 + threadIdx.x) * int64_t{8}; k < K; k += 2048) {
+      float v[8];
+      load8(k, v);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
+    }
+  } else {
+    for (int64_t k = threadIdx.x; k < K; k += blockDim.x) amax = fmaxf(amax, fabsf(load_w<BF16>(w, base + k)));
+  }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
   __shared__ float wave_max[4];
@@ -44,11 +93,26 @@ __global__ __launch_bounds__(256) void int8_quantize_rows_kernel(const void *__r
     if (scales_f32) scales_f32[row] = scale;
     if (scales_bf16) scales_bf16[row] = f32_to_bf16_rne(scale);
   }
-  for (int64_t k = threadIdx.x; k < K; k += blockDim.x) {
-    float v = load_w<BF16>(w, base + k) / scale;  // :66  true division
-    v = rintf(v);                                  // :67  half to even
-    v = fminf(fmaxf(v, -128.f), 127.f);            // :69
-    q[base + k] = static_cast<int8_t>(static_cast<int>(v));
+  const float rcp = __builtin_amdgcn_rcpf(scale);
+  if constexpr (VEC) {
+    const auto store8 = [&](int64_t k, const float (&v)[8]) {
+      u32x2_t o = {0u, 0u};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j >> 2] |= (static_cast<uint32_t>(int8_code(v[j], scale, rcp)) & 255u) << (8 * (j & 3));
+      *reinterpret_cast<u32x2_t *>(q + base + k) = o;
+    };
+#pragma unroll
+    for (int i = 0; i < kHeld; ++i) {
+      const int64_t k = (i * 256 + threadIdx.x) * int64_t{8};
+      if (k < K) store8(k, held[i]);
+    }
+    for (int64_t k = (kHeld * 256 + threadIdx.x) * int64_t{8}; k < K; k += 2048) {
+      float v[8];
+      load8(k, v);
+      store8(k, v);
+    }
+  } else {
+    for (int64_t k = threadIdx.x; k < K; k += blockDim.x) q[base + k] = static_cast<int8_t>(int8_code(load_w<BF16>(w, base + k), scale, rcp));
   }
 }
 
@@ -272,72 +336,134 @@ __global__ __launch_bounds__(256) void int4_dequantize_codes_kernel(const int32_
   w_out[idx] = f32_to_bf16_rne(t + bf16_to_f32(zeros[gi]));                                   // :169 .add(zeros)
 }
 
-// Fused quantize + pack: a workgroup owns one 8-row tile x 256 k.  Lane layout as int4_group_kernel
-// (8 consecutive k per lane); codes go through LDS as bytes and leave as packed words, so the int32
-// code matrix (4 bytes per weight) never touches HBM.
-template <int G>
+// ---- fused quantize + pack ----------------------------------------------------------------------------
+// Lane layout as int4_group_kernel (8 consecutive k per lane, 32 lanes per row, a workgroup 8 rows x 256 k).  Four neighbouring
+// lanes hold the 32 codes of four packed words: word j takes from lane h of the quad code 2 j as nibble h and code 2 j + 1 as
+// nibble 4 + h, so the words form by two ORs across the quad, without LDS, and lane j stores word j.
+
+__device__ __forceinline__ float float_of(uint32_t u) { return __builtin_bit_cast(float, u); }
+
+// nearest bfloat16 by the conversion instruction (no NaN here), as float32
+__device__ __forceinline__ float to_bf16(float v) {
+  return float_of(static_cast<uint32_t>(__builtin_bit_cast(uint16_t, static_cast<__bf16>(v))) << 16);
+}
+
+// value of the lane whose number differs by XOR (1, 2: any; 7, 15: within its row of 16)
+template <int XOR>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+  constexpr int kCtrl = XOR == 1 ? 0xB1 : XOR == 2 ? 0x4E : XOR == 7 ? 0x141 : 0x140;  // quad_perm, row_half_mirror, row_mirror
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), kCtrl, 0xF, 0xF, true));
+}
+
+// minimum and maximum over LPG neighbouring lanes
+template <int LPG>
+__device__ __forceinline__ void group_minmax(float &mn, float &mx) {
+  const auto step = [&](auto other) {
+    const float a = float_of(other(__builtin_bit_cast(uint32_t, mn))), b = float_of(other(__builtin_bit_cast(uint32_t, mx)));
+    mn = fminf(mn, a);
+    mx = fmaxf(mx, b);
+  };
+  step([](uint32_t v) { return lane_xor<1>(v); });
+  step([](uint32_t v) { return lane_xor<2>(v); });
+  if constexpr (LPG >= 8) step([](uint32_t v) { return lane_xor<7>(v); });    // a quad's lanes agree by now
+  if constexpr (LPG >= 16) step([](uint32_t v) { return lane_xor<15>(v); });  // so do eight
+  if constexpr (LPG >= 32) step([](uint32_t v) { return static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), 16)); });
+}
+
+// quantize_one for two values at once and a finite scale >= 1e-6 / 15.  w - min_val and the scale are bfloat16 values, so their quotient
+// Q is exactly a rounding boundary (of bfloat16, or of the integers) or a relative 2^-17 away from one.  q0 = a rcp(s) is within 2^-22 of
+// Q, its residual e = a - q0 s is exact in float32, and q0 + e rcp(s) is Q to 2^-45 before its one rounding: on a boundary it is
+// that value, elsewhere on Q's side.  Adding 1.5 * 2^23 rounds to the integer, ties to even, and leaves it in the low bits.
+__device__ __forceinline__ void quantize_two(float w0, float w1, float scale, float rcp, float min_val, uint32_t &c0, uint32_t &c1) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const uint32_t a = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{w0 - min_val, w1 - min_val}, bf16x2));
+  const float a0 = float_of(a << 16), a1 = float_of(a & 0xFFFF0000u);
+  const float q0 = a0 * rcp, q1 = a1 * rcp;
+  const float r0 = __builtin_fmaf(__builtin_fmaf(-q0, scale, a0), rcp, q0), r1 = __builtin_fmaf(__builtin_fmaf(-q1, scale, a1), rcp, q1);
+  const uint32_t t = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{r0, r1}, bf16x2));
+  c0 = __builtin_bit_cast(uint32_t, fminf(fmaxf(float_of(t << 16), 0.f), 15.f) + 12582912.f) & 15u;
+  c1 = __builtin_bit_cast(uint32_t, fminf(fmaxf(float_of(t & 0xFFFF0000u), 0.f), 15.f) + 12582912.f) & 15u;
+}
+
+// U: spans of 256 k per workgroup, all loaded before the first is worked on.  The bound is HBM once a weight costs about 20 vector
+// instructions: 11008 x 4096 at g128 (112 MB in and out) takes 31 us, 3.6 TB/s beside 4.8 for a large copy.  With IEEE divisions (ten
+// instructions each), software rounding with its NaN branch, shuffles through LDS and 64-bit index divisions it took 67 us.
+// U = 2 measured 30.7 us, 1: 31.5, 4: 31.8, 8: 33.5.
+template <int G, int U>
 __global__ __launch_bounds__(256) void int4_quantize_pack_kernel(const uint16_t *__restrict__ w, uint32_t *__restrict__ packed,
-                                                                 uint16_t *__restrict__ sz, int64_t N, int64_t K, int ikt) {
+                                                                 uint16_t *__restrict__ sz, int64_t N, int64_t K, unsigned spans, int ikt_log2) {
   constexpr int LPG = G / 8;
   constexpr int SPAN = 256;
-  __shared__ uint8_t lds_codes[8][SPAN + 16];
-  const int64_t spans = K / SPAN;
-  const int64_t n_tile = blockIdx.x / spans;
-  const int64_t span = blockIdx.x - n_tile * spans;
-  const int r = threadIdx.x >> 5;        // row within the tile
-  const int kl = (threadIdx.x & 31) * 8;  // k within the span
-  const int64_t n = n_tile * 8 + r;
-  const int64_t k = span * SPAN + kl;
+  const unsigned n_tile = blockIdx.x / spans, span0 = (blockIdx.x - n_tile * spans) * U;
+  const int r = threadIdx.x >> 5;         // row within the tile
+  const int kl = (threadIdx.x & 31) * 8;  // k within a span
+  const int h = threadIdx.x & 3;
+  const int64_t n = static_cast<int64_t>(n_tile) * 8 + r;
+  const int64_t k0 = static_cast<int64_t>(span0) * SPAN;
+  const uint16_t *const src = w + n * K + k0 + kl;
+  u32x4_t raw[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) raw[u] = *reinterpret_cast<const u32x4_t *>(src + u * SPAN);
+  // word (row, h) of the 32-wide piece p of k block k_outer sits at ((n_tile * k blocks + k_outer) * 32 + 4 r + h) * ikt / 2 + p
+  const int kblk_log2 = ikt_log2 + 4, words_log2 = ikt_log2 - 1;
+  uint32_t *const dst = packed + (((static_cast<int64_t>(n_tile) * (K >> kblk_log2) + (k0 >> kblk_log2) + (kl >> kblk_log2)) * 32 + 4 * r + h) << words_log2) +
+                        ((kl >> 5) & ((1 << words_log2) - 1));
+  uint32_t *const sz_dst = reinterpret_cast<uint32_t *>(sz) + ((k0 + kl) / G) * N + n;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = float_of(raw[u][i] << 16);
+      v[2 * i + 1] = float_of(raw[u][i] & 0xFFFF0000u);
+    }
+    float mn = v[0], mx = v[0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) {
+      mn = fminf(mn, v[i]);
+      mx = fmaxf(mx, v[i]);
+    }
+    group_minmax<LPG>(mn, mx);
+    uint32_t c[8], pair;
+    if (mx - mn < 1e37f) {
+      // qparams_from_minmax and requant_min, the division by 15 as quantize_two divides; scale * 8 is exact
+      const float range = fmaxf(to_bf16(mx - mn), bf16_to_f32(0x3586));
+      const float over = range * (1.0f / 15.0f);
+      const float scale = to_bf16(__builtin_fmaf(__builtin_fmaf(-over, 15.0f, range), 1.0f / 15.0f, over));
+      const float zero = to_bf16(mn + scale * 8.0f), min_val = to_bf16(zero - scale * 8.0f), rcp = __builtin_amdgcn_rcpf(scale);
+      pair = __builtin_bit_cast(uint32_t, scale) >> 16 | __builtin_bit_cast(uint32_t, zero);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) quantize_two(v[2 * i], v[2 * i + 1], scale, rcp, min_val, c[2 * i], c[2 * i + 1]);
+    } else {  // infinities or nearly so
+      const GroupQParams qp = qparams_from_minmax(mn, mx);
+      const float min_val = requant_min(qp.scale, qp.zero);
+      pair = static_cast<uint32_t>(f32_to_bf16_rne(qp.scale)) | (static_cast<uint32_t>(f32_to_bf16_rne(qp.zero)) << 16);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) c[i] = static_cast<uint32_t>(quantize_one(v[i], qp.scale, min_val));
+    }
+    if ((kl % G) == 0) sz_dst[u * (SPAN / G) * N] = pair;
+    uint32_t word = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      uint32_t t = (c[2 * j] | c[2 * j + 1] << 16) << (4 * h);
+      t |= lane_xor<1>(t);
+      t |= lane_xor<2>(t);
+      word = h == j ? t : word;
+    }
+    dst[u * SPAN] = word;  // a span of 8 rows is 256 words
+  }
+}
 
-  const u32x4_t raw = *reinterpret_cast<const u32x4_t *>(w + n * K + k);
-  float v[8];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    v[2 * i] = __builtin_bit_cast(float, raw[i] << 16);
-    v[2 * i + 1] = __builtin_bit_cast(float, raw[i] & 0xFFFF0000u);
-  }
-  float mn = v[0], mx = v[0];
-#pragma unroll
-  for (int i = 1; i < 8; ++i) {
-    mn = fminf(mn, v[i]);
-    mx = fmaxf(mx, v[i]);
-  }
-#pragma unroll
-  for (int off = 1; off < LPG; off <<= 1) {
-    mn = fminf(mn, __shfl_xor(mn, off));
-    mx = fmaxf(mx, __shfl_xor(mx, off));
-  }
-  const GroupQParams qp = qparams_from_minmax(mn, mx);
-  const float min_val = requant_min(qp.scale, qp.zero);
-  uint32_t lo = 0, hi = 0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    lo |= static_cast<uint32_t>(quantize_one(v[i], qp.scale, min_val)) << (8 * i);
-    hi |= static_cast<uint32_t>(quantize_one(v[4 + i], qp.scale, min_val)) << (8 * i);
-  }
-  *reinterpret_cast<uint32_t *>(&lds_codes[r][kl]) = lo;
-  *reinterpret_cast<uint32_t *>(&lds_codes[r][kl + 4]) = hi;
-  if ((k % G) == 0) {
-    const uint32_t pair = static_cast<uint32_t>(f32_to_bf16_rne(qp.scale)) | (static_cast<uint32_t>(f32_to_bf16_rne(qp.zero)) << 16);
-    reinterpret_cast<uint32_t *>(sz)[(k / G) * N + n] = pair;
-  }
-  __syncthreads();
-
-  // 8 rows x 256 k = 256 packed words, contiguous in the packed tensor for this (n_tile, span)
-  const int words = ikt / 2;
-  const int kblk = 16 * ikt;
-  const int64_t kt = K / kblk;
-  const int widx_local = threadIdx.x;            // [k_outer_local][t][p]
-  const int p = widx_local % words;
-  const int t = (widx_local / words) % 32;
-  const int ko_local = widx_local / (words * 32);
-  const int row = t >> 2, j = t & 3;
-  const int k0 = ko_local * kblk + 2 * p * 16;
-  uint32_t word = 0;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) word |= static_cast<uint32_t>(lds_codes[row][k0 + nibble_k(i, j)]) << (4 * i);
-  const int64_t k_outer = span * (SPAN / kblk) + ko_local;
-  packed[((n_tile * kt + k_outer) * 32 + t) * words + p] = word;
+template <int G>
+void launch_quantize_pack(const uint16_t *w, uint32_t *packed, uint16_t *sz, int64_t n, int64_t k, int ikt, hipStream_t s) {
+  const unsigned spans = static_cast<unsigned>(k / 256);
+  const int ikt_log2 = ikt == 8 ? 3 : ikt == 4 ? 2 : 1;
+  const unsigned tiles = static_cast<unsigned>(n / 8);
+  if (spans % 2 == 0)
+    hipLaunchKernelGGL((int4_quantize_pack_kernel<G, 2>), dim3(tiles * (spans / 2)), dim3(256), 0, s, w, packed, sz, n, k, spans / 2, ikt_log2);
+  else
+    hipLaunchKernelGGL((int4_quantize_pack_kernel<G, 1>), dim3(tiles * spans), dim3(256), 0, s, w, packed, sz, n, k, spans, ikt_log2);
 }
 
 inline unsigned blocks_for(int64_t items, int per_block) { return static_cast<unsigned>((items + per_block - 1) / per_block); }
@@ -379,10 +505,10 @@ extern "C" int e2h_int8_quantize_per_channel(const void *w, int w_is_bf16, int8_
   if (!w || !q) return E2H_ERR_NULL_POINTER;
   if (n < 1 || k < 1 || n > INT32_MAX) return E2H_ERR_BAD_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (w_is_bf16)
-    hipLaunchKernelGGL((int8_quantize_rows_kernel<true>), dim3(static_cast<unsigned>(n)), dim3(256), 0, s, w, q, scales_f32, scales_bf16, k);
-  else
-    hipLaunchKernelGGL((int8_quantize_rows_kernel<false>), dim3(static_cast<unsigned>(n)), dim3(256), 0, s, w, q, scales_f32, scales_bf16, k);
+  const bool vec = (k % 8) == 0 && aligned16(w) && (reinterpret_cast<uintptr_t>(q) & 7u) == 0;
+  const auto kernel = w_is_bf16 ? (vec ? int8_quantize_rows_kernel<true, true> : int8_quantize_rows_kernel<true, false>)
+                                : (vec ? int8_quantize_rows_kernel<false, true> : int8_quantize_rows_kernel<false, false>);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n)), dim3(256), 0, s, w, q, scales_f32, scales_bf16, k);
   return launch_status();
 }
 
@@ -460,13 +586,12 @@ extern "C" int e2h_int4_quantize_pack(const uint16_t *w, int32_t *packed, uint16
     return E2H_ERR_MISALIGNED;
   if (k % 256 != 0) return E2H_ERR_BAD_SHAPE;  // callers fall back to quantize + pack
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const unsigned blocks = static_cast<unsigned>((n / 8) * (k / 256));
   uint32_t *out = reinterpret_cast<uint32_t *>(packed);
   switch (groupsize) {
-    case 32: hipLaunchKernelGGL((int4_quantize_pack_kernel<32>), dim3(blocks), dim3(256), 0, s, w, out, scales_and_zeros, n, k, inner_k_tiles); break;
-    case 64: hipLaunchKernelGGL((int4_quantize_pack_kernel<64>), dim3(blocks), dim3(256), 0, s, w, out, scales_and_zeros, n, k, inner_k_tiles); break;
-    case 128: hipLaunchKernelGGL((int4_quantize_pack_kernel<128>), dim3(blocks), dim3(256), 0, s, w, out, scales_and_zeros, n, k, inner_k_tiles); break;
-    default: hipLaunchKernelGGL((int4_quantize_pack_kernel<256>), dim3(blocks), dim3(256), 0, s, w, out, scales_and_zeros, n, k, inner_k_tiles); break;
+    case 32: launch_quantize_pack<32>(w, out, scales_and_zeros, n, k, inner_k_tiles, s); break;
+    case 64: launch_quantize_pack<64>(w, out, scales_and_zeros, n, k, inner_k_tiles, s); break;
+    case 128: launch_quantize_pack<128>(w, out, scales_and_zeros, n, k, inner_k_tiles, s); break;
+    default: launch_quantize_pack<256>(w, out, scales_and_zeros, n, k, inner_k_tiles, s); break;
   }
   return launch_status();
 }

@@ -135,3 +135,47 @@ def test_reference_named_functions_on_cpu_tensors():
     deq = e2h.group_dequantize_tensor(codes, sz, 4, 64)
     s_ref, z_ref = qo.unpack_scales_and_zeros(sz_ref)
     np.testing.assert_array_equal(bf16_to_np(deq), qo.int4_dequantize_from_qparams(c_ref, s_ref, z_ref, 4, 64))
+
+
+@pytest.mark.parametrize("g", [32, 64, 128, 256])
+@pytest.mark.parametrize("k", [256, 512, 768])
+def test_fused_quantize_pack_at_ties_and_extremes(g, k):
+    """Quotients exactly on rounding boundaries (small integers over small powers of two), a constant row, tiny and huge ranges,
+    infinities and NaN: the same bits as quantizing with true divisions and packing afterwards."""
+    gen = torch.Generator().manual_seed(g + k)
+    w = torch.randint(-60, 61, (24, k), generator=gen).float()
+    w[4] = 3.0
+    w[5] *= 1e-30
+    w[6] *= 1e36
+    w[7] = torch.randn(k, generator=gen)
+    w[8] /= 64.0
+    w[9] = (torch.randint(0, 31, (k,), generator=gen) - 15).float() * 0.5   # range 15: scale 1, every other value a tie
+    w[10, 3], w[11, 5], w[12, 7] = float("inf"), float("-inf"), float("nan")
+    w[13] = float("nan")
+    wd = w.to(torch.bfloat16).to(DEV)
+    codes, sz = ops.int4_group_quantize(wd, g)
+    for ikt in (2, 4, 8):
+        packed, sz2 = ops.int4_quantize_pack(wd, g, ikt)
+        assert torch.equal(packed, ops._int4_pack_impl(codes, ikt))
+        both = sz.view(torch.int16), sz2.view(torch.int16)
+        assert torch.equal(*both)
+
+
+@pytest.mark.parametrize("k", [1, 7, 8, 40, 2048, 12288, 12296, 22016])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_int8_quantize_rows_next_to_ties_and_of_any_length(k, dtype):
+    """Rows of one value up to more than stay in registers, an unaligned first row, values on and beside n + 1/2."""
+    gen = torch.Generator().manual_seed(k)
+    w = (torch.randint(-255, 256, (6, k), generator=gen).float() * 0.5).to(dtype)
+    w[0, 0], w[1] = 127.5, torch.randn(k, generator=gen).to(dtype)
+    w[2] = 0
+    w[3] = torch.nextafter(w[3].float(), torch.tensor(1e9)).to(dtype)
+    w[4] = 1e-30
+    for shift in (0, 1):
+        flat = torch.empty((w.numel() + shift,), dtype=dtype, device=DEV)
+        wd = flat[shift:].view(w.shape)
+        wd.copy_(w)
+        q, s = ops.int8_quantize_per_channel(wd)
+        q_ref, s_ref, _ = qo.int8_quantize_per_channel(w.float().numpy())
+        np.testing.assert_array_equal(q.cpu().numpy(), q_ref)
+        np.testing.assert_array_equal(s.cpu().numpy(), s_ref)
