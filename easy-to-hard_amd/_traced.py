@@ -435,6 +435,7 @@ def int4_staged_partial_slices(rows, lin):
 _norm_conv_eager = _seq.norm_conv
 _window_attention_eager, _hgrn2_eager, _gated_delta_eager = _seq.window_attention, _seq.hgrn2, _seq.gated_delta
 _rotary_table_eager, _route_eager, _experts_eager = _seq.rotary_table, _seq.route, _seq.experts
+_linear_eager = _seq.linear
 _square_relu_eager, _softcap_eager, _gelu_gate_eager = _seq.square_relu_, _seq.softcap_, _seq.gelu_gate_rows
 
 
@@ -455,6 +456,10 @@ def _seq_square_relu(x: Tensor) -> None:
 
 def _seq_softcap(x: Tensor, cap: float) -> None:
     _softcap_eager(x, cap)
+
+
+def _seq_linear(x: Tensor, weight: Tensor, act: int, cap: float) -> Tensor:
+    return _linear_eager(x, weight, act, cap)
 
 
 def _seq_gelu_gate(gate: Tensor, table: Tensor, tokens: Tensor, column: int) -> Tensor:
@@ -514,6 +519,7 @@ _norm_conv_op = _register(
     mutates=("tail_out",))
 _square_relu_op = _register("seq_square_relu", _seq_square_relu, _nothing, mutates=("x",))
 _softcap_op = _register("seq_softcap", _seq_softcap, _nothing, mutates=("x",))
+_linear_op = _register("seq_linear", _seq_linear, lambda x, weight, act, cap: x.new_empty((*x.shape[:-1], weight.shape[0])))
 _gelu_gate_op = _register("seq_gelu_gate_rows", _seq_gelu_gate, lambda gate, table, tokens, column: torch.empty_like(gate))
 _window_attention_op = _register("seq_window_attention", _seq_window_attention, _nothing, mutates=("k_cache", "v_cache", "out"))
 _hgrn2_op = _register("seq_hgrn2", _seq_hgrn2, _nothing, mutates=("state", "out"))
@@ -542,6 +548,10 @@ def square_relu_(x):
 def softcap_(x, cap):
     _softcap_op(x, cap)
     return x
+
+
+def linear(x, weight, act=0, cap=0.0):
+    return _linear_op(x, weight, act, cap)
 
 
 def gelu_gate_rows(gate, table, tokens, column):
@@ -577,7 +587,7 @@ def experts(x, chosen, up, down, shared_up=None, shared_down=None):
     return out, (shared if shared_up is not None else None)
 
 
-_SEQ_REBOUND = ("norm_conv", "rotary_table", "route", "experts", "square_relu_", "softcap_", "gelu_gate_rows", "window_attention", "hgrn2", "gated_delta")
+_SEQ_REBOUND = ("norm_conv", "rotary_table", "route", "experts", "square_relu_", "softcap_", "linear", "gelu_gate_rows", "window_attention", "hgrn2", "gated_delta")
 
 _REBOUND = (
     "rmsnorm", "add_rmsnorm", "silu_mul", "rope_kv_write", "rope_kv_write_seq", "decode_attention", "argmax_rows", "int4_mm_silu_gate",

@@ -53,8 +53,7 @@ extern "C" int e2h_set_option(const char *name, int value) {
   }
   if (!strcmp(name, "int8_k_groups")) {
     if (value < 0 || value > 2) return E2H_ERR_BAD_OPTION;
-    o.int8_k_groups = value;
-    return E2H_OK;
+    return E2H_OK;  // taken for callers that set it: the split of K over waves is fixed
   }
   if (!strcmp(name, "int8_force_generic")) {
     o.int8_force_generic = value != 0;
@@ -62,8 +61,7 @@ extern "C" int e2h_set_option(const char *name, int value) {
   }
   if (!strcmp(name, "int8_k_slices")) {
     if (value < 0 || value > 16) return E2H_ERR_BAD_OPTION;
-    o.int8_k_slices = value;
-    return E2H_OK;
+    return E2H_OK;  // likewise
   }
   if (!strcmp(name, "int4_no_xsum")) {
     o.int4_no_xsum = value != 0;

@@ -39,14 +39,12 @@ struct Options {
   int int4_k_slices;       // 0 = heuristic, else 1..16 workgroups along K
   int int4_k_groups;       // 0 = heuristic, else 1/2/4 k-groups inside a workgroup
   int int4_col_waves;      // 0 = heuristic, else 1..4 column waves per k-group
-  int int8_rows_per_wave;  // 0 = heuristic, else 16/32/64
-  int int8_k_groups;       // 0 = heuristic, else 1/2
-  int int8_k_slices;       // 0 = heuristic, else 1..16
+  int int8_rows_per_wave;  // 0 = heuristic, else 16/32/64 (calls of more than 64 rows and the generic kernel)
   int int8_force_generic;  // 1 = always use the generic (bounds-checked) int8 kernel
   int int4_no_xsum;        // 1 = many-row int4 calls compute the group sums of x inside the matmul (no pre-pass)
   int int4_no_gemm32;      // 1 = many-row calls (int4 and int8) stay on the 16x16-tile kernels
   int int4_gemm32_min_rows;  // 0 = by workgroup count, else rows from which the 32x32-tile kernels take over
-  int row_tiles;           // 0 = heuristic, else 1/2/4 tiles of 16 activation rows per workgroup (both matmuls)
+  int row_tiles;           // 0 = heuristic, else 1/2/4 tiles of 16 activation rows per workgroup (int4)
   int attention_waves;     // 0 = by cache length, else 4 or 8 waves per decode-attention workgroup
   int attention_no_mfma;   // 1 = grouped-query decode attention stays on the float32 vector kernel
   int int8_gemm_tile;      // 0 = heuristic, else 128 or 256 rows per workgroup in the many-row int8 matmul
@@ -75,8 +73,7 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 int int8_gemm32(const uint16_t *x, const int8_t *q, const uint16_t *scales, uint16_t *y, int M, int N, int K, hipStream_t stream);
 
 // streaming int8 matmul (e2h_int8_stream.hip)
-int int8_stream_mm(const uint16_t *x, const int8_t *q, const uint16_t *scales, uint16_t *y, int M, int N, int K, void *workspace,
-                   int64_t workspace_bytes, hipStream_t stream);
+int int8_stream_mm(const uint16_t *x, const int8_t *q, const uint16_t *scales, uint16_t *y, int M, int N, int K, hipStream_t stream);
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 

@@ -14,6 +14,7 @@
 // chunks and are summed through LDS in a fixed order.  Epilogue as the reference: round the float32 sum
 // to bfloat16 (F.linear's output), multiply by the bfloat16 scale, round again.
 #include "e2h_common.h"
+#include "e2h_stream.h"
 
 namespace e2h {
 namespace {
@@ -200,9 +201,10 @@ extern "C" int e2h_int8_mm(const uint16_t *x, const int8_t *q, const uint16_t *s
     return E2H_ERR_MISALIGNED;
   const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k);
   if (workspace && !aligned16(workspace)) return E2H_ERR_MISALIGNED;
-  // streaming kernel: K in whole 128-wide chunks, 16-byte aligned rows, weight matrix below 4 GB
-  if ((K % 128) == 0 && aligned16(x) && aligned16(q) && n * k < (int64_t{1} << 32) && !options().int8_force_generic)
-    return int8_stream_mm(x, q, scales, y, M, N, K, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+  // streaming kernels: 16-byte aligned rows; many rows also K in whole 128-wide chunks and a weight matrix below 4 GB
+  if (aligned16(x) && aligned16(q) && !options().int8_force_generic &&
+      (stream::takes(M, N, K, 1) || ((K % 128) == 0 && n * k < (int64_t{1} << 32))))
+    return int8_stream_mm(x, q, scales, y, M, N, K, static_cast<hipStream_t>(stream));
   const bool guard = (K % kChunk) != 0 || !aligned16(x) || !aligned16(q);
   const int mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
   int t = options().int8_rows_per_wave / 16;

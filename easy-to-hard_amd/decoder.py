@@ -11,6 +11,7 @@ import torch.nn as nn
 from torch import Tensor
 
 from . import ops, seq_ops
+from .linear import fusable
 from .state import SequenceState, StatePlan, rotary_turns
 
 
@@ -72,9 +73,13 @@ class StatefulDecoder(nn.Module):
             input_pos = input_pos.to(torch.int64).contiguous()
         first = None if left_pad_mask_pos is None else left_pad_mask_pos.to(torch.int64).contiguous()
         h = self._hidden(idx, bsz, seqlen, state, input_pos, first)
-        logits = self.output(h[:, -1:] if greedy_token else h)
-        if self.logit_softcap is not None:
-            logits = seq_ops.softcap_(logits.contiguous(), self.logit_softcap)
+        h = h[:, -1:] if greedy_token else h
+        if self.logit_softcap is not None and fusable(self.output, h):
+            logits = seq_ops.linear(h, self.output.weight, seq_ops.ACT_SOFTCAP, self.logit_softcap)
+        else:
+            logits = self.output(h)
+            if self.logit_softcap is not None:
+                logits = seq_ops.softcap_(logits.contiguous(), self.logit_softcap)
         if not greedy_token:
             return logits
         last = logits[:, -1]

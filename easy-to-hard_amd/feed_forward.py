@@ -7,15 +7,18 @@ import torch.nn as nn
 from torch import Tensor
 
 from . import seq_ops
+from .linear import DecodeLinear, fusable
 
 
 class SquaredReluFF(nn.Module):
     def __init__(self, width: int, hidden: int):
         super().__init__()
-        self.up = nn.Linear(width, hidden, bias=False)
-        self.down = nn.Linear(hidden, width, bias=False)
+        self.up = DecodeLinear(width, hidden, bias=False)
+        self.down = DecodeLinear(hidden, width, bias=False)
 
     def forward(self, h: Tensor) -> Tensor:
+        if fusable(self.up, h):
+            return self.down(seq_ops.linear(h, self.up.weight, seq_ops.ACT_SQUARE_RELU))
         return self.down(seq_ops.square_relu_(self.up(h)))
 
 
@@ -40,7 +43,7 @@ class ExpertMixture(nn.Module):
 
     def forward(self, h: Tensor) -> Tuple[Optional[Tensor], Tensor, Tensor]:
         chosen, weights = seq_ops.route(h, self.router, self.router_bias, self.top)
-        if self.shared is not None and h.shape[0] <= self.STEP_ROWS and type(self.shared.up) is nn.Linear and type(self.shared.down) is nn.Linear:
+        if self.shared is not None and h.shape[0] <= self.STEP_ROWS and all(type(m) in (nn.Linear, DecodeLinear) for m in (self.shared.up, self.shared.down)):
             out, shared = seq_ops.experts(h, chosen, self.up, self.down, self.shared.up.weight, self.shared.down.weight)
             return shared, out, weights
         out, _ = seq_ops.experts(h, chosen, self.up, self.down)

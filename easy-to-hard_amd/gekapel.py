@@ -18,6 +18,7 @@ import torch.nn as nn
 from . import seq_ops
 from .decoder import StatefulDecoder
 from .feed_forward import ExpertMixture
+from .linear import DecodeLinear
 from .mixers import TokenMixer, WindowAttention
 from .state import StatePlan
 
@@ -86,7 +87,7 @@ class Gekapel(StatefulDecoder):
         for i in range(len(config.layers)):
             self.layers.append(GekapelLayer(self.plan, config, i, self.layers))
         self.norm, self.norm_bias = _vector(config.dim), _vector(config.dim)
-        self.output = nn.Linear(config.dim, config.vocab_size, bias=False)
+        self.output = DecodeLinear(config.dim, config.vocab_size, bias=False)
         self.add_rotations()
 
     @classmethod

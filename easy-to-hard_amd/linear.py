@@ -1,0 +1,24 @@
+"""Plain bfloat16 linears of the stateful decoders: nn.Linear to everything that holds, converts or hooks it, with the streamed-weights
+kernel behind the few rows of a decode step."""
+
+import torch.nn as nn
+import torch.nn.functional as F
+from torch import Tensor
+from torch.nn.modules import module as _module
+
+from . import seq_ops
+
+
+class DecodeLinear(nn.Linear):
+    def forward(self, x: Tensor) -> Tensor:
+        if self.bias is None and seq_ops.linear_streams(x, self.weight):
+            return seq_ops.linear(x, self.weight)
+        return F.linear(x, self.weight, self.bias)
+
+
+def fusable(lin: nn.Module, x: Tensor) -> bool:
+    """True where lin(x) may be computed together with what follows it: the module itself (not a replacement), nobody watching its
+    call, and an input that its kernel takes."""
+    return (type(lin) is DecodeLinear and lin.bias is None and seq_ops.linear_streams(x, lin.weight)
+            and not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks
+                     or _module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks))

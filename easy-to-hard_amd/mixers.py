@@ -6,7 +6,7 @@ all their input projections are one linear and all their output projections anot
 outputs, so a mixer costs two matrix products however many branches it has.  A branch's share of the sum is a factor its
 kernel applies before the output projection.
 
-The two linears are plain nn.Linear modules: a QuantHandler can replace them like any other.
+The two linears are nn.Linear modules: a QuantHandler can replace them like any other.
 """
 
 from typing import Optional
@@ -16,6 +16,7 @@ import torch.nn as nn
 from torch import Tensor
 
 from . import seq_ops
+from .linear import DecodeLinear
 from .state import SequenceState, StatePlan
 
 _ALIGN = 8  # projections start at multiples of this many columns (16 bytes in bfloat16)
@@ -139,8 +140,8 @@ class TokenMixer(nn.Module):
         offset = 0
         for b in self.branches:
             offset = b.place(offset)
-        self.in_proj = nn.Linear(width, (offset + _ALIGN - 1) // _ALIGN * _ALIGN, bias=False)
-        self.out_proj = nn.Linear(sum(b.out_width for b in self.branches), width, bias=False)
+        self.in_proj = DecodeLinear(width, (offset + _ALIGN - 1) // _ALIGN * _ALIGN, bias=False)
+        self.out_proj = DecodeLinear(sum(b.out_width for b in self.branches), width, bias=False)
 
     def forward(self, h: Tensor, bsz: int, seqlen: int, state: SequenceState, input_pos: Tensor, first, rotary=()) -> Tensor:
         proj = self.in_proj(h)

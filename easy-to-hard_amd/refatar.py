@@ -18,6 +18,7 @@ import torch.nn as nn
 from . import seq_ops
 from .decoder import StatefulDecoder
 from .feed_forward import SquaredReluFF
+from .linear import DecodeLinear
 from .mixers import GatedDelta, HGRN2, TokenMixer, WindowAttention
 from .state import StatePlan
 
@@ -80,8 +81,8 @@ class RefatarLayer(nn.Module):
             self.norm2, self.norm2b = _vector(w), _vector(w)
             self.canon2 = nn.Parameter(torch.zeros((taps, w), dtype=torch.float32), requires_grad=False)
             self.ring2 = plan.add_ring(w, taps, float32=True)
-        self.side_gate = nn.Linear(w, args.side_dim, bias=False)
-        self.side_proj = nn.Linear(args.side_dim, w, bias=False)
+        self.side_gate = DecodeLinear(w, args.side_dim, bias=False)
+        self.side_proj = DecodeLinear(args.side_dim, w, bias=False)
         self.side_norm = _vector(w)
         self.side_column = index * args.side_dim
 
@@ -108,7 +109,7 @@ class Refatar(StatefulDecoder):
         self.side_embeddings = nn.Embedding(config.vocab_size, len(config.layers) * config.side_dim)
         self.layers = nn.ModuleList(RefatarLayer(self.plan, config, i) for i in range(len(config.layers)))
         self.norm = _vector(config.dim)
-        self.output = nn.Linear(config.dim, config.vocab_size, bias=False)
+        self.output = DecodeLinear(config.dim, config.vocab_size, bias=False)
         self.logit_softcap = config.logit_softcap
 
     @classmethod

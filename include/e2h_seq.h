@@ -73,6 +73,17 @@ typedef struct {
 } e2h_norm_conv_args;
 int e2h_seq_norm_conv(const e2h_norm_conv_args *a, void *stream);
 
+/* y = act(x w^T) for the few rows of a decode step: x [rows, k], w [n, k] (nn.Linear.weight), y [rows, n], all bfloat16 and contiguous,
+ * x and w 16-byte aligned; 1 <= rows <= 64, k a multiple of 8.  Sums are float32; the sum is rounded to bfloat16 before the activation
+ * and after it.  act: E2H_SEQ_ACT_NONE, E2H_SEQ_ACT_SQUARE_RELU, or E2H_SEQ_ACT_SOFTCAP with cap > 0.  Some shapes need scratch memory of
+ * e2h_seq_linear_scratch_bytes (4-byte aligned; 0: none, negative: the shape is refused). */
+#define E2H_SEQ_ACT_NONE 0
+#define E2H_SEQ_ACT_SQUARE_RELU 1
+#define E2H_SEQ_ACT_SOFTCAP 2
+int64_t e2h_seq_linear_scratch_bytes(int64_t rows, int64_t n, int64_t k);
+int e2h_seq_linear(const void *x, const void *w, void *y, int64_t rows, int64_t n, int64_t k, int act, float cap, void *scratch,
+                   int64_t scratch_bytes, void *stream);
+
 /* Elementwise steps.  square_relu: y = max(x, 0)^2.  softcap: y = cap tanh(x / cap).  x and y may be the same memory.
  * gelu_gate_rows: y[r, i] = gelu_tanh(gate[r, i]) * table[tokens[r], column + i], i < dim; table rows are ld values long. */
 int e2h_seq_square_relu(int dtype, const void *x, void *y, int64_t n, void *stream);
