@@ -112,8 +112,7 @@ extern "C" int e2h_set_option(const char *name, int value) {
     return E2H_OK;
   }
   if (!strcmp(name, "staged_no_rows64")) {
-    o.staged_no_rows64 = value != 0;
-    return E2H_OK;
+    return E2H_OK;  // taken for callers that set it: one kernel covers all row counts
   }
   if (!strcmp(name, "attention_no_mfma")) {
     o.attention_no_mfma = value != 0;

@@ -10,20 +10,27 @@
 // group sum of x taken from the staged buffer.  The second sum is a small float32 matrix product over the groups
 // (v_mfma_f32_16x16x4_f32, four groups per instruction).
 //
-// Decomposition: a workgroup is eight waves that split K (each wave a contiguous run of at most C 128-wide chunks of
-// the workgroup's K slice) and all work on the same T tiles of 16 weight rows.  No wave shares anything with another
-// until the end: weights, qparams and activation operands go straight from memory into registers; there is no barrier
-// and no LDS traffic before the last chunk is done.  The code is straight-line over the C chunks with every load at a
-// fixed place in the instruction stream (weights DW chunks ahead, activation operands DX chunks ahead, pinned with
-// scheduling barriers: left alone, the compiler's scheduler sinks each load to its first use).  The eight partial
-// tiles meet once in LDS; wave w adds and finishes the (column tile, row tile) units w, w + 8, .. in k order, a fixed
-// order, so results are deterministic.  S workgroups may split K further (partial epilogue only): their float32 sums
-// go to slice s of a [S][M][N] array for the consumer to add in slice order.
+// Decomposition: a workgroup is eight waves that split K (each wave a contiguous run of 128-wide chunks of the workgroup's K slice)
+// and all work on the same T tiles of 16 weight rows and on all rows of the batch, so that weights are read once.  No wave
+// shares anything with another until the end.  The eight partial tiles meet in LDS; wave w adds and finishes the (column tile, row
+// tile) units w, w + 8, .. in a fixed order, so results are deterministic.  S workgroups may split K further (partial epilogue
+// only): their float32 sums go to slice s of a [S][M][N] array for the consumer to add in slice order.
 //
-// Measured on MI355X at 32 rows, 7B shapes (the kernel this replaces in brackets): 12288 x 4096 10.5 us (13.5),
-// 4096 x 4096 6.0 (8.9), 4096 x 11008 10.5 (13.6), gated 2 x 11008 x 4096 15.9 (19.5).  Timed by omission on
-// 12288 x 4096: launch + first round trip + meeting + stores 4.0 us, arithmetic 0.5, the weight stream 3.2 (25 MB, the
-// HBM rate), the activation operands 2.9 (every CU reads all 256 KB of them from its L2).
+// What a wave needs passes in units of 1 KB through a ring of its own in LDS, written by loads that touch no register: per chunk the
+// packed words of T tiles, their (scale, zero) pairs, then the activation operands 32 k at a time.  A unit is 16 rows of four 16-byte
+// pieces; piece b of row r stands at b ^ (r / 4 mod 4), which keeps the four lanes of a request on one 64-byte segment and the
+// operand reads free of bank conflicts.  Units move from the ring into registers as they land and their places are refilled at once, so
+// 16 KB per wave are on their way while the matrix cores work on a group.  Waits count loads; there is no barrier in the loop.
+//
+// What bounds it: up to 32 rows the stream of the words (4.2 - 5 TB/s where a launch has a full round of workgroups), at 33 .. 64 rows
+// the unpacking and the matrix cores as well.  Loads straight into registers, 16 rows of 64 bytes apart per request and at most two
+// chunks ahead, left the short k runs waiting for memory; slabs of 32 rows read the words twice.  Measured on MI355X, weights from HBM,
+// loads in registers -> ring (rows; N x K, group size):
+//   1 row:    q|k|v 10240 x 8192, g64 16.4 -> 14.3 us; w1|w3 22016 x 8192 46.5 -> 43.6; w2 8192 x 22016 29.6 -> 21.5; head 34.3 -> 31.1
+//   32 rows:  w1|w3 11008 x 4096, g128 16.2 -> 15.8 us; w2 4096 x 11008 10.3 -> 9.6; w2 8192 x 22016, g64 37.8 -> 27.2; head 41.9 -> 35.5
+//   64 rows:  q|k|v 10240 x 8192, g64 36.4 -> 27.0 us; wo 8192 x 8192 21.2 -> 16.8; w1|w3 102 -> 83.8; w2 48.5 -> 42.5; head 76 -> 58.4
+#include <type_traits>
+
 #include "e2h_common.h"
 #include "e2h_int4_unpack.h"
 #include "e2h_staged.h"
@@ -53,25 +60,65 @@ struct StagedArgs {
   unsigned long long *cand;  // [column blocks][M] (arg-max): per row the best (value key << 32 | ~column) of the block's columns
   StagedOut out;        // gate: the result in staged form for the next linear (frag null: not wanted)
   int M, Mpad, N, K;
-  int slabs, col_blocks;
+  int col_blocks;
   StagedRope rope;
 };
 
-// G group size; MT row tiles of 16 per workgroup; T weight tiles of 16 rows per workgroup (GATE: T/2 of each matrix);
-// C chunks a wave has at most; DW / DX prefetch distance of weights / activation operands in chunks.
-template <int G, int MT, int T, int C, int DW, int DX, int EPI>
+typedef __attribute__((address_space(3))) void lds_void;
+
+// until at most n (a constant once the loop around the call is unrolled) of this wave's loads are out
+__device__ __forceinline__ void wait_units(int n) {
+  switch (n) {
+#define E2H_WAIT(N) \
+  case N: asm volatile("s_waitcnt vmcnt(" #N ")" ::: "memory"); break;
+    E2H_WAIT(1) E2H_WAIT(2) E2H_WAIT(3) E2H_WAIT(4) E2H_WAIT(5) E2H_WAIT(6) E2H_WAIT(7) E2H_WAIT(8) E2H_WAIT(9) E2H_WAIT(10) E2H_WAIT(11)
+    E2H_WAIT(12) E2H_WAIT(13) E2H_WAIT(14) E2H_WAIT(15)
+#undef E2H_WAIT
+    default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+}
+
+// until at most n of this wave's LDS reads are out
+__device__ __forceinline__ void wait_reads(int n) {
+  switch (n) {
+#define E2H_WAIT(N) \
+  case N: asm volatile("s_waitcnt lgkmcnt(" #N ")" ::: "memory"); break;
+    E2H_WAIT(0) E2H_WAIT(1) E2H_WAIT(2) E2H_WAIT(3) E2H_WAIT(4) E2H_WAIT(5) E2H_WAIT(6) E2H_WAIT(7) E2H_WAIT(8) E2H_WAIT(9) E2H_WAIT(10)
+    E2H_WAIT(11) E2H_WAIT(12) E2H_WAIT(13) E2H_WAIT(14)
+#undef E2H_WAIT
+    default: asm volatile("s_waitcnt lgkmcnt(15)" ::: "memory");
+  }
+}
+
+// operands of the zero-point term: the groups' sums of 16 (16 bytes each) and their (scale, zero) pairs
+template <int RB, int MT, int T, int L>
+struct ZeroPoint {
+  u32x4_t xs[RB][MT][L];
+  uint32_t sz[RB][T];
+};
+
+// G group size; MT row tiles of 16 (all rows of the batch); T weight tiles of 16 rows per workgroup (GATE: T/2 of each matrix).
+template <int G, int MT, int T, int EPI>
 __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const StagedArgs a) {
   constexpr bool GATE = EPI == kStGate;
   static_assert(!GATE || T % 2 == 0, "gate mode pairs the tiles of two matrices");
   constexpr int TC = GATE ? T / 2 : T;     // distinct column tiles per workgroup
   constexpr int NGRP = 128 / G;            // groups per 128-wide chunk
   constexpr int SPG = G / 32;              // MFMA steps per group
-  constexpr int R = (C * NGRP + 3) / 4;    // float32 MFMAs of the zero-point term per (tile, row tile)
+  constexpr int RB = 4 / SPG;              // rounds of four groups whose zero-point operands are requested together: 512 k
   constexpr int kUnits = TC * MT;          // (column tile, row tile) pairs, each finished by one wave
   constexpr int kUnitsPerWave = (kUnits + kWaves - 1) / kWaves;
-  constexpr int kAccFloats = T * MT * 4 * 64;
+  // units of a chunk in the order of their use: pairs, operands, words
+  constexpr int kSz = GATE ? 2 : (T * NGRP + 15) / 16, kHead = kSz + 4 * MT, UC = kHead + T;
+  constexpr int kRing = UC < 4 ? 8 : 16;         // units of 1 KB per wave
+  constexpr int kAhead = (kRing + UC - 1) / UC;  // chunks that the ring reaches into, at most
+  constexpr int kLate = kAhead * UC - kRing;     // units of the last kAhead chunks that are issued while those run
+  static_assert(kSz + MT < kRing && TC * NGRP <= 16 * (GATE ? 1 : kSz), "ring");
+  constexpr bool kTwoSteps = T * MT > 16;        // the eight parts do not fit LDS at once
+  constexpr int kParts = kTwoSteps ? kWaves / 2 : kWaves;
+  constexpr int kRedBytes = kParts * T * MT * 1024, kRingBytes = kWaves * kRing * 1024;
 
-  __shared__ __attribute__((aligned(16))) float red[kWaves * kAccFloats];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kRedBytes > kRingBytes ? kRedBytes : kRingBytes];
   __shared__ unsigned long long unit_best[EPI == kStArgmax ? kUnits : 1][16];  // arg-max: per unit and row of its tile
 
   const int tid = threadIdx.x;
@@ -79,73 +126,51 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
   const int kg = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave = k part
   const int c = lane & 15, b = lane >> 4;
   const int N = a.N, K = a.K, M = a.M;
-  const int n_tiles8 = N >> 3;
   const int KT = K >> 7;  // packed k-blocks (inner_k_tiles = 8) = chunks
   const int S = gridDim.y, ks = blockIdx.y;
   const int C0 = static_cast<int>((static_cast<unsigned>(KT) * static_cast<unsigned>(ks)) / static_cast<unsigned>(S));
   const int C1 = static_cast<int>((static_cast<unsigned>(KT) * static_cast<unsigned>(ks + 1)) / static_cast<unsigned>(S));
   const int c0 = C0 + ((C1 - C0) * kg) / kWaves;
-  const int c1 = C0 + ((C1 - C0) * (kg + 1)) / kWaves;
-  const int nloc = c1 - c0;  // <= C (the host picks C)
-  // Column block and row slab.  With two row slabs (33 .. 64 rows) the slabs of a column block sit 8 workgroups apart:
-  // workgroup i runs on XCD i % 8, so the second slab finds the weights in the same L2.
-  int col_block = blockIdx.x, slab = 0;
-  if (a.slabs > 1) {
-    slab = (blockIdx.x >> 3) % a.slabs;
-    col_block = (blockIdx.x / (8 * a.slabs)) * 8 + (blockIdx.x & 7);
-    if (col_block >= a.col_blocks) return;  // padding of the folded grid; uniform, before any barrier
-  }
+  const int nloc = C0 + ((C1 - C0) * (kg + 1)) / kWaves - c0;
+  const int col_block = blockIdx.x;
   const int tile16_0 = col_block * TC;
-  const int m_base = slab * (16 * MT);
+  const int tiles = (N >> 4) - tile16_0 < TC ? (N >> 4) - tile16_0 : TC;  // N % 16 == 0
   const uint32_t row_block = static_cast<uint32_t>(a.Mpad) * 64u;  // bytes of one k segment of all rows
 
-  uint32_t wlane[T], szlane[T];
-#pragma unroll
-  for (int t = 0; t < T; ++t) {
-    const int tcol = tile16_0 + (GATE ? t % TC : t);
-    int nt8 = 2 * tcol + (c >> 3);
-    nt8 = nt8 < n_tiles8 ? nt8 : n_tiles8 - 1;
-    wlane[t] = static_cast<uint32_t>((static_cast<size_t>(nt8) * KT * 32 + ((c & 7) * 4 + b)) * 16);
-    int ncol = 16 * tcol + c;
-    ncol = ncol < N ? ncol : N - 1;
-    szlane[t] = static_cast<uint32_t>(ncol) * 4u;
-  }
-  const uint32_t xlane = static_cast<uint32_t>((m_base + c) * 64 + 16 * b);  // lane (b, m = c) of row tile 0
-  const uint32_t w_bytes = static_cast<uint32_t>(static_cast<size_t>(N) * K / 2);
+  // this workgroup's tiles are consecutive in the packed words; a (scale, zero) pair of group g and column n is dword g N + n
+  const size_t w_base = static_cast<size_t>(tile16_0) * KT * 1024;
+  const uint32_t w_bytes = static_cast<uint32_t>(tiles) * KT * 1024u;
   const uint32_t sz_bytes = static_cast<uint32_t>(static_cast<size_t>(K / G) * N * 4);
-  const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(a.wp, w_bytes);
+  const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(reinterpret_cast<const uint8_t *>(a.wp) + w_base, w_bytes);
   const __amdgpu_buffer_rsrc_t sz_rsrc = make_rsrc(a.sz, sz_bytes);
-  const __amdgpu_buffer_rsrc_t w2_rsrc = make_rsrc(GATE ? a.wp2 : a.wp, w_bytes);
+  const __amdgpu_buffer_rsrc_t w2_rsrc = make_rsrc(reinterpret_cast<const uint8_t *>(GATE ? a.wp2 : a.wp) + w_base, w_bytes);
   const __amdgpu_buffer_rsrc_t sz2_rsrc = make_rsrc(GATE ? a.sz2 : a.sz, sz_bytes);
   const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(a.frag, static_cast<uint32_t>(static_cast<size_t>(K / 32) * row_block));
   const __amdgpu_buffer_rsrc_t xs_rsrc = make_rsrc(a.sums, static_cast<uint32_t>(static_cast<size_t>(KT) * a.Mpad * 32));
 
-  struct WRegs {
-    u32x4_t w[T];
-    uint32_t sz[T][NGRP];
-  };
-  struct XRegs {
-    u32x4_t x[MT][4];
-  };
-  auto chunk_at = [&](int i) {
-    const int ci = c0 + (i < nloc ? i : nloc - 1);
-    return ci < C0 ? C0 : ci;  // a wave without chunks re-reads the slice's first chunk (its results are scaled by zero)
-  };
-  auto load_x = [&](XRegs &r, int ci) {
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-        r.x[mt][s] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xlane + mt * 1024, static_cast<uint32_t>(ci * 4 + s) * row_block, 0);
-  };
-  auto load_w = [&](WRegs &r, int ci) {
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-      const bool second = GATE && t >= TC;
-      r.w[t] = __builtin_amdgcn_raw_buffer_load_b128(second ? w2_rsrc : w_rsrc, wlane[t], static_cast<uint32_t>(ci) * 512u, kNt);
-#pragma unroll
-      for (int g = 0; g < NGRP; ++g)
-        r.sz[t][g] = __builtin_amdgcn_raw_buffer_load_b32(second ? sz2_rsrc : sz_rsrc, szlane[t], static_cast<uint32_t>(ci * NGRP + g) * static_cast<uint32_t>(N) * 4u, 0);
+  uint8_t *const ring = lds + kg * (kRing * 1024);
+  // what lane 4 q + s brings: piece s ^ (q / 4 mod 4) of row q
+  const int q4 = lane >> 2;
+  const uint32_t piece = static_cast<uint32_t>((lane & 3) ^ ((lane >> 4) & 3)) * 16u;
+  const uint32_t w_lane = static_cast<uint32_t>(q4 >> 3) * KT * 512u + (q4 & 7) * 64u + piece;  // rows 0 .. 7, 8 .. 15: two packed tiles
+  const uint32_t x_lane = static_cast<uint32_t>(q4) * 64u + piece;
+  const auto column_of = [&](int t) { return 16 * (tile16_0 + (t < tiles ? t : tiles - 1)); };  // past the end: any valid one
+  // unit p (static) of chunk i of this wave's run into ring place `at`
+  const auto issue = [&](int p, int i, int at) {
+    const uint32_t chunk = static_cast<uint32_t>(c0 + i);
+    lds_void *const dst = (lds_void *)(ring + at * 1024);
+    if (p < kSz) {
+      // 16 bytes (four columns) per lane: pair block q4 = (tile, group) of this unit's sixteen
+      const int blk = q4 + (GATE ? 0 : 16 * p), t = blk / NGRP, g = blk % NGRP;
+      const uint32_t off = (static_cast<uint32_t>(g) * N + column_of(t) + 4u * (lane & 3)) * 4u;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(GATE && p > 0 ? sz2_rsrc : sz_rsrc, dst, 16, off, chunk * (NGRP * 4u) * static_cast<uint32_t>(N), 0, 0);
+    } else if (p < kHead) {
+      const int s = (p - kSz) / MT, mt = (p - kSz) % MT;
+      const uint32_t off = 16 * mt + q4 < M ? x_lane + 1024u * mt : 0x80000000u;  // rows past M: out of the buffer's range, zeros
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, dst, 16, off, (chunk * 4u + s) * row_block, 0, 0);
+    } else {
+      const int t = p - kHead;  // past N: out of the buffer's range, zeros
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(t < TC ? w_rsrc : w2_rsrc, dst, 16, w_lane + static_cast<uint32_t>(t % TC) * KT * 1024u, chunk * 512u, 0, kNt);
     }
   };
 
@@ -156,32 +181,80 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
     for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const UnpackConsts uc = unpack_consts();
 
-  auto compute_chunk = [&](const WRegs &r, const XRegs &rx, uint32_t live) {
+  // ---- the zero-point term: four groups per float32 MFMA, lane (b, .) owns group 4 r + b of the wave's run ---------------
+  const int ngroups = nloc * NGRP;
+  typedef ZeroPoint<RB, MT, T, NGRP == 1 ? 2 : 1> Zero;
+  const auto zero_point_load = [&](Zero &z, int r0) {
 #pragma unroll
-    for (int t = 0; t < T; ++t) {
+    for (int r = 0; r < RB; ++r) {
+      const int gi = 4 * (r0 + r) + b;
+      const int gcl = gi < ngroups ? gi : 0;
+      int chunk = c0 + gcl / NGRP;
+      chunk = chunk < KT ? chunk : KT - 1;
+      const int sub = gcl % NGRP;
+      // chunk and sub differ between lanes: everything goes into the vector offset
+      const uint32_t so = static_cast<uint32_t>(chunk) * static_cast<uint32_t>(a.Mpad) * 32u;
 #pragma unroll
-      for (int g = 0; g < NGRP; ++g) {
-        f32x4_t part[MT];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) part[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < SPG; ++s) {
-          const bf16x8_t wf = unpack_word(r.w[t][g * SPG + s], uc);
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt)
-            part[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, rx.x[mt][g * SPG + s]), wf, part[mt], 0, 0, 0);
+      for (int mt = 0; mt < MT; ++mt) {
+        // the group's 8 / NGRP sums of 16
+        const uint32_t off = so + static_cast<uint32_t>((16 * mt + c) * 32 + sub * (32 / NGRP));
+        if constexpr (NGRP == 1) {
+          z.xs[r][mt][0] = __builtin_amdgcn_raw_buffer_load_b128(xs_rsrc, off, 0, 0);
+          z.xs[r][mt][1] = __builtin_amdgcn_raw_buffer_load_b128(xs_rsrc, off + 16, 0, 0);
+        } else if constexpr (NGRP == 2) {
+          z.xs[r][mt][0] = __builtin_amdgcn_raw_buffer_load_b128(xs_rsrc, off, 0, 0);
+        } else {
+          const u32x2_t lo = __builtin_amdgcn_raw_buffer_load_b64(xs_rsrc, off, 0, 0);
+          z.xs[r][mt][0] = u32x4_t{lo[0], lo[1], 0u, 0u};
         }
-        const float scale = __builtin_bit_cast(float, (r.sz[t][g] & live) << 16);  // live == 0: the chunk adds nothing
+      }
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+      for (int t = 0; t < T; ++t)
+        z.sz[r][t] = __builtin_amdgcn_raw_buffer_load_b32(GATE && t >= TC ? sz2_rsrc : sz_rsrc, static_cast<uint32_t>(column_of(t % TC) + c) * 4u +
+                                                             static_cast<uint32_t>(chunk * NGRP + sub) * static_cast<uint32_t>(N) * 4u, 0, 0);
+    }
+  };
+  const auto zero_point_use = [&](const Zero &z, int r0) {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) acc[t][mt][q] = __builtin_fmaf(scale, part[mt][q], acc[t][mt][q]);
+    for (int r = 0; r < RB; ++r) {
+      const bool live = 4 * (r0 + r) + b < ngroups;
+      float xsum[MT];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const f32x4_t lo = __builtin_bit_cast(f32x4_t, z.xs[r][mt][0]);
+        float v;
+        if constexpr (NGRP == 1) {
+          const f32x4_t hi = __builtin_bit_cast(f32x4_t, z.xs[r][mt][1]);
+          v = ((lo[0] + lo[1]) + (lo[2] + lo[3])) + ((hi[0] + hi[1]) + (hi[2] + hi[3]));
+        } else if constexpr (NGRP == 2) {
+          v = (lo[0] + lo[1]) + (lo[2] + lo[3]);
+        } else {
+          v = lo[0] + lo[1];
+        }
+        xsum[mt] = live ? v : 0.f;
+      }
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const float scale = __builtin_bit_cast(float, z.sz[r][t] << 16);
+        const float zero = __builtin_bit_cast(float, z.sz[r][t] & 0xFFFF0000u);
+        const float zc = live ? __builtin_fmaf(-136.0f, scale, zero) : 0.f;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(xsum[mt], zc, acc[t][mt], 0, 0, 0);
       }
     }
   };
 
+  Zero z0, z1;
+  zero_point_load(z0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < kRing; ++u)
+    if (u / UC < nloc) issue(u % UC, u / UC, u);
+  if (4 * RB < ngroups) zero_point_load(z1, RB);
+  __builtin_amdgcn_sched_barrier(0);
+
   // RoPE epilogue: the rotation's cos / sin depend on a position read from memory; both are fetched now, behind the
-  // first weight loads, for the units this wave will finish
+  // first loads, for the units this wave will finish
   int rope_pos = -1;
   float rope_cs[kUnitsPerWave], rope_sn[kUnitsPerWave];
 #pragma unroll
@@ -189,143 +262,170 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
     rope_cs[u] = 1.f;
     rope_sn[u] = 0.f;
   }
-
-  if (C1 > C0) {
-    // ---- the zero-point term: four groups per float32 MFMA, lane (b, .) owns group 4 r + b of the wave's run -----------
-    // Its operands are requested first and used right after the first chunks have been requested: loads return in issue
-    // order, so waiting for them does not wait for the chunks.
-    const int ngroups = nloc * NGRP;
-    u32x4_t xs_raw[R][MT][NGRP == 1 ? 2 : 1];
-    uint32_t zsz[R][T];
-    bool zlive[R];
+  if constexpr (EPI == kStRope) {
+    const int64_t p = a.rope.input_pos[0];
+    rope_pos = p >= 0 && p < a.rope.S ? static_cast<int>(p) : -1;
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int gi = 4 * r + b;  // group of this lane within the wave's run
-      zlive[r] = gi < ngroups;
-      const int gcl = zlive[r] ? gi : 0;
-      int chunk = c0 + gcl / NGRP;
-      chunk = chunk < C1 ? chunk : C1 - 1;
-      const int sub = gcl % NGRP;
-      // chunk and sub differ between lanes: everything goes into the vector offset
-      const uint32_t so = static_cast<uint32_t>(chunk) * static_cast<uint32_t>(a.Mpad) * 32u;
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        // the 128 / NGRP values of the group: 8 / NGRP sums of 16
-        const uint32_t off = so + static_cast<uint32_t>((m_base + 16 * mt + c) * 32 + sub * (32 / NGRP));
-        if constexpr (NGRP == 1) {
-          xs_raw[r][mt][0] = __builtin_amdgcn_raw_buffer_load_b128(xs_rsrc, off, 0, 0);
-          xs_raw[r][mt][1] = __builtin_amdgcn_raw_buffer_load_b128(xs_rsrc, off + 16, 0, 0);
-        } else if constexpr (NGRP == 2) {
-          xs_raw[r][mt][0] = __builtin_amdgcn_raw_buffer_load_b128(xs_rsrc, off, 0, 0);
-        } else {
-          const u32x2_t lo = __builtin_amdgcn_raw_buffer_load_b64(xs_rsrc, off, 0, 0);
-          xs_raw[r][mt][0] = u32x4_t{lo[0], lo[1], 0u, 0u};
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < T; ++t) {
-        const bool second = GATE && t >= TC;
-        zsz[r][t] = __builtin_amdgcn_raw_buffer_load_b32(second ? sz2_rsrc : sz_rsrc,
-                                                         szlane[t] + static_cast<uint32_t>(chunk * NGRP + sub) * static_cast<uint32_t>(N) * 4u, 0, 0);
-      }
-    }
-    WRegs wr[C];
-    XRegs xr[C];
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < (DW > DX ? DW : DX); ++i) {
-      if (i < DW && i < C) load_w(wr[i], chunk_at(i));
-      if (i < DX && i < C) load_x(xr[i], chunk_at(i));
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (EPI == kStRope) {
-      rope_pos = static_cast<int>(a.rope.input_pos[0]);
-#pragma unroll
-      for (int u = 0; u < kUnitsPerWave; ++u) {
-        const int unit = kg + u * kWaves;
-        const int ncol = 16 * (tile16_0 + unit / MT) + c;
-        if (unit < kUnits && ncol < N && rope_pos >= 0 && rope_pos < a.rope.S && ncol < (a.rope.H + a.rope.Hkv) * a.rope.D) {
-          const uint32_t f = reinterpret_cast<const uint32_t *>(a.rope.freqs)[static_cast<size_t>(rope_pos) * (a.rope.D / 2) + ((ncol % a.rope.D) >> 1)];
-          rope_cs[u] = __builtin_bit_cast(float, f << 16);
-          rope_sn[u] = __builtin_bit_cast(float, f & 0xFFFF0000u);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      float xsum[MT];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const f32x4_t lo = __builtin_bit_cast(f32x4_t, xs_raw[r][mt][0]);
-        float v;
-        if constexpr (NGRP == 1) {
-          const f32x4_t hi = __builtin_bit_cast(f32x4_t, xs_raw[r][mt][1]);
-          v = ((lo[0] + lo[1]) + (lo[2] + lo[3])) + ((hi[0] + hi[1]) + (hi[2] + hi[3]));
-        } else if constexpr (NGRP == 2) {
-          v = (lo[0] + lo[1]) + (lo[2] + lo[3]);
-        } else {
-          v = lo[0] + lo[1];
-        }
-        xsum[mt] = zlive[r] ? v : 0.f;
-      }
-#pragma unroll
-      for (int t = 0; t < T; ++t) {
-        const float scale = __builtin_bit_cast(float, zsz[r][t] << 16);
-        const float zero = __builtin_bit_cast(float, zsz[r][t] & 0xFFFF0000u);
-        const float zc = zlive[r] ? __builtin_fmaf(-136.0f, scale, zero) : 0.f;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(xsum[mt], zc, acc[t][mt], 0, 0, 0);
+    for (int u = 0; u < kUnitsPerWave; ++u) {
+      const int unit = kg + u * kWaves;
+      const int ncol = 16 * (tile16_0 + unit / MT) + c;
+      if (unit < kUnits && ncol < N && rope_pos >= 0 && ncol < (a.rope.H + a.rope.Hkv) * a.rope.D) {
+        const uint32_t f = reinterpret_cast<const uint32_t *>(a.rope.freqs)[static_cast<size_t>(rope_pos) * (a.rope.D / 2) + ((ncol % a.rope.D) >> 1)];
+        rope_cs[u] = __builtin_bit_cast(float, f << 16);
+        rope_sn[u] = __builtin_bit_cast(float, f & 0xFFFF0000u);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
-    // straight-line over the C chunks a wave can have: every load sits at a fixed place in the instruction stream, so
-    // the waits for a chunk's operands never include younger prefetches
-#pragma unroll
-    for (int i = 0; i < C; ++i) {
-      if (i + DW < C) load_w(wr[i + DW], chunk_at(i + DW));
-      if (i + DX < C) load_x(xr[i + DX], chunk_at(i + DX));
-      __builtin_amdgcn_sched_barrier(0);
-      compute_chunk(wr[i], xr[i], i < nloc ? 0xFFFFFFFFu : 0u);
-      __builtin_amdgcn_sched_barrier(0);
-    }
   }
+  zero_point_use(z0, 0);
+  if (4 * RB < ngroups) {
+    for (int r0 = 2 * RB; 4 * r0 < ngroups; r0 += RB) {
+      zero_point_load(z0, r0);
+      zero_point_use(z1, r0 - RB);
+      z1 = z0;
+    }
+    zero_point_use(z1, (ngroups - 1) / (4 * RB) * RB);
+  }
+  __builtin_amdgcn_sched_barrier(0);
 
-  // ---- the eight K parts meet in LDS; wave w finishes units w, w + 8, .. --------------------------------------------
-  {
-    float *mine = red + kg * kAccFloats + lane;
+  // ---- the chunks -------------------------------------------------------------------------------------------------
+  const uint32_t read_lane = c * 64u + ((b ^ ((c >> 2) & 3)) * 16u);  // lane (b, c): piece b of row c
+  // kTail -1: a chunk with kAhead or more behind it; 0 .. kAhead - 1: the last ones, for which ever less is left to issue; kAhead: all has landed
+  const auto chunk = [&](auto tail, int i, int at0) {
+    constexpr int kTail = decltype(tail)::value;
+    constexpr bool kSteady = kTail < 0, kDone = kTail == kAhead;
+    // A batch of n units from p0 on, behind one of `before` units whose places are refilled only once this batch's reads are on their
+    // way, so that no wave waits for its own reads.  Loads that may still be out: the ring's younger units.
+    const auto landed = [&](int p0, int n, int before) {
+      if (kDone) return;
+      const int issued = kTail * UC + p0 - before + kRing, all = kAhead * UC;
+      const int younger = kSteady ? kRing - before - n : (issued < all ? issued : all) - (kTail * UC + p0 + n);
+      wait_units(younger);
+    };
+    const auto at = [&](int p) { return (at0 + p) & (kRing - 1); };
+    // the places of units p0 .. p0 + n - 1 of chunk j, whose reads are followed by `later` newer ones; j_tail: kTail of that chunk
+    const auto refill = [&](int j, int j_tail, int j_at0, int p0, int n, int later) {
+      if (kDone) return;
+      wait_reads(later);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int p = p0; p < p0 + n; ++p)
+        if (j_tail < 0 || j_tail * UC + p < kLate) issue((p + kRing) % UC, j + (p + kRing) / UC, (j_at0 + p) & (kRing - 1));
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    uint32_t sz[T][NGRP];
+    landed(0, kSz, 1);
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
+      for (int g = 0; g < NGRP; ++g) {
+        const int blk = (t % TC) * NGRP + g;
+        sz[t][g] = *reinterpret_cast<const uint32_t *>(ring + at(GATE ? t / TC : blk / 16) * 1024 + (blk % 16) * 64 + c * 4);
+      }
+    if (i > 0) refill(i - 1, kTail < 0 ? -1 : kTail - 1, at0 - UC, UC - 1, 1, T * NGRP);  // the previous chunk's last batch
+    bf16x8_t x[4][MT];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) mine[((t * MT + mt) * 4 + q) * 64] = acc[t][mt][q];
+    for (int s = 0; s < 4; ++s) {
+      const int p0 = kSz + s * MT, before = s == 0 ? kSz : MT;
+      landed(p0, MT, before);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) x[s][mt] = *reinterpret_cast<const bf16x8_t *>(ring + at(p0 + mt) * 1024 + read_lane);
+      refill(i, kTail, at0, p0 - before, before, MT);
+    }
+    u32x4_t w[2];
+#pragma unroll
+    for (int t = 0; t < T + 1; ++t) {
+      if (t < T) {
+        const int before = t > 0 ? 1 : MT;
+        landed(kHead + t, 1, before);
+        w[t & 1] = *reinterpret_cast<const u32x4_t *>(ring + at(kHead + t) * 1024 + read_lane);
+        refill(i, kTail, at0, kHead + t - before, before, 1);
+      }
+      if (t == 0) continue;
+#pragma unroll
+      for (int g = 0; g < NGRP; ++g) {
+        f32x4_t part[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) part[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < SPG; ++s) {
+          const bf16x8_t wf = unpack_word(w[(t - 1) & 1][g * SPG + s], uc);
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) part[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[g * SPG + s][mt], wf, part[mt], 0, 0, 0);
+        }
+        const float scale = __builtin_bit_cast(float, sz[t - 1][g] << 16);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) acc[t - 1][mt][q] = __builtin_fmaf(scale, part[mt][q], acc[t - 1][mt][q]);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int i = 0, at0 = 0;
+  const auto run = [&](auto tail) {
+    chunk(tail, i, at0);
+    at0 = (at0 + UC) & (kRing - 1);
+    ++i;
+  };
+#pragma unroll 1
+  while (i < nloc - kAhead) run(std::integral_constant<int, -1>{});
+  if (nloc >= kAhead) {
+    run(std::integral_constant<int, 0>{});
+    if constexpr (kAhead > 1) run(std::integral_constant<int, 1>{});
+    if constexpr (kAhead > 2) run(std::integral_constant<int, 2>{});
+    if constexpr (kAhead > 3) run(std::integral_constant<int, 3>{});
+    static_assert(kAhead <= 4, "ring");
   }
-  __syncthreads();
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll 1
+  while (i < nloc) run(std::integral_constant<int, kAhead>{});  // a wave with fewer chunks than the ring holds
+
+  // ---- the eight K parts meet in LDS as a balanced tree in the order of K; wave w finishes units w, w + 8, .. -------------
+  float *const red = reinterpret_cast<float *>(lds);
+  const auto put = [&](int part) {
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) *reinterpret_cast<f32x4_t *>(red + ((part * T * MT + t * MT + mt) * 64 + lane) * 4) = acc[t][mt];
+  };
+  const auto get = [&](int part, int t, int mt) { return *reinterpret_cast<const f32x4_t *>(red + ((part * T * MT + t * MT + mt) * 64 + lane) * 4); };
+  lds_barrier();  // the rings are done with
+  if constexpr (kTwoSteps) {
+    if (kg & 1) put(kg >> 1);
+    lds_barrier();
+    if (!(kg & 1)) {
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[t][mt] += get(kg >> 1, t, mt);
+    }
+    lds_barrier();
+    if (!(kg & 1)) put(kg >> 1);
+  } else {
+    put(kg);
+  }
+  lds_barrier();
 #pragma unroll
   for (int u = 0; u < kUnitsPerWave; ++u) {
     const int unit = kg + u * kWaves;
     if (unit >= kUnits) break;  // uniform per wave
     const int tc = unit / MT, mt = unit % MT;
-    float v[GATE ? 2 : 1][4];
+    f32x4_t v[GATE ? 2 : 1];
 #pragma unroll
     for (int h = 0; h < (GATE ? 2 : 1); ++h) {
       const int t = tc + h * TC;
+      f32x4_t pair[kWaves / 2];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float *src = red + ((t * MT + mt) * 4 + q) * 64 + lane;
-        float s = src[0];
-#pragma unroll
-        for (int w = 1; w < kWaves; ++w) s += src[w * kAccFloats];
-        v[h][q] = s;
-      }
+      for (int w = 0; w < kWaves / 2; ++w) pair[w] = kTwoSteps ? get(w, t, mt) : get(2 * w, t, mt) + get(2 * w + 1, t, mt);
+      v[h] = (pair[0] + pair[1]) + (pair[2] + pair[3]);
     }
     const int n = 16 * (tile16_0 + tc) + c;
     if constexpr (EPI == kStPartial) {
       float *out = a.partials + static_cast<size_t>(ks) * M * N;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int m = m_base + 16 * mt + 4 * b + q;
+        const int m = 16 * mt + 4 * b + q;
         if (n < N && m < M) out[static_cast<size_t>(m) * N + n] = v[0][q];
       }
     } else if constexpr (EPI == kStGate) {
@@ -334,7 +434,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
       const bool tile_live = 16 * (tile16_0 + tc) < N;  // whole tiles: N % 16 == 0 on this path
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int m = m_base + 16 * mt + 4 * b + q;
+        const int m = 16 * mt + 4 * b + q;
         const float gate = bf16_round(v[0][q]), up = bf16_round(v[1][q]);
         const float act = bf16_round(gate / (1.0f + expf(-gate)));
         const uint16_t o = f32_to_bf16_rne(act * up);
@@ -350,7 +450,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
       const int Dh = rp.D, H = rp.H, Hkv = rp.Hkv;
       const int pos = rope_pos;
       const int head = n / Dh, d = n % Dh;
-      const bool in_range = n < N && pos >= 0 && pos < rp.S;
+      const bool in_range = n < N && pos >= 0;
       const bool rotated = head < H + Hkv;
       const float cs = rope_cs[u], sn = rope_sn[u];
       uint16_t *dst;
@@ -360,12 +460,12 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
         row_stride = static_cast<size_t>(H) * Dh;
       } else {
         const int hk = rotated ? head - H : head - H - Hkv;
-        dst = (rotated ? rp.kc : rp.vc) + (static_cast<size_t>(hk) * rp.S + pos) * Dh + d;
+        dst = (rotated ? rp.kc : rp.vc) + (static_cast<size_t>(hk) * rp.S + (pos < 0 ? 0 : pos)) * Dh + d;
         row_stride = static_cast<size_t>(Hkv) * rp.S * Dh;
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int m = m_base + 16 * mt + 4 * b + q;
+        const int m = 16 * mt + 4 * b + q;
         const float own = bf16_round(v[0][q]);
         const float other = __shfl_xor(own, 1);  // the pair's other column lives in the neighbouring lane
         const float r = (c & 1) ? own * cs + other * sn : own * cs - other * sn;
@@ -391,7 +491,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
     } else {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int m = m_base + 16 * mt + 4 * b + q;
+        const int m = 16 * mt + 4 * b + q;
         if (n < N && m < M) a.y[static_cast<size_t>(m) * N + n] = f32_to_bf16_rne(v[0][q]);
       }
     }
@@ -400,7 +500,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
     // ... then over the workgroup's column tiles: one candidate per row and column block for the reduction kernel
     __syncthreads();
     if (tid < 16 * MT) {
-      const int mt = tid >> 4, m = m_base + tid;
+      const int mt = tid >> 4, m = tid;
       unsigned long long best = 0ull;
 #pragma unroll
       for (int tc = 0; tc < TC; ++tc) best = unit_best[tc * MT + mt][tid & 15] > best ? unit_best[tc * MT + mt][tid & 15] : best;
@@ -439,84 +539,49 @@ __global__ __launch_bounds__(256) void int4_stage_x_kernel(const uint16_t *__res
 
 // ---- launch geometry ---------------------------------------------------------------------------------------------------
 struct Geometry {
-  int t, c, dw, dx;  // kernel instantiation
-  int slices;        // workgroups along K
+  int t, slices;  // weight tiles per workgroup, workgroups along K
 };
 
-// instantiated (T, C, DW, DX) per epilogue; registers: about 8 T (sums) + DW * 5 T (weights) + DX * 32 (operands) + 50
-struct Inst {
-  int t, c, dw, dx;
-};
-constexpr Inst kPlainInsts[] = {{3, 4, 2, 2}, {4, 4, 2, 2}, {8, 4, 1, 1}, {6, 4, 2, 1}, {2, 2, 2, 2}, {4, 2, 2, 2}, {6, 2, 2, 2}, {4, 1, 1, 1}, {4, 3, 3, 1}, {4, 8, 2, 1}, {8, 8, 1, 1}, {2, 1, 1, 1}};
-constexpr Inst kArgmaxInsts[] = {{8, 4, 1, 1}, {4, 4, 2, 2}, {8, 8, 1, 1}, {4, 8, 2, 1}, {4, 1, 1, 1}, {2, 1, 1, 1}};  // LM heads: few K shapes
-constexpr Inst kGateInsts[] = {{6, 4, 2, 1}, {4, 4, 2, 2}, {8, 4, 1, 1}, {6, 8, 1, 1}, {8, 8, 1, 1}};
+// most weight tiles whose sums, words, pairs and operands fit a wave's 256 vector registers beside the group's products
+constexpr int max_tiles(int G, int MT, bool gate) { return MT == 4 ? 6 : gate && G != 32 ? 12 : 8; }
 
-// instantiations that do not fit the 256 vector registers of a wave (they would run, slowly, out of scratch memory):
-// smaller groups carry more (scale, zero) pairs per chunk and more rounds of the zero-point term
-inline bool fits_registers(int groupsize, const Inst &in) {
-  if (groupsize == 32) return !((in.t >= 3 && in.c == 4) || in.t >= 6);
-  if (groupsize == 64) return !(in.t == 8 || (in.t == 4 && in.c == 4));
-  return true;
-}
-
-template <int NI>
-bool pick(const Inst (&insts)[NI], bool gate, int groupsize, int tiles16, int kt, int slabs, int max_slices, Geometry *best) {
-  long best_cost = -1;
-  const int want_t = options().staged_tiles, want_s = options().staged_slices;  // experiments: force a geometry
-  for (int s = 1; s <= max_slices; s *= 2) {
-    if (want_s && s != want_s) continue;
-    if (s > kt) break;
-    const int per_slice = (kt + s - 1) / s;  // the longest slice
-    const int c_need = (per_slice + kWaves - 1) / kWaves;
-    for (const Inst &in : insts) {
-      if (in.c != c_need || !fits_registers(groupsize, in)) continue;
-      if (want_t && !gate && in.t != want_t) continue;
-      const int tc = gate ? in.t / 2 : in.t;
-      const long wgs = static_cast<long>((tiles16 + tc - 1) / tc) * s * slabs;
-      const long rounds = (wgs + kCUs - 1) / kCUs;
-      // per workgroup: a fixed part, the weight tiles, the activation operands of its chunks (about two tiles' worth each);
-      // per slice: what the consumer pays to add it
-      const long cost = rounds * (4 + static_cast<long>(in.t) * in.c + 2L * in.c) * 2 + 2L * s;
-      if (best_cost < 0 || cost < best_cost) {
-        best_cost = cost;
-        *best = Geometry{in.t, in.c, in.dw, in.dx, s};
-      }
-    }
-  }
-  return best_cost >= 0;
-}
-
-template <int G, int MT, int T, int C, int DW, int DX, int EPI>
+template <int G, int MT, int T, int EPI>
 int launch_staged(const StagedArgs &a, int slices, hipStream_t stream) {
-  const unsigned gx = a.slabs > 1 ? static_cast<unsigned>((a.col_blocks + 7) / 8 * 8 * a.slabs) : static_cast<unsigned>(a.col_blocks);
-  hipLaunchKernelGGL((int4_staged_mm_kernel<G, MT, T, C, DW, DX, EPI>), dim3(gx, slices, 1), dim3(64 * kWaves), 0, stream, a);
-  return launch_status();
+  if constexpr (T > max_tiles(G, MT, EPI == kStGate)) {
+    return E2H_ERR_BAD_SHAPE;
+  } else {
+    hipLaunchKernelGGL((int4_staged_mm_kernel<G, MT, T, EPI>), dim3(a.col_blocks, slices), dim3(64 * kWaves), 0, stream, a);
+    return launch_status();
+  }
 }
 
 template <int G, int MT, int EPI>
-int dispatch_inst(const StagedArgs &a, const Geometry &g, hipStream_t stream) {
-#define E2H_ST_CASE(TV, CV, DWV, DXV) \
-  if (g.t == TV && g.c == CV && g.dw == DWV && g.dx == DXV) return launch_staged<G, MT, TV, CV, DWV, DXV, EPI>(a, g.slices, stream);
-  if constexpr (EPI == kStGate) {
-    E2H_ST_CASE(6, 4, 2, 1) E2H_ST_CASE(4, 4, 2, 2) E2H_ST_CASE(8, 4, 1, 1) E2H_ST_CASE(6, 8, 1, 1) E2H_ST_CASE(8, 8, 1, 1)
-  } else if constexpr (EPI == kStArgmax) {
-    E2H_ST_CASE(8, 4, 1, 1) E2H_ST_CASE(4, 4, 2, 2) E2H_ST_CASE(8, 8, 1, 1) E2H_ST_CASE(4, 8, 2, 1) E2H_ST_CASE(4, 1, 1, 1) E2H_ST_CASE(2, 1, 1, 1)
-  } else {
-    E2H_ST_CASE(3, 4, 2, 2) E2H_ST_CASE(4, 4, 2, 2) E2H_ST_CASE(8, 4, 1, 1) E2H_ST_CASE(6, 4, 2, 1) E2H_ST_CASE(2, 2, 2, 2)
-    E2H_ST_CASE(4, 2, 2, 2) E2H_ST_CASE(6, 2, 2, 2) E2H_ST_CASE(4, 1, 1, 1) E2H_ST_CASE(2, 1, 1, 1) E2H_ST_CASE(4, 3, 3, 1) E2H_ST_CASE(4, 8, 2, 1) E2H_ST_CASE(8, 8, 1, 1)
+int dispatch_tiles(const StagedArgs &a, const Geometry &g, hipStream_t stream) {
+  switch (g.t) {
+    case 2: return launch_staged<G, MT, 2, EPI>(a, g.slices, stream);
+    case 4: return launch_staged<G, MT, 4, EPI>(a, g.slices, stream);
+    case 6: return launch_staged<G, MT, 6, EPI>(a, g.slices, stream);
+    case 8: return launch_staged<G, MT, 8, EPI>(a, g.slices, stream);
   }
-#undef E2H_ST_CASE
+  if constexpr (EPI == kStGate) {
+    if (g.t == 12) return launch_staged<G, MT, 12, EPI>(a, g.slices, stream);
+  } else {
+    if (g.t == 1) return launch_staged<G, MT, 1, EPI>(a, g.slices, stream);
+    if (g.t == 3) return launch_staged<G, MT, 3, EPI>(a, g.slices, stream);
+  }
   return E2H_ERR_BAD_SHAPE;
 }
 
 template <int EPI>
 int dispatch_staged(const StagedArgs &a, int groupsize, const Geometry &g, hipStream_t stream) {
-  const bool one = a.M <= 16;
-  switch (groupsize) {
-    case 32: return one ? dispatch_inst<32, 1, EPI>(a, g, stream) : dispatch_inst<32, 2, EPI>(a, g, stream);
-    case 64: return one ? dispatch_inst<64, 1, EPI>(a, g, stream) : dispatch_inst<64, 2, EPI>(a, g, stream);
-    default: return one ? dispatch_inst<128, 1, EPI>(a, g, stream) : dispatch_inst<128, 2, EPI>(a, g, stream);
-  }
+  const int mt = a.M <= 16 ? 1 : a.M <= 32 ? 2 : 4;
+#define E2H_ST_CASE(GV, MV) \
+  if (groupsize == GV && mt == MV) return dispatch_tiles<GV, MV, EPI>(a, g, stream);
+  E2H_ST_CASE(32, 1) E2H_ST_CASE(32, 2) E2H_ST_CASE(32, 4)
+  E2H_ST_CASE(64, 1) E2H_ST_CASE(64, 2) E2H_ST_CASE(64, 4)
+  E2H_ST_CASE(128, 1) E2H_ST_CASE(128, 2) E2H_ST_CASE(128, 4)
+#undef E2H_ST_CASE
+  return E2H_ERR_BAD_GROUPSIZE;
 }
 
 int check_shape(int64_t m, int64_t n, int64_t k, int groupsize) {
@@ -527,7 +592,7 @@ int check_shape(int64_t m, int64_t n, int64_t k, int groupsize) {
   return E2H_OK;
 }
 
-// fills the shape part of the arguments and picks the geometry; false if no instantiation covers the shape
+// fills the shape part of the arguments and picks the geometry; false where there is none
 bool plan(StagedArgs *a, Geometry *g, const void *staged, int64_t m, int64_t n, int64_t k, int groupsize, int epi) {
   a->M = static_cast<int>(m);
   a->Mpad = staged_mpad(m);
@@ -535,16 +600,33 @@ bool plan(StagedArgs *a, Geometry *g, const void *staged, int64_t m, int64_t n, 
   a->K = static_cast<int>(k);
   a->frag = static_cast<const uint8_t *>(staged);
   a->sums = reinterpret_cast<const float *>(a->frag + static_cast<size_t>(a->Mpad) * k * 2);
-  const int mt = a->M <= 16 ? 1 : 2;
-  a->slabs = (a->M + 16 * mt - 1) / (16 * mt);
-  const int tiles16 = static_cast<int>(n / 16);
-  const int kt = static_cast<int>(k / 128);
-  bool ok;
-  if (epi == kStGate) ok = pick(kGateInsts, true, groupsize, tiles16, kt, a->slabs, 1, g);
-  else if (epi == kStArgmax) ok = pick(kArgmaxInsts, false, groupsize, tiles16, kt, a->slabs, 1, g);
-  else ok = pick(kPlainInsts, false, groupsize, tiles16, kt, a->slabs, epi == kStPartial ? 8 : 1, g);
-  if (!ok) return false;
-  const int tc = epi == kStGate ? g->t / 2 : g->t;
+  const int mt = a->M <= 16 ? 1 : a->M <= 32 ? 2 : 4, tiles16 = static_cast<int>(n / 16), kt = static_cast<int>(k / 128);
+  const bool gate = epi == kStGate;
+  const int want_t = options().staged_tiles, want_s = options().staged_slices;  // experiments: force a geometry
+  // The geometry with the least cost; the weights of the cost were fitted to a sweep over T and S at 1 .. 64 rows of the shapes above and
+  // 12288 / 4096 / 32000 x 4096: the chosen geometry is within 6 % of the best one there.  One round of 256 workgroups with many tiles
+  // beats two rounds with few (w1|w3 22016 x 8192, 1 row: T = 12 43.6 us, T = 8 46.0; 32000 x 4096: T = 8 14.6, T = 6 19.0); K slices pay
+  // while a round is not full (w2 4096 x 11008, 32 rows: T = 4, S = 4 10.1 us, the best with S = 1 15.6).
+  double best_cost = -1;
+  for (int s = 1; s <= (epi == kStPartial ? 8 : 1) && s <= kt; s *= 2) {
+    if (want_s && epi == kStPartial && s != want_s) continue;
+    for (int t : {1, 2, 3, 4, 6, 8, 12}) {
+      if (t > max_tiles(groupsize, mt, gate) || (gate && t % 2) || (want_t && !gate && t != want_t)) continue;
+      const int tc = gate ? t / 2 : t;
+      const long wgs = static_cast<long>((tiles16 + tc - 1) / tc) * s;
+      const long rounds = (wgs + kCUs - 1) / kCUs;
+      const double chunks = static_cast<double>(kt) / s / kWaves;
+      // per workgroup: a fixed part, per chunk its weight tiles (at 64 rows their matrix work) and the operands from L2;
+      // per slice: what the consumer pays to add it
+      const double cost = rounds * (6 + chunks * (t * (mt == 4 ? 2.0 : 1.0) + 1.2 * mt)) + 1.0 * s * (mt == 4 ? 2 : 1);
+      if (best_cost < 0 || cost < best_cost) {
+        best_cost = cost;
+        *g = Geometry{t, s};
+      }
+    }
+  }
+  if (best_cost < 0) return false;
+  const int tc = gate ? g->t / 2 : g->t;
   a->col_blocks = (tiles16 + tc - 1) / tc;
   return true;
 }
@@ -625,10 +707,6 @@ extern "C" int e2h_int4_mm_staged_argmax(const void *staged, const int32_t *pack
 extern "C" int e2h_int4_mm_staged_partial_slices(int64_t m, int64_t n, int64_t k, int groupsize) {
   const int rc = check_shape(m, n, k, groupsize);
   if (rc != E2H_OK) return rc;
-  if (m > 32 && !options().staged_no_rows64) {  // one pass over the weights for all rows
-    const int s64 = rows64_partial_slices(m, n, k, groupsize);
-    if (s64 > 0) return s64;
-  }
   StagedArgs a = {};
   Geometry g;
   if (!plan(&a, &g, nullptr, m, n, k, groupsize, kStPartial)) return E2H_ERR_BAD_SHAPE;
@@ -641,8 +719,6 @@ extern "C" int e2h_int4_mm_staged_partials(const void *staged, const int32_t *pa
   const int rc = check_shape(m, n, k, groupsize);
   if (rc != E2H_OK) return rc;
   if (!aligned16(staged) || !aligned16(packed) || !aligned16(scales_and_zeros) || (reinterpret_cast<uintptr_t>(partials) & 3u)) return E2H_ERR_MISALIGNED;
-  if (m > 32 && !options().staged_no_rows64 && rows64_partial_slices(m, n, k, groupsize) > 0)
-    return rows64_partials(staged, packed, scales_and_zeros, partials, m, n, k, groupsize, slices, static_cast<hipStream_t>(stream));
   StagedArgs a = {};
   Geometry g;
   if (!plan(&a, &g, staged, m, n, k, groupsize, kStPartial)) return E2H_ERR_BAD_SHAPE;

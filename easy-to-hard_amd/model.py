@@ -31,7 +31,7 @@ DEFER_SPLIT_K = True         # wo / w2 hand float32 K-slice sums to the residual
 STAGED_DECODE = True         # int4 decode step: activations travel between the kernels in matrix-core operand order
 STAGED_HEAD = True           # ... including the LM head
 FUSE_HEAD_ARGMAX = True      # greedy decoding: the LM head launch reduces its columns to the arg-max, no logits are stored
-STAGED_MAX_ROWS = 64         # 33 .. 64 rows: wo and w2 run the one-pass 64-row kernel, the other launches two 32-row slabs
+STAGED_MAX_ROWS = 64         # the staged kernels read the weights once for up to 64 rows
 
 
 def _fusable(t: Tensor) -> bool:

@@ -226,3 +226,34 @@ def test_staged_argmax_head_is_covered_for_the_benchmark_heads():
     # the 7B head at 32 rows and the 34B head (group size 64) at 64 rows: the configurations the decode benchmark runs
     for rows, n, k, g in ((32, 32000, 4096, 128), (64, 32000, 8192, 64)):
         assert ops._lib.load().e2h_int4_mm_staged_supported(rows, n, k, g, ops.STAGED_ARGMAX) == 1
+
+
+@pytest.mark.parametrize("g", [32, 64, 128])
+@pytest.mark.parametrize("m", [1, 15, 17, 32, 33, 64])
+@pytest.mark.parametrize("n,k", [(16, 128), (16, 256), (48, 1152), (112, 5120), (1040, 13824), (6160, 640), (24592, 128)])
+def test_staged_mm_is_exact_on_integers_at_the_edges(g, m, n, k):
+    """K of fewer chunks than waves, of uneven runs per wave, of less and more than the ring holds; N that ends inside a workgroup's
+    tiles; every row tile count.  Codes 0 .. 15, scale 1 or 2 per group, zero 0 .. 3 and x in -1 .. 1: all terms are integers and all
+    partial sums, the shifted products (128 + q) x included, stay below 13824 * 143 * 2 < 2^22, so float32 is exact in any order."""
+    gen = torch.Generator().manual_seed(n + k + m + g)
+    codes = torch.randint(0, 16, (n, k), generator=gen, dtype=torch.int32)
+    scale = torch.randint(1, 3, (k // g, n), generator=gen).float()
+    zero = torch.randint(0, 4, (k // g, n), generator=gen).float()
+    x = torch.randint(-1, 2, (m, k), generator=gen).float()
+    packed = torch.from_numpy(qo.int4_tile_pack(codes.numpy(), 8)).to(DEV)
+    sz = torch.stack([scale, zero], dim=-1).to(torch.bfloat16).contiguous().to(DEV)
+    w = ((codes.float() - 8).view(n, k // g, g) * scale.t()[:, :, None] + zero.t()[:, :, None]).view(n, k).to(DEV)
+    want = x.to(DEV).double() @ w.double().t()
+    xs = ops.stage_x(x.to(torch.bfloat16).to(DEV))
+    assert torch.equal(ops.int4_mm_staged(xs, packed, g, sz), want.to(torch.bfloat16))
+
+    class Lin:
+        weight, scales_and_zeros, groupsize, in_features, out_features, inner_k_tiles, padding = packed, sz, g, k, n, 8, False
+
+    slices = ops.int4_staged_partial_slices(m, Lin)
+    assert slices >= 1
+    assert torch.equal(ops.int4_mm_staged_partials(xs, packed, g, sz, slices).double().sum(0), want)
+    plain = ops.int4_mm_staged(xs, packed, g, sz)
+    assert torch.equal(ops.int4_mm_staged_argmax(xs, packed, g, sz), ops.argmax_rows(plain))
+    gate, _ = ops.int4_mm_staged_silu_gate(xs, packed, sz, packed, sz, g, want_rows=True, want_staged=False)
+    assert torch.equal(gate, ops.silu_mul(plain, plain))
