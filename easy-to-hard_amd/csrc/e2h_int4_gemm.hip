@@ -3,21 +3,32 @@
 // Same contract and data layouts as e2h_int4_mm.hip (torch.ops.aten._weight_int4pack_mm as called by
 // linear_forward_int4, reference models/quantize.py:445-453), inner_k_tiles = 8, group size 32 / 64 / 128.
 //
-//   y[m,n] = sum_g  s[g,n] * sum_{k in g} x[m,k] * (128 + q[n,k])  +  sum_g (z[g,n] - 136 s[g,n]) * X[m,g]
+//   y[m,n] = sum_g  s[g,n] * sum_{k in g} x[m,k] * (16 + q[n,k])  +  sum_g (z[g,n] - 24 s[g,n]) * X[m,g]
 //
-// with X[m,g] = sum_{k in g} x[m,k] taken from a pre-pass (launch_x_group_sums).  The second sum is a small float32
-// matmul over the groups; it initialises the accumulators through v_mfma_f32_32x32x2_f32 (two groups per
-// instruction) before the main loop, so the loop itself carries no zero-point work at all.
+// with X[m,g] = sum_{k in g} x[m,k] taken from a pre-pass (launch_x_group_sums).  Codes enter the matrix cores as the exact
+// bfloat16 16 + q (rotate, and-or per two codes), so products are exact and sums float32.
 //
-// Main loop, v_mfma_f32_32x32x16_bf16 (A = activations, 32 rows; B = weights, 32 columns; 16 k per instruction):
-// lane L = 32*h + n supplies column n0 + n and k-half h.  A packed word holds 8 codes of one column at
-// k0 + {2j, 2j+1, 2j+8, 2j+9, 2j+16, ...} (j = 0..3); the lane loads the words with j = h (first 16-byte load)
-// and j = 2 + h (second), four 32-wide k spans p each.  Step (p, jp) multiplies the words (j = 2 jp + h, p) with
-// the activation fragment gathered in the same k order, so weights are never shuffled: one word is one B operand.
-// A workgroup of WR x WC waves owns 64 WR rows x 64 WC columns (each wave 64 x 64 = 2 x 2 tiles, 64 accumulator
-// registers).  Activations and packed weights are both staged per 128-wide k chunk into LDS in fragment order (double
-// buffered, one LDS barrier per chunk): the global loads then cover whole contiguous 512-byte weight blocks and whole
-// activation rows, every A fragment read feeds two column tiles and every unpacked word two row tiles.
+// Scales.  An accumulator is kept in units of its column's current scale: entering group g it is multiplied by
+// s[g-1,n] / s[g,n], and the group's products then add to it directly.  No second set of registers for the sums of one group,
+// which is what lets a wave own 128 rows x 64 columns, so that one unpacked fragment feeds four MFMAs and one activation
+// fragment two.  Scales outside 2^-26 .. 2^6 (zeros, infinities, NaN among them; the quantizer's lie between 2^-24 and a few units)
+// could leave float32's range that way: a workgroup that meets one takes a plain loop that forms every group's sum by itself.
+//
+// The zero-point term is a matrix product over the groups.  It starts the accumulators: X and z - 24 s are each split into three
+// bfloat16 parts (exact: 3 x 8 bits), and eight of the nine products of parts (all but low x low, 2^-32) fill one lane's eight k values,
+// two groups per v_mfma_f32_32x32x16_bf16.  That is half the matrix time of the float32 instruction for the same two groups.
+//
+// Main loop, k in natural order: lane L = 32 h + n supplies column n0 + n and the eight k values 16 s + 8 h .. + 7 of step s.  A packed
+// word (column, j, span p) holds the codes at k = 32 p + 8 i + 2 j + {0, 1} in nibbles i and i + 4, so dword j of the operand of step
+// 2 p + a is word[j][p] rotated right by 8 a + 4 h - 3, masked to bits 3 .. 6 and 19 .. 22, over two bfloat16 sixteens.
+// Four waves, 128 x 256 outputs per workgroup, two workgroups per CU: one's start and end run under the other's matrix work.
+// Operands reach LDS by 16-byte loads that write LDS directly:
+//   activations, 128 rows x 64 k per chunk, three stages: 1 KB block b holds rows 8 b .. 8 b + 7, the 16-byte pieces of a row stored at
+//   piece ^ ((row >> 1) & 7);
+//   weights, 64 columns of one wave x 128 k, two stages: 64 bytes per column, pieces at piece ^ ((column >> 2) & 3), read by the wave
+//   that loaded them.
+// One barrier per 64 k.  Where the row count leaves the chip short of workgroups, S of them share K and leave float32 sums for a
+// second kernel to add in order.
 //
 // Workgroup -> tile mapping: workgroup w runs on XCD w % 8; each XCD owns the column blocks cb = xcd (mod 8) and
 // walks them for one row block before moving to the next, so its L2 keeps that slice of the weights.
@@ -28,61 +39,102 @@ namespace e2h {
 namespace {
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef __attribute__((address_space(3))) void lds_void;
 
-constexpr int kChunkK = 128;
-constexpr int kFragB = 1024 + 32;                   // one 32-row x 16-k A fragment block in LDS (64 lanes x 16 B) + skew
-constexpr int kRT = 2, kCT = 2;                     // 32x32 tiles per wave: rows x columns
+constexpr int kCols = 256, kCT = 2;
 
-template <int G, int WR, int WC>
-__global__ __launch_bounds__(64 * WR * WC) void int4_gemm32_kernel(const uint16_t *__restrict__ x, const uint32_t *__restrict__ wp,
-                                                                   const uint32_t *__restrict__ sz, uint16_t *__restrict__ y,
-                                                                   const float *__restrict__ xsum, int xsum_stride, int M, int N, int K,
-                                                                   int n_col_blocks, int cbx) {
-  constexpr int NGRP = kChunkK / G;   // groups per chunk
-  constexpr int SPG = G / 16;         // MFMA steps per group
-  constexpr int kThreads = 64 * WR * WC;
-  constexpr int kRows = 64 * WR, kCols = 64 * WC;
-  constexpr int kStageX = (2 * WR) * 8 * kFragB;      // kRows x 128 k of activations, 8 fragments per 32-row tile
-  constexpr int kStageW = (2 * WC) * 2 * kFragB;      // kCols x 128 k of packed weights, 2 fragments (j pairs) per 32-column tile
-  constexpr int kXRowsPerPass = kThreads / 16;        // 16 pieces of 16 bytes per activation row
-  constexpr int kXPieces = kRows / kXRowsPerPass;
-  constexpr int kWTilesPerPass = kThreads / 32;       // 32 pieces of 16 bytes per 8-column weight block
-  constexpr int kWPieces = (kCols / 8) / kWTilesPerPass;
-  static_assert(kXRowsPerPass % 32 == 0 && kWTilesPerPass % 4 == 0, "staging passes cover whole 32-wide tiles");
-  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * (kStageX + kStageW)];
-  uint8_t *const lds_w = lds + 2 * kStageX;
+__device__ __forceinline__ uint32_t high_halves(float hi, float lo) {  // (bfloat16 bits of lo) | (of hi) << 16, truncated
+  return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo), 0x07060302u);
+}
+
+// v = p[0] + p[1] + p[2], every part a bfloat16 value
+__device__ __forceinline__ void split3(float v, float (&p)[3]) {
+  p[0] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & 0xFFFF0000u);
+  const float r = v - p[0];
+  p[1] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) & 0xFFFF0000u);
+  p[2] = r - p[1];
+}
+
+struct GemmArgs {
+  const uint16_t *x;
+  const uint32_t *wp, *sz;
+  uint16_t *y;
+  float *partials;  // [S][M][N] when K is shared, else null
+  const float *xsum;
+  int xsum_stride, M, N, K, n_col_blocks, cbx;
+};
+
+// kRT row tiles of 32 per wave: 32 kRT rows x 256 columns per workgroup
+template <int G, int kRT>
+__global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
+  constexpr int kRows = 32 * kRT, kXStage = kRows * 128, kWStage = kCols * 64, kLdsW = 3 * kXStage, kLdsBytes = kLdsW + 2 * kWStage;
+  static_assert(2 * kLdsBytes <= 160 * 1024, "two workgroups per CU");
+  constexpr int NGRP = 128 / G, SPG = G / 16;  // groups per 128 k, MFMA steps per group
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kLdsBytes];
+  const int M = a.M, N = a.N, K = a.K;
 
   const int xcd = blockIdx.x & 7;
   const int slot = blockIdx.x >> 3;
-  const int cb = xcd + 8 * (slot % cbx);
-  const int rb = slot / cbx;
-  if (cb >= n_col_blocks) return;  // grid padding; uniform, before any barrier
+  const int cb = xcd + 8 * (slot % a.cbx), rb = slot / a.cbx;
+  if (cb >= a.n_col_blocks) return;  // grid padding; uniform, before any barrier
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wr = wave / WC, wc = wave % WC;
   const int n = lane & 31, h = lane >> 5;
-  const int row0 = rb * kRows + wr * 64;
-  const int col0 = cb * kCols + wc * 64;
-  const int KT = K / kChunkK;
-  const int nchunks = K / kChunkK;
-  const int ngroups = K / G;
+  const int row0 = rb * kRows, col0 = cb * kCols + 64 * wave;
+  const int KT = K >> 7;
+  const int blk0 = static_cast<int>((static_cast<int64_t>(KT) * blockIdx.y) / gridDim.y);
+  const int blk1 = static_cast<int>((static_cast<int64_t>(KT) * (blockIdx.y + 1)) / gridDim.y);
+  const int g_begin = blk0 * NGRP, g_end = blk1 * NGRP;
 
-  const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(wp, static_cast<uint32_t>(static_cast<size_t>(N) * K / 2));
-  const __amdgpu_buffer_rsrc_t sz_rsrc = make_rsrc(sz, static_cast<uint32_t>(static_cast<size_t>(ngroups) * N * 4));
-  const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(x, static_cast<uint32_t>(static_cast<size_t>(M) * K * 2));
-  const __amdgpu_buffer_rsrc_t xs_rsrc = make_rsrc(xsum, static_cast<uint32_t>(static_cast<size_t>(ngroups) * xsum_stride * 4));
+  const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(a.wp, static_cast<uint32_t>(static_cast<size_t>(N) * K / 2));
+  const __amdgpu_buffer_rsrc_t sz_rsrc = make_rsrc(a.sz, static_cast<uint32_t>(static_cast<size_t>(K / G) * N * 4));
+  const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(a.x, static_cast<uint32_t>(static_cast<size_t>(M) * K * 2));
+  const __amdgpu_buffer_rsrc_t xs_rsrc = make_rsrc(a.xsum, static_cast<uint32_t>(static_cast<size_t>(K / G) * a.xsum_stride * 4));
 
-  uint32_t szlane[kCT];  // byte offset of this lane's column inside one [N] row of (scale, zero) pairs
+  // ---- what this lane loads: activation block wave + 4 i, row 8 (wave + 4 i) + lane / 8; weight column 16 i + lane / 4 of the wave's 64
+  uint32_t xsrc[4], wsrc[4];
+#pragma unroll
+  for (int i = 0; i < kRT; ++i) {
+    int row = row0 + 8 * (wave + 4 * i) + (lane >> 3);
+    row = row < M ? row : M - 1;
+    xsrc[i] = static_cast<uint32_t>((static_cast<size_t>(row) * K + ((lane & 7) ^ (((lane >> 4) + 4 * wave) & 7)) * 8) * 2);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    int col = col0 + 16 * i + (lane >> 2);
+    col = col < N ? col : N - 1;
+    wsrc[i] = static_cast<uint32_t>(static_cast<size_t>(col >> 3) * KT * 512 + (col & 7) * 64 + ((lane & 3) ^ ((lane >> 4) & 3)) * 16);
+  }
+  const int last_chunk = 2 * blk1 - 1;
+  const auto load_x = [&](int chunk, uint32_t stage) {  // past the slice: its last chunk again, which nobody uses
+    const uint32_t off = static_cast<uint32_t>(chunk < last_chunk ? chunk : last_chunk) * 128u;
+#pragma unroll
+    for (int i = 0; i < kRT; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, (lds_void *)(lds + stage + (wave + 4 * i) * 1024), 16, xsrc[i], off, 0, 0);
+  };
+  const auto load_w = [&](int blk, uint32_t stage) {
+    const uint32_t off = static_cast<uint32_t>(blk < blk1 - 1 ? blk : blk1 - 1) * 512u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_void *)(lds + stage + (4 * wave + i) * 1024), 16, wsrc[i], off, 0, 0);
+  };
+  uint32_t szlane[kCT];  // this lane's columns inside one [N] row of (scale, zero) pairs
 #pragma unroll
   for (int ct = 0; ct < kCT; ++ct) {
     int col = col0 + 32 * ct + n;
     col = col < N ? col : N - 1;
     szlane[ct] = static_cast<uint32_t>(col) * 4u;
   }
+  const auto load_sz = [&](int ct, int g) {
+    return __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, szlane[ct], static_cast<uint32_t>(g < g_end - 1 ? g : g_end - 1) * N * 4u, 0);
+  };
 
-  // ---- accumulators start as the zero-point term: sum_g X[m,g] * (z - 136 s)[g,n] in float32 MFMAs --------
+  load_w(blk0, kLdsW);
+  load_x(2 * blk0, 0);
+  load_x(2 * blk0 + 1, kXStage);
+
+  // ---- accumulators start as the zero-point term -----------------------------------------------------------------------
   f32x16_t acc[kCT][kRT];
 #pragma unroll
   for (int ct = 0; ct < kCT; ++ct)
@@ -90,178 +142,307 @@ __global__ __launch_bounds__(64 * WR * WC) void int4_gemm32_kernel(const uint16_
     for (int rt = 0; rt < kRT; ++rt)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[ct][rt][e] = 0.f;
-  {
-    uint32_t xslane[kRT];
+  bool odd_scale = false;
+  struct Zero {
+    float xs[4];
+    uint32_t szw[kCT];
+  };
+  constexpr int kBatch = 4;  // pairs of groups per round, requested a round ahead
+  const auto dead = [&](int g0) { return g0 + h < g_end ? 0u : 0x80000000u; };  // lanes with h = 1 take group g0 + 1; past the end: zeros
+  const auto load_zero = [&](Zero (&z)[kBatch], int g0) {
 #pragma unroll
-    for (int rt = 0; rt < kRT; ++rt) xslane[rt] = static_cast<uint32_t>(h * xsum_stride + row0 + 32 * rt + n) * 4u;
-    uint32_t zlane[kCT];
-#pragma unroll
-    for (int ct = 0; ct < kCT; ++ct) zlane[ct] = szlane[ct] + static_cast<uint32_t>(h) * static_cast<uint32_t>(N) * 4u;
-#pragma unroll 4
-    for (int g0 = 0; g0 < ngroups; g0 += 2) {  // lanes with h = 1 take group g0 + 1 (reads past the last group return 0)
-      float a[kRT], zc[kCT];
+    for (int i = 0; i < kBatch; ++i) {
+      const int g = g0 + 2 * i;
+      const uint32_t out = dead(g), gs = static_cast<uint32_t>(g < g_end ? g : g_begin);
 #pragma unroll
       for (int rt = 0; rt < kRT; ++rt)
-        a[rt] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xs_rsrc, xslane[rt], static_cast<uint32_t>(g0) * xsum_stride * 4u, 0));
+        z[i].xs[rt] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xs_rsrc, static_cast<uint32_t>(h * a.xsum_stride + row0 + 32 * rt + n) * 4u | out,
+                                                                                     gs * a.xsum_stride * 4u, 0));
+#pragma unroll
+      for (int ct = 0; ct < kCT; ++ct)
+        z[i].szw[ct] = __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, (szlane[ct] + static_cast<uint32_t>(h) * N * 4u) | out, gs * N * 4u, 0);
+    }
+  };
+  Zero za[kBatch], zb[kBatch];
+  load_zero(za, g_begin);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+  for (int g0 = g_begin; g0 < g_end; g0 += 2 * kBatch) {
+    load_zero(zb, g0 + 2 * kBatch);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      bf16x8_t zf[kCT];
 #pragma unroll
       for (int ct = 0; ct < kCT; ++ct) {
-        const uint32_t szw = __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, zlane[ct], static_cast<uint32_t>(g0) * N * 4u, 0);
-        const float scale = __builtin_bit_cast(float, szw << 16), zero = __builtin_bit_cast(float, szw & 0xFFFF0000u);
-        zc[ct] = __builtin_fmaf(-136.0f, scale, zero);
+        const float scale = __builtin_bit_cast(float, za[i].szw[ct] << 16), zero = __builtin_bit_cast(float, za[i].szw[ct] & 0xFFFF0000u);
+        odd_scale |= !dead(g0 + 2 * i) && !(__builtin_fabsf(scale) >= 0x1p-26f && __builtin_fabsf(scale) <= 0x1p6f && __builtin_fabsf(zero) <= 0x1p100f);
+        float p[3];
+        split3(__builtin_fmaf(-24.0f, scale, zero), p);
+        const uint32_t hm = high_halves(p[1], p[0]);
+        zf[ct] = __builtin_bit_cast(bf16x8_t, u32x4_t{hm, hm, high_halves(p[0], p[2]), high_halves(p[1], p[2])});
       }
 #pragma unroll
-      for (int ct = 0; ct < kCT; ++ct)
+      for (int rt = 0; rt < kRT; ++rt) {
+        float p[3];
+        split3(za[i].xs[rt], p);
+        const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, u32x4_t{high_halves(p[0], p[0]), high_halves(p[1], p[1]), high_halves(p[2], p[0]), high_halves(p[2], p[1])});
 #pragma unroll
-        for (int rt = 0; rt < kRT; ++rt) acc[ct][rt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[rt], zc[ct], acc[ct][rt], 0, 0, 0);
+        for (int ct = 0; ct < kCT; ++ct) acc[ct][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf, zf[ct], acc[ct][rt], 0, 0, 0);
+      }
     }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) za[i] = zb[i];
   }
 
-  // ---- staging.  Activations: piece (row, within): span p = within / 4 of 32 k, quarter u = within % 4; its dword e
-  // belongs to the fragment of step (p, e / 2), lane (h = e % 2, row % 32), register u.  Weights: piece (8-column block,
-  // t) of a 512-byte block = the four words (column 8 blk + t / 4, j = t % 4): fragment (column tile, j / 2), lane
-  // (h = j % 2, column % 32).
-  const int xr0 = tid >> 4, xw = tid & 15;
-  uint32_t xsrc[kXPieces];
+  // do all waves know the same?  (the third activation stage is free until the loop)
+  uint32_t *const votes = reinterpret_cast<uint32_t *>(lds + 2 * kXStage);
+  const bool odd_wave = __builtin_amdgcn_ballot_w64(odd_scale) != 0;
+  if (lane == 0) votes[wave] = odd_wave;
+  lds_barrier();
+  if (__builtin_amdgcn_readfirstlane(votes[0] | votes[1] | votes[2] | votes[3])) {
+    // a scale that the running units do not carry: every group's sum by itself, operands straight from memory
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the loads above still write LDS
+#pragma unroll 1
+    for (int t = 0; t < kCT * kRT; ++t) {
+      const int ct = t / kRT, rt = t % kRT;
+      int row = row0 + 32 * rt + n;
+      row = row < M ? row : M - 1;
+      int col = col0 + 32 * ct + n;
+      col = col < N ? col : N - 1;
+      const uint32_t xo = static_cast<uint32_t>(static_cast<size_t>(row) * K * 2) + 16u * h;
+      const uint32_t wo = static_cast<uint32_t>(static_cast<size_t>(col >> 3) * KT * 512 + (col & 7) * 64);
+      f32x16_t sum = {};
+      for (int g = g_begin; g < g_end; ++g) {
+        f32x16_t part = {};
+        for (int s = 0; s < SPG; ++s) {
+          const int step = g * SPG + s;  // of 16 k
+          const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xo, static_cast<uint32_t>(step) * 32u, 0));
+          u32x4_t u;
 #pragma unroll
-  for (int i = 0; i < kXPieces; ++i) {
-    int row = rb * kRows + xr0 + kXRowsPerPass * i;
-    row = row < M ? row : M - 1;
-    xsrc[i] = static_cast<uint32_t>((static_cast<size_t>(row) * K + xw * 8) * 2);
-  }
-  const int xdst0 = ((xr0 >> 5) * 8 + 2 * (xw >> 2)) * kFragB + (xr0 & 31) * 16 + (xw & 3) * 4;
-  const int wb0 = tid >> 5, wt = tid & 31;  // 8-column block within the pass, piece within the block
-  uint32_t wsrc[kWPieces];
+          for (int j = 0; j < 4; ++j) {
+            const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(w_rsrc, wo + 16u * j, static_cast<uint32_t>(step >> 3) * 512u + ((step >> 1) & 3) * 4u, 0);
+            u[j] = (__builtin_amdgcn_alignbit(w, w, (8 * (step & 1) + 4 * h - 3) & 31) & 0x00780078u) | 0x41804180u;
+          }
+          part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf, __builtin_bit_cast(bf16x8_t, u), part, 0, 0, 0);
+        }
+        const uint32_t szw = __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, static_cast<uint32_t>(col) * 4u, static_cast<uint32_t>(g) * N * 4u, 0);
+        const float scale = __builtin_bit_cast(float, szw << 16), zero = __builtin_bit_cast(float, szw & 0xFFFF0000u);
+        const float zc = __builtin_fmaf(-24.0f, scale, zero);
 #pragma unroll
-  for (int i = 0; i < kWPieces; ++i) {
-    int nt8 = cb * (kCols / 8) + wb0 + kWTilesPerPass * i;
-    nt8 = nt8 < (N >> 3) ? nt8 : (N >> 3) - 1;
-    wsrc[i] = static_cast<uint32_t>((static_cast<size_t>(nt8) * KT * 32 + wt) * 16);
-  }
-  const int wdst0 = ((wb0 >> 2) * 2 + ((wt & 3) >> 1)) * kFragB + ((wt & 1) * 32 + 8 * (wb0 & 3) + (wt >> 2)) * 16;
-
-  struct Staged {
-    u32x4_t x[kXPieces], w[kWPieces];
-  };
-  auto load_next = [&](Staged &r, int ci) {
-    const int cc = ci < nchunks ? ci : nchunks - 1;
-#pragma unroll
-    for (int i = 0; i < kXPieces; ++i) r.x[i] = __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xsrc[i], static_cast<uint32_t>(cc) * (kChunkK * 2), 0);
-#pragma unroll
-    for (int i = 0; i < kWPieces; ++i) r.w[i] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, wsrc[i], static_cast<uint32_t>(cc) * 512u, 0);
-  };
-  auto store_next = [&](const Staged &r, int parity) {
-    uint8_t *bx = lds + (parity & 1) * kStageX + xdst0;
-#pragma unroll
-    for (int i = 0; i < kXPieces; ++i) {
-      uint8_t *d = bx + i * (kXRowsPerPass / 32) * (8 * kFragB);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) *reinterpret_cast<uint32_t *>(d + (e >> 1) * kFragB + (e & 1) * (32 * 16)) = r.x[i][e];
-    }
-    uint8_t *bw = lds_w + (parity & 1) * kStageW + wdst0;
-#pragma unroll
-    for (int i = 0; i < kWPieces; ++i) *reinterpret_cast<u32x4_t *>(bw + i * (kWTilesPerPass / 4) * (2 * kFragB)) = r.w[i];
-  };
-  auto load_scales = [&](uint32_t (&r)[kCT][NGRP], int ci) {
-    const int cc = ci < nchunks ? ci : nchunks - 1;
-#pragma unroll
-    for (int ct = 0; ct < kCT; ++ct)
-#pragma unroll
-      for (int g = 0; g < NGRP; ++g)
-        r[ct][g] = __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, szlane[ct], static_cast<uint32_t>(cc * NGRP + g) * N * 4u, 0);
-  };
-
-  const UnpackConsts uc = unpack_consts();
-  auto compute = [&](const uint32_t (&sc)[kCT][NGRP], int parity) {
-    const uint8_t *bx = lds + (parity & 1) * kStageX + (wr * kRT) * (8 * kFragB) + lane * 16;
-    const uint8_t *bw = lds_w + (parity & 1) * kStageW + (wc * kCT) * (2 * kFragB) + lane * 16;
-    u32x4_t wq[kCT][2];  // [column tile][j pair]: words of the four 32-wide k spans
-#pragma unroll
-    for (int ct = 0; ct < kCT; ++ct)
-#pragma unroll
-      for (int ld = 0; ld < 2; ++ld) wq[ct][ld] = *reinterpret_cast<const u32x4_t *>(bw + (ct * 2 + ld) * kFragB);
-#pragma unroll
-    for (int g = 0; g < NGRP; ++g) {
-      f32x16_t part[kCT][kRT];
-#pragma unroll
-      for (int ct = 0; ct < kCT; ++ct)
-#pragma unroll
-        for (int rt = 0; rt < kRT; ++rt)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) part[ct][rt][e] = 0.f;
-#pragma unroll
-      for (int sg = 0; sg < SPG; ++sg) {
-        const int s = g * SPG + sg;  // step = 2 p + jp
-        bf16x8_t af[kRT];
-#pragma unroll
-        for (int rt = 0; rt < kRT; ++rt) af[rt] = *reinterpret_cast<const bf16x8_t *>(bx + (rt * 8 + s) * kFragB);
-#pragma unroll
-        for (int ct = 0; ct < kCT; ++ct) {
-          const bf16x8_t wf = unpack_word(wq[ct][s & 1][s >> 1], uc);
-#pragma unroll
-          for (int rt = 0; rt < kRT; ++rt) part[ct][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[rt], wf, part[ct][rt], 0, 0, 0);
+        for (int e = 0; e < 16; ++e) {
+          const float xg_e = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xs_rsrc, static_cast<uint32_t>(row0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3)) * 4u,
+                                                                                          static_cast<uint32_t>(g) * a.xsum_stride * 4u, 0));
+          sum[e] = __builtin_fmaf(zc, xg_e, __builtin_fmaf(scale, part[e], sum[e]));
         }
       }
+      if (col0 + 32 * ct + n < N)
+        for (int e = 0; e < 16; ++e) {
+          const int m = row0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3);
+          if (m >= M) continue;
+          if (a.partials) a.partials[(static_cast<size_t>(blockIdx.y) * M + m) * N + col] = sum[e];
+          else a.y[static_cast<size_t>(m) * N + col] = f32_to_bf16_rne(sum[e]);
+        }
+    }
+    return;
+  }
+
+  // ---- fragments: activation (row tile rt, step s): row 32 rt + n, piece 2 s + h; weights (column tile ct): pieces j of column 32 ct + n
+  uint32_t a_lane[4], w_lane[4];
 #pragma unroll
-      for (int ct = 0; ct < kCT; ++ct) {
-        const float scale = __builtin_bit_cast(float, sc[ct][g] << 16);
+  for (int s = 0; s < 4; ++s) a_lane[s] = static_cast<uint32_t>(n * 128 + (((2 * s + h) ^ ((n >> 1) & 7)) << 4));
 #pragma unroll
-        for (int rt = 0; rt < kRT; ++rt)
+  for (int j = 0; j < 4; ++j) w_lane[j] = static_cast<uint32_t>(wave * 4096 + n * 64 + ((j ^ ((n >> 2) & 3)) << 4));
+  bf16x8_t af[2][kRT], wf[2][kCT];
+  u32x4_t wq[kCT][4];
+  const auto read_a = [&](bf16x8_t (&f)[kRT], uint32_t stage, int s) {
 #pragma unroll
-          for (int e = 0; e < 16; ++e) acc[ct][rt][e] = __builtin_fmaf(scale, part[ct][rt][e], acc[ct][rt][e]);
+    for (int rt = 0; rt < kRT; ++rt) f[rt] = *reinterpret_cast<const bf16x8_t *>(lds + stage + a_lane[s] + rt * 4096);
+  };
+  const auto read_w = [&](uint32_t stage) {
+#pragma unroll
+    for (int ct = 0; ct < kCT; ++ct)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) wq[ct][j] = *reinterpret_cast<const u32x4_t *>(lds + stage + w_lane[j] + ct * 2048);
+  };
+  uint32_t mask, magic;  // one scalar and one vector register, so that each pair of codes is one and-or
+  asm volatile("s_mov_b32 %0, 0x00780078" : "=s"(mask));
+  asm volatile("v_mov_b32 %0, 0x41804180" : "=v"(magic));
+  const uint32_t rot0 = (4 * h - 3) & 31, rot1 = (4 * h + 5) & 31;
+  const auto convert = [&](bf16x8_t (&f)[kCT], int s8) {
+#pragma unroll
+    for (int ct = 0; ct < kCT; ++ct) {
+      u32x4_t u;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t w = wq[ct][j][s8 >> 1];
+        u[j] = (__builtin_amdgcn_alignbit(w, w, s8 & 1 ? rot1 : rot0) & mask) | magic;
       }
+      f[ct] = __builtin_bit_cast(bf16x8_t, u);
     }
   };
 
-  // ---- main loop, two chunks per trip so that the scale registers are compile-time names -----------------
-  Staged st;
-  uint32_t sc[2][kCT][NGRP];
-  load_next(st, 0);
-  load_scales(sc[0], 0);
-  store_next(st, 0);
-  lds_barrier();
-  for (int ci = 0; ci < nchunks; ci += 2) {
-    load_next(st, ci + 1);       // in flight during the arithmetic of this chunk
-    load_scales(sc[1], ci + 1);
-    __builtin_amdgcn_sched_barrier(0);  // keep the prefetch ahead of the arithmetic: the scheduler would sink it to its first use
-    compute(sc[0], 0);
-    store_next(st, 1);           // the other stage: everybody left it at the previous barrier
-    lds_barrier();
-    if (ci + 1 >= nchunks) break;  // uniform
-    load_next(st, ci + 2);
-    load_scales(sc[0], ci + 2);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(sc[1], 1);
-    store_next(st, 0);
-    lds_barrier();
+  float unit[kCT] = {1.f, 1.f};  // what one step of the accumulators is worth
+  constexpr int kSc = NGRP < 2 ? NGRP : 2;  // pairs held ahead
+  uint32_t sc[kCT][kSc];
+#pragma unroll
+  for (int ct = 0; ct < kCT; ++ct)
+#pragma unroll
+    for (int g = 0; g < kSc; ++g) sc[ct][g] = load_sz(ct, g_begin + g);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  asm volatile("s_barrier" ::: "memory");
+  read_w(kLdsW);
+  read_a(af[0], 0, 0);
+  convert(wf[0], 0);
+  uint32_t s0 = 0, s1 = kXStage, s2 = 2 * kXStage;  // stage of the chunk in use, of the next one, of the one after
+  uint32_t w_next = kLdsW + kWStage;
+
+  for (int blk = blk0; blk < blk1; ++blk) {
+    load_w(blk + 1, w_next);
+    load_x(2 * blk + 2, s2);
+#pragma unroll
+    for (int s8 = 0; s8 < 8; ++s8) {
+      const int cur = s8 & 1;
+      if (s8 == 4) load_x(2 * blk + 3, s0);  // every wave left that stage at the barrier below
+      // The second chunk is in: loads issued after it are this block's words, its next chunk and the scale pairs of the last half block of each kind.  The
+      // next block's words and first chunk are in: after them came one chunk and this block's scale pairs.
+      if (s8 == 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(4 + kRT + (NGRP == 1 ? 2 : 2 * NGRP)) : "memory");
+      if (s8 == 7) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kRT + 2 * NGRP) : "memory");
+      if (s8 == 7) read_w(w_next);
+      read_a(af[cur ^ 1], s8 < 3 ? s0 : s8 < 7 ? s1 : s2, (s8 + 1) & 3);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ct = 0; ct < kCT; ++ct) {
+        float r = 1.f;
+        if (s8 % SPG == 0) {
+          const float s = __builtin_bit_cast(float, sc[ct][s8 / SPG % kSc] << 16);
+          r = unit[ct] / s;
+          unit[ct] = s;
+          sc[ct][s8 / SPG % kSc] = load_sz(ct, blk * NGRP + s8 / SPG + kSc);
+        }
+#pragma unroll
+        for (int rt = 0; rt < kRT; ++rt) {
+          if (s8 % SPG == 0) {
+            __builtin_amdgcn_sched_barrier(0);  // one tile's rescaling under the previous tile's product
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[ct][rt][e] *= r;
+          }
+          acc[ct][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[cur][rt], wf[cur][ct], acc[ct][rt], 0, 0, 0);
+        }
+      }
+      convert(wf[cur ^ 1], (s8 + 1) & 7);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const uint32_t t = s0;  // two chunks on
+    s0 = s2;
+    s2 = s1;
+    s1 = t;
+    w_next ^= kLdsW ^ (kLdsW + kWStage);
   }
+  // the loads issued past the last block still write LDS: drain them before the stages are reused
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int ct = 0; ct < kCT; ++ct)
+#pragma unroll
+    for (int rt = 0; rt < kRT; ++rt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[ct][rt][e] *= unit[ct];
 
   // ---- store: lane (h, n) holds column col0 + 32 ct + n, rows 8 (e / 4) + 4 h + e % 4 of each tile -----------
-  // (the barrier that ended the last chunk left every wave done with the stages)
+  if (a.partials) {
+    float *out = a.partials + static_cast<size_t>(blockIdx.y) * M * N;
+#pragma unroll
+    for (int ct = 0; ct < kCT; ++ct) {
+      const int col = col0 + 32 * ct + n;
+      if (col >= N) continue;
+#pragma unroll
+      for (int rt = 0; rt < kRT; ++rt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int m = row0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3);
+          if (m < M) out[static_cast<size_t>(m) * N + col] = acc[ct][rt][e];
+        }
+    }
+    return;
+  }
   const float no_scale[kCT] = {};
-  store_tiles_via_lds<kRT, kCT, false>(acc, no_scale, lds + wave * TileStore<kCT>::kBytesPerWave, y, row0, col0, M, N, lane,
-                                    (N & 7) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0);
+  store_tiles_via_lds<kRT, kCT, false>(acc, no_scale, lds + wave * TileStore<kCT>::kBytesPerWave, a.y, row0, col0, M, N, lane,
+                                    (N & 7) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0);
+}
+
+constexpr int kMostSlices = 8;
+
+// y = bf16(sum over the K slices), a balanced tree in the order of K; four columns per thread (N % 8 == 0)
+__global__ __launch_bounds__(256) void add_slices_kernel(const float *__restrict__ partials, uint16_t *__restrict__ y, int64_t quads, int64_t slice, int S) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= quads) return;
+  f32x4_t v[kMostSlices];
+#pragma unroll
+  for (int s = 0; s < kMostSlices; ++s) v[s] = s < S ? *reinterpret_cast<const f32x4_t *>(partials + s * slice + 4 * i) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int step = 1; step < kMostSlices; step *= 2)
+#pragma unroll
+    for (int s = 0; s < kMostSlices; s += 2 * step) v[s] += v[s + step];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) y[4 * i + j] = f32_to_bf16_rne(v[0][j]);
 }
 
 }  // namespace
 
-int int4_gemm32(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint16_t *y, const float *xsum, int xsum_stride,
-                int M, int N, int K, int groupsize, hipStream_t stream) {
-  if (K % kChunkK != 0 || N % 8 != 0) return E2H_ERR_BAD_SHAPE;
-  constexpr int WR = 2, WC = 4;  // 128 rows x 256 columns per workgroup of 8 waves, one workgroup per CU (101 KB of LDS)
-  const int n_col_blocks = (N + 64 * WC - 1) / (64 * WC), n_row_blocks = (M + 64 * WR - 1) / (64 * WR);
-  const int cbx = (n_col_blocks + 7) / 8;
-  const long long wgs = 8LL * cbx * n_row_blocks;
+// Rows per workgroup and K slices by the least expected time in us, from what was measured at 65 .. 8192 rows of the 7B and 34B shapes:
+// a workgroup takes `one` per 128 k when it has its CU to itself and two that share a CU take `two` (64 rows: 1.2 and 1.95, 128 rows:
+// 1.85 and 3.3), a call 3 more, and slices what their sums cost to write and add.  128 rows win once the chip is full (8192 x 12288 x 4096:
+// 688 us, 64 rows 795), 64 rows with one slice or several below (471 x 4096 x 4096: two slices 34 us, one 41, 128 rows 63).
+Int4GemmShape int4_gemm_shape(int M, int N, int K, int groupsize, int64_t scratch_bytes) {
+  const int KT = K >> 7;
+  const int64_t fit = scratch_bytes / (static_cast<int64_t>(M) * N * 4);
+  const int want_rows = options().int4_gemm_tile, want_s = options().int4_k_slices;
+  Int4GemmShape best = {64, 1, -1.0};
+  for (int rows = 64; rows <= (groupsize == 32 ? 64 : 128); rows *= 2) {  // group size 32 at 128 rows does not fit the registers
+    if (want_rows == 128 && groupsize != 32 && rows != 128) continue;
+    const int64_t per_xcd = static_cast<int64_t>((M + rows - 1) / rows) * (((N + kCols - 1) / kCols + 7) / 8);  // one slice; 32 CUs each
+    for (int s = 1; s <= kMostSlices && s <= KT && (s == 1 || s <= fit); s *= 2) {
+      if (want_s > 0 && s != want_s && want_s <= fit && want_s <= kMostSlices) continue;
+      const int64_t per_cu = (per_xcd * s + 31) / 32;
+      const double one = rows == 64 ? 1.2 : 1.85, two = rows == 64 ? 1.95 : 3.3;
+      const double cost = (static_cast<double>(per_cu / 2) * two + (per_cu & 1 ? one : 0)) * KT / s + 3 +
+                          (s > 1 ? 4 + s * (0.6 + 0.9e-6 * static_cast<double>(M) * N) : 0);
+      if (best.us < 0 || cost < best.us) best = Int4GemmShape{rows, s, cost};
+    }
+  }
+  return best;
+}
+
+template <int G>
+void launch_gemm(const GemmArgs &a, int rows, dim3 grid, hipStream_t stream) {
+  if constexpr (G != 32) {
+    if (rows == 128) {
+      hipLaunchKernelGGL((int4_gemm_kernel<G, 4>), grid, dim3(256), 0, stream, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((int4_gemm_kernel<G, 2>), grid, dim3(256), 0, stream, a);
+}
+
+int int4_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint16_t *y, const float *xsum, int xsum_stride,
+              float *partials, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream) {
+  if (K % 128 != 0 || N % 8 != 0) return E2H_ERR_BAD_SHAPE;
+  GemmArgs a = {x, reinterpret_cast<const uint32_t *>(packed), reinterpret_cast<const uint32_t *>(sz), y, shape.slices > 1 ? partials : nullptr,
+                xsum, xsum_stride, M, N, K, (N + kCols - 1) / kCols, 0};
+  a.cbx = (a.n_col_blocks + 7) / 8;
+  const long long wgs = 8LL * a.cbx * ((M + shape.rows - 1) / shape.rows);
   if (wgs > 0x7FFFFFFFLL) return E2H_ERR_BAD_SHAPE;
-  // the pre-pass pads its rows to 64; this kernel's lanes read whole row blocks: rows past the pad return 0 from the
-  // buffer bound or belong to other groups' rows of the same array -- they only ever reach rows >= M, which are not stored
-  dim3 grid(static_cast<unsigned>(wgs)), block(64 * WR * WC);
-  const uint32_t *w = reinterpret_cast<const uint32_t *>(packed);
-  const uint32_t *s = reinterpret_cast<const uint32_t *>(sz);
+  const dim3 grid(static_cast<unsigned>(wgs), static_cast<unsigned>(shape.slices));
   switch (groupsize) {
-    case 32: hipLaunchKernelGGL((int4_gemm32_kernel<32, WR, WC>), grid, block, 0, stream, x, w, s, y, xsum, xsum_stride, M, N, K, n_col_blocks, cbx); break;
-    case 64: hipLaunchKernelGGL((int4_gemm32_kernel<64, WR, WC>), grid, block, 0, stream, x, w, s, y, xsum, xsum_stride, M, N, K, n_col_blocks, cbx); break;
-    case 128: hipLaunchKernelGGL((int4_gemm32_kernel<128, WR, WC>), grid, block, 0, stream, x, w, s, y, xsum, xsum_stride, M, N, K, n_col_blocks, cbx); break;
+    case 32: launch_gemm<32>(a, shape.rows, grid, stream); break;
+    case 64: launch_gemm<64>(a, shape.rows, grid, stream); break;
+    case 128: launch_gemm<128>(a, shape.rows, grid, stream); break;
     default: return E2H_ERR_BAD_GROUPSIZE;
+  }
+  if (shape.slices > 1) {
+    const int64_t quads = static_cast<int64_t>(M) * N / 4;
+    hipLaunchKernelGGL(add_slices_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, stream, partials, y, quads,
+                       static_cast<int64_t>(M) * N, shape.slices);
   }
   return launch_status();
 }

@@ -806,13 +806,20 @@ int int4_mm_impl(const uint16_t *x, const int32_t *packed, const uint16_t *scale
         if (launch_x_group_sums(a.x, xs, a.M, a.K, stride, groupsize, a.stream) != E2H_OK) return E2H_ERR_LAUNCH;
         a.xsum = xs;
         a.xsum_stride = stride;
-        // 32x32-tile kernel for whole 128-row blocks' worth of work
-        // the 128 x 128-output workgroups of that kernel pay off once there are enough of them to fill the chip
-        // (measured crossover on the 7B shapes: about 320 workgroups)
+        // The 32x32-tile kernel wherever the work fills the chip (320 tiles of 128 x 128), and below that where it is expected to take
+        // two thirds of the time of the 16x16-tile kernel of this file at most (both estimates are good to 20 %): that one takes 0.9 us per
+        // 128 k with one weight tile per wave and 1.15 with two, half as much again for every further workgroup on a CU.  Measured (us;
+        // 16x16 / 32x32): 65 rows 4096 x 4096 33 / 21, 471 rows 4096 x 11008 98 / 65; stay: 157 rows 11008 x 4096 47 / 42, 471 rows
+        // 2048 x 2048 20 / 24, 65 rows 512 x 512 8 / 10.
+        const int64_t left = (workspace_bytes - need) & ~int64_t{15};
+        const Int4GemmShape shape = int4_gemm_shape(a.M, a.N, a.K, groupsize, left);
         const long long wgs32 = static_cast<long long>((a.M + 127) / 128) * ((a.N + 127) / 128);
-        const bool use32 = options().int4_gemm32_min_rows > 0 ? a.M >= options().int4_gemm32_min_rows : wgs32 >= 320;
+        const long long wgs16 = static_cast<long long>((tiles16 + 4 * sh.t - 1) / (4 * sh.t)) * ((a.M + 63) / 64);
+        const double us16 = 4 + (sh.t == 2 ? 1.15 : 0.9) * (a.K / 128) * (1 + 0.45 * static_cast<double>((wgs16 - 1) / kCUs));
+        const bool use32 = options().int4_gemm32_min_rows > 0 ? a.M >= options().int4_gemm32_min_rows : wgs32 >= 320 || 1.5 * shape.us < us16;
         if (use32 && !options().int4_no_gemm32) {
-          const int rc32 = int4_gemm32(a.x, a.packed, a.sz, a.y, xs, stride, a.M, a.N, a.K, groupsize, a.stream);
+          float *partials = reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + need);  // need is a multiple of 256
+          const int rc32 = int4_gemm(a.x, a.packed, a.sz, a.y, xs, stride, partials, shape, a.M, a.N, a.K, groupsize, a.stream);
           if (rc32 != E2H_OK) return rc32;
           continue;
         }

@@ -100,9 +100,16 @@ __device__ __forceinline__ void store_tiles_via_lds(const e2h_f32x16_t (&acc)[CT
 // (defined in e2h_int4_mm.hip; groupsize in {32, 64, 128}).
 int launch_x_group_sums(const uint16_t *x, float *out, int M, int K, int stride, int groupsize, hipStream_t stream);
 
-// Many-row int4 matmul on 32x32 MFMA tiles (e2h_int4_gemm.hip); xsum as written by launch_x_group_sums.
-int int4_gemm32(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint16_t *y, const float *xsum, int xsum_stride,
-                int M, int N, int K, int groupsize, hipStream_t stream);
+// Many-row int4 matmul on 32x32 MFMA tiles (e2h_int4_gemm.hip); xsum as written by launch_x_group_sums.  A workgroup owns `rows` rows;
+// K may be shared by `slices` of them through float32 sums in `partials` ([slices][M][N]; unused with one slice).  int4_gemm_shape picks
+// both, with at most as many slices as fit scratch_bytes.
+struct Int4GemmShape {
+  int rows, slices;
+  double us;  // expected time
+};
+Int4GemmShape int4_gemm_shape(int M, int N, int K, int groupsize, int64_t scratch_bytes);
+int int4_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint16_t *y, const float *xsum, int xsum_stride,
+              float *partials, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream);
 
 // Many-row int4 matmul, 256 x 256 outputs per workgroup, weights dequantized to bfloat16 on the way into the matrix
 // cores (e2h_int4_gemm128.hip); needs no scratch memory.

@@ -1,0 +1,84 @@
+"""The many-row int4 matmul (csrc/e2h_int4_gemm.hip) at its edges: rows around its workgroups of 64 and 128, columns that end inside a
+workgroup, odd counts of 128-wide k blocks, K slices, and scales that its running units do not carry.
+
+Operands are chosen so that every product and sum is a small multiple of a power of two (codes, x in -2 .. 2, scales 2^-3 .. 2^3,
+zeros in quarters), below 2^24 of its unit in any order: the result has to be the exactly rounded one."""
+
+import pytest
+import torch
+
+from easy_to_hard_amd import _lib, ops
+from oracle import quant_oracle as qo
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture
+def many_row_kernel():
+    _lib.set_option("int4_gemm32_min_rows", 1)
+    yield
+    _lib.set_option("int4_gemm32_min_rows", 0)
+    _lib.set_option("int4_k_slices", 0)
+    _lib.set_option("int4_gemm_tile", 0)
+
+
+def _case(m, n, k, g, seed=5, low=-3, high=3):
+    gen = torch.Generator().manual_seed(seed + m + n + k + g)
+    codes = torch.randint(0, 16, (n, k), generator=gen, dtype=torch.int32)
+    scale = torch.exp2(torch.randint(low, high + 1, (k // g, n), generator=gen).float())
+    zero = torch.randint(-8, 9, (k // g, n), generator=gen).float() / 4
+    x = torch.randint(-2, 3, (m, k), generator=gen).to(torch.bfloat16).to(DEV)
+    return codes, scale, zero, x
+
+
+def _run(codes, scale, zero, x, g):
+    packed = torch.from_numpy(qo.int4_tile_pack(codes.numpy(), 8)).to(DEV)
+    sz = torch.stack([scale, zero], dim=-1).to(torch.bfloat16).contiguous().to(DEV)
+    n, k = codes.shape
+    w = ((codes.double() - 8).view(n, k // g, g) * scale.double().t()[:, :, None] + zero.double().t()[:, :, None]).view(n, k).to(DEV)
+    return ops.int4_mm(x, packed, g, sz), x.double() @ w.t()
+
+
+@pytest.mark.parametrize("g", [32, 64, 128])
+@pytest.mark.parametrize("slices", [1, 2, 8])
+@pytest.mark.parametrize("tile", [0, 128])
+@pytest.mark.parametrize("m,n,k", [(65, 8, 128), (64 + 1, 264, 384), (128, 256, 1024), (129, 520, 1152), (471, 1032, 2176)])
+def test_exact_on_dyadic_operands(many_row_kernel, g, slices, tile, m, n, k):
+    _lib.set_option("int4_k_slices", slices)
+    _lib.set_option("int4_gemm_tile", tile)
+    got, want = _run(*_case(m, n, k, g), g)
+    assert torch.equal(got, want.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("g", [32, 64, 128])
+@pytest.mark.parametrize("slices", [1, 2])
+def test_scales_outside_the_running_units(many_row_kernel, g, slices):
+    """zero, the smallest and large scales in some columns: those workgroups form every group's sum by itself.  Columns whose scales are
+    all representable stay exact; a column with an infinite or NaN scale is not finite, its neighbours are untouched."""
+    m, n, k = 130, 528, 1024
+    _lib.set_option("int4_k_slices", slices)
+    codes, scale, zero, x = _case(m, n, k, g)
+    scale[0, 3] = 0.0
+    zero[:, 5], scale[:, 5] = 0.0, 2.0**-100
+    zero[:, 260], scale[:, 260] = 0.0, 2.0**40
+    scale[-1, 300] = float("inf")
+    scale[-1, 301] = float("nan")
+    got, want = _run(codes, scale, zero, x, g)
+    finite = torch.ones(n, dtype=torch.bool)
+    finite[[300, 301]] = False
+    assert torch.equal(got[:, finite], want[:, finite].to(torch.bfloat16))
+    assert not torch.isfinite(got[:, 301]).any() and not torch.isfinite(got[:, 300]).all()
+
+
+def test_error_is_that_of_the_final_rounding(many_row_kernel):
+    """random scales over a wide range and x with a mean: against 64 bits the relative error stays that of rounding to bfloat16,
+    at most 2^-9 per value plus the float32 sums' share (K = 4096 terms of up to 31 |x s|, 2^-24 each, far below 2^-12 here)"""
+    gen = torch.Generator().manual_seed(9)
+    m, n, k, g = 200, 512, 4096, 64
+    codes = torch.randint(0, 16, (n, k), generator=gen, dtype=torch.int32)
+    scale = torch.exp2(torch.rand((k // g, n), generator=gen) * 16 - 14).to(torch.bfloat16).float()
+    zero = torch.randn((k // g, n), generator=gen).to(torch.bfloat16).float()
+    x = (torch.randn((m, k), generator=gen) + 1).to(torch.bfloat16).to(DEV)
+    got, want = _run(codes, scale, zero, x, g)
+    assert (got.double() - want).norm() <= 2**-9 * want.norm()
