@@ -11,14 +11,16 @@ from . import seq_ops
 
 class DecodeLinear(nn.Linear):
     def forward(self, x: Tensor) -> Tensor:
-        if self.bias is None and seq_ops.linear_streams(x, self.weight):
-            return seq_ops.linear(x, self.weight)
-        return F.linear(x, self.weight, self.bias)
+        weight, bias = self.weight, self.bias
+        # the count first: the linears of short prompts are bound by what the host does for each of them
+        if x.numel() <= seq_ops.STREAMED_ROWS * self.in_features and bias is None and seq_ops.linear_streams(x, weight):
+            return seq_ops.linear(x, weight)
+        return F.linear(x, weight, bias)
 
 
 def fusable(lin: nn.Module, x: Tensor) -> bool:
     """True where lin(x) may be computed together with what follows it: the module itself (not a replacement), nobody watching its
     call, and an input that its kernel takes."""
-    return (type(lin) is DecodeLinear and lin.bias is None and seq_ops.linear_streams(x, lin.weight)
+    return (type(lin) is DecodeLinear and x.numel() <= seq_ops.STREAMED_ROWS * lin.in_features and lin.bias is None and seq_ops.linear_streams(x, lin.weight)
             and not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks
                      or _module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks))

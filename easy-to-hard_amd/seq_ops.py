@@ -124,10 +124,13 @@ def softcap_(x, cap):
 ACT_NONE, ACT_SQUARE_RELU, ACT_SOFTCAP = 0, 1, 2
 
 
+STREAMED_ROWS = 64
+
+
 def linear_streams(x, weight):
     """True where `linear` takes x [.., k] and weight [n, k]: bfloat16 on the GPU, up to 64 rows, no gradients."""
     k = weight.shape[1]
-    if not 0 < x.numel() <= 64 * k:  # first: prompts come by here with every linear
+    if not 0 < x.numel() <= STREAMED_ROWS * k:
         return False
     if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or not x.is_cuda or weight.device != x.device or x.shape[-1] != k:
         return False
@@ -140,16 +143,21 @@ def linear(x, weight, act=ACT_NONE, cap=0.0):
     """act(x weight^T) of a decode batch, see e2h_seq_linear; operands that are not 16-byte aligned or not contiguous are copied."""
     _need_gpu(x, weight)
     n, k = weight.shape
-    rows2d = x.reshape(-1, k).contiguous()
-    weight = weight.contiguous()
-    rows2d, weight = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (rows2d, weight))
-    y = torch.empty((rows2d.shape[0], n), dtype=x.dtype, device=x.device)
+    rows = x.numel() // k
+    x2d = x if x.is_contiguous() else x.contiguous()  # the kernel reads it as [rows, k]
+    if not weight.is_contiguous():
+        weight = weight.contiguous()
+    if x2d.data_ptr() % 16:
+        x2d = x2d.clone()
+    if weight.data_ptr() % 16:
+        weight = weight.clone()
+    y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
     lib = _lib_for(x)
-    need = lib.e2h_seq_linear_scratch_bytes(rows2d.shape[0], n, k)
+    need = lib.e2h_seq_linear_scratch_bytes(rows, n, k)
     scratch = torch.empty((need,), dtype=torch.uint8, device=x.device) if need > 0 else None
-    _lib.check_seq(lib.e2h_seq_linear(_p(rows2d), _p(weight), _p(y), rows2d.shape[0], n, k, act, cap, _p(scratch), max(need, 0), _stream(x)),
+    _lib.check_seq(lib.e2h_seq_linear(_p(x2d), _p(weight), _p(y), rows, n, k, act, cap, _p(scratch), max(need, 0), _stream(x)),
                    "e2h_seq_linear")
-    return y.view(*x.shape[:-1], n)
+    return y
 
 
 def gelu_gate_rows(gate, table, tokens, column):
