@@ -277,6 +277,7 @@ __global__ __launch_bounds__(64 * kColWaves) void int8_stream_mm_kernel(const ui
       const uint32_t live = i < nchunks ? 0xFFFFFFFFu : 0u;
       if (j % CPP == 0) load_x(xstage[(j / CPP) % XD], phase + XD);
       load_weights(ring[(j + PD) % NB], chunk_at(i + PD));
+      __builtin_amdgcn_sched_barrier(0);  // the scheduler would sink the loads to their first use (65 rows, 4096 x 4096: 40 us, so 31)
       compute_chunk(ring[j % NB], phase, j % CPP, live);
       if (j % CPP == CPP - 1) {
         store_x(xstage[(j / CPP + 1) % XD], phase + 1);
