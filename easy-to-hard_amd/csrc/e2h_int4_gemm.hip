@@ -11,8 +11,10 @@
 // Scales.  An accumulator is kept in units of its column's current scale: entering group g it is multiplied by
 // s[g-1,n] / s[g,n], and the group's products then add to it directly.  No second set of registers for the sums of one group,
 // which is what lets a wave own 128 rows x 64 columns, so that one unpacked fragment feeds four MFMAs and one activation
-// fragment two.  Scales outside 2^-26 .. 2^6 (zeros, infinities, NaN among them; the quantizer's lie between 2^-24 and a few units)
-// could leave float32's range that way: a workgroup that meets one takes a plain loop that forms every group's sum by itself.
+// fragment two.  A workgroup that meets a scale outside 2^-26 .. 2^6 (zeros, infinities, NaN among them; the quantizer's lie between
+// 2^-24 and a few units) takes a plain loop that forms every group's sum by itself.  So does a wave whose sums leave float32's range in
+// units of the scales although they may not by themselves (a zero of 2^100 beside a scale of 2^-20, activations near the type's
+// end): an infinity or NaN in an accumulator stays one to the end, where it is looked for, but for the rows that have one in x.
 //
 // The zero-point term is a matrix product over the groups.  It starts the accumulators: X and z - 24 s are each split into three
 // bfloat16 parts (exact: 3 x 8 bits), and eight of the nine products of parts (all but low x low, 2^-32) fill one lane's eight k values,
@@ -143,6 +145,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[ct][rt][e] = 0.f;
   bool odd_scale = false;
+  float not_finite[kRT] = {};  // NaN once this lane met a group sum of its row that is not finite
   struct Zero {
     float xs[4];
     uint32_t szw[kCT];
@@ -155,9 +158,11 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
       const int g = g0 + 2 * i;
       const uint32_t out = dead(g), gs = static_cast<uint32_t>(g < g_end ? g : g_begin);
 #pragma unroll
-      for (int rt = 0; rt < kRT; ++rt)
-        z[i].xs[rt] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xs_rsrc, static_cast<uint32_t>(h * a.xsum_stride + row0 + 32 * rt + n) * 4u | out,
+      for (int rt = 0; rt < kRT; ++rt) {
+        const int row = row0 + 32 * rt + n;  // past M: zeros, so that nothing there overflows
+        z[i].xs[rt] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xs_rsrc, row < M ? static_cast<uint32_t>(h * a.xsum_stride + row) * 4u | out : 0x80000000u,
                                                                                      gs * a.xsum_stride * 4u, 0));
+      }
 #pragma unroll
       for (int ct = 0; ct < kCT; ++ct)
         z[i].szw[ct] = __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, (szlane[ct] + static_cast<uint32_t>(h) * N * 4u) | out, gs * N * 4u, 0);
@@ -176,7 +181,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
 #pragma unroll
       for (int ct = 0; ct < kCT; ++ct) {
         const float scale = __builtin_bit_cast(float, za[i].szw[ct] << 16), zero = __builtin_bit_cast(float, za[i].szw[ct] & 0xFFFF0000u);
-        odd_scale |= !dead(g0 + 2 * i) && !(__builtin_fabsf(scale) >= 0x1p-26f && __builtin_fabsf(scale) <= 0x1p6f && __builtin_fabsf(zero) <= 0x1p100f);
+        odd_scale |= !dead(g0 + 2 * i) && !(__builtin_fabsf(scale) >= 0x1p-26f && __builtin_fabsf(scale) <= 0x1p6f);
         float p[3];
         split3(__builtin_fmaf(-24.0f, scale, zero), p);
         const uint32_t hm = high_halves(p[1], p[0]);
@@ -185,6 +190,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
 #pragma unroll
       for (int rt = 0; rt < kRT; ++rt) {
         float p[3];
+        not_finite[rt] = __builtin_fmaf(za[i].xs[rt], 0.f, not_finite[rt]);
         split3(za[i].xs[rt], p);
         const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, u32x4_t{high_halves(p[0], p[0]), high_halves(p[1], p[1]), high_halves(p[2], p[0]), high_halves(p[2], p[1])});
 #pragma unroll
@@ -195,179 +201,208 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
     for (int i = 0; i < kBatch; ++i) za[i] = zb[i];
   }
 
+  uint32_t odd_rows[kRT];  // bit r: row r of the tile has a value that is not finite
+#pragma unroll
+  for (int rt = 0; rt < kRT; ++rt) {
+    const uint64_t lanes = __builtin_amdgcn_ballot_w64(!(not_finite[rt] == 0.f));
+    odd_rows[rt] = static_cast<uint32_t>(lanes) | static_cast<uint32_t>(lanes >> 32);
+  }
+
   // do all waves know the same?  (the third activation stage is free until the loop)
   uint32_t *const votes = reinterpret_cast<uint32_t *>(lds + 2 * kXStage);
   const bool odd_wave = __builtin_amdgcn_ballot_w64(odd_scale) != 0;
   if (lane == 0) votes[wave] = odd_wave;
   lds_barrier();
-  if (__builtin_amdgcn_readfirstlane(votes[0] | votes[1] | votes[2] | votes[3])) {
-    // a scale that the running units do not carry: every group's sum by itself, operands straight from memory
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the loads above still write LDS
-#pragma unroll 1
-    for (int t = 0; t < kCT * kRT; ++t) {
-      const int ct = t / kRT, rt = t % kRT;
-      int row = row0 + 32 * rt + n;
-      row = row < M ? row : M - 1;
-      int col = col0 + 32 * ct + n;
-      col = col < N ? col : N - 1;
-      const uint32_t xo = static_cast<uint32_t>(static_cast<size_t>(row) * K * 2) + 16u * h;
-      const uint32_t wo = static_cast<uint32_t>(static_cast<size_t>(col >> 3) * KT * 512 + (col & 7) * 64);
-      f32x16_t sum = {};
-      for (int g = g_begin; g < g_end; ++g) {
-        f32x16_t part = {};
-        for (int s = 0; s < SPG; ++s) {
-          const int step = g * SPG + s;  // of 16 k
-          const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xo, static_cast<uint32_t>(step) * 32u, 0));
-          u32x4_t u;
+  bool plain = __builtin_amdgcn_readfirstlane(votes[0] | votes[1] | votes[2] | votes[3]) != 0;
+  if (!plain) {
+    // ---- fragments: activation (row tile rt, step s): row 32 rt + n, piece 2 s + h; weights (column tile ct): pieces j of column 32 ct + n
+    uint32_t a_lane[4], w_lane[4];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(w_rsrc, wo + 16u * j, static_cast<uint32_t>(step >> 3) * 512u + ((step >> 1) & 3) * 4u, 0);
-            u[j] = (__builtin_amdgcn_alignbit(w, w, (8 * (step & 1) + 4 * h - 3) & 31) & 0x00780078u) | 0x41804180u;
-          }
-          part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf, __builtin_bit_cast(bf16x8_t, u), part, 0, 0, 0);
-        }
-        const uint32_t szw = __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, static_cast<uint32_t>(col) * 4u, static_cast<uint32_t>(g) * N * 4u, 0);
-        const float scale = __builtin_bit_cast(float, szw << 16), zero = __builtin_bit_cast(float, szw & 0xFFFF0000u);
-        const float zc = __builtin_fmaf(-24.0f, scale, zero);
+    for (int s = 0; s < 4; ++s) a_lane[s] = static_cast<uint32_t>(n * 128 + (((2 * s + h) ^ ((n >> 1) & 7)) << 4));
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const float xg_e = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xs_rsrc, static_cast<uint32_t>(row0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3)) * 4u,
-                                                                                          static_cast<uint32_t>(g) * a.xsum_stride * 4u, 0));
-          sum[e] = __builtin_fmaf(zc, xg_e, __builtin_fmaf(scale, part[e], sum[e]));
+    for (int j = 0; j < 4; ++j) w_lane[j] = static_cast<uint32_t>(wave * 4096 + n * 64 + ((j ^ ((n >> 2) & 3)) << 4));
+    bf16x8_t af[2][kRT], wf[2][kCT];
+    u32x4_t wq[kCT][4];
+    const auto read_a = [&](bf16x8_t (&f)[kRT], uint32_t stage, int s) {
+#pragma unroll
+      for (int rt = 0; rt < kRT; ++rt) f[rt] = *reinterpret_cast<const bf16x8_t *>(lds + stage + a_lane[s] + rt * 4096);
+    };
+    const auto read_w = [&](uint32_t stage) {
+#pragma unroll
+      for (int ct = 0; ct < kCT; ++ct)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) wq[ct][j] = *reinterpret_cast<const u32x4_t *>(lds + stage + w_lane[j] + ct * 2048);
+    };
+    uint32_t mask, magic;  // one scalar and one vector register, so that each pair of codes is one and-or
+    asm volatile("s_mov_b32 %0, 0x00780078" : "=s"(mask));
+    asm volatile("v_mov_b32 %0, 0x41804180" : "=v"(magic));
+    const uint32_t rot0 = (4 * h - 3) & 31, rot1 = (4 * h + 5) & 31;
+    const auto convert = [&](bf16x8_t (&f)[kCT], int s8) {
+#pragma unroll
+      for (int ct = 0; ct < kCT; ++ct) {
+        u32x4_t u;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t w = wq[ct][j][s8 >> 1];
+          u[j] = (__builtin_amdgcn_alignbit(w, w, s8 & 1 ? rot1 : rot0) & mask) | magic;
         }
+        f[ct] = __builtin_bit_cast(bf16x8_t, u);
       }
-      if (col0 + 32 * ct + n < N)
-        for (int e = 0; e < 16; ++e) {
-          const int m = row0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3);
-          if (m >= M) continue;
-          if (a.partials) a.partials[(static_cast<size_t>(blockIdx.y) * M + m) * N + col] = sum[e];
-          else a.y[static_cast<size_t>(m) * N + col] = f32_to_bf16_rne(sum[e]);
-        }
-    }
-    return;
-  }
+    };
 
-  // ---- fragments: activation (row tile rt, step s): row 32 rt + n, piece 2 s + h; weights (column tile ct): pieces j of column 32 ct + n
-  uint32_t a_lane[4], w_lane[4];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) a_lane[s] = static_cast<uint32_t>(n * 128 + (((2 * s + h) ^ ((n >> 1) & 7)) << 4));
-#pragma unroll
-  for (int j = 0; j < 4; ++j) w_lane[j] = static_cast<uint32_t>(wave * 4096 + n * 64 + ((j ^ ((n >> 2) & 3)) << 4));
-  bf16x8_t af[2][kRT], wf[2][kCT];
-  u32x4_t wq[kCT][4];
-  const auto read_a = [&](bf16x8_t (&f)[kRT], uint32_t stage, int s) {
-#pragma unroll
-    for (int rt = 0; rt < kRT; ++rt) f[rt] = *reinterpret_cast<const bf16x8_t *>(lds + stage + a_lane[s] + rt * 4096);
-  };
-  const auto read_w = [&](uint32_t stage) {
+    float unit[kCT] = {1.f, 1.f};  // what one step of the accumulators is worth
+    constexpr int kSc = NGRP < 2 ? NGRP : 2;  // pairs held ahead
+    uint32_t sc[kCT][kSc];
 #pragma unroll
     for (int ct = 0; ct < kCT; ++ct)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) wq[ct][j] = *reinterpret_cast<const u32x4_t *>(lds + stage + w_lane[j] + ct * 2048);
-  };
-  uint32_t mask, magic;  // one scalar and one vector register, so that each pair of codes is one and-or
-  asm volatile("s_mov_b32 %0, 0x00780078" : "=s"(mask));
-  asm volatile("v_mov_b32 %0, 0x41804180" : "=v"(magic));
-  const uint32_t rot0 = (4 * h - 3) & 31, rot1 = (4 * h + 5) & 31;
-  const auto convert = [&](bf16x8_t (&f)[kCT], int s8) {
+      for (int g = 0; g < kSc; ++g) sc[ct][g] = load_sz(ct, g_begin + g);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    asm volatile("s_barrier" ::: "memory");
+    read_w(kLdsW);
+    read_a(af[0], 0, 0);
+    convert(wf[0], 0);
+    uint32_t s0 = 0, s1 = kXStage, s2 = 2 * kXStage;  // stage of the chunk in use, of the next one, of the one after
+    uint32_t w_next = kLdsW + kWStage;
+
+    for (int blk = blk0; blk < blk1; ++blk) {
+      load_w(blk + 1, w_next);
+      load_x(2 * blk + 2, s2);
 #pragma unroll
-    for (int ct = 0; ct < kCT; ++ct) {
-      u32x4_t u;
+      for (int s8 = 0; s8 < 8; ++s8) {
+        const int cur = s8 & 1;
+        if (s8 == 4) load_x(2 * blk + 3, s0);  // every wave left that stage at the barrier below
+        // The second chunk is in: loads issued after it are this block's words, its next chunk and the scale pairs of the last half block of each kind.  The
+        // next block's words and first chunk are in: after them came one chunk and this block's scale pairs.
+        if (s8 == 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(4 + kRT + (NGRP == 1 ? 2 : 2 * NGRP)) : "memory");
+        if (s8 == 7) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kRT + 2 * NGRP) : "memory");
+        if (s8 == 7) read_w(w_next);
+        read_a(af[cur ^ 1], s8 < 3 ? s0 : s8 < 7 ? s1 : s2, (s8 + 1) & 3);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t w = wq[ct][j][s8 >> 1];
-        u[j] = (__builtin_amdgcn_alignbit(w, w, s8 & 1 ? rot1 : rot0) & mask) | magic;
+        for (int ct = 0; ct < kCT; ++ct) {
+          float r = 1.f;
+          if (s8 % SPG == 0) {
+            const float s = __builtin_bit_cast(float, sc[ct][s8 / SPG % kSc] << 16);
+            r = unit[ct] / s;
+            unit[ct] = s;
+            sc[ct][s8 / SPG % kSc] = load_sz(ct, blk * NGRP + s8 / SPG + kSc);
+          }
+#pragma unroll
+          for (int rt = 0; rt < kRT; ++rt) {
+            if (s8 % SPG == 0) {
+              __builtin_amdgcn_sched_barrier(0);  // one tile's rescaling under the previous tile's product
+#pragma unroll
+              for (int e = 0; e < 16; ++e) acc[ct][rt][e] *= r;
+            }
+            acc[ct][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[cur][rt], wf[cur][ct], acc[ct][rt], 0, 0, 0);
+          }
+        }
+        convert(wf[cur ^ 1], (s8 + 1) & 7);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      f[ct] = __builtin_bit_cast(bf16x8_t, u);
+      const uint32_t t = s0;  // two chunks on
+      s0 = s2;
+      s2 = s1;
+      s1 = t;
+      w_next ^= kLdsW ^ (kLdsW + kWStage);
     }
-  };
-
-  float unit[kCT] = {1.f, 1.f};  // what one step of the accumulators is worth
-  constexpr int kSc = NGRP < 2 ? NGRP : 2;  // pairs held ahead
-  uint32_t sc[kCT][kSc];
+    // the loads issued past the last block still write LDS: drain them before the stages are reused
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // Is a sum not finite in its column's units?  A row whose x is not finite stays out: nothing could make it so.
+    bool over = false;
 #pragma unroll
-  for (int ct = 0; ct < kCT; ++ct)
-#pragma unroll
-    for (int g = 0; g < kSc; ++g) sc[ct][g] = load_sz(ct, g_begin + g);
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-  asm volatile("s_barrier" ::: "memory");
-  read_w(kLdsW);
-  read_a(af[0], 0, 0);
-  convert(wf[0], 0);
-  uint32_t s0 = 0, s1 = kXStage, s2 = 2 * kXStage;  // stage of the chunk in use, of the next one, of the one after
-  uint32_t w_next = kLdsW + kWStage;
-
-  for (int blk = blk0; blk < blk1; ++blk) {
-    load_w(blk + 1, w_next);
-    load_x(2 * blk + 2, s2);
-#pragma unroll
-    for (int s8 = 0; s8 < 8; ++s8) {
-      const int cur = s8 & 1;
-      if (s8 == 4) load_x(2 * blk + 3, s0);  // every wave left that stage at the barrier below
-      // The second chunk is in: loads issued after it are this block's words, its next chunk and the scale pairs of the last half block of each kind.  The
-      // next block's words and first chunk are in: after them came one chunk and this block's scale pairs.
-      if (s8 == 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(4 + kRT + (NGRP == 1 ? 2 : 2 * NGRP)) : "memory");
-      if (s8 == 7) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kRT + 2 * NGRP) : "memory");
-      if (s8 == 7) read_w(w_next);
-      read_a(af[cur ^ 1], s8 < 3 ? s0 : s8 < 7 ? s1 : s2, (s8 + 1) & 3);
-      __builtin_amdgcn_sched_barrier(0);
+    for (int rt = 0; rt < kRT; ++rt) {
 #pragma unroll
       for (int ct = 0; ct < kCT; ++ct) {
-        float r = 1.f;
-        if (s8 % SPG == 0) {
-          const float s = __builtin_bit_cast(float, sc[ct][s8 / SPG % kSc] << 16);
-          r = unit[ct] / s;
-          unit[ct] = s;
-          sc[ct][s8 / SPG % kSc] = load_sz(ct, blk * NGRP + s8 / SPG + kSc);
-        }
+        float t[2] = {0.f, 0.f};  // zero times an infinity or a NaN is a NaN
+        if (odd_rows[rt] == 0) {
 #pragma unroll
-        for (int rt = 0; rt < kRT; ++rt) {
-          if (s8 % SPG == 0) {
-            __builtin_amdgcn_sched_barrier(0);  // one tile's rescaling under the previous tile's product
+          for (int e = 0; e < 16; ++e) t[e & 1] = __builtin_fmaf(acc[ct][rt][e], 0.f, t[e & 1]);
+        } else {
+          const uint32_t mine = odd_rows[rt] >> (4 * h);
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[ct][rt][e] *= r;
-          }
-          acc[ct][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[cur][rt], wf[cur][ct], acc[ct][rt], 0, 0, 0);
+          for (int e = 0; e < 16; ++e) t[e & 1] = __builtin_fmaf(mine >> (8 * (e >> 2) + (e & 3)) & 1 ? 0.f : acc[ct][rt][e], 0.f, t[e & 1]);
         }
+        over |= !(t[0] + t[1] == 0.f);
       }
-      convert(wf[cur ^ 1], (s8 + 1) & 7);
-      __builtin_amdgcn_sched_barrier(0);
     }
-    const uint32_t t = s0;  // two chunks on
-    s0 = s2;
-    s2 = s1;
-    s1 = t;
-    w_next ^= kLdsW ^ (kLdsW + kWStage);
-  }
-  // the loads issued past the last block still write LDS: drain them before the stages are reused
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    plain = __builtin_amdgcn_ballot_w64(over) != 0;
+    if (!plain) {
 #pragma unroll
-  for (int ct = 0; ct < kCT; ++ct)
+      for (int ct = 0; ct < kCT; ++ct)
 #pragma unroll
-    for (int rt = 0; rt < kRT; ++rt)
+        for (int rt = 0; rt < kRT; ++rt)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[ct][rt][e] *= unit[ct];
+          for (int e = 0; e < 16; ++e) acc[ct][rt][e] *= unit[ct];
 
-  // ---- store: lane (h, n) holds column col0 + 32 ct + n, rows 8 (e / 4) + 4 h + e % 4 of each tile -----------
-  if (a.partials) {
-    float *out = a.partials + static_cast<size_t>(blockIdx.y) * M * N;
+      // ---- store: lane (h, n) holds column col0 + 32 ct + n, rows 8 (e / 4) + 4 h + e % 4 of each tile -----------
+      if (a.partials) {
+        float *out = a.partials + static_cast<size_t>(blockIdx.y) * M * N;
 #pragma unroll
-    for (int ct = 0; ct < kCT; ++ct) {
-      const int col = col0 + 32 * ct + n;
-      if (col >= N) continue;
+        for (int ct = 0; ct < kCT; ++ct) {
+          const int col = col0 + 32 * ct + n;
+          if (col >= N) continue;
 #pragma unroll
-      for (int rt = 0; rt < kRT; ++rt)
+          for (int rt = 0; rt < kRT; ++rt)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int m = row0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3);
-          if (m < M) out[static_cast<size_t>(m) * N + col] = acc[ct][rt][e];
+            for (int e = 0; e < 16; ++e) {
+              const int m = row0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3);
+              if (m < M) out[static_cast<size_t>(m) * N + col] = acc[ct][rt][e];
+            }
         }
+        return;
+      }
+      const float no_scale[kCT] = {};
+      store_tiles_via_lds<kRT, kCT, false>(acc, no_scale, lds + wave * TileStore<kCT>::kBytesPerWave, a.y, row0, col0, M, N, lane,
+                                          (N & 7) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0);
+      return;
     }
-    return;
   }
-  const float no_scale[kCT] = {};
-  store_tiles_via_lds<kRT, kCT, false>(acc, no_scale, lds + wave * TileStore<kCT>::kBytesPerWave, a.y, row0, col0, M, N, lane,
-                                    (N & 7) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0);
+
+  // Every group's sum by itself, operands straight from memory, nothing shared with the other waves.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the first loads still write LDS
+#pragma unroll 1
+  for (int t = 0; t < kCT * kRT; ++t) {
+    const int ct = t / kRT, rt = t % kRT;
+    int row = row0 + 32 * rt + n;
+    row = row < M ? row : M - 1;
+    int col = col0 + 32 * ct + n;
+    col = col < N ? col : N - 1;
+    const uint32_t xo = static_cast<uint32_t>(static_cast<size_t>(row) * K * 2) + 16u * h;
+    const uint32_t wo = static_cast<uint32_t>(static_cast<size_t>(col >> 3) * KT * 512 + (col & 7) * 64);
+    f32x16_t sum = {};
+    for (int g = g_begin; g < g_end; ++g) {
+      f32x16_t part = {};
+      for (int s = 0; s < SPG; ++s) {
+        const int step = g * SPG + s;  // of 16 k
+        const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xo, static_cast<uint32_t>(step) * 32u, 0));
+        u32x4_t u;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(w_rsrc, wo + 16u * j, static_cast<uint32_t>(step >> 3) * 512u + ((step >> 1) & 3) * 4u, 0);
+          u[j] = (__builtin_amdgcn_alignbit(w, w, (8 * (step & 1) + 4 * h - 3) & 31) & 0x00780078u) | 0x41804180u;
+        }
+        part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf, __builtin_bit_cast(bf16x8_t, u), part, 0, 0, 0);
+      }
+      const uint32_t szw = __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, static_cast<uint32_t>(col) * 4u, static_cast<uint32_t>(g) * N * 4u, 0);
+      const float scale = __builtin_bit_cast(float, szw << 16), zero = __builtin_bit_cast(float, szw & 0xFFFF0000u);
+      const float zc = __builtin_fmaf(-24.0f, scale, zero);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float xg_e = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xs_rsrc, static_cast<uint32_t>(row0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3)) * 4u,
+                                                                                        static_cast<uint32_t>(g) * a.xsum_stride * 4u, 0));
+        sum[e] = __builtin_fmaf(zc, xg_e, __builtin_fmaf(scale, part[e], sum[e]));
+      }
+    }
+    if (col0 + 32 * ct + n < N)
+      for (int e = 0; e < 16; ++e) {
+        const int m = row0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3);
+        if (m >= M) continue;
+        if (a.partials) a.partials[(static_cast<size_t>(blockIdx.y) * M + m) * N + col] = sum[e];
+        else a.y[static_cast<size_t>(m) * N + col] = f32_to_bf16_rne(sum[e]);
+      }
+  }
 }
 
 constexpr int kMostSlices = 8;

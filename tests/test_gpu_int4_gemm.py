@@ -82,3 +82,40 @@ def test_error_is_that_of_the_final_rounding(many_row_kernel):
     x = (torch.randn((m, k), generator=gen) + 1).to(torch.bfloat16).to(DEV)
     got, want = _run(codes, scale, zero, x, g)
     assert (got.double() - want).norm() <= 2**-9 * want.norm()
+
+
+@pytest.mark.parametrize("g", [32, 64, 128])
+@pytest.mark.parametrize("slices", [1, 2])
+@pytest.mark.parametrize("tile", [0, 128])
+def test_sums_that_only_the_running_units_cannot_hold(many_row_kernel, g, slices, tile):
+    """A sum in units of its column's scale may leave float32's range although the sum itself does not: a large zero beside a small scale,
+    and rows of x near the end of the type.  All terms of a column are multiples of one power of two below 2^24 of it
+    (K * 31 * 2 * 2^6 = 2^22 for the products, and the columns with large zeros have products far below half a unit of the sum), so results are exact."""
+    m, n, k = 150, 528, 1024
+    _lib.set_option("int4_k_slices", slices)
+    _lib.set_option("int4_gemm_tile", tile)
+    codes, scale, zero, x = _case(m, n, k, g, low=-20, high=-14)
+    zero = zero.mul(4) * 2.0**-20
+    for col, z in ((5, 2.0**100), (259, -(2.0**99)), (527, 2.0**110)):
+        scale[:, col], zero[:, col] = 2.0**-26, z
+    codes[[5, 259, 527]] = 8
+    x[0], x[70] = 2.0**114, x[70] * 2.0**112  # a group of products alone stays below 128 * 31 * 2^114 < 2^126
+    x[149] = 0
+    cols = torch.ones(n, dtype=torch.bool)
+    cols[[5, 259, 527]] = False
+    got, want = _run(codes, scale, zero, x, g)
+    assert want[:, cols].abs().max() < 2.0**127 and want[0, cols].abs().max() > 2.0**100
+    assert torch.equal(got[:, cols], want[:, cols].to(torch.bfloat16))
+    small = torch.ones(m, dtype=torch.bool)
+    small[[0, 70]] = False
+    assert torch.equal(got[small][:, ~cols], want[small][:, ~cols].to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_a_row_that_is_not_finite_touches_no_other(many_row_kernel, value):
+    codes, scale, zero, x = _case(140, 264, 512, 64)
+    x[3, 77] = value
+    got, want = _run(codes, scale, zero, x, 64)
+    rest = torch.arange(140) != 3
+    assert not torch.isfinite(got[3]).any()
+    assert torch.equal(got[rest], want[rest].to(torch.bfloat16))
