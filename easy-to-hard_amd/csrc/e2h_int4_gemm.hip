@@ -11,10 +11,13 @@
 // Scales.  An accumulator is kept in units of its column's current scale: entering group g it is multiplied by
 // s[g-1,n] / s[g,n], and the group's products then add to it directly.  No second set of registers for the sums of one group,
 // which is what lets a wave own 128 rows x 64 columns, so that one unpacked fragment feeds four MFMAs and one activation
-// fragment two.  A workgroup that meets a scale outside 2^-26 .. 2^6 (zeros, infinities, NaN among them; the quantizer's lie between
-// 2^-24 and a few units) takes a plain loop that forms every group's sum by itself.  So does a wave whose sums leave float32's range in
-// units of the scales although they may not by themselves (a zero of 2^100 beside a scale of 2^-20, activations near the type's
-// end): an infinity or NaN in an accumulator stays one to the end, where it is looked for, but for the rows that have one in x.
+// fragment two.  In a group whose scale is zero a column's operands are zeros and its unit stays.  Scales between 2^-100 and 2^13 (the
+// quantizer's lie between 2^-24 and a few units) run like that: rescaling by up to 2^113 loses at most 2^-136 of a sum, below the smallest
+// bfloat16.  A workgroup that meets any other (infinities, NaN) forms every group's sum by itself in a plain loop, which takes five to nine
+// times as long (8192 x 11008 x 4096, group size 128, such a scale in every workgroup: 5850 us beside 680).  So does a wave whose
+// sums leave float32's range in units of the scales although they may not by themselves (a zero of 2^100 beside a scale of 2^-20,
+// activations near the type's end): an infinity or NaN in an accumulator stays one to the end, where it is looked for, but for the
+// rows that have one in x.
 //
 // The zero-point term is a matrix product over the groups.  It starts the accumulators: X and z - 24 s are each split into three
 // bfloat16 parts (exact: 3 x 8 bits), and eight of the nine products of parts (all but low x low, 2^-32) fill one lane's eight k values,
@@ -55,6 +58,14 @@ __device__ __forceinline__ void split3(float v, float (&p)[3]) {
   const float r = v - p[0];
   p[1] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) & 0xFFFF0000u);
   p[2] = r - p[1];
+}
+
+// a / b, correctly rounded, for bfloat16 values between 2^-100 and 2^13: the first guess is a few units in the last place off, its residual
+// is exact, and a quotient of two 8-bit significands is no closer to a rounding boundary than 2^-33 of itself.  (A division takes ten
+// instructions; with one per group and column the kernel took 1.2 % longer at group size 64.)
+__device__ __forceinline__ float quotient(float a, float b) {
+  const float rcp = __builtin_amdgcn_rcpf(b), q = a * rcp;
+  return __builtin_fmaf(__builtin_fmaf(-q, b, a), rcp, q);
 }
 
 struct GemmArgs {
@@ -181,7 +192,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
 #pragma unroll
       for (int ct = 0; ct < kCT; ++ct) {
         const float scale = __builtin_bit_cast(float, za[i].szw[ct] << 16), zero = __builtin_bit_cast(float, za[i].szw[ct] & 0xFFFF0000u);
-        odd_scale |= !dead(g0 + 2 * i) && !(__builtin_fabsf(scale) >= 0x1p-26f && __builtin_fabsf(scale) <= 0x1p6f);
+        odd_scale |= !dead(g0 + 2 * i) && !(scale == 0.f || (__builtin_fabsf(scale) >= 0x1p-100f && __builtin_fabsf(scale) <= 0x1p13f));
         float p[3];
         split3(__builtin_fmaf(-24.0f, scale, zero), p);
         const uint32_t hm = high_halves(p[1], p[0]);
@@ -233,9 +244,14 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) wq[ct][j] = *reinterpret_cast<const u32x4_t *>(lds + stage + w_lane[j] + ct * 2048);
     };
-    uint32_t mask, magic;  // one scalar and one vector register, so that each pair of codes is one and-or
-    asm volatile("s_mov_b32 %0, 0x00780078" : "=s"(mask));
-    asm volatile("v_mov_b32 %0, 0x41804180" : "=v"(magic));
+    // of a column's group, so that each pair of codes is one and-or; both zero where the scale is zero: the group adds nothing
+    uint32_t mask[kCT], magic[kCT];
+    const auto enter = [&](int ct, uint32_t pair) {
+      const bool live = (pair & 0x7FFFu) != 0;
+      mask[ct] = live ? 0x00780078u : 0u;
+      magic[ct] = live ? 0x41804180u : 0u;
+      asm volatile("" : "+v"(mask[ct]), "+v"(magic[ct]));  // two registers, not a select behind every pair
+    };
     const uint32_t rot0 = (4 * h - 3) & 31, rot1 = (4 * h + 5) & 31;
     const auto convert = [&](bf16x8_t (&f)[kCT], int s8) {
 #pragma unroll
@@ -244,7 +260,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const uint32_t w = wq[ct][j][s8 >> 1];
-          u[j] = (__builtin_amdgcn_alignbit(w, w, s8 & 1 ? rot1 : rot0) & mask) | magic;
+          u[j] = (__builtin_amdgcn_alignbit(w, w, s8 & 1 ? rot1 : rot0) & mask[ct]) | magic[ct];
         }
         f[ct] = __builtin_bit_cast(bf16x8_t, u);
       }
@@ -261,6 +277,8 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
     asm volatile("s_barrier" ::: "memory");
     read_w(kLdsW);
     read_a(af[0], 0, 0);
+#pragma unroll
+    for (int ct = 0; ct < kCT; ++ct) enter(ct, sc[ct][0]);
     convert(wf[0], 0);
     uint32_t s0 = 0, s1 = kXStage, s2 = 2 * kXStage;  // stage of the chunk in use, of the next one, of the one after
     uint32_t w_next = kLdsW + kWStage;
@@ -283,8 +301,8 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
         for (int ct = 0; ct < kCT; ++ct) {
           float r = 1.f;
           if (s8 % SPG == 0) {
-            const float s = __builtin_bit_cast(float, sc[ct][s8 / SPG % kSc] << 16);
-            r = unit[ct] / s;
+            const float scale = __builtin_bit_cast(float, sc[ct][s8 / SPG % kSc] << 16), s = scale != 0.f ? scale : unit[ct];
+            r = quotient(unit[ct], s);
             unit[ct] = s;
             sc[ct][s8 / SPG % kSc] = load_sz(ct, blk * NGRP + s8 / SPG + kSc);
           }
@@ -298,6 +316,9 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
             acc[ct][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[cur][rt], wf[cur][ct], acc[ct][rt], 0, 0, 0);
           }
         }
+        if ((s8 + 1) % SPG == 0)
+#pragma unroll
+          for (int ct = 0; ct < kCT; ++ct) enter(ct, sc[ct][(s8 + 1) % 8 / SPG % kSc]);
         convert(wf[cur ^ 1], (s8 + 1) & 7);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -360,47 +381,63 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
     }
   }
 
-  // Every group's sum by itself, operands straight from memory, nothing shared with the other waves.
+  // Every group's sum by itself, two row tiles at a time, operands straight from memory, nothing shared with the other waves.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the first loads still write LDS
 #pragma unroll 1
-  for (int t = 0; t < kCT * kRT; ++t) {
-    const int ct = t / kRT, rt = t % kRT;
-    int row = row0 + 32 * rt + n;
-    row = row < M ? row : M - 1;
-    int col = col0 + 32 * ct + n;
-    col = col < N ? col : N - 1;
-    const uint32_t xo = static_cast<uint32_t>(static_cast<size_t>(row) * K * 2) + 16u * h;
+  for (int t = 0; t < kCT * kRT / 2; ++t) {
+    int r0 = row0 + 64 * (t / kCT);
+    asm volatile("" : "+s"(r0));  // keeps the addresses of all rows out of the registers of the loops
+    int col = col0 + 32 * (t % kCT) + n;
+    const bool live = col < N;
+    col = live ? col : N - 1;
     const uint32_t wo = static_cast<uint32_t>(static_cast<size_t>(col >> 3) * KT * 512 + (col & 7) * 64);
-    f32x16_t sum = {};
+    uint32_t xo[2];
+    f32x16_t sum[2] = {};
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      const int row = r0 + 32 * rt + n;
+      xo[rt] = static_cast<uint32_t>(static_cast<size_t>(row < M ? row : M - 1) * K * 2) + 16u * h;
+    }
+#pragma unroll 1
     for (int g = g_begin; g < g_end; ++g) {
-      f32x16_t part = {};
+      f32x16_t part[2] = {};
+#pragma unroll 4
       for (int s = 0; s < SPG; ++s) {
         const int step = g * SPG + s;  // of 16 k
-        const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xo, static_cast<uint32_t>(step) * 32u, 0));
         u32x4_t u;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(w_rsrc, wo + 16u * j, static_cast<uint32_t>(step >> 3) * 512u + ((step >> 1) & 3) * 4u, 0);
           u[j] = (__builtin_amdgcn_alignbit(w, w, (8 * (step & 1) + 4 * h - 3) & 31) & 0x00780078u) | 0x41804180u;
         }
-        part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf, __builtin_bit_cast(bf16x8_t, u), part, 0, 0, 0);
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) {
+          const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, xo[rt], static_cast<uint32_t>(step) * 32u, 0));
+          part[rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf, __builtin_bit_cast(bf16x8_t, u), part[rt], 0, 0, 0);
+        }
       }
       const uint32_t szw = __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, static_cast<uint32_t>(col) * 4u, static_cast<uint32_t>(g) * N * 4u, 0);
       const float scale = __builtin_bit_cast(float, szw << 16), zero = __builtin_bit_cast(float, szw & 0xFFFF0000u);
       const float zc = __builtin_fmaf(-24.0f, scale, zero);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const float xg_e = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xs_rsrc, static_cast<uint32_t>(row0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3)) * 4u,
-                                                                                        static_cast<uint32_t>(g) * a.xsum_stride * 4u, 0));
-        sum[e] = __builtin_fmaf(zc, xg_e, __builtin_fmaf(scale, part[e], sum[e]));
-      }
+      for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {  // rows 8 q + 4 h .. + 3 of the tile
+          const f32x4_t xg = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(xs_rsrc, static_cast<uint32_t>(r0 + 32 * rt + 8 * q + 4 * h) * 4u,
+                                                                                              static_cast<uint32_t>(g) * a.xsum_stride * 4u, 0));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sum[rt][4 * q + e] = __builtin_fmaf(zc, xg[e], __builtin_fmaf(scale, part[rt][4 * q + e], sum[rt][4 * q + e]));
+        }
     }
-    if (col0 + 32 * ct + n < N)
+    if (!live) continue;
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int m = row0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3);
+        const int m = r0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3);
         if (m >= M) continue;
-        if (a.partials) a.partials[(static_cast<size_t>(blockIdx.y) * M + m) * N + col] = sum[e];
-        else a.y[static_cast<size_t>(m) * N + col] = f32_to_bf16_rne(sum[e]);
+        if (a.partials) a.partials[(static_cast<size_t>(blockIdx.y) * M + m) * N + col] = sum[rt][e];
+        else a.y[static_cast<size_t>(m) * N + col] = f32_to_bf16_rne(sum[rt][e]);
       }
   }
 }

@@ -119,3 +119,26 @@ def test_a_row_that_is_not_finite_touches_no_other(many_row_kernel, value):
     rest = torch.arange(140) != 3
     assert not torch.isfinite(got[3]).any()
     assert torch.equal(got[rest], want[rest].to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("g", [32, 64, 128])
+@pytest.mark.parametrize("slices", [1, 2])
+@pytest.mark.parametrize("tile", [0, 128])
+def test_groups_whose_scale_is_zero_add_nothing(many_row_kernel, g, slices, tile):
+    """the first group, the last, neighbours, every second one and all of a column, a negative zero, and scales at the ends of what
+    the running units carry; only a row's zero-point term is left where all scales are zero"""
+    m, n, k = 150, 528, 1152
+    _lib.set_option("int4_k_slices", slices)
+    _lib.set_option("int4_gemm_tile", tile)
+    codes, scale, zero, x = _case(m, n, k, g)
+    scale[0, 3] = scale[-1, 4] = scale[2:5, 5] = 0.0
+    scale[::2, 6] = scale[1::2, 7] = 0.0
+    scale[:, 8] = 0.0
+    scale[:, 300], zero[:, 300] = 0.0, 0.0
+    scale[1, 301] = -0.0
+    zero[:, 400:402] = 0.0
+    scale[:, 400], scale[:, 401] = 2.0**-100, 2.0**13
+    scale[1::2, 400] = 0.0
+    got, want = _run(codes, scale, zero, x, g)
+    assert torch.equal(got, want.to(torch.bfloat16))
+    assert not got[:, 300].any()
