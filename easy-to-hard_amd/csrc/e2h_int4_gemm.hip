@@ -18,6 +18,8 @@
 // sums leave float32's range in units of the scales although they may not by themselves (a zero of 2^100 beside a scale of 2^-20,
 // activations near the type's end): an infinity or NaN in an accumulator stays one to the end, where it is looked for, but for the
 // rows that have one in x.
+// Group size 32 keeps that second set of registers (64 rows per workgroup, so they fit): rescaling 64 sums every two steps costs the same
+// multiplications as adding 64 group sums, and the quotients and masks on top, 6 % of the kernel.  Every finite scale runs like that.
 //
 // The zero-point term is a matrix product over the groups.  It starts the accumulators: X and z - 24 s are each split into three
 // bfloat16 parts (exact: 3 x 8 bits), and eight of the nine products of parts (all but low x low, 2^-32) fill one lane's eight k values,
@@ -83,6 +85,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
   constexpr int kRows = 32 * kRT, kXStage = kRows * 128, kWStage = kCols * 64, kLdsW = 3 * kXStage, kLdsBytes = kLdsW + 2 * kWStage;
   static_assert(2 * kLdsBytes <= 160 * 1024, "two workgroups per CU");
   constexpr int NGRP = 128 / G, SPG = G / 16;  // groups per 128 k, MFMA steps per group
+  constexpr bool kGroupSums = G == 32;         // a group's products in registers of their own, scaled when it ends
   __shared__ __attribute__((aligned(1024))) uint8_t lds[kLdsBytes];
   const int M = a.M, N = a.N, K = a.K;
 
@@ -192,7 +195,9 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
 #pragma unroll
       for (int ct = 0; ct < kCT; ++ct) {
         const float scale = __builtin_bit_cast(float, za[i].szw[ct] << 16), zero = __builtin_bit_cast(float, za[i].szw[ct] & 0xFFFF0000u);
-        odd_scale |= !dead(g0 + 2 * i) && !(scale == 0.f || (__builtin_fabsf(scale) >= 0x1p-100f && __builtin_fabsf(scale) <= 0x1p13f));
+        const bool carried = kGroupSums ? __builtin_isfinite(scale) && __builtin_isfinite(zero)
+                                        : scale == 0.f || (__builtin_fabsf(scale) >= 0x1p-100f && __builtin_fabsf(scale) <= 0x1p13f);
+        odd_scale |= !dead(g0 + 2 * i) && !carried;
         float p[3];
         split3(__builtin_fmaf(-24.0f, scale, zero), p);
         const uint32_t hm = high_halves(p[1], p[0]);
@@ -244,13 +249,21 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) wq[ct][j] = *reinterpret_cast<const u32x4_t *>(lds + stage + w_lane[j] + ct * 2048);
     };
-    // of a column's group, so that each pair of codes is one and-or; both zero where the scale is zero: the group adds nothing
+    // registers, so that each pair of codes is one and-or; per column, both zero where a group's scale is zero: it adds nothing
     uint32_t mask[kCT], magic[kCT];
+    if constexpr (kGroupSums) {
+      asm volatile("s_mov_b32 %0, 0x00780078" : "=s"(mask[0]));
+      asm volatile("v_mov_b32 %0, 0x41804180" : "=v"(magic[0]));
+      mask[1] = mask[0];
+      magic[1] = magic[0];
+    }
     const auto enter = [&](int ct, uint32_t pair) {
-      const bool live = (pair & 0x7FFFu) != 0;
-      mask[ct] = live ? 0x00780078u : 0u;
-      magic[ct] = live ? 0x41804180u : 0u;
-      asm volatile("" : "+v"(mask[ct]), "+v"(magic[ct]));  // two registers, not a select behind every pair
+      if constexpr (!kGroupSums) {
+        const bool live = (pair & 0x7FFFu) != 0;
+        mask[ct] = live ? 0x00780078u : 0u;
+        magic[ct] = live ? 0x41804180u : 0u;
+        asm volatile("" : "+v"(mask[ct]), "+v"(magic[ct]));  // no select behind every pair
+      }
     };
     const uint32_t rot0 = (4 * h - 3) & 31, rot1 = (4 * h + 5) & 31;
     const auto convert = [&](bf16x8_t (&f)[kCT], int s8) {
@@ -266,7 +279,8 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
       }
     };
 
-    float unit[kCT] = {1.f, 1.f};  // what one step of the accumulators is worth
+    float unit[kCT] = {1.f, 1.f};  // what one step of the accumulators is worth (group sums: the group's scale)
+    [[maybe_unused]] f32x16_t part[kCT][kGroupSums ? kRT : 1];
     constexpr int kSc = NGRP < 2 ? NGRP : 2;  // pairs held ahead
     uint32_t sc[kCT][kSc];
 #pragma unroll
@@ -301,21 +315,33 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
         for (int ct = 0; ct < kCT; ++ct) {
           float r = 1.f;
           if (s8 % SPG == 0) {
-            const float scale = __builtin_bit_cast(float, sc[ct][s8 / SPG % kSc] << 16), s = scale != 0.f ? scale : unit[ct];
-            r = quotient(unit[ct], s);
+            const float scale = __builtin_bit_cast(float, sc[ct][s8 / SPG % kSc] << 16), s = kGroupSums || scale != 0.f ? scale : unit[ct];
+            if (!kGroupSums) r = quotient(unit[ct], s);
             unit[ct] = s;
             sc[ct][s8 / SPG % kSc] = load_sz(ct, blk * NGRP + s8 / SPG + kSc);
           }
 #pragma unroll
           for (int rt = 0; rt < kRT; ++rt) {
-            if (s8 % SPG == 0) {
-              __builtin_amdgcn_sched_barrier(0);  // one tile's rescaling under the previous tile's product
+            if constexpr (kGroupSums) {
+              part[ct][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[cur][rt], wf[cur][ct], s8 % SPG == 0 ? f32x16_t{} : part[ct][rt], 0, 0, 0);
+            } else {
+              if (s8 % SPG == 0) {
+                __builtin_amdgcn_sched_barrier(0);  // one tile's rescaling under the previous tile's product
 #pragma unroll
-              for (int e = 0; e < 16; ++e) acc[ct][rt][e] *= r;
+                for (int e = 0; e < 16; ++e) acc[ct][rt][e] *= r;
+              }
+              acc[ct][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[cur][rt], wf[cur][ct], acc[ct][rt], 0, 0, 0);
             }
-            acc[ct][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[cur][rt], wf[cur][ct], acc[ct][rt], 0, 0, 0);
           }
         }
+        if constexpr (kGroupSums)
+          if ((s8 + 1) % SPG == 0)
+#pragma unroll
+            for (int ct = 0; ct < kCT; ++ct)
+#pragma unroll
+              for (int rt = 0; rt < kRT; ++rt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[ct][rt][e] = __builtin_fmaf(unit[ct], part[ct][rt][e], acc[ct][rt][e]);
         if ((s8 + 1) % SPG == 0)
 #pragma unroll
           for (int ct = 0; ct < kCT; ++ct) enter(ct, sc[ct][(s8 + 1) % 8 / SPG % kSc]);
@@ -333,7 +359,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
     // Is a sum not finite in its column's units?  A row whose x is not finite stays out: nothing could make it so.
     bool over = false;
 #pragma unroll
-    for (int rt = 0; rt < kRT; ++rt) {
+    for (int rt = 0; rt < (kGroupSums ? 0 : kRT); ++rt) {
 #pragma unroll
       for (int ct = 0; ct < kCT; ++ct) {
         float t[2] = {0.f, 0.f};  // zero times an infinity or a NaN is a NaN
@@ -351,7 +377,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
     plain = __builtin_amdgcn_ballot_w64(over) != 0;
     if (!plain) {
 #pragma unroll
-      for (int ct = 0; ct < kCT; ++ct)
+      for (int ct = 0; ct < (kGroupSums ? 0 : kCT); ++ct)
 #pragma unroll
         for (int rt = 0; rt < kRT; ++rt)
 #pragma unroll
