@@ -8,6 +8,7 @@ float32.
 import ctypes
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from .ops import _need_gpu, _OnDevice, _stream
@@ -127,8 +128,20 @@ ACT_NONE, ACT_SQUARE_RELU, ACT_SOFTCAP = 0, 1, 2
 STREAMED_ROWS = 64
 
 
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
+def _watched(*tensors):
+    """True where something besides autograd's graph follows what happens to the tensors and would lose sight of it in a launch through
+    ctypes: subclasses, forward-mode derivatives, function transforms (vmap, jvp, ..), dispatch modes, torch.jit traces.  (The two last
+    do not look through a compiler's trace: that records the registered op.)"""
+    if any(type(t) not in _PLAIN_TYPES for t in tensors) or forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active():
+        return True
+    return not torch.compiler.is_compiling() and (torch._C._len_torch_dispatch_stack() > 0 or torch._C._get_tracing_state() is not None)
+
+
 def linear_streams(x, weight):
-    """True where `linear` takes x [.., k] and weight [n, k]: bfloat16 on the GPU, up to 64 rows, no gradients."""
+    """True where `linear` takes x [.., k] and weight [n, k]: bfloat16 on the GPU, up to 64 rows, no gradients, nobody watching."""
     k = weight.shape[1]
     if not 0 < x.numel() <= STREAMED_ROWS * k:
         return False
@@ -136,7 +149,7 @@ def linear_streams(x, weight):
         return False
     if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
         return False
-    return k % 8 == 0 and k < 1 << 22 and not torch.is_autocast_enabled()
+    return k % 8 == 0 and k < 1 << 22 and not torch.is_autocast_enabled() and not _watched(x, weight)
 
 
 def linear(x, weight, act=ACT_NONE, cap=0.0):

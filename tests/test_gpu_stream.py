@@ -86,3 +86,39 @@ def test_module_routes_and_refusals():
     assert (lin.float()(x.float()) - ref).abs().max() <= 1e-4 * ref.abs().max()
     with pytest.raises(RuntimeError):
         seq_ops.linear(torch.zeros((65, 256), dtype=torch.bfloat16, device=DEV), torch.zeros((96, 256), dtype=torch.bfloat16, device=DEV))
+
+
+def test_module_shows_transforms_and_traces_what_nn_linear_shows():
+    """forward-mode derivatives, function transforms, dispatch modes, traces and subclasses see the product: none of them may end in a
+    launch that they know nothing of"""
+    from torch.autograd import forward_ad
+    from torch.utils.flop_counter import FlopCounterMode
+
+    gen = torch.Generator().manual_seed(6)
+    lin = DecodeLinear(256, 96, bias=False).to(DEV, torch.bfloat16).requires_grad_(False)
+    x, t = (torch.randn((5, 256), generator=gen).to(torch.bfloat16).to(DEV) for _ in range(2))
+    assert seq_ops.linear_streams(x, lin.weight)
+    want = torch.nn.functional.linear(t, lin.weight)
+    with forward_ad.dual_level():
+        assert torch.equal(forward_ad.unpack_dual(lin(forward_ad.make_dual(x, t))).tangent, want)
+        weight = torch.randn((96, 256), generator=gen).to(torch.bfloat16).to(DEV)
+        dual = torch.func.functional_call(lin, {"weight": forward_ad.make_dual(lin.weight, weight)}, (x,))
+        assert torch.equal(forward_ad.unpack_dual(dual).tangent, torch.nn.functional.linear(x, weight))
+    assert torch.equal(torch.func.jvp(lin, (x,), (t,))[1], want)
+    seen = []
+
+    def route(row):
+        seen.append(seq_ops.linear_streams(row, lin.weight))
+        return row
+
+    torch.func.vmap(route)(x)
+    assert seen == [False]
+    with FlopCounterMode(display=False) as flops:
+        lin(x)
+    assert flops.get_total_flops() == 2 * 5 * 96 * 256
+    assert torch.equal(torch.jit.trace(lin, x, check_trace=False)(t), want)
+
+    class Named(torch.Tensor):
+        pass
+
+    assert type(lin(x.as_subclass(Named))) is Named
