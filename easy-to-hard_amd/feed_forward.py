@@ -7,7 +7,7 @@ import torch.nn as nn
 from torch import Tensor
 
 from . import seq_ops
-from .linear import DecodeLinear, fusable
+from .linear import DecodeLinear, fusable, unwatched
 
 
 class SquaredReluFF(nn.Module):
@@ -43,11 +43,16 @@ class ExpertMixture(nn.Module):
 
     def forward(self, h: Tensor) -> Tuple[Optional[Tensor], Tensor, Tensor]:
         chosen, weights = seq_ops.route(h, self.router, self.router_bias, self.top)
-        if self.shared is not None and h.shape[0] <= self.STEP_ROWS and all(type(m) in (nn.Linear, DecodeLinear) for m in (self.shared.up, self.shared.down)):
+        if self.shared is not None and h.shape[0] <= self.STEP_ROWS and self._shared_joins():
             out, shared = seq_ops.experts(h, chosen, self.up, self.down, self.shared.up.weight, self.shared.down.weight)
             return shared, out, weights
         out, _ = seq_ops.experts(h, chosen, self.up, self.down)
         return (None if self.shared is None else self.shared(h)), out, weights
+
+    def _shared_joins(self) -> bool:
+        """the shared expert is the modules built here, and nobody watches their calls"""
+        linears = (self.shared.up, self.shared.down)
+        return all(type(m) in (nn.Linear, DecodeLinear) for m in linears) and unwatched(self.shared) and all(unwatched(m) for m in linears)
 
     def from_checkpoint(self, get, prefix: str, linear_dtype) -> dict:
         n = self.router.shape[0]
