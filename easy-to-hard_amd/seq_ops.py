@@ -153,23 +153,24 @@ def linear_streams(x, weight):
 
 
 def linear(x, weight, act=ACT_NONE, cap=0.0):
-    """act(x weight^T) of a decode batch, see e2h_seq_linear; operands that are not 16-byte aligned or not contiguous are copied."""
+    """act(x weight^T) of a decode batch, see e2h_seq_linear; x is copied if it is not 16-byte aligned or not contiguous.  A weight that
+    is not takes the library's product, which reads it where it lies."""
     _need_gpu(x, weight)
     n, k = weight.shape
     rows = x.numel() // k
-    x2d = x if x.is_contiguous() else x.contiguous()  # the kernel reads it as [rows, k]
-    if not weight.is_contiguous():
-        weight = weight.contiguous()
-    if x2d.data_ptr() % 16:
-        x2d = x2d.clone()
-    if weight.data_ptr() % 16:
-        weight = weight.clone()
-    y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
     lib = _lib_for(x)
     need = lib.e2h_seq_linear_scratch_bytes(rows, n, k)
+    if need < 0:
+        _lib.check_seq(need, "e2h_seq_linear")
+    if not weight.is_contiguous() or weight.data_ptr() % 16:
+        y = torch.nn.functional.linear(x, weight)
+        return square_relu_(y) if act == ACT_SQUARE_RELU else softcap_(y, cap) if act == ACT_SOFTCAP else y
+    x2d = x if x.is_contiguous() else x.contiguous()  # the kernel reads it as [rows, k]
+    if x2d.data_ptr() % 16:
+        x2d = x2d.clone()
+    y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
     scratch = torch.empty((need,), dtype=torch.uint8, device=x.device) if need > 0 else None
-    _lib.check_seq(lib.e2h_seq_linear(_p(x2d), _p(weight), _p(y), rows, n, k, act, cap, _p(scratch), max(need, 0), _stream(x)),
-                   "e2h_seq_linear")
+    _lib.check_seq(lib.e2h_seq_linear(_p(x2d), _p(weight), _p(y), rows, n, k, act, cap, _p(scratch), need, _stream(x)), "e2h_seq_linear")
     return y
 
 

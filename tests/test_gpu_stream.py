@@ -122,3 +122,23 @@ def test_module_shows_transforms_and_traces_what_nn_linear_shows():
         pass
 
     assert type(lin(x.as_subclass(Named))) is Named
+
+
+@pytest.mark.parametrize("act,cap", [(seq_ops.ACT_NONE, 0.0), (seq_ops.ACT_SQUARE_RELU, 0.0), (seq_ops.ACT_SOFTCAP, 30.0)])
+def test_a_weight_that_the_kernel_does_not_read_is_not_copied(act, cap):
+    """rows cut out of wider ones and a weight off 16 bytes, as views of a checkpoint's buffer are: integers, so the result is exact"""
+    n, k = 4096, 4096
+    x = ints((5, k), 1, torch.bfloat16, 1)
+    wide = ints((n, k + 8), 2, torch.bfloat16, 1)
+    shifted = torch.empty((n * k + 1,), dtype=torch.bfloat16, device=DEV)[1:].view(n, k)
+    shifted.copy_(wide[:, :k])
+    aligned = shifted.clone()
+    want = seq_ops.linear(x, aligned, act, cap)
+    for w in (wide[:, :k], shifted, aligned.t().contiguous().t()):
+        seq_ops.linear(x, w, act, cap)  # the library's own workspace
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        got = seq_ops.linear(x, w, act, cap)
+        assert torch.cuda.max_memory_allocated() - before < n * k
+        assert torch.equal(got, want)
