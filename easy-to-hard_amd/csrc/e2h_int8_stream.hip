@@ -318,7 +318,7 @@ int partial_slices8_for(int64_t m, int64_t n, int64_t k) {
   if (m < 1 || m > 64 || n < 8 || (n % 8) != 0 || k < 128 || (k % 128) != 0 || n > INT32_MAX || k > INT32_MAX || n * k >= (int64_t{1} << 32))
     return E2H_ERR_BAD_SHAPE;
   if (m > 32 && (n + 63) / 64 >= kCUs8) return E2H_ERR_BAD_SHAPE;
-  return 2;
+  return stream::takes(m, n, k, 1) ? 2 : E2H_ERR_BAD_SHAPE;
 }
 
 }  // namespace
@@ -396,7 +396,6 @@ extern "C" int e2h_int8_mm_partials(const uint16_t *x, const int8_t *q, float *p
   if (want < 0) return want;
   if (slices != want) return E2H_ERR_BAD_SHAPE;
   if (!aligned16(x) || !aligned16(q) || (reinterpret_cast<uintptr_t>(partials) & 3u)) return E2H_ERR_MISALIGNED;
-  if (!stream::takes(m, n, k, 1)) return E2H_ERR_BAD_SHAPE;
   return stream::run<stream::Int8Weights, Partial8>({x, q, q, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k)}, {partials},
                                                     static_cast<hipStream_t>(stream));
 }

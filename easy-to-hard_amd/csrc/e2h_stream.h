@@ -21,6 +21,7 @@
 namespace e2h {
 namespace stream {
 
+constexpr int64_t kMaxBytes = int64_t{1} << 31;  // of a buffer: offsets of 2^31 are what is sent out of range
 constexpr int kWaves = 8;
 constexpr int kMaxUnits = 16;  // (column tile, row tile) pairs of a workgroup: 8 KB of LDS each when the waves meet
 constexpr int kUnitBytes = 2048, kRing = 8;  // per wave: 14 KB on their way while 2 KB are in use (18 KB measured the same)
@@ -247,6 +248,7 @@ inline int pick_tiles(int M, int N, int K, int slices = 1) {
   for (int t : {1, 2, 3, 4, 6, 8}) {
     if (t > cap || (GATE && t % 2)) continue;
     const int tc = GATE ? t / 2 : t;
+    if (int64_t{16} * tc * K * W::kBytes >= kMaxBytes) continue;
     const int rounds = ((tiles + tc - 1) / tc * slices + 255) / 256;
     const double cost = rounds * (16.0 * t * W::kBytes + 0.25 * 2 * M + 16384.0 / K);
     if (!best || cost < best_cost) best = t, best_cost = cost;
@@ -279,9 +281,11 @@ int launch_rows(const Args &a, const typename Epi::Args &ea, int t, int slices, 
   }
 }
 
-// rows in pieces of 16 bytes, a workgroup's weights and x below 2^31 bytes; x and w 16-byte aligned
+// rows in pieces of 16 bytes, whole row tiles of x and a tile of weights below 2^31 bytes; x and w 16-byte aligned
 inline bool takes(int64_t M, int64_t N, int64_t K, int bytes) {
-  return M >= 1 && M <= 64 && N >= 1 && N < (int64_t{1} << 31) - 128 && K >= 1 && K * bytes % 16 == 0 && 128 * K * 2 < (int64_t{1} << 31);
+  const int64_t x_rows = M <= 16 ? 16 : M <= 32 ? 32 : 64;
+  return M >= 1 && M <= 64 && N >= 1 && N < (int64_t{1} << 31) - 128 && K >= 1 && K < (int64_t{1} << 30) && K * bytes % 16 == 0 &&
+         x_rows * K * 2 < kMaxBytes && 16 * K * bytes < kMaxBytes;
 }
 
 // slices > 1: workgroups split K too, and the epilogue stores its slice's sums (blockIdx.y)

@@ -142,3 +142,22 @@ def test_a_weight_that_the_kernel_does_not_read_is_not_copied(act, cap):
         got = seq_ops.linear(x, w, act, cap)
         assert torch.cuda.max_memory_allocated() - before < n * k
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("m,k", [(1, 1 << 23), (17, (1 << 23) + 128), (33, 1 << 23), (3, 1 << 25)])
+def test_int8_fused_launches_take_very_long_rows(m, k):
+    """rows of 2^23 values and more, where a workgroup's tiles have to stay below 2^31 bytes: some 64 values per row of x are not zero, so
+    the sums of integers are exact; gate, K halves and the plain form"""
+    n = 48
+    gen = torch.Generator().manual_seed(k + m)
+    x = torch.zeros((m, k), dtype=torch.bfloat16, device=DEV)
+    at = torch.unique(torch.cat([torch.randint(0, k, (62,), generator=gen), torch.tensor([0, k - 1])])).to(DEV)
+    x[:, at] = ints((m, len(at)), 3, torch.bfloat16)
+    w, w3 = (torch.randint(-4, 5, (n, k), dtype=torch.int8, device=DEV, generator=torch.Generator(DEV).manual_seed(s)) for s in (1, 2))
+    scales = torch.full((n,), 0.5, dtype=torch.bfloat16, device=DEV)
+    want, want3 = (exact(x[:, at], q[:, at]) for q in (w, w3))
+    lin, up = ((t.to(torch.bfloat16).float() * 0.5).to(torch.bfloat16) for t in (want, want3))
+    assert torch.equal(ops.int8_mm_direct(x, w, scales), lin)
+    assert torch.equal(ops.int8_mm_silu_gate(x, w, scales, w3, scales), ops.silu_mul(lin, up))
+    sums = ops.int8_mm_partials(x, w, scales, ops._lib.load().e2h_int8_mm_partial_slices(m, n, k)).partials
+    assert torch.equal(sums.double().sum(0), want)
