@@ -494,13 +494,17 @@ __global__ __launch_bounds__(256) void add_slices_kernel(const float *__restrict
 Int4GemmShape int4_gemm_shape(int M, int N, int K, int groupsize, int64_t scratch_bytes) {
   const int KT = K >> 7;
   const int64_t fit = scratch_bytes / (static_cast<int64_t>(M) * N * 4);
-  const int want_rows = options().int4_gemm_tile, want_s = options().int4_k_slices;
+  const int want_rows = options().int4_gemm_tile, most = options().int4_k_slices > 0 ? options().int4_k_slices : kMostSlices;
+  const auto possible = [&](int s) { return s <= kMostSlices && s <= KT && s <= most && (s == 1 || s <= fit); };
+  int forced = 0;  // the option's count, or the largest one below it that there is
+  if (options().int4_k_slices > 0)
+    for (int s = 1; possible(s); s *= 2) forced = s;
   Int4GemmShape best = {64, 1, -1.0};
   for (int rows = 64; rows <= (groupsize == 32 ? 64 : 128); rows *= 2) {  // group size 32 at 128 rows does not fit the registers
     if (want_rows == 128 && groupsize != 32 && rows != 128) continue;
     const int64_t per_xcd = static_cast<int64_t>((M + rows - 1) / rows) * (((N + kCols - 1) / kCols + 7) / 8);  // one slice; 32 CUs each
-    for (int s = 1; s <= kMostSlices && s <= KT && (s == 1 || s <= fit); s *= 2) {
-      if (want_s > 0 && s != want_s && want_s <= fit && want_s <= kMostSlices) continue;
+    for (int s = 1; possible(s); s *= 2) {
+      if (forced && s != forced) continue;
       const int64_t per_cu = (per_xcd * s + 31) / 32;
       const double one = rows == 64 ? 1.2 : 1.85, two = rows == 64 ? 1.95 : 3.3;
       const double cost = (static_cast<double>(per_cu / 2) * two + (per_cu & 1 ? one : 0)) * KT / s + 3 +

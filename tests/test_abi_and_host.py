@@ -320,3 +320,29 @@ def test_reward_model_loader_builds_the_two_row_head_and_rejects_quantized_files
     assert tuple(first.shape) == (2, 8) and torch.equal(first, big.output.weight) and float(first.abs().max()) > 0
     with pytest.raises(ValueError):
         apply_reward_modeling_head(big, init_scheme="other")
+
+
+@pytest.mark.parametrize("k", [128, 384, 1024, 4096])
+@pytest.mark.parametrize("want", [1, 2, 3, 5, 6, 7, 8, 16])
+@pytest.mark.parametrize("tile,groupsize", [(0, 64), (128, 64), (128, 128), (0, 32)])
+def test_a_forced_slice_count_leaves_a_real_geometry(k, want, tile, groupsize):
+    """the many-row int4 matmul picks rows per workgroup and K slices by expected time; a forced count that is no power of two, or more than
+    K or the scratch memory allow, becomes the next possible one, with its time, and a forced tile stays"""
+
+    class Shape(ctypes.Structure):
+        _fields_ = [("rows", ctypes.c_int), ("slices", ctypes.c_int), ("us", ctypes.c_double)]
+
+    lib = _lib.load()
+    shape = lib["_ZN3e2h15int4_gemm_shapeEiiiil"]  # e2h::int4_gemm_shape(int, int, int, int, long)
+    shape.restype, shape.argtypes = Shape, [ctypes.c_int] * 4 + [ctypes.c_int64]
+    m, n = 130, 512
+    for fit in (0, 2, 64):
+        try:
+            assert lib.e2h_set_option(b"int4_k_slices", want) == 0 and lib.e2h_set_option(b"int4_gemm_tile", tile) == 0
+            got = shape(m, n, k, groupsize, fit * m * n * 4)
+        finally:
+            lib.e2h_set_option(b"int4_k_slices", 0)
+            lib.e2h_set_option(b"int4_gemm_tile", 0)
+        most = min(want, 8, k // 128, max(fit, 1))
+        assert got.slices == max(s for s in (1, 2, 4, 8) if s <= most)
+        assert got.us > 0 and got.rows == (128 if tile == 128 else 64)
