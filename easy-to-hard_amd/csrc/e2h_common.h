@@ -36,7 +36,7 @@ __host__ __device__ inline float bf16_round(float f) { return bf16_to_f32(f32_to
 
 struct Options {
   int int4_rows_per_wave;  // 0 = heuristic, else 16/32/64
-  int int4_k_slices;       // 0 = heuristic, else 1..16 workgroups along K
+  int int4_k_slices;       // 0 = heuristic, else 1..16 workgroups along K (many rows: the largest power of two up to that which is possible)
   int int4_k_groups;       // 0 = heuristic, else 1/2/4 k-groups inside a workgroup
   int int4_col_waves;      // 0 = heuristic, else 1..4 column waves per k-group
   int int8_rows_per_wave;  // 0 = heuristic, else 16/32/64 (calls of more than 64 rows and the generic kernel)

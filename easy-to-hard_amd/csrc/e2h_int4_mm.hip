@@ -771,9 +771,8 @@ int int4_mm_impl(const uint16_t *x, const int32_t *packed, const uint16_t *scale
   int64_t max_rows = rows_by_bytes < rows_by_grid ? rows_by_bytes : rows_by_grid;
   max_rows -= max_rows % (16 * mt);
   if (max_rows < 16 * mt) return E2H_ERR_BAD_SHAPE;
-  // Many rows run on the 128-row kernel (exact products, scale and zero applied to float32 group sums: the arithmetic of
-  // every other int4 kernel here, so a row's result does not depend on how many rows share the call).  The 256 x 256
-  // kernel that dequantizes to bfloat16 on the way into the matrix cores (the reference kernel's arithmetic, 15-20 %
+  // Many rows run on the 32x32-tile kernel (exact products, float32 sums, scales and zero points, one rounding, as in every other
+  // int4 kernel here; only the order of the sums differs between them).  The 256 x 256 kernel that dequantizes to bfloat16 on the way into the matrix cores (the reference kernel's arithmetic, 15-20 %
   // faster at thousands of rows) is taken only on request, option "int4_gemm_tile" = 256, and then for every slice of
   // the call alike.
   const auto takes_256_row_kernel = [&](int64_t) {

@@ -40,10 +40,11 @@ int e2h_abi_version(void);
 const char *e2h_status_string(int status);
 
 /* Tuning knobs for experiments: launch-geometry overrides such as "int4_rows_per_wave", "int4_k_slices", "int4_k_groups",
- * "int4_col_waves", "int8_rows_per_wave", "int8_k_groups", "int8_k_slices", "int8_force_generic", "row_tiles", "int4_no_xsum",
- * "int4_no_gemm32", "int4_gemm32_min_rows", "int4_gemm_tile", "int8_gemm_tile", "int8_gemm_waves", "int8_gemm_wave_cols", "attention_waves",
- * "attention_no_mfma", "staged_tiles", "staged_slices"; "staged_no_rows64" is taken and has no effect;
- * value 0 restores the built-in heuristic.  Not thread safe; set before launching. */
+ * "int4_col_waves", "int8_rows_per_wave", "int8_force_generic", "row_tiles" (int4), "int4_no_xsum", "int4_no_gemm32",
+ * "int4_gemm32_min_rows", "int4_gemm_tile", "int8_gemm_tile", "int8_gemm_waves", "int8_gemm_wave_cols", "attention_waves",
+ * "attention_no_mfma", "staged_tiles", "staged_slices"; value 0 restores the built-in heuristic.  "int8_k_groups",
+ * "int8_k_slices" and "staged_no_rows64" are taken, with the range checks they had, and have no effect.
+ * Not thread safe; set before launching. */
 int e2h_set_option(const char *name, int value);
 
 /* ------------------------------------------------------------------------------------------------
@@ -65,8 +66,9 @@ int e2h_int8_quantize_per_channel(const void *w, int w_is_bf16, int8_t *q, float
 /* WeightOnlyInt8Linear.forward, reference :428-429:  y = F.linear(x, weight.to(bf16)) * scales.
  *   x [m, k] bf16, q [n, k] int8, scales [n] bf16, y [m, n] bf16.  float32 accumulation; the result
  *   is rounded to bfloat16 before and after the multiplication by the scale, as in the reference.
- * Any m >= 1, n >= 1, k >= 1 (k % 128 == 0 with 16-byte aligned x and q takes the streaming kernel).
- * workspace / workspace_bytes: optional scratch as for e2h_int4_mm (NULL / 0 allowed). */
+ * Any m >= 1, n >= 1, k >= 1.  With 16-byte aligned x and q the streaming kernels run: up to 64 rows for k % 16 == 0, above
+ * for k % 128 == 0 and n * k < 2^32; anything else takes the generic one.
+ * workspace / workspace_bytes: NULL / 0 or 16-byte aligned; no kernel uses it. */
 int e2h_int8_mm(const uint16_t *x, const int8_t *q, const uint16_t *scales, uint16_t *y, int64_t m,
                 int64_t n, int64_t k, void *workspace, int64_t workspace_bytes, void *stream);
 
@@ -126,11 +128,13 @@ int e2h_int4_dequantize_codes(const int32_t *codes, const uint16_t *scales, cons
  *              recommended size) that lets small problems split K across workgroups.  It must be zero
  *              when first used and is left zeroed where it matters by every launch; launches that share
  *              it must be ordered on one stream.  NULL / 0 selects the single-slice kernels.
- * Every kernel behind this entry point forms exact bf16 x code products and applies scale and zero per group in
- * float32, so a row's result does not depend on how many rows share the call.  Only with
- * e2h_set_option("int4_gemm_tile", 256) calls of more than 64 rows (k % 256 == 0, g <= 128, ikt 8) run a kernel that
- * rounds every weight to bfloat16 first (the arithmetic of the kernel the reference calls; 15-20 % faster at thousands
- * of rows): results then differ from the default by that rounding, for every row of such a call alike. */
+ * Every kernel behind this entry point forms exact bf16 x code products, keeps all sums, scales and zero-point terms in
+ * float32 and rounds once.  The order of the sums follows the launch geometry, which depends on m, n, k, the workspace and
+ * the options: the same call gives the same bits, but a row may differ by float32 rounding before the one to bfloat16 when
+ * another number of rows shares the call, or another workspace.  Only with e2h_set_option("int4_gemm_tile", 256) calls of
+ * more than 64 rows (k % 256 == 0, g <= 128, ikt 8) run a kernel that rounds every weight to bfloat16 first (the arithmetic
+ * of the kernel the reference calls; 15-20 % faster at thousands of rows): results then differ from the default by that
+ * rounding, for every row of such a call alike. */
 int e2h_int4_mm(const uint16_t *x, const int32_t *packed, const uint16_t *scales_and_zeros, uint16_t *y,
                 int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles, void *workspace,
                 int64_t workspace_bytes, void *stream);
@@ -180,7 +184,8 @@ int e2h_int4_mm_rope_kv(const uint16_t *x, const int32_t *packed, const uint16_t
  * models/quantize.py:405-429, in FeedForward.forward models/model.py:343-344 and Attention.forward :283-296).
  * Each linear's output is formed with the reference's two roundings, bf16(bf16(x @ q^T) * scales), before the SiLU-gate
  * or the rotation is applied, so the results equal the unfused sequence of calls bit for bit.
- *   q_* int8 [n, k] row-major, scales_* bf16 [n]; 1 <= m (batch) <= 64, k % 128 == 0, 16-byte aligned x and q rows;
+ *   q_* int8 [n, k] row-major, scales_* bf16 [n]; 1 <= m (batch) <= 64, k % 128 == 0, 16-byte aligned x and q rows; n * k < 2^32,
+ *   k < 2^26 for up to 16 rows, 2^25 for up to 32, 2^24 for up to 64 (x below 2 GiB);
  *   the other arguments as in e2h_int4_mm_silu_gate / e2h_int4_mm_rope_kv. */
 int e2h_int8_mm_silu_gate(const uint16_t *x, const int8_t *q_gate, const uint16_t *scales_gate, const int8_t *q_up,
                           const uint16_t *scales_up, uint16_t *y, int64_t m, int64_t n, int64_t k, void *stream);

@@ -40,6 +40,7 @@ def _run(codes, scale, zero, x, g):
     return ops.int4_mm(x, packed, g, sz), x.double() @ w.t()
 
 
+# slices: at most, as many as there are blocks of 128 k; tile 128: 128 rows per workgroup but at group size 32
 @pytest.mark.parametrize("g", [32, 64, 128])
 @pytest.mark.parametrize("slices", [1, 2, 8])
 @pytest.mark.parametrize("tile", [0, 128])
@@ -142,3 +143,28 @@ def test_groups_whose_scale_is_zero_add_nothing(many_row_kernel, g, slices, tile
     got, want = _run(codes, scale, zero, x, g)
     assert torch.equal(got, want.to(torch.bfloat16))
     assert not got[:, 300].any()
+
+
+@pytest.mark.parametrize("g", [32, 64, 128])
+@pytest.mark.parametrize("n,k", [(1032, 1024), (4096, 1024), (4096, 4096)])
+def test_a_row_differs_by_float32_rounding_at_most_between_row_counts(g, n, k):
+    """The kernels for 1 .. 64 rows, 65 and more, many, and every choice of K slices add the same exact products in another order.  A sum
+    of N additions is within N 2^-24 A of the exact one, A the sum of the magnitudes added, and rounding to bfloat16 adds 2^-8 of the
+    value between two results.  A chain has at most K / 16 products' steps, two additions per group and 16 for the parts that
+    meet; the magnitudes are those of 128 + q <= 143 and of z - 136 s.  The same call gives the same bits."""
+    m = 1030
+    gen = torch.Generator().manual_seed(n + k + g)
+    codes = torch.randint(0, 16, (n, k), generator=gen, dtype=torch.int32)
+    scale = (torch.rand((k // g, n), generator=gen) * 0.02 + 0.01).to(torch.bfloat16)
+    zero = (torch.randn((k // g, n), generator=gen) * 0.02).to(torch.bfloat16)
+    x = torch.randn((m, k), generator=gen).to(torch.bfloat16).to(DEV)
+    packed = torch.from_numpy(qo.int4_tile_pack(codes.numpy(), 8)).to(DEV)
+    sz = torch.stack([scale, zero], dim=-1).contiguous().to(DEV)
+    full = ops.int4_mm(x, packed, g, sz)
+    size = (143 * scale + 136 * scale + zero.abs()).double().to(DEV)  # [K / g, N]
+    magnitude = x.double().abs().view(m, k // g, g).sum(-1) @ size
+    bound = 2 * (k / 16 + 2 * k / g + 16) * 2.0**-24 * magnitude + 2.0**-8 * full.double().abs()
+    for rows in (1, 16, 17, 33, 64, 65, 128, 129, 300, 512, 640):
+        part = ops.int4_mm(x[:rows], packed, g, sz)
+        assert torch.equal(part, ops.int4_mm(x[:rows], packed, g, sz))
+        assert ((part.double() - full[:rows].double()).abs() <= bound[:rows]).all()
