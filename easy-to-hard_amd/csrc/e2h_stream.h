@@ -2,8 +2,9 @@
 // decode-batch matmul of int8 linears (e2h_int8_stream.hip) and of bfloat16 ones (e2h_seq_linear.hip).
 //
 // A workgroup is eight waves that split K and all work on the same T tiles of 16 weight rows, so that a CU streams 16 T rows and
-// reads x once.  The split of K depends on K alone, so a row's result depends neither on the rows beside it nor on N, and every
-// epilogue sees the same sums.  The waves meet once, at the end: wave w adds and finishes the (column tile, row tile) units w,
+// reads x once.  The split of K over the waves of a workgroup depends on K alone, so with one slice a row's result depends neither on the rows
+// beside it nor on N, and every epilogue sees the same sums.  (Slices over several workgroups, which e2h_seq_linear takes for some shapes,
+// sum in another order: there a row's result changes by float32 rounding with the choice.)  The waves meet once, at the end: wave w adds and finishes the (column tile, row tile) units w,
 // w + 8, .. in k order.
 //
 // Everything a wave needs passes as units of 2 KB -- 16 rows of x or of a weight tile, 128 bytes each -- through a ring of its own in
@@ -64,8 +65,7 @@ __device__ __forceinline__ void wait_loads(int n) {
   switch (n) {
 #define E2H_WAIT(N) \
   case N: asm volatile("s_waitcnt vmcnt(" #N ")" ::: "memory"); break;
-    E2H_WAIT(7) E2H_WAIT(8) E2H_WAIT(9) E2H_WAIT(10) E2H_WAIT(11) E2H_WAIT(12) E2H_WAIT(13) E2H_WAIT(14) E2H_WAIT(15) E2H_WAIT(16) E2H_WAIT(17)
-    E2H_WAIT(18)
+    E2H_WAIT(7) E2H_WAIT(8) E2H_WAIT(9) E2H_WAIT(10) E2H_WAIT(11) E2H_WAIT(12) E2H_WAIT(13) E2H_WAIT(14)
 #undef E2H_WAIT
     default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }

@@ -161,3 +161,20 @@ def test_int8_fused_launches_take_very_long_rows(m, k):
     assert torch.equal(ops.int8_mm_silu_gate(x, w, scales, w3, scales), ops.silu_mul(lin, up))
     sums = ops.int8_mm_partials(x, w, scales, ops._lib.load().e2h_int8_mm_partial_slices(m, n, k)).partials
     assert torch.equal(sums.double().sum(0), want)
+
+
+def test_sliced_launches_change_a_row_by_float32_rounding_at_most():
+    """From 17 rows on K is cut over four workgroups (N <= 4096, K >= 8192): among those a row depends on no other row and no other column;
+    beside one workgroup's sum the order differs.  Either is within N 2^-24 A of the exact sum (N <= K / 32 + 12 additions in a chain, A
+    the sum of the magnitudes), and rounding to bfloat16 adds 2^-8 of the value."""
+    gen = torch.Generator().manual_seed(8)
+    k = 8192
+    x, w = (torch.randn(s, generator=gen).to(torch.bfloat16).to(DEV) for s in ((64, k), (4112, k)))
+    narrow = w[:4096]
+    full = seq_ops.linear(x, narrow)
+    for rows in (17, 32, 33):
+        assert torch.equal(seq_ops.linear(x[:rows], narrow), full[:rows])
+    assert torch.equal(seq_ops.linear(x, w[:700]), full[:, :700])
+    bound = 2 * (k / 32 + 12) * 2.0**-24 * (x.double().abs() @ narrow.double().abs().t()) + 2.0**-8 * full.double().abs()
+    assert ((seq_ops.linear(x[:16], narrow).double() - full[:16].double()).abs() <= bound[:16]).all()
+    assert ((seq_ops.linear(x, w)[:, :4096].double() - full.double()).abs() <= bound).all()
