@@ -110,7 +110,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
   constexpr int kUnitsPerWave = (kUnits + kWaves - 1) / kWaves;
   // units of a chunk in the order of their use: pairs, operands, words
   constexpr int kSz = GATE ? 2 : (T * NGRP + 15) / 16, kHead = kSz + 4 * MT, UC = kHead + T;
-  constexpr int kRing = UC < 4 ? 8 : 16;         // units of 1 KB per wave
+  constexpr int kRing = 16;                      // units of 1 KB per wave
   constexpr int kAhead = (kRing + UC - 1) / UC;  // chunks that the ring reaches into, at most
   constexpr int kLate = kAhead * UC - kRing;     // units of the last kAhead chunks that are issued while those run
   static_assert(kSz + MT < kRing && TC * NGRP <= 16 * (GATE ? 1 : kSz), "ring");
@@ -374,8 +374,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
     run(std::integral_constant<int, 0>{});
     if constexpr (kAhead > 1) run(std::integral_constant<int, 1>{});
     if constexpr (kAhead > 2) run(std::integral_constant<int, 2>{});
-    if constexpr (kAhead > 3) run(std::integral_constant<int, 3>{});
-    static_assert(kAhead <= 4, "ring");
+    static_assert(kAhead <= 3, "ring");
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll 1

@@ -317,7 +317,7 @@ constexpr int kCUs8 = 256;
 int partial_slices8_for(int64_t m, int64_t n, int64_t k) {
   if (m < 1 || m > 64 || n < 8 || (n % 8) != 0 || k < 128 || (k % 128) != 0 || n > INT32_MAX || k > INT32_MAX || n * k >= (int64_t{1} << 32))
     return E2H_ERR_BAD_SHAPE;
-  if (m > 32 && (n + 63) / 64 >= kCUs8) return E2H_ERR_BAD_SHAPE;
+  if (m > 32 && (n + 63) / 64 >= kCUs8) return E2H_ERR_BAD_SHAPE;  // never offered: wider than any model's residual stream
   return stream::takes(m, n, k, 1) ? 2 : E2H_ERR_BAD_SHAPE;
 }
 

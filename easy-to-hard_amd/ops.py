@@ -129,7 +129,7 @@ def _int8_mm_impl(x, q, scales):
     y = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
     if m == 0:
         return y
-    ws = _workspace(x.device)
+    ws = _workspace(x.device)  # no int8 kernel uses it, but a first eager call of either kind is what a later capture of int4 calls relies on
     rc = _lib_for(x).e2h_int8_mm(_ptr(x), _ptr(q), _ptr(scales), _ptr(y), m, n, k, _ptr(ws), ws.numel(), _stream(x))
     _lib.check(rc, "e2h_int8_mm")
     return y
