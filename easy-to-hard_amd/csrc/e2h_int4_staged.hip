@@ -118,9 +118,8 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
   constexpr int kParts = kTwoSteps ? kWaves / 2 : kWaves;
   constexpr int kRedBytes = kParts * T * MT * 1024, kRingBytes = kWaves * kRing * 1024;
 
-  // One object for everything: beside a second one the compiler tells loads into LDS from its reads by object and waits for all of them
-  // before each (head 32000 x 4096 with the candidates in an array of their own: 27.6 us at 32 rows, so 20.1).
   __shared__ __attribute__((aligned(1024))) uint8_t lds[kRedBytes > kRingBytes ? kRedBytes : kRingBytes];
+  __shared__ unsigned long long unit_best[EPI == kStArgmax ? kUnits : 1][16];  // arg-max: per unit and row of its tile
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -406,7 +405,6 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
     put(kg);
   }
   lds_barrier();
-  unsigned long long row_best[EPI == kStArgmax ? kUnitsPerWave : 1][4];  // arg-max: best candidate of a unit's rows 4 b + q
 #pragma unroll
   for (int u = 0; u < kUnitsPerWave; ++u) {
     const int unit = kg + u * kWaves;
@@ -487,7 +485,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
           const unsigned long long other = __shfl_xor(best, off);
           best = other > best ? other : best;
         }
-        row_best[u][q] = best;
+        if (c == 0) unit_best[unit][4 * b + q] = best;
       }
     } else {
 #pragma unroll
@@ -499,22 +497,12 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
   }
   if constexpr (EPI == kStArgmax) {
     // ... then over the workgroup's column tiles: one candidate per row and column block for the reduction kernel
-    unsigned long long *const unit_best = reinterpret_cast<unsigned long long *>(lds);  // [kUnits][16], over sums that every wave has read
-    lds_barrier();
-#pragma unroll
-    for (int u = 0; u < kUnitsPerWave; ++u)
-      if (kg + u * kWaves < kUnits && c == 0)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) unit_best[(kg + u * kWaves) * 16 + 4 * b + q] = row_best[u][q];
     __syncthreads();
     if (tid < 16 * MT) {
       const int mt = tid >> 4, m = tid;
       unsigned long long best = 0ull;
 #pragma unroll
-      for (int tc = 0; tc < TC; ++tc) {
-        const unsigned long long other = unit_best[(tc * MT + mt) * 16 + (tid & 15)];
-        best = other > best ? other : best;
-      }
+      for (int tc = 0; tc < TC; ++tc) best = unit_best[tc * MT + mt][tid & 15] > best ? unit_best[tc * MT + mt][tid & 15] : best;
       if (m < M) a.cand[static_cast<size_t>(col_block) * M + m] = best;
     }
   }
