@@ -17,6 +17,8 @@
 //
 // int8 -> bf16 is exact (sign-extending byte convert, keep the high half).  No per-group arithmetic: the float32 accumulators
 // run over all of K and the epilogue reproduces the reference's two roundings, bf16(acc) then bf16(t * scale).
+#include <type_traits>
+
 #include "e2h_common.h"
 #include "e2h_stream.h"
 
@@ -153,6 +155,11 @@ struct Partial8 {
 };
 
 // ---- more than 64 rows ------------------------------------------------------------------------------------------------
+// What is too little work for the 32x32-tile kernels: few rows, or a head of one or two columns over many.  A chunk is one round of LDS
+// reads, products and a barrier, so its latency is the time.  The activations' fragments are read before the chunk's loads are issued
+// (behind the fence that keeps those in place they waited for the issue), and waves past the last column only help with staging: with
+// one column the fragment reads of the other three took most of the LDS bandwidth.  us before / fragments first / and idle waves out,
+// K = 4096: 65 rows x 1 column 26.7 / 24.9 / 17.6, 4096 x 1 30.3 / 28.5 / 21.8, 65 x 4096 31.7 / 29.4 / 28.9, 512 x 1024 31.4 / 29.2 / 28.8.
 
 template <int T>
 __global__ __launch_bounds__(64 * kColWaves) void int8_stream_mm_kernel(const uint16_t *__restrict__ x, const int8_t *__restrict__ q,
@@ -236,13 +243,15 @@ __global__ __launch_bounds__(64 * kColWaves) void int8_stream_mm_kernel(const ui
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  auto compute_chunk = [&](const WeightRegs8<T> &r, int parity, int qc, uint32_t live) {
+  bf16x8_t xf[MT][kSteps];
+  auto read_x = [&](int parity, int qc) {
     const uint8_t *buf = lds + (parity & 1) * kStageBytes + qc * kBufBytes + lane * 16;
-    bf16x8_t xf[MT][kSteps];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int s = 0; s < kSteps; ++s) xf[mt][s] = *reinterpret_cast<const bf16x8_t *>(buf + (mt * kSteps + s) * kFragBytes);
+  };
+  auto compute_chunk = [&](const WeightRegs8<T> &r, uint32_t live) {
 #pragma unroll
     for (int t = 0; t < T; ++t) {
 #pragma unroll
@@ -269,22 +278,32 @@ __global__ __launch_bounds__(64 * kColWaves) void int8_stream_mm_kernel(const ui
   for (int i = 0; i < PD; ++i) load_weights(ring[i], chunk_at(i));
   store_x(xstage[0], 0);
   lds_barrier();
-  for (int base = 0; base < nchunks; base += U) {
+  const auto chunks = [&](auto has_columns) {
+    for (int base = 0; base < nchunks; base += U) {
 #pragma unroll
-    for (int j = 0; j < U; ++j) {
-      const int i = base + j;
-      const int phase = i / CPP;
-      const uint32_t live = i < nchunks ? 0xFFFFFFFFu : 0u;
-      if (j % CPP == 0) load_x(xstage[(j / CPP) % XD], phase + XD);
-      load_weights(ring[(j + PD) % NB], chunk_at(i + PD));
-      __builtin_amdgcn_sched_barrier(0);  // the scheduler would sink the loads to their first use (65 rows, 4096 x 4096: 40 us, so 31)
-      compute_chunk(ring[j % NB], phase, j % CPP, live);
-      if (j % CPP == CPP - 1) {
-        store_x(xstage[(j / CPP + 1) % XD], phase + 1);
-        lds_barrier();
+      for (int j = 0; j < U; ++j) {
+        const int i = base + j;
+        const int phase = i / CPP;
+        const uint32_t live = i < nchunks ? 0xFFFFFFFFu : 0u;
+        if constexpr (has_columns) read_x(phase, j % CPP);
+        if (j % CPP == 0) load_x(xstage[(j / CPP) % XD], phase + XD);
+        if constexpr (has_columns) {
+          load_weights(ring[(j + PD) % NB], chunk_at(i + PD));
+          __builtin_amdgcn_sched_barrier(0);  // the scheduler would sink the loads to their first use (65 rows, 4096 x 4096: 40 us, so 31)
+          compute_chunk(ring[j % NB], live);
+        }
+        if (j % CPP == CPP - 1) {
+          store_x(xstage[(j / CPP + 1) % XD], phase + 1);
+          lds_barrier();
+        }
       }
     }
+  };
+  if (16 * tile16_0 >= N) {
+    chunks(std::false_type{});
+    return;
   }
+  chunks(std::true_type{});
 
 #pragma unroll
   for (int t = 0; t < T; ++t) {

@@ -45,6 +45,13 @@ def test_int8_mm_is_exact_on_integers(rows, n, k):
     assert torch.equal(ops.int8_mm_direct(x, w, scales), want)
 
 
+@pytest.mark.parametrize("rows", [65, 128, 200])
+@pytest.mark.parametrize("n,k", [(1, 128), (16, 384), (17, 256), (48, 4096), (64, 128), (65, 384), (129, 256)])
+def test_int8_mm_of_many_rows_and_few_columns_is_exact_on_integers(rows, n, k):
+    """one to all four waves of the last workgroup have columns; odd and even numbers of chunks"""
+    test_int8_mm_is_exact_on_integers(rows, n, k)
+
+
 @pytest.mark.parametrize("k", [128, 4096, 4224])
 def test_int8_extreme_codes(k):
     """codes -128 and 127 keep their sign and value; the products cancel in pairs"""
