@@ -613,8 +613,10 @@ bool plan(StagedArgs *a, Geometry *g, const void *staged, int64_t m, int64_t n, 
   // The geometry with the least cost; the weights of the cost were fitted to a sweep over T and S at 1 .. 64 rows of the shapes above and
   // 12288 / 4096 / 32000 x 4096: the chosen geometry is within 6 % of the best one there.  One round of 256 workgroups with many tiles
   // beats two rounds with few (w1|w3 22016 x 8192, 1 row: T = 12 43.6 us, T = 8 46.0; 32000 x 4096: T = 8 14.6, T = 6 19.0); K slices pay
-  // while a round is not full (w2 4096 x 11008, 32 rows: T = 4, S = 4 10.1 us, the best with S = 1 15.6).  At group size 32
-  // slices pay later (wo 4096 x 4096, 32 rows, with the norm behind it: two slices 12.0 us, four 13.2; group size 128 10.9 / 11.4).
+  // while a round is not full (w2 4096 x 11008, 32 rows: T = 4, S = 4 10.1 us, the best with S = 1 15.6).  What a slice costs the norm that
+  // adds it grows with rows and columns: fitted with the norm's time to 1 .. 64 rows of 1024 x 2048 .. 8192 x 22016 at every group size, where
+  // the choice is within 0.2 % of the best one on average and 6 % at most (one unit per slice whatever its size: 2.6 %, 31 %; 8192 x 8192 at
+  // group size 128 and 32 rows 19.9 us, now 18.6; 4096 x 4096 at group size 64 and 64 rows 15.5, now 13.7).
   double best_cost = -1;
   for (int s = 1; s <= (epi == kStPartial ? 8 : 1) && s <= kt; s *= 2) {
     if (want_s && epi == kStPartial && s != want_s) continue;
@@ -625,8 +627,8 @@ bool plan(StagedArgs *a, Geometry *g, const void *staged, int64_t m, int64_t n, 
       const long rounds = (wgs + kCUs - 1) / kCUs;
       const double chunks = static_cast<double>(kt) / s / kWaves;
       // per workgroup: a fixed part, per chunk its weight tiles (at 64 rows their matrix work) and the operands from L2;
-      // per slice: what the consumer pays to add it
-      const double cost = rounds * (6 + chunks * (t * (mt == 4 ? 2.0 : 1.0) + 1.2 * mt)) + s * (mt == 4 || groupsize == 32 ? 2.0 : 1.0);
+      // per slice: what the norm pays to add it
+      const double cost = rounds * (6 + chunks * (t * (mt == 4 ? 2.0 : 1.0) + 1.2 * mt)) + s * (0.5 + 0.6 * mt * n / 4096);
       if (best_cost < 0 || cost < best_cost) {
         best_cost = cost;
         *g = Geometry{t, s};
