@@ -11,8 +11,8 @@
 // (v_mfma_f32_16x16x4_f32, four groups per instruction).
 //
 // Decomposition: a workgroup is eight waves that split K (each wave a contiguous run of 128-wide chunks of the workgroup's K slice)
-// and all work on the same T tiles of 16 weight rows and on all rows of the batch, so that weights are read once.  No wave
-// shares anything with another until the end.  The eight partial tiles meet in LDS; wave w adds and finishes the (column tile, row
+// and all work on the same T tiles of 16 weight rows and on all rows of the batch, so that weights are read once (small weights beside 33
+// and more rows: on half of them, see plan).  No wave shares anything with another until the end.  The eight partial tiles meet in LDS; wave w adds and finishes the (column tile, row
 // tile) units w, w + 8, .. in a fixed order, so results are deterministic.  S workgroups may split K further (partial epilogue
 // only): their float32 sums go to slice s of a [S][M][N] array for the consumer to add in slice order.
 //
@@ -97,7 +97,7 @@ struct ZeroPoint {
   uint32_t sz[RB][T];
 };
 
-// G group size; MT row tiles of 16 (all rows of the batch); T weight tiles of 16 rows per workgroup (GATE: T/2 of each matrix).
+// G group size; MT row tiles of 16 (all rows of the batch, or one of its halves); T weight tiles of 16 rows per workgroup (GATE: T/2 of each matrix).
 template <int G, int MT, int T, int EPI>
 __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const StagedArgs a) {
   constexpr bool GATE = EPI == kStGate;
@@ -138,6 +138,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
   const int c0 = C0 + ((C1 - C0) * kg) / kWaves;
   const int nloc = C0 + ((C1 - C0) * (kg + 1)) / kWaves - c0;
   const int col_block = blockIdx.x;
+  const int row0 = blockIdx.z * (16 * MT);
   const int tile16_0 = col_block * TC;
   const int tiles = (N >> 4) - tile16_0 < TC ? (N >> 4) - tile16_0 : TC;  // N % 16 == 0
   const uint32_t row_block = static_cast<uint32_t>(a.Mpad) * 64u;  // bytes of one k segment of all rows
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
   const int q4 = lane >> 2;
   const uint32_t piece = static_cast<uint32_t>((lane & 3) ^ ((lane >> 4) & 3)) * 16u;
   const uint32_t w_lane = static_cast<uint32_t>(q4 >> 3) * KT * 512u + (q4 & 7) * 64u + piece;  // rows 0 .. 7, 8 .. 15: two packed tiles
-  const uint32_t x_lane = static_cast<uint32_t>(q4) * 64u + piece;
+  const uint32_t x_lane = static_cast<uint32_t>(row0 + q4) * 64u + piece;
   const auto column_of = [&](int t) { return 16 * (tile16_0 + (t < tiles ? t : tiles - 1)); };  // past the end: any valid one
   // unit p (static) of chunk i of this wave's run into ring place `at`
   const auto issue = [&](int p, int i, int at) {
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
       __builtin_amdgcn_raw_ptr_buffer_load_lds(GATE && p > 0 ? sz2_rsrc : sz_rsrc, dst, 16, off, chunk * (NGRP * 4u) * static_cast<uint32_t>(N), 0, 0);
     } else if (p < kHead) {
       const int s = (p - kSz) / MT, mt = (p - kSz) % MT;
-      const uint32_t off = 16 * mt + q4 < M ? x_lane + 1024u * mt : 0x80000000u;  // rows past M: out of the buffer's range, zeros
+      const uint32_t off = row0 + 16 * mt + q4 < M ? x_lane + 1024u * mt : 0x80000000u;  // rows past M: out of the buffer's range, zeros
       __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, dst, 16, off, (chunk * 4u + s) * row_block, 0, 0);
     } else {
       const int t = p - kHead;  // past N: out of the buffer's range, zeros
@@ -202,7 +203,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         // the group's 8 / NGRP sums of 16
-        const uint32_t off = so + static_cast<uint32_t>((16 * mt + c) * 32 + sub * (32 / NGRP));
+        const uint32_t off = so + static_cast<uint32_t>((row0 + 16 * mt + c) * 32 + sub * (32 / NGRP));
         if constexpr (NGRP == 1) {
           z.xs[r][mt][0] = __builtin_amdgcn_raw_buffer_load_b128(xs_rsrc, off, 0, 0);
           z.xs[r][mt][1] = __builtin_amdgcn_raw_buffer_load_b128(xs_rsrc, off + 16, 0, 0);
@@ -429,7 +430,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
       float *out = a.partials + static_cast<size_t>(ks) * M * N;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int m = 16 * mt + 4 * b + q;
+        const int m = row0 + 16 * mt + 4 * b + q;
         if (n < N && m < M) out[static_cast<size_t>(m) * N + n] = v[0][q];
       }
     } else if constexpr (EPI == kStGate) {
@@ -438,7 +439,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
       const bool tile_live = 16 * (tile16_0 + tc) < N;  // whole tiles: N % 16 == 0 on this path
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int m = 16 * mt + 4 * b + q;
+        const int m = row0 + 16 * mt + 4 * b + q;
         const float gate = bf16_round(v[0][q]), up = bf16_round(v[1][q]);
         const float act = bf16_round(gate / (1.0f + expf(-gate)));
         const uint16_t o = f32_to_bf16_rne(act * up);
@@ -469,7 +470,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int m = 16 * mt + 4 * b + q;
+        const int m = row0 + 16 * mt + 4 * b + q;
         const float own = bf16_round(v[0][q]);
         const float other = __shfl_xor(own, 1);  // the pair's other column lives in the neighbouring lane
         const float r = (c & 1) ? own * cs + other * sn : own * cs - other * sn;
@@ -495,7 +496,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
     } else {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int m = 16 * mt + 4 * b + q;
+        const int m = row0 + 16 * mt + 4 * b + q;
         if (n < N && m < M) a.y[static_cast<size_t>(m) * N + n] = f32_to_bf16_rne(v[0][q]);
       }
     }
@@ -504,7 +505,7 @@ __global__ __launch_bounds__(64 * kWaves) void int4_staged_mm_kernel(const Stage
     // ... then over the workgroup's column tiles: one candidate per row and column block for the reduction kernel
     __syncthreads();
     if (tid < 16 * MT) {
-      const int mt = tid >> 4, m = tid;
+      const int mt = tid >> 4, m = row0 + tid;
       unsigned long long best = 0ull;
 #pragma unroll
       for (int tc = 0; tc < TC; ++tc) {
@@ -546,18 +547,18 @@ __global__ __launch_bounds__(256) void int4_stage_x_kernel(const uint16_t *__res
 
 // ---- launch geometry ---------------------------------------------------------------------------------------------------
 struct Geometry {
-  int t, slices;  // weight tiles per workgroup, workgroups along K
+  int t, slices, mt, halves;  // weight tiles per workgroup, workgroups along K, row tiles per workgroup, workgroups along the rows
 };
 
 // most weight tiles whose sums, words, pairs and operands fit a wave's 256 vector registers beside the group's products
 constexpr int max_tiles(int G, int MT, bool gate) { return MT == 4 ? 6 : gate && G != 32 ? 12 : 8; }
 
 template <int G, int MT, int T, int EPI>
-int launch_staged(const StagedArgs &a, int slices, hipStream_t stream) {
+int launch_staged(const StagedArgs &a, const Geometry &g, hipStream_t stream) {
   if constexpr (T > max_tiles(G, MT, EPI == kStGate)) {
     return E2H_ERR_BAD_SHAPE;
   } else {
-    hipLaunchKernelGGL((int4_staged_mm_kernel<G, MT, T, EPI>), dim3(a.col_blocks, slices), dim3(64 * kWaves), 0, stream, a);
+    hipLaunchKernelGGL((int4_staged_mm_kernel<G, MT, T, EPI>), dim3(a.col_blocks, g.slices, g.halves), dim3(64 * kWaves), 0, stream, a);
     return launch_status();
   }
 }
@@ -565,25 +566,24 @@ int launch_staged(const StagedArgs &a, int slices, hipStream_t stream) {
 template <int G, int MT, int EPI>
 int dispatch_tiles(const StagedArgs &a, const Geometry &g, hipStream_t stream) {
   switch (g.t) {
-    case 2: return launch_staged<G, MT, 2, EPI>(a, g.slices, stream);
-    case 4: return launch_staged<G, MT, 4, EPI>(a, g.slices, stream);
-    case 6: return launch_staged<G, MT, 6, EPI>(a, g.slices, stream);
-    case 8: return launch_staged<G, MT, 8, EPI>(a, g.slices, stream);
+    case 2: return launch_staged<G, MT, 2, EPI>(a, g, stream);
+    case 4: return launch_staged<G, MT, 4, EPI>(a, g, stream);
+    case 6: return launch_staged<G, MT, 6, EPI>(a, g, stream);
+    case 8: return launch_staged<G, MT, 8, EPI>(a, g, stream);
   }
   if constexpr (EPI == kStGate) {
-    if (g.t == 12) return launch_staged<G, MT, 12, EPI>(a, g.slices, stream);
+    if (g.t == 12) return launch_staged<G, MT, 12, EPI>(a, g, stream);
   } else {
-    if (g.t == 1) return launch_staged<G, MT, 1, EPI>(a, g.slices, stream);
-    if (g.t == 3) return launch_staged<G, MT, 3, EPI>(a, g.slices, stream);
+    if (g.t == 1) return launch_staged<G, MT, 1, EPI>(a, g, stream);
+    if (g.t == 3) return launch_staged<G, MT, 3, EPI>(a, g, stream);
   }
   return E2H_ERR_BAD_SHAPE;
 }
 
 template <int EPI>
 int dispatch_staged(const StagedArgs &a, int groupsize, const Geometry &g, hipStream_t stream) {
-  const int mt = a.M <= 16 ? 1 : a.M <= 32 ? 2 : 4;
 #define E2H_ST_CASE(GV, MV) \
-  if (groupsize == GV && mt == MV) return dispatch_tiles<GV, MV, EPI>(a, g, stream);
+  if (groupsize == GV && g.mt == MV) return dispatch_tiles<GV, MV, EPI>(a, g, stream);
   E2H_ST_CASE(32, 1) E2H_ST_CASE(32, 2) E2H_ST_CASE(32, 4)
   E2H_ST_CASE(64, 1) E2H_ST_CASE(64, 2) E2H_ST_CASE(64, 4)
   E2H_ST_CASE(128, 1) E2H_ST_CASE(128, 2) E2H_ST_CASE(128, 4)
@@ -607,8 +607,14 @@ bool plan(StagedArgs *a, Geometry *g, const void *staged, int64_t m, int64_t n, 
   a->K = static_cast<int>(k);
   a->frag = static_cast<const uint8_t *>(staged);
   a->sums = reinterpret_cast<const float *>(a->frag + static_cast<size_t>(a->Mpad) * k * 2);
-  const int mt = a->M <= 16 ? 1 : a->M <= 32 ? 2 : 4, tiles16 = static_cast<int>(n / 16), kt = static_cast<int>(k / 128);
+  const int tiles16 = static_cast<int>(n / 16), kt = static_cast<int>(k / 128);
   const bool gate = epi == kStGate;
+  // Above 32 rows: four row tiles per workgroup, so that the weights are read once, or two workgroups of two row tiles each while the weights
+  // are small enough for L2 to hand them out twice and too small to fill the chip (64 rows, group size 128, us, one / two: 1024 x 2048 6.9 / 5.3,
+  // 6144 x 4096 with the rotation 13.0 / 10.9, 2 x 5504 x 2048 gated 12.0 / 11.5, 4096 x 4096 with its norm 13.5 / 13.0; 12288 x 4096
+  // 15.0 / 14.3 but 13.4 / 13.8 at 33 rows, 4096 x 11008 with its norm 19.2 / 19.7, 10240 x 8192 26.3 / 29.0, 2 x 11008 x 4096 24.7 / 27.4).
+  const int halves = a->M > 32 && n * k * (gate ? 2 : 1) <= (int64_t{1} << 25) ? 2 : 1;
+  const int mt = a->M <= 16 ? 1 : a->M <= 32 || halves == 2 ? 2 : 4;
   const int want_t = options().staged_tiles, want_s = options().staged_slices;  // experiments: force a geometry
   // The geometry with the least cost; the weights of the cost were fitted to a sweep over T and S at 1 .. 64 rows of the shapes above and
   // 12288 / 4096 / 32000 x 4096: the chosen geometry is within 6 % of the best one there.  One round of 256 workgroups with many tiles
@@ -623,15 +629,15 @@ bool plan(StagedArgs *a, Geometry *g, const void *staged, int64_t m, int64_t n, 
     for (int t : {1, 2, 3, 4, 6, 8, 12}) {
       if (t > max_tiles(groupsize, mt, gate) || (gate && t % 2) || (want_t && !gate && t != want_t)) continue;
       const int tc = gate ? t / 2 : t;
-      const long wgs = static_cast<long>((tiles16 + tc - 1) / tc) * s;
+      const long wgs = static_cast<long>((tiles16 + tc - 1) / tc) * s * halves;
       const long rounds = (wgs + kCUs - 1) / kCUs;
       const double chunks = static_cast<double>(kt) / s / kWaves;
       // per workgroup: a fixed part, per chunk its weight tiles (at 64 rows their matrix work) and the operands from L2;
       // per slice: what the norm pays to add it
-      const double cost = rounds * (6 + chunks * (t * (mt == 4 ? 2.0 : 1.0) + 1.2 * mt)) + s * (0.5 + 0.6 * mt * n / 4096);
+      const double cost = rounds * (6 + chunks * (t * (mt == 4 ? 2.0 : 1.0) + 1.2 * mt)) + s * (0.5 + 0.6 * mt * halves * n / 4096);
       if (best_cost < 0 || cost < best_cost) {
         best_cost = cost;
-        *g = Geometry{t, s};
+        *g = Geometry{t, s, mt, halves};
       }
     }
   }

@@ -257,3 +257,40 @@ def test_staged_mm_is_exact_on_integers_at_the_edges(g, m, n, k):
     assert torch.equal(ops.int4_mm_staged_argmax(xs, packed, g, sz), ops.argmax_rows(plain))
     gate, _ = ops.int4_mm_staged_silu_gate(xs, packed, sz, packed, sz, g, want_rows=True, want_staged=False)
     assert torch.equal(gate, ops.silu_mul(plain, plain))
+
+
+@pytest.mark.parametrize("g", [32, 64, 128])
+@pytest.mark.parametrize("m", [33, 48, 49, 64])
+@pytest.mark.parametrize("n,k", [(2048, 8192), (2064, 8192), (4096, 8192), (4112, 8192)])
+def test_staged_mm_on_both_sides_of_the_line_between_halves_and_whole_batches(g, m, n, k):
+    """33 rows and more: two workgroups share the rows up to 2^25 weights (of both matrices in the gated launch), one takes them all above.
+    Integers as above: sums stay below 8192 * 143 * 2 < 2^22."""
+    test_staged_mm_is_exact_on_integers_at_the_edges(g, m, n, k)
+
+
+@pytest.mark.parametrize("m", [33, 48, 64])
+def test_halves_hand_on_the_staged_gate_of_all_rows(m):
+    gen = torch.Generator().manual_seed(m)
+    w = torch.randn((2, 256, 512), generator=gen).to(torch.bfloat16).to(DEV)
+    (p1, z1), (p2, z2) = (ops.int4_quantize_pack(v, 64, 8) for v in w)
+    xs = ops.stage_x(torch.randn((m, 512), generator=gen).to(torch.bfloat16).to(DEV))
+    rows, staged = ops.int4_mm_staged_silu_gate(xs, p1, z1, p2, z2, 64, want_rows=True)
+    again = ops.stage_x(rows)
+    packed, sz = ops.int4_quantize_pack(torch.randn((64, 256), generator=gen).to(torch.bfloat16).to(DEV), 64, 8)
+    # the next linear sees the same operands whether they were staged by the launch or from its rows
+    assert torch.equal(ops.int4_mm_staged(staged, packed, 64, sz), ops.int4_mm_staged(again, packed, 64, sz))
+
+
+@pytest.mark.parametrize("bsz", [33, 48, 64])
+def test_halves_rotate_and_cache_every_row(bsz):
+    n_head, n_kv, hd, k, g, s_max = 3, 1, 64, 512, 64, 16
+    from easy_to_hard_amd.model import precompute_freqs_cis
+
+    freqs = precompute_freqs_cis(s_max, hd, 10000, device=DEV)
+    packed, sz = ops.int4_quantize_pack(randn_bf16(((n_head + 2 * n_kv) * hd, k), seed=5).to(DEV), g, 8)
+    xs = ops.stage_x(randn_bf16((bsz, k), seed=9).to(DEV))
+    pos = torch.tensor([7], dtype=torch.int64, device=DEV)
+    kc, vc, kc2, vc2 = (torch.zeros((bsz, n_kv, s_max, hd), dtype=torch.bfloat16, device=DEV) for _ in range(4))
+    q = ops.int4_mm_staged_rope_kv(xs, packed, sz, g, freqs, kc, vc, pos, n_head, n_kv, hd)
+    q2 = ops.rope_kv_write(ops.int4_mm_staged(xs, packed, g, sz), freqs, kc2, vc2, pos, n_head, n_kv, hd)
+    assert torch.equal(q, q2) and torch.equal(kc, kc2) and torch.equal(vc, vc2)
