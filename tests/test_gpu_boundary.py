@@ -331,7 +331,9 @@ def test_decode_step_with_deferred_slices_equals_the_step_without(bsz, mode, mon
 def test_staged_decode_step_agrees_with_the_row_major_fused_step(monkeypatch):
     """The single-token step on staged activations (model.STAGED_DECODE) against the same step on the row-major fused
     kernels, two layers of the 7B shape at 32 and 5 rows: same arithmetic up to the order of the float32 sums over K, so the
-    logits agree to bfloat16 rounding noise; the staged step replayed from a HIP graph equals its eager run bit for bit."""
+    logits agree to bfloat16 rounding noise; the staged step replayed from a HIP graph equals its eager run bit for bit.  Both are fed the tokens
+    that the row-major step picks: with its own, a row whose two largest logits are one bfloat16 unit apart (4.8125 and 4.78125 in the second
+    step here) could go on as another sequence, of which the bound says nothing."""
     import easy_to_hard_amd.model as model_mod
     from easy_to_hard_amd.model import ModelArgs, random_quantized_transformer
 
@@ -341,16 +343,19 @@ def test_staged_decode_step_agrees_with_the_row_major_fused_step(monkeypatch):
     t = 7
     for bsz in (32, 5):
         prompt = torch.randint(0, cfg.vocab_size, (bsz, t), generator=torch.Generator().manual_seed(4)).to(DEV)
-        logits = {}
+        logits, tokens = {}, []
         for staged in (False, True):
             monkeypatch.setattr(model_mod, "STAGED_DECODE", staged)
             model.max_seq_length = -1
             model.setup_caches(bsz, 32)
             assert model.staged_step_supported(bsz) == staged
             cur = prefill(model, prompt, torch.arange(0, t, device=DEV))
+            assert not tokens or torch.equal(cur, tokens[0])
             out = []
             for i in range(3):
-                lg = model(cur, torch.tensor([t + i], device=DEV))
+                if not staged:
+                    tokens.append(cur)
+                lg = model(tokens[i], torch.tensor([t + i], device=DEV))
                 out.append(lg[:, -1].clone())
                 cur = torch.argmax(lg[:, -1].float(), dim=-1, keepdim=True)
             logits[staged] = torch.stack(out).float()
@@ -358,8 +363,7 @@ def test_staged_decode_step_agrees_with_the_row_major_fused_step(monkeypatch):
         assert err <= 2e-2, err
         stepper = GraphedDecodeStep(model, bsz, DEV)
         prefill(model, prompt, torch.arange(0, t, device=DEV))
-        first = torch.argmax(logits[True][0], dim=-1, keepdim=True)
-        tok = stepper.step(first, torch.tensor([t + 1], device=DEV)).clone()
+        tok = stepper.step(tokens[1], torch.tensor([t + 1], device=DEV)).clone()
         assert torch.equal(tok, torch.argmax(logits[True][1], dim=-1, keepdim=True))
 
 
