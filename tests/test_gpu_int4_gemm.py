@@ -55,13 +55,14 @@ def test_exact_on_dyadic_operands(many_row_kernel, g, slices, tile, m, n, k):
 @pytest.mark.parametrize("g", [32, 64, 128])
 @pytest.mark.parametrize("slices", [1, 2])
 def test_scales_outside_the_running_units(many_row_kernel, g, slices):
-    """zero, the smallest and large scales in some columns: those workgroups form every group's sum by itself.  Columns whose scales are
-    all representable stay exact; a column with an infinite or NaN scale is not finite, its neighbours are untouched."""
+    """a scale of zero, and columns of scales that the units do not carry, whose workgroups form every group's sum by itself.  Columns whose
+    scales are finite stay exact; a column with an infinite or NaN scale is not finite, its neighbours are untouched."""
     m, n, k = 130, 528, 1024
     _lib.set_option("int4_k_slices", slices)
     codes, scale, zero, x = _case(m, n, k, g)
     scale[0, 3] = 0.0
     zero[:, 5], scale[:, 5] = 0.0, 2.0**-100
+    zero[:, 7], scale[:, 7] = 0.0, 2.0**-101
     zero[:, 260], scale[:, 260] = 0.0, 2.0**40
     scale[-1, 300] = float("inf")
     scale[-1, 301] = float("nan")

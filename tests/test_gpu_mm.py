@@ -672,13 +672,9 @@ def test_int8_gate_matches_oracle_and_unfused_path(m, n, k):
     a = qo.int8_linear_fp32(bf16_to_np(x), q1, s1).astype(np.float64)
     b = qo.int8_linear_fp32(bf16_to_np(x), q2, s2).astype(np.float64)
     assert qo.normwise_rel_err(bf16_to_np(y), a / (1.0 + np.exp(-a)) * b) <= TOL
-    # same accumulation order as the single-matrix kernel with one K slice: identical bits
-    _lib.set_option("int8_k_slices", 1)
-    try:
-        ya = ops.int8_mm_direct(xd, q1_d, s1_d)
-        yb = ops.int8_mm_direct(xd, q2_d, s2_d)
-    finally:
-        _lib.set_option("int8_k_slices", 0)
+    # same accumulation order as the single-matrix launch: identical bits
+    ya = ops.int8_mm_direct(xd, q1_d, s1_d)
+    yb = ops.int8_mm_direct(xd, q2_d, s2_d)
     assert torch.equal(y, ops.silu_mul(ya, yb) if (m * n) % 8 == 0 else torch.nn.functional.silu(ya) * yb)
     with pytest.raises(RuntimeError):
         ops.int8_mm_silu_gate(randn_bf16((65, k), seed=3).to(DEV), q1_d, s1_d, q2_d, s2_d)  # more than 64 rows
@@ -700,11 +696,7 @@ def test_int8_rope_kv_matches_two_kernel_path(bsz, n_head, n_kv, d, k):
     input_pos = torch.tensor([pos], device=DEV)
     kc, vc = kc0.clone(), vc0.clone()
     q = ops.int8_mm_rope_kv(x, q_d, s_d, freqs, kc, vc, input_pos, n_head, n_kv, d)
-    _lib.set_option("int8_k_slices", 1)
-    try:
-        qkv = ops.int8_mm_direct(x, q_d, s_d)
-    finally:
-        _lib.set_option("int8_k_slices", 0)
+    qkv = ops.int8_mm_direct(x, q_d, s_d)
     kc2, vc2 = kc0.clone(), vc0.clone()
     q2 = ops.rope_kv_write(qkv, freqs, kc2, vc2, input_pos, n_head, n_kv, d)
     assert torch.equal(q, q2) and torch.equal(kc, kc2) and torch.equal(vc, vc2)

@@ -36,8 +36,7 @@ def test_column_shards_concatenate_to_the_full_output(kind, world):
     n, k = 512, 1024
     full = _quantized(kind, n, k)
     x = randn_bf16((5, k), seed=3).to(DEV)
-    _lib.set_option("int4_k_slices", 1)   # same accumulation order whatever the shard's width
-    _lib.set_option("int8_k_slices", 1)
+    _lib.set_option("int4_k_slices", 1)   # same accumulation order whatever the shard's width (int8 has one order)
     try:
         y = full(x)
         parts = []
@@ -48,7 +47,6 @@ def test_column_shards_concatenate_to_the_full_output(kind, world):
             parts.append(shard(x))
     finally:
         _lib.set_option("int4_k_slices", 0)
-        _lib.set_option("int8_k_slices", 0)
     assert torch.equal(torch.cat(parts, dim=-1), y)
 
 
@@ -75,7 +73,6 @@ def test_fused_qkv_is_sharded_part_by_part(kind):
     full = _quantized(kind, dim + 2 * kv, 512)
     x = randn_bf16((3, 512), seed=5).to(DEV)
     _lib.set_option("int4_k_slices", 1)
-    _lib.set_option("int8_k_slices", 1)
     try:
         q, k_, v = full(x).split([dim, kv, kv], dim=-1)
         for r in range(world):
@@ -87,7 +84,6 @@ def test_fused_qkv_is_sharded_part_by_part(kind):
             assert torch.equal(vs, v[:, r * kv // world:(r + 1) * kv // world])
     finally:
         _lib.set_option("int4_k_slices", 0)
-        _lib.set_option("int8_k_slices", 0)
 
 
 def test_uneven_shards_are_refused():
