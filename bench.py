@@ -34,7 +34,7 @@ HBM_PEAK_GBPS = 8000.0
 # profiles/int4_staged_mm_7b_decode_bs32.md (int4_skinny_mm_7b_decode_bs32.md for the row-major kernels).  Counters cannot be read from inside this process, so the figure is
 # recorded here for the configuration and kernel set it was measured on and reported as null for any other.
 MEASURED_TRAFFIC_BYTES = {("7B", "int4", 128, 32, "int4_skinny_mm_kernel"): 33_440_000,
-                          ("7B", "int4", 128, 32, "int4_staged_mm_kernel"): 32_370_000}
+                          ("7B", "int4", 128, 32, "int4_staged_mm_kernel"): 32_390_000}
 
 
 def parse_args():
@@ -184,7 +184,7 @@ def measure_gemv_roofline(model, batch, reps, traffic_key=None):
             calls.append(lambda x=x, m=mod: m(x))
             bytes_pass += algorithmic_bytes(mod, batch)
     if kernel_set is None:
-        kernel_set = "int4_skinny_mm_kernel" if "Int4" in type(by_name[next(iter(by_name))]).__name__ else "int8_stream_mm_kernel"
+        kernel_set = "int4_skinny_mm_kernel" if "Int4" in type(by_name[next(iter(by_name))]).__name__ else "stream_mm_kernel"
 
     def one_pass():
         out = None
