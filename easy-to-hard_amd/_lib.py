@@ -121,6 +121,8 @@ _SEQ_SIGNATURES = {
     "e2h_seq_linear": (c_int, [_P, _P, _P, c_int64, c_int64, c_int64, c_int, c_float, _P, c_int64, _P]),
     "e2h_seq_rotary_table": (c_int, [_P, _P, _P, _P, c_int64, c_int64, c_int64, _P]),
     "e2h_seq_window_attention": (c_int, [_A(WindowAttentionArgs), _P]),
+    "e2h_seq_window_attention_scratch_bytes": (c_int64, [_A(WindowAttentionArgs)]),
+    "e2h_seq_window_attention_split": (c_int, [_A(WindowAttentionArgs), _P, c_int64, _P]),
     "e2h_seq_hgrn2_scratch_bytes": (c_int64, [_A(Hgrn2Args)]),
     "e2h_seq_hgrn2": (c_int, [_A(Hgrn2Args), _P]),
     "e2h_seq_delta_scratch_bytes": (c_int64, [_A(DeltaArgs)]),

@@ -576,11 +576,16 @@ __global__ __launch_bounds__(256) void attention_prefill_kernel(const e2h_window
   }
 }
 
-// ---- bfloat16, one token per sequence: one workgroup per (sequence, key/value head) ------------------------------------------
-// The lane columns are the query heads of the group (up to 16); the waves take key tiles of 32 round robin and are combined at
-// the end.  The workgroup appends its own new key and value row first.
+// ---- bfloat16, one token per sequence: `splits` workgroups per (sequence, key/value head) --------------------------------------
+// The lane columns are the query heads of the group (up to 16); the waves of all its workgroups take key tiles of 32 round robin and
+// are combined at the end: in LDS, then, where there are several workgroups, by attention_combine_kernel from `part`
+// ([sequence and key/value head][split][head of the group][DV sums, maximum, sum of weights]).  The workgroup whose tile holds the new
+// token's row appends that row first.
+// A tile is a serial chain of 2.4 us (load, product, softmax, product), so what bounds few sequences is tiles per wave and not
+// bytes: 4 sequences x 8 key heads over 2048 keys took 25.5 us with one workgroup each (9 tiles per wave on 32 of 256 CUs), 12.9 with eight; 1 sequence 23.9 and 11.6; 30000 keys 273 and
+// 29.  32 sequences (256 workgroups, no split) read 6 TB/s.
 template <int KS, int VT, int NW, bool VEC>
-__global__ __launch_bounds__(64 * NW) void attention_step_kernel(const e2h_window_attention_args a) {
+__global__ __launch_bounds__(64 * NW) void attention_step_kernel(const e2h_window_attention_args a, int splits, float *part) {
   constexpr int kVRow = VT * 32 + 8;  // bytes per value row in LDS
   constexpr int kWaveLds = 32 * kVRow;
   constexpr int kEndLds = NW * (16 * VT * 16 + 32) * 4;
@@ -589,15 +594,20 @@ __global__ __launch_bounds__(64 * NW) void attention_step_kernel(const e2h_windo
   const int lane = threadIdx.x & 63, c = lane & 15, b4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int D = static_cast<int>(a.dim), DV = static_cast<int>(a.vdim);
-  const int bi = blockIdx.x / static_cast<int>(a.kv_heads), g = blockIdx.x % static_cast<int>(a.kv_heads);
+  const int split = static_cast<int>(blockIdx.x % splits), pair = static_cast<int>(blockIdx.x / splits);
+  const int bi = pair / static_cast<int>(a.kv_heads), g = pair % static_cast<int>(a.kv_heads);
   const int rep = static_cast<int>(a.heads / a.kv_heads);
   const int pos = static_cast<int>(a.input_pos[0]);
   const int first = a.first ? static_cast<int>(a.first[bi]) : 0;
+  const int last = pos < a.cache_len ? pos : static_cast<int>(a.cache_len) - 1;
+  const KeyList kl = key_list(pos, last, first, static_cast<int>(a.window), static_cast<int>(a.keep_first));
+  // the list ends with the new token's row
+  const bool appends = split == (kl.count > 0 ? (kl.count - 1) / 32 / NW % splits : 0);
   const bf16_t *proj = static_cast<const bf16_t *>(a.proj) + static_cast<size_t>(bi) * a.ld;
   bf16_t *kc = static_cast<bf16_t *>(a.k_cache) + (static_cast<size_t>(bi) * a.kv_heads + g) * a.cache_len * D;
   bf16_t *vc = static_cast<bf16_t *>(a.v_cache) + (static_cast<size_t>(bi) * a.kv_heads + g) * a.cache_len * DV;
   const bool prepared = a.k_norm || a.rotary;
-  if (a.k_off >= 0 && pos >= 0 && pos < a.cache_len) {
+  if (appends && a.k_off >= 0 && pos >= 0 && pos < a.cache_len) {
     if (prepared && wave == 0) {  // norm and rotation by the first wave, the others copy the value
       const int d = 8 * lane;
       float v[8];
@@ -641,8 +651,6 @@ __global__ __launch_bounds__(64 * NW) void attention_step_kernel(const e2h_windo
   __threadfence_block();
   __syncthreads();  // the new row is visible to the workgroup
 
-  const int last = pos < a.cache_len ? pos : static_cast<int>(a.cache_len) - 1;
-  const KeyList kl = key_list(pos, last, first, static_cast<int>(a.window), static_cast<int>(a.keep_first));
   f32x4_t oacc[VT];
   float m_run = kMasked, l_run = 0.f;
 #pragma unroll
@@ -651,7 +659,7 @@ __global__ __launch_bounds__(64 * NW) void attention_step_kernel(const e2h_windo
   uint8_t *v_lds = lds + wave * kWaveLds;
   constexpr int kVPer = (32 * VT * 2 + 63) / 64;
 
-  for (int n0 = wave * 32; n0 < kl.count; n0 += NW * 32) {
+  for (int n0 = (split * NW + wave) * 32; n0 < kl.count; n0 += splits * NW * 32) {
     u32x4_t kf[2][KS], vr[kVPer];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -749,12 +757,92 @@ __global__ __launch_bounds__(64 * NW) void attention_step_kernel(const e2h_windo
       l += sh_l[w * 16 + r] * cw;
       o += sh_o[(w * 16 + r) * VT * 16 + d] * cw;
     }
+    if (part) {
+      float *row = part + (static_cast<size_t>(blockIdx.x) * rep + r) * (DV + 2);
+      row[d] = o;
+      if (d == 0) {
+        row[DV] = m;
+        row[DV + 1] = l;
+      }
+      continue;
+    }
     if (a.sink) l += __builtin_amdgcn_exp2f(__builtin_fmaf(a.sink[g * rep + r], kLog2e, -m));
     const int col = (g * rep + r) * DV + d;
     o = l > 0.f ? o / l * a.out_scale : 0.f;
     if (a.g_off >= 0) o *= sigmoid_f32(to_f32(proj[a.g_off + col]));
     static_cast<bf16_t *>(a.out)[static_cast<size_t>(bi) * a.ld_out + a.out_off + col] = from_f32<bf16_t>(o);
   }
+}
+
+// one value of one head per thread: the splits' sums, each in units of its own maximum, brought to the largest
+__global__ __launch_bounds__(256) void attention_combine_kernel(const e2h_window_attention_args a, int splits, const float *part) {
+  const int H = static_cast<int>(a.heads), G = static_cast<int>(a.kv_heads), DV = static_cast<int>(a.vdim), rep = H / G;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= a.batch * H * DV) return;
+  const int d = static_cast<int>(i % DV), h = static_cast<int>(i / DV % H), bi = static_cast<int>(i / DV / H), stride = rep * (DV + 2);
+  const float *row = part + (static_cast<size_t>(bi) * G + h / rep) * splits * stride + (h % rep) * (DV + 2);
+  constexpr int kAtOnce = 8;
+  float m = kMasked, l = 0.f, o = 0.f;
+  for (int s0 = 0; s0 < splits; s0 += kAtOnce) {
+    float ms[kAtOnce], ls[kAtOnce], os[kAtOnce];
+#pragma unroll
+    for (int k = 0; k < kAtOnce; ++k) {
+      const bool there = s0 + k < splits;
+      const float *p = row + static_cast<size_t>(there ? s0 + k : s0) * stride;
+      ms[k] = there ? p[DV] : kMasked;
+      ls[k] = there ? p[DV + 1] : 0.f;
+      os[k] = there ? p[d] : 0.f;
+    }
+    float m_new = m;
+#pragma unroll
+    for (int k = 0; k < kAtOnce; ++k) m_new = fmaxf(m_new, ms[k]);
+    const float corr = __builtin_amdgcn_exp2f(m - m_new);
+    l *= corr;
+    o *= corr;
+    m = m_new;
+#pragma unroll
+    for (int k = 0; k < kAtOnce; ++k) {
+      const float c = __builtin_amdgcn_exp2f(ms[k] - m);
+      l = __builtin_fmaf(ls[k], c, l);
+      o = __builtin_fmaf(os[k], c, o);
+    }
+  }
+  if (a.sink) l += __builtin_amdgcn_exp2f(__builtin_fmaf(a.sink[h], kLog2e, -m));
+  o = l > 0.f ? o / l * a.out_scale : 0.f;
+  if (a.g_off >= 0) o *= sigmoid_f32(to_f32(static_cast<const bf16_t *>(a.proj)[static_cast<size_t>(bi) * a.ld + a.g_off + static_cast<int64_t>(h) * DV + d]));
+  static_cast<bf16_t *>(a.out)[static_cast<size_t>(bi) * a.ld_out + a.out_off + static_cast<int64_t>(h) * DV + d] = from_f32<bf16_t>(o);
+}
+
+bool on_matrix_cores(const e2h_window_attention_args &a) {
+  return a.dtype == E2H_SEQ_BF16 && a.heads / a.kv_heads <= 16 && a.scale > 0.f;
+}
+
+// waves per workgroup of the step: one walks 32 keys at a time; more of them pay once there are enough keys to share
+int64_t step_span(const e2h_window_attention_args &a) {
+  return a.window > 0 && a.window <= INT32_MAX && a.keep_first <= INT32_MAX && a.window + a.keep_first < a.cache_len ? a.window + a.keep_first : a.cache_len;
+}
+int step_waves(const e2h_window_attention_args &a) {
+  const int64_t d = a.dim > a.vdim ? a.dim : a.vdim;
+  const int nw = seq_options().attention_decode_waves ? seq_options().attention_decode_waves : (step_span(a) > 256 ? 8 : 4);
+  return d <= 128 ? nw : 4;
+}
+
+// Workgroups per (sequence, key/value head) of the step, so that there is one per CU at most (two cost more than they share: 8 sequences x
+// 8 key heads over 2052 keys in 4 parts 18.8 us, in 8 parts 24.2).  A tile takes a wave 2.4 us and the combining launch 4 to 5, so fewer than
+// three tiles per wave are not shared (300 keys, 4 sequences: 9.2 us whole, 10.9 in two parts), and two parts never pay: 86 and more
+// workgroups already read at the memory's rate (16 sequences 27.2 us whole, 28.3 in two parts).
+constexpr int kMostSplits = 64;
+int step_splits(const e2h_window_attention_args &a) {
+  if (a.seqlen != 1 || !on_matrix_cores(a)) return 1;
+  const int64_t rounds = (step_span(a) + 32 * step_waves(a) - 1) / (32 * step_waves(a));  // tiles of a wave
+  const int64_t fit = 256 / (a.batch * a.kv_heads);
+  int64_t s = rounds < fit ? rounds : fit;
+  s = s < kMostSplits ? s : kMostSplits;
+  return s < 3 ? 1 : static_cast<int>(s);
+}
+
+int64_t step_scratch_bytes(const e2h_window_attention_args &a, int splits) {
+  return splits < 2 ? 0 : a.batch * a.heads * splits * (a.vdim + 2) * 4;
 }
 
 void launch_append(const e2h_window_attention_args &a, bool vec, hipStream_t s) {
@@ -781,14 +869,15 @@ void launch_append(const e2h_window_attention_args &a, bool vec, hipStream_t s) 
 }
 
 template <int KS, int VT, bool VEC>
-void launch_mfma(const e2h_window_attention_args &a, hipStream_t s) {
+void launch_mfma(const e2h_window_attention_args &a, float *part, int64_t part_bytes, hipStream_t s) {
   if (a.seqlen == 1) {
-    const dim3 grid(static_cast<unsigned>(a.batch * a.kv_heads));
-    // one wave walks 32 keys at a time; more waves pay once there are enough keys to share
-    const int64_t span = a.window > 0 && a.window + a.keep_first < a.cache_len ? a.window + a.keep_first : a.cache_len;
-    const int nw = seq_options().attention_decode_waves ? seq_options().attention_decode_waves : (span > 256 ? 8 : 4);
-    if (nw == 8 && KS <= 4) hipLaunchKernelGGL((attention_step_kernel<KS, VT, (KS <= 4 ? 8 : 4), VEC>), grid, dim3(KS <= 4 ? 512 : 256), 0, s, a);
-    else hipLaunchKernelGGL((attention_step_kernel<KS, VT, 4, VEC>), grid, dim3(256), 0, s, a);
+    int splits = step_splits(a);
+    if (!part || step_scratch_bytes(a, splits) > part_bytes) splits = 1;
+    if (splits == 1) part = nullptr;
+    const dim3 grid(static_cast<unsigned>(a.batch * a.kv_heads * splits));
+    if (step_waves(a) == 8) hipLaunchKernelGGL((attention_step_kernel<KS, VT, (KS <= 4 ? 8 : 4), VEC>), grid, dim3(KS <= 4 ? 512 : 256), 0, s, a, splits, part);
+    else hipLaunchKernelGGL((attention_step_kernel<KS, VT, 4, VEC>), grid, dim3(256), 0, s, a, splits, part);
+    if (part) hipLaunchKernelGGL(attention_combine_kernel, dim3(static_cast<unsigned>((a.batch * a.heads * a.vdim + 255) / 256)), dim3(256), 0, s, a, splits, part);
     return;
   }
   launch_append(a, VEC && aligned16(a.k_bias) && aligned16(a.v_bias) && a.k_off % 8 == 0 && a.v_off % 8 == 0, s);
@@ -797,12 +886,12 @@ void launch_mfma(const e2h_window_attention_args &a, hipStream_t s) {
 }
 
 template <bool VEC>
-void launch_mfma_by_size(const e2h_window_attention_args &a, hipStream_t s) {
+void launch_mfma_by_size(const e2h_window_attention_args &a, float *part, int64_t part_bytes, hipStream_t s) {
   const int64_t d = a.dim > a.vdim ? a.dim : a.vdim;
-  if (d <= 32) launch_mfma<1, 2, VEC>(a, s);
-  else if (d <= 64) launch_mfma<2, 4, VEC>(a, s);
-  else if (d <= 128) launch_mfma<4, 8, VEC>(a, s);
-  else launch_mfma<8, 16, VEC>(a, s);
+  if (d <= 32) launch_mfma<1, 2, VEC>(a, part, part_bytes, s);
+  else if (d <= 64) launch_mfma<2, 4, VEC>(a, part, part_bytes, s);
+  else if (d <= 128) launch_mfma<4, 8, VEC>(a, part, part_bytes, s);
+  else launch_mfma<8, 16, VEC>(a, part, part_bytes, s);
 }
 
 void launch_rows(const e2h_window_attention_args &a, hipStream_t s) {
@@ -828,7 +917,7 @@ extern "C" int e2h_seq_rotary_table(const double *turns, const int64_t *input_po
   return launch_status();
 }
 
-extern "C" int e2h_seq_window_attention(const e2h_window_attention_args *a, void *stream) {
+static int check_attention(const e2h_window_attention_args *a) {
   if (!a || !a->proj || !a->k_cache || !a->v_cache || !a->input_pos || !a->out) return E2H_ERR_NULL_POINTER;
   if (a->dtype != E2H_SEQ_BF16 && a->dtype != E2H_SEQ_F32) return E2H_ERR_BAD_SHAPE;
   if (a->batch < 1 || a->seqlen < 1 || a->heads < 1 || a->kv_heads < 1 || a->heads % a->kv_heads != 0 || a->dim < 1 || a->vdim < 1 ||
@@ -843,20 +932,36 @@ extern "C" int e2h_seq_window_attention(const e2h_window_attention_args *a, void
     return E2H_ERR_BAD_SHAPE;
   if (a->batch * a->seqlen * a->heads > INT32_MAX || a->batch * a->seqlen * a->kv_heads * (a->dim + a->vdim) / 256 > INT32_MAX - 1)
     return E2H_ERR_BAD_SHAPE;
+  return E2H_OK;
+}
+
+extern "C" int64_t e2h_seq_window_attention_scratch_bytes(const e2h_window_attention_args *a) {
+  if (const int rc = check_attention(a)) return rc;
+  return step_scratch_bytes(*a, step_splits(*a));
+}
+
+extern "C" int e2h_seq_window_attention(const e2h_window_attention_args *a, void *stream) {
+  return e2h_seq_window_attention_split(a, nullptr, 0, stream);
+}
+
+extern "C" int e2h_seq_window_attention_split(const e2h_window_attention_args *a, void *scratch, int64_t scratch_bytes, void *stream) {
+  if (const int rc = check_attention(a)) return rc;
+  if (reinterpret_cast<uintptr_t>(scratch) & 3) return E2H_ERR_MISALIGNED;
   hipStream_t s = static_cast<hipStream_t>(stream);
   e2h_window_attention_args v = *a;
   const int64_t most = INT32_MAX / 2;  // no limit, as far as any cache reaches
   v.window = v.window == 0 || v.window > most ? most : v.window;
   v.keep_first = v.keep_first > most ? most : v.keep_first;
   a = &v;
-  if (a->dtype == E2H_SEQ_F32 || a->heads / a->kv_heads > 16 || !(a->scale > 0.f)) {
+  if (!on_matrix_cores(*a)) {
     launch_rows(*a, s);
     return launch_status();
   }
   const bool vec = a->dim % 8 == 0 && a->vdim % 8 == 0 && a->ld % 8 == 0 && a->q_off % 8 == 0 && (a->g_off < 0 || a->g_off % 4 == 0) &&
                    a->ld_out % 4 == 0 && a->out_off % 4 == 0 && aligned16(a->proj) && aligned16(a->k_cache) && aligned16(a->v_cache) && aligned16(a->out) &&
                    aligned16(a->q_norm) && aligned16(a->k_norm);
-  if (vec) launch_mfma_by_size<true>(*a, s);
-  else launch_mfma_by_size<false>(*a, s);
+  float *const part = static_cast<float *>(scratch);
+  if (vec) launch_mfma_by_size<true>(*a, part, scratch_bytes, s);
+  else launch_mfma_by_size<false>(*a, part, scratch_bytes, s);
   return launch_status();
 }

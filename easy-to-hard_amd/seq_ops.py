@@ -227,7 +227,10 @@ def window_attention(proj, batch, seqlen, heads, kv_heads, dim, vdim, offsets, b
         a.rotary, a.rot_pairs = _vec(rotary, batch * seqlen * rotary.shape[-2] * 2, "window_attention rotary"), rotary.shape[-2]
     a.sink = _vec(sink, heads, "window_attention sink")
     a.input_pos, a.first = _positions(input_pos, first, batch, seqlen, "window_attention")
-    _lib.check_seq(_lib_for(proj).e2h_seq_window_attention(ctypes.byref(a), _stream(proj)), "e2h_seq_window_attention")
+    lib = _lib_for(proj)
+    n = max(0, lib.e2h_seq_window_attention_scratch_bytes(ctypes.byref(a))) if seqlen == 1 else 0  # a refused call is refused below
+    scratch = torch.empty((n,), dtype=torch.uint8, device=proj.device) if n else None
+    _lib.check_seq(lib.e2h_seq_window_attention_split(ctypes.byref(a), _p(scratch), n, _stream(proj)), "e2h_seq_window_attention")
 
 
 def _scratch(args, query, like):

@@ -127,6 +127,12 @@ typedef struct {
 } e2h_window_attention_args;
 int e2h_seq_window_attention(const e2h_window_attention_args *a, void *stream);
 
+/* The same for callers with scratch memory: one-token calls of few sequences share their keys among several workgroups, whose sums meet in
+ * scratch_bytes of it (4-byte aligned; e2h_seq_window_attention_scratch_bytes says how many are used, 0: none, negative: the call is
+ * refused).  With less, or NULL, they run as above. */
+int64_t e2h_seq_window_attention_scratch_bytes(const e2h_window_attention_args *a);
+int e2h_seq_window_attention_split(const e2h_window_attention_args *a, void *scratch, int64_t scratch_bytes, void *stream);
+
 /* HGRN2.  Per head: q = silu(q_proj), f = lower + (1 - lower) sigmoid(f_proj + f_bias), S = diag(f) S + (1 - f) v^T,
  * o = S^T q; result out_scale * o / rms(o) * norm_weight at out + row * ld_out + out_off. */
 typedef struct {

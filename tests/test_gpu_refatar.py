@@ -205,6 +205,22 @@ def test_decode_attention_over_many_keys_with_either_wave_count(waves):
     assert rel(got[-1], want[-1]) < 1e-2
 
 
+@pytest.mark.parametrize("t,window,keep,waves", [(545, 4000, 0, 8), (769, 700, 3, 8), (1057, 2000, 0, 4), (2050, 1030, 30, 8)])
+@pytest.mark.parametrize("h,g,d,dv", [(4, 2, 64, 64), (5, 1, 20, 12), (2, 2, 136, 200)])
+def test_decode_attention_shared_by_workgroups(t, window, keep, waves, h, g, d, dv):
+    """A step whose keys are split: sequences of two keys, of one tile and a remainder, and of all positions side by side; the far keys
+    carry much of the weight.  The float32 sums are combined in another order only, so the tolerance is that of the whole step."""
+    _lib.set_seq_option("attention_decode_waves", waves)
+    pads = [0, t - 2, t - 33]
+    q, k, v, gate = (randn(3, t, n, s, seed=i, dtype=torch.bfloat16) for i, (n, s) in enumerate(((h, d), (g, d), (g, dv), (h, dv))))
+    k[0, 5:40, 0] += 0.5 * q[0, -1, 0]
+    first = torch.tensor(pads, device=DEV)
+    got = f64(run_attention(q, k, v, gate, torch.bfloat16, 0.3, window, keep, [t - 1, 1], first=first))
+    for i, f in enumerate(pads):
+        want = ro.window_attention(f64(q)[i, f:], f64(k)[i, f:], f64(v)[i, f:], 0.3, window, keep)[-1] * ro.sigmoid(f64(gate)[i, -1])
+        assert rel(got[i, -1], want) < 1e-2, (i, f)
+
+
 # ---- HGRN2 -----------------------------------------------------------------------------------------------------------------------
 
 def run_hgrn2(q, f, v, fb, low, nw, eps, dtype, portions, first=None, state=None, out_scale=1.0):
