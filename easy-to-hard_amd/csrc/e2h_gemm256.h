@@ -1,0 +1,189 @@
+// Matrix product of two 16-bit operands, 256 x 256 outputs per tile: the loop that the many-row kernels share.
+//
+//   out[row][col] = sum_k x[row][k] w[col][k]      x rows and w rows of K values, K a multiple of 64 and at least 192
+//
+// What bounds it: the matrix pipelines, and with all of them busy the chip's power (1.6 - 1.75 GHz instead of 2.4), so that everything
+// that costs energy beside the products costs time.  One workgroup per CU of four waves, each 128 x 128 outputs in 256 accumulation registers
+// (an LDS read of 16 values per lane feeds 64 products of 16 x 16 x 32; 256 x 64 per wave would read 1.25 times as much).  Operands reach LDS by
+// 16-byte loads that write LDS directly, in units of 256 rows x 64 k (32 KB, whole 128-byte lines: units of 32 k, which ask the L2 for every line
+// twice, ran at 1300 TFLOP/s where this runs at 1420 - 1520).  All 160 KB of LDS are a ring of five such units, x_0 w_0 x_1 w_1 ..: a unit's place
+// is free as soon as the fragments of its second half are in registers, so that a chunk of 64 k is requested two chunks ahead of its use.
+// One barrier per chunk, in its middle.  The walk over tiles is one pipeline: the first chunks of a tile are on their way while the
+// one before it is finished and stored.
+//   8192 rows, bfloat16: 12288 x 4096 545 us (1510 TFLOP/s), 4096 x 11008 480 us (1540).
+//
+// 16-byte pieces of a row stand at position piece ^ f(row) of its 128 bytes, f chosen so that the 16 rows of a fragment read fall on different
+// bank groups: rows of x in order, f = (row / 2) % 8; of w the fragments i = 2 p and 2 p + 1 of a wave hold columns 32 p + 8 (r / 4) + 4 (i % 2) + r % 4
+// (r: the fragment's row), so that a lane ends up with eight neighbouring outputs of a row, f = (column / 2) % 2 + 2 ((column / 8) % 4).
+#pragma once
+
+#include "e2h_common.h"
+
+namespace e2h {
+namespace gemm256 {
+
+constexpr int kSide = 256, kLeastK = 192;
+constexpr int kStores = 32;  // vector stores of a wave per tile, exactly (see below)
+constexpr uint32_t kUnit = 256 * 128, kRing = 5 * kUnit;
+constexpr uint32_t kNowhere = 0xFFFFFFF0u;  // an offset past every buffer: the store is dropped
+
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(3))) void lds_void_t;
+
+// In-place accumulation on an accumulation register: left to itself the register allocator, with all 256 of them taken, moves
+// accumulators about inside the loop (twice the time).
+template <bool F16>
+__device__ __forceinline__ void mma(f32x4_t &d, u32x4_t a, u32x4_t b) {
+  if constexpr (F16) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(d) : "v"(a), "v"(b));
+  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(d) : "v"(a), "v"(b));
+}
+
+// P names the tiles and what surrounds them.  P::Tile holds uniform values.
+//   bool first(Tile &), bool next(Tile &)     the workgroup's tiles, false: no more
+//   int chunks()                              K / 64
+//   rsrc x_rsrc(Tile), w_rsrc(Tile)           the operands
+//   Fetch, fetch(Tile, lane, wave, Fetch &)   what the two below need from memory (requested a tile ahead)
+//   uint32_t x_at(Tile, Fetch, i, row), w_at(Tile, col)   byte offset of row (0 .. 255, the i-th of this lane) and column of the tile, inside the buffer
+//   Dest, dest(Tile, row of the lane's first output, col, Dest &)   what store needs from memory
+//   store(Tile, Dest, j, p, row, col, v)      stores the eight outputs (row, col .. col + 7), one vector store in every case
+template <bool F16, class P>
+__device__ __forceinline__ void walk(P &p, uint8_t *lds) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave & 1, wn = wave >> 1, chunks = p.chunks();
+  typename P::Tile cur, nxt;
+  if (!p.first(cur)) return;  // uniform, before any barrier
+
+  // loads: wave w brings the 1 KB blocks w, w + 4, .. of a unit (8 rows each), lane l position l % 8 of row l / 8
+  const uint32_t xpiece = ((lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7)) * 16, wpiece = ((lane & 7) ^ (((lane >> 4) & 1) + 2 * wave)) * 16;
+  uint32_t xsrc[8], wsrc[8];
+  typename P::Fetch fetched;
+  __amdgpu_buffer_rsrc_t xr = p.x_rsrc(cur), wr = p.w_rsrc(cur);
+  auto aim_x = [&](const typename P::Tile &t) {
+    xr = p.x_rsrc(t);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) xsrc[i] = p.x_at(t, fetched, i, 8 * (wave + 4 * i) + (lane >> 3)) + xpiece;
+  };
+  auto aim_w = [&](const typename P::Tile &t) {
+    wr = p.w_rsrc(t);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) wsrc[i] = p.w_at(t, 8 * (wave + 4 * i) + (lane >> 3)) + wpiece;
+  };
+  auto load_x = [&](int chunk, uint32_t unit, int i) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t *)(lds + unit + (wave + 4 * i) * 1024), 16, xsrc[i], static_cast<uint32_t>(chunk) * 128, 0, 0);
+  };
+  auto load_w = [&](int chunk, uint32_t unit, int i) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_t *)(lds + unit + (wave + 4 * i) * 1024), 16, wsrc[i], static_cast<uint32_t>(chunk) * 128, 0, 0);
+  };
+
+  // fragments of a half chunk: lane (h, n) reads piece 4 s + h of its rows
+  const int n = lane & 15, h = lane >> 4;
+  const uint32_t xa = (128 * wm + n) * 128 + ((h ^ ((n >> 1) & 7)) << 4);
+  const uint32_t wa = (128 * wn + 8 * (n >> 2) + (n & 3)) * 128 + ((h ^ (((n >> 1) & 1) + 2 * (n >> 2))) << 4);
+  u32x4_t xf[2][8], wf[2][8];
+  auto read_x = [&](uint32_t unit, int s, int i) { return *reinterpret_cast<const u32x4_t *>(lds + unit + (xa ^ (64 * s)) + i * 2048); };
+  auto read_w = [&](uint32_t unit, int s, int i) {
+    return *reinterpret_cast<const u32x4_t *>(lds + unit + (wa ^ (64 * s)) + (i >> 1) * 4096 + (i & 1) * 512);
+  };
+  auto after = [](uint32_t unit) { return unit + kUnit == kRing ? 0u : unit + kUnit; };
+
+  p.fetch(cur, lane, wave, fetched);
+  aim_x(cur);
+  aim_w(cur);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) load_x(0, 0, i);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) load_w(0, kUnit, i);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) load_x(1, 2 * kUnit, i);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) load_w(1, 3 * kUnit, i);
+  asm volatile("s_waitcnt vmcnt(16)\n\ts_barrier" ::: "memory");
+  nxt = cur;
+  bool more = p.next(nxt);
+  if (more) p.fetch(nxt, lane, wave, fetched);
+  typename P::Dest dest;
+  const int row0 = 128 * wm + n, col0 = 128 * wn + 8 * h;
+  p.dest(cur, row0, col0, dest);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) xf[0][i] = read_x(0, 0, i);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) wf[0][i] = read_w(kUnit, 0, i);
+  f32x4_t acc[8][8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  uint32_t xu = 0, wu = kUnit, loading = 3 * kUnit;
+  int ahead = 2;         // the chunk that the next loads bring, of this tile or (once it has come round) of the next one
+  bool stored = false;   // this tile's first chunk has the stores of another one in front of its loads
+  while (true) {
+#pragma unroll
+    for (int i = 0; i < 64; ++i) asm volatile("" : "+a"(acc[i / 8][i % 8]));
+    asm volatile("s_nop 7");  // the accumulators are set by here, and the products may read them
+    for (int c = 0; c < chunks; ++c) {
+      const uint32_t nxu = after(wu), nwu = after(nxu);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        if (s == 1) {
+          // The next chunk has landed once at most what was issued behind it is open: the eight loads of the first half, and in a tile's first
+          // chunk the stores of the tile before it.  Behind the barrier nobody reads this chunk's units any more.
+          if (c == 0 && stored) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(8 + kStores) : "memory");
+          else asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        }
+        loading = after(loading);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            mma<F16>(acc[i][j], wf[s][i], xf[s][j]);
+            const int slot = 8 * i + j, r = slot / 2;
+            if (slot % 2 == 0 && r < 16) {  // the next half's fragments, in the order of their use
+              if (r == 0) wf[s ^ 1][0] = read_w(s ? nwu : wu, s ^ 1, 0);
+              else if (r <= 8) xf[s ^ 1][r - 1] = read_x(s ? nxu : xu, s ^ 1, r - 1);
+              else wf[s ^ 1][r - 8] = read_w(s ? nwu : wu, s ^ 1, r - 8);
+            }
+            if (slot % 4 == 1 && slot < 32) {
+              if (s == 0) load_x(ahead, loading, slot / 4);
+              else load_w(ahead, loading, slot / 4);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        // behind the last tile the loads go on reading it: nobody uses them
+        if (s == 0 && ahead + 1 == chunks && more) aim_x(nxt);
+        if (s == 1 && ++ahead == chunks) {
+          ahead = 0;
+          if (more) aim_w(nxt);
+        }
+      }
+      xu = nxu;
+      wu = nwu;
+    }
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last products' results can be read
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        asm volatile("" : "+a"(acc[2 * q][j]), "+a"(acc[2 * q + 1][j]));  // read here: all 256 at once would not fit
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = acc[2 * q + (e >> 2)][j][e & 3];
+        acc[2 * q][j] = acc[2 * q + 1][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        p.store(cur, dest, j, q, row0 + 16 * j, col0 + 32 * q, v);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    if (!more) break;
+    stored = true;
+    cur = nxt;
+    more = p.next(nxt);
+    if (more) p.fetch(nxt, lane, wave, fetched);
+    p.dest(cur, row0, col0, dest);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // loads past the last tile must land before the workgroup gives its LDS away
+}
+#endif
+
+}  // namespace gemm256
+}  // namespace e2h

@@ -9,6 +9,7 @@
 //               brought into LDS by direct 16-byte loads (token rows gathered by the loads themselves).
 //   otherwise   expert_plain_kernel on the vector units (float32, sizes that are not multiples of 8).
 // Matrix products are transposed (weights are the A operand), so a lane holds four neighbouring outputs of one token.
+#include "e2h_gemm256.h"
 #include "e2h_seq_common.h"
 
 namespace e2h {
@@ -213,27 +214,31 @@ struct Tile {
   int expert, base, count, m, n;  // rows base .. base + count - 1 of the sorted order; tile m of them, column tile n; expert < 0: none
 };
 
-__device__ __forceinline__ Tile find_tile(const int32_t *offsets, int experts, int rows, int tile_rows, int n_tiles) {
+// tiles of expert e; all tiles
+__device__ __forceinline__ int tiles_of(const int32_t *offsets, int experts, int rows, int tile_rows, int e) {
+  if (e >= experts) return 0;
+  const int n = offsets ? offsets[e + 1] - offsets[e] : rows;
+  return (n + tile_rows - 1) / tile_rows;
+}
+
+__device__ __forceinline__ int count_tiles(const int32_t *offsets, int experts, int rows, int tile_rows, int n_tiles) {
   const int lane = threadIdx.x & 63;
-  auto tiles_of = [&](int e) {
-    if (e >= experts) return 0;
-    const int n = offsets ? offsets[e + 1] - offsets[e] : rows;
-    return (n + tile_rows - 1) / tile_rows;
-  };
   int total = 0;
   for (int e0 = 0; e0 < experts; e0 += 64) {
-    int v = tiles_of(e0 + lane);
+    int v = tiles_of(offsets, experts, rows, tile_rows, e0 + lane);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
     total += v;
   }
-  total = __builtin_amdgcn_readfirstlane(total) * n_tiles;
-  const int chunk = (total + 7) / 8, slot = blockIdx.x >> 3;
-  int t = static_cast<int>(blockIdx.x & 7) * chunk + slot;
+  return __builtin_amdgcn_readfirstlane(total) * n_tiles;
+}
+
+// tile t, below the total
+__device__ __forceinline__ Tile tile_at(const int32_t *offsets, int experts, int rows, int tile_rows, int n_tiles, int t) {
+  const int lane = threadIdx.x & 63;
   Tile r = {-1, 0, 0, 0, 0};
-  if (slot >= chunk || t >= total) return r;
   for (int e0 = 0; e0 < experts; e0 += 64) {
-    const int mt = tiles_of(e0 + lane);
+    const int mt = tiles_of(offsets, experts, rows, tile_rows, e0 + lane);
     int upto = mt;  // tiles of experts e0 .. e0 + lane
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -257,6 +262,13 @@ __device__ __forceinline__ Tile find_tile(const int32_t *offsets, int experts, i
   // the same in all lanes, which the compiler cannot know
   return {__builtin_amdgcn_readfirstlane(r.expert), __builtin_amdgcn_readfirstlane(r.base), __builtin_amdgcn_readfirstlane(r.count),
           __builtin_amdgcn_readfirstlane(r.m), __builtin_amdgcn_readfirstlane(r.n)};
+}
+
+__device__ __forceinline__ Tile find_tile(const int32_t *offsets, int experts, int rows, int tile_rows, int n_tiles) {
+  const int total = count_tiles(offsets, experts, rows, tile_rows, n_tiles);
+  const int chunk = (total + 7) / 8, slot = blockIdx.x >> 3, t = static_cast<int>(blockIdx.x & 7) * chunk + slot;
+  if (slot >= chunk || t >= total) return {-1, 0, 0, 0, 0};
+  return tile_at(offsets, experts, rows, tile_rows, n_tiles, t);
 }
 
 // One matrix product over sorted rows: y[to(p)] = f(weight[e] x[from(p)]).  UP: x row = slot / top, y row = p, f = squared ReLU;
@@ -374,6 +386,87 @@ __global__ __launch_bounds__(256, 2) void expert_tiles_kernel(const Product p) {
       if (n < N) store4(y + n, v);
     }
   }
+}
+
+// The same on tiles of 256 x 256 (e2h_gemm256.h): a workgroup per CU walks its XCD's tiles.  8192 rows x 8 of 64 experts, 4096 x 1024:
+// both products 985 us (1116 TFLOP/s), 1301 on the tiles above; a ninth of the products are for rows past an expert's last one, and the last
+// round of tiles fills half the chip in the up product.
+template <bool UP>
+struct ExpertWalk {
+  typedef e2h::Tile Tile;
+  const Product &p;
+  int t, end, stride;
+  __amdgpu_buffer_rsrc_t y;
+
+  __device__ __forceinline__ explicit ExpertWalk(const Product &product) : p(product) {
+    const int total = count_tiles(p.offsets, p.experts, p.rows, gemm256::kSide, p.n_tiles), xcd = blockIdx.x & 7;
+    stride = static_cast<int>(gridDim.x >> 3);
+    end = static_cast<int>(static_cast<int64_t>(total) * (xcd + 1) / 8);
+    t = static_cast<int>(static_cast<int64_t>(total) * xcd / 8) + static_cast<int>(blockIdx.x >> 3) - stride;
+    y = make_rsrc(p.y, static_cast<uint32_t>(static_cast<size_t>(p.rows) * p.N * 2));
+  }
+  __device__ __forceinline__ bool next(Tile &tile) {
+    t += stride;
+    if (t >= end) return false;
+    tile = tile_at(p.offsets, p.experts, p.rows, gemm256::kSide, p.n_tiles, t);
+    return true;
+  }
+  __device__ __forceinline__ bool first(Tile &tile) { return next(tile); }
+  __device__ __forceinline__ int chunks() const { return p.K / 64; }
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t x_rsrc(const Tile &) const { return make_rsrc(p.x, static_cast<uint32_t>(p.x_rows * p.K * 2)); }
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t w_rsrc(const Tile &tile) const {
+    return make_rsrc(static_cast<const bf16_t *>(p.weight) + tile.expert * p.weight_stride, static_cast<uint32_t>(static_cast<size_t>(p.N) * p.K * 2));
+  }
+  __device__ __forceinline__ int sorted_row(const Tile &tile, int row) const {
+    const int m = tile.m * gemm256::kSide + row;
+    return tile.base + (m < tile.count ? m : tile.count - 1);
+  }
+  struct Fetch {
+    int slot[8];
+  };
+  __device__ __forceinline__ void fetch(const Tile &tile, int lane, int wave, Fetch &f) const {
+    if (!UP) return;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f.slot[i] = slot_of(p, sorted_row(tile, 8 * (wave + 4 * i) + (lane >> 3)));
+  }
+  __device__ __forceinline__ uint32_t x_at(const Tile &tile, const Fetch &f, int i, int row) const {
+    return static_cast<uint32_t>(UP ? f.slot[i] / p.top : sorted_row(tile, row)) * static_cast<uint32_t>(p.K) * 2;
+  }
+  __device__ __forceinline__ uint32_t w_at(const Tile &tile, int col) const {
+    const int n = tile.n * gemm256::kSide + col;
+    return static_cast<uint32_t>(n < p.N ? n : p.N - 1) * static_cast<uint32_t>(p.K) * 2;
+  }
+  struct Dest {
+    int slot[UP ? 1 : 8];
+  };
+  __device__ __forceinline__ void dest(const Tile &tile, int row, int, Dest &d) const {
+    if (UP) return;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) d.slot[UP ? 0 : j] = slot_of(p, sorted_row(tile, row + 16 * j));
+  }
+  __device__ __forceinline__ void store(const Tile &tile, const Dest &d, int j, int, int row, int col, float (&v)[8]) const {
+    if (UP) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float r = fmaxf(v[e], 0.f);
+        v[e] = r * r;
+      }
+    }
+    const int n = tile.n * gemm256::kSide + col, out = UP ? tile.base + tile.m * gemm256::kSide + row : d.slot[UP ? 0 : j];
+    const uint32_t at = (static_cast<uint32_t>(out) * static_cast<uint32_t>(p.N) + static_cast<uint32_t>(n)) * 2;
+    const bool there = tile.m * gemm256::kSide + row < tile.count && n < p.N;
+    __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]), pack_bf16(v[4], v[5]), pack_bf16(v[6], v[7])}, y,
+                                           there ? at : gemm256::kNowhere, 0, 0);
+  }
+};
+
+template <bool UP>
+__global__ __launch_bounds__(256, 1) void expert_big_tiles_kernel(const Product p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[gemm256::kRing];
+  ExpertWalk<UP> tiles(p);
+  gemm256::walk<false>(tiles, lds);
+#endif
 }
 
 // 32 rows x 32 columns per workgroup, float32 products
@@ -559,10 +652,22 @@ int check_experts(const e2h_experts_args &a) {
   return E2H_OK;
 }
 
+// 256-row tiles: from 104 rows per expert on, where an expert's second tile of 128 rows begins to cost (64 experts, 4096 x 1024: 80 rows each 275 us with
+// tiles of 128 and 295 with 256, 96 278 and 288, 112 349 and 303, 256 450 and 386, 1024 1301 and 985), and with enough of them for half the CUs,
+// below which two workgroups per CU of the other form divide the work better.
+bool big_tiles_pay(const Product &p) {
+  const int64_t tiles = (static_cast<int64_t>(p.rows) / gemm256::kSide + (p.experts + 1) / 2) * p.n_tiles;
+  return p.K % 64 == 0 && p.K >= gemm256::kLeastK && static_cast<int64_t>(p.rows) * p.N <= static_cast<int64_t>(UINT32_MAX) / 2 - 16 && p.rows >= 104LL * p.experts && tiles >= 128;
+}
+
 template <bool UP>
 void launch_product(Product p, int form, bool bf16, hipStream_t s) {
   const int cols = form == kTiles ? kTileCols : 32, side = form == kTiles ? kTileRows : 32;
   p.n_tiles = (p.N + cols - 1) / cols;
+  if (form == kTiles && big_tiles_pay(p)) {
+    hipLaunchKernelGGL((expert_big_tiles_kernel<UP>), dim3(256), dim3(256), 0, s, p);
+    return;
+  }
   const int64_t tiles = (static_cast<int64_t>(p.rows) / side + p.experts) * p.n_tiles;  // at least one per expert and begun block of rows
   const dim3 grid(static_cast<unsigned>((tiles + 7) / 8 * 8)), block(256);
   if (form == kTiles) hipLaunchKernelGGL((expert_tiles_kernel<UP>), grid, block, 0, s, p);

@@ -292,6 +292,25 @@ def test_experts(dtype, form, rows, width, n, top, ff, shared):
         assert rel(f64(sh), want_experts(x, one, su[None], sd[None])) < tol
 
 
+@pytest.mark.parametrize("width,ff,n,counts", [
+    (192, 16392, 2, (1, 255)),                      # the shortest K of the 256-row tiles, a last column tile of eight columns; then K = 16392 on the others
+    (4096, 192, 8, (0, 1, 256, 257, 513, 15, 640, 300)),
+    (8192, 256, 4, (700, 2, 0, 258)),
+    (320, 640, 70, (731,) * 10 + (0,) * 59 + (40,)),
+])
+def test_experts_on_256_row_tiles(width, ff, n, counts):
+    """Lists that end at, before and behind a tile's last row, empty ones, and none at all; chosen by the sizes alone.  Sums of K products of
+    random signs lie within a few rounding errors of their terms, so the tolerance is that of the bfloat16 results between and behind the products."""
+    top = 2
+    chosen = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])
+    chosen = chosen[torch.randperm(len(chosen), generator=torch.Generator().manual_seed(7))][: len(chosen) // top * top].reshape(-1, top).to(torch.int32).to(DEV)
+    x, up, down = randn(len(chosen), width, seed=1, dtype=torch.bfloat16), randn(n, ff, width, seed=2, std=width ** -0.5, dtype=torch.bfloat16), randn(
+        n, width, ff, seed=3, std=ff ** -0.5, dtype=torch.bfloat16)
+    assert chosen.numel() > 0
+    _lib.set_seq_option("expert_form", 3)
+    assert rel(f64(seq_ops.experts(x, chosen, up, down)[0]), want_experts(x, chosen, up, down)) < 1.2e-2
+
+
 @pytest.mark.parametrize("form", [1, 2, 3])
 def test_experts_with_uneven_loads(form):
     """All rows at one expert, most experts unused, a row that repeats an expert, and an index that is no expert."""
