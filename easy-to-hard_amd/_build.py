@@ -18,7 +18,7 @@ CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libe2h_quant.so"
 SEQ_LIB_PATH = PKG_DIR / "libe2h_seq.so"
 
-SOURCES = ["e2h_abi.hip", "e2h_quantize.hip", "e2h_int4_mm.hip", "e2h_int4_staged.hip", "e2h_int8_mm.hip", "e2h_int8_stream.hip", "e2h_int4_gemm.hip", "e2h_int4_gemm128.hip", "e2h_int8_gemm.hip", "e2h_attention.hip", "e2h_sample.hip", "e2h_probe.hip"]
+SOURCES = ["e2h_abi.hip", "e2h_quantize.hip", "e2h_int4_mm.hip", "e2h_int4_staged.hip", "e2h_int8_mm.hip", "e2h_int8_stream.hip", "e2h_int4_gemm.hip", "e2h_int4_gemm128.hip", "e2h_int8_gemm.hip", "e2h_unpacked_gemm.hip", "e2h_attention.hip", "e2h_sample.hip", "e2h_probe.hip"]
 
 SEQ_SOURCES = ["e2h_seq_norm.hip", "e2h_seq_linear.hip", "e2h_seq_attention.hip", "e2h_seq_hgrn2.hip", "e2h_seq_delta.hip", "e2h_seq_moe.hip"]
 

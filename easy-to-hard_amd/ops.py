@@ -116,6 +116,22 @@ def int8_quantize_per_channel(w):
     return q, scales
 
 
+_UNPACK_ROWS = 1024  # no smaller call is offered scratch memory
+
+
+def _unpacked_weight(query, m, n, k, device):
+    """Scratch for the 16-bit weights of a call with many rows, or None: the sizes are not for that form, or there is no memory left for it."""
+    if m < _UNPACK_ROWS:
+        return None
+    need = query(m, n, k)
+    if need <= 0:
+        return None
+    try:
+        return torch.empty((need,), dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def _int8_mm_impl(x, q, scales):
     _need_gpu(x, q, scales)
     if x.dtype != torch.bfloat16 or q.dtype != torch.int8 or scales.dtype != torch.bfloat16:
@@ -130,7 +146,13 @@ def _int8_mm_impl(x, q, scales):
     if m == 0:
         return y
     ws = _workspace(x.device)  # no int8 kernel uses it, but a first eager call of either kind is what a later capture of int4 calls relies on
-    rc = _lib_for(x).e2h_int8_mm(_ptr(x), _ptr(q), _ptr(scales), _ptr(y), m, n, k, _ptr(ws), ws.numel(), _stream(x))
+    lib = _lib_for(x)
+    unpacked = _unpacked_weight(lib.e2h_int8_mm_scratch_bytes, m, n, k, x.device)
+    if unpacked is not None:
+        rc = lib.e2h_int8_mm_scratch(_ptr(x), _ptr(q), _ptr(scales), _ptr(y), m, n, k, _ptr(unpacked), unpacked.numel(), _stream(x))
+        _lib.check(rc, "e2h_int8_mm_scratch")
+        return y
+    rc = lib.e2h_int8_mm(_ptr(x), _ptr(q), _ptr(scales), _ptr(y), m, n, k, _ptr(ws), ws.numel(), _stream(x))
     _lib.check(rc, "e2h_int8_mm")
     return y
 

@@ -72,6 +72,13 @@ int e2h_int8_quantize_per_channel(const void *w, int w_is_bf16, int8_t *q, float
 int e2h_int8_mm(const uint16_t *x, const int8_t *q, const uint16_t *scales, uint16_t *y, int64_t m,
                 int64_t n, int64_t k, void *workspace, int64_t workspace_bytes, void *stream);
 
+/* The same for callers with memory to spare: over thousands of rows the weights are first unpacked to bfloat16 in `scratch` (16-byte aligned), of which
+ * e2h_int8_mm_scratch_bytes says how much is used (0: this shape runs as above).  With less, or where x, q, scales or y is not 16-byte
+ * aligned, the call is e2h_int8_mm. */
+int64_t e2h_int8_mm_scratch_bytes(int64_t m, int64_t n, int64_t k);
+int e2h_int8_mm_scratch(const uint16_t *x, const int8_t *q, const uint16_t *scales, uint16_t *y, int64_t m, int64_t n, int64_t k,
+                        void *scratch, int64_t scratch_bytes, void *stream);
+
 /* ------------------------------------------------------------------------------------------------
  * int4, group-wise asymmetric
  * ---------------------------------------------------------------------------------------------- */

@@ -489,6 +489,33 @@ def test_int8_many_rows_at_the_reward_scoring_size():
     y_int = qo.int8_linear_reference_rounding(bf16_to_np(x[-3:]), q, s)
     assert np.array_equal(bf16_to_np(y[-3:].cpu()), y_int)
 
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(4100, 4104, 384), (2304, 8456, 256), (70000, 264, 256), (70000, 8, 256), (1040, 16392, 640), (3100, 5128, 1024)])
+def test_int8_unpacked_weights_match_the_other_kernels_bit_for_bit(m, n, k):
+    """Sizes at which the weights are unpacked to bfloat16 first: the shortest K, odd chunk counts, ragged last tiles down to eight columns and four rows, more tiles
+    than CUs.  Integer activations, so every partial sum is exact; the same call without scratch memory and with misaligned rows takes the other kernels."""
+    lib = _lib.load()
+    q, s, q_d, s_d = _int8_case(n, k, seed=m + k)
+    q = q.copy()
+    q[0, :4] = (-128, 127, -128, 127)
+    q_d = torch.from_numpy(q).to(DEV)
+    need = lib.e2h_int8_mm_scratch_bytes(m, n, k)
+    assert need == 2 * n * k
+    x = torch.randint(-2, 3, (m, k), generator=torch.Generator().manual_seed(5)).to(torch.bfloat16)
+    x_d, scratch = x.to(DEV), torch.empty((need,), dtype=torch.uint8, device=DEV)
+    y = ops.int8_mm_direct(x_d, q_d, s_d)
+    for given in (need, need - 16, 0):
+        z = torch.full_like(y, float("nan"))
+        rc = lib.e2h_int8_mm_scratch(ops._ptr(x_d), ops._ptr(q_d), ops._ptr(s_d), ops._ptr(z), m, n, k, ops._ptr(scratch) if given else None, given, ops._stream(x_d))
+        assert rc == 0 and torch.equal(y, z)
+    shifted = torch.empty((m * n + 8,), dtype=torch.bfloat16, device=DEV)[1:1 + m * n].view(m, n)
+    rc = lib.e2h_int8_mm_scratch(ops._ptr(x_d), ops._ptr(q_d), ops._ptr(s_d), ops._ptr(shifted), m, n, k, ops._ptr(scratch), need, ops._stream(x_d))
+    assert rc == 0 and torch.equal(y, shifted)
+    rows = np.r_[0:64, 255:258, m - 70:m]
+    assert np.array_equal(bf16_to_np(y.cpu())[rows], qo.int8_linear_reference_rounding(bf16_to_np(x)[rows], q, s))
+
+
 @pytest.mark.parametrize("g", [32, 64, 128])
 @pytest.mark.parametrize("m,n,k", [(300, 264, 512), (1000, 520, 256), (257, 136, 768), (257, 136, 384), (512, 4096, 4096)])
 def test_int4_gemm128_dequantizing_kernel_matches_oracle_and_32x32_tile_kernel(m, n, k, g):
