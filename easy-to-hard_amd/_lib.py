@@ -16,6 +16,8 @@ _SIGNATURES = {
     "e2h_status_string": (c_char_p, [c_int]),
     "e2h_set_option": (c_int, [c_char_p, c_int]),
     "e2h_int8_quantize_per_channel": (c_int, [_P, c_int, _P, _P, _P, c_int64, c_int64, _P]),
+    "e2h_int4_mm_scratch_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int, c_int]),
+    "e2h_int4_mm_scratch": (c_int, [_P, _P, _P, _P, c_int64, c_int64, c_int64, c_int, c_int, _P, c_int64, _P, c_int64, _P]),
     "e2h_int8_mm_scratch_bytes": (c_int64, [c_int64, c_int64, c_int64]),
     "e2h_int8_mm_scratch": (c_int, [_P, _P, _P, _P, c_int64, c_int64, c_int64, _P, c_int64, _P]),
     "e2h_int8_mm": (c_int, [_P, _P, _P, _P, c_int64, c_int64, c_int64, _P, c_int64, _P]),

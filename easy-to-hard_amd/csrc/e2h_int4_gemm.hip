@@ -77,6 +77,7 @@ struct GemmArgs {
   float *partials;  // [S][M][N] when K is shared, else null
   const float *xsum;
   int xsum_stride, M, N, K, n_col_blocks, cbx;
+  const int *run_if;  // not null: nothing is done where it holds zero
 };
 
 // kRT row tiles of 32 per wave: 32 kRT rows x 256 columns per workgroup
@@ -88,6 +89,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
   constexpr bool kGroupSums = G == 32;         // a group's products in registers of their own, scaled when it ends
   __shared__ __attribute__((aligned(1024))) uint8_t lds[kLdsBytes];
   const int M = a.M, N = a.N, K = a.K;
+  if (a.run_if && *a.run_if == 0) return;  // the whole grid
 
   const int xcd = blockIdx.x & 7;
   const int slot = blockIdx.x >> 3;
@@ -527,10 +529,10 @@ void launch_gemm(const GemmArgs &a, int rows, dim3 grid, hipStream_t stream) {
 }
 
 int int4_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint16_t *y, const float *xsum, int xsum_stride,
-              float *partials, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream) {
+              float *partials, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream, const int *run_if) {
   if (K % 128 != 0 || N % 8 != 0) return E2H_ERR_BAD_SHAPE;
   GemmArgs a = {x, reinterpret_cast<const uint32_t *>(packed), reinterpret_cast<const uint32_t *>(sz), y, shape.slices > 1 ? partials : nullptr,
-                xsum, xsum_stride, M, N, K, (N + kCols - 1) / kCols, 0};
+                xsum, xsum_stride, M, N, K, (N + kCols - 1) / kCols, 0, run_if};
   a.cbx = (a.n_col_blocks + 7) / 8;
   const long long wgs = 8LL * a.cbx * ((M + shape.rows - 1) / shape.rows);
   if (wgs > 0x7FFFFFFFLL) return E2H_ERR_BAD_SHAPE;

@@ -102,14 +102,14 @@ int launch_x_group_sums(const uint16_t *x, float *out, int M, int K, int stride,
 
 // Many-row int4 matmul on 32x32 MFMA tiles (e2h_int4_gemm.hip); xsum as written by launch_x_group_sums.  A workgroup owns `rows` rows;
 // K may be shared by `slices` of them through float32 sums in `partials` ([slices][M][N]; unused with one slice).  int4_gemm_shape picks
-// both, with at most as many slices as fit scratch_bytes.
+// both, with at most as many slices as fit scratch_bytes.  run_if, in device memory: the launch does nothing where it holds zero (one slice only).
 struct Int4GemmShape {
   int rows, slices;
   double us;  // expected time
 };
 Int4GemmShape int4_gemm_shape(int M, int N, int K, int groupsize, int64_t scratch_bytes);
 int int4_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint16_t *y, const float *xsum, int xsum_stride,
-              float *partials, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream);
+              float *partials, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream, const int *run_if = nullptr);
 
 // Many-row int4 matmul, 256 x 256 outputs per workgroup, weights dequantized to bfloat16 on the way into the matrix
 // cores (e2h_int4_gemm128.hip); needs no scratch memory.

@@ -4,11 +4,22 @@
 // int8: y = bf16( bf16( x @ q^T ) * scales ).  A code has at most eight significant bits, so its bfloat16 value is exact and the result is that
 // of the kernels which convert on the way into the matrix cores (e2h_int8_gemm.hip).  Those are bound by the energy and the LDS traffic of 64-byte rows and
 // by conversions beside the products.
+//
+// int4: y = bf16( sum_g sum_{k in g} x[m,k] (s[g,n] (q[n,k] - 8)) + sum_g z[g,n] X[m,g] ), X[m,g] = sum_{k in g} x[m,k].
+// s (q - 8) is an eight-bit significand times a three-bit integer (or eight): it fits the eleven bits of a float16, and x (eight bits) does too.  So both become
+// float16 without rounding, a row of x and a column of weights each in units of a power of two of its own that puts its largest value near the
+// type's end; products are exact and sums float32, as in the kernel that multiplies codes (e2h_int4_gemm.hip: 1.1 - 1.2 PFLOP/s, bound by unpacking and rescaling
+// beside the products).  The zero-point term is three more columns per group: X split exactly into three float16 parts (an infinity of them
+// apart, which the next paragraph keeps out), against z three times.  K grows by 2.4 % at group size 128.
+// What does not fit is multiplied by that other kernel: the passes that unpack raise a flag at a scale or zero that is not finite, would be rounded
+// (2^-28 of its column's largest) or lies outside 2^-48 .. 2^27 or so, at a value of x that is not finite, and at a row of x of which a sixteenth is
+// smaller than 2^-31 of its largest value; up to there what is rounded is less than 2^-39 of the row's largest value, below the rounding of
+// float32 sums that hold it.  With the flag the product's workgroups end at once, without it those of the other kernel do.
 #include <algorithm>
 
 #include "e2h_common.h"
 #include "e2h_gemm256.h"
-#include "e2h_unpacked_gemm.h"
+#include "e2h_int4_unpack.h"
 
 namespace e2h {
 namespace {
@@ -123,6 +134,243 @@ __global__ __launch_bounds__(256, 1) void int8_unpacked_gemm_kernel(const uint16
 #endif
 }
 
+// ---- int4 ------------------------------------------------------------------------------------------------------------------------
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t pack_f16(float lo, float hi) {  // round to nearest even; most callers' values are exact
+  return __builtin_bit_cast(uint32_t, f16x2_t{static_cast<_Float16>(lo), static_cast<_Float16>(hi)});
+}
+
+constexpr int kTopX = 13, kTopW = 15;  // largest value of a row of x: 2^kTopX .. 2^(kTopX + 1); of a column: below 2^kTopW
+constexpr float kWhole = 0x1p-17f;     // eight bits from here on fit a float16
+
+struct Int4Scratch {
+  int *flag;         // [1] this call needs the other kernel
+  int *row_exp;      // [M] x is multiplied by 2^row_exp
+  int *row_flag;     // [M]
+  float *col_unit;   // [N] what one step of a column's sums is worth
+  float *xsum;       // [K / G][stride] group sums, for the other kernel
+  uint32_t *sz;      // [K / 128][N] pairs of group size 256, each twice
+  uint16_t *x, *w;   // [M][KE], [N][KE]
+  int64_t bytes;
+};
+int extended(int K, int G) { return (K + 3 * (K / G) + 63) / 64 * 64; }  // G: 32, 64 or 128
+int sum_stride(int64_t M) { return static_cast<int>((M + 63) / 64 * 64); }
+
+Int4Scratch int4_scratch(uint8_t *base, int64_t M, int64_t N, int64_t K, int groupsize) {
+  const int G = groupsize == 256 ? 128 : groupsize;
+  int64_t at = 0;
+  const auto take = [&](int64_t n) {
+    uint8_t *p = base + at;
+    at += (n + 255) / 256 * 256;
+    return p;
+  };
+  Int4Scratch s;
+  const int64_t KE = extended(static_cast<int>(K), G);
+  s.flag = reinterpret_cast<int *>(take(4));
+  s.row_exp = reinterpret_cast<int *>(take(M * 4));
+  s.row_flag = reinterpret_cast<int *>(take(M * 4));
+  s.col_unit = reinterpret_cast<float *>(take(N * 4));
+  s.xsum = reinterpret_cast<float *>(take(K / G * sum_stride(M) * 4));
+  s.sz = reinterpret_cast<uint32_t *>(take(groupsize == 256 ? K / 128 * N * 4 : 0));
+  s.x = reinterpret_cast<uint16_t *>(take(M * KE * 2));
+  s.w = reinterpret_cast<uint16_t *>(take(N * KE * 2));
+  s.bytes = at;
+  return s;
+}
+
+__device__ __forceinline__ int exponent_of(float v) { return static_cast<int>((__builtin_bit_cast(uint32_t, v) >> 23) & 0xFFu) - 127; }
+
+// One wave per row, two passes over it (the second from the cache): largest value, then float16 values, group sums and their parts.
+// Bound by memory: 8192 x 4096 (133 MB moved) 36 us.
+template <int G>
+__global__ __launch_bounds__(256) void int4_unpack_x_kernel(const uint16_t *__restrict__ x, int M, int K, int KE, Int4Scratch s, int stride) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *s.flag = 0;  // raised by the next launch
+  const int lane = threadIdx.x & 63, m = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (m >= M) return;
+  const u32x4_t *row = reinterpret_cast<const u32x4_t *>(x + static_cast<size_t>(m) * K);
+  const int pieces = K / 8;  // a multiple of 16
+  uint32_t top = 0;
+#pragma unroll 4
+  for (int p = lane; p < pieces; p += 64) {
+    const u32x4_t v = row[p];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const uint32_t lo = v[d] & 0x7FFFu, hi = (v[d] >> 16) & 0x7FFFu;
+      top = top > lo ? top : lo;
+      top = top > hi ? top : hi;
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const uint32_t o = static_cast<uint32_t>(__shfl_xor(static_cast<int>(top), off));
+    top = top > o ? top : o;
+  }
+  const bool finite = top < 0x7F80u;
+  const int up = top == 0 || !finite ? 0 : kTopX - exponent_of(bf16_to_f32(static_cast<uint16_t>(top)));
+  uint16_t *out = s.x + static_cast<size_t>(m) * KE;
+  int lost = 0;
+#pragma unroll 2
+  for (int p = lane; p < pieces; p += 64) {
+    const u32x4_t v = row[p];
+    u32x4_t h;
+    float sum[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const float a = __builtin_bit_cast(float, v[d] << 16), b = __builtin_bit_cast(float, v[d] & 0xFFFF0000u);
+      sum[d] = a + b;
+      const float as = __builtin_ldexpf(a, up), bs = __builtin_ldexpf(b, up);
+      lost += (as != 0.f && __builtin_fabsf(as) < kWhole) + (bs != 0.f && __builtin_fabsf(bs) < kWhole);
+      h[d] = pack_f16(as, bs);
+    }
+    reinterpret_cast<u32x4_t *>(out)[p] = h;
+    float t = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+#pragma unroll
+    for (int off = 1; off < G / 8; off <<= 1) t += __shfl_xor(t, off);  // the lanes of a group are all here or none
+    if (lane % (G / 8) == 0) {
+      const int g = p / (G / 8);
+      s.xsum[static_cast<size_t>(g) * stride + m] = t;
+      const float ts = __builtin_ldexpf(t, up) * (1.0f / G);
+      const _Float16 p0 = static_cast<_Float16>(ts);
+      const float r = ts - static_cast<float>(p0);
+      const _Float16 p1 = static_cast<_Float16>(r), p2 = static_cast<_Float16>(r - static_cast<float>(p1));
+      out[K + 3 * g] = __builtin_bit_cast(uint16_t, p0);
+      out[K + 3 * g + 1] = __builtin_bit_cast(uint16_t, p1);
+      out[K + 3 * g + 2] = __builtin_bit_cast(uint16_t, p2);
+    }
+  }
+  for (int k = K + 3 * (K / G) + lane; k < KE; k += 64) out[k] = 0;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) lost += __shfl_xor(lost, off);
+  if (lane == 0) {
+    s.row_exp[m] = up;
+    s.row_flag[m] = !finite || lost * 16 > K;
+  }
+}
+
+// Sixteen columns and a share of K per workgroup: the columns' units first (every share finds them for itself), then a lane per 16-byte piece
+// of the result.  Bound by memory: 12288 x 4096 (130 MB moved) 36 us.
+template <int G>
+__global__ __launch_bounds__(256) void int4_unpack_w_kernel(const uint32_t *__restrict__ wp, const uint32_t *__restrict__ sz, int twice, int M, int N, int K, int KE,
+                                                            Int4Scratch s) {
+  __shared__ float top_of[16][17];
+  __shared__ int raised;
+  const int groups = K / G, tid = threadIdx.x, col0 = blockIdx.x * 16;
+  if (tid == 0) raised = 0;
+  __syncthreads();
+  // every row's flag, shared among all workgroups
+  int odd = 0;
+  for (int64_t m = (static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x) * 256 + tid; m < M; m += static_cast<int64_t>(gridDim.x) * gridDim.y * 256) odd |= s.row_flag[m];
+  const int c1 = tid & 15, g1 = tid >> 4;
+  const bool live1 = col0 + c1 < N;
+  float top = 0.f;
+  if (live1)
+    for (int g = g1; g < groups; g += 16) {
+      const uint32_t pair = sz[static_cast<size_t>(g >> twice) * N + col0 + c1];
+      const float scale = __builtin_bit_cast(float, pair << 16), zero = __builtin_bit_cast(float, pair & 0xFFFF0000u);
+      odd |= !__builtin_isfinite(scale) || !__builtin_isfinite(zero);
+      top = fmaxf(top, fmaxf(8.f * __builtin_fabsf(scale), static_cast<float>(G) * __builtin_fabsf(zero)));
+    }
+  top_of[c1][g1] = top;
+  __syncthreads();
+  const auto unit_of = [&](int c) {  // the power of two that the column is multiplied by
+    float t = 0.f;
+#pragma unroll
+    for (int g = 0; g < 16; ++g) t = fmaxf(t, top_of[c][g]);
+    return t == 0.f ? 0 : kTopW - 1 - exponent_of(t);
+  };
+  const int up1 = unit_of(c1);
+  odd |= live1 && (up1 < -30 || up1 > 60);
+  if (live1)
+    for (int g = g1; g < groups; g += 16) {
+      const uint32_t pair = sz[static_cast<size_t>(g >> twice) * N + col0 + c1];
+      const float scale = __builtin_bit_cast(float, pair << 16), zero = __builtin_bit_cast(float, pair & 0xFFFF0000u);
+      const float a = __builtin_fabsf(__builtin_ldexpf(scale, up1)), z = __builtin_ldexpf(zero, up1) * static_cast<float>(G);
+      odd |= (scale != 0.f && a < kWhole) || (zero != 0.f && __builtin_fabsf(z) < kWhole);
+      if (blockIdx.y == 0) {
+        uint16_t *ext = s.w + static_cast<size_t>(col0 + c1) * KE + K + 3 * g;
+        ext[0] = ext[1] = ext[2] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(z));
+        if (twice) s.sz[static_cast<size_t>(g) * N + col0 + c1] = pair;
+      }
+    }
+  if (blockIdx.y == 0 && live1) {
+    for (int k = K + 3 * groups + g1; k < KE; k += 16) s.w[static_cast<size_t>(col0 + c1) * KE + k] = 0;
+    if (g1 == 0) s.col_unit[col0 + c1] = __builtin_ldexpf(1.f, -up1);
+  }
+  if (odd) raised = 1;  // any of them: the same value
+  __syncthreads();
+  if (tid == 0 && raised) atomicOr(s.flag, 1);
+
+  // piece (span p, part i) of column c: codes k = 128 b + 32 p + 8 i + 2 j + {0, 1} in nibbles i and i + 4 of word [j][p]
+  const int c = tid >> 4, p = (tid >> 2) & 3, i = tid & 3, col = col0 + c, KT = K >> 7;
+  if (col >= N) return;
+  const int up = unit_of(c);
+  const uint32_t *words = wp + static_cast<size_t>(col >> 3) * KT * 128 + (col & 7) * 16 + p;
+  uint16_t *out = s.w + static_cast<size_t>(col) * KE + 32 * p + 8 * i;
+  const int b1 = static_cast<int>(static_cast<int64_t>(KT) * (blockIdx.y + 1) / gridDim.y);
+#pragma unroll 4
+  for (int b = static_cast<int>(static_cast<int64_t>(KT) * blockIdx.y / gridDim.y); b < b1; ++b) {
+    const int g = (128 * b + 32 * p + 8 * i) / G;
+    const float scale = __builtin_ldexpf(__builtin_bit_cast(float, sz[static_cast<size_t>(g >> twice) * N + col] << 16), up);
+    u32x4_t h;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t w = words[static_cast<size_t>(b) * 128 + 4 * j];
+      const float q0 = static_cast<float>((w >> (4 * i)) & 15u), q1 = static_cast<float>((w >> (4 * i + 16)) & 15u);
+      h[j] = pack_f16(__builtin_fmaf(q0, scale, -8.f * scale), __builtin_fmaf(q1, scale, -8.f * scale));
+    }
+    *reinterpret_cast<u32x4_t *>(out + static_cast<size_t>(b) * 128) = h;
+  }
+}
+
+struct Int4Walk : PlainWalk {
+  const float *col_unit;
+  const int *row_exp;
+  __device__ __forceinline__ Int4Walk(const Int4Scratch &s, uint16_t *y_, int M_, int N_, int KE) : PlainWalk(s.x, s.w, y_, M_, N_, KE), col_unit(s.col_unit), row_exp(s.row_exp) {}
+  struct Dest {
+    f32x4_t unit[4][2];  // of the eight columns of each store of a row
+    int up[8];           // of the rows
+  };
+  __device__ __forceinline__ void dest(const Tile &tile, int row, int col, Dest &d) const {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int n = tile.cb * 256 + col + 32 * q;
+      const f32x4_t *u = reinterpret_cast<const f32x4_t *>(col_unit + (n < N ? n : N - 8));
+      d.unit[q][0] = u[0];
+      d.unit[q][1] = u[1];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int m = tile.rb * 256 + row + 16 * j;
+      d.up[j] = row_exp[m < M ? m : M - 1];
+    }
+  }
+  __device__ __forceinline__ void store(const Tile &tile, const Dest &d, int j, int q, int row, int col, float (&v)[8]) const {
+    u32x4_t out;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = __builtin_ldexpf(v[e] * d.unit[q][e >> 2][e & 3], -d.up[j]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = pack_bf16(v[2 * e], v[2 * e + 1]);
+    __builtin_amdgcn_raw_buffer_store_b128(out, y_rsrc(tile), y_at(tile, row, col), 0, 0);
+  }
+};
+
+__global__ __launch_bounds__(256, 1) void int4_unpacked_gemm_kernel(const Int4Scratch s, uint16_t *y, int M, int N, int KE) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (*s.flag) return;  // the whole grid
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[gemm256::kRing];
+  Int4Walk tiles(s, y, M, N, KE);
+  gemm256::walk<true>(tiles, lds);
+#endif
+}
+
+template <int G>
+void launch_unpack(const uint16_t *x, const uint32_t *wp, const uint32_t *sz, const Int4Scratch &s, int twice, int M, int N, int K, int KE, hipStream_t stream) {
+  hipLaunchKernelGGL(int4_unpack_x_kernel<G>, dim3(static_cast<unsigned>((M + 3) / 4)), dim3(256), 0, stream, x, M, K, KE, s, sum_stride(M));
+  const int cols = (N + 15) / 16, shares = std::max(1, std::min(K / 512, (4096 + cols - 1) / cols));  // at least four blocks of 128 k each
+  hipLaunchKernelGGL(int4_unpack_w_kernel<G>, dim3(static_cast<unsigned>(cols), static_cast<unsigned>(shares)), dim3(256), 0, stream, wp, sz, twice, M, N, K, KE, s);
+}
+
 unsigned grid_of(int64_t M, int64_t N) {
   const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
   return static_cast<unsigned>(8 * std::min<int64_t>(32, (tiles + 7) / 8));
@@ -169,7 +417,54 @@ int int8_unpacked_gemm(const uint16_t *x, const int8_t *q, const uint16_t *scale
   return launch_status();
 }
 
+// Taken where it is the cheaper one, the unpacking (two and a half bytes a weight, four a value of x, at 4.8 TB/s; 8 us of launches) included.  Measured, us, here (codes multiplied
+// in the loop): 8192 rows 12288 x 4096 g128 647 (695), 32000 x 4096 1664 (1793), 12288 x 4096 g32 699 (1056), g256 644; 2048 rows 12288 x 4096 g128 230
+// (204), left to the other form.
+int64_t int4_unpacked_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int inner_k_tiles) {
+  if (inner_k_tiles != 8 || (groupsize != 32 && groupsize != 64 && groupsize != 128 && groupsize != 256)) return 0;
+  const int G = groupsize == 256 ? 128 : groupsize;
+  if (M <= 64 || N < 8 || N % 8 != 0 || K < 256 || K % 128 != 0 || K % groupsize != 0 || M > INT32_MAX / 64 || N > INT32_MAX / 64 || K > INT32_MAX / 64) return 0;
+  const Options &o = options();
+  if (o.int4_no_gemm32 || o.int4_gemm_tile || o.int4_gemm32_min_rows || o.int4_no_xsum || o.int4_k_slices || o.int4_rows_per_wave || o.row_tiles) return 0;  // another form is asked for
+  const int64_t KE = extended(static_cast<int>(K), G);
+  if (M * KE * 2 >= (int64_t{1} << 32) || N * KE * 2 >= (int64_t{1} << 32) || K / G * sum_stride(M) * 4 >= (int64_t{1} << 32)) return 0;
+  const int64_t bytes = int4_scratch(nullptr, M, N, K, groupsize).bytes;
+  const double unpack = (static_cast<double>(N) * static_cast<double>(K) * 2.5 + static_cast<double>(M) * static_cast<double>(K) * 4) / 4.8e6 + 8;
+  const double other = int4_gemm_shape(static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), G, 32 << 20).us * (G == 32 ? 1.3 : 1.0);  // its estimate for group size 32 is that much low
+  return unpacked_cost(M, N, KE, unpack) < other ? bytes : 0;
+}
+
+int int4_unpacked_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *scales_and_zeros, uint16_t *y, int M, int N, int K, int groupsize, void *scratch,
+                       hipStream_t stream) {
+  const Int4Scratch s = int4_scratch(static_cast<uint8_t *>(scratch), M, N, K, groupsize);
+  const int twice = groupsize == 256, G = twice ? 128 : groupsize, KE = extended(K, G);
+  const uint32_t *wp = reinterpret_cast<const uint32_t *>(packed), *sz = reinterpret_cast<const uint32_t *>(scales_and_zeros);
+  switch (G) {
+    case 32: launch_unpack<32>(x, wp, sz, s, twice, M, N, K, KE, stream); break;
+    case 64: launch_unpack<64>(x, wp, sz, s, twice, M, N, K, KE, stream); break;
+    default: launch_unpack<128>(x, wp, sz, s, twice, M, N, K, KE, stream); break;
+  }
+  hipLaunchKernelGGL(int4_unpacked_gemm_kernel, dim3(grid_of(M, N)), dim3(256), 0, stream, s, y, M, N, KE);
+  return int4_gemm(x, packed, twice ? reinterpret_cast<const uint16_t *>(s.sz) : scales_and_zeros, y, s.xsum, sum_stride(M), nullptr, int4_gemm_shape(M, N, K, G, 0), M, N, K,
+                   G, stream, s.flag);
+}
+
 }  // namespace e2h
+
+extern "C" int64_t e2h_int4_mm_scratch_bytes(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles) {
+  return e2h::int4_unpacked_bytes(m, n, k, groupsize, inner_k_tiles);
+}
+
+extern "C" int e2h_int4_mm_scratch(const uint16_t *x, const int32_t *packed, const uint16_t *scales_and_zeros, uint16_t *y, int64_t m, int64_t n, int64_t k, int groupsize,
+                                   int inner_k_tiles, void *workspace, int64_t workspace_bytes, void *scratch, int64_t scratch_bytes, void *stream) {
+  using namespace e2h;
+  if (!x || !packed || !scales_and_zeros || !y) return E2H_ERR_NULL_POINTER;
+  const int64_t need = int4_unpacked_bytes(m, n, k, groupsize, inner_k_tiles);
+  if (!scratch || need == 0 || scratch_bytes < need || !aligned16(x) || !aligned16(packed) || !aligned16(scales_and_zeros) || !aligned16(y) || !aligned16(scratch) ||
+      (workspace && !aligned16(workspace)) || n * k / 2 >= (int64_t{1} << 32) || (k / groupsize) * n * 4 >= (int64_t{1} << 32))
+    return e2h_int4_mm(x, packed, scales_and_zeros, y, m, n, k, groupsize, inner_k_tiles, workspace, workspace_bytes, stream);
+  return int4_unpacked_gemm(x, packed, scales_and_zeros, y, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), groupsize, scratch, static_cast<hipStream_t>(stream));
+}
 
 extern "C" int64_t e2h_int8_mm_scratch_bytes(int64_t m, int64_t n, int64_t k) { return e2h::int8_unpacked_bytes(m, n, k); }
 

@@ -119,11 +119,11 @@ def int8_quantize_per_channel(w):
 _UNPACK_ROWS = 1024  # no smaller call is offered scratch memory
 
 
-def _unpacked_weight(query, m, n, k, device):
+def _unpacked_weight(m, device, query, *sizes):
     """Scratch for the 16-bit weights of a call with many rows, or None: the sizes are not for that form, or there is no memory left for it."""
     if m < _UNPACK_ROWS:
         return None
-    need = query(m, n, k)
+    need = query(m, *sizes)
     if need <= 0:
         return None
     try:
@@ -147,7 +147,7 @@ def _int8_mm_impl(x, q, scales):
         return y
     ws = _workspace(x.device)  # no int8 kernel uses it, but a first eager call of either kind is what a later capture of int4 calls relies on
     lib = _lib_for(x)
-    unpacked = _unpacked_weight(lib.e2h_int8_mm_scratch_bytes, m, n, k, x.device)
+    unpacked = _unpacked_weight(m, x.device, lib.e2h_int8_mm_scratch_bytes, n, k)
     if unpacked is not None:
         rc = lib.e2h_int8_mm_scratch(_ptr(x), _ptr(q), _ptr(scales), _ptr(y), m, n, k, _ptr(unpacked), unpacked.numel(), _stream(x))
         _lib.check(rc, "e2h_int8_mm_scratch")
@@ -313,7 +313,13 @@ def _int4_mm_impl(x, packed, groupsize, scales_and_zeros):
     if m == 0:
         return y
     ws = _workspace(x.device)
-    rc = _lib_for(x).e2h_int4_mm(_ptr(x), _ptr(packed), _ptr(sz), _ptr(y), m, n, k, groupsize, ikt, _ptr(ws), ws.numel(), _stream(x))
+    lib = _lib_for(x)
+    unpacked = _unpacked_weight(m, x.device, lib.e2h_int4_mm_scratch_bytes, n, k, groupsize, ikt)
+    if unpacked is not None:
+        rc = lib.e2h_int4_mm_scratch(_ptr(x), _ptr(packed), _ptr(sz), _ptr(y), m, n, k, groupsize, ikt, _ptr(ws), ws.numel(), _ptr(unpacked), unpacked.numel(), _stream(x))
+        _lib.check(rc, "e2h_int4_mm_scratch")
+        return y
+    rc = lib.e2h_int4_mm(_ptr(x), _ptr(packed), _ptr(sz), _ptr(y), m, n, k, groupsize, ikt, _ptr(ws), ws.numel(), _stream(x))
     _lib.check(rc, "e2h_int4_mm")
     return y
 

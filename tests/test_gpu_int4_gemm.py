@@ -169,3 +169,92 @@ def test_a_row_differs_by_float32_rounding_at_most_between_row_counts(g, n, k):
         part = ops.int4_mm(x[:rows], packed, g, sz)
         assert torch.equal(part, ops.int4_mm(x[:rows], packed, g, sz))
         assert ((part.double() - full[:rows].double()).abs() <= bound[:rows]).all()
+
+
+# ---- weights unpacked to float16 first (csrc/e2h_unpacked_gemm.hip) ---------------------------------------------------------------------
+
+def _unpacked(codes, scale, zero, x, g):
+    """(with scratch memory, without, bytes of it), through the C interface"""
+    lib = _lib.load()
+    packed = torch.from_numpy(qo.int4_tile_pack(codes.numpy(), 8)).to(DEV)
+    sz = torch.stack([scale, zero], dim=-1).to(torch.bfloat16).contiguous().to(DEV)
+    (m, k), n, ws = x.shape, codes.shape[0], ops._workspace(x.device)
+    need = lib.e2h_int4_mm_scratch_bytes(m, n, k, g, 8)
+    scratch = torch.full((max(need, 16),), 255, dtype=torch.uint8, device=DEV)  # a NaN wherever it is read unwritten
+    out = []
+    for given in (need, 0):
+        y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+        rc = lib.e2h_int4_mm_scratch(ops._ptr(x), ops._ptr(packed), ops._ptr(sz), ops._ptr(y), m, n, k, g, 8, ops._ptr(ws), ws.numel(), ops._ptr(scratch), given, ops._stream(x))
+        assert rc == 0
+        out.append(y)
+    return (*out, need)
+
+
+def _double(codes, scale, zero, x, g, rows):
+    n, k = codes.shape
+    w = ((codes.double() - 8).view(n, k // g, g) * scale.double().t()[:, :, None] + zero.double().t()[:, :, None]).view(n, k).to(DEV)
+    return x[rows].double() @ w.t()
+
+
+UNPACKED = [(70000, 264, 256), (70000, 8, 256), (66049, 520, 512)]  # the shortest K, few and ragged columns, a last tile of one row
+
+
+@pytest.mark.parametrize("g", [32, 64, 128, 256])
+@pytest.mark.parametrize("m,n,k", UNPACKED)
+def test_unpacked_weights_are_exact_on_dyadic_operands(m, n, k, g):
+    case = _case(m, n, k, g)
+    got, other, need = _unpacked(*case, g)
+    assert need > 0 and torch.equal(got, other)
+    rows = torch.cat([torch.arange(0, 300), torch.arange(m - 300, m)]).to(DEV)
+    assert torch.equal(got[rows], _double(*case, g, rows).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("g", [32, 128, 256])
+def test_unpacked_weights_round_once(g):
+    """Rows in units from 2^-60 to 2^60 with values 2^-28 .. 1 of them, scales over 2^-20 .. 1 in one column, zeros: all held without rounding, so the error is that of
+    the result's rounding (half a unit of eight significant bits: 2^-8 of the value at most) and of float32 sums of K = 512 terms (2^-24 each)."""
+    m, n, k = 66049, 264, 512
+    gen = torch.Generator().manual_seed(3)
+    codes = torch.randint(0, 16, (n, k), generator=gen, dtype=torch.int32)
+    scale = torch.exp2(torch.rand((k // g, n), generator=gen) * 20 - 20).to(torch.bfloat16).float()
+    zero = (torch.randn((k // g, n), generator=gen) * 8 * scale).to(torch.bfloat16).float()
+    x = torch.exp2(torch.randint(-28, 1, (m, k), generator=gen).float() + torch.randint(-60, 61, (m, 1), generator=gen).float()).to(torch.bfloat16)
+    x = (x * (torch.randint(0, 2, (m, k), generator=gen) * 2 - 1)).to(DEV)
+    x[5] = 0
+    got, _, need = _unpacked(codes, scale, zero, x, g)
+    rows = torch.cat([torch.arange(0, 512), torch.arange(m - 512, m)]).to(DEV)
+    want = _double(codes, scale, zero, x, g, rows)
+    err, size = (got[rows].double() - want).abs(), want.abs()
+    terms = (x[rows].double().abs() @ ((codes.double() - 8).abs().view(n, k // g, g) * scale.double().t()[:, :, None] + zero.double().abs().t()[:, :, None]).view(n, k).to(DEV).t())
+    assert need > 0 and bool((err <= 2**-8 * size + 2**-15 * terms).all()) and bool((got[5] == 0).all())
+    assert (err / terms.clamp(min=1e-300)).mean() < 2**-9
+
+
+@pytest.mark.parametrize("what", ["scale ratio", "infinite scale", "NaN zero", "tiny zero", "large scales", "small scales", "infinite x", "NaN x", "small x"])
+def test_what_float16_does_not_hold_is_left_to_the_other_kernel(what):
+    """bit for bit what the call without scratch memory gives, wherever in x or the weights it stands"""
+    m, n, k, g = 70000, 264, 256, 128
+    codes, scale, zero, x = _case(m, n, k, g)
+    if what == "scale ratio":
+        scale[1, 77], zero[1, 77] = 2.0**-40, 0.0
+    elif what == "infinite scale":
+        scale[0, 263] = float("inf")
+    elif what == "NaN zero":
+        zero[1, 0] = float("nan")
+    elif what == "tiny zero":
+        zero[0, 100] = 2.0**-60
+    elif what == "large scales":
+        scale[:, 3], zero[:, 3] = 2.0**50, 0.0
+    elif what == "small scales":
+        scale[:, 3], zero[:, 3] = 2.0**-70, 0.0
+    elif what == "infinite x":
+        x[m - 1, 255] = float("inf")
+    elif what == "NaN x":
+        x[0, 0] = float("nan")
+    else:
+        x[12345] = 2.0**-50
+        x[12345, 9] = 1.0
+    got, other, need = _unpacked(codes, scale, zero, x, g)
+    assert need > 0
+    same = torch.where(torch.isnan(other), torch.isnan(got), got == other)
+    assert bool(same.all())
