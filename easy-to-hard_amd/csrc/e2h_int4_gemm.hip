@@ -311,8 +311,9 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
         if (s8 == 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(4 + kRT + (NGRP == 1 ? 2 : 2 * NGRP)) : "memory");
         if (s8 == 7) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kRT + 2 * NGRP) : "memory");
         if (s8 == 7) read_w(w_next);
+        if (!kGroupSums) __builtin_amdgcn_sched_barrier(0);  // the counts of the waits above hold for this order of loads
         read_a(af[cur ^ 1], s8 < 3 ? s0 : s8 < 7 ? s1 : s2, (s8 + 1) & 3);
-        __builtin_amdgcn_sched_barrier(0);
+        if (kGroupSums) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int ct = 0; ct < kCT; ++ct) {
           float r = 1.f;
@@ -328,7 +329,6 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
               part[ct][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[cur][rt], wf[cur][ct], s8 % SPG == 0 ? f32x16_t{} : part[ct][rt], 0, 0, 0);
             } else {
               if (s8 % SPG == 0) {
-                __builtin_amdgcn_sched_barrier(0);  // one tile's rescaling under the previous tile's product
 #pragma unroll
                 for (int e = 0; e < 16; ++e) acc[ct][rt][e] *= r;
               }
@@ -348,6 +348,16 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
 #pragma unroll
           for (int ct = 0; ct < kCT; ++ct) enter(ct, sc[ct][(s8 + 1) % 8 / SPG % kSc]);
         convert(wf[cur ^ 1], (s8 + 1) & 7);
+        if constexpr (!kGroupSums) {
+#pragma unroll
+          for (int i = 0; i < kCT * kRT; ++i) {
+            if (s8 % SPG == 0) __builtin_amdgcn_sched_group_barrier(0x2, 16, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            if (s8 == 7) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            else __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
+          }
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
       const uint32_t t = s0;  // two chunks on
@@ -412,7 +422,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
   // Every group's sum by itself, two row tiles at a time, operands straight from memory, nothing shared with the other waves.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the first loads still write LDS
 #pragma unroll 1
-  for (int t = 0; t < kCT * kRT / 2; ++t) {
+  for (int t = 0; t < kCT * ((kRT + 1) / 2); ++t) {
     int r0 = row0 + 64 * (t / kCT);
     asm volatile("" : "+s"(r0));  // keeps the addresses of all rows out of the registers of the loops
     int col = col0 + 32 * (t % kCT) + n;
@@ -463,7 +473,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int m = r0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3);
-        if (m >= M) continue;
+        if (m >= M || m >= row0 + kRows) continue;
         if (a.partials) a.partials[(static_cast<size_t>(blockIdx.y) * M + m) * N + col] = sum[rt][e];
         else a.y[static_cast<size_t>(m) * N + col] = f32_to_bf16_rne(sum[rt][e]);
       }
@@ -502,13 +512,14 @@ Int4GemmShape int4_gemm_shape(int M, int N, int K, int groupsize, int64_t scratc
   if (options().int4_k_slices > 0)
     for (int s = 1; possible(s); s *= 2) forced = s;
   Int4GemmShape best = {64, 1, -1.0};
-  for (int rows = 64; rows <= (groupsize == 32 ? 64 : 128); rows *= 2) {  // group size 32 at 128 rows does not fit the registers
+  for (int rows = 64; rows <= (groupsize == 32 ? 64 : 128); rows += 32) {
+  // group size 32 at 128 rows does not fit the registers
     if (want_rows == 128 && groupsize != 32 && rows != 128) continue;
     const int64_t per_xcd = static_cast<int64_t>((M + rows - 1) / rows) * (((N + kCols - 1) / kCols + 7) / 8);  // one slice; 32 CUs each
     for (int s = 1; possible(s); s *= 2) {
       if (forced && s != forced) continue;
       const int64_t per_cu = (per_xcd * s + 31) / 32;
-      const double one = rows == 64 ? 1.2 : 1.85, two = rows == 64 ? 1.95 : 3.3;
+      const double one = rows == 64 ? 1.2 : rows == 96 ? 1.47 : 1.85, two = rows == 64 ? 1.95 : rows == 96 ? 2.42 : 3.3;
       const double cost = (static_cast<double>(per_cu / 2) * two + (per_cu & 1 ? one : 0)) * KT / s + 3 +
                           (s > 1 ? 4 + s * (0.6 + 0.9e-6 * static_cast<double>(M) * N) : 0);
       if (best.us < 0 || cost < best.us) best = Int4GemmShape{rows, s, cost};
@@ -520,8 +531,9 @@ Int4GemmShape int4_gemm_shape(int M, int N, int K, int groupsize, int64_t scratc
 template <int G>
 void launch_gemm(const GemmArgs &a, int rows, dim3 grid, hipStream_t stream) {
   if constexpr (G != 32) {
-    if (rows == 128) {
-      hipLaunchKernelGGL((int4_gemm_kernel<G, 4>), grid, dim3(256), 0, stream, a);
+    if (rows != 64) {
+      if (rows == 128) hipLaunchKernelGGL((int4_gemm_kernel<G, 4>), grid, dim3(256), 0, stream, a);
+      else hipLaunchKernelGGL((int4_gemm_kernel<G, 3>), grid, dim3(256), 0, stream, a);
       return;
     }
   }
