@@ -1,7 +1,8 @@
 // int4 group-wise matmul for many rows of x (prefill, scoring): MFMA-bound, 32x32 tiles.
 //
 // Same contract and data layouts as e2h_int4_mm.hip (torch.ops.aten._weight_int4pack_mm as called by
-// linear_forward_int4, reference models/quantize.py:445-453), inner_k_tiles = 8, group size 32 / 64 / 128.
+// linear_forward_int4, reference models/quantize.py:445-453), inner_k_tiles = 8, group size 32 / 64 / 128, and 256 as pairs of groups of 128
+// that share a scale and a zero.
 //
 //   y[m,n] = sum_g  s[g,n] * sum_{k in g} x[m,k] * (16 + q[n,k])  +  sum_g (z[g,n] - 24 s[g,n]) * X[m,g]
 //
@@ -77,6 +78,7 @@ struct GemmArgs {
   float *partials;  // [S][M][N] when K is shared, else null
   const float *xsum;
   int xsum_stride, M, N, K, n_col_blocks, cbx;
+  int shared;         // 1: two neighbouring groups have one (scale, zero) pair (group size 256), else 0
   const int *run_if;  // not null: nothing is done where it holds zero
 };
 
@@ -106,7 +108,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
   const int g_begin = blk0 * NGRP, g_end = blk1 * NGRP;
 
   const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(a.wp, static_cast<uint32_t>(static_cast<size_t>(N) * K / 2));
-  const __amdgpu_buffer_rsrc_t sz_rsrc = make_rsrc(a.sz, static_cast<uint32_t>(static_cast<size_t>(K / G) * N * 4));
+  const __amdgpu_buffer_rsrc_t sz_rsrc = make_rsrc(a.sz, static_cast<uint32_t>(static_cast<size_t>((K / G) >> a.shared) * N * 4));
   const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(a.x, static_cast<uint32_t>(static_cast<size_t>(M) * K * 2));
   const __amdgpu_buffer_rsrc_t xs_rsrc = make_rsrc(a.xsum, static_cast<uint32_t>(static_cast<size_t>(K / G) * a.xsum_stride * 4));
 
@@ -145,7 +147,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
     szlane[ct] = static_cast<uint32_t>(col) * 4u;
   }
   const auto load_sz = [&](int ct, int g) {
-    return __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, szlane[ct], static_cast<uint32_t>(g < g_end - 1 ? g : g_end - 1) * N * 4u, 0);
+    return __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, szlane[ct], static_cast<uint32_t>((g < g_end - 1 ? g : g_end - 1) >> a.shared) * N * 4u, 0);
   };
 
   load_w(blk0, kLdsW);
@@ -181,7 +183,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
       }
 #pragma unroll
       for (int ct = 0; ct < kCT; ++ct)
-        z[i].szw[ct] = __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, (szlane[ct] + static_cast<uint32_t>(h) * N * 4u) | out, gs * N * 4u, 0);
+        z[i].szw[ct] = __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, (szlane[ct] + ((gs + h) >> a.shared) * static_cast<uint32_t>(N) * 4u) | out, 0, 0);
     }
   };
   Zero za[kBatch], zb[kBatch];
@@ -454,7 +456,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
           part[rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf, __builtin_bit_cast(bf16x8_t, u), part[rt], 0, 0, 0);
         }
       }
-      const uint32_t szw = __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, static_cast<uint32_t>(col) * 4u, static_cast<uint32_t>(g) * N * 4u, 0);
+      const uint32_t szw = __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, static_cast<uint32_t>(col) * 4u, static_cast<uint32_t>(g >> a.shared) * N * 4u, 0);
       const float scale = __builtin_bit_cast(float, szw << 16), zero = __builtin_bit_cast(float, szw & 0xFFFF0000u);
       const float zc = __builtin_fmaf(-24.0f, scale, zero);
 #pragma unroll
@@ -543,8 +545,10 @@ void launch_gemm(const GemmArgs &a, int rows, dim3 grid, hipStream_t stream) {
 int int4_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint16_t *y, const float *xsum, int xsum_stride,
               float *partials, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream, const int *run_if) {
   if (K % 128 != 0 || N % 8 != 0) return E2H_ERR_BAD_SHAPE;
+  const int shared = groupsize == 256;
+  if (shared) groupsize = 128;
   GemmArgs a = {x, reinterpret_cast<const uint32_t *>(packed), reinterpret_cast<const uint32_t *>(sz), y, shape.slices > 1 ? partials : nullptr,
-                xsum, xsum_stride, M, N, K, (N + kCols - 1) / kCols, 0, run_if};
+                xsum, xsum_stride, M, N, K, (N + kCols - 1) / kCols, 0, shared, run_if};
   a.cbx = (a.n_col_blocks + 7) / 8;
   const long long wgs = 8LL * a.cbx * ((M + shape.rows - 1) / shape.rows);
   if (wgs > 0x7FFFFFFFLL) return E2H_ERR_BAD_SHAPE;

@@ -32,6 +32,8 @@
 // fixed order, so results are deterministic -- and writes bf16.
 #include <atomic>
 
+#include <algorithm>
+
 #include "e2h_common.h"
 #include "e2h_int4_unpack.h"
 
@@ -778,11 +780,11 @@ int int4_mm_impl(const uint16_t *x, const int32_t *packed, const uint16_t *scale
   const auto takes_256_row_kernel = [&](int64_t) {
     return mt == 4 && wide_ok && !options().int4_no_gemm32 && a.K % 256 == 0 && options().int4_gemm_tile == 256;
   };
-  if (mt == 4 && wide_ok && workspace && !options().int4_no_xsum && !takes_256_row_kernel(a.M)) {
+  if (((mt == 4 && wide_ok) || (groupsize == 256 && inner_k_tiles == 8 && a.M > 64)) && workspace && !options().int4_no_xsum && !takes_256_row_kernel(a.M)) {
     // many rows: the pre-pass keeps (K / g) sums per row in the workspace; slice M so that they fit rather than fall
     // back to the kernels that form the sums themselves (K = 22016 at g = 64: 24k rows per slice with 32 MB)
     const int64_t avail = workspace_bytes - static_cast<int64_t>(kTicketBytes);
-    const int64_t rows_by_xsum = avail / (static_cast<int64_t>(a.K / groupsize) * 4) / 256 * 256;
+    const int64_t rows_by_xsum = avail / (static_cast<int64_t>(a.K / (groupsize == 256 ? 128 : groupsize)) * 4) / 256 * 256;
     if (rows_by_xsum >= 2048 && rows_by_xsum < max_rows) max_rows = rows_by_xsum;
   }
   const int m_total = a.M;
@@ -796,6 +798,23 @@ int int4_mm_impl(const uint16_t *x, const int32_t *packed, const uint16_t *scale
       if (rc128 != E2H_OK) return rc128;
       continue;
     }
+    // Group size 256 over many rows: pairs of groups of 128 on the 32x32-tile kernel where their sums of x fit and it is expected to be the faster one.  The kernel of this file takes
+    // 0.36 us per 128 k and round of its 32 x 64 outputs over the CUs.  Measured (us; here / 32x32): 66 rows 12288 x 4096 39 / 30, 400 rows 108 / 56, 4096 rows
+    // 1083 / 355, 300 rows 4096 x 4096 36 / 30; stay: 157 rows 25 / 25, 400 rows 2048 x 2048 16 / 24.
+    if (groupsize == 256 && inner_k_tiles == 8 && a.M > 64 && workspace && !options().int4_no_xsum && !options().int4_no_gemm32 && !options().row_tiles) {
+      const int stride = ((a.M + 63) / 64) * 64;
+      const int64_t need = static_cast<int64_t>(kTicketBytes) + static_cast<int64_t>(a.K / 128) * stride * 4;
+      const Int4GemmShape shape = int4_gemm_shape(a.M, a.N, a.K, 128, std::max<int64_t>(0, workspace_bytes - need) & ~int64_t{15});
+      const double rounds = static_cast<double>((a.N + 63) / 64) * ((a.M + 31) / 32) / kCUs;
+      if (need <= workspace_bytes && 1.1 * shape.us + 1.6 < 6 + 0.36 * (a.K / 128) * std::max(1.0, rounds)) {
+        float *xs = reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + kTicketBytes);
+        if (launch_x_group_sums(a.x, xs, a.M, a.K, stride, 128, a.stream) != E2H_OK) return E2H_ERR_LAUNCH;
+        float *partials = reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + need);
+        const int rc = int4_gemm(a.x, a.packed, a.sz, a.y, xs, stride, partials, shape, a.M, a.N, a.K, 256, a.stream);
+        if (rc != E2H_OK) return rc;
+        continue;
+      }
+    }
     if (mt == 4 && wide_ok && (sh.t == 1 || sh.t == 2) && workspace && !options().int4_no_xsum) {
       // many rows: one pass over x leaves its group sums in the workspace's partial-tile area (unused here: no K split)
       const int stride = ((a.M + 63) / 64) * 64;
@@ -806,22 +825,24 @@ int int4_mm_impl(const uint16_t *x, const int32_t *packed, const uint16_t *scale
         a.xsum = xs;
         a.xsum_stride = stride;
         // The 32x32-tile kernel wherever the work fills the chip (320 tiles of 128 x 128), and below that where it is expected to take
-        // two thirds of the time of the 16x16-tile kernel of this file at most (both estimates are good to 20 %): that one takes 0.9 us per
-        // 128 k with one weight tile per wave and 1.15 with two, half as much again for every further workgroup on a CU.  Measured (us;
-        // 16x16 / 32x32): 65 rows 4096 x 4096 33 / 21, 471 rows 4096 x 11008 98 / 65; stay: 157 rows 11008 x 4096 47 / 42, 471 rows
-        // 2048 x 2048 20 / 24, 65 rows 512 x 512 8 / 10.
+        // less time than the 16x16-tile kernel of this file by more than the estimates are off: that one takes 0.9 us per 128 k with one weight tile per wave (1.35 at group size
+        // 32) and 1.15 with two (1.85 at 64, 3 at 32), not quite half as much again for every further workgroup on a CU.  Measured (us;
+        // 16x16 / 32x32): 300 rows 12288 x 4096 g128 52 / 44, g64 82 / 55, g32 131 / 69, 1100 rows 4096 x 11008 g128 202 / 125; stay: 400 rows
+        // 2048 x 2048 g128 21 / 23, g64 20 / 24.
         const int64_t left = (workspace_bytes - need) & ~int64_t{15};
         const Int4GemmShape shape = int4_gemm_shape(a.M, a.N, a.K, groupsize, left);
         const long long wgs32 = static_cast<long long>((a.M + 127) / 128) * ((a.N + 127) / 128);
         const long long wgs16 = static_cast<long long>((tiles16 + 4 * sh.t - 1) / (4 * sh.t)) * ((a.M + 63) / 64);
-        const double us16 = 4 + (sh.t == 2 ? 1.15 : 0.9) * (a.K / 128) * (1 + 0.45 * static_cast<double>((wgs16 - 1) / kCUs));
-        const bool use32 = options().int4_gemm32_min_rows > 0 ? a.M >= options().int4_gemm32_min_rows : wgs32 >= 320 || 1.5 * shape.us < us16;
+        const double per_wg = sh.t == 2 ? (groupsize == 32 ? 3.0 : groupsize == 64 ? 1.85 : 1.15) : groupsize == 32 ? 1.35 : 0.9;
+        const double us16 = 4 + per_wg * (a.K / 128) * std::max(1.0, 0.75 + 0.45 * static_cast<double>(wgs16) / kCUs);
+        const bool use32 = options().int4_gemm32_min_rows > 0 ? a.M >= options().int4_gemm32_min_rows : wgs32 >= 320 || 1.1 * shape.us + 1.6 < us16;
         if (use32 && !options().int4_no_gemm32) {
           float *partials = reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + need);  // need is a multiple of 256
           const int rc32 = int4_gemm(a.x, a.packed, a.sz, a.y, xs, stride, partials, shape, a.M, a.N, a.K, groupsize, a.stream);
           if (rc32 != E2H_OK) return rc32;
           continue;
         }
+        if (a.S > 1) a.xsum = nullptr;  // forced K slices leave their partial tiles where the sums lie: the kernel forms them itself
       }
     }
     int rc;

@@ -100,7 +100,7 @@ __device__ __forceinline__ void store_tiles_via_lds(const e2h_f32x16_t (&acc)[CT
 // (defined in e2h_int4_mm.hip; groupsize in {32, 64, 128}).
 int launch_x_group_sums(const uint16_t *x, float *out, int M, int K, int stride, int groupsize, hipStream_t stream);
 
-// Many-row int4 matmul on 32x32 MFMA tiles (e2h_int4_gemm.hip); xsum as written by launch_x_group_sums.  A workgroup owns `rows` rows;
+// Many-row int4 matmul on 32x32 MFMA tiles (e2h_int4_gemm.hip); xsum as written by launch_x_group_sums (for group size 256: of 128).  A workgroup owns `rows` rows;
 // K may be shared by `slices` of them through float32 sums in `partials` ([slices][M][N]; unused with one slice).  int4_gemm_shape picks
 // both, with at most as many slices as fit scratch_bytes.  run_if, in device memory: the launch does nothing where it holds zero (one slice only).
 struct Int4GemmShape {

@@ -150,7 +150,6 @@ struct Int4Scratch {
   int *row_flag;     // [M]
   float *col_unit;   // [N] what one step of a column's sums is worth
   float *xsum;       // [K / G][stride] group sums, for the other kernel
-  uint32_t *sz;      // [K / 128][N] pairs of group size 256, each twice
   uint16_t *x, *w;   // [M][KE], [N][KE]
   int64_t bytes;
 };
@@ -172,7 +171,6 @@ Int4Scratch int4_scratch(uint8_t *base, int64_t M, int64_t N, int64_t K, int gro
   s.row_flag = reinterpret_cast<int *>(take(M * 4));
   s.col_unit = reinterpret_cast<float *>(take(N * 4));
   s.xsum = reinterpret_cast<float *>(take(K / G * sum_stride(M) * 4));
-  s.sz = reinterpret_cast<uint32_t *>(take(groupsize == 256 ? K / 128 * N * 4 : 0));
   s.x = reinterpret_cast<uint16_t *>(take(M * KE * 2));
   s.w = reinterpret_cast<uint16_t *>(take(N * KE * 2));
   s.bytes = at;
@@ -290,7 +288,6 @@ __global__ __launch_bounds__(256) void int4_unpack_w_kernel(const uint32_t *__re
       if (blockIdx.y == 0) {
         uint16_t *ext = s.w + static_cast<size_t>(col0 + c1) * KE + K + 3 * g;
         ext[0] = ext[1] = ext[2] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(z));
-        if (twice) s.sz[static_cast<size_t>(g) * N + col0 + c1] = pair;
       }
     }
   if (blockIdx.y == 0 && live1) {
@@ -445,8 +442,7 @@ int int4_unpacked_gemm(const uint16_t *x, const int32_t *packed, const uint16_t 
     default: launch_unpack<128>(x, wp, sz, s, twice, M, N, K, KE, stream); break;
   }
   hipLaunchKernelGGL(int4_unpacked_gemm_kernel, dim3(grid_of(M, N)), dim3(256), 0, stream, s, y, M, N, KE);
-  return int4_gemm(x, packed, twice ? reinterpret_cast<const uint16_t *>(s.sz) : scales_and_zeros, y, s.xsum, sum_stride(M), nullptr, int4_gemm_shape(M, N, K, G, 0), M, N, K,
-                   G, stream, s.flag);
+  return int4_gemm(x, packed, scales_and_zeros, y, s.xsum, sum_stride(M), nullptr, int4_gemm_shape(M, N, K, G, 0), M, N, K, groupsize, stream, s.flag);
 }
 
 }  // namespace e2h

@@ -52,6 +52,18 @@ def test_exact_on_dyadic_operands(many_row_kernel, g, slices, tile, m, n, k):
     assert torch.equal(got, want.to(torch.bfloat16))
 
 
+# three blocks of 128 k per slice and an odd first one; workgroups of 64, 96 and 128 rows by their own rule
+@pytest.mark.parametrize("slices", [0, 1, 2, 4])
+@pytest.mark.parametrize("g,m,n,k", [(256, 130, 3080, 768), (256, 471, 1032, 2304), (256, 513, 12288, 1024), (128, 470, 12296, 384), (64, 195, 5128, 640), (64, 97, 8200, 1408)])
+def test_pairs_of_groups_and_96_row_workgroups_are_exact(g, m, n, k, slices):
+    _lib.set_option("int4_k_slices", slices)
+    try:
+        got, want = _run(*_case(m, n, k, g), g)
+    finally:
+        _lib.set_option("int4_k_slices", 0)
+    assert torch.equal(got, want.to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("g", [32, 64, 128])
 @pytest.mark.parametrize("slices", [1, 2])
 def test_scales_outside_the_running_units(many_row_kernel, g, slices):
@@ -258,3 +270,16 @@ def test_what_float16_does_not_hold_is_left_to_the_other_kernel(what):
     assert need > 0
     same = torch.where(torch.isnan(other), torch.isnan(got), got == other)
     assert bool(same.all())
+
+
+@pytest.mark.parametrize("g,m,n,k", [(64, 470, 12296, 640), (128, 470, 12296, 384), (256, 470, 12296, 768)])
+def test_odd_scales_in_96_row_workgroups(g, m, n, k):
+    """471 rows of 12288 columns are work for five rows of workgroups; the plain loop walks pairs of row tiles, of which the last holds one"""
+    codes, scale, zero, x = _case(m, n, k, g)
+    zero[:, 5], scale[:, 5] = 0.0, 2.0**-101
+    zero[:, 12290], scale[:, 12290] = 0.0, 2.0**40
+    scale[-1, 300] = float("nan")
+    got, want = _run(codes, scale, zero, x, g)
+    finite = torch.ones(n, dtype=torch.bool)
+    finite[300] = False
+    assert torch.equal(got[:, finite], want[:, finite].to(torch.bfloat16)) and not torch.isfinite(got[:, 300]).any()
