@@ -13,6 +13,7 @@
 // Norm and rotation of a query happen where a kernel loads it (a lane of the matrix kernels holds 8 neighbouring dimensions, so the
 // rotated pairs are in-lane and a head's sum of squares is two shuffles); those of a key where it is appended.  A sink joins the
 // softmax sum at the end.
+#include "e2h_attention_tiles.h"
 #include "e2h_seq_common.h"
 
 namespace e2h {
@@ -576,6 +577,71 @@ __global__ __launch_bounds__(256) void attention_prefill_kernel(const e2h_window
   }
 }
 
+// ---- the same for heads of 64 or 128 dimensions: 4 waves x 32 queries (e2h_attention_tiles.h) -----------------------------------------
+template <int D>
+__global__ __launch_bounds__(256, 2) void attention_prompt_kernel(const e2h_window_attention_args a, int q_blocks) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int KS = D / 32, VT = D / 16;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[attention::kLdsBytes<D>];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, b4 = lane >> 4;
+  const int seqlen = static_cast<int>(a.seqlen);
+  const int rep = static_cast<int>(a.heads / a.kv_heads);
+  const attention::Place at = attention::place(blockIdx.x, static_cast<int>(a.batch * a.kv_heads), rep, q_blocks);
+  const int qb = q_blocks - 1 - at.back, g = at.pair % static_cast<int>(a.kv_heads), bi = at.pair / static_cast<int>(a.kv_heads), h = g * rep + at.rep;
+  const int pos0 = static_cast<int>(a.input_pos[0]), first = a.first ? static_cast<int>(a.first[bi]) : 0;
+  const int t0 = qb * attention::kQueries, t1 = t0 + attention::kQueries - 1 < seqlen - 1 ? t0 + attention::kQueries - 1 : seqlen - 1;
+  const int cache_last = static_cast<int>(a.cache_len) - 1, pb = pos0 + t1 < cache_last ? pos0 + t1 : cache_last;
+  const KeyList list = key_list(pos0 + t0, pb, first, static_cast<int>(a.window), static_cast<int>(a.keep_first));
+  const attention::Keys keys = {list.first, list.kept, list.start, list.count};
+  const attention::Rule rule = {first, static_cast<int>(a.window), static_cast<int>(a.keep_first)};
+  const bf16_t *proj = static_cast<const bf16_t *>(a.proj);
+  const size_t row0 = static_cast<size_t>(bi) * seqlen, head = static_cast<size_t>(bi) * a.kv_heads + g;
+  bf16x8_t qf[2][KS];
+  int pos[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int tq = t0 + wave * 32 + 16 * i + c, tc = tq < seqlen ? tq : seqlen - 1;
+    pos[i] = pos0 + tq;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int64_t d = static_cast<int64_t>(h) * D + 32 * s + 8 * b4;
+      u32x4_t raw = *reinterpret_cast<const u32x4_t *>(proj + (row0 + tc) * a.ld + a.q_off + d);
+      if (a.q_bias) raw = add_bias8(raw, a.q_bias + d, 8);
+      qf[i][s] = __builtin_bit_cast(bf16x8_t, raw);
+    }
+    prepare_query<KS, true>(qf[i], a, row0 + tc, D, b4);
+  }
+  f32x4_t o[2][VT];
+  float m[2], l[2];
+  const float sc = a.scale * kLog2e;
+  const int lo = pos0 + t0 + wave * 32;
+  attention::attend<D, true>(qf, pos, lo, lo + 31, keys, rule, sc, static_cast<const bf16_t *>(a.k_cache) + head * a.cache_len * D,
+                             static_cast<const bf16_t *>(a.v_cache) + head * a.cache_len * D, static_cast<uint32_t>(a.cache_len), lds, o, m, l);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int tq = t0 + wave * 32 + 16 * i + c;
+    float sum = l[i];
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    if (a.sink) sum += __builtin_amdgcn_exp2f(__builtin_fmaf(a.sink[h], kLog2e, -m[i] * sc));
+    const float inv = sum > 0.f ? a.out_scale / sum : 0.f;
+    if (tq >= seqlen) continue;
+    const size_t row = row0 + tq;
+#pragma unroll
+    for (int v = 0; v < VT; ++v) {
+      const int64_t d = static_cast<int64_t>(h) * D + 16 * v + 4 * b4;
+      f32x4_t out = o[i][v] * inv;
+      if (a.g_off >= 0) {
+        const f32x4_t gate = load4(proj + row * a.ld + a.g_off + d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[e] *= fast_sigmoid(gate[e]);
+      }
+      store4(static_cast<bf16_t *>(a.out) + row * a.ld_out + a.out_off + d, out);
+    }
+  }
+#endif
+}
+
 // ---- bfloat16, one token per sequence: `splits` workgroups per (sequence, key/value head) --------------------------------------
 // The lane columns are the query heads of the group (up to 16); the waves of all its workgroups take key tiles of 32 round robin and
 // are combined at the end: in LDS, then, where there are several workgroups, by attention_combine_kernel from `part`
@@ -881,6 +947,14 @@ void launch_mfma(const e2h_window_attention_args &a, float *part, int64_t part_b
     return;
   }
   launch_append(a, VEC && aligned16(a.k_bias) && aligned16(a.v_bias) && a.k_off % 8 == 0 && a.v_off % 8 == 0, s);
+  if constexpr (VEC && (KS == 2 || KS == 4) && VT == 2 * KS) {
+    constexpr int D = 32 * KS;
+    if (a.dim == D && a.vdim == D && a.cache_len <= static_cast<int64_t>(UINT32_MAX) / (2 * D)) {
+      const int blocks = static_cast<int>((a.seqlen + attention::kQueries - 1) / attention::kQueries);
+      hipLaunchKernelGGL(attention_prompt_kernel<D>, dim3(static_cast<unsigned>(a.batch * a.heads * blocks)), dim3(256), 0, s, a, blocks);
+      return;
+    }
+  }
   const int q_blocks = static_cast<int>((a.seqlen + 63) / 64);
   hipLaunchKernelGGL((attention_prefill_kernel<KS, VT, VEC>), dim3(static_cast<unsigned>(a.batch * a.heads * q_blocks)), dim3(256), 0, s, a, q_blocks);
 }

@@ -172,6 +172,24 @@ def test_window_edges_with_one_key_that_stands_out(dtype, window, keep):
             assert rel(got, want) < (1e-5 if dtype == torch.float32 else 1e-2)
 
 
+@pytest.mark.parametrize("h,g,d", [(4, 2, 64), (8, 8, 128), (5, 1, 128), (3, 3, 64)])
+@pytest.mark.parametrize("window,keep", [(0, 0), (100, 70), (300, 5), (1, 0)])
+def test_prompt_attention_in_blocks_of_128_queries(h, g, d, window, keep):
+    """Prompts and portions that end at, before and behind a block of 128 queries and a tile of 64 keys, kept keys that end inside a tile, windows that leave whole tiles
+    out, sequences with no, one tile's and more than a block's padding side by side, and numbers of heads that do and do not divide by the eight XCDs.  The weights are held
+    as two bfloat16 terms, so the tolerance is that of the values' and the result's rounding."""
+    t, pads = 390, [0, 70, 200]
+    q, k, v, gate = (randn(3, t, n, d, seed=i, dtype=torch.bfloat16) for i, n in enumerate((h, g, g, h)))
+    k[0, 5:40, 0] += 0.5 * q[0, -1, 0]  # far keys carry weight
+    first = torch.tensor(pads, device=DEV)
+    for portions in ([t], [129, 128, 1, 127, 5], [63, 65, 256, 6]):
+        got = f64(run_attention(q, k, v, gate, torch.bfloat16, 0.3, window, keep, portions, first=first))
+        for i, f in enumerate(pads):
+            want = ro.window_attention(f64(q)[i, f:], f64(k)[i, f:], f64(v)[i, f:], 0.3, window or 10 ** 9, keep) * ro.sigmoid(f64(gate)[i, f:])
+            assert rel(got[i, f:], want) < 1e-2, (portions, i)
+            assert (got[i, :f] == 0).all()
+
+
 @BOTH
 def test_attention_of_padded_and_shorter_sequences_side_by_side(dtype):
     b, t, h, g, d, dv, window, keep = 3, 90, 4, 2, 32, 48, 11, 4
