@@ -42,6 +42,7 @@ _SIGNATURES = {
     "e2h_int8_mm_partials": (c_int, [_P, _P, _P, c_int64, c_int64, c_int64, c_int, _P]),
     "e2h_add_rmsnorm_partials": (c_int, [_P, _P, c_int, _P, _P, _P, _P, c_int64, c_int64, c_float, _P]),
     "e2h_rope_kv_write": (c_int, [_P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, _P]),
+    "e2h_prefill_attention": (c_int, [_P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_float, _P]),
     "e2h_rope_kv_write_seq": (c_int, [_P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, _P]),
     "e2h_silu_mul": (c_int, [_P, _P, _P, c_int64, _P]),
     "e2h_int4_mm_rope_kv": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_int, _P]),

@@ -3,9 +3,11 @@
 //   e2h_rmsnorm            RMSNorm with the reference's rounding points
 //   e2h_rope_kv_write      rotary embedding of q and k + write of k, v into the cache at input_pos
 //   e2h_silu_mul           silu(a) * b
+// and, over many new tokens, e2h_prefill_attention: causal attention with left padding.
 // They restate, for one new token per sequence, what the reference's model code does with stock ops
 // (models/model.py: KVCache.update :121-129, Attention.forward :310-349, RMSNorm :363-377, apply_rotary_emb
 // :400-412, FeedForward.forward :359-360; decode loop inference_generate.py:110-157).
+#include "e2h_attention_tiles.h"
 #include "e2h_common.h"
 #include "e2h_staged.h"
 
@@ -612,6 +614,79 @@ int launch_attention(int rep, dim3 grid, hipStream_t s, const uint16_t *q, const
   return launch_attention_nw<D, 4>(rep, grid, s, q, kc, vc, out, input_pos, left_pad, H, Hkv, S, scale, staged);
 }
 
+// ---- causal attention of many new tokens (e2h_attention_tiles.h) --------------------------------------------------------------
+// 128 queries of one head per workgroup.  A query at position p sees the keys left_pad .. p and, in front of its sequence, its own key alone: there the result is
+// that value as it is.  Weights are rounded to bfloat16 for their product with the values, their sum is not.
+// 64 x 768 tokens, 32 heads of 128: the stock kernel took 1640 us and a copy to token order 204.
+template <int D>
+__global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restrict__ kc, const uint16_t *__restrict__ vc,
+                                                                   uint16_t *__restrict__ out, const int64_t *__restrict__ input_pos,
+                                                                   const int64_t *__restrict__ left_pad, int B, int T, int H, int Hkv, int S, float scale, int q_blocks) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int KS = D / 32, VT = D / 16;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[attention::kLdsBytes<D>];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, b4 = lane >> 4;
+  const int rep = H / Hkv;
+  const attention::Place at = attention::place(blockIdx.x, B * Hkv, rep, q_blocks);
+  const int hk = at.pair % Hkv, b = at.pair / Hkv, h = hk * rep + at.rep, t0 = (q_blocks - 1 - at.back) * attention::kQueries;
+  const int first = left_pad ? static_cast<int>(left_pad[b]) : 0;
+  const auto position = [&](int t) { return input_pos ? static_cast<int>(input_pos[t < T ? t : T - 1]) : t < T ? t : T - 1; };
+  // positions may come in any order: the largest of the block bounds its keys
+  int top = position(t0 + lane) > position(t0 + 64 + lane) ? position(t0 + lane) : position(t0 + 64 + lane);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const int o = __shfl_xor(top, off);
+    top = top > o ? top : o;
+  }
+  top = __builtin_amdgcn_readfirstlane(top);
+  top = top < S - 1 ? top : S - 1;
+  const attention::Rule rule = {first > 0 ? first : 0, INT32_MAX / 2, 0};
+  const attention::Keys keys = {rule.first, 0, rule.first, top >= rule.first ? top - rule.first + 1 : 0};
+
+  bf16x8_t qf[2][KS];
+  int pos[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int t = t0 + wave * 32 + 16 * i + c, tc = t < T ? t : T - 1;
+    pos[i] = position(t);
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      qf[i][s] = *reinterpret_cast<const bf16x8_t *>(q + ((static_cast<size_t>(b) * H + h) * T + tc) * D + 32 * s + 8 * b4);
+  }
+  int lo = pos[0] < pos[1] ? pos[0] : pos[1], hi = pos[0] < pos[1] ? pos[1] : pos[0];
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1) {
+    const int l2 = __shfl_xor(lo, off), h2 = __shfl_xor(hi, off);
+    lo = lo < l2 ? lo : l2;
+    hi = hi > h2 ? hi : h2;
+  }
+  lo = __builtin_amdgcn_readfirstlane(lo);
+  hi = __builtin_amdgcn_readfirstlane(hi);
+  const size_t head = (static_cast<size_t>(b) * Hkv + hk) * S * D;
+  f32x4_t o[2][VT];
+  float m[2], l[2];
+  attention::attend<D, false>(qf, pos, lo, hi, keys, rule, scale * attention::kLog2E, kc + head, vc + head, static_cast<uint32_t>(S), lds, o, m, l);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int t = t0 + wave * 32 + 16 * i + c;
+    float sum = l[i];
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    if (t >= T) continue;
+    const float inv = 1.0f / sum;
+    uint16_t *dst = out + (static_cast<size_t>(b) * T + t) * H * D + static_cast<size_t>(h) * D + 4 * b4;
+    const bool own = pos[i] < rule.first && pos[i] >= 0 && pos[i] < S;
+    const uint16_t *value = vc + head + static_cast<size_t>(own ? pos[i] : 0) * D + 4 * b4;
+#pragma unroll
+    for (int v = 0; v < VT; ++v) {
+      u32x2_t w = {attention::pack_bf16_pair(o[i][v][0] * inv, o[i][v][1] * inv), attention::pack_bf16_pair(o[i][v][2] * inv, o[i][v][3] * inv)};
+      if (own) w = *reinterpret_cast<const u32x2_t *>(value + 16 * v);
+      *reinterpret_cast<u32x2_t *>(dst + 16 * v) = w;
+    }
+  }
+#endif
+}
+
 }  // namespace
 }  // namespace e2h
 
@@ -693,6 +768,29 @@ extern "C" int e2h_add_rmsnorm_staged(const uint16_t *x, const uint16_t *delta, 
     return E2H_ERR_MISALIGNED;
   launch_rmsnorm(x, delta, partials, partials ? slices : 0, partials ? col_scales : nullptr, weight, h_out, y, staged_out(staged, rows, dim), rows, dim,
                  eps, static_cast<hipStream_t>(stream));
+  return launch_status();
+}
+
+extern "C" int e2h_prefill_attention(const uint16_t *q, const uint16_t *k_cache, const uint16_t *v_cache, uint16_t *out, const int64_t *input_pos,
+                                     const int64_t *left_pad, int64_t batch, int64_t seqlen, int64_t n_head, int64_t n_kv_head, int64_t cache_len,
+                                     int64_t head_dim, float scale, void *stream) {
+  if (!q || !k_cache || !v_cache || !out) return E2H_ERR_NULL_POINTER;
+  if (batch < 1 || seqlen < 1 || n_head < 1 || n_kv_head < 1 || n_head % n_kv_head != 0 || (head_dim != 64 && head_dim != 128) || cache_len < 1 ||
+      cache_len > static_cast<int64_t>(UINT32_MAX) / (2 * head_dim) || cache_len > INT32_MAX / 2 || seqlen > INT32_MAX / 2 || (!input_pos && seqlen > cache_len) || !(scale > 0.f))
+    return E2H_ERR_BAD_SHAPE;
+  if (!aligned16(q) || !aligned16(k_cache) || !aligned16(v_cache) || !aligned16(out) || (reinterpret_cast<uintptr_t>(input_pos) & 7u) ||
+      (reinterpret_cast<uintptr_t>(left_pad) & 7u))
+    return E2H_ERR_MISALIGNED;
+  const int64_t blocks = (seqlen + attention::kQueries - 1) / attention::kQueries;
+  if (n_head > INT32_MAX / batch || batch * n_head > INT32_MAX / blocks) return E2H_ERR_BAD_SHAPE;
+  const dim3 grid(static_cast<unsigned>(batch * n_head * blocks));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (head_dim == 64)
+    hipLaunchKernelGGL(prefill_attention_kernel<64>, grid, dim3(256), 0, s, q, k_cache, v_cache, out, input_pos, left_pad, (int)batch, (int)seqlen, (int)n_head, (int)n_kv_head,
+                       (int)cache_len, scale, (int)blocks);
+  else
+    hipLaunchKernelGGL(prefill_attention_kernel<128>, grid, dim3(256), 0, s, q, k_cache, v_cache, out, input_pos, left_pad, (int)batch, (int)seqlen, (int)n_head, (int)n_kv_head,
+                       (int)cache_len, scale, (int)blocks);
   return launch_status();
 }
 

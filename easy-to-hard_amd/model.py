@@ -17,7 +17,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 from torch import Tensor
 
-from . import ops
+from . import ops, seq_ops
+from .linear import unwatched
 from .quantize import WeightOnlyInt4Linear, WeightOnlyInt8Linear, find_multiple
 from .state import KVCache
 
@@ -147,6 +148,7 @@ class Attention(nn.Module):
         self.kv_cache = None
         self.freqs_table = None        # full (cos, sin) table, set by Transformer.setup_caches
         self.left_pad_mask_pos = None  # per-step padding mask positions, set by Transformer.forward
+        self.mask_of = None            # while Transformer.forward passes no mask (causal by input_pos, with left_pad_mask_pos): what would build it
         self.n_head = config.n_head
         self.head_dim = config.head_dim
         self.n_local_heads = config.n_local_heads
@@ -210,6 +212,10 @@ class Attention(nn.Module):
                 k, v = self.kv_cache.k_cache, self.kv_cache.v_cache
             q = ops.rope_kv_write_seq(qkv, self.freqs_table, k, v, input_pos, self.n_head, self.n_local_heads, self.head_dim,
                                       rows_by_token=fully_causal)
+            if ((fully_causal or (mask is None and self.mask_of is not None)) and not torch.compiler.is_compiling()
+                    and ops.prefill_attention_fits(seqlen, self.n_head, k, v) and not seq_ops.watched(q, k, v)):
+                y = ops.prefill_attention(q, k, v, None if fully_causal else input_pos, None if fully_causal else self.left_pad_mask_pos)
+                return self.wo(y)
             k, v = k[:bsz], v[:bsz]
         else:
             q, k, v = self.wqkv(x).split([self.dim, kv_size, kv_size], dim=-1)
@@ -222,6 +228,8 @@ class Attention(nn.Module):
         if rep > 1:
             k = k.repeat_interleave(rep, dim=1)
             v = v.repeat_interleave(rep, dim=1)
+        if mask is None and self.mask_of is not None:
+            mask = self.mask_of(input_pos, self.left_pad_mask_pos)
         if fully_causal and q.size(2) == k.size(2):
             y = F.scaled_dot_product_attention(q, k, v, is_causal=True)
         else:
@@ -417,12 +425,9 @@ class Transformer(nn.Module):
         x = self.tok_embeddings(idx)
         mask = None
         fused_step = self.layers[0].attention.can_fuse_decode(x, fully_causal)
-        if not fully_causal and not fused_step:
-            mask = self.causal_mask[None, None, input_pos]
-            if left_pad_mask_pos is not None:
-                visible = torch.arange(mask.size(-1), device=mask.device).view(1, -1) >= left_pad_mask_pos.view(-1, 1)
-                mask = torch.logical_and(mask, visible[:, None, None, :])
-                mask = torch.logical_or(mask, self.self_mask[None, None, input_pos])
+        by_position = not fully_causal and not fused_step and self._masks_by_position(x, input_pos)
+        if not fully_causal and not fused_step and not by_position:
+            mask = self._mask(input_pos, left_pad_mask_pos)
         freqs_cis = None if fused_step else self.freqs_cis[input_pos].to(dtype=x.dtype)
         if fused_step and input_pos.dtype != torch.int64:
             # the reference decodes with an int32 position tensor (inference_generate.py:205); the fused kernels read int64
@@ -441,15 +446,45 @@ class Transformer(nn.Module):
                 return ops.int4_mm_staged(xs, out.weight, out.groupsize, out.scales_and_zeros).view(rows, 1, -1)
             _, normed = ops.add_rmsnorm(h, delta, self.norm.weight, self.norm.eps)
             return self.output(normed.view(rows, 1, -1))
-        if _fusable(x) and x.shape[-1] % 8 == 0 and self.norm.weight.dtype == torch.bfloat16:
-            delta = None
+        if by_position:
+            for blk in self.layers:
+                blk.attention.mask_of = self._mask
+        try:
+            if _fusable(x) and x.shape[-1] % 8 == 0 and self.norm.weight.dtype == torch.bfloat16:
+                delta = None
+                for layer in self.layers:
+                    x, delta = layer.forward_deferred(x, delta, input_pos, freqs_cis, mask, fully_causal)
+                _, normed = ops.add_rmsnorm(x, delta, self.norm.weight, self.norm.eps)
+                return self.output(normed)
             for layer in self.layers:
-                x, delta = layer.forward_deferred(x, delta, input_pos, freqs_cis, mask, fully_causal)
-            _, normed = ops.add_rmsnorm(x, delta, self.norm.weight, self.norm.eps)
-            return self.output(normed)
-        for layer in self.layers:
-            x = layer(x, input_pos, freqs_cis, mask, fully_causal)
-        return self.output(self.norm(x))
+                x = layer(x, input_pos, freqs_cis, mask, fully_causal)
+            return self.output(self.norm(x))
+        finally:
+            if by_position:
+                for blk in self.layers:
+                    blk.attention.mask_of = None
+
+    def _mask(self, input_pos: Tensor, left_pad_mask_pos: Optional[Tensor]) -> Tensor:
+        mask = self.causal_mask[None, None, input_pos]
+        if left_pad_mask_pos is not None:
+            visible = torch.arange(mask.size(-1), device=mask.device).view(1, -1) >= left_pad_mask_pos.view(-1, 1)
+            mask = torch.logical_and(mask, visible[:, None, None, :])
+            mask = torch.logical_or(mask, self.self_mask[None, None, input_pos])
+        return mask
+
+    def _masks_by_position(self, x: Tensor, input_pos: Optional[Tensor]) -> bool:
+        """True where every attention of a prompt runs on ops.prefill_attention, which needs no mask tensor: built for them all otherwise, and where somebody
+        watches the blocks' or the attentions' calls (hooks are shown the mask) or a trace is being made."""
+        if torch.compiler.is_compiling() or input_pos is None or not (input_pos.is_cuda and input_pos.dtype == torch.int64 and input_pos.dim() == 1):
+            return False
+        if seq_ops.watched(x, input_pos):
+            return False
+        for blk in self.layers:
+            att = blk.attention
+            if not (type(att) is Attention and type(blk) is TransformerBlock and unwatched(blk) and unwatched(att) and att._can_fuse_prefill_rope(x, input_pos, False)
+                    and ops.prefill_attention_fits(x.shape[1], att.n_head, att.kv_cache.k_cache, att.kv_cache.v_cache)):
+                return False
+        return True
 
 
 class RewardModel(nn.Module):

@@ -555,6 +555,31 @@ def rope_kv_write_seq(qkv, freqs_cis, k_cache, v_cache, input_pos, n_head, n_kv_
     return q
 
 
+def prefill_attention_fits(t, n_head, k, v):
+    """True when T queries of n_head heads and (k, v [>= B, Hkv, S, D]) fit e2h_prefill_attention and there are enough tokens for its blocks of queries."""
+    return (t >= 16 and k.is_cuda and k.shape[3] in (64, 128) and n_head % k.shape[1] == 0 and k.shape[2] * k.shape[3] < 2 ** 30
+            and all(c.dtype == torch.bfloat16 and c.is_contiguous() and c.data_ptr() % 16 == 0 for c in (k, v)))
+
+
+def prefill_attention(q, k, v, input_pos=None, left_pad=None):
+    """Causal attention of T new tokens per sequence, q bf16 [B, H, T, D] over keys and values [>= B, Hkv, S, D] -> [B, T, H * D].  Token t stands at
+    input_pos[t] (int64 on the device), or at t; left_pad int64 [B] or None: keys in front of it are seen by nobody but their own query."""
+    _need_gpu(q, k, v)
+    bsz, h, t, d = q.shape
+    hkv, s = k.shape[1], k.shape[2]
+    assert q.dtype == torch.bfloat16 and k.dtype == torch.bfloat16 and v.dtype == torch.bfloat16 and q.is_contiguous() and k.is_contiguous() and v.is_contiguous()
+    assert k.shape[0] >= bsz and k.shape[3] == d and v.shape == k.shape and h % hkv == 0
+    assert input_pos is None or (input_pos.is_cuda and input_pos.dtype == torch.int64 and input_pos.numel() == t)
+    assert left_pad is None or (left_pad.is_cuda and left_pad.numel() in (1, bsz))
+    pos = None if input_pos is None else input_pos.contiguous()
+    pad = None if left_pad is None else left_pad.reshape(-1).to(torch.int64).expand(bsz).contiguous()
+    out = torch.empty((bsz, t, h * d), dtype=torch.bfloat16, device=q.device)
+    rc = _lib_for(q).e2h_prefill_attention(_ptr(q), _ptr(k), _ptr(v), _ptr(out), None if pos is None else _ptr(pos), None if pad is None else _ptr(pad), bsz, t, h, hkv, s, d,
+                                           d ** -0.5, _stream(q))
+    _lib.check(rc, "e2h_prefill_attention")
+    return out
+
+
 def int4_rope_kv_supported(x, wqkv, freqs_cis, k_cache):
     """True when the fused projection + RoPE + cache write covers (x [B, 1, K], a WeightOnlyInt4Linear)."""
     if not (x.is_cuda and x.dtype == torch.bfloat16 and x.numel() // x.shape[-1] <= 64):

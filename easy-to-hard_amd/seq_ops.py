@@ -131,7 +131,7 @@ STREAMED_ROWS = 64
 _PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
-def _watched(*tensors):
+def watched(*tensors):
     """True where something besides autograd's graph follows what happens to the tensors and would lose sight of it in a launch through
     ctypes: subclasses, forward-mode derivatives, function transforms (vmap, jvp, ..), dispatch modes, torch.jit traces.  (The two last
     do not look through a compiler's trace: that records the registered op.)"""
@@ -149,7 +149,7 @@ def linear_streams(x, weight):
         return False
     if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
         return False
-    return k % 8 == 0 and k < 1 << 22 and not torch.is_autocast_enabled() and not _watched(x, weight)
+    return k % 8 == 0 and k < 1 << 22 and not torch.is_autocast_enabled() and not watched(x, weight)
 
 
 def linear(x, weight, act=ACT_NONE, cap=0.0):

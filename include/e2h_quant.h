@@ -370,6 +370,15 @@ int e2h_rope_kv_write_seq(const uint16_t *qkv, const uint16_t *freqs_cis, uint16
                           uint16_t *v_cache, const int64_t *input_pos, int64_t batch, int64_t seqlen, int64_t n_head,
                           int64_t n_kv_head, int64_t cache_len, int64_t head_dim, int rows_by_token, void *stream);
 
+/* Causal attention of many new tokens (prefill, scoring): what the reference computes with scaled_dot_product_attention under its mask (:221-228, :341-349).
+ * q [batch, n_head, seqlen, head_dim], k_cache / v_cache [>= batch, n_kv_head, cache_len, head_dim] that hold every key a query sees, out
+ * [batch, seqlen, n_head * head_dim], all bf16 and 16-byte aligned; head_dim 64 or 128, n_head a multiple of n_kv_head.  Token t stands at position input_pos[t], or t
+ * where input_pos is NULL; a query at position p sees keys left_pad[b] .. p and key p (left_pad NULL: 0 .. p).  float32 scores and sums; weights are rounded to
+ * bfloat16 for their product with the values. */
+int e2h_prefill_attention(const uint16_t *q, const uint16_t *k_cache, const uint16_t *v_cache, uint16_t *out, const int64_t *input_pos,
+                          const int64_t *left_pad, int64_t batch, int64_t seqlen, int64_t n_head, int64_t n_kv_head, int64_t cache_len,
+                          int64_t head_dim, float scale, void *stream);
+
 /* F.silu(a) * b with bf16 rounding after each op (reference FeedForward.forward :359-360). n elements, n % 8 == 0. */
 int e2h_silu_mul(const uint16_t *a, const uint16_t *b, uint16_t *y, int64_t n, void *stream);
 

@@ -204,3 +204,57 @@ def test_grouped_query_attention_on_matrix_cores_matches_sdpa_and_vector_kernel(
             finally:
                 _lib.set_option("attention_no_mfma", 0)
             assert (y.float() - y_vec.float()).abs().max() < 1e-2 * scale
+
+
+@pytest.mark.parametrize("h,hkv,d", [(4, 4, 128), (8, 2, 64), (5, 1, 128), (6, 3, 64)])
+@pytest.mark.parametrize("t,start,s_len", [(16, 0, 16), (127, 0, 136), (129, 40, 200), (300, 64, 600)])
+def test_prefill_attention_against_float64(h, hkv, d, t, start, s_len):
+    """Blocks of 128 queries and tiles of 64 keys that end inside, a prompt behind cached tokens, unequal padding (none, inside the prompt, more than all of it), positions
+    in any order, and tokens that stand at their index.  Rows in front of a sequence are their own value.  Cache rows nobody sees hold NaN.  Error against 64 bits: at most that of
+    the stock kernel on the same inputs (both round weights and results to bfloat16), with a margin for single inputs."""
+    gen = torch.Generator().manual_seed(t + h)
+    b = 3
+    q = torch.randn((b, h, t, d), generator=gen).to(torch.bfloat16).to(DEV)
+    k, v = (torch.randn((b + 1, hkv, s_len, d), generator=gen).to(torch.bfloat16).to(DEV) for _ in range(2))
+    pads = torch.tensor([0, min(start + t - 1, 70), start + t + 3], device=DEV)
+    order = torch.arange(start, start + t, device=DEV)
+    for pos, pad in ((order, None), (order, pads), (order[torch.randperm(t, generator=gen).to(DEV)], pads), (None, None)):
+        at = torch.arange(t, device=DEV) if pos is None else pos
+        key = torch.arange(s_len, device=DEV)
+        mask = (key[None, None] <= at[None, :, None]).expand(b, t, s_len)
+        if pad is not None:
+            mask = (mask & (key[None, None] >= pad[:, None, None])) | (key[None, None] == at[None, :, None])
+        kn, vn = k.clone(), v.clone()
+        far = int(at.max()) + 64 - int(at.max()) % 64  # tiles behind the last visible key; in a tile that is seen in part, a value meets a weight of zero
+        kn[:, :, far:], vn[:, :, far:] = float("nan"), float("nan")
+        got = ops.prefill_attention(q, kn, vn, pos, pad)
+        rep = lambda c: c[:b].repeat_interleave(h // hkv, dim=1)  # noqa: E731
+        scores = (q.double() @ rep(k).double().transpose(-1, -2).contiguous()) * d ** -0.5
+        want = (scores.masked_fill(~mask[:, None], float("-inf")).softmax(-1) @ rep(v).double()).transpose(1, 2).reshape(b, t, h * d)
+        stock = torch.nn.functional.scaled_dot_product_attention(q, rep(k), rep(v), attn_mask=mask[:, None]).transpose(1, 2).reshape(b, t, h * d)
+        err, err_stock = ((x.double() - want).norm() / want.norm() for x in (got, stock))
+        assert err <= 1.05 * err_stock, (err, err_stock)
+        if pad is not None:
+            for i in range(b):
+                front = (at < pad[i]).nonzero().flatten()
+                assert torch.equal(got[i, front], rep(v)[i][:, at[front]].transpose(0, 1).reshape(len(front), h * d))
+
+
+def test_prompts_of_a_watched_attention_are_shown_the_mask():
+    """A hook on one attention keeps the stock operator and its mask for the whole model; nothing of the unwatched pass stays behind, and both give the same logits up to
+    the rounding of two layers."""
+    model = Transformer(model_mod.ModelArgs(block_size=128, vocab_size=256, n_layer=2, n_head=4, n_local_heads=2, dim=256, intermediate_size=512))
+    init_random_(model, seed=3)
+    model = model.to(device=DEV, dtype=torch.bfloat16).eval()
+    model.setup_caches(3, 64)
+    ids, pos, pads = torch.randint(0, 256, (3, 40), generator=torch.Generator().manual_seed(5)).to(DEV), torch.arange(40, device=DEV), torch.tensor([0, 7, 39], device=DEV)
+    with torch.no_grad():
+        plain = model(ids, pos, pads).float()
+        assert all(blk.attention.mask_of is None for blk in model.layers)
+        seen = []
+        handle = model.layers[1].attention.register_forward_pre_hook(lambda m, args: seen.append(args[2]))
+        watched = model(ids, pos, pads).float()
+        handle.remove()
+        assert torch.equal(model(ids, pos, pads).float(), plain)
+    assert len(seen) == 1 and seen[0].dtype == torch.bool and tuple(seen[0].shape) == (3, 1, 40, 64)
+    assert (plain - watched).norm() <= 2e-2 * watched.norm()
