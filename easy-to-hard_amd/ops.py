@@ -9,7 +9,6 @@ torch.compile(fullgraph=True) and capture into HIP graphs (fixed launch geometry
 allocation outside the caching allocator, kernels on the current stream).
 """
 
-import ctypes
 
 import torch
 
@@ -20,11 +19,20 @@ _VALID_IKT = (2, 4, 8)
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()  # the entry points' argument types turn the number into a pointer
+
+
+# (A call of a small linear is bound by what happens here: a Stream object takes 2 us to make, its handle 0.2.)
+_current_device = torch._C._cuda_getDevice if hasattr(torch._C, "_cuda_getDevice") else torch.cuda.current_device
+if hasattr(torch._C, "_cuda_getCurrentRawStream"):
+    _raw_stream = torch._C._cuda_getCurrentRawStream
+else:
+    def _raw_stream(index):
+        return torch.cuda.current_stream(index).cuda_stream
 
 
 def _stream(t):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return _raw_stream(t.get_device())
 
 
 def _need_gpu(*tensors):
@@ -57,7 +65,7 @@ def _workspace(device):
                 "run one warm-up call before capturing a HIP graph"
             )
         return ws
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index, _raw_stream(device.index))
     ws = _workspaces.get(key)
     if ws is None:
         if ("capture", device.index) not in _workspaces:
@@ -87,7 +95,7 @@ class _OnDevice:
 
 def _lib_for(t):
     lib = _lib.load()
-    if t.device.index == torch.cuda.current_device():
+    if t.get_device() == _current_device():
         return lib
     return _OnDevice(lib, t.device)
 

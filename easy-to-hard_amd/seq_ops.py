@@ -11,7 +11,7 @@ import torch
 from torch.autograd import forward_ad
 
 from . import _lib
-from .ops import _need_gpu, _OnDevice, _stream
+from .ops import _current_device, _need_gpu, _OnDevice, _stream
 
 _DTYPES = {torch.bfloat16: _lib.SEQ_BF16, torch.float32: _lib.SEQ_F32}
 
@@ -24,7 +24,7 @@ def _dtype(t, what):
 
 def _lib_for(t):
     lib = _lib.load_seq()
-    return lib if t.device.index == torch.cuda.current_device() else _OnDevice(lib, t.device)
+    return lib if t.get_device() == _current_device() else _OnDevice(lib, t.device)
 
 
 def _p(t):
