@@ -251,6 +251,28 @@ def test_router(dtype, rows, width, n, top):
     assert np.abs(w - e / e.sum(1, keepdims=True)).max() < 1e-5
 
 
+@BOTH
+@pytest.mark.parametrize("rows,n,top", [(1, 1, 1), (4, 2, 2), (5, 63, 63), (4, 64, 64), (3, 64, 1), (17, 64, 8), (2, 65, 64)])
+def test_router_order_of_ties_and_infinities(dtype, rows, n, top):
+    """A router that copies the row's first channels into the logits: small whole numbers tie in every row, -inf and nan go last in
+    the order of their indices.  The weights are float32 softmax terms: each within 2 units in the last place, their sum of at
+    most 64 as many times 2^-24 more."""
+    x = torch.randint(-3, 4, (rows, 72), generator=torch.Generator().manual_seed(5)).float()
+    bias = torch.zeros(n)
+    if n > 4:
+        bias[n // 2] = float("-inf")
+        bias[1] = float("nan")
+    r = torch.zeros(n, 72)
+    r[torch.arange(n), torch.arange(n)] = 1
+    chosen, weights = seq_ops.route(x.to(DEV, dtype), r.to(DEV, dtype), bias.to(DEV), top)
+    z = x[:, :n] + bias
+    z = torch.where(z > -3e38, z, torch.tensor(-3e38))  # the router's rule for what is no number
+    order = z.sort(dim=1, descending=True, stable=True)
+    assert torch.equal(chosen.cpu().long(), order.indices[:, :top])
+    want = order.values[:, :top].double().softmax(1)
+    assert ((weights.cpu().double() - want).abs() <= (4 + 64) * 2.0 ** -23 * want + 1e-37).all()
+
+
 def test_router_prefers_the_lower_index_of_equal_logits_and_survives_non_numbers():
     x, r = torch.zeros((6, 64), device=DEV), torch.zeros((70, 64), device=DEV)
     chosen, weights = seq_ops.route(x, r, None, 5)
