@@ -222,9 +222,11 @@ __device__ __forceinline__ void update_state(const float *sk, const float *sc, c
   }
 }
 
-// step 1
+// step 1.  Head sizes up to 128 (DT 8) run three waves per SIMD, which no register has to be spilled for; without the bound the
+// compiler moves the state to accumulator registers and keeps two (8192 tokens, 32 heads of 128: 191 us, with it 170).  Larger
+// heads would spill.
 template <typename T, int DT, int VTW, int NW>
-__global__ __launch_bounds__(64 * NW) void hgrn2_chunk_state_kernel(const e2h_hgrn2_args a, ChunkPlan plan) {
+__global__ __launch_bounds__(64 * NW, DT <= 8 ? 3 : 1) void hgrn2_chunk_state_kernel(const e2h_hgrn2_args a, ChunkPlan plan) {
   constexpr int DP = DT * 16, VP = VTW * NW * 16, NT = 64 * NW;
   __shared__ __attribute__((aligned(16))) float sk[kBlockTokens * (DP + 4)], sc[kBlockTokens * (DP + 4)], sv[kBlockTokens * (VP + 4)];
   const int D = static_cast<int>(a.dim), DV = static_cast<int>(a.vdim);
@@ -297,13 +299,15 @@ __global__ __launch_bounds__(256) void hgrn2_scan_kernel(const e2h_hgrn2_args a,
   // the last chunk's own contribution comes from step 3, which starts from the state stored above
 }
 
-// step 3
+// step 3.  Between its barriers a wave waits for LDS and exponentials more than for the matrix cores, so two workgroups per CU are
+// what counts: with 313 registers there was room for one (8192 tokens, 32 heads of 128: 600 us), with the bound for two (430 us).
+// Eight waves with half the value columns each read the same keys twice as often: 550 us.  Heads of more than 128 would spill.
 template <typename T, int DT, int VTW, int NW>
-__global__ __launch_bounds__(64 * NW) void hgrn2_chunk_output_kernel(const e2h_hgrn2_args a, ChunkPlan plan) {
+__global__ __launch_bounds__(64 * NW, DT <= 8 ? 2 : 1) void hgrn2_chunk_output_kernel(const e2h_hgrn2_args a, ChunkPlan plan) {
   constexpr int DP = DT * 16, VP = VTW * NW * 16, NT = 64 * NW;
   constexpr int kLevels = 5;
   __shared__ __attribute__((aligned(16))) float sq[kBlockTokens * (DP + 4)], sk[kBlockTokens * (DP + 4)], sc[kBlockTokens * (DP + 4)];
-  __shared__ __attribute__((aligned(16))) float sv[kBlockTokens * (VP + 4)], sqd[kBlockTokens * (DP + 4)];
+  __shared__ __attribute__((aligned(16))) float sv[kBlockTokens * (VP + 4)];
   __shared__ __attribute__((aligned(16))) float sa[16 * 20], spart[NW][16 * 17], snorm[NW][16];
   const int D = static_cast<int>(a.dim), DV = static_cast<int>(a.vdim), seqlen = static_cast<int>(a.seqlen);
   const int bh_count = static_cast<int>(a.batch * a.heads);
@@ -364,13 +368,10 @@ __global__ __launch_bounds__(64 * NW) void hgrn2_chunk_output_kernel(const e2h_h
         if (t > c && ((t ^ c) >> l) == 1) v = lev[l + 1][r];
       spart[wave][t * 17 + c] = v;
     }
-    for (int i = threadIdx.x; i < kBlockTokens * DP; i += NT) {
-      const int t = i / DP, d = i % DP;
-      sqd[t * (DP + 4) + d] = sq[t * (DP + 4) + d] * __builtin_amdgcn_exp2f(sc[t * (DP + 4) + d]);
-    }
     __syncthreads();
     for (int i = threadIdx.x; i < kBlockTokens * DP; i += NT) {
       const int t = i / DP, d = i % DP;
+      sq[t * (DP + 4) + d] *= __builtin_amdgcn_exp2f(sc[t * (DP + 4) + d]);
       sk[t * (DP + 4) + d] *= __builtin_amdgcn_exp2f(sc[(kBlockTokens - 1) * (DP + 4) + d] - sc[t * (DP + 4) + d]);
     }
     if (threadIdx.x < 256) {
@@ -392,7 +393,7 @@ __global__ __launch_bounds__(64 * NW) void hgrn2_chunk_output_kernel(const e2h_h
     }
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
-      const f32x4_t q = load4(sqd + c * (DP + 4) + dt * 16 + 4 * b4);
+      const f32x4_t q = load4(sq + c * (DP + 4) + dt * 16 + 4 * b4);
 #pragma unroll
       for (int v = 0; v < VTW; ++v) o[v] = mfma4(q, s[dt][v], o[v]);
     }
