@@ -29,7 +29,8 @@
 // Main loop, k in natural order: lane L = 32 h + n supplies column n0 + n and the eight k values 16 s + 8 h .. + 7 of step s.  A packed
 // word (column, j, span p) holds the codes at k = 32 p + 8 i + 2 j + {0, 1} in nibbles i and i + 4, so dword j of the operand of step
 // 2 p + a is word[j][p] rotated right by 8 a + 4 h - 3, masked to bits 3 .. 6 and 19 .. 22, over two bfloat16 sixteens.
-// Four waves, 128 x 256 outputs per workgroup, two workgroups per CU: one's start and end run under the other's matrix work.
+// Four waves, 64, 96 or 128 rows x 256 columns per workgroup (kRT row tiles of 32), two workgroups per CU: one's start and end run under the
+// other's matrix work.
 // Operands reach LDS by 16-byte loads that write LDS directly:
 //   activations, 128 rows x 64 k per chunk, three stages: 1 KB block b holds rows 8 b .. 8 b + 7, the 16-byte pieces of a row stored at
 //   piece ^ ((row >> 1) & 7);
@@ -350,6 +351,10 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
 #pragma unroll
           for (int ct = 0; ct < kCT; ++ct) enter(ct, sc[ct][(s8 + 1) % 8 / SPG % kSc]);
         convert(wf[cur ^ 1], (s8 + 1) & 7);
+        // A product takes 32 clocks and leaves its wave's vector unit free.  Left to itself the compiler issues a step's products in a
+        // row and its vector work behind them, so a wave pays for both; in this order (entering a group first, then a product, an LDS
+        // read, three vector instructions) most of the unpacking runs under the products.  With the 96-row form
+        // 471 x 12288 x 4096, group size 128, went from 69 to 58 us.
         if constexpr (!kGroupSums) {
 #pragma unroll
           for (int i = 0; i < kCT * kRT; ++i) {
@@ -502,8 +507,8 @@ __global__ __launch_bounds__(256) void add_slices_kernel(const float *__restrict
 }  // namespace
 
 // Rows per workgroup and K slices by the least expected time in us, from what was measured at 65 .. 8192 rows of the 7B and 34B shapes:
-// a workgroup takes `one` per 128 k when it has its CU to itself and two that share a CU take `two` (64 rows: 1.2 and 1.95, 128 rows:
-// 1.85 and 3.3), a call 3 more, and slices what their sums cost to write and add.  128 rows win once the chip is full (8192 x 12288 x 4096:
+// a workgroup takes `one` per 128 k when it has its CU to itself and two that share a CU take `two` (64 rows: 1.2 and 1.95, 96 rows:
+// 1.47 and 2.42, 128 rows: 1.85 and 3.3), a call 3 more, and slices what their sums cost to write and add.  128 rows win once the chip is full (8192 x 12288 x 4096:
 // 688 us, 64 rows 795), 64 rows with one slice or several below (471 x 4096 x 4096: two slices 34 us, one 41, 128 rows 63).
 Int4GemmShape int4_gemm_shape(int M, int N, int K, int groupsize, int64_t scratch_bytes) {
   const int KT = K >> 7;
