@@ -138,6 +138,15 @@ def _project_deferred(lin, y2d: Tensor, lead_shape) -> Tensor:
     return lin(y2d.view(*lead_shape, -1))
 
 
+class _MaskByPosition:
+    """Stands in for the mask of one call, causal by input_pos with the call's padding, where the attention kernel takes those instead.  It is an
+    argument like the mask and no state of the modules, so calls of several threads don't see each other's."""
+    __slots__ = ("build", "left_pad")
+
+    def __init__(self, build, left_pad):
+        self.build, self.left_pad = build, left_pad
+
+
 class Attention(nn.Module):
     def __init__(self, config: ModelArgs):
         super().__init__()
@@ -148,7 +157,6 @@ class Attention(nn.Module):
         self.kv_cache = None
         self.freqs_table = None        # full (cos, sin) table, set by Transformer.setup_caches
         self.left_pad_mask_pos = None  # per-step padding mask positions, set by Transformer.forward
-        self.mask_of = None            # while Transformer.forward passes no mask (causal by input_pos, with left_pad_mask_pos): what would build it
         self.n_head = config.n_head
         self.head_dim = config.head_dim
         self.n_local_heads = config.n_local_heads
@@ -212,9 +220,9 @@ class Attention(nn.Module):
                 k, v = self.kv_cache.k_cache, self.kv_cache.v_cache
             q = ops.rope_kv_write_seq(qkv, self.freqs_table, k, v, input_pos, self.n_head, self.n_local_heads, self.head_dim,
                                       rows_by_token=fully_causal)
-            if ((fully_causal or (mask is None and self.mask_of is not None)) and not torch.compiler.is_compiling()
+            if ((fully_causal or isinstance(mask, _MaskByPosition)) and not torch.compiler.is_compiling()
                     and ops.prefill_attention_fits(seqlen, self.n_head, k, v) and not seq_ops.watched(q, k, v)):
-                y = ops.prefill_attention(q, k, v, None if fully_causal else input_pos, None if fully_causal else self.left_pad_mask_pos)
+                y = ops.prefill_attention(q, k, v, None if fully_causal else input_pos, None if fully_causal else mask.left_pad)
                 return self.wo(y)
             k, v = k[:bsz], v[:bsz]
         else:
@@ -228,8 +236,8 @@ class Attention(nn.Module):
         if rep > 1:
             k = k.repeat_interleave(rep, dim=1)
             v = v.repeat_interleave(rep, dim=1)
-        if mask is None and self.mask_of is not None:
-            mask = self.mask_of(input_pos, self.left_pad_mask_pos)
+        if isinstance(mask, _MaskByPosition):
+            mask = mask.build(input_pos, mask.left_pad)
         if fully_causal and q.size(2) == k.size(2):
             y = F.scaled_dot_product_attention(q, k, v, is_causal=True)
         else:
@@ -425,9 +433,9 @@ class Transformer(nn.Module):
         x = self.tok_embeddings(idx)
         mask = None
         fused_step = self.layers[0].attention.can_fuse_decode(x, fully_causal)
-        by_position = not fully_causal and not fused_step and self._masks_by_position(x, input_pos)
-        if not fully_causal and not fused_step and not by_position:
-            mask = self._mask(input_pos, left_pad_mask_pos)
+        if not fully_causal and not fused_step:
+            by_position = self._masks_by_position(x, input_pos)
+            mask = _MaskByPosition(self._mask, left_pad_mask_pos) if by_position else self._mask(input_pos, left_pad_mask_pos)
         freqs_cis = None if fused_step else self.freqs_cis[input_pos].to(dtype=x.dtype)
         if fused_step and input_pos.dtype != torch.int64:
             # the reference decodes with an int32 position tensor (inference_generate.py:205); the fused kernels read int64
@@ -446,23 +454,15 @@ class Transformer(nn.Module):
                 return ops.int4_mm_staged(xs, out.weight, out.groupsize, out.scales_and_zeros).view(rows, 1, -1)
             _, normed = ops.add_rmsnorm(h, delta, self.norm.weight, self.norm.eps)
             return self.output(normed.view(rows, 1, -1))
-        if by_position:
-            for blk in self.layers:
-                blk.attention.mask_of = self._mask
-        try:
-            if _fusable(x) and x.shape[-1] % 8 == 0 and self.norm.weight.dtype == torch.bfloat16:
-                delta = None
-                for layer in self.layers:
-                    x, delta = layer.forward_deferred(x, delta, input_pos, freqs_cis, mask, fully_causal)
-                _, normed = ops.add_rmsnorm(x, delta, self.norm.weight, self.norm.eps)
-                return self.output(normed)
+        if _fusable(x) and x.shape[-1] % 8 == 0 and self.norm.weight.dtype == torch.bfloat16:
+            delta = None
             for layer in self.layers:
-                x = layer(x, input_pos, freqs_cis, mask, fully_causal)
-            return self.output(self.norm(x))
-        finally:
-            if by_position:
-                for blk in self.layers:
-                    blk.attention.mask_of = None
+                x, delta = layer.forward_deferred(x, delta, input_pos, freqs_cis, mask, fully_causal)
+            _, normed = ops.add_rmsnorm(x, delta, self.norm.weight, self.norm.eps)
+            return self.output(normed)
+        for layer in self.layers:
+            x = layer(x, input_pos, freqs_cis, mask, fully_causal)
+        return self.output(self.norm(x))
 
     def _mask(self, input_pos: Tensor, left_pad_mask_pos: Optional[Tensor]) -> Tensor:
         mask = self.causal_mask[None, None, input_pos]

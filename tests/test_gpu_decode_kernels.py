@@ -241,7 +241,7 @@ def test_prefill_attention_against_float64(h, hkv, d, t, start, s_len):
 
 
 def test_prompts_of_a_watched_attention_are_shown_the_mask():
-    """A hook on one attention keeps the stock operator and its mask for the whole model; nothing of the unwatched pass stays behind, and both give the same logits up to
+    """A hook on one attention keeps the stock operator and its mask for the whole model, and both give the same logits up to
     the rounding of two layers."""
     model = Transformer(model_mod.ModelArgs(block_size=128, vocab_size=256, n_layer=2, n_head=4, n_local_heads=2, dim=256, intermediate_size=512))
     init_random_(model, seed=3)
@@ -250,7 +250,6 @@ def test_prompts_of_a_watched_attention_are_shown_the_mask():
     ids, pos, pads = torch.randint(0, 256, (3, 40), generator=torch.Generator().manual_seed(5)).to(DEV), torch.arange(40, device=DEV), torch.tensor([0, 7, 39], device=DEV)
     with torch.no_grad():
         plain = model(ids, pos, pads).float()
-        assert all(blk.attention.mask_of is None for blk in model.layers)
         seen = []
         handle = model.layers[1].attention.register_forward_pre_hook(lambda m, args: seen.append(args[2]))
         watched = model(ids, pos, pads).float()
@@ -258,3 +257,26 @@ def test_prompts_of_a_watched_attention_are_shown_the_mask():
         assert torch.equal(model(ids, pos, pads).float(), plain)
     assert len(seen) == 1 and seen[0].dtype == torch.bool and tuple(seen[0].shape) == (3, 1, 40, 64)
     assert (plain - watched).norm() <= 2e-2 * watched.norm()
+
+
+def test_a_prompt_keeps_its_padding_while_another_call_runs():
+    """A call of the same model without padding, made between the layers of a padded prompt (as another thread's may be), leaves the
+    prompt's logits as they are: the second layer still sees this call's padding."""
+    model = Transformer(model_mod.ModelArgs(block_size=128, vocab_size=256, n_layer=2, n_head=4, n_local_heads=2, dim=256, intermediate_size=512))
+    init_random_(model, seed=3)
+    model = model.to(device=DEV, dtype=torch.bfloat16).eval()
+    model.setup_caches(3, 64)
+    ids, pos, pads = torch.randint(0, 256, (3, 40), generator=torch.Generator().manual_seed(5)).to(DEV), torch.arange(40, device=DEV), torch.tensor([0, 7, 39], device=DEV)
+    inner = []
+
+    def between(*_):
+        if not inner:
+            inner.append(None)
+            inner[0] = model(ids, pos)
+
+    with torch.no_grad():
+        plain = model(ids, pos, pads)
+        handle = model.layers[0].feed_forward.register_forward_pre_hook(between)
+        got = model(ids, pos, pads)
+        handle.remove()
+    assert torch.equal(got, plain) and not torch.equal(inner[0], plain)
