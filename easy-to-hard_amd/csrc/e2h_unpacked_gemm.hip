@@ -9,12 +9,14 @@
 // s (q - 8) is an eight-bit significand times a three-bit integer (or eight): it fits the eleven bits of a float16, and x (eight bits) does too.  So both become
 // float16 without rounding, a row of x and a column of weights each in units of a power of two of its own that puts its largest value near the
 // type's end; products are exact and sums float32, as in the kernel that multiplies codes (e2h_int4_gemm.hip: 1.1 - 1.2 PFLOP/s, bound by unpacking and rescaling
-// beside the products).  The zero-point term is three more columns per group: X split exactly into three float16 parts (an infinity of them
-// apart, which the next paragraph keeps out), against z three times.  K grows by 2.4 % at group size 128.
+// beside the products).  The zero-point term is three more columns per group: X as g p0 + p1 + p2 of float16 values, against g z, z and z.  K grows by 2.4 % at
+// group size 128.
+// A value of x below about 2^-30 of its row's largest can have bits that its float16 does not hold, and so can the sum of a group of such values.  What is lacking
+// stands in a list of the row's, and the store adds its products in float32 before the rounding (ordinary activations have such a value in one row of ten thousand).
 // What does not fit is multiplied by that other kernel: the passes that unpack raise a flag at a scale or zero that is not finite, would be rounded
-// (2^-28 of its column's largest) or lies outside 2^-48 .. 2^27 or so, at a value of x that is not finite, and at a row of x of which a sixteenth is
-// smaller than 2^-31 of its largest value; up to there what is rounded is less than 2^-39 of the row's largest value, below the rounding of
-// float32 sums that hold it.  With the flag the product's workgroups end at once, without it those of the other kernel do.
+// (a scale below about 2^-28, a zero below 2^-31 of the larger of its column's 8 s and g z) or whose column's largest such value lies outside 2^-46 .. 2^45, at a value
+// or group sum of x that is not finite, and at a row of x with more lacking values than its list holds.  With the flag the product's workgroups end at once, without
+// it those of the other kernel do.
 #include <algorithm>
 
 #include "e2h_common.h"
@@ -144,10 +146,17 @@ __device__ __forceinline__ uint32_t pack_f16(float lo, float hi) {  // round to 
 constexpr int kTopX = 13, kTopW = 15;  // largest value of a row of x: 2^kTopX .. 2^(kTopX + 1); of a column: below 2^kTopW
 constexpr float kWhole = 0x1p-17f;     // eight bits from here on fit a float16
 
+struct Lacking {
+  int at;    // column of the extended K
+  float by;  // value of x, or sum of a group, less what its float16 values hold
+};
+constexpr int kMostLacking = 16;
+
 struct Int4Scratch {
   int *flag;         // [1] this call needs the other kernel
-  int *row_exp;      // [M] x is multiplied by 2^row_exp
+  int *row_exp;      // [M] low half: x is multiplied by 2^that; high half: entries of the row's list
   int *row_flag;     // [M]
+  Lacking *lacking;  // [M][kMostLacking]
   float *col_unit;   // [N] what one step of a column's sums is worth
   float *xsum;       // [K / G][stride] group sums, for the other kernel
   uint16_t *x, *w;   // [M][KE], [N][KE]
@@ -169,6 +178,7 @@ Int4Scratch int4_scratch(uint8_t *base, int64_t M, int64_t N, int64_t K, int gro
   s.flag = reinterpret_cast<int *>(take(4));
   s.row_exp = reinterpret_cast<int *>(take(M * 4));
   s.row_flag = reinterpret_cast<int *>(take(M * 4));
+  s.lacking = reinterpret_cast<Lacking *>(take(M * kMostLacking * static_cast<int64_t>(sizeof(Lacking))));
   s.col_unit = reinterpret_cast<float *>(take(N * 4));
   s.xsum = reinterpret_cast<float *>(take(K / G * sum_stride(M) * 4));
   s.x = reinterpret_cast<uint16_t *>(take(M * KE * 2));
@@ -207,42 +217,63 @@ __global__ __launch_bounds__(256) void int4_unpack_x_kernel(const uint16_t *__re
   const bool finite = top < 0x7F80u;
   const int up = top == 0 || !finite ? 0 : kTopX - exponent_of(bf16_to_f32(static_cast<uint16_t>(top)));
   uint16_t *out = s.x + static_cast<size_t>(m) * KE;
-  int lost = 0;
+  Lacking *list = s.lacking + static_cast<size_t>(m) * kMostLacking;
+  int lacking = 0;  // entries so far, in lane 0, which takes part in every round
+  bool endless = !finite;
+  const auto enter = [&](int at, float by) {  // of the lanes here, those whose `by` is not zero
+    const uint64_t all = __builtin_amdgcn_ballot_w64(by != 0.f);
+    const int i = lacking + __builtin_popcountll(all & ((uint64_t{1} << lane) - 1));
+    if (by != 0.f && i < kMostLacking) list[i] = Lacking{at, by};
+    lacking += __builtin_popcountll(all);
+  };
 #pragma unroll 2
   for (int p = lane; p < pieces; p += 64) {
     const u32x4_t v = row[p];
     u32x4_t h;
     float sum[4];
+    bool small = false;
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
       const float a = __builtin_bit_cast(float, v[d] << 16), b = __builtin_bit_cast(float, v[d] & 0xFFFF0000u);
       sum[d] = a + b;
       const float as = __builtin_ldexpf(a, up), bs = __builtin_ldexpf(b, up);
-      lost += (as != 0.f && __builtin_fabsf(as) < kWhole) + (bs != 0.f && __builtin_fabsf(bs) < kWhole);
+      small |= (a != 0.f && __builtin_fabsf(as) < kWhole) || (b != 0.f && __builtin_fabsf(bs) < kWhole);
       h[d] = pack_f16(as, bs);
     }
     reinterpret_cast<u32x4_t *>(out)[p] = h;
+    if (__builtin_amdgcn_ballot_w64(small)) {  // hardly ever
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const uint32_t pair = h[d];  // (a bit cast of the element itself reads the vector's first one)
+        const f16x2_t held = __builtin_bit_cast(f16x2_t, pair);
+        enter(8 * p + 2 * d, __builtin_bit_cast(float, v[d] << 16) - __builtin_ldexpf(static_cast<float>(held[0]), -up));
+        enter(8 * p + 2 * d + 1, __builtin_bit_cast(float, v[d] & 0xFFFF0000u) - __builtin_ldexpf(static_cast<float>(held[1]), -up));
+      }
+    }
     float t = (sum[0] + sum[1]) + (sum[2] + sum[3]);
 #pragma unroll
     for (int off = 1; off < G / 8; off <<= 1) t += __shfl_xor(t, off);  // the lanes of a group are all here or none
+    const int g = p / (G / 8);
+    const float ts = __builtin_ldexpf(t, up);
+    const _Float16 p0 = static_cast<_Float16>(ts * (1.0f / G));
+    const float r = ts - static_cast<float>(p0) * G;
+    const _Float16 p1 = static_cast<_Float16>(r), p2 = static_cast<_Float16>(r - static_cast<float>(p1));
+    endless |= !__builtin_isfinite(t);
+    float by = 0.f;
     if (lane % (G / 8) == 0) {
-      const int g = p / (G / 8);
       s.xsum[static_cast<size_t>(g) * stride + m] = t;
-      const float ts = __builtin_ldexpf(t, up) * (1.0f / G);
-      const _Float16 p0 = static_cast<_Float16>(ts);
-      const float r = ts - static_cast<float>(p0);
-      const _Float16 p1 = static_cast<_Float16>(r), p2 = static_cast<_Float16>(r - static_cast<float>(p1));
       out[K + 3 * g] = __builtin_bit_cast(uint16_t, p0);
       out[K + 3 * g + 1] = __builtin_bit_cast(uint16_t, p1);
       out[K + 3 * g + 2] = __builtin_bit_cast(uint16_t, p2);
+      by = t - __builtin_ldexpf((static_cast<float>(p0) * G + static_cast<float>(p1)) + static_cast<float>(p2), -up);
     }
+    if (__builtin_amdgcn_ballot_w64(by != 0.f)) enter(K + 3 * g + 1, by);
   }
   for (int k = K + 3 * (K / G) + lane; k < KE; k += 64) out[k] = 0;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) lost += __shfl_xor(lost, off);
+  const bool odd = __builtin_amdgcn_ballot_w64(endless) != 0 || lacking > kMostLacking;
   if (lane == 0) {
-    s.row_exp[m] = up;
-    s.row_flag[m] = !finite || lost * 16 > K;
+    s.row_exp[m] = (up & 0xFFFF) | (odd ? 0 : lacking << 16);
+    s.row_flag[m] = odd;
   }
 }
 
@@ -283,11 +314,12 @@ __global__ __launch_bounds__(256) void int4_unpack_w_kernel(const uint32_t *__re
     for (int g = g1; g < groups; g += 16) {
       const uint32_t pair = sz[static_cast<size_t>(g >> twice) * N + col0 + c1];
       const float scale = __builtin_bit_cast(float, pair << 16), zero = __builtin_bit_cast(float, pair & 0xFFFF0000u);
-      const float a = __builtin_fabsf(__builtin_ldexpf(scale, up1)), z = __builtin_ldexpf(zero, up1) * static_cast<float>(G);
+      const float a = __builtin_fabsf(__builtin_ldexpf(scale, up1)), z = __builtin_ldexpf(zero, up1);
       odd |= (scale != 0.f && a < kWhole) || (zero != 0.f && __builtin_fabsf(z) < kWhole);
       if (blockIdx.y == 0) {
         uint16_t *ext = s.w + static_cast<size_t>(col0 + c1) * KE + K + 3 * g;
-        ext[0] = ext[1] = ext[2] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(z));
+        ext[0] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(z * static_cast<float>(G)));
+        ext[1] = ext[2] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(z));
       }
     }
   if (blockIdx.y == 0 && live1) {
@@ -323,10 +355,12 @@ __global__ __launch_bounds__(256) void int4_unpack_w_kernel(const uint32_t *__re
 struct Int4Walk : PlainWalk {
   const float *col_unit;
   const int *row_exp;
-  __device__ __forceinline__ Int4Walk(const Int4Scratch &s, uint16_t *y_, int M_, int N_, int KE) : PlainWalk(s.x, s.w, y_, M_, N_, KE), col_unit(s.col_unit), row_exp(s.row_exp) {}
+  const Lacking *lacking;
+  __device__ __forceinline__ Int4Walk(const Int4Scratch &s, uint16_t *y_, int M_, int N_, int KE)
+      : PlainWalk(s.x, s.w, y_, M_, N_, KE), col_unit(s.col_unit), row_exp(s.row_exp), lacking(s.lacking) {}
   struct Dest {
     f32x4_t unit[4][2];  // of the eight columns of each store of a row
-    int up[8];           // of the rows
+    int up[8];           // row_exp of the rows
   };
   __device__ __forceinline__ void dest(const Tile &tile, int row, int col, Dest &d) const {
 #pragma unroll
@@ -345,7 +379,22 @@ struct Int4Walk : PlainWalk {
   __device__ __forceinline__ void store(const Tile &tile, const Dest &d, int j, int q, int row, int col, float (&v)[8]) const {
     u32x4_t out;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = __builtin_ldexpf(v[e] * d.unit[q][e >> 2][e & 3], -d.up[j]);
+    for (int e = 0; e < 8; ++e) v[e] = __builtin_ldexpf(v[e] * d.unit[q][e >> 2][e & 3], -static_cast<int>(static_cast<int16_t>(d.up[j])));
+    if (__builtin_expect(d.up[j] >= 1 << 16, 0)) {
+      const int m = tile.rb * 256 + row, n = tile.cb * 256 + col;
+      const Lacking *list = lacking + static_cast<size_t>(m < M ? m : M - 1) * kMostLacking;
+      const __amdgpu_buffer_rsrc_t wr = w_rsrc(tile);
+#pragma unroll 1
+      for (int i = 0; i < d.up[j] >> 16; ++i) {
+        const Lacking l = list[i];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {  // (columns past N: of column 0, not stored)
+          const uint32_t at = (static_cast<uint32_t>(n < N ? n + e : 0) * static_cast<uint32_t>(K) + static_cast<uint32_t>(l.at)) * 2;
+          const float w = static_cast<float>(__builtin_bit_cast(_Float16, __builtin_amdgcn_raw_buffer_load_b16(wr, at, 0, 0)));
+          v[e] = __builtin_fmaf(l.by, w * d.unit[q][e >> 2][e & 3], v[e]);
+        }
+      }
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) out[e] = pack_bf16(v[2 * e], v[2 * e + 1]);
     __builtin_amdgcn_raw_buffer_store_b128(out, y_rsrc(tile), y_at(tile, row, col), 0, 0);

@@ -185,8 +185,9 @@ def test_a_row_differs_by_float32_rounding_at_most_between_row_counts(g, n, k):
 
 # ---- weights unpacked to float16 first (csrc/e2h_unpacked_gemm.hip) ---------------------------------------------------------------------
 
-def _unpacked(codes, scale, zero, x, g):
-    """(with scratch memory, without, bytes of it), through the C interface"""
+def _unpacked(codes, scale, zero, x, g, flag=None):
+    """(with scratch memory, without, bytes of it), through the C interface; flag: a list that is given the scratch memory's first number, not zero where the other
+    kernel was asked for"""
     lib = _lib.load()
     packed = torch.from_numpy(qo.int4_tile_pack(codes.numpy(), 8)).to(DEV)
     sz = torch.stack([scale, zero], dim=-1).to(torch.bfloat16).contiguous().to(DEV)
@@ -198,6 +199,8 @@ def _unpacked(codes, scale, zero, x, g):
         y = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
         rc = lib.e2h_int4_mm_scratch(ops._ptr(x), ops._ptr(packed), ops._ptr(sz), ops._ptr(y), m, n, k, g, 8, ops._ptr(ws), ws.numel(), ops._ptr(scratch), given, ops._stream(x))
         assert rc == 0
+        if flag is not None and given:
+            flag.append(int(scratch[:4].view(torch.int32)))
         out.append(y)
     return (*out, need)
 
@@ -230,6 +233,7 @@ def test_unpacked_weights_round_once(g):
     codes = torch.randint(0, 16, (n, k), generator=gen, dtype=torch.int32)
     scale = torch.exp2(torch.rand((k // g, n), generator=gen) * 20 - 20).to(torch.bfloat16).float()
     zero = (torch.randn((k // g, n), generator=gen) * 8 * scale).to(torch.bfloat16).float()
+    zero[zero.abs() < 2.0**-30 * torch.maximum(8 * scale, 128 * zero.abs()).max(0).values] = 0.0  # smaller ones send the call to the other kernel
     x = torch.exp2(torch.randint(-28, 1, (m, k), generator=gen).float() + torch.randint(-60, 61, (m, 1), generator=gen).float()).to(torch.bfloat16)
     x = (x * (torch.randint(0, 2, (m, k), generator=gen) * 2 - 1)).to(DEV)
     x[5] = 0
@@ -240,6 +244,26 @@ def test_unpacked_weights_round_once(g):
     terms = (x[rows].double().abs() @ ((codes.double() - 8).abs().view(n, k // g, g) * scale.double().t()[:, :, None] + zero.double().abs().t()[:, :, None]).view(n, k).to(DEV).t())
     assert need > 0 and bool((err <= 2**-8 * size + 2**-15 * terms).all()) and bool((got[5] == 0).all())
     assert (err / terms.clamp(min=1e-300)).mean() < 2**-9
+
+
+@pytest.mark.parametrize("count", [14, 15])
+def test_unpacked_x_keeps_what_its_float16_values_lack(count):
+    """Values of x far below their row's largest, which meets a group whose scale and zero are zero in the first columns: there they alone are the result.  One to fourteen of
+    them in one and two groups, which with the groups' sums a row's list of sixteen holds, and fifteen in three, which it does not; up to 2^-174 of the largest.  2^-31 of it
+    is held by the float16 values themselves.  Every sum is of at most 16 multiples of one power of two, so the result is the exactly rounded one."""
+    m, n, k, g = 66049, 264, 512, 128
+    codes, scale, zero, x = _case(m, n, k, g)
+    scale[0, :130], zero[0, :130] = 0.0, 0.0
+    special = {0: (2.0**110, 2.0**-64, 10), 77: (1.0, 2.0**-40, 1), 300: (-1.0, -(2.0**-31), 16), 4097: (2.0**40, 3 * 2.0**-20, count), m - 1: (2.0**-30, 2.0**-70, 5)}
+    for row, (largest, small, n_small) in special.items():
+        x[row] = 0
+        x[row, row % g] = largest
+        x[row, k - 1 - 19 * torch.arange(n_small)] = small
+    flag = []
+    got, _, need = _unpacked(codes, scale, zero, x, g, flag)
+    rows = torch.tensor(list(special) + [1, 78, 4096, m - 2], device=DEV)
+    assert need > 0 and (flag[0] != 0) == (count > 14)
+    assert torch.equal(got[rows][:, :130], _double(codes, scale, zero, x, g, rows)[:, :130].to(torch.bfloat16))
 
 
 @pytest.mark.parametrize("what", ["scale ratio", "infinite scale", "NaN zero", "tiny zero", "large scales", "small scales", "infinite x", "NaN x", "small x"])
