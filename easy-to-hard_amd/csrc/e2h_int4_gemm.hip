@@ -80,7 +80,7 @@ struct GemmArgs {
   const float *xsum;
   int xsum_stride, M, N, K, n_col_blocks, cbx;
   int shared;         // 1: two neighbouring groups have one (scale, zero) pair (group size 256), else 0
-  const int *run_if;  // not null: nothing is done where it holds zero
+  const int *run_if, *row_flag;  // not null: run_if[0] = 1 asks for everything, 2 for the rows m with row_flag[m] only, 0 for nothing
 };
 
 // kRT row tiles of 32 per wave: 32 kRT rows x 256 columns per workgroup
@@ -92,8 +92,6 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
   constexpr bool kGroupSums = G == 32;         // a group's products in registers of their own, scaled when it ends
   __shared__ __attribute__((aligned(1024))) uint8_t lds[kLdsBytes];
   const int M = a.M, N = a.N, K = a.K;
-  if (a.run_if && *a.run_if == 0) return;  // the whole grid
-
   const int xcd = blockIdx.x & 7;
   const int slot = blockIdx.x >> 3;
   const int cb = xcd + 8 * (slot % a.cbx), rb = slot / a.cbx;
@@ -103,6 +101,17 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
   const int row0 = rb * kRows, col0 = cb * kCols + 64 * wave;
+  const int *only = nullptr;
+  if (a.run_if) {
+    const int asked = *a.run_if;
+    if (asked == 0) return;  // the whole grid
+    if ((asked & 1) == 0) {
+      int any = 0;
+      for (int r = lane; r < kRows; r += 64) any |= row0 + r < M ? a.row_flag[row0 + r] : 0;
+      if (__builtin_amdgcn_ballot_w64(any != 0) == 0) return;  // the whole workgroup
+      only = a.row_flag;
+    }
+  }
   const int KT = K >> 7;
   const int blk0 = static_cast<int>((static_cast<int64_t>(KT) * blockIdx.y) / gridDim.y);
   const int blk1 = static_cast<int>((static_cast<int64_t>(KT) * (blockIdx.y + 1)) / gridDim.y);
@@ -421,7 +430,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
       }
       const float no_scale[kCT] = {};
       store_tiles_via_lds<kRT, kCT, false>(acc, no_scale, lds + wave * TileStore<kCT>::kBytesPerWave, a.y, row0, col0, M, N, lane,
-                                          (N & 7) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0);
+                                          (N & 7) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0, only);
       return;
     }
   }
@@ -480,7 +489,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int m = r0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3);
-        if (m >= M || m >= row0 + kRows) continue;
+        if (m >= M || m >= row0 + kRows || (only && !only[m])) continue;
         if (a.partials) a.partials[(static_cast<size_t>(blockIdx.y) * M + m) * N + col] = sum[rt][e];
         else a.y[static_cast<size_t>(m) * N + col] = f32_to_bf16_rne(sum[rt][e]);
       }
@@ -548,12 +557,12 @@ void launch_gemm(const GemmArgs &a, int rows, dim3 grid, hipStream_t stream) {
 }
 
 int int4_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint16_t *y, const float *xsum, int xsum_stride,
-              float *partials, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream, const int *run_if) {
+              float *partials, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream, const int *run_if, const int *row_flag) {
   if (K % 128 != 0 || N % 8 != 0) return E2H_ERR_BAD_SHAPE;
   const int shared = groupsize == 256;
   if (shared) groupsize = 128;
   GemmArgs a = {x, reinterpret_cast<const uint32_t *>(packed), reinterpret_cast<const uint32_t *>(sz), y, shape.slices > 1 ? partials : nullptr,
-                xsum, xsum_stride, M, N, K, (N + kCols - 1) / kCols, 0, shared, run_if};
+                xsum, xsum_stride, M, N, K, (N + kCols - 1) / kCols, 0, shared, run_if, row_flag};
   a.cbx = (a.n_col_blocks + 7) / 8;
   const long long wgs = 8LL * a.cbx * ((M + shape.rows - 1) / shape.rows);
   if (wgs > 0x7FFFFFFFLL) return E2H_ERR_BAD_SHAPE;

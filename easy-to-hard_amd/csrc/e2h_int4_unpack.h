@@ -35,6 +35,7 @@ __device__ __forceinline__ bf16x8_t unpack_word(uint32_t w, const UnpackConsts &
 // instruction).  kScale: the int8 contract y = bf16(bf16(acc) * scale[column]); otherwise y = bf16(acc).
 // pieces (uniform): N % 8 == 0 and y 16-byte aligned, so that every piece is one aligned 16-byte store; otherwise the
 // eight values of a piece leave one by one, bounds-checked against N.
+// only: not null, rows m with only[m] = 0 are not stored.
 typedef float e2h_float2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 e2h_bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float e2h_f32x16_t __attribute__((ext_vector_type(16)));
@@ -52,7 +53,7 @@ __device__ __forceinline__ uint32_t pack_bf16x2_rne(float a, float b) {
 template <int RT, int CT, bool kScale>
 __device__ __forceinline__ void store_tiles_via_lds(const e2h_f32x16_t (&acc)[CT][RT], const float (&scale)[CT], uint8_t *tile,
                                                     uint16_t *__restrict__ y, int row0, int col0, int M, int N, int lane,
-                                                    bool pieces) {
+                                                    bool pieces, const int *only = nullptr) {
   constexpr int kTileStride = TileStore<CT>::kTileStride;
   constexpr int kPiecesPerRow = 4 * CT;             // 16-byte pieces per tile row
   constexpr int kRowsPerPass = 64 / kPiecesPerRow;  // tile rows one 64-lane read covers
@@ -82,7 +83,7 @@ __device__ __forceinline__ void store_tiles_via_lds(const e2h_f32x16_t (&acc)[CT
       const int trow = pass * kRowsPerPass + lane / kPiecesPerRow, piece = lane % kPiecesPerRow;
       const u32x4_t v = *reinterpret_cast<const u32x4_t *>(tile + trow * kTileStride + piece * 16);
       const int row = row0 + 32 * rt + trow, col = col0 + 8 * piece;
-      if (row < M && col < N) {
+      if (row < M && col < N && (!only || only[row])) {
         uint16_t *dst = y + static_cast<size_t>(row) * N + col;
         if (pieces) {
           __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t *>(dst));  // streamed: the tiles in L2 are the operands
@@ -102,14 +103,15 @@ int launch_x_group_sums(const uint16_t *x, float *out, int M, int K, int stride,
 
 // Many-row int4 matmul on 32x32 MFMA tiles (e2h_int4_gemm.hip); xsum as written by launch_x_group_sums (for group size 256: of 128).  A workgroup owns `rows` rows;
 // K may be shared by `slices` of them through float32 sums in `partials` ([slices][M][N]; unused with one slice).  int4_gemm_shape picks
-// both, with at most as many slices as fit scratch_bytes.  run_if, in device memory: the launch does nothing where it holds zero (one slice only).
+// both, with at most as many slices as fit scratch_bytes.  run_if and row_flag, in device memory (one slice only): where run_if holds 1 the launch does everything,
+// where 2 the rows m whose row_flag[m] is not zero, where 0 nothing.
 struct Int4GemmShape {
   int rows, slices;
   double us;  // expected time
 };
 Int4GemmShape int4_gemm_shape(int M, int N, int K, int groupsize, int64_t scratch_bytes);
 int int4_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint16_t *y, const float *xsum, int xsum_stride,
-              float *partials, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream, const int *run_if = nullptr);
+              float *partials, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream, const int *run_if = nullptr, const int *row_flag = nullptr);
 
 // Many-row int4 matmul, 256 x 256 outputs per workgroup, weights dequantized to bfloat16 on the way into the matrix
 // cores (e2h_int4_gemm128.hip); needs no scratch memory.

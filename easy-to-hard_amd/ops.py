@@ -128,7 +128,8 @@ _UNPACK_ROWS = 1024  # no smaller call is offered scratch memory
 
 
 def _unpacked_weight(m, device, query, *sizes):
-    """Scratch for the 16-bit weights of a call with many rows, or None: the sizes are not for that form, or there is no memory left for it."""
+    """Scratch for the 16-bit weights of a call with many rows, or None: the sizes are not for that form, or there is no memory left for it (the
+    call then adds the same products in another order, which float32 rounding may show)."""
     if m < _UNPACK_ROWS:
         return None
     need = query(m, *sizes)

@@ -149,7 +149,8 @@ int e2h_int4_mm(const uint16_t *x, const int32_t *packed, const uint16_t *scales
 /* The same for callers with memory to spare: over thousands of rows x and the weights are first unpacked to 16-bit values in `scratch` (16-byte
  * aligned, shared by nobody while the call runs), of which e2h_int4_mm_scratch_bytes says how much is used (0: this shape runs as above; not in the count:
  * workspace, as above).  Products are exact, sums float32 and rounded once, as above: what 16-bit values do not hold of a row of x is multiplied
- * by itself where it is little, and runs on the kernels above otherwise, as scales and zeros do that they do not hold.  With less scratch, or a y that is not 16-byte aligned, the call is e2h_int4_mm. */
+ * by itself where it is little, and runs on the kernels above otherwise, as scales and zeros do that they do not hold. A row's result does not depend on
+ * what stands in other rows; as above it may differ by float32 rounding with another number of rows, and with or without scratch.  With less scratch, or a y that is not 16-byte aligned, the call is e2h_int4_mm. */
 int64_t e2h_int4_mm_scratch_bytes(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles);
 int e2h_int4_mm_scratch(const uint16_t *x, const int32_t *packed, const uint16_t *scales_and_zeros, uint16_t *y, int64_t m, int64_t n,
                         int64_t k, int groupsize, int inner_k_tiles, void *workspace, int64_t workspace_bytes, void *scratch,

@@ -296,6 +296,36 @@ def test_what_float16_does_not_hold_is_left_to_the_other_kernel(what):
     assert bool(same.all())
 
 
+@pytest.mark.parametrize("g", [32, 128])
+def test_rows_of_an_unpacked_call_stand_alone(g):
+    """Rows that the float16 form does not take (a NaN, an infinity, values over 2^60) leave every other row as it is without them, bit for bit, first, last and
+    neighbours of them included, with operands whose sums are rounded.  The wide rows are as exact as float32 sums are: K = 512 terms, each within 2^-15 of the magnitudes added."""
+    m, n, k = 66049, 264, 512
+    gen = torch.Generator().manual_seed(g)
+    codes = torch.randint(0, 16, (n, k), generator=gen, dtype=torch.int32)
+    scale = (torch.rand((k // g, n), generator=gen) * 0.02 + 0.01).to(torch.bfloat16).float()
+    zero = (torch.randn((k // g, n), generator=gen) * 0.02).to(torch.bfloat16).float()
+    x = torch.randn((m, k), generator=gen).to(torch.bfloat16).to(DEV)
+    flag = []
+    plain, _, need = _unpacked(codes, scale, zero, x, g, flag)
+    wide = [1, 128, 40000, *range(512, 768)]  # a whole block of the product's rows among them
+    odd = [0, 127, 4100, m - 1]
+    for row in wide:
+        x[row] *= torch.exp2(torch.randint(-60, 1, (k,), generator=gen).float()).to(torch.bfloat16).to(DEV)
+    x[0, 3] = x[127, 511] = float("nan")
+    x[4100, 7] = x[m - 1, 0] = float("inf")
+    got, _, _ = _unpacked(codes, scale, zero, x, g, flag)
+    assert need > 0 and flag == [0, 2]
+    rest = torch.ones(m, dtype=torch.bool)
+    rest[wide + odd] = False
+    assert torch.equal(got[rest], plain[rest])
+    assert not torch.isfinite(got[odd]).any()
+    w = torch.tensor(wide, device=DEV)
+    want = _double(codes, scale, zero, x, g, w)
+    size = ((codes.double() + 24).view(n, k // g, g) * scale.double().t()[:, :, None] + zero.double().abs().t()[:, :, None]).view(n, k).to(DEV)
+    assert bool(((got[w].double() - want).abs() <= 2**-8 * want.abs() + 2**-15 * (x[w].double().abs() @ size.t())).all())
+
+
 @pytest.mark.parametrize("g,m,n,k", [(64, 470, 12296, 640), (128, 470, 12296, 384), (256, 470, 12296, 768)])
 def test_odd_scales_in_96_row_workgroups(g, m, n, k):
     """471 rows of 12288 columns are work for five rows of workgroups; the plain loop walks pairs of row tiles, of which the last holds one"""
