@@ -665,7 +665,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const uint16_
   const size_t head = (static_cast<size_t>(b) * Hkv + hk) * S * D;
   f32x4_t o[2][VT];
   float m[2], l[2];
-  attention::attend<D, false>(qf, pos, lo, hi, keys, rule, scale * attention::kLog2E, kc + head, vc + head, static_cast<uint32_t>(S), lds, o, m, l);
+  attention::attend<D, false, true>(qf, pos, lo, hi, keys, rule, scale * attention::kLog2E, kc + head, vc + head, static_cast<uint32_t>(S), lds, o, m, l);
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int t = t0 + wave * 32 + 16 * i + c;

@@ -15,7 +15,7 @@ namespace e2h {
 namespace attention {
 
 constexpr int kQueries = 128, kKeys = 64;
-constexpr float kMaskedScore = -1e30f, kLog2E = 1.4426950408889634f;
+constexpr float kMaskedScore = -__builtin_inff(), kLog2E = 1.4426950408889634f;
 template <int D>
 constexpr int kLdsBytes = 2 * 2 * kKeys * D * 2;
 
@@ -74,10 +74,72 @@ __device__ __forceinline__ void weights(const float (&p)[8], bf16x8_t &hi, bf16x
   lo = __builtin_bit_cast(bf16x8_t, l);
 }
 
+// The same result for one wave without LDS, fragments straight from memory, scores taken relative to the largest one before anything is multiplied: for scores of any
+// size.  Two walks over the keys, the first for the largest scores.
+template <int D>
+__device__ __forceinline__ void attend_far(const bf16x8_t (&qf)[2][D / 32], const int (&pos)[2], const Keys &kl, const Rule &rule, float sc, const uint16_t *kc, const uint16_t *vc,
+                                           f32x4_t (&o)[2][D / 16], float (&m)[2], float (&l)[2]) {
+  constexpr int KS = D / 32, VT = D / 16;
+  const int lane = threadIdx.x & 63, c = lane & 15, b4 = lane >> 4;
+  const auto key = [&](int n) { return kl.at(n < kl.count ? n : kl.count - 1); };
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    m[i] = kMaskedScore;
+    l[i] = 0.f;
+#pragma unroll
+    for (int v = 0; v < VT; ++v) o[i][v] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int walk = 0; walk < 2; ++walk) {
+      const float top = m[i] > kMaskedScore ? m[i] : 0.f;
+#pragma unroll 1
+      for (int n0 = 0; n0 < kl.count; n0 += 32) {
+        float p[8];  // keys n0 + 16 (e / 4) + 4 b + e % 4
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+          f32x4_t st = {0.f, 0.f, 0.f, 0.f};
+          const uint16_t *row = kc + static_cast<size_t>(key(n0 + 16 * kt + c)) * D + 8 * b4;
+#pragma unroll
+          for (int s = 0; s < KS; ++s) st = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8_t *>(row + 32 * s), qf[i][s], st, 0, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int n = n0 + 16 * kt + 4 * b4 + e;
+            p[4 * kt + e] = n < kl.count && rule.sees(pos[i], kl.at(n)) ? st[e] : kMaskedScore;
+          }
+        }
+        if (walk == 0) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) m[i] = fmaxf(m[i], p[e]);
+          continue;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          p[e] = __builtin_amdgcn_exp2f((p[e] - top) * sc);
+          l[i] += p[e];
+        }
+        bf16x8_t wh, wl;
+        weights<false>(p, wh, wl);
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+          u32x4_t a;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int n = n0 + 16 * (e >> 1) + 4 * b4 + 2 * (e & 1);
+            a[e] = vc[static_cast<size_t>(key(n)) * D + 16 * v + c] | static_cast<uint32_t>(vc[static_cast<size_t>(key(n + 1)) * D + 16 * v + c]) << 16;
+          }
+          o[i][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), wh, o[i][v], 0, 0, 0);
+        }
+      }
+      m[i] = fmaxf(m[i], __shfl_xor(m[i], 16));
+      m[i] = fmaxf(m[i], __shfl_xor(m[i], 32));
+    }
+  }
+}
+
 // qf[i][s]: dimensions 32 s + 8 b .. + 7 of query 16 i + c of the wave (lane 16 b + c), at position pos[i]; lo, hi: the wave's smallest and largest position.
 // kc, vc: [rows, D], 16-byte aligned.  Results, lane (b, c): o[i][v] = weighted sums of value columns 16 v + 4 b .. + 3 of query 16 i + c in units of 2^(its
-// largest score times sc), m[i] that score, l[i] this lane's share of the sum of weights.
-template <int D, bool SPLIT>
+// largest score times sc), m[i] that score (no key seen: minus infinity, and units of 1), l[i] this lane's share of the sum of weights.
+// ANY: scores may have any size (with SPLIT there are no registers left for it).
+template <int D, bool SPLIT, bool ANY>
 __device__ __forceinline__ void attend(const bf16x8_t (&qf)[2][D / 32], const int (&pos)[2], int lo, int hi, const Keys &kl, const Rule &rule, float sc, const uint16_t *kc,
                                        const uint16_t *vc, uint32_t rows, uint8_t *lds, f32x4_t (&o)[2][D / 16], float (&m)[2], float (&l)[2]) {
   constexpr int KS = D / 32, VT = D / 16, kRow = D * 2, kOperand = kKeys * kRow, kStage = 2 * kOperand;
@@ -154,8 +216,8 @@ __device__ __forceinline__ void attend(const bf16x8_t (&qf)[2][D / 32], const in
       mx = fmaxf(mx, __shfl_xor(mx, 16));
       mx = fmaxf(mx, __shfl_xor(mx, 32));
       const float m_new = fmaxf(m[i], mx);
-      // while a query has seen no key its maximum is the mask value: exponents are then taken against 0, where masked scores give 0
-      const float ref = m_new > 0.5f * kMaskedScore ? m_new * sc : 0.f;
+      // while a query has seen no key its maximum is the mask value, which no finite score reaches: exponents are then taken against 0, where masked scores give 0
+      const float ref = m_new > kMaskedScore ? m_new * sc : 0.f;
       // sums enter and leave the branch as whole registers: element by element they would be copied once per tile
 #pragma unroll
       for (int v = 0; v < VT; ++v) asm volatile("" : "+v"(o[i][v]));
@@ -204,6 +266,13 @@ __device__ __forceinline__ void attend(const bf16x8_t (&qf)[2][D / 32], const in
       }
     }
   }
+  if constexpr (!ANY) return;
+  // An exponent above is one multiply-add against a rounded reference, 2^-24 of the largest score's own exponent off.  Where that is beyond 4096, or sums have left float32's range
+  // on the way (the largest score may have been farther from zero before), the wave starts over without it.
+  bool far = false;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) far |= (m[i] > kMaskedScore && __builtin_fabsf(m[i] * sc) > 4096.f) || !__builtin_isfinite(l[i]);
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(far) != 0, 0)) attend_far<D>(qf, pos, kl, rule, sc, kc, vc, o, m, l);
 }
 #endif
 

@@ -615,7 +615,7 @@ __global__ __launch_bounds__(256, 2) void attention_prompt_kernel(const e2h_wind
   float m[2], l[2];
   const float sc = a.scale * kLog2e;
   const int lo = pos0 + t0 + wave * 32;
-  attention::attend<D, true>(qf, pos, lo, lo + 31, keys, rule, sc, static_cast<const bf16_t *>(a.k_cache) + head * a.cache_len * D,
+  attention::attend<D, true, false>(qf, pos, lo, lo + 31, keys, rule, sc, static_cast<const bf16_t *>(a.k_cache) + head * a.cache_len * D,
                              static_cast<const bf16_t *>(a.v_cache) + head * a.cache_len * D, static_cast<uint32_t>(a.cache_len), lds, o, m, l);
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -623,7 +623,7 @@ __global__ __launch_bounds__(256, 2) void attention_prompt_kernel(const e2h_wind
     float sum = l[i];
     sum += __shfl_xor(sum, 16);
     sum += __shfl_xor(sum, 32);
-    if (a.sink) sum += __builtin_amdgcn_exp2f(__builtin_fmaf(a.sink[h], kLog2e, -m[i] * sc));
+    if (a.sink) sum += __builtin_amdgcn_exp2f(__builtin_fmaf(a.sink[h], kLog2e, m[i] > attention::kMaskedScore ? -m[i] * sc : 0.f));
     const float inv = sum > 0.f ? a.out_scale / sum : 0.f;
     if (tq >= seqlen) continue;
     const size_t row = row0 + tq;

@@ -240,6 +240,25 @@ def test_prefill_attention_against_float64(h, hkv, d, t, start, s_len):
                 assert torch.equal(got[i, front], rep(v)[i][:, at[front]].transpose(0, 1).reshape(len(front), h * d))
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("t,start", [(40, 0), (200, 70)])
+@pytest.mark.parametrize("sign", [-1, 1])
+def test_prefill_attention_of_scores_far_from_zero(d, t, start, sign):
+    """Every score near -2^109 or 2^109: the softmax of what a query sees is as it is anywhere else, the largest score's value (the mean of several alike, rounded to bfloat16: 2^-8
+    of values below 8), and no masked key takes part."""
+    gen = torch.Generator().manual_seed(d)
+    b, h, s_len = 2, 3, start + t
+    q = torch.full((b, h, t, d), 2.0**51).to(torch.bfloat16).to(DEV)
+    k = (sign * 2.0**52 * (1 + torch.randint(0, 64, (b, h, s_len, 1), generator=gen) / 64)).expand(b, h, s_len, d).to(torch.bfloat16).contiguous().to(DEV)
+    v = torch.randn((b, h, s_len, d), generator=gen).to(torch.bfloat16).to(DEV)
+    pos, pad = torch.arange(start, s_len, device=DEV), torch.tensor([0, start + 9], device=DEV)
+    key = torch.arange(s_len, device=DEV)
+    mask = ((key[None, None] <= pos[None, :, None]) & (key[None, None] >= pad[:, None, None])) | (key[None, None] == pos[None, :, None])
+    scores = (q.double() @ k.double().transpose(-1, -2).contiguous()) * d ** -0.5
+    want = (scores.masked_fill(~mask[:, None], float("-inf")).softmax(-1) @ v.double()).transpose(1, 2).reshape(b, t, h * d)
+    assert ((ops.prefill_attention(q, k, v, pos, pad).double() - want).abs() <= 2**-5).all()
+
+
 def test_prompts_of_a_watched_attention_are_shown_the_mask():
     """A hook on one attention keeps the stock operator and its mask for the whole model, and both give the same logits up to
     the rounding of two layers."""
