@@ -16,6 +16,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 from torch import Tensor
+from torch.utils._device import DeviceContext
 
 from . import ops, seq_ops
 from .linear import unwatched
@@ -138,6 +139,14 @@ def _project_deferred(lin, y2d: Tensor, lead_shape) -> Tensor:
     return lin(y2d.view(*lead_shape, -1))
 
 
+def _stock_attention_wanted() -> bool:
+    """True where somebody intercepts torch functions (a default device does so too, but looks at no attention), or has switched off the backend whose place the
+    package's attention of prompts takes."""
+    if torch._C._len_torch_function_stack() and any(type(m) is not DeviceContext for m in torch.overrides._get_current_function_mode_stack()):
+        return True
+    return not torch.backends.cuda.flash_sdp_enabled()
+
+
 class _MaskByPosition:
     """Stands in for the mask of one call, causal by input_pos with the call's padding, where the attention kernel takes those instead.  It is an
     argument like the mask and no state of the modules, so calls of several threads don't see each other's."""
@@ -221,7 +230,7 @@ class Attention(nn.Module):
             q = ops.rope_kv_write_seq(qkv, self.freqs_table, k, v, input_pos, self.n_head, self.n_local_heads, self.head_dim,
                                       rows_by_token=fully_causal)
             if ((fully_causal or isinstance(mask, _MaskByPosition)) and not torch.compiler.is_compiling()
-                    and ops.prefill_attention_fits(seqlen, self.n_head, k, v) and not seq_ops.watched(q, k, v)):
+                    and ops.prefill_attention_fits(seqlen, self.n_head, k, v) and not seq_ops.watched(q, k, v) and not _stock_attention_wanted()):
                 y = ops.prefill_attention(q, k, v, None if fully_causal else input_pos, None if fully_causal else mask.left_pad)
                 return self.wo(y)
             k, v = k[:bsz], v[:bsz]
@@ -477,7 +486,7 @@ class Transformer(nn.Module):
         watches the blocks' or the attentions' calls (hooks are shown the mask) or a trace is being made."""
         if torch.compiler.is_compiling() or input_pos is None or not (input_pos.is_cuda and input_pos.dtype == torch.int64 and input_pos.dim() == 1):
             return False
-        if seq_ops.watched(x, input_pos):
+        if seq_ops.watched(x, input_pos) or _stock_attention_wanted():
             return False
         for blk in self.layers:
             att = blk.attention

@@ -278,6 +278,40 @@ def test_prompts_of_a_watched_attention_are_shown_the_mask():
     assert (plain - watched).norm() <= 2e-2 * watched.norm()
 
 
+@pytest.mark.parametrize("fully_causal", [False, True])
+def test_prompts_use_the_stock_attention_where_it_is_watched_or_chosen(monkeypatch, fully_causal):
+    """A function mode sees every layer's attention, and a choice among the operator's backends is kept; a default device is neither."""
+    model = Transformer(model_mod.ModelArgs(block_size=128, vocab_size=256, n_layer=2, n_head=4, n_local_heads=2, dim=256, intermediate_size=512))
+    init_random_(model, seed=3)
+    model = model.to(device=DEV, dtype=torch.bfloat16).eval()
+    model.setup_caches(3, 64, kv_cache=not fully_causal)
+    ids, pos = torch.randint(0, 256, (3, 40), generator=torch.Generator().manual_seed(5)).to(DEV), torch.arange(40, device=DEV)
+    pads = None if fully_causal else torch.tensor([0, 7, 39], device=DEV)
+    own, seen, launch = [], [], ops.prefill_attention
+
+    class Watch(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            if func is torch.nn.functional.scaled_dot_product_attention:
+                seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    monkeypatch.setattr(ops, "prefill_attention", lambda *a: own.append(None) or launch(*a))
+    run = lambda: model(ids, pos, pads, fully_causal=fully_causal).float()  # noqa: E731
+    with torch.no_grad():
+        plain = run()
+        with torch.device(DEV):
+            assert torch.equal(run(), plain)
+        assert len(own) == 4
+        with Watch():
+            watched = run()
+        assert len(seen) == 2
+        with torch.nn.attention.sdpa_kernel(torch.nn.attention.SDPBackend.MATH):
+            chosen = run()
+        assert len(own) == 4
+    for other in (watched, chosen):
+        assert (plain - other).norm() <= 2e-2 * other.norm()
+
+
 def test_a_prompt_keeps_its_padding_while_another_call_runs():
     """A call of the same model without padding, made between the layers of a padded prompt (as another thread's may be), leaves the
     prompt's logits as they are: the second layer still sees this call's padding."""
