@@ -629,7 +629,11 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const uint16_
   const int rep = H / Hkv;
   const attention::Place at = attention::place(blockIdx.x, B * Hkv, rep, q_blocks);
   const int hk = at.pair % Hkv, b = at.pair / Hkv, h = hk * rep + at.rep, t0 = (q_blocks - 1 - at.back) * attention::kQueries;
-  const int first = left_pad ? static_cast<int>(left_pad[b]) : 0;
+  int first = 0;
+  if (left_pad) {
+    const int64_t pad = left_pad[b];  // any number
+    first = pad < 0 ? 0 : pad > S ? S : static_cast<int>(pad);
+  }
   const auto position = [&](int t) { return input_pos ? static_cast<int>(input_pos[t < T ? t : T - 1]) : t < T ? t : T - 1; };
   // positions may come in any order: the largest of the block bounds its keys
   int top = position(t0 + lane) > position(t0 + 64 + lane) ? position(t0 + lane) : position(t0 + 64 + lane);
@@ -640,7 +644,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const uint16_
   }
   top = __builtin_amdgcn_readfirstlane(top);
   top = top < S - 1 ? top : S - 1;
-  const attention::Rule rule = {first > 0 ? first : 0, INT32_MAX / 2, 0};
+  const attention::Rule rule = {first, INT32_MAX / 2, 0};
   const attention::Keys keys = {rule.first, 0, rule.first, top >= rule.first ? top - rule.first + 1 : 0};
 
   bf16x8_t qf[2][KS];

@@ -443,7 +443,7 @@ class Transformer(nn.Module):
         mask = None
         fused_step = self.layers[0].attention.can_fuse_decode(x, fully_causal)
         if not fully_causal and not fused_step:
-            by_position = self._masks_by_position(x, input_pos)
+            by_position = self._masks_by_position(x, input_pos, left_pad_mask_pos)
             mask = _MaskByPosition(self._mask, left_pad_mask_pos) if by_position else self._mask(input_pos, left_pad_mask_pos)
         freqs_cis = None if fused_step else self.freqs_cis[input_pos].to(dtype=x.dtype)
         if fused_step and input_pos.dtype != torch.int64:
@@ -481,11 +481,13 @@ class Transformer(nn.Module):
             mask = torch.logical_or(mask, self.self_mask[None, None, input_pos])
         return mask
 
-    def _masks_by_position(self, x: Tensor, input_pos: Optional[Tensor]) -> bool:
+    def _masks_by_position(self, x: Tensor, input_pos: Optional[Tensor], left_pad: Optional[Tensor]) -> bool:
         """True where every attention of a prompt runs on ops.prefill_attention, which needs no mask tensor: built for them all otherwise, and where somebody
         watches the blocks' or the attentions' calls (hooks are shown the mask) or a trace is being made."""
         if torch.compiler.is_compiling() or input_pos is None or not (input_pos.is_cuda and input_pos.dtype == torch.int64 and input_pos.dim() == 1):
             return False
+        if left_pad is not None and (left_pad.is_floating_point() or left_pad.is_complex()):
+            return False  # the mask compares them as they are
         if seq_ops.watched(x, input_pos) or _stock_attention_wanted():
             return False
         for blk in self.layers:

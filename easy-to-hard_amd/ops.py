@@ -579,7 +579,7 @@ def prefill_attention(q, k, v, input_pos=None, left_pad=None):
     assert q.dtype == torch.bfloat16 and k.dtype == torch.bfloat16 and v.dtype == torch.bfloat16 and q.is_contiguous() and k.is_contiguous() and v.is_contiguous()
     assert k.shape[0] >= bsz and k.shape[3] == d and v.shape == k.shape and h % hkv == 0
     assert input_pos is None or (input_pos.is_cuda and input_pos.dtype == torch.int64 and input_pos.numel() == t)
-    assert left_pad is None or (left_pad.is_cuda and left_pad.numel() in (1, bsz))
+    assert left_pad is None or (left_pad.is_cuda and left_pad.numel() in (1, bsz) and not left_pad.is_floating_point())
     pos = None if input_pos is None else input_pos.contiguous()
     pad = None if left_pad is None else left_pad.reshape(-1).to(torch.int64).expand(bsz).contiguous()
     out = torch.empty((bsz, t, h * d), dtype=torch.bfloat16, device=q.device)

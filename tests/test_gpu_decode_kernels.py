@@ -278,6 +278,25 @@ def test_prompts_of_a_watched_attention_are_shown_the_mask():
     assert (plain - watched).norm() <= 2e-2 * watched.norm()
 
 
+@pytest.mark.parametrize("pads,same", [([2.5, 39.25, 0.0], [3, 40, 0]), ([2**32, 2**40 + 5, 0], [64, 64, 0]), ([-(2**32) + 9, -1, 70], [0, 0, 64])])
+def test_padding_of_any_number(pads, same):
+    """Positions that lie between two tokens, and such as no 32 bits hold, mask what they mask as numbers: the prompt's logits are those of the whole number that masks the
+    same (of the stock operator for fractions, up to the rounding of two layers)."""
+    model = Transformer(model_mod.ModelArgs(block_size=128, vocab_size=256, n_layer=2, n_head=4, n_local_heads=2, dim=256, intermediate_size=512))
+    init_random_(model, seed=3)
+    model = model.to(device=DEV, dtype=torch.bfloat16).eval()
+    model.setup_caches(3, 64)
+    ids, pos = torch.randint(0, 256, (3, 40), generator=torch.Generator().manual_seed(5)).to(DEV), torch.arange(40, device=DEV)
+    with torch.no_grad():
+        got, want = (model(ids, pos, torch.tensor(p, device=DEV)).float() for p in (pads, same))
+    if isinstance(pads[0], int):
+        assert torch.equal(got, want)
+    else:
+        assert (got - want).norm() <= 1.5e-2 * want.norm()
+        with torch.no_grad():
+            assert (model(ids, pos, torch.tensor(pads, device=DEV).long()).float() - want).norm() > 5e-2 * want.norm()  # what cutting them off would give
+
+
 @pytest.mark.parametrize("fully_causal", [False, True])
 def test_prompts_use_the_stock_attention_where_it_is_watched_or_chosen(monkeypatch, fully_causal):
     """A function mode sees every layer's attention, and a choice among the operator's backends is kept; a default device is neither."""
