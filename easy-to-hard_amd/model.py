@@ -377,6 +377,7 @@ class Transformer(nn.Module):
         self.max_batch_size = -1
         self.max_seq_length = -1
         self.kv_cache_enabled = False
+        self._note_masks()
 
     @classmethod
     def from_name(cls, name: str):
@@ -402,6 +403,27 @@ class Transformer(nn.Module):
             blk.attention.freqs_table = self.freqs_cis
         self.causal_mask = torch.tril(torch.ones(max_seq_length, max_seq_length, dtype=torch.bool, device=device))
         self.self_mask = torch.eye(max_seq_length, dtype=torch.bool, device=device)
+        self._note_masks()
+
+    def _note_masks(self) -> None:
+        masks = (self.causal_mask, self.self_mask)
+        # (a tensor made in inference mode counts no changes)
+        self._masks_built = tuple((m, None if m is None or m.is_inference() else m._version) for m in masks)
+
+    def _masks_as_built(self) -> bool:
+        """False once somebody has put another mask in place of setup_caches' or written into it: prompts then have to read the tensor."""
+        return all(now is built and (version is None or now._version == version)
+                   for now, (built, version) in zip((self.causal_mask, self.self_mask), self._masks_built))
+
+    def __getstate__(self):
+        return {**self.__dict__, "_masks_built": self._masks_as_built()}
+
+    def __setstate__(self, state) -> None:  # a copy's masks count their changes anew
+        super().__setstate__(state)
+        built = state.get("_masks_built", False)
+        self._note_masks()
+        if not built:
+            self._masks_built = ((None, None), (None, None))
 
     def staged_step_supported(self, rows: int) -> bool:
         """True when a single-token step of `rows` sequences runs on the decode-batch int4 kernels with staged activations
@@ -483,12 +505,12 @@ class Transformer(nn.Module):
 
     def _masks_by_position(self, x: Tensor, input_pos: Optional[Tensor], left_pad: Optional[Tensor]) -> bool:
         """True where every attention of a prompt runs on ops.prefill_attention, which needs no mask tensor: built for them all otherwise, and where somebody
-        watches the blocks' or the attentions' calls (hooks are shown the mask) or a trace is being made."""
+        watches the blocks' or the attentions' calls (hooks are shown the mask), has changed the masks, or a trace is being made."""
         if torch.compiler.is_compiling() or input_pos is None or not (input_pos.is_cuda and input_pos.dtype == torch.int64 and input_pos.dim() == 1):
             return False
         if left_pad is not None and (left_pad.is_floating_point() or left_pad.is_complex()):
             return False  # the mask compares them as they are
-        if seq_ops.watched(x, input_pos) or _stock_attention_wanted():
+        if not self._masks_as_built() or seq_ops.watched(x, input_pos) or _stock_attention_wanted():
             return False
         for blk in self.layers:
             att = blk.attention

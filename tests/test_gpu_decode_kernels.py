@@ -1,6 +1,8 @@
 """GPU checks of the decode-step kernels around the linears (RMSNorm, SiLU*mul, RoPE + KV write, single-query
 attention) against the stock torch ops the harness otherwise uses, through the C ABI."""
 
+import copy
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -276,6 +278,35 @@ def test_prompts_of_a_watched_attention_are_shown_the_mask():
         assert torch.equal(model(ids, pos, pads).float(), plain)
     assert len(seen) == 1 and seen[0].dtype == torch.bool and tuple(seen[0].shape) == (3, 1, 40, 64)
     assert (plain - watched).norm() <= 2e-2 * watched.norm()
+
+
+@pytest.mark.parametrize("how", ["written", "replaced", "copied", "written after a copy"])
+def test_a_prompt_reads_masks_that_were_changed(how):
+    """A prompt whose first ten tokens see each other, by the model's own mask tensor: the first token's logits change, and go back with the mask.  A copy of a model keeps
+    what its masks are."""
+    model = Transformer(model_mod.ModelArgs(block_size=128, vocab_size=256, n_layer=2, n_head=4, n_local_heads=2, dim=256, intermediate_size=512))
+    init_random_(model, seed=3)
+    model = model.to(device=DEV, dtype=torch.bfloat16).eval()
+    model.setup_caches(2, 64)
+    ids, pos = torch.randint(0, 256, (2, 40), generator=torch.Generator().manual_seed(5)).to(DEV), torch.arange(40, device=DEV)
+    with torch.no_grad():
+        plain = model(ids, pos).float()
+        assert model._masks_by_position(model.tok_embeddings(ids), pos, None)
+        if how == "written after a copy":
+            model = copy.deepcopy(model)
+            assert model._masks_by_position(model.tok_embeddings(ids), pos, None) and torch.equal(model(ids, pos).float(), plain)
+        if how == "replaced":
+            model.causal_mask = model.causal_mask.clone()
+            model.causal_mask[:10, :10] = True
+        else:
+            model.causal_mask[:10, :10] = True
+        if how == "copied":
+            model = copy.deepcopy(model)
+        changed = model(ids, pos).float()
+        model.causal_mask[:10, :10] = torch.ones(10, 10, device=DEV).tril().bool()
+        back = model(ids, pos).float()
+    assert (changed[:, 0] - plain[:, 0]).norm() > 5e-2 * plain[:, 0].norm()
+    assert (back - plain).norm() <= 2e-2 * plain.norm()
 
 
 @pytest.mark.parametrize("pads,same", [([2.5, 39.25, 0.0], [3, 40, 0]), ([2**32, 2**40 + 5, 0], [64, 64, 0]), ([-(2**32) + 9, -1, 70], [0, 0, 64])])
