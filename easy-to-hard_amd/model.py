@@ -230,7 +230,7 @@ class Attention(nn.Module):
             q = ops.rope_kv_write_seq(qkv, self.freqs_table, k, v, input_pos, self.n_head, self.n_local_heads, self.head_dim,
                                       rows_by_token=fully_causal)
             if ((fully_causal or isinstance(mask, _MaskByPosition)) and not torch.compiler.is_compiling()
-                    and ops.prefill_attention_fits(seqlen, self.n_head, k, v) and not seq_ops.watched(q, k, v) and not _stock_attention_wanted()):
+                    and ops.prefill_attention_fits(bsz, seqlen, self.n_head, k, v, not fully_causal) and not seq_ops.watched(q, k, v) and not _stock_attention_wanted()):
                 y = ops.prefill_attention(q, k, v, None if fully_causal else input_pos, None if fully_causal else mask.left_pad)
                 return self.wo(y)
             k, v = k[:bsz], v[:bsz]
@@ -515,7 +515,7 @@ class Transformer(nn.Module):
         for blk in self.layers:
             att = blk.attention
             if not (type(att) is Attention and type(blk) is TransformerBlock and unwatched(blk) and unwatched(att) and att._can_fuse_prefill_rope(x, input_pos, False)
-                    and ops.prefill_attention_fits(x.shape[1], att.n_head, att.kv_cache.k_cache, att.kv_cache.v_cache)):
+                    and ops.prefill_attention_fits(x.shape[0], x.shape[1], att.n_head, att.kv_cache.k_cache, att.kv_cache.v_cache, True)):
                 return False
         return True
 

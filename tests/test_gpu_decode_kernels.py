@@ -280,6 +280,13 @@ def test_prompts_of_a_watched_attention_are_shown_the_mask():
     assert (plain - watched).norm() <= 2e-2 * watched.norm()
 
 
+@pytest.mark.parametrize("b,t,h,s_len,masked,own", [(32, 16, 32, 16, True, False), (32, 47, 32, 56, True, False), (32, 48, 32, 56, True, True), (32, 16, 32, 64, True, True),
+                                                     (31, 16, 32, 16, True, True), (32, 16, 32, 16, False, True), (1, 15, 4, 64, True, False), (1, 16, 4, 16, True, True)])
+def test_where_prompts_take_the_own_attention(b, t, h, s_len, masked, own):
+    k = torch.empty((b, h, s_len, 64), dtype=torch.bfloat16, device=DEV)
+    assert ops.prefill_attention_fits(b, t, h, k, k, masked) == own
+
+
 @pytest.mark.parametrize("how", ["written", "replaced", "copied", "written after a copy"])
 def test_a_prompt_reads_masks_that_were_changed(how):
     """A prompt whose first ten tokens see each other, by the model's own mask tensor: the first token's logits change, and go back with the mask.  A copy of a model keeps
