@@ -577,7 +577,7 @@ __global__ __launch_bounds__(256) void attention_prefill_kernel(const e2h_window
   }
 }
 
-// ---- the same for heads of 64 or 128 dimensions: 4 waves x 32 queries (e2h_attention_tiles.h) -----------------------------------------
+// ---- the same for many queries with heads of 64 or 128 dimensions: 4 waves x 32 queries (e2h_attention_tiles.h) -----------------------------------------
 template <int D>
 __global__ __launch_bounds__(256, 2) void attention_prompt_kernel(const e2h_window_attention_args a, int q_blocks) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -911,6 +911,15 @@ int64_t step_scratch_bytes(const e2h_window_attention_args &a, int splits) {
   return splits < 2 ? 0 : a.batch * a.heads * splits * (a.vdim + 2) * 4;
 }
 
+// Queries per workgroup of a prompt, heads of 64 or 128 dimensions.  64 (16 per wave) while the workgroups are one per CU at most, and for portions that would leave half of a
+// 128-query workgroup's waves without a query: such a launch is as long as its longest workgroup, and a wave with 16 queries walks its keys sooner.  us, 64 / 128 queries, heads of 128
+// (of 64): 32 heads x 128 tokens 12.1 / 15.0 (9.5 / 13.0), 512 tokens, 256 workgroups, 26.3 / 27.6 (19.1 / 22.1), 768 tokens 39.8 / 36.3 (26.8 / 28.2), behind 1024
+// cached 81.7 / 68.6 (54.8 / 50.1); 1024 56.6 / 45.0 (37.2 / 34.0); 512 heads x 16 tokens 10.8 / 11.6, x 64 behind 1024 cached 60.4 / 65.9, x 96 115 / 73.
+int prompt_queries(const e2h_window_attention_args &a) {
+  if (seq_options().attention_prompt_queries) return seq_options().attention_prompt_queries;
+  return a.seqlen <= 64 || a.batch * a.heads * ((a.seqlen + 63) / 64) <= 256 ? 64 : 128;
+}
+
 void launch_append(const e2h_window_attention_args &a, bool vec, hipStream_t s) {
   if (a.k_off < 0) return;
   if (a.k_norm || a.rotary) {
@@ -949,7 +958,7 @@ void launch_mfma(const e2h_window_attention_args &a, float *part, int64_t part_b
   launch_append(a, VEC && aligned16(a.k_bias) && aligned16(a.v_bias) && a.k_off % 8 == 0 && a.v_off % 8 == 0, s);
   if constexpr (VEC && (KS == 2 || KS == 4) && VT == 2 * KS) {
     constexpr int D = 32 * KS;
-    if (a.dim == D && a.vdim == D && a.cache_len <= static_cast<int64_t>(UINT32_MAX) / (2 * D)) {
+    if (prompt_queries(a) == 128 && a.dim == D && a.vdim == D && a.cache_len <= static_cast<int64_t>(UINT32_MAX) / (2 * D)) {
       const int blocks = static_cast<int>((a.seqlen + attention::kQueries - 1) / attention::kQueries);
       hipLaunchKernelGGL(attention_prompt_kernel<D>, dim3(static_cast<unsigned>(a.batch * a.heads * blocks)), dim3(256), 0, s, a, blocks);
       return;

@@ -418,6 +418,9 @@ extern "C" int e2h_seq_set_option(const char *name, int value) {
   } else if (!strcmp(name, "attention_decode_waves")) {
     if (value != 0 && value != 4 && value != 8) return E2H_ERR_BAD_OPTION;
     o.attention_decode_waves = value;
+  } else if (!strcmp(name, "attention_prompt_queries")) {
+    if (value != 0 && value != 64 && value != 128) return E2H_ERR_BAD_OPTION;
+    o.attention_prompt_queries = value;
   } else if (!strcmp(name, "expert_form")) {
     if (value < 0 || value > 3) return E2H_ERR_BAD_OPTION;
     o.expert_form = value;

@@ -22,7 +22,7 @@ BOTH = pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f
 @pytest.fixture(autouse=True)
 def _default_options():
     yield
-    for name in ("recurrence_form", "recurrence_chunk", "norm_run", "attention_decode_waves"):
+    for name in ("recurrence_form", "recurrence_chunk", "norm_run", "attention_decode_waves", "attention_prompt_queries"):
         _lib.set_seq_option(name, 0)
 
 
@@ -174,10 +174,12 @@ def test_window_edges_with_one_key_that_stands_out(dtype, window, keep):
 
 @pytest.mark.parametrize("h,g,d", [(4, 2, 64), (8, 8, 128), (5, 1, 128), (3, 3, 64)])
 @pytest.mark.parametrize("window,keep", [(0, 0), (100, 70), (300, 5), (1, 0)])
-def test_prompt_attention_in_blocks_of_128_queries(h, g, d, window, keep):
-    """Prompts and portions that end at, before and behind a block of 128 queries and a tile of 64 keys, kept keys that end inside a tile, windows that leave whole tiles
+@pytest.mark.parametrize("queries", [64, 128])
+def test_prompt_attention_in_blocks_of_64_and_128_queries(h, g, d, window, keep, queries):
+    """Prompts and portions that end at, before and behind a block of 64 and 128 queries and a tile of 64 keys, kept keys that end inside a tile, windows that leave whole tiles
     out, sequences with no, one tile's and more than a block's padding side by side, and numbers of heads that do and do not divide by the eight XCDs.  The weights are held
     as two bfloat16 terms, so the tolerance is that of the values' and the result's rounding."""
+    _lib.set_seq_option("attention_prompt_queries", queries)
     t, pads = 390, [0, 70, 200]
     q, k, v, gate = (randn(3, t, n, d, seed=i, dtype=torch.bfloat16) for i, n in enumerate((h, g, g, h)))
     k[0, 5:40, 0] += 0.5 * q[0, -1, 0]  # far keys carry weight
