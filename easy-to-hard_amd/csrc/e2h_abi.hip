@@ -97,7 +97,7 @@ extern "C" int e2h_set_option(const char *name, int value) {
     return E2H_OK;
   }
   if (!strcmp(name, "int4_gemm_tile")) {
-    if (value != 0 && value != 128 && value != 256) return E2H_ERR_BAD_OPTION;
+    if (value != 0 && value != 96 && value != 128 && value != 256) return E2H_ERR_BAD_OPTION;
     o.int4_gemm_tile = value;
     return E2H_OK;
   }

@@ -530,7 +530,7 @@ Int4GemmShape int4_gemm_shape(int M, int N, int K, int groupsize, int64_t scratc
   Int4GemmShape best = {64, 1, -1.0};
   for (int rows = 64; rows <= (groupsize == 32 ? 64 : 128); rows += 32) {
   // group size 32 at 128 rows does not fit the registers
-    if (want_rows == 128 && groupsize != 32 && rows != 128) continue;
+    if ((want_rows == 96 || want_rows == 128) && groupsize != 32 && rows != want_rows) continue;
     const int64_t per_xcd = static_cast<int64_t>((M + rows - 1) / rows) * (((N + kCols - 1) / kCols + 7) / 8);  // one slice; 32 CUs each
     for (int s = 1; possible(s); s *= 2) {
       if (forced && s != forced) continue;

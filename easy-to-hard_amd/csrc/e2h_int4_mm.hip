@@ -806,7 +806,8 @@ int int4_mm_impl(const uint16_t *x, const int32_t *packed, const uint16_t *scale
       const int64_t need = static_cast<int64_t>(kTicketBytes) + static_cast<int64_t>(a.K / 128) * stride * 4;
       const Int4GemmShape shape = int4_gemm_shape(a.M, a.N, a.K, 128, std::max<int64_t>(0, workspace_bytes - need) & ~int64_t{15});
       const double rounds = static_cast<double>((a.N + 63) / 64) * ((a.M + 31) / 32) / kCUs;
-      if (need <= workspace_bytes && 1.1 * shape.us + 1.6 < 6 + 0.36 * (a.K / 128) * std::max(1.0, rounds)) {
+      const bool use32 = options().int4_gemm32_min_rows > 0 ? a.M >= options().int4_gemm32_min_rows : 1.1 * shape.us + 1.6 < 6 + 0.36 * (a.K / 128) * std::max(1.0, rounds);
+      if (need <= workspace_bytes && use32) {
         float *xs = reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + kTicketBytes);
         if (launch_x_group_sums(a.x, xs, a.M, a.K, stride, 128, a.stream) != E2H_OK) return E2H_ERR_LAUNCH;
         float *partials = reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + need);

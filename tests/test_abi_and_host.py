@@ -324,7 +324,7 @@ def test_reward_model_loader_builds_the_two_row_head_and_rejects_quantized_files
 
 @pytest.mark.parametrize("k", [128, 384, 1024, 4096])
 @pytest.mark.parametrize("want", [1, 2, 3, 5, 6, 7, 8, 16])
-@pytest.mark.parametrize("tile,groupsize", [(0, 64), (128, 64), (128, 128), (0, 32)])
+@pytest.mark.parametrize("tile,groupsize", [(0, 64), (96, 64), (96, 128), (128, 64), (128, 128), (0, 32), (96, 32)])
 def test_a_forced_slice_count_leaves_a_real_geometry(k, want, tile, groupsize):
     """the many-row int4 matmul picks rows per workgroup and K slices by expected time; a forced count that is no power of two, or more than
     K or the scratch memory allow, becomes the next possible one, with its time, and a forced tile stays"""
@@ -345,4 +345,4 @@ def test_a_forced_slice_count_leaves_a_real_geometry(k, want, tile, groupsize):
             lib.e2h_set_option(b"int4_gemm_tile", 0)
         most = min(want, 8, k // 128, max(fit, 1))
         assert got.slices == max(s for s in (1, 2, 4, 8) if s <= most)
-        assert got.us > 0 and got.rows == (128 if tile == 128 else 64)
+        assert got.us > 0 and got.rows == (tile if tile and groupsize != 32 else 64)

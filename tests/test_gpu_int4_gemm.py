@@ -52,15 +52,14 @@ def test_exact_on_dyadic_operands(many_row_kernel, g, slices, tile, m, n, k):
     assert torch.equal(got, want.to(torch.bfloat16))
 
 
-# three blocks of 128 k per slice and an odd first one; workgroups of 64, 96 and 128 rows by their own rule
+# slices of an odd number of blocks of 128 k, so that pairs of groups are cut; (256, 513, 12288, 1024) has no room for sums of slices and keeps one
 @pytest.mark.parametrize("slices", [0, 1, 2, 4])
+@pytest.mark.parametrize("tile", [0, 96, 128])
 @pytest.mark.parametrize("g,m,n,k", [(256, 130, 3080, 768), (256, 471, 1032, 2304), (256, 513, 12288, 1024), (128, 470, 12296, 384), (64, 195, 5128, 640), (64, 97, 8200, 1408)])
-def test_pairs_of_groups_and_96_row_workgroups_are_exact(g, m, n, k, slices):
+def test_pairs_of_groups_and_96_row_workgroups_are_exact(many_row_kernel, g, m, n, k, tile, slices):
     _lib.set_option("int4_k_slices", slices)
-    try:
-        got, want = _run(*_case(m, n, k, g), g)
-    finally:
-        _lib.set_option("int4_k_slices", 0)
+    _lib.set_option("int4_gemm_tile", tile)
+    got, want = _run(*_case(m, n, k, g), g)
     assert torch.equal(got, want.to(torch.bfloat16))
 
 
@@ -327,8 +326,9 @@ def test_rows_of_an_unpacked_call_stand_alone(g):
 
 
 @pytest.mark.parametrize("g,m,n,k", [(64, 470, 12296, 640), (128, 470, 12296, 384), (256, 470, 12296, 768)])
-def test_odd_scales_in_96_row_workgroups(g, m, n, k):
-    """471 rows of 12288 columns are work for five rows of workgroups; the plain loop walks pairs of row tiles, of which the last holds one"""
+def test_odd_scales_in_96_row_workgroups(many_row_kernel, g, m, n, k):
+    """Five rows of workgroups, the last of 86 rows; the plain loop walks pairs of row tiles, of which the last holds one, and stores nothing of the next workgroup's rows"""
+    _lib.set_option("int4_gemm_tile", 96)
     codes, scale, zero, x = _case(m, n, k, g)
     zero[:, 5], scale[:, 5] = 0.0, 2.0**-101
     zero[:, 12290], scale[:, 12290] = 0.0, 2.0**40
