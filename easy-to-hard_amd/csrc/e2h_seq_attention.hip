@@ -649,7 +649,13 @@ __global__ __launch_bounds__(256, 2) void attention_prompt_kernel(const e2h_wind
 // token's row appends that row first.
 // A tile is a serial chain of 2.4 us (load, product, softmax, product), so what bounds few sequences is tiles per wave and not
 // bytes: 4 sequences x 8 key heads over 2048 keys took 25.5 us with one workgroup each (9 tiles per wave on 32 of 256 CUs), 12.9 with eight; 1 sequence 23.9 and 11.6; 30000 keys 273 and
-// 29.  32 sequences (256 workgroups, no split) read 6 TB/s.
+// 29.  32 sequences (256 workgroups, no split) read 5.2 TB/s.
+// `splits` is for the cache's capacity; workgroups beyond the keys that there are end at once, and where one is left it writes the result itself.
+__device__ __forceinline__ int parts_with_keys(int count, int waves, int splits) {
+  const int rounds = (count + 32 * waves - 1) / (32 * waves);  // tiles of a wave of one workgroup
+  return rounds < 2 ? 1 : rounds < splits ? rounds : splits;
+}
+
 template <int KS, int VT, int NW, bool VEC>
 __global__ __launch_bounds__(64 * NW) void attention_step_kernel(const e2h_window_attention_args a, int splits, float *part) {
   constexpr int kVRow = VT * 32 + 8;  // bytes per value row in LDS
@@ -667,8 +673,11 @@ __global__ __launch_bounds__(64 * NW) void attention_step_kernel(const e2h_windo
   const int first = a.first ? static_cast<int>(a.first[bi]) : 0;
   const int last = pos < a.cache_len ? pos : static_cast<int>(a.cache_len) - 1;
   const KeyList kl = key_list(pos, last, first, static_cast<int>(a.window), static_cast<int>(a.keep_first));
+  const int parts = parts_with_keys(kl.count, NW, splits);
+  if (split >= parts) return;  // the whole workgroup
+  if (parts == 1) part = nullptr;
   // the list ends with the new token's row
-  const bool appends = split == (kl.count > 0 ? (kl.count - 1) / 32 / NW % splits : 0);
+  const bool appends = split == (kl.count > 0 ? (kl.count - 1) / 32 / NW % parts : 0);
   const bf16_t *proj = static_cast<const bf16_t *>(a.proj) + static_cast<size_t>(bi) * a.ld;
   bf16_t *kc = static_cast<bf16_t *>(a.k_cache) + (static_cast<size_t>(bi) * a.kv_heads + g) * a.cache_len * D;
   bf16_t *vc = static_cast<bf16_t *>(a.v_cache) + (static_cast<size_t>(bi) * a.kv_heads + g) * a.cache_len * DV;
@@ -725,7 +734,7 @@ __global__ __launch_bounds__(64 * NW) void attention_step_kernel(const e2h_windo
   uint8_t *v_lds = lds + wave * kWaveLds;
   constexpr int kVPer = (32 * VT * 2 + 63) / 64;
 
-  for (int n0 = (split * NW + wave) * 32; n0 < kl.count; n0 += splits * NW * 32) {
+  for (int n0 = (split * NW + wave) * 32; n0 < kl.count; n0 += parts * NW * 32) {
     u32x4_t kf[2][KS], vr[kVPer];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -841,19 +850,22 @@ __global__ __launch_bounds__(64 * NW) void attention_step_kernel(const e2h_windo
 }
 
 // one value of one head per thread: the splits' sums, each in units of its own maximum, brought to the largest
-__global__ __launch_bounds__(256) void attention_combine_kernel(const e2h_window_attention_args a, int splits, const float *part) {
+__global__ __launch_bounds__(256) void attention_combine_kernel(const e2h_window_attention_args a, int waves, int splits, const float *part) {
   const int H = static_cast<int>(a.heads), G = static_cast<int>(a.kv_heads), DV = static_cast<int>(a.vdim), rep = H / G;
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= a.batch * H * DV) return;
   const int d = static_cast<int>(i % DV), h = static_cast<int>(i / DV % H), bi = static_cast<int>(i / DV / H), stride = rep * (DV + 2);
+  const int pos = static_cast<int>(a.input_pos[0]), last = pos < a.cache_len ? pos : static_cast<int>(a.cache_len) - 1;
+  const int parts = parts_with_keys(key_list(pos, last, a.first ? static_cast<int>(a.first[bi]) : 0, static_cast<int>(a.window), static_cast<int>(a.keep_first)).count, waves, splits);
+  if (parts == 1) return;  // the step has written the result
   const float *row = part + (static_cast<size_t>(bi) * G + h / rep) * splits * stride + (h % rep) * (DV + 2);
   constexpr int kAtOnce = 8;
   float m = kMasked, l = 0.f, o = 0.f;
-  for (int s0 = 0; s0 < splits; s0 += kAtOnce) {
+  for (int s0 = 0; s0 < parts; s0 += kAtOnce) {
     float ms[kAtOnce], ls[kAtOnce], os[kAtOnce];
 #pragma unroll
     for (int k = 0; k < kAtOnce; ++k) {
-      const bool there = s0 + k < splits;
+      const bool there = s0 + k < parts;
       const float *p = row + static_cast<size_t>(there ? s0 + k : s0) * stride;
       ms[k] = there ? p[DV] : kMasked;
       ls[k] = there ? p[DV + 1] : 0.f;
@@ -893,10 +905,12 @@ int step_waves(const e2h_window_attention_args &a) {
   return d <= 128 ? nw : 4;
 }
 
-// Workgroups per (sequence, key/value head) of the step, so that there is one per CU at most (two cost more than they share: 8 sequences x
+// Workgroups per (sequence, key/value head) of the step, by the cache's capacity (the position is on the device), so that there is one per CU at most (two cost more than they share: 8 sequences x
 // 8 key heads over 2052 keys in 4 parts 18.8 us, in 8 parts 24.2).  A tile takes a wave 2.4 us and the combining launch 4 to 5, so fewer than
 // three tiles per wave are not shared (300 keys, 4 sequences: 9.2 us whole, 10.9 in two parts), and two parts never pay: 86 and more
-// workgroups already read at the memory's rate (16 sequences 27.2 us whole, 28.3 in two parts).
+// workgroups already read at the memory's rate (16 sequences 27.2 us whole, 28.3 in two parts).  A position with few keys in a long cache pays 1.7 to 2
+// us for a launch that combines little or nothing (8 key heads, cache of 8192; one workgroup / this, us: 1 sequence, 17 keys 6.7 / 8.5, 500 11.1 / 12.7, 700 13.4 / 12.5, 2000 25 / 13;
+// 4 sequences 6.7 / 8.6, 11.9 / 13.9, 15.7 / 14.2, 32 / 18; with all workgroups of the capacity at work 11.9 at 17 keys of 1 sequence).
 constexpr int kMostSplits = 64;
 int step_splits(const e2h_window_attention_args &a) {
   if (a.seqlen != 1 || !on_matrix_cores(a)) return 1;
@@ -952,7 +966,7 @@ void launch_mfma(const e2h_window_attention_args &a, float *part, int64_t part_b
     const dim3 grid(static_cast<unsigned>(a.batch * a.kv_heads * splits));
     if (step_waves(a) == 8) hipLaunchKernelGGL((attention_step_kernel<KS, VT, (KS <= 4 ? 8 : 4), VEC>), grid, dim3(KS <= 4 ? 512 : 256), 0, s, a, splits, part);
     else hipLaunchKernelGGL((attention_step_kernel<KS, VT, 4, VEC>), grid, dim3(256), 0, s, a, splits, part);
-    if (part) hipLaunchKernelGGL(attention_combine_kernel, dim3(static_cast<unsigned>((a.batch * a.heads * a.vdim + 255) / 256)), dim3(256), 0, s, a, splits, part);
+    if (part) hipLaunchKernelGGL(attention_combine_kernel, dim3(static_cast<unsigned>((a.batch * a.heads * a.vdim + 255) / 256)), dim3(256), 0, s, a, step_waves(a), splits, part);
     return;
   }
   launch_append(a, VEC && aligned16(a.k_bias) && aligned16(a.v_bias) && a.k_off % 8 == 0 && a.v_off % 8 == 0, s);

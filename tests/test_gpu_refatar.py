@@ -2,6 +2,8 @@
 in float32 and bfloat16, prompts against token-by-token decoding and against portions, sequences side by side, reused rows, and
 generation through the package's own entry points."""
 
+import copy
+import ctypes
 import io
 import json
 
@@ -239,6 +241,43 @@ def test_decode_attention_shared_by_workgroups(t, window, keep, waves, h, g, d, 
     for i, f in enumerate(pads):
         want = ro.window_attention(f64(q)[i, f:], f64(k)[i, f:], f64(v)[i, f:], 0.3, window, keep)[-1] * ro.sigmoid(f64(gate)[i, -1])
         assert rel(got[i, -1], want) < 1e-2, (i, f)
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("keys", [1, 31, 255, 256, 257, 511, 512, 513, 900])
+def test_few_keys_in_a_long_cache_are_not_shared(waves, keys):
+    """Steps early in a cache for 4096 positions: the launch is that of a full cache, the result bit for bit that of one workgroup while its waves have one tile each at most,
+    without a look at the scratch memory, and beyond that within the rounding of the step; a sequence that begins late has fewer keys than its neighbours."""
+    _lib.set_seq_option("attention_decode_waves", waves)
+    b, h, g, d = 3, 8, 2, 64
+    cache = KVCache(b, 4096, g, d, torch.bfloat16, DEV)
+    cache.k_cache.copy_(randn(b, g, 4096, d, seed=1, dtype=torch.bfloat16))
+    cache.v_cache.copy_(randn(b, g, 4096, d, seed=2, dtype=torch.bfloat16))
+    proj = randn(b, (h + 2 * g) * d, seed=3, dtype=torch.bfloat16)
+    first = torch.tensor([0, keys // 3, keys - 1], device=DEV)
+    outs, caches = [], []
+    for whole in (False, True):
+        lib = _lib.load_seq()
+        mine, out = copy.deepcopy(cache), torch.zeros((b, h * d), dtype=torch.bfloat16, device=DEV)
+        a = _lib.WindowAttentionArgs(dtype=_lib.SEQ_BF16, batch=b, seqlen=1, heads=h, kv_heads=g, dim=d, vdim=d, cache_len=4096, proj=proj.data_ptr(), ld=proj.shape[1], q_off=0,
+                                     k_off=h * d, v_off=(h + g) * d, g_off=-1, k_cache=mine.k_cache.data_ptr(), v_cache=mine.v_cache.data_ptr(), window=0, keep_first=0, scale=0.125,
+                                     out_scale=1.0, out=out.data_ptr(), ld_out=h * d, out_off=0)
+        pos = positions(keys - 1, 1)
+        a.input_pos, a.first = pos.data_ptr(), first.data_ptr()
+        need = lib.e2h_seq_window_attention_scratch_bytes(ctypes.byref(a))
+        assert need > 0
+        scratch = torch.full((need // 4,), float("nan"), dtype=torch.float32, device=DEV)
+        assert lib.e2h_seq_window_attention_split(ctypes.byref(a), None if whole else scratch.data_ptr(), 0 if whole else need, torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        outs.append(out)
+        caches.append(mine)
+        if not whole:
+            scratch_used = not bool(scratch.isnan().all())
+    assert torch.equal(caches[0].k_cache, caches[1].k_cache) and torch.equal(caches[0].v_cache, caches[1].v_cache)
+    if keys <= 32 * waves:
+        assert torch.equal(outs[0], outs[1])
+    assert scratch_used == (keys > 32 * waves)
+    assert rel(f64(outs[0]), f64(outs[1])) < 4e-3  # one rounding to bfloat16 may fall the other way
 
 
 # ---- HGRN2 -----------------------------------------------------------------------------------------------------------------------
