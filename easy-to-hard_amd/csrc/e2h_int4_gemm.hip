@@ -428,8 +428,10 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
         }
         return;
       }
+      int late = lane;
+      asm volatile("" : "+v"(late));  // keeps the rows' addresses out of the registers of the main loop (the 128-row form of group size 64 would spill two)
       const float no_scale[kCT] = {};
-      store_tiles_via_lds<kRT, kCT, false>(acc, no_scale, lds + wave * TileStore<kCT>::kBytesPerWave, a.y, row0, col0, M, N, lane,
+      store_tiles_via_lds<kRT, kCT, false>(acc, no_scale, lds + wave * TileStore<kCT>::kBytesPerWave, a.y, row0, col0, M, N, late,
                                           (N & 7) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0, only);
       return;
     }
