@@ -684,6 +684,21 @@ int launch_x_group_sums(const uint16_t *x, float *out, int M, int K, int stride,
 }
 }  // namespace e2h
 
+namespace e2h {
+// More than 64 rows: whether the 32x32-tile kernel, which takes us32, is expected to take less time than this file's kernels.  Of these a workgroup takes `one` us per 128 k when it has its CU
+// to itself and two that share a CU `two` (64 rows and 4 x 16 columns, or 8 x 16 where `tiles` is 2, group sums of x included; at group size 256 32 rows and 64 columns); 3 to 6 % off 540
+// measured calls per group size.
+bool int4_rows_on_32x32(int M, int N, int K, int groupsize, int tiles, double us32) {
+  const int64_t wgs = groupsize == 256 ? static_cast<int64_t>((N + 63) / 64) * ((M + 31) / 32) : static_cast<int64_t>(((N + 15) / 16 + 4 * tiles - 1) / (4 * tiles)) * ((M + 63) / 64);
+  const int64_t per_cu = (wgs + kCUs - 1) / kCUs;
+  double one = 0.34, two = 0.62;
+  if (groupsize == 32) one = tiles == 2 ? 1.9 : 1.23, two = tiles == 2 ? 3.8 : 2.46;
+  if (groupsize == 64) one = tiles == 2 ? 1.2 : 0.8, two = tiles == 2 ? 2.4 : 1.23;
+  if (groupsize == 128) one = tiles == 2 ? 1.05 : 0.83, two = tiles == 2 ? 1.43 : 1.07;
+  return us32 < 6 + (K / 128) * (static_cast<double>(per_cu / 2) * two + (per_cu & 1 ? one : 0));
+}
+}  // namespace e2h
+
 extern "C" int64_t e2h_workspace_bytes(void) { return static_cast<int64_t>(e2h::kTicketBytes) + (int64_t{32} << 20); }
 
 namespace e2h {
@@ -798,15 +813,13 @@ int int4_mm_impl(const uint16_t *x, const int32_t *packed, const uint16_t *scale
       if (rc128 != E2H_OK) return rc128;
       continue;
     }
-    // Group size 256 over many rows: pairs of groups of 128 on the 32x32-tile kernel where their sums of x fit and it is expected to be the faster one.  The kernel of this file takes
-    // 0.36 us per 128 k and round of its 32 x 64 outputs over the CUs.  Measured (us; here / 32x32): 66 rows 12288 x 4096 39 / 30, 400 rows 108 / 56, 4096 rows
-    // 1083 / 355, 300 rows 4096 x 4096 36 / 30; stay: 157 rows 25 / 25, 400 rows 2048 x 2048 16 / 24.
+    // Group size 256 over many rows: pairs of groups of 128 on the 32x32-tile kernel where their sums of x fit and it is expected to be the faster one.  Measured (us; here /
+    // 32x32): 66 rows 12288 x 4096 39 / 30, 400 rows 108 / 56, 4096 rows 1083 / 355, 300 rows 4096 x 4096 36 / 30; stay: 157 rows 25 / 28, 400 rows 2048 x 2048 16 / 24.
     if (groupsize == 256 && inner_k_tiles == 8 && a.M > 64 && workspace && !options().int4_no_xsum && !options().int4_no_gemm32 && !options().row_tiles) {
       const int stride = ((a.M + 63) / 64) * 64;
       const int64_t need = static_cast<int64_t>(kTicketBytes) + static_cast<int64_t>(a.K / 128) * stride * 4;
       const Int4GemmShape shape = int4_gemm_shape(a.M, a.N, a.K, 128, std::max<int64_t>(0, workspace_bytes - need) & ~int64_t{15});
-      const double rounds = static_cast<double>((a.N + 63) / 64) * ((a.M + 31) / 32) / kCUs;
-      const bool use32 = options().int4_gemm32_min_rows > 0 ? a.M >= options().int4_gemm32_min_rows : 1.1 * shape.us + 1.6 < 6 + 0.36 * (a.K / 128) * std::max(1.0, rounds);
+      const bool use32 = options().int4_gemm32_min_rows > 0 ? a.M >= options().int4_gemm32_min_rows : int4_rows_on_32x32(a.M, a.N, a.K, 256, 1, shape.us);
       if (need <= workspace_bytes && use32) {
         float *xs = reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + kTicketBytes);
         if (launch_x_group_sums(a.x, xs, a.M, a.K, stride, 128, a.stream) != E2H_OK) return E2H_ERR_LAUNCH;
@@ -825,18 +838,15 @@ int int4_mm_impl(const uint16_t *x, const int32_t *packed, const uint16_t *scale
         if (launch_x_group_sums(a.x, xs, a.M, a.K, stride, groupsize, a.stream) != E2H_OK) return E2H_ERR_LAUNCH;
         a.xsum = xs;
         a.xsum_stride = stride;
-        // The 32x32-tile kernel wherever the work fills the chip (320 tiles of 128 x 128), and below that where it is expected to take
-        // less time than the 16x16-tile kernel of this file by more than the estimates are off: that one takes 0.9 us per 128 k with one weight tile per wave (1.35 at group size
-        // 32) and 1.15 with two (1.85 at 64, 3 at 32), not quite half as much again for every further workgroup on a CU.  Measured (us;
-        // 16x16 / 32x32): 300 rows 12288 x 4096 g128 52 / 44, g64 82 / 55, g32 131 / 69, 1100 rows 4096 x 11008 g128 202 / 125; stay: 400 rows
-        // 2048 x 2048 g128 21 / 23, g64 20 / 24.
+        // The 32x32-tile kernel wherever the work fills the chip (320 tiles of 128 x 128), and below that where it is expected to take less time than the 16x16-tile kernel of this
+        // file.  Measured (us; 16x16 / 32x32): 300 rows 12288 x 4096 g128 52 / 44, g64
+        // 82 / 55, g32 131 / 69, 1100 rows 4096 x 11008 g128 202 / 125; stay: 471 rows 2048 x 2048 g128 19 / 25, g64 19 / 25, 256 rows 8192 x 2048 g128 22 / 29, 200 rows
+        // 4096 x 1024 g32 16 / 21.
         const int64_t left = (workspace_bytes - need) & ~int64_t{15};
         const Int4GemmShape shape = int4_gemm_shape(a.M, a.N, a.K, groupsize, left);
         const long long wgs32 = static_cast<long long>((a.M + 127) / 128) * ((a.N + 127) / 128);
-        const long long wgs16 = static_cast<long long>((tiles16 + 4 * sh.t - 1) / (4 * sh.t)) * ((a.M + 63) / 64);
-        const double per_wg = sh.t == 2 ? (groupsize == 32 ? 3.0 : groupsize == 64 ? 1.85 : 1.15) : groupsize == 32 ? 1.35 : 0.9;
-        const double us16 = 4 + per_wg * (a.K / 128) * std::max(1.0, 0.75 + 0.45 * static_cast<double>(wgs16) / kCUs);
-        const bool use32 = options().int4_gemm32_min_rows > 0 ? a.M >= options().int4_gemm32_min_rows : wgs32 >= 320 || 1.1 * shape.us + 1.6 < us16;
+        const bool use32 = options().int4_gemm32_min_rows > 0 ? a.M >= options().int4_gemm32_min_rows
+                                                              : wgs32 >= 320 || int4_rows_on_32x32(a.M, a.N, a.K, groupsize, sh.t, shape.us);
         if (use32 && !options().int4_no_gemm32) {
           float *partials = reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + need);  // need is a multiple of 256
           const int rc32 = int4_gemm(a.x, a.packed, a.sz, a.y, xs, stride, partials, shape, a.M, a.N, a.K, groupsize, a.stream);

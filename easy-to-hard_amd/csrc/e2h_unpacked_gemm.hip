@@ -447,6 +447,19 @@ double unpacked_cost(int64_t M, int64_t N, int64_t K, double unpack) {
   return unpack + 4 + rounds * (static_cast<double>(K) / 64 * 1.36 + 5);
 }
 
+// The same of the kernel that multiplies codes (e2h_int4_gemm.hip) with a thousand rows and more and one K slice: the cost that int4_gemm_shape picks its rows per workgroup by, which holds
+// for chips full of matrix work (its expected time is fitted to fewer rows).
+double int4_codes_cost(int64_t M, int64_t N, int64_t K, int groupsize) {
+  constexpr double kOne[] = {1.2, 1.47, 1.85}, kTwo[] = {1.95, 2.42, 3.3};
+  double best = -1;
+  for (int i = 0; i < (groupsize == 32 ? 1 : 3); ++i) {
+    const int64_t rows = 64 + 32 * i, per_cu = ((M + rows - 1) / rows * (((N + 255) / 256 + 7) / 8) + 31) / 32;
+    const double cost = (static_cast<double>(per_cu / 2) * kTwo[i] + (per_cu & 1 ? kOne[i] : 0)) * static_cast<double>(K / 128) + 3;
+    if (best < 0 || cost < best) best = cost;
+  }
+  return groupsize == 32 ? 1.3 * best : best;
+}
+
 // The same of int8_gemm32 (e2h_int8_gemm.hip), by its own rule: 256-row tiles dealt to the XCDs by whole column blocks, 1.52 per chunk, or
 // rounds of 128-row ones, 1.03 per chunk.
 double int8_gemm32_cost(int64_t M, int64_t N, int64_t K) {
@@ -458,6 +471,7 @@ double int8_gemm32_cost(int64_t M, int64_t N, int64_t K) {
 
 // Taken where it is the cheaper one, the unpacking (three bytes a weight at 4.8 TB/s) included: 8192 rows 12288 x 4096 571 us (611 converting in the loop),
 // 11008 x 4096 542 (591), 5120 x 13824 875 (1250: 20 column blocks on 8 XCDs); 2048 rows 4096 x 11008 209 (177), left to the other form.
+// Known to be off over a short K, where a last round that is not full takes as long as a full one: 1280 rows 16384 x 1024 66 us, 57 in the other form.
 int64_t int8_unpacked_bytes(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || N < 8 || N % 8 != 0 || K % 128 != 0 || K < 256 || N > INT32_MAX || K > INT32_MAX || N * K * 2 >= (int64_t{1} << 32)) return 0;
   const Options &o = options();
@@ -491,8 +505,7 @@ int64_t int4_unpacked_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int 
   if (M * KE * 2 >= (int64_t{1} << 32) || N * KE * 2 >= (int64_t{1} << 32) || K / G * sum_stride(M) * 4 >= (int64_t{1} << 32)) return 0;
   const int64_t bytes = int4_scratch(nullptr, M, N, K, groupsize).bytes;
   const double unpack = (static_cast<double>(N) * static_cast<double>(K) * 2.5 + static_cast<double>(M) * static_cast<double>(K) * 4) / 4.8e6 + 8;
-  const double other = int4_gemm_shape(static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), G, 32 << 20).us * (G == 32 ? 1.3 : 1.0);  // its estimate for group size 32 is that much low
-  return unpacked_cost(M, N, KE, unpack) < other ? bytes : 0;
+  return unpacked_cost(M, N, KE, unpack) < int4_codes_cost(M, N, K, G) ? bytes : 0;
 }
 
 int int4_unpacked_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *scales_and_zeros, uint16_t *y, int M, int N, int K, int groupsize, void *scratch,

@@ -346,3 +346,21 @@ def test_a_forced_slice_count_leaves_a_real_geometry(k, want, tile, groupsize):
         most = min(want, 8, k // 128, max(fit, 1))
         assert got.slices == max(s for s in (1, 2, 4, 8) if s <= most)
         assert got.us > 0 and got.rows == (tile if tile and groupsize != 32 else 64)
+
+
+@pytest.mark.parametrize("m,n,k,groupsize,big", [(471, 2048, 2048, 64, False), (471, 2048, 2048, 128, False), (256, 8192, 2048, 128, False), (300, 6144, 2048, 128, False), (200, 4096, 1024, 32, False),
+                                                 (1300, 520, 1024, 32, False), (200, 4096, 4096, 256, False), (300, 3072, 3072, 64, False), (300, 12288, 4096, 128, True), (471, 4096, 4096, 128, True),
+                                                 (65, 4096, 11008, 64, True), (471, 12288, 4096, 32, True), (400, 12288, 4096, 256, True), (1024, 2048, 4096, 128, True)])
+def test_rows_between_the_two_int4_kernels(m, n, k, groupsize, big):
+    """more rows than a decode batch: the 32x32-tile kernel where it was measured to be the faster one"""
+
+    class Shape(ctypes.Structure):
+        _fields_ = [("rows", ctypes.c_int), ("slices", ctypes.c_int), ("us", ctypes.c_double)]
+
+    lib = _lib.load()
+    shape, on_32x32 = lib["_ZN3e2h15int4_gemm_shapeEiiiil"], lib["_ZN3e2h18int4_rows_on_32x32Eiiiiid"]
+    shape.restype, shape.argtypes = Shape, [ctypes.c_int] * 4 + [ctypes.c_int64]
+    on_32x32.restype, on_32x32.argtypes = ctypes.c_bool, [ctypes.c_int] * 5 + [ctypes.c_double]
+    tiles = 2 if (n + 127) // 128 * ((m + 63) // 64) >= 256 else 1
+    us = shape(m, n, k, min(groupsize, 128), 31 << 20).us
+    assert on_32x32(m, n, k, groupsize, tiles, us) == big
