@@ -448,7 +448,7 @@ double unpacked_cost(int64_t M, int64_t N, int64_t K, double unpack) {
 }
 
 // The same of the kernel that multiplies codes (e2h_int4_gemm.hip) with a thousand rows and more and one K slice: the cost that int4_gemm_shape picks its rows per workgroup by, which holds
-// for chips full of matrix work (its expected time is fitted to fewer rows).
+// for chips full of matrix work (its expected time is fitted to fewer rows), and what more of the rescaling group sizes 32 and 64 cost there.
 double int4_codes_cost(int64_t M, int64_t N, int64_t K, int groupsize) {
   constexpr double kOne[] = {1.2, 1.47, 1.85}, kTwo[] = {1.95, 2.42, 3.3};
   double best = -1;
@@ -457,7 +457,7 @@ double int4_codes_cost(int64_t M, int64_t N, int64_t K, int groupsize) {
     const double cost = (static_cast<double>(per_cu / 2) * kTwo[i] + (per_cu & 1 ? kOne[i] : 0)) * static_cast<double>(K / 128) + 3;
     if (best < 0 || cost < best) best = cost;
   }
-  return groupsize == 32 ? 1.3 * best : best;
+  return groupsize == 32 ? 1.3 * best : groupsize == 64 ? 1.15 * best : best;
 }
 
 // The same of int8_gemm32 (e2h_int8_gemm.hip), by its own rule: 256-row tiles dealt to the XCDs by whole column blocks, 1.52 per chunk, or
@@ -493,7 +493,7 @@ int int8_unpacked_gemm(const uint16_t *x, const int8_t *q, const uint16_t *scale
 }
 
 // Taken where it is the cheaper one, the unpacking (two and a half bytes a weight, four a value of x, at 4.8 TB/s; 8 us of launches) included.  Measured, us, here (codes multiplied
-// in the loop): 8192 rows 12288 x 4096 g128 647 (695), 32000 x 4096 1664 (1793), 12288 x 4096 g32 699 (1056), g256 644; 2048 rows 12288 x 4096 g128 230
+// in the loop): 8192 rows 12288 x 4096 g128 647 (695), 32000 x 4096 1664 (1793), 12288 x 4096 g32 699 (1056), g64 656 (765), g256 644; 3000 rows 32000 x 4096 g64 685 (804), 2048 rows 12288 x 4096 g128 230
 // (204), left to the other form.
 int64_t int4_unpacked_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int inner_k_tiles) {
   if (inner_k_tiles != 8 || (groupsize != 32 && groupsize != 64 && groupsize != 128 && groupsize != 256)) return 0;

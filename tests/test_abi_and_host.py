@@ -364,3 +364,9 @@ def test_rows_between_the_two_int4_kernels(m, n, k, groupsize, big):
     tiles = 2 if (n + 127) // 128 * ((m + 63) // 64) >= 256 else 1
     us = shape(m, n, k, min(groupsize, 128), 31 << 20).us
     assert on_32x32(m, n, k, groupsize, tiles, us) == big
+
+
+@pytest.mark.parametrize("m,n,k,groupsize,unpacked", [(6000, 32000, 4096, 64, True), (8192, 12288, 4096, 64, True), (2048, 22016, 8192, 64, True), (8192, 12288, 4096, 128, True), (8192, 12288, 4096, 32, True),
+                                                      (1300, 10240, 8192, 64, False), (1700, 22016, 8192, 64, False), (2048, 11008, 4096, 64, False), (2048, 12288, 4096, 128, False)])
+def test_int4_operands_are_unpacked_where_that_is_faster(m, n, k, groupsize, unpacked):
+    assert (_lib.load().e2h_int4_mm_scratch_bytes(m, n, k, groupsize, 8) > 0) == unpacked
