@@ -857,20 +857,25 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const e2h_window
   const int d = static_cast<int>(i % DV), h = static_cast<int>(i / DV % H), bi = static_cast<int>(i / DV / H), stride = rep * (DV + 2);
   const int pos = static_cast<int>(a.input_pos[0]), last = pos < a.cache_len ? pos : static_cast<int>(a.cache_len) - 1;
   const int parts = parts_with_keys(key_list(pos, last, a.first ? static_cast<int>(a.first[bi]) : 0, static_cast<int>(a.window), static_cast<int>(a.keep_first)).count, waves, splits);
-  if (parts == 1) return;  // the step has written the result
   const float *row = part + (static_cast<size_t>(bi) * G + h / rep) * splits * stride + (h % rep) * (DV + 2);
   constexpr int kAtOnce = 8;
   float m = kMasked, l = 0.f, o = 0.f;
-  for (int s0 = 0; s0 < parts; s0 += kAtOnce) {
+  int s0 = 0;
+  do {  // the first sums are requested while the count of parts is on its way: what no part has written is read and left
     float ms[kAtOnce], ls[kAtOnce], os[kAtOnce];
 #pragma unroll
     for (int k = 0; k < kAtOnce; ++k) {
-      const bool there = s0 + k < parts;
-      const float *p = row + static_cast<size_t>(there ? s0 + k : s0) * stride;
-      ms[k] = there ? p[DV] : kMasked;
-      ls[k] = there ? p[DV + 1] : 0.f;
-      os[k] = there ? p[d] : 0.f;
+      const float *p = row + static_cast<size_t>(s0 + k < splits ? s0 + k : 0) * stride;
+      ms[k] = p[DV];
+      ls[k] = p[DV + 1];
+      os[k] = p[d];
     }
+#pragma unroll
+    for (int k = 0; k < kAtOnce; ++k)
+      if (s0 + k >= parts) {
+        ms[k] = kMasked;
+        ls[k] = os[k] = 0.f;
+      }
     float m_new = m;
 #pragma unroll
     for (int k = 0; k < kAtOnce; ++k) m_new = fmaxf(m_new, ms[k]);
@@ -884,7 +889,9 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const e2h_window
       l = __builtin_fmaf(ls[k], c, l);
       o = __builtin_fmaf(os[k], c, o);
     }
-  }
+    s0 += kAtOnce;
+  } while (s0 < parts);
+  if (parts == 1) return;  // the step has written the result
   if (a.sink) l += __builtin_amdgcn_exp2f(__builtin_fmaf(a.sink[h], kLog2e, -m));
   o = l > 0.f ? o / l * a.out_scale : 0.f;
   if (a.g_off >= 0) o *= sigmoid_f32(to_f32(static_cast<const bf16_t *>(a.proj)[static_cast<size_t>(bi) * a.ld + a.g_off + static_cast<int64_t>(h) * DV + d]));
@@ -908,9 +915,9 @@ int step_waves(const e2h_window_attention_args &a) {
 // Workgroups per (sequence, key/value head) of the step, by the cache's capacity (the position is on the device), so that there is one per CU at most (two cost more than they share: 8 sequences x
 // 8 key heads over 2052 keys in 4 parts 18.8 us, in 8 parts 24.2).  A tile takes a wave 2.4 us and the combining launch 4 to 5, so fewer than
 // three tiles per wave are not shared (300 keys, 4 sequences: 9.2 us whole, 10.9 in two parts), and two parts never pay: 86 and more
-// workgroups already read at the memory's rate (16 sequences 27.2 us whole, 28.3 in two parts).  A position with few keys in a long cache pays 1.7 to 2
-// us for a launch that combines little or nothing (8 key heads, cache of 8192; one workgroup / this, us: 1 sequence, 17 keys 6.7 / 8.5, 500 11.1 / 12.7, 700 13.4 / 12.5, 2000 25 / 13;
-// 4 sequences 6.7 / 8.6, 11.9 / 13.9, 15.7 / 14.2, 32 / 18; with all workgroups of the capacity at work 11.9 at 17 keys of 1 sequence).
+// workgroups already read at the memory's rate (16 sequences 27.2 us whole, 28.3 in two parts).  A position with few keys in a long cache pays 1 to 3.5
+// us for a launch that combines little or nothing (8 key heads, cache of 8192; one workgroup / this, us: 1 sequence, 17 keys 6.7 / 8.9, 256 8.8 / 11.5, 500 11.1 / 12.2, 700 13.4 / 12.2,
+// 2000 25 / 12.6; 4 sequences 6.7 / 9.1, 9.3 / 12.8, 11.9 / 13.5, 15.8 / 14.0, 32 / 17.8; with all workgroups of the capacity at work 11.9 and 14.4 at 17 and 256 keys of 1 sequence).
 constexpr int kMostSplits = 64;
 int step_splits(const e2h_window_attention_args &a) {
   if (a.seqlen != 1 || !on_matrix_cores(a)) return 1;
