@@ -3,8 +3,9 @@
 // Four waves of 32 queries, key tiles of 64.  Both products on v_mfma_f32_16x16x32_bf16 in transposed form: S^T = K Q^T puts one query into each
 // lane column (lane 16 b + c holds keys 4 b .. 4 b + 3 of query c), so statistics are in-lane sums plus two shuffles, and the weights are the second operand of
 // O^T = V^T P^T without moving, over the key order 4 b .. 4 b + 3, 16 + 4 b .. 16 + 4 b + 3 of each 32.
-// What bounds it: products and the vector work between them take about as long, so two workgroups share a CU (64 KB of LDS each) and one computes
-// under the other's products.  32 queries per wave rather than 16, so that a fragment of K or V read from LDS feeds two or four products (with 16 the
+// What bounds it: the vector work between the products (scores, maxima, exponents, rounding) takes one and a half times as long as they do (8192 tokens, window 2048: matrix pipelines
+// busy 36 %, vector units 56 %; 64 x 768 tokens 24 and 44 %), and waves wait for a third of their time and more.  Two workgroups share a CU (64 KB of LDS each), so that one computes
+// under the other's products and waits.  32 queries per wave rather than 16, so that a fragment of K or V read from LDS feeds two or four products (with 16 the
 // LDS took longer than the products); K and V reach LDS by loads that write it directly, two stages, one barrier per tile, and V's
 // fragments leave it through the transposing read (written transposed by two-byte stores, V cost as much LDS time as both products' reads).
 #pragma once

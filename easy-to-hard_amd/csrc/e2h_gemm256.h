@@ -2,8 +2,8 @@
 //
 //   out[row][col] = sum_k x[row][k] w[col][k]      x rows and w rows of K values, K a multiple of 64 and at least 192
 //
-// What bounds it: the matrix pipelines, and with all of them busy the chip's power (1.6 - 1.75 GHz instead of 2.4), so that everything
-// that costs energy beside the products costs time.  One workgroup per CU of four waves, each 128 x 128 outputs in 256 accumulation registers
+// What bounds it: the matrix pipelines (busy 75 - 78 % of a launch that fills the chip, the library's kernel 83 %), and with all of them at work the chip's power (1.75 - 1.85 GHz instead of
+// 2.4), so that everything that costs energy beside the products costs time.  One workgroup per CU of four waves, each 128 x 128 outputs in 256 accumulation registers
 // (an LDS read of 16 values per lane feeds 64 products of 16 x 16 x 32; 256 x 64 per wave would read 1.25 times as much).  Operands reach LDS by
 // 16-byte loads that write LDS directly, in units of 256 rows x 64 k (32 KB, whole 128-byte lines: units of 32 k, which ask the L2 for every line
 // twice, ran at 1300 TFLOP/s where this runs at 1420 - 1520).  All 160 KB of LDS are a ring of five such units, x_0 w_0 x_1 w_1 ..: a unit's place

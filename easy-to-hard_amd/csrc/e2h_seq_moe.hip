@@ -6,7 +6,8 @@
 //   few rows    expert_step_kernel: a workgroup per expert in use (and 16 or 32 of its weight rows) finds the expert's slots itself
 //               and streams those weights once; waves split K.  The shared expert is part of the same launch.
 //   many rows   sort_slots_kernel orders the slots by expert, then expert_tiles_kernel: 256 x 128 outputs per workgroup, operands
-//               brought into LDS by direct 16-byte loads (token rows gathered by the loads themselves).
+//               brought into LDS by direct 16-byte loads (token rows gathered by the loads themselves); from 104 rows per expert on
+//               expert_big_tiles_kernel: 256 x 256 outputs (e2h_gemm256.h).
 //   otherwise   expert_plain_kernel on the vector units (float32, sizes that are not multiples of 8).
 // Matrix products are transposed (weights are the A operand), so a lane holds four neighbouring outputs of one token.
 #include "e2h_gemm256.h"
