@@ -295,6 +295,19 @@ def test_what_float16_does_not_hold_is_left_to_the_other_kernel(what):
     assert bool(same.all())
 
 
+@pytest.mark.parametrize("exponent,held", [(-50, False), (-49, True), (41, True), (42, False)])
+def test_units_of_columns_on_both_sides_of_their_ends(exponent, held):
+    """A column of scales 2^-49 .. 2^41 (8 s from 2^-46 to below 2^45) has a unit, one beyond sends the call to the other kernel; exact either way."""
+    m, n, k, g = 66049, 264, 512, 128
+    codes, scale, zero, x = _case(m, n, k, g)
+    scale[:, 3], zero[:, 3] = 2.0**exponent, 0.0
+    flag = []
+    got, _, need = _unpacked(codes, scale, zero, x, g, flag)
+    assert need > 0 and (flag[0] == 0) == held
+    rows = torch.tensor([0, 255, 4097, m - 1], device=DEV)
+    assert torch.equal(got[rows], _double(codes, scale, zero, x, g, rows).to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("g", [32, 128])
 def test_rows_of_an_unpacked_call_stand_alone(g):
     """Rows that the float16 form does not take (a NaN, an infinity, values over 2^60) leave every other row as it is without them, bit for bit, first, last and
