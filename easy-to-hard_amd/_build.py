@@ -18,7 +18,7 @@ CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libe2h_quant.so"
 SEQ_LIB_PATH = PKG_DIR / "libe2h_seq.so"
 
-SOURCES = ["e2h_abi.hip", "e2h_quantize.hip", "e2h_int4_mm.hip", "e2h_int4_staged.hip", "e2h_int8_mm.hip", "e2h_int8_stream.hip", "e2h_int4_gemm.hip", "e2h_int4_gemm128.hip", "e2h_int8_gemm.hip", "e2h_unpacked_gemm.hip", "e2h_attention.hip", "e2h_sample.hip", "e2h_probe.hip"]
+SOURCES = ["e2h_abi.hip", "e2h_quantize.hip", "e2h_int4_mm.hip", "e2h_int4_staged.hip", "e2h_int4_staged_g32.hip", "e2h_int4_staged_g64.hip", "e2h_int4_staged_g128.hip", "e2h_int8_mm.hip", "e2h_int8_stream.hip", "e2h_int4_gemm.hip", "e2h_int4_gemm128.hip", "e2h_int8_gemm.hip", "e2h_unpacked_gemm.hip", "e2h_attention.hip", "e2h_sample.hip", "e2h_probe.hip"]
 
 SEQ_SOURCES = ["e2h_seq_norm.hip", "e2h_seq_linear.hip", "e2h_seq_attention.hip", "e2h_seq_hgrn2.hip", "e2h_seq_delta.hip", "e2h_seq_moe.hip"]
 
@@ -40,7 +40,8 @@ HIPCC_FLAGS = [
 # Per-source additions.  The 32x32-tile matmul mixes MFMA accumulators with float32 FMAs on the same values; with
 # the accumulators in the accumulation register file every FMA needs copies in and out (3 extra instructions per FMA),
 # so that file is compiled with MFMA results kept in ordinary vector registers.
-EXTRA_FLAGS = {"e2h_int4_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "e2h_int4_staged.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}  # (the int8 kernel of the same shape has no such FMAs)
+_VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
+EXTRA_FLAGS = {s: _VGPR_FORM for s in ("e2h_int4_gemm.hip", "e2h_int4_staged_g32.hip", "e2h_int4_staged_g64.hip", "e2h_int4_staged_g128.hip")}  # (the int8 kernel of the same shape has no such FMAs)
 
 
 def _hipcc():

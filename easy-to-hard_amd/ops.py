@@ -742,7 +742,7 @@ def decode_attention(q, k_cache, v_cache, input_pos, left_pad_mask_pos=None, sca
 
 
 # ---------------------------------------------------------------------------------------------
-# decode batches on staged activations: the int4 kernels of csrc/e2h_int4_staged.hip read their activations in
+# decode batches on staged activations: the int4 kernels of csrc/e2h_int4_staged_kernel.h read their activations in
 # matrix-core operand order, written by the kernel that produces them (norm, attention, gated feed-forward) or
 # by stage_x for activations that arrive row-major
 # ---------------------------------------------------------------------------------------------

@@ -1,4 +1,4 @@
-"""GPU parity of the decode-batch int4 kernels that read staged activations (csrc/e2h_int4_staged.hip), through the
+"""GPU parity of the decode-batch int4 kernels that read staged activations (csrc/e2h_int4_staged_kernel.h), through the
 C ABI: the staging pass and every producer of staged activations against a numpy restatement of the layout, the
 matmul epilogues against the float32 dequantize-then-matmul oracle (gate max|y - y_ref| / max|y_ref| <= 1e-2) and,
 bit for bit, against each other."""
@@ -265,6 +265,15 @@ def test_staged_mm_is_exact_on_integers_at_the_edges(g, m, n, k):
 def test_staged_mm_on_both_sides_of_the_line_between_halves_and_whole_batches(g, m, n, k):
     """33 rows and more: two workgroups share the rows up to 2^25 weights (of both matrices in the gated launch), one takes them all above.
     Integers as above: sums stay below 8192 * 143 * 2 < 2^22."""
+    test_staged_mm_is_exact_on_integers_at_the_edges(g, m, n, k)
+
+
+@pytest.mark.parametrize("g", [32, 64, 128])
+@pytest.mark.parametrize("m", [1, 17, 64])
+@pytest.mark.parametrize("n,k", [(33040, 1152), (48, 16384), (4112, 8192)])
+def test_staged_mm_beyond_one_round_and_with_turned_chunks(g, m, n, k):
+    """More workgroups than compute units run as two of four waves on each, here with uneven runs of chunks; in rows of a multiple of 32 KB (K = 8192, 16384) every workgroup
+    starts with another chunk of its waves' runs.  Integers as above: sums stay below 16384 * 143 * 2 < 2^23."""
     test_staged_mm_is_exact_on_integers_at_the_edges(g, m, n, k)
 
 
