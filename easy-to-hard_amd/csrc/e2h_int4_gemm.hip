@@ -36,6 +36,7 @@
 //   piece ^ ((row >> 1) & 7);
 //   weights, 64 columns of one wave x 128 k, two stages: 64 bytes per column, pieces at piece ^ ((column >> 2) & 3), read by the wave
 //   that loaded them.
+// A gated launch (both matrices of silu(x w1) * (x w3)) gives a wave 32 columns of each, so that a lane holds both products of its outputs and multiplies them on the way out.
 // One barrier per 64 k.  Where the row count leaves the chip short of workgroups, S of them share K and leave float32 sums for a
 // second kernel to add in order.
 //
@@ -72,9 +73,15 @@ __device__ __forceinline__ float quotient(float a, float b) {
   return __builtin_fmaf(__builtin_fmaf(-q, b, a), rcp, q);
 }
 
+// F.silu(a) * b on bfloat16 tensors, before the last rounding
+__device__ __forceinline__ float gated(float a, float b) {
+  const float gate = bf16_round(a);
+  return bf16_round(gate / (1.0f + expf(-gate))) * bf16_round(b);
+}
+
 struct GemmArgs {
   const uint16_t *x;
-  const uint32_t *wp, *sz;
+  const uint32_t *wp, *sz, *wp2, *sz2;  // wp2, sz2: the second matrix of a gated launch
   uint16_t *y;
   float *partials;  // [S][M][N] when K is shared, else null
   const float *xsum;
@@ -83,8 +90,9 @@ struct GemmArgs {
   const int *run_if, *row_flag;  // not null: run_if[0] = 1 asks for everything, 2 for the rows m with row_flag[m] only, 0 for nothing
 };
 
-// kRT row tiles of 32 per wave: 32 kRT rows x 256 columns per workgroup
-template <int G, int kRT>
+// kRT row tiles of 32 per wave: 32 kRT rows x 256 columns per workgroup.  GATE: 128 columns of each of two matrices, a wave's first column tile from
+// the one and its second from the other, so that a lane ends up with both products of its outputs: y = bf16( bf16(silu(bf16 a)) * bf16 b ).
+template <int G, int kRT, bool GATE>
 __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
   constexpr int kRows = 32 * kRT, kXStage = kRows * 128, kWStage = kCols * 64, kLdsW = 3 * kXStage, kLdsBytes = kLdsW + 2 * kWStage;
   static_assert(2 * kLdsBytes <= 160 * 1024, "two workgroups per CU");
@@ -100,7 +108,9 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
-  const int row0 = rb * kRows, col0 = cb * kCols + 64 * wave;
+  constexpr int kWide = GATE ? 32 : 64;  // columns of a matrix per wave
+  const int row0 = rb * kRows, col0 = cb * (4 * kWide) + kWide * wave;
+  const auto column = [&](int ct) { return col0 + (GATE ? 0 : 32 * ct); };  // first one of a column tile
   const int *only = nullptr;
   if (a.run_if) {
     const int asked = *a.run_if;
@@ -119,6 +129,8 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
 
   const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(a.wp, static_cast<uint32_t>(static_cast<size_t>(N) * K / 2));
   const __amdgpu_buffer_rsrc_t sz_rsrc = make_rsrc(a.sz, static_cast<uint32_t>(static_cast<size_t>((K / G) >> a.shared) * N * 4));
+  const __amdgpu_buffer_rsrc_t w2_rsrc = make_rsrc(GATE ? a.wp2 : a.wp, static_cast<uint32_t>(static_cast<size_t>(N) * K / 2));
+  const __amdgpu_buffer_rsrc_t sz2_rsrc = make_rsrc(GATE ? a.sz2 : a.sz, static_cast<uint32_t>(static_cast<size_t>((K / G) >> a.shared) * N * 4));
   const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(a.x, static_cast<uint32_t>(static_cast<size_t>(M) * K * 2));
   const __amdgpu_buffer_rsrc_t xs_rsrc = make_rsrc(a.xsum, static_cast<uint32_t>(static_cast<size_t>(K / G) * a.xsum_stride * 4));
 
@@ -132,7 +144,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    int col = col0 + 16 * i + (lane >> 2);
+    int col = col0 + (GATE ? 16 * (i & 1) : 16 * i) + (lane >> 2);
     col = col < N ? col : N - 1;
     wsrc[i] = static_cast<uint32_t>(static_cast<size_t>(col >> 3) * KT * 512 + (col & 7) * 64 + ((lane & 3) ^ ((lane >> 4) & 3)) * 16);
   }
@@ -147,17 +159,17 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
     const uint32_t off = static_cast<uint32_t>(blk < blk1 - 1 ? blk : blk1 - 1) * 512u;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_void *)(lds + stage + (4 * wave + i) * 1024), 16, wsrc[i], off, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(GATE && i >= 2 ? w2_rsrc : w_rsrc, (lds_void *)(lds + stage + (4 * wave + i) * 1024), 16, wsrc[i], off, 0, 0);
   };
   uint32_t szlane[kCT];  // this lane's columns inside one [N] row of (scale, zero) pairs
 #pragma unroll
   for (int ct = 0; ct < kCT; ++ct) {
-    int col = col0 + 32 * ct + n;
+    int col = column(ct) + n;
     col = col < N ? col : N - 1;
     szlane[ct] = static_cast<uint32_t>(col) * 4u;
   }
   const auto load_sz = [&](int ct, int g) {
-    return __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, szlane[ct], static_cast<uint32_t>((g < g_end - 1 ? g : g_end - 1) >> a.shared) * N * 4u, 0);
+    return __builtin_amdgcn_raw_buffer_load_b32(GATE && ct > 0 ? sz2_rsrc : sz_rsrc, szlane[ct], static_cast<uint32_t>((g < g_end - 1 ? g : g_end - 1) >> a.shared) * N * 4u, 0);
   };
 
   load_w(blk0, kLdsW);
@@ -193,7 +205,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
       }
 #pragma unroll
       for (int ct = 0; ct < kCT; ++ct)
-        z[i].szw[ct] = __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, (szlane[ct] + ((gs + h) >> a.shared) * static_cast<uint32_t>(N) * 4u) | out, 0, 0);
+        z[i].szw[ct] = __builtin_amdgcn_raw_buffer_load_b32(GATE && ct > 0 ? sz2_rsrc : sz_rsrc, (szlane[ct] + ((gs + h) >> a.shared) * static_cast<uint32_t>(N) * 4u) | out, 0, 0);
     }
   };
   Zero za[kBatch], zb[kBatch];
@@ -416,7 +428,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
         float *out = a.partials + static_cast<size_t>(blockIdx.y) * M * N;
 #pragma unroll
         for (int ct = 0; ct < kCT; ++ct) {
-          const int col = col0 + 32 * ct + n;
+          const int col = column(ct) + n;
           if (col >= N) continue;
 #pragma unroll
           for (int rt = 0; rt < kRT; ++rt)
@@ -430,20 +442,34 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
       }
       int late = lane;
       asm volatile("" : "+v"(late));  // keeps the rows' addresses out of the registers of the main loop (the 128-row form of group size 64 would spill two)
-      const float no_scale[kCT] = {};
-      store_tiles_via_lds<kRT, kCT, false>(acc, no_scale, lds + wave * TileStore<kCT>::kBytesPerWave, a.y, row0, col0, M, N, late,
-                                          (N & 7) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0, only);
+      const bool pieces = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
+      if constexpr (GATE) {
+        const float no_scale[1] = {};
+        uint8_t *const tile = lds + wave * TileStore<1>::kBytesPerWave;
+#pragma unroll
+        for (int rt = 0; rt < kRT; ++rt) {
+          f32x16_t out[1][1];
+#pragma unroll
+          for (int e = 0; e < 16; ++e) out[0][0][e] = gated(acc[0][rt][e], acc[1][rt][e]);
+          store_tiles_via_lds<1, 1, false>(out, no_scale, tile, a.y, row0 + 32 * rt, col0, M, N, late, pieces, only);
+        }
+      } else {
+        const float no_scale[kCT] = {};
+        store_tiles_via_lds<kRT, kCT, false>(acc, no_scale, lds + wave * TileStore<kCT>::kBytesPerWave, a.y, row0, col0, M, N, late, pieces, only);
+      }
       return;
     }
   }
 
   // Every group's sum by itself, two row tiles at a time, operands straight from memory, nothing shared with the other waves.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the first loads still write LDS
+  [[maybe_unused]] f32x16_t first[2];
 #pragma unroll 1
-  for (int t = 0; t < kCT * ((kRT + 1) / 2); ++t) {
+  for (int t = 0; t < kCT * ((kRT + 1) / 2); ++t) {  // (gated: the two tiles of the same outputs after each other)
+    const bool second = GATE && (t & 1);
     int r0 = row0 + 64 * (t / kCT);
     asm volatile("" : "+s"(r0));  // keeps the addresses of all rows out of the registers of the loops
-    int col = col0 + 32 * (t % kCT) + n;
+    int col = column(t % kCT) + n;
     const bool live = col < N;
     col = live ? col : N - 1;
     const uint32_t wo = static_cast<uint32_t>(static_cast<size_t>(col >> 3) * KT * 512 + (col & 7) * 64);
@@ -463,7 +489,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
         u32x4_t u;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(w_rsrc, wo + 16u * j, static_cast<uint32_t>(step >> 3) * 512u + ((step >> 1) & 3) * 4u, 0);
+          const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(second ? w2_rsrc : w_rsrc, wo + 16u * j, static_cast<uint32_t>(step >> 3) * 512u + ((step >> 1) & 3) * 4u, 0);
           u[j] = (__builtin_amdgcn_alignbit(w, w, (8 * (step & 1) + 4 * h - 3) & 31) & 0x00780078u) | 0x41804180u;
         }
 #pragma unroll
@@ -472,7 +498,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
           part[rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf, __builtin_bit_cast(bf16x8_t, u), part[rt], 0, 0, 0);
         }
       }
-      const uint32_t szw = __builtin_amdgcn_raw_buffer_load_b32(sz_rsrc, static_cast<uint32_t>(col) * 4u, static_cast<uint32_t>(g >> a.shared) * N * 4u, 0);
+      const uint32_t szw = __builtin_amdgcn_raw_buffer_load_b32(second ? sz2_rsrc : sz_rsrc, static_cast<uint32_t>(col) * 4u, static_cast<uint32_t>(g >> a.shared) * N * 4u, 0);
       const float scale = __builtin_bit_cast(float, szw << 16), zero = __builtin_bit_cast(float, szw & 0xFFFF0000u);
       const float zc = __builtin_fmaf(-24.0f, scale, zero);
 #pragma unroll
@@ -485,6 +511,11 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
           for (int e = 0; e < 4; ++e) sum[rt][4 * q + e] = __builtin_fmaf(zc, xg[e], __builtin_fmaf(scale, part[rt][4 * q + e], sum[rt][4 * q + e]));
         }
     }
+    if (GATE && !second) {
+      first[0] = sum[0];
+      first[1] = sum[1];
+      continue;
+    }
     if (!live) continue;
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt)
@@ -493,7 +524,7 @@ __global__ __launch_bounds__(256, 2) void int4_gemm_kernel(const GemmArgs a) {
         const int m = r0 + 32 * rt + 8 * (e >> 2) + 4 * h + (e & 3);
         if (m >= M || m >= row0 + kRows || (only && !only[m])) continue;
         if (a.partials) a.partials[(static_cast<size_t>(blockIdx.y) * M + m) * N + col] = sum[rt][e];
-        else a.y[static_cast<size_t>(m) * N + col] = f32_to_bf16_rne(sum[rt][e]);
+        else a.y[static_cast<size_t>(m) * N + col] = f32_to_bf16_rne(GATE ? gated(first[rt][e], sum[rt][e]) : sum[rt][e]);
       }
   }
 }
@@ -562,16 +593,34 @@ Int4GemmShape int4_gemm_shape(int M, int N, int K, int groupsize, int64_t scratc
   return best;
 }
 
-template <int G>
+template <int G, bool GATE>
 void launch_gemm(const GemmArgs &a, int rows, dim3 grid, hipStream_t stream) {
   if constexpr (G != 32) {
     if (rows != 64) {
-      if (rows == 128) hipLaunchKernelGGL((int4_gemm_kernel<G, 4>), grid, dim3(256), 0, stream, a);
-      else hipLaunchKernelGGL((int4_gemm_kernel<G, 3>), grid, dim3(256), 0, stream, a);
+      if (rows == 128) hipLaunchKernelGGL((int4_gemm_kernel<G, 4, GATE>), grid, dim3(256), 0, stream, a);
+      else hipLaunchKernelGGL((int4_gemm_kernel<G, 3, GATE>), grid, dim3(256), 0, stream, a);
       return;
     }
   }
-  hipLaunchKernelGGL((int4_gemm_kernel<G, 2>), grid, dim3(256), 0, stream, a);
+  hipLaunchKernelGGL((int4_gemm_kernel<G, 2, GATE>), grid, dim3(256), 0, stream, a);
+}
+
+template <bool GATE>
+int launch_gemm(const GemmArgs &args, int groupsize, Int4GemmShape shape, hipStream_t stream) {
+  GemmArgs a = args;
+  const int wide = GATE ? kCols / 2 : kCols;
+  a.n_col_blocks = (a.N + wide - 1) / wide;
+  a.cbx = (a.n_col_blocks + 7) / 8;
+  const long long wgs = 8LL * a.cbx * ((a.M + shape.rows - 1) / shape.rows);
+  if (wgs > 0x7FFFFFFFLL) return E2H_ERR_BAD_SHAPE;
+  const dim3 grid(static_cast<unsigned>(wgs), static_cast<unsigned>(shape.slices));
+  switch (groupsize) {
+    case 32: launch_gemm<32, GATE>(a, shape.rows, grid, stream); break;
+    case 64: launch_gemm<64, GATE>(a, shape.rows, grid, stream); break;
+    case 128: launch_gemm<128, GATE>(a, shape.rows, grid, stream); break;
+    default: return E2H_ERR_BAD_GROUPSIZE;
+  }
+  return E2H_OK;
 }
 
 int int4_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint16_t *y, const float *xsum, int xsum_stride,
@@ -579,18 +628,10 @@ int int4_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint
   if (K % 128 != 0 || N % 8 != 0) return E2H_ERR_BAD_SHAPE;
   const int shared = groupsize == 256;
   if (shared) groupsize = 128;
-  GemmArgs a = {x, reinterpret_cast<const uint32_t *>(packed), reinterpret_cast<const uint32_t *>(sz), y, shape.slices > 1 ? partials : nullptr,
-                xsum, xsum_stride, M, N, K, (N + kCols - 1) / kCols, 0, shared, run_if, row_flag};
-  a.cbx = (a.n_col_blocks + 7) / 8;
-  const long long wgs = 8LL * a.cbx * ((M + shape.rows - 1) / shape.rows);
-  if (wgs > 0x7FFFFFFFLL) return E2H_ERR_BAD_SHAPE;
-  const dim3 grid(static_cast<unsigned>(wgs), static_cast<unsigned>(shape.slices));
-  switch (groupsize) {
-    case 32: launch_gemm<32>(a, shape.rows, grid, stream); break;
-    case 64: launch_gemm<64>(a, shape.rows, grid, stream); break;
-    case 128: launch_gemm<128>(a, shape.rows, grid, stream); break;
-    default: return E2H_ERR_BAD_GROUPSIZE;
-  }
+  const GemmArgs a = {x, reinterpret_cast<const uint32_t *>(packed), reinterpret_cast<const uint32_t *>(sz), nullptr, nullptr, y, shape.slices > 1 ? partials : nullptr,
+                      xsum, xsum_stride, M, N, K, 0, 0, shared, run_if, row_flag};
+  const int rc = launch_gemm<false>(a, groupsize, shape, stream);
+  if (rc != E2H_OK) return rc;
   if (shape.slices > 1) {
     const int64_t quads = static_cast<int64_t>(M) * N / 4;
     hipLaunchKernelGGL(add_slices_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, stream, partials, y, quads,
@@ -599,4 +640,64 @@ int int4_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint
   return launch_status();
 }
 
+int int4_gemm_gate(const uint16_t *x, const int32_t *packed, const uint16_t *sz, const int32_t *packed2, const uint16_t *sz2, uint16_t *y, const float *xsum,
+                   int xsum_stride, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream) {
+  if (K % 128 != 0 || N % 8 != 0 || shape.slices != 1) return E2H_ERR_BAD_SHAPE;
+  const int shared = groupsize == 256;
+  const GemmArgs a = {x, reinterpret_cast<const uint32_t *>(packed), reinterpret_cast<const uint32_t *>(sz), reinterpret_cast<const uint32_t *>(packed2),
+                      reinterpret_cast<const uint32_t *>(sz2), y, nullptr, xsum, xsum_stride, M, N, K, 0, 0, shared, nullptr, nullptr};
+  const int rc = launch_gemm<true>(a, shared ? 128 : groupsize, shape, stream);
+  return rc != E2H_OK ? rc : launch_status();
+}
+
 }  // namespace e2h
+
+namespace e2h {
+int64_t int4_unpacked_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int inner_k_tiles);
+constexpr int kUnpackRows = 1024;  // from here on callers offer memory for unpacked operands
+
+// Group sums of x, the only scratch of a gated call, or 0 where two calls and a pass that multiplies are expected to be no slower or a form is asked for by an option.
+// The launch of both matrices has twice the workgroups, spares one pass over x for its group sums, the two products' way to memory and back, and a launch.  Measured, us, two calls and
+// the pass / here: 2 x 11008 x 4096 g128 65 rows 61 / 54, 128 rows 72 / 51, 471 rows 117 / 97, 1500 rows 298 / 273; g64 471 rows 141 / 112; g32 192 rows 132 / 96; 2 x 5504 x 2048
+// g128 256 rows 53 / 32.  Over 440 shapes and rows (65 .. 4096) 21 % less; the expected times, 7 % in favour of the calls, leave four that are slower, by 2.5 % at most (2 x 22016 x 8192, 320
+// rows, where the calls fill their last rounds, 266 / 288: left to them).  Calls on unpacked operands (e2h_unpacked_gemm.hip) stay with those.
+int64_t int4_gate_rows_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int inner_k_tiles) {
+  if (inner_k_tiles != 8 || (groupsize != 32 && groupsize != 64 && groupsize != 128 && groupsize != 256)) return 0;
+  if (M <= 64 || N < 8 || N % 8 != 0 || K < 128 || K % 128 != 0 || K % groupsize != 0 || M > INT32_MAX / 64 || N > INT32_MAX / 64 || K > INT32_MAX / 64) return 0;
+  if (M * K * 2 >= (int64_t{1} << 32) || N * K / 2 >= (int64_t{1} << 32) || K / groupsize * N * 4 >= (int64_t{1} << 32)) return 0;
+  const int G = groupsize == 256 ? 128 : groupsize;
+  const int64_t bytes = K / G * ((M + 63) / 64 * 64) * 4;
+  if (bytes >= (int64_t{1} << 32)) return 0;
+  const Options &o = options();
+  if (o.int4_no_gemm32 || o.int4_gemm_tile || o.int4_gemm32_min_rows || o.int4_no_xsum || o.int4_k_slices || o.int4_rows_per_wave || o.row_tiles) return 0;
+  const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
+  if (M >= kUnpackRows && int4_unpacked_bytes(M, N, K, groupsize, inner_k_tiles) > 0) return 0;
+  const double calls = 2 * int4_gemm_shape(m, n, k, G, int64_t{32} << 20).us + 3 + static_cast<double>(M) * static_cast<double>(N) * 6 / 5e6;  // the pass moves six bytes an output
+  return 1.07 * int4_gemm_shape(m, 2 * n, k, G, 0).us < calls ? bytes : 0;
+}
+}  // namespace e2h
+
+extern "C" int64_t e2h_int4_mm_silu_gate_rows_scratch_bytes(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles) {
+  return e2h::int4_gate_rows_bytes(m, n, k, groupsize, inner_k_tiles);
+}
+
+extern "C" int e2h_int4_mm_silu_gate_rows(const uint16_t *x, const int32_t *packed_gate, const uint16_t *sz_gate, const int32_t *packed_up, const uint16_t *sz_up,
+                                          uint16_t *y, int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles, void *scratch, int64_t scratch_bytes,
+                                          void *stream) {
+  using namespace e2h;
+  if (!x || !packed_gate || !sz_gate || !packed_up || !sz_up || !y || !scratch) return E2H_ERR_NULL_POINTER;
+  if (groupsize != 32 && groupsize != 64 && groupsize != 128 && groupsize != 256) return E2H_ERR_BAD_GROUPSIZE;
+  if (inner_k_tiles != 8) return E2H_ERR_BAD_INNER_K_TILES;
+  const int64_t need = int4_gate_rows_bytes(m, n, k, groupsize, inner_k_tiles);
+  if (need == 0) return E2H_ERR_BAD_SHAPE;
+  if (scratch_bytes < need) return E2H_ERR_SCRATCH_TOO_SMALL;
+  if (!aligned16(x) || !aligned16(packed_gate) || !aligned16(sz_gate) || !aligned16(packed_up) || !aligned16(sz_up) || !aligned16(scratch) ||
+      (reinterpret_cast<uintptr_t>(y) & 1u))
+    return E2H_ERR_MISALIGNED;
+  const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k), G = groupsize == 256 ? 128 : groupsize, stride = (M + 63) / 64 * 64;
+  float *xsum = static_cast<float *>(scratch);
+  const int rc = launch_x_group_sums(x, xsum, M, K, stride, G, static_cast<hipStream_t>(stream));
+  if (rc != E2H_OK) return rc;
+  return int4_gemm_gate(x, packed_gate, sz_gate, packed_up, sz_up, y, xsum, stride, int4_gemm_shape(M, 2 * N, K, G, 0), M, N, K, groupsize,
+                        static_cast<hipStream_t>(stream));
+}

@@ -276,6 +276,26 @@ class FeedForward(nn.Module):
             return False
         return ops.int8_gate_supported(x, w1, w3)
 
+    def _gate_rows(self, x: Tensor) -> Optional[Tensor]:
+        """silu(w1 x) * w3 x of a prompt with one launch for both products, or None where the modules are to be called: few rows, weights that differ in form or do not fit x,
+        somebody who watches their calls, or no gain."""
+        w1, w3 = self.w1, self.w3
+        if not (FUSE_GATE and _fusable(x) and type(w1) is WeightOnlyInt4Linear and type(w3) is WeightOnlyInt4Linear) or torch.compiler.is_compiling():
+            return None
+        k, n, group = w1.in_features, w1.out_features, w1.groupsize
+        if x.shape[-1] != k or x.numel() <= 64 * k or w1.padding or w3.padding or w3.groupsize != group:
+            return None
+        for w in (w1, w3):
+            p, sz = w.weight, w.scales_and_zeros
+            if not (p.dtype == torch.int32 and sz.dtype == torch.bfloat16 and p.device == x.device and sz.device == x.device and p.dim() == 4
+                    and p.shape[3] == 4 and p.shape[2] == 32 and p.shape[0] * 8 == n == w.out_features and p.shape[1] * 128 == k
+                    and tuple(sz.shape) == (k // group, n, 2) and unwatched(w)):
+                return None
+        if seq_ops.watched(x, w1.weight, w1.scales_and_zeros, w3.weight, w3.scales_and_zeros):
+            return None
+        y = ops.int4_mm_silu_gate_rows(x.reshape(-1, k), w1.weight, w1.scales_and_zeros, w3.weight, w3.scales_and_zeros, group)
+        return None if y is None else y.view(*x.shape[:-1], n)
+
     def forward(self, x: Tensor, defer_output: bool = False) -> Tensor:
         if defer_output and self._gate_fusable_int8(x):
             y = ops.int8_mm_silu_gate(x.reshape(-1, x.shape[-1]), self.w1.weight, self.w1.scales, self.w3.weight, self.w3.scales)
@@ -292,6 +312,9 @@ class FeedForward(nn.Module):
             y = ops.int4_mm_silu_gate(x.reshape(-1, x.shape[-1]), self.w1.weight, self.w1.scales_and_zeros,
                                       self.w3.weight, self.w3.scales_and_zeros, self.w1.groupsize)
             return self.w2(y.reshape(*x.shape[:-1], y.shape[-1]))
+        y = self._gate_rows(x)
+        if y is not None:
+            return self.w2(y)
         a, b = self.w1(x), self.w3(x)
         if _fusable(a) and a.numel() % 8 == 0:
             return self.w2(ops.silu_mul(a, b))

@@ -367,6 +367,45 @@ def int4_mm_silu_gate(x, packed_gate, sz_gate, packed_up, sz_up, groupsize):
     return y
 
 
+def int4_gate_rows_scratch(m, n, k, groupsize, inner_k_tiles, device):
+    """Scratch for int4_mm_silu_gate_rows, or None: the sizes are not for that launch, or there is no memory left for it."""
+    need = _lib.load().e2h_int4_mm_silu_gate_rows_scratch_bytes(m, n, k, groupsize, inner_k_tiles)
+    if need <= 0:
+        return None
+    try:
+        return torch.empty((need,), dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
+def int4_mm_silu_gate_rows(x, packed_gate, sz_gate, packed_up, sz_up, groupsize):
+    """bf16(bf16(silu(int4_mm(x, gate))) * int4_mm(x, up)) over more than 64 rows in one product launch, or None where two calls of int4_mm are
+    no slower (or there is no memory for the launch's scratch)."""
+    _need_gpu(x, packed_gate, sz_gate, packed_up, sz_up)
+    if x.dtype != torch.bfloat16 or sz_gate.dtype != torch.bfloat16 or sz_up.dtype != torch.bfloat16:
+        raise TypeError("int4_mm_silu_gate_rows: bfloat16 activations and scales_and_zeros expected")
+    assert x.dim() == 2
+    n, k, ikt = _packed_dims(packed_gate)
+    if _packed_dims(packed_up) != (n, k, ikt):
+        raise RuntimeError("int4_mm_silu_gate_rows: the two packed weights differ in shape")
+    m = x.shape[0]
+    if x.shape[1] != k:
+        raise RuntimeError(f"int4_mm_silu_gate_rows: x has K={x.shape[1]}, packed weights have K={k}")
+    for sz in (sz_gate, sz_up):
+        if groupsize not in _VALID_GROUPS or k % groupsize != 0 or tuple(sz.shape) != (k // groupsize, n, 2):
+            raise RuntimeError(f"int4_mm_silu_gate_rows: groupsize={groupsize} does not fit scales_and_zeros {tuple(sz.shape)} and K={k}")
+    scratch = int4_gate_rows_scratch(m, n, k, groupsize, ikt, x.device)
+    if scratch is None:
+        return None
+    x, packed_gate, sz_gate = x.contiguous(), packed_gate.contiguous(), sz_gate.contiguous()
+    packed_up, sz_up = packed_up.contiguous(), sz_up.contiguous()
+    y = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    rc = _lib_for(x).e2h_int4_mm_silu_gate_rows(_ptr(x), _ptr(packed_gate), _ptr(sz_gate), _ptr(packed_up), _ptr(sz_up), _ptr(y), m, n, k, groupsize, ikt,
+                                                _ptr(scratch), scratch.numel(), _stream(x))
+    _lib.check(rc, "e2h_int4_mm_silu_gate_rows")
+    return y
+
+
 # ---------------------------------------------------------------------------------------------
 # torch.library registrations (operator boundary that replaces the two aten int4 ops and the
 # F.linear * scales pair of the reference)

@@ -197,6 +197,16 @@ int e2h_int4_mm_rope_kv(const uint16_t *x, const int32_t *packed, const uint16_t
                         int64_t head_dim, int64_t cache_len, int64_t k, int groupsize, int inner_k_tiles,
                         void *stream);
 
+/* The gated launch over many rows, y = bf16(bf16(silu(x @ gate^T)) * (x @ up^T)) with both products rounded to bfloat16 first: what two calls of
+ * e2h_int4_mm and e2h_silu_mul give, with the same sums in float32 as e2h_int4_mm has over the 32 x 32 tiles of such calls with one K slice.
+ *   65 <= m, any group size of e2h_int4_mm, inner_k_tiles == 8, k % 128 == 0, n % 8 == 0; scratch 16-byte aligned, scratch_bytes >= what
+ *   e2h_int4_mm_silu_gate_rows_scratch_bytes returns, which is 0 where the shape is not taken (or not faster than those calls: the entry point then returns
+ *   E2H_ERR_BAD_SHAPE).  The launch neither allocates nor keeps anything. */
+int64_t e2h_int4_mm_silu_gate_rows_scratch_bytes(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles);
+int e2h_int4_mm_silu_gate_rows(const uint16_t *x, const int32_t *packed_gate, const uint16_t *sz_gate, const int32_t *packed_up,
+                               const uint16_t *sz_up, uint16_t *y, int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles,
+                               void *scratch, int64_t scratch_bytes, void *stream);
+
 /* int8 forms of the two fused decode-step launches above (WeightOnlyInt8Linear modules, reference
  * models/quantize.py:405-429, in FeedForward.forward models/model.py:343-344 and Attention.forward :283-296).
  * Each linear's output is formed with the reference's two roundings, bf16(bf16(x @ q^T) * scales), before the SiLU-gate

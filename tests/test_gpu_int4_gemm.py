@@ -182,6 +182,76 @@ def test_a_row_differs_by_float32_rounding_at_most_between_row_counts(g, n, k):
         assert ((part.double() - full[:rows].double()).abs() <= bound[:rows]).all()
 
 
+# ---- both matrices of a gated feed-forward in one launch --------------------------------------------------------------------------------
+# workgroups of 64, 96 and 128 rows (the last three), columns that end inside a wave's 32 and a workgroup's 128, odd counts of 128-wide k blocks; scales up to 2^15
+# leave the running units (above 2^13) in some workgroups only
+@pytest.mark.parametrize("g", [32, 64, 128, 256])
+@pytest.mark.parametrize("high", [-4, 15])
+@pytest.mark.parametrize("m,n,k", [(65, 8, 256), (129, 264, 768), (471, 1032, 1280), (190, 12296, 256), (200, 12296, 512), (1000, 2056, 256)])
+def test_gated_rows_are_the_two_exact_products_gated(g, high, m, n, k):
+    """Dyadic operands as above: both products have to be exactly rounded, and the gate is what ops.silu_mul makes of them."""
+    halves = [_case(m, n, k, g, seed=seed, low=-9, high=-4) for seed in (5, 77)]
+    halves[1][1][:, 3::97] = 2.0 ** high
+    halves[1][2][:, 3::97] = 0.0  # (multiples of 2^15 beside quarters would not fit 24 bits; without them these columns are multiples of their scale below 2^24 of it)
+    x = halves[0][3]
+    weights = []
+    for codes, scale, zero, _ in halves:
+        weights += [torch.from_numpy(qo.int4_tile_pack(codes.numpy(), 8)).to(DEV), torch.stack([scale, zero], dim=-1).to(torch.bfloat16).contiguous().to(DEV)]
+    got = ops.int4_mm_silu_gate_rows(x, *weights, g)
+    assert got is not None  # these sizes are taken
+    a, b = (x.double() @ ((c.double() - 8).view(n, k // g, g) * s.double().t()[:, :, None] + z.double().t()[:, :, None]).view(n, k).to(DEV).t() for c, s, z, _ in halves)
+    assert torch.equal(got, ops.silu_mul(a.to(torch.bfloat16), b.to(torch.bfloat16)))
+
+
+@pytest.mark.parametrize("g", [32, 64, 128, 256])
+def test_gated_rows_form_what_float32_units_do_not_hold(g):
+    """Infinite and NaN scales, sums that leave float32's range only in units of a scale, rows of x that are not finite: as two calls of the kernel give them."""
+    m, n, k = 471, 1032, 1280
+    gen = torch.Generator().manual_seed(g)
+    x = torch.randn((m, k), generator=gen).to(torch.bfloat16)
+    x[3, 5], x[200, 7] = float("inf"), float("nan")
+    w = [ops.int4_quantize_pack((torch.randn((n, k), generator=gen) * 0.02).to(torch.bfloat16).to(DEV), g, 8) for _ in range(2)]
+    w[0][1][0, 17, 0], w[0][1][-1, 600, 0], w[1][1][0, 333, 0] = float("inf"), float("nan"), 2.0 ** -20
+    w[1][1][0, 333, 1] = 2.0 ** 100
+    x = x.to(DEV)
+    got = ops.int4_mm_silu_gate_rows(x, *w[0], *w[1], g)
+    _lib.set_option("int4_gemm32_min_rows", 1)
+    try:
+        want = ops.silu_mul(*(ops.int4_mm(x, p, g, sz) for p, sz in w))
+    finally:
+        _lib.set_option("int4_gemm32_min_rows", 0)
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    fine = torch.isfinite(want)
+    assert torch.equal(got[~fine & ~torch.isnan(want)], want[~fine & ~torch.isnan(want)])
+    # one product may differ by a rounding to bfloat16 (K slices of the two calls), the gate of it by its slope: at most 1.1 in relative size away from its zero
+    assert ((got[fine].double() - want[fine].double()).norm() <= 2 ** -8 * want[fine].double().norm()).item()
+
+
+def test_gated_rows_leave_watched_modules_and_other_forms_to_the_modules():
+    from easy_to_hard_amd.model import FeedForward, ModelArgs
+    from easy_to_hard_amd.quantize import WeightOnlyInt4QuantHandler, prepare_int4_weight_and_scales_and_zeros
+
+    args = ModelArgs(dim=512, intermediate_size=1024, n_head=4, n_layer=1)
+    ff = FeedForward(args)
+    WeightOnlyInt4QuantHandler(ff, groupsize=64).convert_for_runtime()
+    gen = torch.Generator().manual_seed(1)
+    for lin in (ff.w1, ff.w2, ff.w3):
+        w = (torch.randn((lin.out_features, lin.in_features), generator=gen) * 0.05).to(torch.bfloat16).to(DEV)
+        lin.weight, lin.scales_and_zeros = prepare_int4_weight_and_scales_and_zeros(w, 64, 8)
+    x = torch.randn((3, 40, 512), generator=gen).to(torch.bfloat16).to(DEV)
+    whole = ff(x)
+    assert ff._gate_rows(x).shape == (3, 40, 1024)
+    seen = []
+    handle = ff.w3.register_forward_hook(lambda *_: seen.append(1))
+    assert ff._gate_rows(x) is None
+    assert seen == [] and (ff(x).double() - whole.double()).norm() <= 2 ** -7 * whole.double().norm() and seen == [1]
+    handle.remove()
+    assert ff._gate_rows(x[:, :20]) is None  # 60 rows: the decode launch
+    assert ff._gate_rows(x.float()) is None and ff._gate_rows(x[..., :384]) is None
+    strided = x.transpose(0, 1)
+    assert torch.equal(ff._gate_rows(strided), ff._gate_rows(x).transpose(0, 1))
+
+
 # ---- weights unpacked to float16 first (csrc/e2h_unpacked_gemm.hip) ---------------------------------------------------------------------
 
 def _unpacked(codes, scale, zero, x, g, flag=None):
