@@ -2,6 +2,8 @@
 Llama decode step) and libe2h_seq.so (include/e2h_seq.h, the layers with per-sequence state and
 mixtures of experts).
 
+A third, small object is a CPython extension module: the host side of calls of small linears (_calls.so, csrc/e2h_calls.cpp).
+
 The libraries are built in-tree, next to this file, so that they travel with the source tree; nothing is
 installed into site-packages and no JIT cache is involved.  They are separate so that a model that needs one of them
 compiles only that one.
@@ -17,6 +19,7 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libe2h_quant.so"
 SEQ_LIB_PATH = PKG_DIR / "libe2h_seq.so"
+CALLS_PATH = PKG_DIR / "_calls.so"
 
 SOURCES = ["e2h_abi.hip", "e2h_quantize.hip", "e2h_int4_mm.hip", "e2h_int4_staged.hip", "e2h_int4_staged_g32.hip", "e2h_int4_staged_g64.hip", "e2h_int4_staged_g128.hip", "e2h_int8_mm.hip", "e2h_int8_stream.hip", "e2h_int4_gemm.hip", "e2h_int4_gemm128.hip", "e2h_int8_gemm.hip", "e2h_unpacked_gemm.hip", "e2h_attention.hip", "e2h_sample.hip", "e2h_probe.hip"]
 
@@ -89,6 +92,28 @@ def build_seq_library(verbose=False):
     return _compile_and_link(SEQ_SOURCES, SEQ_LIB_PATH, verbose)
 
 
+def build_calls(verbose=False):
+    """The host-side extension module of small calls (csrc/e2h_calls.cpp), against the installed torch."""
+    import sysconfig
+
+    import torch
+
+    home = Path(torch.__file__).resolve().parent
+    cxx = shutil.which(os.environ.get("CXX", "g++"))
+    if cxx is None:
+        raise RuntimeError("no host C++ compiler found; the extension module of small calls cannot be built")
+    rocm = Path(_hipcc()).resolve().parent.parent
+    tmp = CALLS_PATH.with_name(CALLS_PATH.name + ".tmp")
+    out = _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+                *(f"-I{d}" for d in (home / "include", home / "include" / "torch" / "csrc" / "api" / "include", rocm / "include", sysconfig.get_paths()["include"])),
+                str(CSRC / "e2h_calls.cpp"), "-o", str(tmp), f"-L{home / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"])
+    if verbose and out.strip():
+        print(out)
+    os.replace(tmp, CALLS_PATH)
+    return CALLS_PATH
+
+
 if __name__ == "__main__":
+    print(build_calls(verbose=True))
     print(build_library(verbose=True))
     print(build_seq_library(verbose=True))

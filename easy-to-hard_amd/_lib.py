@@ -5,9 +5,10 @@ no fallback implementation behind these entry points.
 """
 
 import ctypes
+import importlib.util
 from ctypes import c_char_p, c_float, c_int, c_int32, c_int64, c_void_p
 
-from ._build import LIB_PATH, SEQ_LIB_PATH, build_library, build_seq_library
+from ._build import CALLS_PATH, LIB_PATH, SEQ_LIB_PATH, build_library, build_seq_library
 
 _P = c_void_p
 _SIGNATURES = {
@@ -15,6 +16,7 @@ _SIGNATURES = {
     "e2h_abi_version": (c_int, []),
     "e2h_status_string": (c_char_p, [c_int]),
     "e2h_set_option": (c_int, [c_char_p, c_int]),
+    "e2h_stream_capturing": (c_int, [_P]),
     "e2h_int8_quantize_per_channel": (c_int, [_P, c_int, _P, _P, _P, c_int64, c_int64, _P]),
     "e2h_int4_mm_scratch_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int, c_int]),
     "e2h_int4_mm_scratch": (c_int, [_P, _P, _P, _P, c_int64, c_int64, c_int64, c_int, c_int, _P, c_int64, _P, c_int64, _P]),
@@ -182,6 +184,25 @@ def load_seq(build_if_missing=False):
     if _seq_lib is None:
         _seq_lib = _open(SEQ_LIB_PATH, build_seq_library, build_if_missing, _SEQ_SIGNATURES, "e2h_seq_abi_version", 2)
     return _seq_lib
+
+
+_calls = None
+
+
+def calls():
+    """The extension module of small calls (csrc/e2h_calls.cpp), bound to libe2h_quant.so and the workspaces of `ops`."""
+    global _calls
+    if _calls is None:
+        if not CALLS_PATH.exists():
+            raise E2HLibraryError(f"{CALLS_PATH} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`")
+        from . import ops
+
+        spec = importlib.util.spec_from_file_location(f"{__package__}._calls", CALLS_PATH)
+        module, lib = importlib.util.module_from_spec(spec), load()
+        spec.loader.exec_module(module)
+        module.bind(*(ctypes.cast(f, c_void_p).value for f in (lib.e2h_int4_mm, lib.e2h_int8_mm, lib.e2h_stream_capturing)), ops._workspaces)
+        _calls = module
+    return _calls
 
 
 _STATUS_TEXT = {-1: "a required pointer is NULL", -2: "unsupported shape", -5: "pointer not aligned as required", -6: "HIP kernel launch failed",

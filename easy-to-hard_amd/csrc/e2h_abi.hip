@@ -120,3 +120,8 @@ extern "C" int e2h_set_option(const char *name, int value) {
   }
   return E2H_ERR_BAD_OPTION;
 }
+
+extern "C" int e2h_stream_capturing(void *stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status) != hipSuccess || status != hipStreamCaptureStatusNone;
+}

@@ -223,6 +223,9 @@ int e2h_int8_mm_rope_kv(const uint16_t *x, const int8_t *q, const uint16_t *scal
 /* Recommended size in bytes of the workspace accepted by the matmul entry points (no reference counterpart). */
 int64_t e2h_workspace_bytes(void);
 
+/* 0 where the stream records no graph (what a caller that keeps a workspace per stream asks before it uses the eager one), else 1. */
+int e2h_stream_capturing(void *stream);
+
 /* ------------------------------------------------------------------------------------------------
  * Decode-step kernels around the quantized linears (callers of the hot path; stock-op equivalents in the
  * reference's models/model.py).  bf16 everywhere, float32 arithmetic inside.
