@@ -365,32 +365,29 @@ __global__ __launch_bounds__(64 * NW) void decode_attention_gqa_kernel(const uin
 // ------------------------------------------------------------------------------------------------
 // One workgroup of BLOCK threads per row.  With `delta` the kernel first forms h = bf16(x + delta) (the residual add
 // of TransformerBlock.forward, reference :279-282), stores it to h_out and normalises h.  The first kPieces pieces of
-// 8 values per thread stay in registers and all their loads are issued before anything is waited for (one memory
+// 8 values per thread stay in registers and all their loads, slices and weights included, are issued before anything is waited for (one memory
 // round trip for the whole row up to BLOCK * 8 * kPieces values); longer rows re-read the rest.
-template <int BLOCK>
+// What bounds it in a decode step: the launch and one memory round trip.  64 rows of 8192 with two slices: 7.2 us with 512 threads, whose second pieces asked for their
+// slices when the first had arrived, 5.7 with 1024; 32 rows of 4096 5.1 either way.
+enum NormTerm { kNothing = 0, kDelta = 1, kSums = 2 };  // what is added to x first
+
+template <int BLOCK, NormTerm SRC>
 __global__ __launch_bounds__(BLOCK) void rmsnorm_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ delta,
                                                         const float *__restrict__ psum, int slices,
                                                         const uint16_t *__restrict__ col_scales,
                                                         const uint16_t *__restrict__ w, uint16_t *__restrict__ h_out,
                                                         uint16_t *__restrict__ y, StagedOut staged, int dim, float eps) {
-  constexpr int kPieces = 2, kStride = BLOCK * 8, kWaves = BLOCK / 64;
+  constexpr int kPieces = BLOCK == 256 ? 2 : 1, kStride = BLOCK * 8, kWaves = BLOCK / 64;
   constexpr int kMaxSlices = 4;  // slices whose loads are all issued before the first addition
   const size_t row = blockIdx.x;
   const uint16_t *xr = x + row * dim;
-  const uint16_t *dr_row = delta ? delta + row * dim : nullptr;
+  const uint16_t *dr_row = SRC == kDelta ? delta + row * dim : nullptr;
   // psum: the term to add arrives as float32 partial sums [slices][rows][dim] of a matmul split along K; the term is
   // bf16(p[0] + p[1] + .. in slice order), the value the matmul's own combine step would have stored -- with
   // col_scales (int8 weights) bf16(that * scale[column]), the two roundings of the int8 linear
   const size_t slice_floats = static_cast<size_t>(gridDim.x) * dim;
-  const float *pr = psum ? psum + row * dim : nullptr;
-  auto sum_slices = [&](int i) {
-    f32x4_t lo[kMaxSlices], hi[kMaxSlices];
-#pragma unroll
-    for (int u = 0; u < kMaxSlices; ++u) {
-      const int s2 = u < slices ? u : slices - 1;
-      lo[u] = *reinterpret_cast<const f32x4_t *>(pr + s2 * slice_floats + i);
-      hi[u] = *reinterpret_cast<const f32x4_t *>(pr + s2 * slice_floats + i + 4);
-    }
+  const float *pr = SRC == kSums ? psum + row * dim : nullptr;
+  auto sum_slices = [&](const f32x4_t (&lo)[kMaxSlices], const f32x4_t (&hi)[kMaxSlices], u32x4_t cs, int i) {
     f32x4_t a = lo[0], b = hi[0];
 #pragma unroll
     for (int u = 1; u < kMaxSlices; ++u)
@@ -398,12 +395,11 @@ __global__ __launch_bounds__(BLOCK) void rmsnorm_kernel(const uint16_t *__restri
         a += lo[u];
         b += hi[u];
       }
-    for (int s2 = kMaxSlices; s2 < slices; ++s2) {
+    for (int s2 = kMaxSlices; s2 < slices && i < dim; ++s2) {
       a += *reinterpret_cast<const f32x4_t *>(pr + s2 * slice_floats + i);
       b += *reinterpret_cast<const f32x4_t *>(pr + s2 * slice_floats + i + 4);
     }
     if (col_scales) {
-      const u32x4_t cs = *reinterpret_cast<const u32x4_t *>(col_scales + i);
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         a[2 * j] = bf16_round(a[2 * j]) * __builtin_bit_cast(float, cs[j] << 16);
@@ -419,7 +415,7 @@ __global__ __launch_bounds__(BLOCK) void rmsnorm_kernel(const uint16_t *__restri
     d[3] = static_cast<uint32_t>(f32_to_bf16_rne(b[2])) | (static_cast<uint32_t>(f32_to_bf16_rne(b[3])) << 16);
     return d;
   };
-  const bool adds = delta || psum;
+  constexpr bool adds = SRC != kNothing;
   auto add_round = [](u32x4_t a, u32x4_t d) {  // bf16(x + delta), value by value
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -452,16 +448,28 @@ __global__ __launch_bounds__(BLOCK) void rmsnorm_kernel(const uint16_t *__restri
     if (staged.frag) staged_store_piece(staged, static_cast<int>(row), i >> 3, o);
   };
 
-  u32x4_t keep[kPieces], keepd[kPieces], keepw[kPieces];
+  u32x4_t keep[kPieces], keepd[kPieces], keepw[kPieces], keepc[kPieces];
+  f32x4_t lo[kPieces][kMaxSlices], hi[kPieces][kMaxSlices];
 #pragma unroll
   for (int p = 0; p < kPieces; ++p) {
-    const int i = threadIdx.x * 8 + p * kStride;
-    if (i < dim) {
-      keep[p] = *reinterpret_cast<const u32x4_t *>(xr + i);
-      if (delta) keepd[p] = *reinterpret_cast<const u32x4_t *>(dr_row + i);
-      else if (psum) keepd[p] = sum_slices(i);
-      keepw[p] = *reinterpret_cast<const u32x4_t *>(w + i);  // needed only after the reduction
+    const int i = threadIdx.x * 8 + p * kStride, at = i < dim ? i : 0;  // past the row: its first piece, not used
+    keep[p] = *reinterpret_cast<const u32x4_t *>(xr + at);
+    if (SRC == kDelta) keepd[p] = *reinterpret_cast<const u32x4_t *>(dr_row + at);
+    if (SRC == kSums) {
+#pragma unroll
+      for (int u = 0; u < kMaxSlices; ++u)
+        if (u < slices) {
+          lo[p][u] = *reinterpret_cast<const f32x4_t *>(pr + u * slice_floats + at);
+          hi[p][u] = *reinterpret_cast<const f32x4_t *>(pr + u * slice_floats + at + 4);
+        }
+      if (col_scales) keepc[p] = *reinterpret_cast<const u32x4_t *>(col_scales + at);
     }
+    keepw[p] = *reinterpret_cast<const u32x4_t *>(w + at);  // needed only after the reduction
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (SRC == kSums) {
+#pragma unroll
+    for (int p = 0; p < kPieces; ++p) keepd[p] = sum_slices(lo[p], hi[p], keepc[p], threadIdx.x * 8 + p * kStride);
   }
   float ss = 0.f;
 #pragma unroll
@@ -478,7 +486,20 @@ __global__ __launch_bounds__(BLOCK) void rmsnorm_kernel(const uint16_t *__restri
   for (int i = threadIdx.x * 8 + kPieces * kStride; i < dim; i += kStride) {
     u32x4_t raw = *reinterpret_cast<const u32x4_t *>(xr + i);
     if (adds) {
-      raw = add_round(raw, delta ? *reinterpret_cast<const u32x4_t *>(dr_row + i) : sum_slices(i));
+      u32x4_t term;
+      if constexpr (SRC == kSums) {
+        f32x4_t l[kMaxSlices], h[kMaxSlices];
+#pragma unroll
+        for (int u = 0; u < kMaxSlices; ++u)
+          if (u < slices) {
+            l[u] = *reinterpret_cast<const f32x4_t *>(pr + u * slice_floats + i);
+            h[u] = *reinterpret_cast<const f32x4_t *>(pr + u * slice_floats + i + 4);
+          }
+        term = sum_slices(l, h, col_scales ? *reinterpret_cast<const u32x4_t *>(col_scales + i) : u32x4_t{}, i);
+      } else {
+        term = *reinterpret_cast<const u32x4_t *>(dr_row + i);
+      }
+      raw = add_round(raw, term);
       *reinterpret_cast<u32x4_t *>(h_out + row * dim + i) = raw;
     }
     ss = sum_sq(raw, ss);
@@ -571,15 +592,22 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t *__restric
   reinterpret_cast<u32x4_t *>(y)[idx] = o;
 }
 
-// few rows (decode): 512 threads so that a 4096-wide row is one piece per thread; many rows: 256-thread workgroups
+template <int BLOCK>
+void launch_rmsnorm_block(const uint16_t *x, const uint16_t *delta, const float *psum, int slices, const uint16_t *col_scales, const uint16_t *w,
+                          uint16_t *h_out, uint16_t *y, StagedOut staged, int64_t rows, int64_t dim, float eps, hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>(rows)), block(BLOCK);
+  const int width = static_cast<int>(dim);
+  if (delta) hipLaunchKernelGGL((rmsnorm_kernel<BLOCK, kDelta>), grid, block, 0, stream, x, delta, psum, slices, col_scales, w, h_out, y, staged, width, eps);
+  else if (psum) hipLaunchKernelGGL((rmsnorm_kernel<BLOCK, kSums>), grid, block, 0, stream, x, delta, psum, slices, col_scales, w, h_out, y, staged, width, eps);
+  else hipLaunchKernelGGL((rmsnorm_kernel<BLOCK, kNothing>), grid, block, 0, stream, x, delta, psum, slices, col_scales, w, h_out, y, staged, width, eps);
+}
+
+// few rows (decode): one piece per thread up to 8192 values; many rows: 256-thread workgroups
 void launch_rmsnorm(const uint16_t *x, const uint16_t *delta, const float *psum, int slices, const uint16_t *col_scales, const uint16_t *w,
                     uint16_t *h_out, uint16_t *y, StagedOut staged, int64_t rows, int64_t dim, float eps, hipStream_t stream) {
-  if (rows <= 512 && dim >= 4096)
-    hipLaunchKernelGGL(rmsnorm_kernel<512>, dim3(static_cast<unsigned>(rows)), dim3(512), 0, stream, x, delta, psum, slices, col_scales, w, h_out,
-                       y, staged, static_cast<int>(dim), eps);
-  else
-    hipLaunchKernelGGL(rmsnorm_kernel<256>, dim3(static_cast<unsigned>(rows)), dim3(256), 0, stream, x, delta, psum, slices, col_scales, w, h_out,
-                       y, staged, static_cast<int>(dim), eps);
+  if (rows <= 512 && dim > 4096) launch_rmsnorm_block<1024>(x, delta, psum, slices, col_scales, w, h_out, y, staged, rows, dim, eps, stream);
+  else if (rows <= 512 && dim >= 4096) launch_rmsnorm_block<512>(x, delta, psum, slices, col_scales, w, h_out, y, staged, rows, dim, eps, stream);
+  else launch_rmsnorm_block<256>(x, delta, psum, slices, col_scales, w, h_out, y, staged, rows, dim, eps, stream);
 }
 
 template <int D, int NW>

@@ -50,6 +50,27 @@ def test_add_rmsnorm_matches_stock_ops():
         assert (y == ref).float().mean() > 0.99
 
 
+@pytest.mark.parametrize("scaled", [False, True])
+@pytest.mark.parametrize("slices", [1, 2, 4, 5, 8])
+@pytest.mark.parametrize("rows,dim", [(1, 4096), (2, 4104), (33, 8192), (2, 8200), (1, 20480), (600, 4104), (5, 512)])
+def test_norm_of_slices_equals_the_norm_of_their_sum(rows, dim, slices, scaled):
+    """Rows of one piece per thread, of a piece beyond, of the re-read rest; slices within and beyond those requested at once; rows of both block sizes."""
+    gen = torch.Generator().manual_seed(rows + dim + slices)
+    x = torch.randn((rows, dim), generator=gen).to(torch.bfloat16).to(DEV)
+    w = (1 + 0.1 * torch.randn((dim,), generator=gen)).to(torch.bfloat16).to(DEV)
+    parts = torch.randn((slices, rows, dim), generator=gen).to(DEV)
+    scales = torch.rand((dim,), generator=gen).to(torch.bfloat16).to(DEV) if scaled else None
+    total = parts[0].clone()
+    for i in range(1, slices):
+        total += parts[i]
+    delta = total.to(torch.bfloat16)
+    if scaled:
+        delta = delta * scales
+    h, y = ops.add_rmsnorm(x, ops.ScaledPartials(parts, scales) if scaled else parts, w, 1e-5)
+    want_h, want_y = ops.add_rmsnorm(x, delta, w, 1e-5)
+    assert torch.equal(h, want_h) and torch.equal(h, x + delta) and torch.equal(y, want_y)
+
+
 def test_silu_mul_matches_stock_ops():
     a = randn_bf16((32, 11008), std=2.0, seed=1).to(DEV)
     b = randn_bf16((32, 11008), std=1.0, seed=2).to(DEV)
