@@ -8,9 +8,10 @@
 // G_t the decay from the chunk's start through token t,
 //   u_t + sum_{s<t} beta_t (G_t / G_s) (k_t . k_s) u_s = beta_t (v_t - G_t S0^T k_t)
 //   o_t = G_t S0^T q_t + sum_{s<=t} (G_t / G_s) (q_t . k_s) u_s,   S = G_end S0 + sum_s (G_end / G_s) k_s u_s^T
-// 1. delta_chunk_kernel, parallel over chunks: T = (I + M)^-1 diag(beta) for the strictly lower triangular M above (the four
-//    16 x 16 diagonal blocks by substitution, the others from products of blocks), and the masked, decayed products q k^T;
-// 2. delta_scan_kernel, one workgroup per (sequence, head, 16 value columns), chunk after chunk: read-outs, u = T (v - G S0^T k),
+// 1. delta_chunk_kernel, parallel over chunks, everything that needs no state: T = (I + M)^-1 diag(beta) for the strictly lower
+//    triangular M above (the four 16 x 16 diagonal blocks by substitution, the others from products of blocks), W = T diag(G) K
+//    and U0 = T V, so that u = U0 - W S0, and the masked, decayed products q k^T;
+// 2. delta_scan_kernel, one workgroup per (sequence, head, 16 value columns), chunk after chunk: u and q's read-out, then
 //    outputs and the next state;
 // 3. delta_gate_kernel: RMS norm over the head and the silu gate.
 #include "e2h_seq_common.h"
@@ -21,12 +22,25 @@ namespace {
 constexpr int kMaxDim = 256;
 constexpr float kUnitEps = 1e-6f;
 
+constexpr int kChunk = 64;  // tokens that the chunked form takes together
+
 struct Prepared {
-  float *q, *k;   // [rows, kv_heads, dim] unit vectors, q scaled
+  float *q, *k;   // unit vectors, q scaled: [rows, kv_heads, dim], or by fragments of matrix operands where tiles > 0 (see head_value)
   float *v;       // [rows, heads, vdim]
   float *beta;    // [rows, heads]
   float *log_g;   // [rows, heads] logarithm of the decay
+  int tiles, chunks;  // the chunked form: tiles of 16 channels that hold a head's keys, and chunks of a sequence
 };
+
+// Where channel d of token t's query or key stands.  By fragments: [sequence, chunk, head][block of 16 tokens][tile of 16 channels]
+// [four channels][token][channel], so that what a wave wants of a tile, lane (c, b4) the channels 4 b4 .. of token c, is one run
+// of 1 KB.  From rows of tokens every lane of a quarter wave meets another cache line, and such a load takes the L1 cache 64 clocks
+// instead of 16.
+__device__ __forceinline__ size_t head_value(const Prepared &o, int b, int t, size_t row, int head, int kvh, int D, int d) {
+  if (o.tiles == 0) return (row * kvh + head) * D + d;
+  const size_t block = ((static_cast<size_t>(b) * o.chunks + t / kChunk) * kvh + head) * (kChunk / 16) + t % kChunk / 16;
+  return ((block * o.tiles + d / 16) * 64 + d % 16 / 4 * 16 + t % 16) * 4 + d % 4;
+}
 
 // causal convolution of one channel ending at token t (position pos0 + t), then silu
 template <typename T>
@@ -87,11 +101,11 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(const e2h_delta_args
     scale = 1.0f / sqrtf(wave_add(ss) + kUnitEps);
     if (is_q) scale /= sqrtf(static_cast<float>(D));
   }
-  float *dst = is_q ? o.q + (row * kvh + head) * D : is_k ? o.k + (row * kvh + head) * D : o.v + (row * H + head) * DV;
+  const int padded = o.tiles > 0 ? o.tiles * 16 : n;  // zeros in the head's last tile
 #pragma unroll
   for (int i = 0; i < kMaxDim / 64; ++i) {
     const int d = i * 64 + lane;
-    if (d < n) dst[d] = x[i] * scale;
+    if (d < (is_q || is_k ? padded : n)) *(is_q || is_k ? (is_q ? o.q : o.k) + head_value(o, b, t, row, head, kvh, D, d) : o.v + (row * H + head) * DV + d) = x[i] * scale;
   }
   // the last taps - 1 convolution inputs of the call; those from before it (a call shorter than the convolution) are carried over
   if (a.taps > 1 && t >= seqlen - (a.taps - 1)) {
@@ -111,6 +125,8 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(const e2h_delta_args
 // The same for convolutions of up to four taps with everything in multiples of four channels: `cp` lanes (a power of two) hold
 // one head's channels, four each, and walk kPrepareRun tokens with the previous inputs in registers.
 constexpr int kPrepareRun = 8;
+constexpr int kRunPitch = kPrepareRun * 4 + 4;
+static_assert(kPrepareRun == 8, "a run of tokens is half a block of 16");
 
 template <typename T>
 __global__ __launch_bounds__(256) void delta_prepare4_kernel(const e2h_delta_args a, Prepared o, int cp, int runs) {
@@ -133,6 +149,11 @@ __global__ __launch_bounds__(256) void delta_prepare4_kernel(const e2h_delta_arg
   const size_t row0 = static_cast<size_t>(b) * seqlen;
   const T *src = static_cast<const T *>(a.proj) + row0 * a.ld + col;
   const T *tail = static_cast<const T *>(a.tail_in) + static_cast<size_t>(b) * taps * channels + ch;
+  __shared__ __attribute__((aligned(16))) float turned[4 * 64 * kRunPitch];
+  float *const mem = turned + (threadIdx.x >> 6) * 64 * kRunPitch;
+  // where the run's first token goes if it goes by fragments, or 0; a head's last tile is filled with zeros
+  const bool by_fragments = o.tiles > 0 && (is_q || is_k) && d < o.tiles * 16;
+  const auto place = by_fragments ? reinterpret_cast<unsigned long long>((is_q ? o.q : o.k) + head_value(o, b, t_begin, 0, head, kvh, D, d)) : 0ull;
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
   f32x4_t w[4];  // shallower convolutions: zero weights in front
 #pragma unroll
@@ -175,7 +196,20 @@ __global__ __launch_bounds__(256) void delta_prepare4_kernel(const e2h_delta_arg
     for (int off = 1; off < cp; off <<= 1) ss += __shfl_xor(ss, off);
     if (is_q || is_k) y *= is_q ? 1.0f / (sqrtf(ss + kUnitEps) * sqrtf(static_cast<float>(D))) : 1.0f / sqrtf(ss + kUnitEps);
     const size_t row = row0 + t;
-    if (mine) store4(is_q ? o.q + (row * kvh + head) * D + d : is_k ? o.k + (row * kvh + head) * D + d : o.v + (row * H + head) * DV + d, y);
+    if (place) store4(mem + lane * kRunPitch + i * 4, y);
+    else if (mine) store4(is_q || is_k ? (is_q ? o.q : o.k) + (row * kvh + head) * D + d : o.v + (row * H + head) * DV + d, y);
+  }
+  // a run is half a block's tokens, 128 bytes of each four channels in a row: eight lanes take one of them (by a lane's 16 bytes at a
+  // time this kernel took 209 us for 8192 tokens of 64 heads of 128, so 142)
+  if (o.tiles > 0) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int from = i * 8 + lane / 8, t = lane % 8;
+      float *const to = reinterpret_cast<float *>(__shfl(place, from));
+      if (to && t_begin + t < t_end) store4(to + t * 4, load4(mem + from * kRunPitch + t * 4));
+    }
   }
   if (taps > 1 && t_end == seqlen && mine) {  // the last taps - 1 inputs, some of them carried over when the call is that short
     T *dst = static_cast<T *>(a.tail_out) + static_cast<size_t>(b) * taps * channels + ch;
@@ -372,135 +406,218 @@ __global__ __launch_bounds__(BLOCK) void delta_tokens_kernel(const e2h_delta_arg
 }
 
 // ---- chunked form ----------------------------------------------------------------------------------------------------------
-constexpr int kChunk = 64;
-
 struct ChunkScratch {
-  float *t;  // [batch * heads, chunks, 64, 64]
-  float *p;  // [batch * heads, chunks, 64, 64]
-  int chunks;
+  float *w;     // [batch * heads, chunks] by fragments as the keys
+  float *p;     // [batch * heads, chunks] by fragments, four tiles
+  float *g, *e; // [batch * heads, chunks, 64] decay from the chunk's start through the token, and from the token to the chunk's end
 };
 
-// four consecutive values of a row at column d; zero beyond the row's n values (n % 4 == 0) or when the row does not exist
-__device__ __forceinline__ f32x4_t row4(const float *base, bool exists, int d, int n) {
-  return exists && d < n ? load4(base + d) : f32x4_t{0.f, 0.f, 0.f, 0.f};
-}
-
-// step 1: 4 waves, one (sequence, head, chunk) each; wave w owns the token rows 16 w .. 16 w + 15
-__global__ __launch_bounds__(256) void delta_chunk_kernel(const e2h_delta_args a, Prepared p, ChunkScratch cs) {
-  constexpr int kRow = kChunk + 4;
-  __shared__ __attribute__((aligned(16))) float sm[kChunk * kRow];  // M, then its blocks are replaced by the inverse's
-  __shared__ __attribute__((aligned(16))) float si[kChunk * kRow];  // inverse
-  __shared__ float sg[kChunk], sb[kChunk];
-  const int D = static_cast<int>(a.dim), H = static_cast<int>(a.heads), kvh = static_cast<int>(a.kv_heads), seqlen = static_cast<int>(a.seqlen);
-  const int chunk = blockIdx.x % cs.chunks, bh = blockIdx.x / cs.chunks;
+// step 1: 4 waves, one (sequence, head, chunk) each; wave w owns the token rows 16 w .. 16 w + 15.  TILES: tiles of 16 that hold a
+// head's keys and its values.  U0 takes the place of the values.  Products are formed turned, a lane its token's row of four keys:
+// that is both the layout of the left operand that M's blocks become and 16 bytes of a fragment.
+// What bounds it: 76 us of float32 matrix work and 560 MB at 8192 tokens of 32 heads of 128, with phases that wait for one another;
+// 52 KB of LDS and 112 registers let three workgroups of a CU overlap theirs.  290 us with M in LDS and two workgroups, 190 so; the
+// two products that it took over from the scan cost it 50.
+template <int TILES>
+__global__ __launch_bounds__(256, TILES <= 8 ? 3 : 1) void delta_chunk_kernel(const e2h_delta_args a, Prepared p, ChunkScratch cs) {
+  constexpr int kRow = kChunk + 4, kWide = TILES * 16 + 4, kQuads = TILES * 4, kEvery = 256 / kQuads;
+  __shared__ __attribute__((aligned(16))) float sw[kChunk * kWide];  // keys, then values
+  __shared__ __attribute__((aligned(16))) float si[kChunk * kRow];  // inverse; M's diagonal blocks stand in blocks above its diagonal
+  __shared__ __attribute__((aligned(16))) float sg[kChunk], sb[kChunk];
+  const int D = static_cast<int>(a.dim), DV = static_cast<int>(a.vdim), H = static_cast<int>(a.heads), kvh = static_cast<int>(a.kv_heads), seqlen = static_cast<int>(a.seqlen);
+  const int chunk = blockIdx.x % p.chunks, bh = blockIdx.x / p.chunks;
   const int b = bh / H, h = bh % H, hk = h / (H / kvh);
-  const int wave = threadIdx.x >> 6, c = threadIdx.x & 15, b4 = (threadIdx.x & 63) >> 4;
+  // the last rows take four times the first ones' products: neighbours on a CU hand them to different SIMDs (205 to 201 us)
+  const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) + blockIdx.x / 8 + blockIdx.x / 256) & 3;
+  const int lane = threadIdx.x & 63, c = lane & 15, b4 = lane >> 4;
   const size_t row0 = static_cast<size_t>(b) * seqlen + static_cast<size_t>(chunk) * kChunk;
   const int live = seqlen - chunk * kChunk < kChunk ? seqlen - chunk * kChunk : kChunk;  // tokens past the end: beta 0, decay 1, q = k = 0
+  const f32x4_t none = {0.f, 0.f, 0.f, 0.f};
+  // tokens past the sequence's end are read from its last one or as whatever the memory holds, and masked when they are used: no
+  // load waits in a branch
+  const size_t gate_row = (row0 + (lane < live ? lane : live - 1)) * H + h;
+  const float log_g = p.log_g[gate_row], beta = p.beta[gate_row];
+  f32x4_t mine[TILES], query[TILES];  // this wave's rows of keys and queries
+  const size_t head = (((static_cast<size_t>(b) * p.chunks + chunk) * kvh + hk) * (kChunk / 16) + wave) * p.tiles * 256 + lane * 4;
+  const int tr = 16 * wave + c;
+#pragma unroll
+  for (int dt = 0; dt < TILES; ++dt) {
+    const int there = dt < p.tiles ? dt : p.tiles - 1;
+    mine[dt] = load4(p.k + head + there * 256);
+    query[dt] = load4(p.q + head + there * 256);
+  }
   if (threadIdx.x < 64) {
     const int t = threadIdx.x;
-    float g = t < live ? p.log_g[(row0 + t) * H + h] : 0.f;
+    float g = t < live ? log_g : 0.f;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
       const float up = __shfl_up(g, off);
       if (t >= off) g += up;
     }
     sg[t] = g * kLog2e;
-    sb[t] = t < live ? p.beta[(row0 + t) * H + h] : 0.f;
+    sb[t] = t < live ? beta : 0.f;
   }
-  for (int i = threadIdx.x; i < kChunk * kRow; i += 256) si[i] = 0.f;
-  // k k^T and q k^T for the column blocks up to this wave's
-  f32x4_t kk[4], qk[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) kk[j] = qk[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const size_t stride = static_cast<size_t>(kvh) * D;
-  const float *kb = p.k + (row0 * kvh + hk) * D, *qb = p.q + (row0 * kvh + hk) * D;
-  const int tr = 16 * wave + c;
-  for (int d = 4 * b4; d < (D + 15) / 16 * 16; d += 16) {
-    const f32x4_t ka = row4(kb + tr * stride, tr < live, d, D), qa = row4(qb + tr * stride, tr < live, d, D);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (j > wave) break;
-      const f32x4_t kc = j == wave ? ka : row4(kb + (16 * j + c) * stride, 16 * j + c < live, d, D);
-      kk[j] = mfma4(ka, kc, kk[j]);
-      qk[j] = mfma4(qa, kc, qk[j]);
-    }
+  for (int dt = 0; dt < TILES; ++dt) {
+    const bool there = tr < live && dt < p.tiles;
+    mine[dt] = there ? mine[dt] : none;
+    query[dt] = there ? query[dt] : none;
+    store4(sw + tr * kWide + dt * 16 + 4 * b4, mine[dt]);
   }
-  __syncthreads();
-  float *pt = cs.p + (static_cast<size_t>(bh) * cs.chunks + chunk) * kChunk * kChunk;
+  lds_barrier();
+  // M's blocks left of the diagonal, and q k^T for the blocks up to it
+  f32x4_t m[4];
+  float *pt = cs.p + (static_cast<size_t>(bh) * p.chunks + chunk) * kChunk * kChunk + wave * 1024 + lane * 4;
+  const float g_mine = sg[tr], b_mine = sb[tr];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    if (j > wave) break;
+    m[j] = none;
+    if (j > wave) continue;
+    f32x4_t kk = none, kq = none;
+#pragma unroll
+    for (int dt = 0; dt < TILES; ++dt) {
+      const f32x4_t kc = load4(sw + (16 * j + c) * kWide + dt * 16 + 4 * b4);
+      kk = mfma4(kc, mine[dt], kk);
+      kq = mfma4(kc, query[dt], kq);
+    }
+    const f32x4_t g = load4(sg + 16 * j + 4 * b4);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int t = 16 * wave + 4 * b4 + r, s = 16 * j + c;
-      const float dec = s <= t ? __builtin_amdgcn_exp2f(sg[t] - sg[s]) : 0.f;
-      sm[t * kRow + s] = s < t ? sb[t] * dec * kk[j][r] : 0.f;
-      pt[t * kChunk + s] = dec * qk[j][r];
+      const int key = 16 * j + 4 * b4 + r;
+      const float dec = __builtin_amdgcn_exp2f(key <= tr ? g_mine - g[r] : -INFINITY);
+      m[j][r] = key < tr ? b_mine * dec * kk[r] : 0.f;
+      kq[r] *= dec;
     }
+    store4(pt + j * 256, kq);
   }
-  __syncthreads();
   // inverse of the unit lower triangular diagonal blocks: wave w, lane c = column c of block w, substitution down the rows
+  float *const diagonal = si + (wave < 3 ? 16 * wave * kRow + 16 * (wave + 1) : 32);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (j == wave) store4(diagonal + c * kRow + 4 * b4, m[j]);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
   if (b4 == 0) {
+    f32x4_t row[2][4];  // of this step and the next
     float x[16];
-    const float *m = sm + (16 * wave) * kRow + 16 * wave;
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if (t < 15 && 4 * s <= t) row[(t + 1) & 1][s] = load4(diagonal + (t + 1) * kRow + 4 * s);
       float v = t == c ? 1.f : 0.f;
 #pragma unroll
       for (int s = 0; s < 16; ++s)
-        if (s < t) v = __builtin_fmaf(-m[t * kRow + s], x[s], v);
+        if (s < t) v = __builtin_fmaf(-row[t & 1][s / 4][s % 4], x[s], v);
       x[t] = v;
       si[(16 * wave + t) * kRow + 16 * wave + c] = v;
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
-  __syncthreads();
+  lds_barrier();
+  // the values in whole rows, a thread four columns of every kEvery-th token, are wanted behind the products of the keys
+  const int vt = threadIdx.x / kQuads, vd = threadIdx.x % kQuads * 4;
+  f32x4_t val[kChunk / kEvery];
+#pragma unroll
+  for (int i = 0; i < kChunk / kEvery; ++i) {
+    const int t = vt + i * kEvery;
+    val[i] = load4(p.v + ((row0 + (t < live ? t : live - 1)) * H + h) * DV + (vd < DV ? vd : 0));
+  }
   // blocks off the diagonal, by distance: I_ij = -I_ii sum_{j <= l < i} M_il I_lj
 #pragma unroll
   for (int dist = 1; dist < 4; ++dist) {
     const int i = wave, j = wave - dist;
-    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    f32x4_t acc = none;
     if (j >= 0) {
-      for (int l = j; l < i; ++l) {
+#pragma unroll
+      for (int l = 0; l < 3; ++l) {
+        if (l < j || l >= i) continue;
         f32x4_t bb;
 #pragma unroll
         for (int r = 0; r < 4; ++r) bb[r] = si[(16 * l + 4 * b4 + r) * kRow + 16 * j + c];
-        acc = mfma4(load4(sm + (16 * i + c) * kRow + 16 * l + 4 * b4), bb, acc);
+        acc = mfma4(m[l], bb, acc);
       }
-      const f32x4_t res = mfma4(load4(si + (16 * i + c) * kRow + 16 * i + 4 * b4), acc, f32x4_t{0.f, 0.f, 0.f, 0.f});
+      const f32x4_t res = mfma4(load4(si + (16 * i + c) * kRow + 16 * i + 4 * b4), acc, none);
 #pragma unroll
       for (int r = 0; r < 4; ++r) si[(16 * i + 4 * b4 + r) * kRow + 16 * j + c] = -res[r];
     }
-    __syncthreads();
+    lds_barrier();
   }
-  float *tt = cs.t + (static_cast<size_t>(bh) * cs.chunks + chunk) * kChunk * kChunk;
-  for (int i = threadIdx.x; i < kChunk * kChunk; i += 256) {
-    const int s = i & 63;
-    tt[i] = si[(i >> 6) * kRow + s] * sb[s];
+  const size_t at = static_cast<size_t>(bh) * p.chunks + chunk;
+  if (threadIdx.x < kChunk) {
+    cs.g[at * kChunk + threadIdx.x] = __builtin_amdgcn_exp2f(sg[threadIdx.x]);
+    cs.e[at * kChunk + threadIdx.x] = __builtin_amdgcn_exp2f(sg[kChunk - 1] - sg[threadIdx.x]);
+  }
+  // rows 16 w .. of (I + M)^-1 diag(coefficient), which multiply the rows in sw, two tiles of columns at a time
+  f32x4_t inv[4], by[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    inv[j] = by[j] = none;
+    if (j > wave) continue;
+    const f32x4_t g = load4(sg + 16 * j + 4 * b4);
+    by[j] = load4(si + tr * kRow + 16 * j + 4 * b4) * load4(sb + 16 * j + 4 * b4);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) inv[j][r] = by[j][r] * __builtin_amdgcn_exp2f(g[r]);
+  }
+  const auto column = [&](int j, int tile) {
+    f32x4_t x;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[r] = sw[(16 * j + 4 * b4 + r) * kWide + tile * 16 + c];
+    return x;
+  };
+  float *wt = cs.w + at * kChunk * 16 * p.tiles + wave * p.tiles * 256 + lane * 4;
+  for (int tile = 0; tile < p.tiles; tile += 2) {
+    f32x4_t w0 = none, w1 = none;  // turned
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j <= wave) {
+        w0 = mfma4(column(j, tile), inv[j], w0);
+        w1 = mfma4(column(j, tile + 1), inv[j], w1);
+      }
+    store4(wt + tile * 256, w0);
+    if (tile + 1 < p.tiles) store4(wt + tile * 256 + 256, w1);
+  }
+  lds_barrier();  // the keys have been read
+#pragma unroll
+  for (int i = 0; i < kChunk / kEvery; ++i) store4(sw + (vt + i * kEvery) * kWide + vd, vt + i * kEvery < live && vd < DV ? val[i] : none);
+  lds_barrier();
+  float *const u_at = p.v + ((row0 + 16 * wave + 4 * b4) * H + h) * DV + c;
+  const size_t u_stride = static_cast<size_t>(H) * DV;
+  for (int tile = 0; tile * 16 < DV; tile += 2) {
+    f32x4_t u0 = none, u1 = none;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j <= wave) {
+        u0 = mfma4(by[j], column(j, tile), u0);
+        u1 = mfma4(by[j], column(j, tile + 1), u1);
+      }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (16 * wave + 4 * b4 + r >= live) continue;
+      if (tile * 16 + c < DV) u_at[r * u_stride + tile * 16] = u0[r];
+      if (tile * 16 + 16 + c < DV) u_at[r * u_stride + tile * 16 + 16] = u1[r];
+    }
   }
 }
 
-// What one wave of the scan reads of a chunk: its 16 token rows of k, T and v, or of q and the decayed q k^T.  None of it
-// depends on the state, so it is fetched a chunk ahead.
-template <int DT>
-struct ChunkRows {
-  f32x4_t rows[DT], square[4], v;
-  float log_g;
-};
-
 // step 2: DT = head dimension in tiles of 16.  Eight waves: wave w < 4 owns the token rows 16 w .. 16 w + 15 on the writing side
-// (k, T, v: what u is made of), wave w + 4 the same rows on the reading side (q and the outputs); the state's row tiles w, w + 8
+// (u = U0 - W S0), wave w + 4 the same rows on the reading side (q and the outputs); the state's row tiles w, w + 8
 // are wave w's.  The state is kept twice: in accumulators by its owner, and in LDS, transposed, as the B operand of
-// everybody's read-outs.  The keys go through LDS once to be read transposed in the state update.
-// WHOLE: the head dimension fills its tiles, so no load needs a mask (rows past the end are read from the last token: their beta is
-// 0, which keeps them out of u, and their outputs are not stored).
+// everybody's read-outs.  The keys, decayed to the chunk's end, go through LDS once to be read transposed in the state update.
+// What bounds it: one workgroup per CU of dependent chunks (32 heads of 128 values, one sequence), each two matrix phases in
+// float32 with a barrier behind either, 2048 and up to 1536 matrix clocks a SIMD of the 6600 that a chunk takes, and 112 KB that
+// pass the L1 cache at 64 bytes a clock (1800).  All of it comes by fragments, 1 KB to a load: from rows of tokens a chunk took
+// 1.0 us more, and 1.2 us more with the loads in one block ahead of the products instead of between them.  With T applied here
+// (u = T (v - G S0^T k), a phase and a barrier more), decays formed by every lane, sums by single LDS words and rows of
+// tokens, 8192 tokens took 709 us; now 400.
+// WHOLE: the head dimension fills its tiles, so that every tile's place is a constant from the first one's.
 template <int DT, bool WHOLE>
 __global__ __launch_bounds__(512) void delta_scan_kernel(const e2h_delta_args a, Prepared p, ChunkScratch cs, int v_blocks) {
-  constexpr int DP = DT * 16, OWN = (DT + 7) / 8, kRow = DP + 4, kTok = 20;
-  __shared__ __attribute__((aligned(16))) float st[16 * kRow];                         // state, [value column][row]
-  __shared__ __attribute__((aligned(16))) float sk[kChunk * kRow];                     // keys, [token][channel]
-  __shared__ __attribute__((aligned(16))) float sx[kChunk * kTok], su[kChunk * kTok];  // [token][value column]
-  __shared__ float sg[2][kChunk];
+  constexpr int DP = DT * 16, OWN = (DT + 7) / 8, kRow = DP + 4, kTok = kChunk + 4;
+  constexpr bool kTwo = DT <= 8;  // the next chunk's rows are requested between this one's products; two sets of more do not fit the registers
+  __shared__ __attribute__((aligned(16))) float st[16 * kRow];       // state, [value column][row]
+  __shared__ __attribute__((aligned(16))) float sk[kChunk * kRow];   // keys, [token][channel]
+  __shared__ __attribute__((aligned(16))) float su[16 * kTok];       // u, [value column][token]
   const int D = static_cast<int>(a.dim), DV = static_cast<int>(a.vdim), H = static_cast<int>(a.heads), kvh = static_cast<int>(a.kv_heads);
   const int seqlen = static_cast<int>(a.seqlen), bh_count = static_cast<int>(a.batch) * H;
   // the value blocks of one head read the same keys and queries: keep them on one die (workgroups go round robin over 8)
@@ -534,111 +651,126 @@ __global__ __launch_bounds__(512) void delta_scan_kernel(const e2h_delta_args a,
     }
     if (dt < DT) store4(st + c * kRow + dt * 16 + 4 * b4, s[i]);
   }
-  const size_t stride = static_cast<size_t>(kvh) * D;
-  const int tr = 16 * block + c;
-  const size_t seq0 = static_cast<size_t>(b) * seqlen;
-  const float *squares = (reader ? cs.p : cs.t) + static_cast<size_t>(bh) * cs.chunks * kChunk * kChunk;
-  const float *vectors = reader ? p.q : p.k;
+  const int tr = 16 * block + c, half = reader ? DT / 2 : 0;  // first tile of the keys that this wave brings
+  const size_t seq0 = static_cast<size_t>(b) * seqlen, first_chunk = static_cast<size_t>(bh) * p.chunks;
 
-  auto fetch = [&](int chunk, ChunkRows<DT> &x) {
-    const size_t row0 = seq0 + static_cast<size_t>(chunk) * kChunk;
-    const int live = seqlen - chunk * kChunk < kChunk ? seqlen - chunk * kChunk : kChunk;
-    const float *mine = vectors + ((row0 + (tr < live ? tr : live - 1)) * kvh + hk) * D;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) x.rows[dt] = WHOLE ? load4(mine + dt * 16 + 4 * b4) : row4(mine, true, dt * 16 + 4 * b4, D);
-    const float *sq = squares + static_cast<size_t>(chunk) * kChunk * kChunk + tr * kChunk + 4 * b4;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (j <= block) x.square[j] = load4(sq + 16 * j);
-    if (!reader) {
+  // a chunk's place is uniform, a lane's part of it one offset of 32 bits
+  const uint32_t v_stride = static_cast<uint32_t>(H) * static_cast<uint32_t>(DV), lane4 = static_cast<uint32_t>(threadIdx.x & 63) * 4;
+  const uint32_t my_rows = static_cast<uint32_t>(block * p.tiles) * 256 + lane4, my_square = static_cast<uint32_t>(block) * 1024 + lane4;
+  const uint32_t my_v = static_cast<uint32_t>(16 * block + 4 * b4) * v_stride, my_col = col_ok ? col : 0;
+  const size_t head_size = static_cast<size_t>(kChunk) * 16 * p.tiles;
+  const auto head_at = [&](int chunk) { return ((static_cast<size_t>(b) * p.chunks + chunk) * kvh + hk) * head_size; };
+  // a tile of this wave's 16 tokens; rows past the sequence's end are whatever the memory holds, tiles past the head's last one that one again: they
+  // meet the state's zeros, since keys are put away as zeros there.  Nothing is masked on arrival: that would wait for each load in turn.
+  const f32x4_t none = {0.f, 0.f, 0.f, 0.f};
+  const auto tile = [&](const float *from, int dt) { return load4(from + (my_rows + (WHOLE || dt < p.tiles ? dt : p.tiles - 1) * 256)); };
+  // rows of W or of q; of dead tokens: u that is set to zero, and outputs that are not stored
+  const auto rows_of = [&](int chunk) { return reader ? p.q + head_at(chunk) : cs.w + (first_chunk + chunk) * head_size; };
+  f32x4_t key[DT / 2], square[4], v = none, g = none;  // v: writers, square and g: readers
+  float e, decay;
+  const auto bring_keys = [&](int chunk) {
+    const size_t at = first_chunk + chunk;
+    const float *const keys = p.k + head_at(chunk);
+    e = cs.e[at * kChunk + tr];
+    decay = cs.g[at * kChunk + kChunk - 1];
+    if (reader) {
+      g = load4(cs.g + at * kChunk + (16 * block + 4 * b4));
+    } else {
+      const float *const values = p.v + ((seq0 + static_cast<size_t>(chunk) * kChunk) * H + h) * DV;
+      const uint32_t last = static_cast<uint32_t>(seqlen - chunk * kChunk < kChunk ? seqlen - chunk * kChunk : kChunk) - 1;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int t = 16 * block + 4 * b4 + r;
-        x.v[r] = p.v[((row0 + (t < live ? t : live - 1)) * H + h) * DV + (col_ok ? col : 0)];
+        const uint32_t t = my_v + r * v_stride;
+        v[r] = values[(t < last * v_stride ? t : last * v_stride) + my_col];
       }
     }
-    if (wave == 0) x.log_g = p.log_g[(row0 + (static_cast<int>(threadIdx.x) < live ? threadIdx.x : live - 1)) * H + h];
+#pragma unroll
+    for (int i = 0; i < DT / 2; ++i) key[i] = tile(keys, half + i);
+  };
+  const auto bring_square = [&](int chunk) {
+    const float *const from = cs.p + (first_chunk + chunk) * kChunk * kChunk;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) square[j] = load4(from + (my_square + 256 * j));
   };
 
-  ChunkRows<DT> cur, next;
-  fetch(0, cur);
-  for (int chunk = 0; chunk < cs.chunks; ++chunk) {
+  const auto step = [&](int chunk, f32x4_t (&cur)[DT], f32x4_t (&next)[DT]) {
     const int live = seqlen - chunk * kChunk < kChunk ? seqlen - chunk * kChunk : kChunk;
-    float *g = sg[chunk & 1];
-    if (wave == 0) {
-      float x = static_cast<int>(threadIdx.x) < live ? cur.log_g : 0.f;
+    const int after = chunk + 1 < p.chunks ? chunk + 1 : chunk;
+    const float *const next_rows = rows_of(after);
+    f32x4_t y = none;  // W S0 or S0^T q
+    f32x4_t sf[DT];
+    sf[0] = load4(st + c * kRow + 4 * b4);
+    sf[1] = load4(st + c * kRow + 16 + 4 * b4);
 #pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const float up = __shfl_up(x, off);
-        if (static_cast<int>(threadIdx.x) >= off) x += up;
-      }
-      g[threadIdx.x] = x * kLog2e;
+    for (int dt = 0; dt < DT; ++dt) {
+      if (kTwo) next[dt] = tile(next_rows, dt);
+      if (dt + 2 < DT) sf[dt + 2] = load4(st + c * kRow + (dt + 2) * 16 + 4 * b4);
+      y = mfma4(cur[dt], sf[dt], y);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    if (!reader) {
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) store4(sk + tr * kRow + dt * 16 + 4 * b4, cur.rows[dt]);
-    }
-    if (chunk + 1 < cs.chunks) fetch(chunk + 1, next);
-    lds_barrier();  // state, keys and decays of this chunk are in LDS; the loads above stay in flight
-    f32x4_t y = {0.f, 0.f, 0.f, 0.f}, gt;  // S0^T k or S0^T q, decayed to each token
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) y = mfma4(cur.rows[dt], load4(st + c * kRow + dt * 16 + 4 * b4), y);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      gt[r] = __builtin_amdgcn_exp2f(g[16 * block + 4 * b4 + r]);
-      y[r] *= gt[r];
-      if (!reader) sx[(16 * block + 4 * b4 + r) * kTok + c] = cur.v[r] - y[r];
-    }
-    lds_barrier();
-    if (!reader) {
-      f32x4_t u = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (j > block) break;
-        f32x4_t x;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) x[r] = sx[(16 * j + 4 * b4 + r) * kTok + c];
-        u = mfma4(cur.square[j], x, u);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) su[(16 * block + 4 * b4 + r) * kTok + c] = u[r];
-    }
-    lds_barrier();
-    f32x4_t ub[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) ub[j][r] = su[(16 * j + 4 * b4 + r) * kTok + c];
-      if (reader && j <= block) y = mfma4(cur.square[j], ub[j], y);
-    }
+    const float into = decay;
     if (reader) {
+      y *= g;
+    } else {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {  // over the values this workgroup has read
-        const int t = 16 * block + 4 * b4 + r;
-        if (t < live && col_ok) p.v[((seq0 + static_cast<size_t>(chunk) * kChunk + t) * H + h) * DV + col] = y[r];
-      }
+      for (int r = 0; r < 4; ++r) y[r] = 16 * block + 4 * b4 + r < live ? v[r] - y[r] : 0.f;
+      store4(su + c * kTok + 16 * block + 4 * b4, y);
     }
-    const float g_end = g[kChunk - 1], dec = __builtin_amdgcn_exp2f(g_end);
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int i = 0; i < DT / 2; ++i) store4(sk + tr * kRow + (half + i) * 16 + 4 * b4, tr < live && (WHOLE || half + i < p.tiles) ? key[i] * e : none);
+    lds_barrier();  // u and the keys are in LDS, the state has been read; the loads above stay in flight
+    bring_keys(after);
+    if (!kTwo) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) ub[j][r] *= __builtin_amdgcn_exp2f(g_end - g[16 * j + 4 * b4 + r]);
+      for (int dt = 0; dt < DT; ++dt) next[dt] = tile(next_rows, dt);
+    }
+    f32x4_t u[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) u[j] = load4(su + c * kTok + 16 * j + 4 * b4);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < OWN; ++i) {
       if (wave + 8 * i >= DT) break;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) s[i][r] *= dec;
+      s[i] *= into;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         f32x4_t kt;
 #pragma unroll
         for (int r = 0; r < 4; ++r) kt[r] = sk[(16 * j + 4 * b4 + r) * kRow + (wave + 8 * i) * 16 + c];
-        s[i] = mfma4(kt, ub[j], s[i]);
+        s[i] = mfma4(kt, u[j], s[i]);
       }
       store4(st + c * kRow + (wave + 8 * i) * 16 + 4 * b4, s[i]);
     }
-    lds_barrier();  // the keys have been read; the next chunk's take their place
-    cur = next;
+    if (reader) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (j <= block) y = mfma4(square[j], u[j], y);
+      bring_square(after);
+      float *const out = p.v + ((seq0 + static_cast<size_t>(chunk) * kChunk) * H + h) * DV;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)  // over the values this workgroup has read
+        if (16 * block + 4 * b4 + r < live && col_ok) out[my_v + r * v_stride + my_col] = y[r];
+    }
+    lds_barrier();  // the next state is in LDS, and the keys and u have been read
+  };
+  f32x4_t even[DT], odd[kTwo ? DT : 1];
+  {
+    const float *const rows = rows_of(0);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) even[dt] = tile(rows, dt);
+  }
+  bring_keys(0);
+  if (reader) bring_square(0);
+  lds_barrier();
+  if constexpr (kTwo) {
+#pragma unroll 1
+    for (int chunk = 0; chunk < p.chunks; chunk += 2) {
+      step(chunk, even, odd);
+      if (chunk + 1 < p.chunks) step(chunk + 1, odd, even);
+    }
+  } else {
+#pragma unroll 1
+    for (int chunk = 0; chunk < p.chunks; ++chunk) step(chunk, even, even);
   }
 #pragma unroll
   for (int i = 0; i < OWN; ++i)
@@ -696,8 +828,11 @@ void launch_scan(const e2h_delta_args &a, const Prepared &p, const ChunkScratch 
 
 template <typename T>
 void launch_chunks(const e2h_delta_args &a, const Prepared &p, const ChunkScratch &cs, hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>(a.batch * a.heads * cs.chunks)), block(256);
-  hipLaunchKernelGGL(delta_chunk_kernel, grid, block, 0, s, a, p, cs);
+  const dim3 grid(static_cast<unsigned>(a.batch * a.heads * p.chunks)), block(256);
+  const int64_t widest = a.dim > a.vdim ? a.dim : a.vdim;
+  if (widest <= 64) hipLaunchKernelGGL(delta_chunk_kernel<4>, grid, block, 0, s, a, p, cs);
+  else if (widest <= 128) hipLaunchKernelGGL(delta_chunk_kernel<8>, grid, block, 0, s, a, p, cs);
+  else hipLaunchKernelGGL(delta_chunk_kernel<16>, grid, block, 0, s, a, p, cs);
   if (a.dim <= 64) launch_scan<4>(a, p, cs, s);
   else if (a.dim <= 128) launch_scan<8>(a, p, cs, s);
   else launch_scan<16>(a, p, cs, s);
@@ -721,8 +856,10 @@ int64_t round256(int64_t n) { return (n + 255) / 256 * 256; }
 // scratch layout; returns its size in bytes
 int64_t carve(const e2h_delta_args &a, Prepared *p, ChunkScratch *cs) {
   if (a.seqlen == 1) return 0;
-  const int64_t rows = a.batch * a.seqlen;
-  const int64_t qk = round256(rows * a.kv_heads * a.dim * 4), v = round256(rows * a.heads * a.vdim * 4), g = round256(rows * a.heads * 4);
+  const bool chunked = use_chunks(a);
+  const int64_t rows = a.batch * a.seqlen, chunks = (a.seqlen + kChunk - 1) / kChunk, tiles = (a.dim + 15) / 16;
+  const int64_t qk = round256((chunked ? a.batch * chunks * kChunk * a.kv_heads * tiles * 16 : rows * a.kv_heads * a.dim) * 4);
+  const int64_t v = round256(rows * a.heads * a.vdim * 4), g = round256(rows * a.heads * 4);
   if (p) {
     uint8_t *base = static_cast<uint8_t *>(a.scratch);
     p->q = reinterpret_cast<float *>(base);
@@ -730,16 +867,20 @@ int64_t carve(const e2h_delta_args &a, Prepared *p, ChunkScratch *cs) {
     p->v = reinterpret_cast<float *>(base + 2 * qk);
     p->beta = reinterpret_cast<float *>(base + 2 * qk + v);
     p->log_g = reinterpret_cast<float *>(base + 2 * qk + v + g);
+    p->tiles = chunked ? static_cast<int>(tiles) : 0;
+    p->chunks = static_cast<int>(chunks);
   }
   const int64_t prepared = 2 * qk + v + 2 * g;
-  if (!use_chunks(a)) return prepared;
-  const int64_t chunks = (a.seqlen + kChunk - 1) / kChunk, squares = a.batch * a.heads * chunks * kChunk * kChunk * 4;
+  if (!chunked) return prepared;
+  const int64_t gates = a.batch * a.heads * chunks * kChunk * 4, w = gates * tiles * 16, squares = gates * kChunk;
   if (cs) {
-    cs->t = reinterpret_cast<float *>(static_cast<uint8_t *>(a.scratch) + prepared);
-    cs->p = reinterpret_cast<float *>(static_cast<uint8_t *>(a.scratch) + prepared + squares);
-    cs->chunks = static_cast<int>(chunks);
+    uint8_t *base = static_cast<uint8_t *>(a.scratch) + prepared;
+    cs->w = reinterpret_cast<float *>(base);
+    cs->p = reinterpret_cast<float *>(base + w);
+    cs->g = reinterpret_cast<float *>(base + w + squares);
+    cs->e = reinterpret_cast<float *>(base + w + squares + gates);
   }
-  return prepared + 2 * squares;
+  return prepared + w + squares + 2 * gates;
 }
 
 template <typename T>
@@ -752,7 +893,8 @@ int launch_delta(const e2h_delta_args &a, hipStream_t s) {
   ChunkScratch cs = {};
   carve(a, &p, &cs);
   if (a.taps <= 4 && quads_ok(a)) {
-    const int cp = lanes_for(a.dim > a.vdim ? a.dim : a.vdim), runs = static_cast<int>((a.seqlen + kPrepareRun - 1) / kPrepareRun);
+    const int64_t widest = a.dim > a.vdim ? a.dim : a.vdim;
+    const int cp = lanes_for(p.tiles > 0 && widest < 16 ? 16 : widest), runs = static_cast<int>((a.seqlen + kPrepareRun - 1) / kPrepareRun);
     const int64_t waves = a.batch * runs * ((2 * a.kv_heads + a.heads + 64 / cp - 1) / (64 / cp));
     hipLaunchKernelGGL(delta_prepare4_kernel<T>, dim3(static_cast<unsigned>((waves + 3) / 4)), dim3(256), 0, s, a, p, cp, runs);
     hipLaunchKernelGGL(delta_gates_kernel<T>, dim3(static_cast<unsigned>((a.batch * a.seqlen * a.heads + 255) / 256)), dim3(256), 0, s, a, p);

@@ -483,6 +483,29 @@ def test_delta_batches_padding_and_reused_rows(dtype, form):
     assert rel(f64(again)[0], f64(got)[0]) < tol
 
 
+@pytest.mark.parametrize("heads,kvh,d,dv,taps,t", [(2, 1, 4, 4, 4, 24), (2, 1, 12, 8, 4, 65), (3, 3, 64, 64, 4, 63), (2, 2, 68, 20, 4, 129), (4, 2, 128, 128, 4, 200),
+                                                   (2, 1, 36, 128, 5, 66), (2, 1, 132, 20, 4, 130), (1, 1, 192, 256, 6, 127), (1, 1, 256, 40, 4, 128)])
+def test_delta_chunks_read_nothing_that_was_not_written(heads, kvh, d, dv, taps, t, monkeypatch):
+    """Heads that end inside a tile of 16 or leave tiles of their kernel empty, chunks whose last tokens do not exist, an odd and an even number of
+    chunks; scratch memory is full of NaN beforehand.  Tolerance: as for all shapes."""
+    made = seq_ops._scratch
+
+    def poisoned(args, query, like):
+        buf = made(args, query, like)
+        if buf is not None:
+            buf.fill_(255)
+        return buf
+
+    monkeypatch.setattr(seq_ops, "_scratch", poisoned)
+    _lib.set_seq_option("recurrence_form", 2)
+    b, eps = 2, 1e-5
+    x, c, p = delta_case(b, t, heads, kvh, d, dv, taps, torch.float32)
+    got, state = run_delta(x, c, p, heads, kvh, d, dv, taps, eps, torch.float32, [t])
+    for i in range(b):
+        want, s = want_delta(x, c, p, heads, kvh, d, dv, eps, i)
+        assert rel(f64(got)[i], want) < 4e-5 and rel(f64(state)[i], s) < 2e-5
+
+
 # ---- whole models ------------------------------------------------------------------------------------------------------------------
 
 CONFIGS = {
