@@ -4,7 +4,8 @@
 // lane column (lane 16 b + c holds keys 4 b .. 4 b + 3 of query c), so statistics are in-lane sums plus two shuffles, and the weights are the second operand of
 // O^T = V^T P^T without moving, over the key order 4 b .. 4 b + 3, 16 + 4 b .. 16 + 4 b + 3 of each 32.
 // What bounds it: the vector work between the products (scores, maxima, exponents, rounding) takes one and a half times as long as they do (8192 tokens, window 2048: matrix pipelines
-// busy 36 %, vector units 56 %; 64 x 768 tokens 24 and 44 %), and waves wait for a third of their time and more.  Two workgroups share a CU (64 KB of LDS each), so that one computes
+// busy 36 %, vector units 56 %; 64 x 768 tokens 24 and 44 %), and waves wait for a third of their time and more.  (Measured with masks taken key by key and the next
+// tile's loads waited for before V is read; without either 526 us have become 493 and 667 have become 646, 8 x 1024 tokens 185 and 174.)  Two workgroups share a CU (64 KB of LDS each), so that one computes
 // under the other's products and waits.  32 queries per wave rather than 16, so that a fragment of K or V read from LDS feeds two or four products (with 16 the
 // LDS took longer than the products); K and V reach LDS by loads that write it directly, two stages, one barrier per tile, and V's
 // fragments leave it through the transposing read (written transposed by two-byte stores, V cost as much LDS time as both products' reads).
@@ -40,6 +41,10 @@ __device__ __forceinline__ uint32_t pack_bf16_pair(float lo, float hi) {
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
+
+// The transposing read.  __restrict__ is what tells the compiler that loads into LDS under way do not write here: without it, it waits for
+// all of them before the first such read of a tile, which are the next tile's.
+__device__ __forceinline__ s16x4_t read_turned(const uint8_t *__restrict__ at) { return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t *)at); }
 
 // Workgroup -> (sequence, key head), query head of its group, block of queries counted from the last one.  Workgroups are dealt out to the eight XCDs in turn.
 // Where the (sequence, key head) pairs, or else the heads, divide by eight, each XCD walks its own ones, all blocks of one after each other and those with the most
@@ -196,7 +201,21 @@ __device__ __forceinline__ void attend(const bf16x8_t (&qf)[2][D / 32], const in
       }
     }
     // a tile inside every query's window needs no masks: whole, behind the kept keys, not beyond the first query, not out of the last one's window
-    if (!(n0 >= kl.kept && n0 + kKeys <= kl.count && j1 <= lo && hi - j0 < rule.window && j0 >= rule.first)) {
+    if (n0 >= kl.kept && n0 + kKeys <= kl.count && j1 <= lo && hi - j0 < rule.window && j0 >= rule.first) {
+    } else if (n0 >= kl.kept && j0 - rule.first >= rule.keep) {
+      // one run of keys, none of them kept: key t of the lane's (t = 16 kt + e) is `from` - t back from the query, and seen if that is in one range.
+      // 100 instructions for a tile instead of 1000, of 700 in all: prompts shorter than the window have a tile or two of these in five.
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int from = pos[i] - (j0 + 4 * b4), end = pos[i] - rule.first + 1 < rule.window ? pos[i] - rule.first + 1 : rule.window;
+        const int behind = from - (kl.count - n0 - 4 * b4) + 1, begin = behind > 0 ? behind : 0;
+        const uint32_t span = end > begin ? static_cast<uint32_t>(end - begin) : 0u;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) st[i][kt][e] = static_cast<uint32_t>(from - begin - (16 * kt + e)) < span ? st[i][kt][e] : kMaskedScore;
+      }
+    } else {
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
@@ -255,8 +274,7 @@ __device__ __forceinline__ void attend(const bf16x8_t (&qf)[2][D / 32], const in
       }
 #pragma unroll
       for (int v = 0; v < VT; ++v) {
-        const s16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t *)(lds + stage + v_at[v] + half * 32 * kRow));
-        const s16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t *)(lds + stage + v_at[v] + (half * 32 + 16) * kRow));
+        const s16x4_t v0 = read_turned(lds + stage + v_at[v] + half * 32 * kRow), v1 = read_turned(lds + stage + v_at[v] + (half * 32 + 16) * kRow);
         const u32x2_t a = __builtin_bit_cast(u32x2_t, v0), b = __builtin_bit_cast(u32x2_t, v1);
         const bf16x8_t vfrag = __builtin_bit_cast(bf16x8_t, u32x4_t{a[0], a[1], b[0], b[1]});
 #pragma unroll

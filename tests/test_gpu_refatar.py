@@ -194,6 +194,26 @@ def test_prompt_attention_in_blocks_of_64_and_128_queries(h, g, d, window, keep,
             assert (got[i, :f] == 0).all()
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("window,keep", [(0, 0), (1, 0), (2, 1), (63, 0), (64, 64), (65, 3), (128, 0), (200, 130)])
+def test_prompt_attention_counts_every_key_that_is_seen(d, window, keep):
+    """All scores zero and a value column per position modulo the head's size: a result is the number of seen keys of its column over all seen keys.  One key more or less in a
+    tile shows.  Tolerance: two bfloat16 roundings, of the result and of what it is divided by."""
+    _lib.set_seq_option("attention_prompt_queries", 128)
+    t, pads = 333, [0, 1, 63, 64, 130]
+    q = torch.zeros((len(pads), t, 2, d), dtype=torch.bfloat16, device=DEV)
+    k = randn(len(pads), t, 1, d, seed=1, dtype=torch.bfloat16)
+    v = torch.nn.functional.one_hot(torch.arange(t, device=DEV) % d, d).to(torch.bfloat16).view(1, t, 1, d).repeat(len(pads), 1, 1, 1)
+    for portions in ([t], [130, 203]):
+        got = f64(run_attention(q, k, v, None, torch.bfloat16, 0.3, window, keep, portions, first=torch.tensor(pads, device=DEV)))
+        for b, f in enumerate(pads):
+            i, j = np.arange(t)[:, None], np.arange(t)[None]
+            seen = (j <= i) & (j >= f) & ((i - j < (window or t)) | (j - f < keep))
+            count = np.stack([seen[:, c::d].sum(1) for c in range(d)], 1)
+            want = count / np.maximum(seen.sum(1, keepdims=True), 1)
+            assert (np.abs(got[b] - want[:, None]) <= 2.0 ** -8 * want[:, None]).all(), (portions, b)
+
+
 @BOTH
 def test_attention_of_padded_and_shorter_sequences_side_by_side(dtype):
     b, t, h, g, d, dv, window, keep = 3, 90, 4, 2, 32, 48, 11, 4
