@@ -814,7 +814,8 @@ bool quads_ok(const e2h_delta_args &a) {
 }
 
 bool use_chunks(const e2h_delta_args &a) {
-  if (a.seqlen == 1 || seq_options().recurrence_form == 1 || !quads_ok(a)) return false;
+  // (the scan counts a chunk's values in 31 bits)
+  if (a.seqlen == 1 || seq_options().recurrence_form == 1 || !quads_ok(a) || a.heads * a.vdim > INT32_MAX / kChunk) return false;
   return seq_options().recurrence_form == 2 || a.seqlen >= 24;
 }
 
