@@ -46,6 +46,8 @@ __device__ __forceinline__ void mma(f32x4_t &d, u32x4_t a, u32x4_t b) {
 }
 
 // P names the tiles and what surrounds them.  P::Tile holds uniform values.
+//   static constexpr bool kHalves             whether tiles may have 128 rows and fewer, bool half(Tile): whether this one does; only the products of those are
+//                                             formed then, and the rows 32 j + 16 wm + r of a tile are wave wm's instead of 128 wm + 16 j + r
 //   bool first(Tile &), bool next(Tile &)     the workgroup's tiles, false: no more
 //   int chunks()                              K / 64
 //   rsrc x_rsrc(Tile), w_rsrc(Tile)           the operands
@@ -57,6 +59,8 @@ template <bool F16, class P>
 __device__ __forceinline__ void walk(P &p, uint8_t *lds) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave & 1, wn = wave >> 1, chunks = p.chunks();
+  // a wave's 16-row blocks: neighbours, or every second one where tiles may be half empty
+  constexpr int kXWave = P::kHalves ? 16 : 128, kXStep = P::kHalves ? 32 : 16;
   typename P::Tile cur, nxt;
   if (!p.first(cur)) return;  // uniform, before any barrier
 
@@ -84,10 +88,10 @@ __device__ __forceinline__ void walk(P &p, uint8_t *lds) {
 
   // fragments of a half chunk: lane (h, n) reads piece 4 s + h of its rows
   const int n = lane & 15, h = lane >> 4;
-  const uint32_t xa = (128 * wm + n) * 128 + ((h ^ ((n >> 1) & 7)) << 4);
+  const uint32_t xa = (kXWave * wm + n) * 128 + ((h ^ ((n >> 1) & 7)) << 4);
   const uint32_t wa = (128 * wn + 8 * (n >> 2) + (n & 3)) * 128 + ((h ^ (((n >> 1) & 1) + 2 * (n >> 2))) << 4);
   u32x4_t xf[2][8], wf[2][8];
-  auto read_x = [&](uint32_t unit, int s, int i) { return *reinterpret_cast<const u32x4_t *>(lds + unit + (xa ^ (64 * s)) + i * 2048); };
+  auto read_x = [&](uint32_t unit, int s, int i) { return *reinterpret_cast<const u32x4_t *>(lds + unit + (xa ^ (64 * s)) + i * (kXStep * 128)); };
   auto read_w = [&](uint32_t unit, int s, int i) {
     return *reinterpret_cast<const u32x4_t *>(lds + unit + (wa ^ (64 * s)) + (i >> 1) * 4096 + (i & 1) * 512);
   };
@@ -109,19 +113,19 @@ __device__ __forceinline__ void walk(P &p, uint8_t *lds) {
   bool more = p.next(nxt);
   if (more) p.fetch(nxt, lane, wave, fetched);
   typename P::Dest dest;
-  const int row0 = 128 * wm + n, col0 = 128 * wn + 8 * h;
+  const int row0 = kXWave * wm + n, col0 = 128 * wn + 8 * h;
   p.dest(cur, row0, col0, dest);
 #pragma unroll
   for (int i = 0; i < 8; ++i) xf[0][i] = read_x(0, 0, i);
 #pragma unroll
   for (int i = 0; i < 8; ++i) wf[0][i] = read_w(kUnit, 0, i);
-  f32x4_t acc[8][8];
 
   uint32_t xu = 0, wu = kUnit, loading = 3 * kUnit;
   int ahead = 2;         // the chunk that the next loads bring, of this tile or (once it has come round) of the next one
   bool stored = false;   // this tile's first chunk has the stores of another one in front of its loads
-  auto chunk = [&](auto first) {
+  auto chunk = [&](auto first, auto blocks, f32x4_t (&acc)[8][8]) {
     constexpr bool kFirst = decltype(first)::value;  // of a tile
+    constexpr int kBlocks = decltype(blocks)::value;  // of 16 rows per wave
     const uint32_t nxu = after(wu), nwu = after(nxu);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
@@ -135,10 +139,10 @@ __device__ __forceinline__ void walk(P &p, uint8_t *lds) {
 #pragma unroll
       for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < kBlocks; ++j) {
           if (kFirst && s == 0) mma<F16, true>(acc[i][j], wf[s][i], xf[s][j]);
           else mma<F16, false>(acc[i][j], wf[s][i], xf[s][j]);
-          const int slot = 8 * i + j, r = slot / 2;
+          const int slot = kBlocks * i + j, r = slot / 2;
           if (slot % 2 == 0 && r < 16) {  // the next half's fragments, in the order of their use
             if (r == 0) wf[s ^ 1][0] = read_w(s ? nwu : wu, s ^ 1, 0);
             else if (r <= 8) xf[s ^ 1][r - 1] = read_x(s ? nxu : xu, s ^ 1, r - 1);
@@ -161,29 +165,44 @@ __device__ __forceinline__ void walk(P &p, uint8_t *lds) {
     wu = nwu;
   };
   while (true) {
-    chunk(std::true_type{});
-    int c = 1;
-    do chunk(std::false_type{});  // at least three chunks: whoever waits for what a tile's start has requested can count on that
-    while (++c < chunks);
-    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last products' results can be read
-    __builtin_amdgcn_sched_barrier(0);
+    const auto chunks_of = [&](auto blocks) {
+      f32x4_t acc[8][8];
+      chunk(std::true_type{}, blocks, acc);
+      int c = 1;
+      do chunk(std::false_type{}, blocks, acc);  // at least three chunks: whoever waits for what a tile's start has requested can count on that
+      while (++c < chunks);
+      asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last products' results can be read
+      __builtin_amdgcn_sched_barrier(0);
+      int row = row0, col = col0;
+      asm volatile("" : "+v"(row), "+v"(col));  // what is derived from them is formed here: held through the tiles, it would not fit the registers
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+      for (int j = 0; j < 8; ++j)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        asm volatile("" : "+a"(acc[2 * q][j]), "+a"(acc[2 * q + 1][j]));  // read here: all 256 at once would not fit
-        float v[8];
+        for (int q = 0; q < 4; ++q) {
+          float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // rows that are not there: stored nowhere, but counted
+          if (j < decltype(blocks)::value) {
+            asm volatile("" : "+a"(acc[2 * q][j]), "+a"(acc[2 * q + 1][j]));  // read here: all 256 at once would not fit
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = acc[2 * q + (e >> 2)][j][e & 3];
-        p.store(cur, dest, j, q, row0 + 16 * j, col0 + 32 * q, v);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+            for (int e = 0; e < 8; ++e) v[e] = acc[2 * q + (e >> 2)][j][e & 3];
+          }
+          p.store(cur, dest, j, q, row + kXStep * j, col + 32 * q, v);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    if constexpr (P::kHalves) {
+      if (p.half(cur)) chunks_of(std::integral_constant<int, 4>{});
+      else chunks_of(std::integral_constant<int, 8>{});
+    } else {
+      chunks_of(std::integral_constant<int, 8>{});
+    }
     if (!more) break;
     stored = true;
     cur = nxt;
     more = p.next(nxt);
     if (more) p.fetch(nxt, lane, wave, fetched);
-    p.dest(cur, row0, col0, dest);
+    int row = row0, col = col0;
+    asm volatile("" : "+v"(row), "+v"(col));
+    p.dest(cur, row, col, dest);
     __builtin_amdgcn_sched_barrier(0);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // loads past the last tile must land before the workgroup gives its LDS away

@@ -420,11 +420,12 @@ __global__ __launch_bounds__(256, 2) void expert_tiles_kernel(const Product p) {
 }
 
 // The same on tiles of 256 x 256 (e2h_gemm256.h): a workgroup per CU walks its XCD's tiles.  8192 rows x 8 of 64 experts, 4096 x 1024:
-// both products 985 us (1116 TFLOP/s), 1301 on the tiles above; a ninth of the products are for rows past an expert's last one, and the last
-// round of tiles fills half the chip in the up product.
+// both products 904 us (1216 TFLOP/s), 1301 on the tiles above.  An expert's last tile forms the products of 128 rows where it has no more (both products
+// 937 us with whole tiles throughout, a ninth of the products for rows that are not there); the last round of tiles fills half the chip in the up product.
 template <bool UP>
 struct ExpertWalk {
   typedef e2h::Tile Tile;
+  static constexpr bool kHalves = true;
   const Product &p;
   int t, end, stride;
   int begin, after;  // tiles before the present expert's first, and up to its last
@@ -467,6 +468,7 @@ struct ExpertWalk {
     tile.m = (t - begin) - tile.n * rows;
     return true;
   }
+  __device__ __forceinline__ bool half(const Tile &tile) const { return tile.count - tile.m * gemm256::kSide <= gemm256::kSide / 2; }
   __device__ __forceinline__ int chunks() const { return p.K / 64; }
   __device__ __forceinline__ __amdgpu_buffer_rsrc_t x_rsrc(const Tile &) const { return make_rsrc(p.x, static_cast<uint32_t>(p.x_rows * p.K * 2)); }
   __device__ __forceinline__ __amdgpu_buffer_rsrc_t w_rsrc(const Tile &tile) const {
@@ -498,7 +500,7 @@ struct ExpertWalk {
   __device__ __forceinline__ void dest(const Tile &tile, int row, int, Dest &d) const {
     if (UP) return;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) d.slot[UP ? 0 : j] = slot_of(p, sorted_row(tile, row + 16 * j));
+    for (int j = 0; j < 8; ++j) d.slot[UP ? 0 : j] = slot_of(p, sorted_row(tile, row + 32 * j));
   }
   __device__ __forceinline__ void store(const Tile &tile, const Dest &d, int j, int, int row, int col, float (&v)[8]) const {
     if (UP) {
@@ -707,12 +709,12 @@ int check_experts(const e2h_experts_args &a) {
   return E2H_OK;
 }
 
-// 256-row tiles: from 104 rows per expert on, where an expert's second tile of 128 rows begins to cost (64 experts, 4096 x 1024: 80 rows each 275 us with
-// tiles of 128 and 295 with 256, 96 278 and 288, 112 349 and 303, 256 450 and 386, 1024 1301 and 985), and with enough of them for half the CUs,
-// below which two workgroups per CU of the other form divide the work better.
+// 256-row tiles: from 24 rows per expert on, where rows that are not there cost half a tile at most (64 experts, 4096 x 1024, both products: 24 rows each 252 us with
+// tiles of 128 and 240 with 256, 64 271 and 263, 96 285 and 272; 32 experts, 2048 x 1024: 24 rows 75.4 and 74.5, 96 87.9 and 83.1; below nothing was
+// measured), and with enough of them for half the CUs, below which two workgroups per CU of the other form divide the work better.
 bool big_tiles_pay(const Product &p) {
   const int64_t tiles = (static_cast<int64_t>(p.rows) / gemm256::kSide + (p.experts + 1) / 2) * p.n_tiles;
-  return p.K % 64 == 0 && p.K >= gemm256::kLeastK && static_cast<int64_t>(p.rows) * p.N <= static_cast<int64_t>(UINT32_MAX) / 2 - 16 && p.rows >= 104LL * p.experts && tiles >= 128;
+  return p.K % 64 == 0 && p.K >= gemm256::kLeastK && static_cast<int64_t>(p.rows) * p.N <= static_cast<int64_t>(UINT32_MAX) / 2 - 16 && p.rows >= 24LL * p.experts && tiles >= 128;
 }
 
 template <bool UP>

@@ -55,6 +55,7 @@ __global__ __launch_bounds__(256) void unpack_int8_kernel(const int8_t *__restri
 // The tiles of one plain product, dealt to the XCDs in contiguous runs of equal length: panels of eight column blocks, all row
 // blocks of a panel after each other, so that the 32 tiles at work on an XCD share four row blocks and eight column blocks.
 struct PlainWalk {
+  static constexpr bool kHalves = false;
   static constexpr int kPanel = 8;
   struct Tile {
     int rb, cb;

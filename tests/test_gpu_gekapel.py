@@ -318,6 +318,7 @@ def test_experts(dtype, form, rows, width, n, top, ff, shared):
     (192, 16392, 2, (1, 255)),                      # the shortest K of the 256-row tiles, a last column tile of eight columns; then K = 16392 on the others
     (4096, 192, 8, (0, 1, 256, 257, 513, 15, 640, 300)),
     (8192, 256, 4, (700, 2, 0, 258)),
+    (4096, 256, 6, (128, 129, 384, 385, 130, 896)),   # last tiles of 128 rows, which are half ones, and of one row more; one behind the other
     (320, 640, 70, (731,) * 10 + (0,) * 59 + (40,)),
 ])
 def test_experts_on_256_row_tiles(width, ff, n, counts):
