@@ -200,7 +200,7 @@ def calls():
         spec = importlib.util.spec_from_file_location(f"{__package__}._calls", CALLS_PATH)
         module, lib = importlib.util.module_from_spec(spec), load()
         spec.loader.exec_module(module)
-        module.bind(*(ctypes.cast(f, c_void_p).value for f in (lib.e2h_int4_mm, lib.e2h_int8_mm, lib.e2h_stream_capturing)), ops._workspaces)
+        module.bind(*(ctypes.cast(f, c_void_p).value for f in (lib.e2h_int4_mm, lib.e2h_int8_mm, lib.e2h_stream_capturing)), ops._workspaces, check)
         _calls = module
     return _calls
 

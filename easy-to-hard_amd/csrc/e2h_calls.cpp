@@ -3,7 +3,8 @@
 // A call of a small linear is bound by the host.  4096 x 4096 at one row, group size 128: the kernel takes 6.2 us, and the checks, the allocation, the workspace's lookup and
 // the ctypes call of the Python path together with nn.Module's part 11.6; from here 7.4 (see WeightOnlyInt4Linear.forward).  Anything out of the ordinary -- tensor subclasses
 // and wrappers, modes, traces, other types, strides, devices or shapes, captures, a workspace that is not there yet -- returns None, and the Python path takes the call or
-// raises its error.
+// raises its error, and so it does where an entry point refuses its arguments.  A launch that failed is reported from here: asked once more, the
+// runtime may take it, over whatever of a call of several launches has begun.
 //
 // Both functions take (x, weight, scales, .., out_features) and return a new tensor or None.
 #include <Python.h>
@@ -30,8 +31,12 @@ Int4Mm int4_mm_entry = nullptr;
 Int8Mm int8_mm_entry = nullptr;
 Capturing capturing_entry = nullptr;
 PyObject *workspaces = nullptr;  // ops._workspaces: (device index, stream) -> tensor
+PyObject *check = nullptr;       // _lib.check: raises what a status stands for
 
 constexpr int64_t kMostRows = 1023;  // larger calls may use memory of their own
+
+// E2H_ERR_LAUNCH and E2H_ERR_NO_DEVICE of e2h_quant.h: what does not follow from the arguments
+bool failed(int status) { return status == -6 || status == -7; }
 
 // a tensor of this device and type whose elements lie as its shape says, with nothing that follows what happens to it
 bool plain(const at::Tensor &t, c10::DeviceIndex device, at::ScalarType type) {
@@ -72,7 +77,7 @@ at::Tensor result_for(const at::Tensor &x, int64_t n) {
 }
 
 template <class Launch>
-PyObject *run(const at::Tensor &x, int64_t n, c10::DeviceIndex device, Launch launch) {
+PyObject *run(const char *entry, const at::Tensor &x, int64_t n, c10::DeviceIndex device, Launch launch) {
   void *const stream = c10::hip::getCurrentHIPStream(device).stream();
   void *ws = nullptr;
   int64_t ws_bytes = 0;
@@ -82,6 +87,10 @@ PyObject *run(const at::Tensor &x, int64_t n, c10::DeviceIndex device, Launch la
   Py_BEGIN_ALLOW_THREADS  // a full queue makes the launch wait
   rc = launch(y.data_ptr(), ws, ws_bytes, stream);
   Py_END_ALLOW_THREADS
+  if (failed(rc)) {
+    Py_XDECREF(PyObject_CallFunction(check, "is", rc, entry));
+    return nullptr;
+  }
   if (rc != 0) Py_RETURN_NONE;  // the Python path meets the same status and raises it
   return THPVariable_Wrap(std::move(y));
 }
@@ -103,7 +112,7 @@ PyObject *int4_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   const int64_t n = w.size(0) * 8, k = w.size(1) * 128, m = k > 0 ? x.numel() / k : 0;
   if (x.size(-1) != k || n != out || m < 1 || m > kMostRows || (g != 32 && g != 64 && g != 128 && g != 256) || k % g != 0) Py_RETURN_NONE;
   if (sz.size(0) != k / g || sz.size(1) != n || sz.size(2) != 2) Py_RETURN_NONE;
-  return run(x, n, device, [&](void *y, void *ws, int64_t ws_bytes, void *stream) {
+  return run("e2h_int4_mm", x, n, device, [&](void *y, void *ws, int64_t ws_bytes, void *stream) {
     return int4_mm_entry(x.data_ptr(), w.data_ptr(), sz.data_ptr(), y, m, n, k, static_cast<int>(g), 8, ws, ws_bytes, stream);
   });
   END_HANDLE_TH_ERRORS
@@ -125,20 +134,23 @@ PyObject *int8_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   if (x.dim() < 1 || q.dim() != 2 || scales.dim() != 1) Py_RETURN_NONE;
   const int64_t n = q.size(0), k = q.size(1), m = k > 0 ? x.numel() / k : 0;
   if (x.size(-1) != k || n != out || n < 1 || m < 1 || m > kMostRows || scales.size(0) != n) Py_RETURN_NONE;
-  return run(x, n, device, [&](void *y, void *ws, int64_t ws_bytes, void *stream) {
+  return run("e2h_int8_mm", x, n, device, [&](void *y, void *ws, int64_t ws_bytes, void *stream) {
     return int8_mm_entry(x.data_ptr(), q.data_ptr(), scales.data_ptr(), y, m, n, k, ws, ws_bytes, stream);
   });
   END_HANDLE_TH_ERRORS
 }
 
-// bind(address of e2h_int4_mm, of e2h_int8_mm, of e2h_stream_capturing, ops._workspaces)
+// bind(address of e2h_int4_mm, of e2h_int8_mm, of e2h_stream_capturing, ops._workspaces, _lib.check)
 PyObject *bind(PyObject *, PyObject *args) {
   unsigned long long int4 = 0, int8 = 0, capturing = 0;
-  PyObject *dict = nullptr;
-  if (!PyArg_ParseTuple(args, "KKKO!", &int4, &int8, &capturing, &PyDict_Type, &dict)) return nullptr;
+  PyObject *dict = nullptr, *raises = nullptr;
+  if (!PyArg_ParseTuple(args, "KKKO!O", &int4, &int8, &capturing, &PyDict_Type, &dict, &raises)) return nullptr;
   Py_INCREF(dict);
+  Py_INCREF(raises);
   Py_XDECREF(workspaces);
+  Py_XDECREF(check);
   workspaces = dict;
+  check = raises;
   int4_mm_entry = reinterpret_cast<Int4Mm>(static_cast<uintptr_t>(int4));
   int8_mm_entry = reinterpret_cast<Int8Mm>(static_cast<uintptr_t>(int8));
   capturing_entry = reinterpret_cast<Capturing>(static_cast<uintptr_t>(capturing));

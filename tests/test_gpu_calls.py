@@ -1,5 +1,7 @@
 """Small calls of the quantized linears in one native call (csrc/e2h_calls.cpp): the same bits as the Python path, and everything out of the ordinary left to it."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -113,3 +115,31 @@ def test_modules_with_other_forms_of_weights_run_as_before():
     lin.out_features = 256  # refused where the weight has another number of rows
     with pytest.raises(RuntimeError):
         lin(x)
+
+
+@pytest.mark.parametrize("mode", ["int4", "int8"])
+def test_a_failed_launch_is_reported_and_not_tried_again(mode):
+    """The entry point's address is that of a function which launches nothing and returns a status."""
+    lin, x = _linear(mode), _x(4, 512)
+    want = lin(x)
+    lib, calls, asked = _lib.load(), _lib.calls(), []
+
+    def bind(int4, int8):
+        calls.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (int4, int8, lib.e2h_stream_capturing)), ops._workspaces, _lib.check)
+
+    def answer(real, code):
+        return ctypes.CFUNCTYPE(ctypes.c_int, *real.argtypes)(lambda *a: asked.append(code) or code)
+
+    try:
+        for code in (-6, -7):
+            fakes = answer(lib.e2h_int4_mm, code), answer(lib.e2h_int8_mm, code)
+            bind(*fakes)
+            with pytest.raises(RuntimeError, match=rf"e2h_{mode}_mm: .*status {code}"):
+                lin(x)
+        assert asked == [-6, -7]
+        fakes = answer(lib.e2h_int4_mm, -5), answer(lib.e2h_int8_mm, -5)  # refused arguments: the Python path's to meet
+        bind(*fakes)
+        assert torch.equal(lin(x), want) and asked == [-6, -7, -5]
+    finally:
+        bind(lib.e2h_int4_mm, lib.e2h_int8_mm)
+    assert torch.equal(lin(x), want)
