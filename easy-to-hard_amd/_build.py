@@ -93,18 +93,17 @@ def build_seq_library(verbose=False):
 
 
 def build_calls(verbose=False):
-    """The host-side extension module of small calls (csrc/e2h_calls.cpp), against the installed torch."""
+    """The host-side extension module of small calls (csrc/e2h_calls.cpp), for the installed torch and no other."""
     import sysconfig
 
     import torch
 
     home = Path(torch.__file__).resolve().parent
-    cxx = shutil.which(os.environ.get("CXX", "g++"))
-    if cxx is None:
-        raise RuntimeError("no host C++ compiler found; the extension module of small calls cannot be built")
     rocm = Path(_hipcc()).resolve().parent.parent
+    cxx = shutil.which(os.environ.get("CXX", "g++")) or rocm / "llvm" / "bin" / "clang++"  # else the one that hipcc drives
     tmp = CALLS_PATH.with_name(CALLS_PATH.name + ".tmp")
     out = _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+                f'-DE2H_TORCH_VERSION="{torch.__version__}"',
                 *(f"-I{d}" for d in (home / "include", home / "include" / "torch" / "csrc" / "api" / "include", rocm / "include", sysconfig.get_paths()["include"])),
                 str(CSRC / "e2h_calls.cpp"), "-o", str(tmp), f"-L{home / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python"])
     if verbose and out.strip():
@@ -114,6 +113,6 @@ def build_calls(verbose=False):
 
 
 if __name__ == "__main__":
-    print(build_calls(verbose=True))
     print(build_library(verbose=True))
     print(build_seq_library(verbose=True))
+    print(build_calls(verbose=True))

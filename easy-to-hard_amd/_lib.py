@@ -6,7 +6,10 @@ no fallback implementation behind these entry points.
 
 import ctypes
 import importlib.util
+import warnings
 from ctypes import c_char_p, c_float, c_int, c_int32, c_int64, c_void_p
+
+import torch
 
 from ._build import CALLS_PATH, LIB_PATH, SEQ_LIB_PATH, build_library, build_seq_library
 
@@ -189,19 +192,44 @@ def load_seq(build_if_missing=False):
 _calls = None
 
 
+class _PythonCalls:
+    """Stands for the extension module where that cannot be used: every call is left to the Python path, which launches the same kernels."""
+
+    @staticmethod
+    def int4_linear(*_):
+        return None
+
+    int8_linear = int4_linear
+
+
+def _load_calls(lib):
+    if not CALLS_PATH.exists():
+        return "is missing"
+    from . import ops
+
+    spec = importlib.util.spec_from_file_location(f"{__package__}._calls", CALLS_PATH)
+    try:
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+    except ImportError as e:
+        return f"cannot be loaded ({e})"
+    if module.torch_version != torch.__version__:  # it reads tensors' structures as that torch laid them out
+        return f"was built for torch {module.torch_version}, this is {torch.__version__}"
+    module.bind(*(ctypes.cast(f, c_void_p).value for f in (lib.e2h_int4_mm, lib.e2h_int8_mm, lib.e2h_stream_capturing)), ops._workspaces, check)
+    return module
+
+
 def calls():
-    """The extension module of small calls (csrc/e2h_calls.cpp), bound to libe2h_quant.so and the workspaces of `ops`."""
+    """The extension module of small calls (csrc/e2h_calls.cpp), bound to libe2h_quant.so and the workspaces of `ops`.  Without one that was built for this torch, a warning
+    and a stand-in: such calls then cost the host what they cost through Python."""
     global _calls
     if _calls is None:
-        if not CALLS_PATH.exists():
-            raise E2HLibraryError(f"{CALLS_PATH} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`")
-        from . import ops
-
-        spec = importlib.util.spec_from_file_location(f"{__package__}._calls", CALLS_PATH)
-        module, lib = importlib.util.module_from_spec(spec), load()
-        spec.loader.exec_module(module)
-        module.bind(*(ctypes.cast(f, c_void_p).value for f in (lib.e2h_int4_mm, lib.e2h_int8_mm, lib.e2h_stream_capturing)), ops._workspaces, check)
-        _calls = module
+        got = _load_calls(load())
+        if isinstance(got, str):
+            warnings.warn(f"{CALLS_PATH} {got}: small calls of the quantized linears go through Python until it is built with "
+                          "`python -c 'import __graft_entry__ as g; g.build()'`", RuntimeWarning, stacklevel=2)
+            got = _PythonCalls
+        _calls = got
     return _calls
 
 

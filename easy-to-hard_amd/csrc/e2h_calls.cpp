@@ -165,4 +165,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_calls", nullptr, -1, methods};
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__calls(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__calls(void) {
+  PyObject *m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", E2H_TORCH_VERSION) != 0) Py_CLEAR(m);  // compared before anything here touches a tensor
+  return m;
+}

@@ -61,6 +61,26 @@ def test_argument_validation_returns_codes_without_launching():
     assert lib.e2h_set_option(b"int4_rows_per_wave", 0) == 0
 
 
+@pytest.mark.parametrize("why", ["is missing", "cannot be loaded", "was built for torch"])
+def test_small_calls_without_a_module_for_this_torch_are_left_to_python(why, monkeypatch, tmp_path):
+    monkeypatch.setattr(_lib, "_calls", None)
+    if why == "was built for torch":
+        monkeypatch.setattr(torch, "__version__", "0.0.0")
+    else:
+        monkeypatch.setattr(_lib, "CALLS_PATH", tmp_path / "_calls.so")
+        if why == "cannot be loaded":
+            (tmp_path / "_calls.so").write_bytes(b"not a library")
+    with pytest.warns(RuntimeWarning, match=why):
+        calls = _lib.calls()
+    assert calls.int4_linear(None, None, None, 128, 8) is None and calls.int8_linear(None, None, None, 8) is None
+    assert _lib.calls() is calls  # one warning in a process
+
+
+def test_the_module_of_small_calls_is_used_where_it_was_built_for_this_torch(monkeypatch):
+    monkeypatch.setattr(_lib, "_calls", None)
+    assert _lib.calls().torch_version == torch.__version__
+
+
 def test_ops_refuse_cpu_tensors():
     x = torch.zeros(1, 128, dtype=torch.bfloat16)
     packed = torch.zeros(1, 1, 32, 4, dtype=torch.int32)
