@@ -367,18 +367,19 @@ __global__ __launch_bounds__(64 * NW) void decode_attention_gqa_kernel(const uin
 // of TransformerBlock.forward, reference :279-282), stores it to h_out and normalises h.  The first kPieces pieces of
 // 8 values per thread stay in registers and all their loads, slices and weights included, are issued before anything is waited for (one memory
 // round trip for the whole row up to BLOCK * 8 * kPieces values); longer rows re-read the rest.
-// What bounds it in a decode step: the launch and one memory round trip.  64 rows of 8192 with two slices: 7.2 us with 512 threads, whose second pieces asked for their
-// slices when the first had arrived, 5.7 with 1024; 32 rows of 4096 5.1 either way.
+// What bounds it in a decode step: the launch and one memory round trip.  64 rows of 8192 with two slices, launches after each other: 6.2 us with 512 threads, whose second
+// pieces asked for their slices when the first had arrived, 5.0 with 1024.
+// kMaxSlices (2 or 4) slices are requested without asking how many there are, the first one in the place of those that are not: a branch for each of four
+// cost 64 rows of 2048 4.2 us instead of 3.5 (4096: 4.3 and 4.0), always four cost two slices 0.2.
 enum NormTerm { kNothing = 0, kDelta = 1, kSums = 2 };  // what is added to x first
 
-template <int BLOCK, NormTerm SRC>
+template <int BLOCK, int kPieces, NormTerm SRC, int kMaxSlices>
 __global__ __launch_bounds__(BLOCK) void rmsnorm_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ delta,
                                                         const float *__restrict__ psum, int slices,
                                                         const uint16_t *__restrict__ col_scales,
                                                         const uint16_t *__restrict__ w, uint16_t *__restrict__ h_out,
                                                         uint16_t *__restrict__ y, StagedOut staged, int dim, float eps) {
-  constexpr int kPieces = BLOCK == 256 ? 2 : 1, kStride = BLOCK * 8, kWaves = BLOCK / 64;
-  constexpr int kMaxSlices = 4;  // slices whose loads are all issued before the first addition
+  constexpr int kStride = BLOCK * 8, kWaves = BLOCK / 64;
   const size_t row = blockIdx.x;
   const uint16_t *xr = x + row * dim;
   const uint16_t *dr_row = SRC == kDelta ? delta + row * dim : nullptr;
@@ -453,15 +454,16 @@ __global__ __launch_bounds__(BLOCK) void rmsnorm_kernel(const uint16_t *__restri
 #pragma unroll
   for (int p = 0; p < kPieces; ++p) {
     const int i = threadIdx.x * 8 + p * kStride, at = i < dim ? i : 0;  // past the row: its first piece, not used
+    if (p > 0 && __builtin_amdgcn_readfirstlane(i) >= dim) break;
     keep[p] = *reinterpret_cast<const u32x4_t *>(xr + at);
     if (SRC == kDelta) keepd[p] = *reinterpret_cast<const u32x4_t *>(dr_row + at);
     if (SRC == kSums) {
 #pragma unroll
-      for (int u = 0; u < kMaxSlices; ++u)
-        if (u < slices) {
-          lo[p][u] = *reinterpret_cast<const f32x4_t *>(pr + u * slice_floats + at);
-          hi[p][u] = *reinterpret_cast<const f32x4_t *>(pr + u * slice_floats + at + 4);
-        }
+      for (int u = 0; u < kMaxSlices; ++u) {
+        const float *const from = pr + (u < slices ? u : 0) * slice_floats + at;
+        lo[p][u] = *reinterpret_cast<const f32x4_t *>(from);
+        hi[p][u] = *reinterpret_cast<const f32x4_t *>(from + 4);
+      }
       if (col_scales) keepc[p] = *reinterpret_cast<const u32x4_t *>(col_scales + at);
     }
     keepw[p] = *reinterpret_cast<const u32x4_t *>(w + at);  // needed only after the reduction
@@ -490,11 +492,11 @@ __global__ __launch_bounds__(BLOCK) void rmsnorm_kernel(const uint16_t *__restri
       if constexpr (SRC == kSums) {
         f32x4_t l[kMaxSlices], h[kMaxSlices];
 #pragma unroll
-        for (int u = 0; u < kMaxSlices; ++u)
-          if (u < slices) {
-            l[u] = *reinterpret_cast<const f32x4_t *>(pr + u * slice_floats + i);
-            h[u] = *reinterpret_cast<const f32x4_t *>(pr + u * slice_floats + i + 4);
-          }
+        for (int u = 0; u < kMaxSlices; ++u) {
+          const float *const from = pr + (u < slices ? u : 0) * slice_floats + i;
+          l[u] = *reinterpret_cast<const f32x4_t *>(from);
+          h[u] = *reinterpret_cast<const f32x4_t *>(from + 4);
+        }
         term = sum_slices(l, h, col_scales ? *reinterpret_cast<const u32x4_t *>(col_scales + i) : u32x4_t{}, i);
       } else {
         term = *reinterpret_cast<const u32x4_t *>(dr_row + i);
@@ -592,22 +594,29 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t *__restric
   reinterpret_cast<u32x4_t *>(y)[idx] = o;
 }
 
-template <int BLOCK>
+template <int BLOCK, int PIECES>
 void launch_rmsnorm_block(const uint16_t *x, const uint16_t *delta, const float *psum, int slices, const uint16_t *col_scales, const uint16_t *w,
                           uint16_t *h_out, uint16_t *y, StagedOut staged, int64_t rows, int64_t dim, float eps, hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>(rows)), block(BLOCK);
-  const int width = static_cast<int>(dim);
-  if (delta) hipLaunchKernelGGL((rmsnorm_kernel<BLOCK, kDelta>), grid, block, 0, stream, x, delta, psum, slices, col_scales, w, h_out, y, staged, width, eps);
-  else if (psum) hipLaunchKernelGGL((rmsnorm_kernel<BLOCK, kSums>), grid, block, 0, stream, x, delta, psum, slices, col_scales, w, h_out, y, staged, width, eps);
-  else hipLaunchKernelGGL((rmsnorm_kernel<BLOCK, kNothing>), grid, block, 0, stream, x, delta, psum, slices, col_scales, w, h_out, y, staged, width, eps);
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(rows)), dim3(BLOCK), 0, stream, x, delta, psum, slices, col_scales, w, h_out, y, staged, static_cast<int>(dim), eps);
+  };
+  if (delta) launch(rmsnorm_kernel<BLOCK, PIECES, kDelta, 1>);
+  else if (!psum) launch(rmsnorm_kernel<BLOCK, PIECES, kNothing, 1>);
+  else if (slices <= 2) launch(rmsnorm_kernel<BLOCK, PIECES, kSums, 2>);
+  else launch(rmsnorm_kernel<BLOCK, PIECES, kSums, 4>);
 }
 
-// few rows (decode): one piece per thread up to 8192 values; many rows: 256-thread workgroups
+// Up to 512 rows (decode): one piece per thread up to 8192 values, so that the row is one round trip.  Where sums are added to more rows than there are CUs two pieces, since
+// 1024 threads leave a CU one row at a time (512 rows of 8192, two slices: 14.4 us, with two pieces 13.2; 320 of 5120 8.2 and 7.3; without sums 5.5 and 5.9: left).
+// More rows: workgroups of 256.  Rows of 2048 and fewer are one piece of those (64 rows, four slices 3.5 us; with a second, empty piece 4.2).
 void launch_rmsnorm(const uint16_t *x, const uint16_t *delta, const float *psum, int slices, const uint16_t *col_scales, const uint16_t *w,
                     uint16_t *h_out, uint16_t *y, StagedOut staged, int64_t rows, int64_t dim, float eps, hipStream_t stream) {
-  if (rows <= 512 && dim > 4096) launch_rmsnorm_block<1024>(x, delta, psum, slices, col_scales, w, h_out, y, staged, rows, dim, eps, stream);
-  else if (rows <= 512 && dim >= 4096) launch_rmsnorm_block<512>(x, delta, psum, slices, col_scales, w, h_out, y, staged, rows, dim, eps, stream);
-  else launch_rmsnorm_block<256>(x, delta, psum, slices, col_scales, w, h_out, y, staged, rows, dim, eps, stream);
+  const bool few = rows <= 512;
+  const auto launch = dim <= 2048 ? launch_rmsnorm_block<256, 1>
+                      : !few || dim < 4096 ? launch_rmsnorm_block<256, 2>
+                      : dim == 4096 ? launch_rmsnorm_block<512, 1>
+                      : (psum || delta) && rows > 256 ? launch_rmsnorm_block<512, 2> : launch_rmsnorm_block<1024, 1>;
+  launch(x, delta, psum, slices, col_scales, w, h_out, y, staged, rows, dim, eps, stream);
 }
 
 template <int D, int NW>

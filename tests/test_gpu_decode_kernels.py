@@ -71,6 +71,16 @@ def test_norm_of_slices_equals_the_norm_of_their_sum(rows, dim, slices, scaled):
     assert torch.equal(h, want_h) and torch.equal(h, x + delta) and torch.equal(y, want_y)
 
 
+@pytest.mark.parametrize("slices", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("rows,dim", [(2, 8), (3, 2048), (3, 2056), (256, 4608), (257, 4608), (300, 8200), (512, 4104), (513, 4608)])
+def test_norm_of_slices_on_both_sides_of_its_lines(rows, dim, slices):
+    """Rows of one piece and of two, waves without a second piece, and row counts that change the workgroup."""
+    test_norm_of_slices_equals_the_norm_of_their_sum(rows, dim, slices, False)
+    x = randn_bf16((rows, dim), std=1.5, seed=rows).to(DEV)
+    w = (1 + 0.1 * randn_bf16((dim,), seed=dim).float()).to(torch.bfloat16).to(DEV)
+    assert torch.allclose(ops.rmsnorm(x, w, 1e-5).float(), _rmsnorm_reference(x, w, 1e-5).float(), rtol=2 ** -6, atol=1e-6)
+
+
 def test_silu_mul_matches_stock_ops():
     a = randn_bf16((32, 11008), std=2.0, seed=1).to(DEV)
     b = randn_bf16((32, 11008), std=1.0, seed=2).to(DEV)
