@@ -56,6 +56,7 @@ _SIGNATURES = {
     "e2h_int8_mm_silu_gate": (c_int, [_P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, _P]),
     "e2h_int8_mm_rope_kv": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, _P]),
     "e2h_int4_mm_silu_gate_rows_scratch_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int, c_int]),
+    "e2h_int4_mm_silu_gate_rows_pays": (c_int, [c_int64, c_int64, c_int64, c_int, c_int]),
     "e2h_int4_mm_silu_gate_rows": (c_int, [_P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int, c_int, _P, c_int64, _P]),
     "e2h_int4_mm_silu_gate": (c_int, [_P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int, c_int, _P]),
     "e2h_int4_staged_bytes": (c_int64, [c_int64, c_int64]),

@@ -42,6 +42,8 @@
 //
 // Workgroup -> tile mapping: workgroup w runs on XCD w % 8; each XCD owns the column blocks cb = xcd (mod 8) and
 // walks them for one row block before moving to the next, so its L2 keeps that slice of the weights.
+#include <algorithm>
+
 #include "e2h_common.h"
 #include "e2h_int4_unpack.h"
 
@@ -656,11 +658,9 @@ namespace e2h {
 int64_t int4_unpacked_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int inner_k_tiles);
 constexpr int kUnpackRows = 1024;  // from here on callers offer memory for unpacked operands
 
-// Group sums of x, the only scratch of a gated call, or 0 where two calls and a pass that multiplies are expected to be no slower or a form is asked for by an option.
-// The launch of both matrices has twice the workgroups, spares one pass over x for its group sums, the two products' way to memory and back, and a launch.  Measured, us, two calls and
-// the pass / here: 2 x 11008 x 4096 g128 65 rows 61 / 54, 128 rows 72 / 51, 471 rows 117 / 97, 1500 rows 298 / 273; g64 471 rows 141 / 112; g32 192 rows 132 / 96; 2 x 5504 x 2048
-// g128 256 rows 53 / 32.  Over 440 shapes and rows (65 .. 4096) 21 % less; the expected times, 7 % in favour of the calls, leave four that are slower, by 2.5 % at most (2 x 22016 x 8192, 320
-// rows, where the calls fill their last rounds, 266 / 288: left to them).  Calls on unpacked operands (e2h_unpacked_gemm.hip) stay with those.
+// Group sums of x, the only scratch of a gated call, or 0 where two calls of the 32x32-tile kernel and a pass that multiplies are expected to be no slower or a form is asked for by an
+// option.  The launch of both matrices has twice the workgroups, spares one pass over x for its group sums, the two products' way to memory and back, and a launch.  Calls on unpacked
+// operands (e2h_unpacked_gemm.hip) stay with those.
 int64_t int4_gate_rows_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int inner_k_tiles) {
   if (inner_k_tiles != 8 || (groupsize != 32 && groupsize != 64 && groupsize != 128 && groupsize != 256)) return 0;
   if (M <= 64 || N < 8 || N % 8 != 0 || K < 128 || K % 128 != 0 || K % groupsize != 0 || M > INT32_MAX / 64 || N > INT32_MAX / 64 || K > INT32_MAX / 64) return 0;
@@ -675,10 +675,30 @@ int64_t int4_gate_rows_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int
   const double calls = 2 * int4_gemm_shape(m, n, k, G, int64_t{32} << 20).us + 3 + static_cast<double>(M) * static_cast<double>(N) * 6 / 5e6;  // the pass moves six bytes an output
   return 1.07 * int4_gemm_shape(m, 2 * n, k, G, 0).us < calls ? bytes : 0;
 }
+
+// Whether a model's calls gain by it: sizes that are taken, beside calls of whichever kernel they would run (small weights, of group size 256 above all: the one of 16 x 16 tiles).  The
+// gated launch takes 5 us and a tenth more than expected of a product of both widths.  Measured, us, two calls and the pass / here: 2 x 11008 x 4096 g128 65 rows 61 / 54, 128 rows
+// 72 / 51, 471 rows 117 / 97, 1500 rows 298 / 273; g64 471 rows 141 / 112; 2 x 5504 x 2048 g128 256 rows 51 / 31; left to the calls: 2 x 2816 x 1024 g256 72 rows 17 / 21, 2 x 2048 x 4096
+// g256 192 rows 35 / 47, 2 x 1024 x 512 g256 192 rows 15 / 16.  Of 834 shapes and rows (65 .. 4096) that are taken 779 pay, 19 % less on average and 3 % more at most; the other 55 would
+// take up to 34 % more and none 2 % less.
+bool int4_gate_rows_pay(int64_t M, int64_t N, int64_t K, int groupsize, int inner_k_tiles) {
+  if (int4_gate_rows_bytes(M, N, K, groupsize, inner_k_tiles) == 0) return false;
+  const int G = groupsize == 256 ? 128 : groupsize, m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
+  double call = int4_gemm_shape(m, n, k, G, int64_t{32} << 20).us;
+  if (groupsize == 256 || (M + 127) / 128 * ((N + 127) / 128) < 320) {  // as e2h_int4_mm chooses
+    const int tiles = groupsize != 256 && (N + 127) / 128 * ((M + 63) / 64) >= 256 ? 2 : 1;
+    call = std::min(call, int4_rows_us(m, n, k, groupsize, tiles));
+  }
+  return 1.03 * int4_gemm_shape(m, 2 * n, k, G, 0).us + 6 < 2 * call + 3 + static_cast<double>(M) * static_cast<double>(N) * 6 / 5e6;
+}
 }  // namespace e2h
 
 extern "C" int64_t e2h_int4_mm_silu_gate_rows_scratch_bytes(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles) {
   return e2h::int4_gate_rows_bytes(m, n, k, groupsize, inner_k_tiles);
+}
+
+extern "C" int e2h_int4_mm_silu_gate_rows_pays(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles) {
+  return e2h::int4_gate_rows_pay(m, n, k, groupsize, inner_k_tiles);
 }
 
 extern "C" int e2h_int4_mm_silu_gate_rows(const uint16_t *x, const int32_t *packed_gate, const uint16_t *sz_gate, const int32_t *packed_up, const uint16_t *sz_up,

@@ -685,18 +685,20 @@ int launch_x_group_sums(const uint16_t *x, float *out, int M, int K, int stride,
 }  // namespace e2h
 
 namespace e2h {
-// More than 64 rows: whether the 32x32-tile kernel, which takes us32, is expected to take less time than this file's kernels.  Of these a workgroup takes `one` us per 128 k when it has its CU
-// to itself and two that share a CU `two` (64 rows and 4 x 16 columns, or 8 x 16 where `tiles` is 2, group sums of x included; at group size 256 32 rows and 64 columns); 3 to 6 % off 540
-// measured calls per group size.
-bool int4_rows_on_32x32(int M, int N, int K, int groupsize, int tiles, double us32) {
+// More than 64 rows: what a call of this file's kernels is expected to take.  A workgroup takes `one` us per 128 k when it has its CU to itself and two that share a CU `two` (64 rows and 4 x 16
+// columns, or 8 x 16 where `tiles` is 2, group sums of x included; at group size 256 32 rows and 64 columns); 3 to 6 % off 540 measured calls per group size.
+double int4_rows_us(int M, int N, int K, int groupsize, int tiles) {
   const int64_t wgs = groupsize == 256 ? static_cast<int64_t>((N + 63) / 64) * ((M + 31) / 32) : static_cast<int64_t>(((N + 15) / 16 + 4 * tiles - 1) / (4 * tiles)) * ((M + 63) / 64);
   const int64_t per_cu = (wgs + kCUs - 1) / kCUs;
   double one = 0.34, two = 0.62;
   if (groupsize == 32) one = tiles == 2 ? 1.9 : 1.23, two = tiles == 2 ? 3.8 : 2.46;
   if (groupsize == 64) one = tiles == 2 ? 1.2 : 0.8, two = tiles == 2 ? 2.4 : 1.23;
   if (groupsize == 128) one = tiles == 2 ? 1.05 : 0.83, two = tiles == 2 ? 1.43 : 1.07;
-  return us32 < 6 + (K / 128) * (static_cast<double>(per_cu / 2) * two + (per_cu & 1 ? one : 0));
+  return 6 + (K / 128) * (static_cast<double>(per_cu / 2) * two + (per_cu & 1 ? one : 0));
 }
+
+// whether the 32x32-tile kernel, which takes us32, is expected to take less time
+bool int4_rows_on_32x32(int M, int N, int K, int groupsize, int tiles, double us32) { return us32 < int4_rows_us(M, N, K, groupsize, tiles); }
 }  // namespace e2h
 
 extern "C" int64_t e2h_workspace_bytes(void) { return static_cast<int64_t>(e2h::kTicketBytes) + (int64_t{32} << 20); }

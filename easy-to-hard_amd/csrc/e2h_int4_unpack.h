@@ -113,6 +113,9 @@ Int4GemmShape int4_gemm_shape(int M, int N, int K, int groupsize, int64_t scratc
 int int4_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint16_t *y, const float *xsum, int xsum_stride,
               float *partials, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream, const int *run_if = nullptr, const int *row_flag = nullptr);
 
+// More than 64 rows: us that a call is expected to take on the 16x16-tile kernels (e2h_int4_mm.hip), with `tiles` column tiles per wave.
+double int4_rows_us(int M, int N, int K, int groupsize, int tiles);
+
 // y = silu(x w) * (x w2) of two matrices of one shape in one launch of that kernel, rounded as the two products and F.silu(a) * b would be; `shape` as
 // int4_gemm_shape gives it for the columns of both, with one slice.
 int int4_gemm_gate(const uint16_t *x, const int32_t *packed, const uint16_t *sz, const int32_t *packed2, const uint16_t *sz2, uint16_t *y, const float *xsum,

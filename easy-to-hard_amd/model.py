@@ -283,7 +283,7 @@ class FeedForward(nn.Module):
         if not (FUSE_GATE and _fusable(x) and type(w1) is WeightOnlyInt4Linear and type(w3) is WeightOnlyInt4Linear) or torch.compiler.is_compiling():
             return None
         k, n, group = w1.in_features, w1.out_features, w1.groupsize
-        if x.shape[-1] != k or x.numel() <= 64 * k or w1.padding or w3.padding or w3.groupsize != group:
+        if x.shape[-1] != k or x.numel() <= 64 * k or w1.padding or w3.padding or w3.groupsize != group or not ops.int4_gate_rows_pay(x.numel() // k, n, k, group):
             return None
         for w in (w1, w3):
             p, sz = w.weight, w.scales_and_zeros

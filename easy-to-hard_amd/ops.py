@@ -378,9 +378,14 @@ def int4_gate_rows_scratch(m, n, k, groupsize, inner_k_tiles, device):
         return None
 
 
+def int4_gate_rows_pay(m, n, k, groupsize, inner_k_tiles=8) -> bool:
+    """True where int4_mm_silu_gate_rows is expected to take less time than two calls of int4_mm and silu_mul."""
+    return bool(_lib.load().e2h_int4_mm_silu_gate_rows_pays(m, n, k, groupsize, inner_k_tiles))
+
+
 def int4_mm_silu_gate_rows(x, packed_gate, sz_gate, packed_up, sz_up, groupsize):
-    """bf16(bf16(silu(int4_mm(x, gate))) * int4_mm(x, up)) over more than 64 rows in one product launch, or None where two calls of int4_mm are
-    no slower (or there is no memory for the launch's scratch)."""
+    """bf16(bf16(silu(int4_mm(x, gate))) * int4_mm(x, up)) over more than 64 rows in one product launch, or None where the sizes are not taken
+    (or there is no memory for the launch's scratch)."""
     _need_gpu(x, packed_gate, sz_gate, packed_up, sz_up)
     if x.dtype != torch.bfloat16 or sz_gate.dtype != torch.bfloat16 or sz_up.dtype != torch.bfloat16:
         raise TypeError("int4_mm_silu_gate_rows: bfloat16 activations and scales_and_zeros expected")

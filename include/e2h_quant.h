@@ -203,6 +203,8 @@ int e2h_int4_mm_rope_kv(const uint16_t *x, const int32_t *packed, const uint16_t
  *   e2h_int4_mm_silu_gate_rows_scratch_bytes returns, which is 0 where the shape is not taken (or not faster than those calls: the entry point then returns
  *   E2H_ERR_BAD_SHAPE).  The launch neither allocates nor keeps anything. */
 int64_t e2h_int4_mm_silu_gate_rows_scratch_bytes(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles);
+/* 1 where that launch is expected to take less time than two calls of e2h_int4_mm and e2h_silu_mul, whichever kernels those run, else 0 (a subset of the shapes that are taken). */
+int e2h_int4_mm_silu_gate_rows_pays(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles);
 int e2h_int4_mm_silu_gate_rows(const uint16_t *x, const int32_t *packed_gate, const uint16_t *sz_gate, const int32_t *packed_up,
                                const uint16_t *sz_up, uint16_t *y, int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles,
                                void *scratch, int64_t scratch_bytes, void *stream);

@@ -386,6 +386,12 @@ def test_rows_between_the_two_int4_kernels(m, n, k, groupsize, big):
     assert on_32x32(m, n, k, groupsize, tiles, us) == big
 
 
+@pytest.mark.parametrize("m,n,k,groupsize,pays", [(471, 11008, 4096, 128, True), (65, 11008, 4096, 256, True), (256, 5504, 2048, 128, True), (320, 2816, 1024, 256, True), (65, 2816, 1024, 128, True),
+                                                  (72, 2816, 1024, 256, False), (192, 2048, 4096, 256, False), (400, 1024, 2048, 256, False), (320, 1408, 1024, 256, False), (64, 11008, 4096, 128, False)])
+def test_gated_rows_where_they_were_measured_to_be_faster_than_the_calls(m, n, k, groupsize, pays):
+    assert _lib.load().e2h_int4_mm_silu_gate_rows_pays(m, n, k, groupsize, 8) == pays
+
+
 @pytest.mark.parametrize("m,n,k,groupsize,unpacked", [(6000, 32000, 4096, 64, True), (8192, 12288, 4096, 64, True), (2048, 22016, 8192, 64, True), (8192, 12288, 4096, 128, True), (8192, 12288, 4096, 32, True),
                                                       (1300, 10240, 8192, 64, False), (1700, 22016, 8192, 64, False), (2048, 11008, 4096, 64, False), (2048, 12288, 4096, 128, False)])
 def test_int4_operands_are_unpacked_where_that_is_faster(m, n, k, groupsize, unpacked):

@@ -252,6 +252,24 @@ def test_gated_rows_leave_watched_modules_and_other_forms_to_the_modules():
     assert torch.equal(ff._gate_rows(strided), ff._gate_rows(x).transpose(0, 1))
 
 
+def test_gated_rows_are_left_to_calls_that_are_faster():
+    """Group size 256 on small weights, whose products run on 16 x 16 tiles."""
+    from easy_to_hard_amd.model import FeedForward, ModelArgs
+    from easy_to_hard_amd.quantize import WeightOnlyInt4QuantHandler, prepare_int4_weight_and_scales_and_zeros
+
+    ff = FeedForward(ModelArgs(dim=1024, intermediate_size=1408, n_head=8, n_layer=1))
+    WeightOnlyInt4QuantHandler(ff, groupsize=128).convert_for_runtime()
+    gen = torch.Generator().manual_seed(2)
+    for lin in (ff.w1, ff.w3):
+        lin.groupsize = 256
+    for lin in (ff.w1, ff.w2, ff.w3):
+        w = (torch.randn((lin.out_features, lin.in_features), generator=gen) * 0.05).to(torch.bfloat16).to(DEV)
+        lin.weight, lin.scales_and_zeros = prepare_int4_weight_and_scales_and_zeros(w, lin.groupsize, 8)
+    x = torch.randn((2, 64, 1024), generator=gen).to(torch.bfloat16).to(DEV)
+    assert ff._gate_rows(x) is None
+    assert torch.equal(ff(x), ff.w2(ops.silu_mul(ff.w1(x), ff.w3(x))))
+
+
 # ---- weights unpacked to float16 first (csrc/e2h_unpacked_gemm.hip) ---------------------------------------------------------------------
 
 def _unpacked(codes, scale, zero, x, g, flag=None):
