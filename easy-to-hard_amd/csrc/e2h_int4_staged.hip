@@ -72,12 +72,12 @@ bool plan(StagedArgs *a, Geometry *g, const void *staged, int64_t m, int64_t n, 
   const int halves = a->M > 32 && n * k * (gate ? 2 : 1) <= (int64_t{1} << 25) ? 2 : 1;
   const int mt = a->M <= 16 ? 1 : a->M <= 32 || halves == 2 ? 2 : 4;
   const int want_t = options().staged_tiles, want_s = options().staged_slices;  // experiments: force a geometry
-  // The geometry with the least cost; the weights of the cost were fitted to a sweep over T and S at 1 .. 64 rows of the shapes above and
-  // 12288 / 4096 / 32000 x 4096: the chosen geometry is within 6 % of the best one there.  One round of 256 workgroups with many tiles
-  // beats two rounds with few (w1|w3 22016 x 8192, 1 row: T = 12 43.6 us, T = 8 46.0; 32000 x 4096: T = 8 14.6, T = 6 19.0); K slices pay
+  // The geometry with the least cost; the weights of the cost were fitted to a sweep over T and S, with workgroups of eight waves throughout, at 1 .. 64 rows of the shapes above and
+  // 12288 / 4096 / 32000 x 4096: the chosen geometry was within 6 % of the best one there, and the 7B, 13B and 34B shapes have kept theirs.  One round of 256 workgroups with many tiles
+  // beats two rounds with few (of eight waves: w1|w3 22016 x 8192, 1 row: T = 12 43.6 us, T = 8 46.0; 32000 x 4096: T = 8 14.6, T = 6 19.0); K slices pay
   // while a round is not full (w2 4096 x 11008, 32 rows: T = 4, S = 4 10.1 us, the best with S = 1 15.6).  What a slice costs the norm that
-  // adds it grows with rows and columns: fitted with the norm's time to 1 .. 64 rows of 1024 x 2048 .. 8192 x 22016 at every group size, where
-  // the choice is within 0.2 % of the best one on average and 6 % at most (one unit per slice whatever its size: 2.6 %, 31 %; 8192 x 8192 at
+  // adds it grows with rows and columns: fitted with the norm's time, in the same form, to 1 .. 64 rows of 1024 x 2048 .. 8192 x 22016 at every group size, where
+  // the choice was within 0.2 % of the best one on average and 6 % at most (one unit per slice whatever its size: 2.6 %, 31 %; 8192 x 8192 at
   // group size 128 and 32 rows 19.9 us, now 18.6; 4096 x 4096 at group size 64 and 64 rows 15.5, now 13.7).
   double best_cost = -1;
   for (int s = 1; s <= (epi == kStPartial ? 8 : 1) && s <= kt; s *= 2) {

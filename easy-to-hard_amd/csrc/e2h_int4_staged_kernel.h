@@ -14,7 +14,8 @@
 // 128-wide chunks of the workgroup's K slice)
 // and all work on the same T tiles of 16 weight rows and on all rows of the batch, so that weights are read once (small weights beside 33
 // and more rows: on half of them, see plan).  No wave shares anything with another until the end.  The waves' partial tiles meet in LDS; wave w adds and finishes the (column tile, row
-// tile) units w, w + 8, .. (w + 4, ..) in a fixed order, so results are deterministic.  S workgroups may split K further (partial epilogue
+// tile) units w, w + 8, .. (w + 4, ..) in a fixed order, so results are deterministic; the order of a sum follows from the number of waves and the chunk they begin with, which
+// another epilogue of the same weights may have otherwise (a gated launch has twice the tiles of a plain one).  S workgroups may split K further (partial epilogue
 // only): their float32 sums go to slice s of a [S][M][N] array for the consumer to add in slice order.
 //
 // What a wave needs passes in units of 1 KB through a ring of its own in LDS, written by loads that touch no register: per chunk the
@@ -127,6 +128,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void int4_staged_mm_kernel(const St
   const int col_block = blockIdx.x;
   // Rows of a multiple of 32 KB: workgroups that all start with their first chunk ask few of the memory's channels at a time, so each starts with another one
   // (w1|w3 22016 x 8192, g64, 1 row 48.5 -> 40.4 us, 32 rows 55.7 -> 50.4; head 32000 x 8192, 1 row 35.2 -> 28.6; 12288 x 4096, which has rows of 16 KB, 7.8 either way).
+  // Workgroups of four waves begin alike: turned chunks make no difference to them (w1|w3, g64, 33 rows 73.2 us, turned 73.1, 64 rows 75.5 and 76.3; head, 64 rows 54.0 and 53.4).
   const int turn = kWaves == 8 && KT % 64 == 0 && nloc > 0 ? static_cast<int>(static_cast<unsigned>(col_block) % static_cast<unsigned>(nloc)) : 0;
   const int row0 = blockIdx.z * (16 * MT);
   const int tile16_0 = col_block * TC;
@@ -145,7 +147,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void int4_staged_mm_kernel(const St
   const __amdgpu_buffer_rsrc_t xs_rsrc = make_rsrc(a.sums, static_cast<uint32_t>(static_cast<size_t>(KT) * a.Mpad * 32));
 
   uint8_t *const ring = lds + kg * (kRing * 1024);
-  // what lane 4 q + s brings: piece s ^ (q / 4 mod 4) of row q
+  // what lane 4 q + s brings: piece s ^ turned(q / 4 mod 4) of row q
   const int q4 = lane >> 2;
   const uint32_t piece = static_cast<uint32_t>((lane & 3) ^ turned(lane >> 4)) * 16u;
   const uint32_t w_lane = static_cast<uint32_t>(q4 >> 3) * KT * 512u + (q4 & 7) * 64u + piece;  // rows 0 .. 7, 8 .. 15: two packed tiles
@@ -383,7 +385,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void int4_staged_mm_kernel(const St
 #pragma unroll 1
   while (i < nloc) run(std::integral_constant<int, kAhead>{});  // a wave with fewer chunks than the ring holds
 
-  // ---- the eight K parts meet in LDS as a balanced tree in the order of K; wave w finishes units w, w + 8, .. -------------
+  // ---- the waves' K parts meet in LDS as a balanced tree in the order of K; wave w finishes units w, w + kWaves, .. -------
   float *const red = reinterpret_cast<float *>(lds);
   const auto put = [&](int part) {
 #pragma unroll
