@@ -1,7 +1,7 @@
 // Calls of a quantized linear on plain tensors, host side: what ops._int4_mm_impl and ops._int8_mm_impl do for up to 1023 rows, in one native call.
 //
-// A call of a small linear is bound by the host.  4096 x 4096 at one row, group size 128: the kernel takes 6.2 us, and the checks, the allocation, the workspace's lookup and
-// the ctypes call of the Python path together with nn.Module's part 11.6; from here 7.4 (see WeightOnlyInt4Linear.forward).  Anything out of the ordinary -- tensor subclasses
+// A call of a small linear through Python is bound by the host.  4096 x 4096 at one row, group size 128: the kernel takes 7.0 us, and the checks, the allocation, the workspace's lookup
+// and the ctypes call of the Python path together with nn.Module's part 11.6; from here 7.3 (see WeightOnlyInt4Linear.forward).  Anything out of the ordinary -- tensor subclasses
 // and wrappers, modes, traces, other types, strides, devices or shapes, captures, a workspace that is not there yet -- returns None, and the Python path takes the call or
 // raises its error, and so it does where an entry point refuses its arguments.  A launch that failed is reported from here: asked once more, the
 // runtime may take it, over whatever of a call of several launches has begun.

@@ -709,9 +709,11 @@ int check_experts(const e2h_experts_args &a) {
   return E2H_OK;
 }
 
-// 256-row tiles: from 24 rows per expert on, where rows that are not there cost half a tile at most (64 experts, 4096 x 1024, both products: 24 rows each 252 us with
-// tiles of 128 and 240 with 256, 64 271 and 263, 96 285 and 272; 32 experts, 2048 x 1024: 24 rows 75.4 and 74.5, 96 87.9 and 83.1; below nothing was
-// measured), and with enough of them for half the CUs, below which two workgroups per CU of the other form divide the work better.
+// 256-row tiles: from 24 rows per expert on, where rows that are not there cost half a tile at most, and with enough of them for half the CUs, below which two workgroups per CU of the other
+// form divide the work better.  Both products, us, tiles of 128 / of 256, the same number of rows for every expert on average: 64 experts, 4096 x 1024, 24 rows each 236 / 233, 64 256 / 252,
+// 96 272 / 263, 256 381 / 360; 32 experts, 2048 x 1024, 24 rows 72 / 72, 64 78 / 76, 96 84 / 81.  Rows by Zipf's law, 64 experts: 24 rows on average 313 / 239, 32 314 / 242, but 48 310 / 317,
+// 64 325 / 333 and 96 327 / 335; by its square 32 304 / 242, 48 292 / 313, 64 313 / 329, 96 318 / 330, 128 362 / 349.  Below 24 the two are within 2 % where experts have equal shares
+// (8 rows 227 / 227, 16 232 / 228; 32 experts, 16 rows 69 / 69), and few uneven ones gain (20 rows by Zipf's law 313 / 234).
 bool big_tiles_pay(const Product &p) {
   const int64_t tiles = (static_cast<int64_t>(p.rows) / gemm256::kSide + (p.experts + 1) / 2) * p.n_tiles;
   return p.K % 64 == 0 && p.K >= gemm256::kLeastK && static_cast<int64_t>(p.rows) * p.N <= static_cast<int64_t>(UINT32_MAX) / 2 - 16 && p.rows >= 24LL * p.experts && tiles >= 128;

@@ -178,6 +178,8 @@ typedef struct {
   void *out;
   int64_t ld_out, out_off;
 } e2h_delta_args;
+/* Prompts of 24 tokens and more hold queries, keys, and a product of either with a chunk's system by whole chunks of 64 tokens and tiles of 16 channels: 474 MB for 8192 tokens of
+ * 32 heads (16 key heads) of 128, 3.1 GB for 1024 sequences of 24 such tokens. */
 int64_t e2h_seq_delta_scratch_bytes(const e2h_delta_args *a);
 int e2h_seq_delta(const e2h_delta_args *a, void *stream);
 
