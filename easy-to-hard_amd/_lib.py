@@ -14,6 +14,12 @@ import torch
 from ._build import CALLS_PATH, LIB_PATH, SEQ_LIB_PATH, build_library, build_seq_library
 
 _P = c_void_p
+
+
+class RowNorm(ctypes.Structure):
+    _fields_ = [("x", _P), ("partials", _P), ("col_scales", _P), ("weight", _P), ("h_out", _P), ("slices", c_int), ("eps", c_float)]
+
+
 _SIGNATURES = {
     # name: (restype, argtypes)
     "e2h_abi_version": (c_int, []),
@@ -55,6 +61,10 @@ _SIGNATURES = {
     "e2h_argmax_rows": (c_int, [_P, c_int64, _P, c_int64, c_int64, _P]),
     "e2h_int8_mm_silu_gate": (c_int, [_P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, _P]),
     "e2h_int8_mm_rope_kv": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, _P]),
+    "e2h_int8_norm_mm_supported": (c_int, [c_int64, c_int64, c_int64]),
+    "e2h_int8_norm_mm": (c_int, [ctypes.POINTER(RowNorm), _P, _P, _P, c_int64, c_int64, c_int64, _P]),
+    "e2h_int8_norm_mm_silu_gate": (c_int, [ctypes.POINTER(RowNorm), _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, _P]),
+    "e2h_int8_norm_mm_rope_kv": (c_int, [ctypes.POINTER(RowNorm), _P, _P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, _P]),
     "e2h_int4_mm_silu_gate_rows_scratch_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int, c_int]),
     "e2h_int4_mm_silu_gate_rows_pays": (c_int, [c_int64, c_int64, c_int64, c_int, c_int]),
     "e2h_int4_mm_silu_gate_rows": (c_int, [_P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int, c_int, _P, c_int64, _P]),

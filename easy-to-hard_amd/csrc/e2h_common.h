@@ -37,6 +37,15 @@ __host__ __device__ inline uint16_t f32_to_bf16_rne(float f) {
 // float32 value rounded to the nearest bfloat16, kept as float32
 __host__ __device__ inline float bf16_round(float f) { return bf16_to_f32(f32_to_bf16_rne(f)); }
 
+#if defined(__HIPCC__)
+// two of them in one dword, one conversion
+__device__ __forceinline__ uint32_t f32x2_to_bf16_rne(float lo, float hi) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
+}
+#endif
+
 // ---- option store (set through e2h_set_option) --------------------------------------------------
 
 struct Options {

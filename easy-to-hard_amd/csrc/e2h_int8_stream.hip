@@ -418,3 +418,62 @@ extern "C" int e2h_int8_mm_partials(const uint16_t *x, const int8_t *q, float *p
   return stream::run<stream::Int8Weights, Partial8>({x, q, q, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k)}, {partials},
                                                     static_cast<hipStream_t>(stream));
 }
+
+// ---- the same three behind the norm that makes their rows ---------------------------------------------------------------------------
+namespace e2h {
+namespace {
+int check_norm(const e2h_row_norm *norm, int64_t m, int64_t n, int64_t k) {
+  if (!norm || !norm->x || !norm->weight || (norm->partials && !norm->h_out)) return E2H_ERR_NULL_POINTER;
+  if (!e2h_int8_norm_mm_supported(m, n, k) || (norm->partials && (norm->slices < 1 || norm->slices > 2))) return E2H_ERR_BAD_SHAPE;
+  if (!aligned16(norm->x) || !aligned16(norm->partials) || !aligned16(norm->col_scales) || !aligned16(norm->weight) || !aligned16(norm->h_out)) return E2H_ERR_MISALIGNED;
+  return E2H_OK;
+}
+stream::RowNorm row_norm(const e2h_row_norm &n) { return {n.x, n.partials, n.partials ? n.col_scales : nullptr, n.weight, n.h_out, n.slices, n.eps}; }
+}  // namespace
+}  // namespace e2h
+
+extern "C" int e2h_int8_norm_mm_supported(int64_t m, int64_t n, int64_t k) {
+  return n >= 1 && n <= INT32_MAX && e2h::stream::norm_fits(m, k) && n * k < (int64_t{1} << 32) && e2h::stream::takes(m, n, k, 1) ? 1 : 0;
+}
+
+extern "C" int e2h_int8_norm_mm(const e2h_row_norm *norm, const int8_t *q, const uint16_t *scales, uint16_t *y, int64_t m, int64_t n, int64_t k, void *stream) {
+  using namespace e2h;
+  if (!q || !scales || !y) return E2H_ERR_NULL_POINTER;
+  const int rc = check_norm(norm, m, n, k);
+  if (rc != E2H_OK) return rc;
+  if (!aligned16(q) || (reinterpret_cast<uintptr_t>(scales) & 1u) || (reinterpret_cast<uintptr_t>(y) & 1u)) return E2H_ERR_MISALIGNED;
+  return stream::run_norm<stream::Int8Weights, Plain8>({norm->x, q, q, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k)}, {scales, y}, row_norm(*norm),
+                                                       static_cast<hipStream_t>(stream));
+}
+
+extern "C" int e2h_int8_norm_mm_silu_gate(const e2h_row_norm *norm, const int8_t *q_gate, const uint16_t *scales_gate, const int8_t *q_up, const uint16_t *scales_up,
+                                          uint16_t *y, int64_t m, int64_t n, int64_t k, void *stream) {
+  using namespace e2h;
+  if (!q_gate || !scales_gate || !q_up || !scales_up || !y) return E2H_ERR_NULL_POINTER;
+  const int rc = check_norm(norm, m, n, k);
+  if (rc != E2H_OK) return rc;
+  if (!aligned16(q_gate) || !aligned16(q_up) || ((reinterpret_cast<uintptr_t>(scales_gate) | reinterpret_cast<uintptr_t>(scales_up) | reinterpret_cast<uintptr_t>(y)) & 1u))
+    return E2H_ERR_MISALIGNED;
+  return stream::run_norm<stream::Int8Weights, Gate8>({norm->x, q_gate, q_up, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k)}, {scales_gate, scales_up, y},
+                                                      row_norm(*norm), static_cast<hipStream_t>(stream));
+}
+
+extern "C" int e2h_int8_norm_mm_rope_kv(const e2h_row_norm *norm, const int8_t *q, const uint16_t *scales, const uint16_t *freqs_cis, uint16_t *q_out, uint16_t *k_cache,
+                                        uint16_t *v_cache, const int64_t *input_pos, int64_t batch, int64_t n_head, int64_t n_kv_head, int64_t head_dim, int64_t cache_len,
+                                        int64_t k, void *stream) {
+  using namespace e2h;
+  if (!q || !scales || !freqs_cis || !q_out || !k_cache || !v_cache || !input_pos) return E2H_ERR_NULL_POINTER;
+  if (n_head < 1 || n_kv_head < 1 || head_dim < 2 || (head_dim % 2) != 0 || cache_len < 1 || cache_len > INT32_MAX || n_head > INT32_MAX || n_kv_head > INT32_MAX ||
+      head_dim > INT32_MAX / (n_head + 2 * n_kv_head))
+    return E2H_ERR_BAD_SHAPE;
+  const int64_t n = (n_head + 2 * n_kv_head) * head_dim;
+  const int rc = check_norm(norm, batch, n, k);
+  if (rc != E2H_OK) return rc;
+  if (!aligned16(q) || (reinterpret_cast<uintptr_t>(scales) & 1u) || (reinterpret_cast<uintptr_t>(freqs_cis) & 3u) || (reinterpret_cast<uintptr_t>(q_out) & 1u) ||
+      (reinterpret_cast<uintptr_t>(k_cache) & 1u) || (reinterpret_cast<uintptr_t>(v_cache) & 1u) || (reinterpret_cast<uintptr_t>(input_pos) & 7u))
+    return E2H_ERR_MISALIGNED;
+  return stream::run_norm<stream::Int8Weights, Rope8>({norm->x, q, q, static_cast<int>(batch), static_cast<int>(n), static_cast<int>(k)},
+                                                      {scales, freqs_cis, q_out, k_cache, v_cache, input_pos, static_cast<int>(n_head), static_cast<int>(n_kv_head),
+                                                       static_cast<int>(cache_len), static_cast<int>(head_dim)},
+                                                      row_norm(*norm), static_cast<hipStream_t>(stream));
+}

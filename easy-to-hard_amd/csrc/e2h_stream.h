@@ -17,10 +17,30 @@
 // are sent out of the buffer's range: they return zeros and move no data.
 #pragma once
 
+#include <type_traits>
+
 #include "e2h_common.h"
 
 namespace e2h {
 namespace stream {
+
+// One row whose RMSNorm is x, formed by every workgroup for itself behind the requests for its first weights, in the round trip that those take as well.
+// h = bf16(x + term), term = bf16(sum of the slices) or bf16(bf16(sum) * column scale), or h = x where there are no partial sums; rounding points and orders of sums are those of
+// e2h_add_rmsnorm_partials.  Workgroup 0 stores h.  A step of one sequence through four int8 7B layers and the head, nine such products: 281 us with the norms as launches of their
+// own (2.8 each), 268.  With two rows what every workgroup reads and does for itself takes as long as the launch (two layers of 7B, 163 us and 164).
+struct RowNorm {
+  const uint16_t *x;
+  const float *partials;       // [slices][K], null: h = x
+  const uint16_t *col_scales;  // may be null
+  const uint16_t *weight;
+  uint16_t *h_out;
+  int slices;                  // 1 or 2
+  float eps;
+};
+struct NoNorm {};
+constexpr int kNormPieces = 2, kNormPiece = 4096;  // pieces of the row, eight values per thread each
+constexpr int kNormSums = 128, kNormBytes = kNormSums + kNormPieces * kNormPiece * 2;  // LDS: the waves' sums of squares, the row
+inline bool norm_fits(int64_t M, int64_t K) { return M == 1 && K >= 128 && K % 128 == 0 && K <= kNormPieces * kNormPiece; }
 
 constexpr int64_t kMaxBytes = int64_t{1} << 31;  // of a buffer: offsets of 2^31 are what is sent out of range
 constexpr int kWaves = 8;
@@ -71,19 +91,101 @@ __device__ __forceinline__ void wait_loads(int n) {
   }
 }
 
+// What a thread holds of the row to be normalised: eight values of every piece, all requested before anything is waited for.
+struct NormLoads {
+  u32x4_t x[kNormPieces], w[kNormPieces], cs[kNormPieces];
+  f32x4_t lo[kNormPieces][2], hi[kNormPieces][2];
+
+  __device__ __forceinline__ void request(const RowNorm &n, int K) {
+#pragma unroll
+    for (int p = 0; p < kNormPieces; ++p) {
+      const int i = p * kNormPiece + static_cast<int>(threadIdx.x) * 8, at = i < K ? i : 0;  // past the row: its first piece, not used
+      if (K <= p * kNormPiece) break;
+      x[p] = *reinterpret_cast<const u32x4_t *>(n.x + at);
+      if (n.partials) {
+        const float *const from = n.partials + at, *const other = from + (n.slices > 1 ? K : 0);
+        lo[p][0] = *reinterpret_cast<const f32x4_t *>(from);
+        hi[p][0] = *reinterpret_cast<const f32x4_t *>(from + 4);
+        lo[p][1] = *reinterpret_cast<const f32x4_t *>(other);
+        hi[p][1] = *reinterpret_cast<const f32x4_t *>(other + 4);
+        if (n.col_scales) cs[p] = *reinterpret_cast<const u32x4_t *>(n.col_scales + at);
+      }
+      w[p] = *reinterpret_cast<const u32x4_t *>(n.weight + at);
+    }
+  }
+
+  // the normalised row to lds + kNormSums, the waves' sums of squares in front of it
+  __device__ __forceinline__ void finish(const RowNorm &n, int K, uint8_t *lds, bool store) {
+    float *const sums = reinterpret_cast<float *>(lds);
+    const auto low = [](uint32_t v) { return __builtin_bit_cast(float, v << 16); };
+    const auto high = [](uint32_t v) { return __builtin_bit_cast(float, v & 0xFFFF0000u); };
+#pragma unroll
+    for (int p = 0; p < kNormPieces; ++p) {
+      const int i = p * kNormPiece + static_cast<int>(threadIdx.x) * 8;
+      float ss = 0.f;
+      if (K > p * kNormPiece) {
+        if (n.partials) {
+          f32x4_t a = lo[p][0], b = hi[p][0];
+          if (n.slices > 1) a += lo[p][1], b += hi[p][1];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            float t0 = j < 2 ? a[2 * j] : b[2 * j - 4], t1 = j < 2 ? a[2 * j + 1] : b[2 * j - 3];
+            if (n.col_scales) t0 = bf16_round(t0) * low(cs[p][j]), t1 = bf16_round(t1) * high(cs[p][j]);
+            x[p][j] = f32x2_to_bf16_rne(low(x[p][j]) + bf16_round(t0), high(x[p][j]) + bf16_round(t1));
+          }
+          if (store && i < K) *reinterpret_cast<u32x4_t *>(n.h_out + i) = x[p];
+        }
+        if (i < K) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float h0 = low(x[p][j]), h1 = high(x[p][j]);
+            ss = __builtin_fmaf(h0, h0, ss);
+            ss = __builtin_fmaf(h1, h1, ss);
+          }
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
+      }
+      if ((threadIdx.x & 63) == 0) sums[p * kWaves + (threadIdx.x >> 6)] = ss;
+    }
+    lds_barrier();
+    float ss = 0.f;
+#pragma unroll
+    for (int q = 0; q < kNormPieces * kWaves; ++q) ss += sums[q];
+    const float inv = rsqrtf(ss / static_cast<float>(K) + n.eps);
+#pragma unroll
+    for (int p = 0; p < kNormPieces; ++p) {
+      const int i = p * kNormPiece + static_cast<int>(threadIdx.x) * 8;
+      if (i >= K) break;
+      u32x4_t o;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t v = f32x2_to_bf16_rne(low(x[p][j]) * inv, high(x[p][j]) * inv);
+        o[j] = f32x2_to_bf16_rne(low(v) * low(w[p][j]), high(v) * high(w[p][j]));
+      }
+      *reinterpret_cast<u32x4_t *>(lds + kNormSums + static_cast<uint32_t>(i) * 2) = o;
+    }
+    lds_barrier();
+  }
+};
+
 // Epi: struct with kGate (two matrices, T / 2 tiles of each), kHalves (acc and acc2 are the sums over the two halves of K), Args, and per
 // unit a state: load(args, n, N) issues what it needs early, finish(args, acc, acc2, m0, M, n, N) stores rows m0 .. m0 + 3 of column n.
 // XR: rows of x in a tile that can be present (8: M <= 8, one load per unit of x instead of two).
-template <typename W, int MT, int XR, int T, typename Epi>
-__global__ __launch_bounds__(64 * kWaves) void stream_mm_kernel(const Args a, const typename Epi::Args ea) {
+// Norm: NoNorm, or RowNorm, which takes the place of a.x; the normalised row stands behind the rings, and units are weights only.
+template <typename W, int MT, int XR, int T, typename Epi, typename Norm>
+__global__ __launch_bounds__(64 * kWaves) void stream_mm_kernel(const Args a, const typename Epi::Args ea, const Norm norm) {
+  constexpr bool kNorm = std::is_same<Norm, RowNorm>::value;
+  static_assert(!kNorm || (MT == 1 && W::kXUnits == 2), "a row in front of 8-bit weights");
   static_assert(T * MT <= kMaxUnits && (!Epi::kGate || T % 2 == 0), "shape");
   constexpr int TC = Epi::kGate ? T / 2 : T;
-  constexpr int XN = MT * W::kXUnits, U = XN + T;        // units of a step: activations first
+  constexpr int XN = kNorm ? 0 : MT * W::kXUnits, U = XN + T;  // units of a step: activations first
   constexpr int kAhead = (kRing + U - 1) / U;             // steps that the ring's units reach into, at most
   constexpr int kLate = kAhead * U - kRing;               // units of the last kAhead steps that are issued while those run
   constexpr int kUnits = TC * MT, kPerWave = (kUnits + kWaves - 1) / kWaves;
   constexpr int kRingBytes = kWaves * kRing * kUnitBytes, kRedBytes = kWaves * T * MT * 1024;
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[kRingBytes > kRedBytes ? kRingBytes : kRedBytes];
+  constexpr int kLoopBytes = kRingBytes > kRedBytes ? kRingBytes : kRedBytes;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kLoopBytes + (kNorm ? kNormBytes : 0)];
 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, b = lane >> 4;
@@ -122,7 +224,8 @@ __global__ __launch_bounds__(64 * kWaves) void stream_mm_kernel(const Args a, co
     const uint32_t o0 = (16u * tile + r8) * pitch + piece0, o1 = (16u * tile + 8u + r8) * pitch + piece1;
     const __amdgpu_buffer_rsrc_t rs = is_x ? x_rsrc : (t < TC ? w_rsrc : w2_rsrc);
     // (at_k >= pitch: the second unit of activations of a last step of 64 bytes of weights or less)
-    const bool in0 = at_k < pitch && piece0 < left, in1 = at_k < pitch && piece1 < left;
+    bool in0 = at_k < pitch && piece0 < left, in1 = at_k < pitch && piece1 < left;
+    if (kNorm) in0 &= s < nloc, in1 &= s < nloc;  // (issued without a branch at the start, so that the waits for the row can count them)
     if (is_x) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)(ring + at), 16, in0 ? o0 : 0x80000000u, at_k, 0, 0);
       if (kXLoads == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void *)(ring + at + 1024), 16, in1 ? o1 : 0x80000000u, at_k, 0, 0);
@@ -167,9 +270,25 @@ __global__ __launch_bounds__(64 * kWaves) void stream_mm_kernel(const Args a, co
   };
   const auto next = [](uint32_t at) { return at == (kRing - 1) * kUnitBytes ? 0u : at + kUnitBytes; };
 
+  [[maybe_unused]] NormLoads row_in;
+  if constexpr (kNorm) row_in.request(norm, a.K);
 #pragma unroll
   for (int q = 0; q < kRing; ++q)
-    if (q / U < nloc) issue(q % U, q / U, q * kUnitBytes);
+    if (kNorm || q / U < nloc) issue(q % U, q / U, q * kUnitBytes);
+  if constexpr (kNorm) {
+    __builtin_amdgcn_sched_barrier(0);
+    row_in.finish(norm, a.K, lds + kLoopBytes, blockIdx.x == 0 && blockIdx.y == 0);
+  }
+  // the activations of step s, where they stand behind the rings
+  const auto take_x = [&](int s) {
+    if constexpr (kNorm) {
+      const int turned = s + turn, step = s0 + (turned < nloc ? turned : turned - nloc);
+      const uint32_t row = kLoopBytes + kNormSums, at_k = static_cast<uint32_t>(step) * 256u;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)  // every lane column holds it; what the others give is not stored
+        xf[0][i] = *reinterpret_cast<const bf16x8_t *>(lds + row + at_k + 128u * (i >> 1) + (2u * b + (i & 1)) * 16u);
+    }
+  };
   Epi epi[kPerWave];
 #pragma unroll
   for (int i = 0; i < kPerWave; ++i) {
@@ -181,6 +300,7 @@ __global__ __launch_bounds__(64 * kWaves) void stream_mm_kernel(const Args a, co
   int s = 0;
 #pragma unroll 1
   for (; s < nloc - kAhead; ++s) {
+    take_x(s);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       wait_loads(behind(u));  // (loads of the epilogue only make it wait longer)
@@ -191,6 +311,7 @@ __global__ __launch_bounds__(64 * kWaves) void stream_mm_kernel(const Args a, co
   }
   // the last steps: what is left to issue, then nothing more is on its way than what they need
   if (s < nloc && nloc >= kAhead) {
+    take_x(s);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (u < kLate) wait_loads(behind(u));
@@ -204,12 +325,14 @@ __global__ __launch_bounds__(64 * kWaves) void stream_mm_kernel(const Args a, co
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
 #pragma unroll 1
-  for (; s < nloc; ++s)
+  for (; s < nloc; ++s) {
+    take_x(s);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       use(u, at);
       at = next(at);
     }
+  }
 
   lds_barrier();  // the rings become the meeting place
   f32x4_t *const red = reinterpret_cast<f32x4_t *>(lds);
@@ -256,27 +379,27 @@ inline int pick_tiles(int M, int N, int K, int slices = 1) {
   return best;
 }
 
-template <typename W, typename Epi, int MT, int XR, int T>
-int launch(const Args &a, const typename Epi::Args &ea, int slices, hipStream_t stream) {
+template <typename W, typename Epi, int MT, int XR, int T, typename Norm>
+int launch(const Args &a, const typename Epi::Args &ea, int slices, hipStream_t stream, const Norm &norm) {
   if constexpr (T * MT > kMaxUnits || (Epi::kGate && T % 2)) {
     return E2H_ERR_BAD_SHAPE;
   } else {
     constexpr int TC = Epi::kGate ? T / 2 : T;
     const int tiles = (a.N + 15) / 16;
-    hipLaunchKernelGGL((stream_mm_kernel<W, MT, XR, T, Epi>), dim3((tiles + TC - 1) / TC, slices), dim3(64 * kWaves), 0, stream, a, ea);
+    hipLaunchKernelGGL((stream_mm_kernel<W, MT, XR, T, Epi, Norm>), dim3((tiles + TC - 1) / TC, slices), dim3(64 * kWaves), 0, stream, a, ea, norm);
     return launch_status();
   }
 }
 
-template <typename W, typename Epi, int MT, int XR>
-int launch_rows(const Args &a, const typename Epi::Args &ea, int t, int slices, hipStream_t stream) {
+template <typename W, typename Epi, int MT, int XR, typename Norm = NoNorm>
+int launch_rows(const Args &a, const typename Epi::Args &ea, int t, int slices, hipStream_t stream, const Norm &norm = Norm{}) {
   switch (t) {
-    case 1: return launch<W, Epi, MT, XR, 1>(a, ea, slices, stream);
-    case 2: return launch<W, Epi, MT, XR, 2>(a, ea, slices, stream);
-    case 3: return launch<W, Epi, MT, XR, 3>(a, ea, slices, stream);
-    case 4: return launch<W, Epi, MT, XR, 4>(a, ea, slices, stream);
-    case 6: return launch<W, Epi, MT, XR, 6>(a, ea, slices, stream);
-    case 8: return launch<W, Epi, MT, XR, 8>(a, ea, slices, stream);
+    case 1: return launch<W, Epi, MT, XR, 1>(a, ea, slices, stream, norm);
+    case 2: return launch<W, Epi, MT, XR, 2>(a, ea, slices, stream, norm);
+    case 3: return launch<W, Epi, MT, XR, 3>(a, ea, slices, stream, norm);
+    case 4: return launch<W, Epi, MT, XR, 4>(a, ea, slices, stream, norm);
+    case 6: return launch<W, Epi, MT, XR, 6>(a, ea, slices, stream, norm);
+    case 8: return launch<W, Epi, MT, XR, 8>(a, ea, slices, stream, norm);
     default: return E2H_ERR_BAD_SHAPE;
   }
 }
@@ -296,6 +419,12 @@ int run(const Args &a, const typename Epi::Args &ea, hipStream_t stream, int sli
   if (a.M <= 16) return launch_rows<W, Epi, 1, 16>(a, ea, t, slices, stream);
   if (a.M <= 32) return launch_rows<W, Epi, 2, 16>(a, ea, t, slices, stream);
   return launch_rows<W, Epi, 4, 16>(a, ea, t, slices, stream);
+}
+
+// the same over a row that a norm forms first (norm_fits)
+template <typename W, typename Epi>
+int run_norm(const Args &a, const typename Epi::Args &ea, const RowNorm &norm, hipStream_t stream) {
+  return launch_rows<W, Epi, 1, 8>(a, ea, pick_tiles<W, Epi::kGate>(a.M, a.N, a.K), 1, stream, norm);
 }
 
 }  // namespace stream

@@ -343,6 +343,8 @@ class TransformerBlock(nn.Module):
     def forward_deferred(self, x: Tensor, delta: Optional[Tensor], input_pos, freqs_cis, mask, fully_causal: bool = False):
         """Fused-path variant: `delta` is the previous block's feed-forward output that has not been added to the
         residual stream yet; the add is folded into this block's first norm.  Returns (h, this block's pending delta)."""
+        if not fully_causal and x.shape[1] == 1 and self._norms_fold(x, delta):
+            return self._forward_folded(x, delta, input_pos)
         if delta is None:
             normed = ops.rmsnorm(x, self.attention_norm.weight, self.attention_norm.eps)
         else:
@@ -350,6 +352,31 @@ class TransformerBlock(nn.Module):
         attn = self.attention(normed, freqs_cis, mask, input_pos, fully_causal, defer_output=DEFER_SPLIT_K)
         h, normed2 = ops.add_rmsnorm(x, attn, self.ffn_norm.weight, self.ffn_norm.eps)
         return h, self.feed_forward(normed2, defer_output=DEFER_SPLIT_K)
+
+
+    def _norms_fold(self, x: Tensor, delta) -> bool:
+        """True for the single-token step of one sequence through an int8 model whose modules nobody watches: the products behind the norms form their row themselves."""
+        att, ff = self.attention, self.feed_forward
+        if x.shape[0] != 1 or not (FUSE_ROPE_PROJECTION and FUSE_GATE and DEFER_SPLIT_K and type(att) is Attention and type(ff) is FeedForward
+                                  and type(self.attention_norm) is RMSNorm and type(self.ffn_norm) is RMSNorm and att.can_fuse_decode(x, False)):
+            return False
+        lins = (att.wqkv, att.wo, ff.w1, ff.w3, ff.w2)
+        if not all(type(m) is WeightOnlyInt8Linear for m in lins) or not all(unwatched(m) for m in (self.attention_norm, self.ffn_norm, att, ff, *lins)):
+            return False
+        rows, cache = x.shape[0], att.kv_cache.k_cache
+        return (ops.int8_rope_kv_supported(x, att.wqkv, att.freqs_table, cache) and ops.int8_gate_supported(x, ff.w1, ff.w3)
+                and ops.int8_norm_fits(x, self.attention_norm.weight, delta, att.wqkv) and ops.int8_norm_fits(x, self.ffn_norm.weight, None, ff.w1, ff.w3)
+                and att.wo.scales.dtype == torch.bfloat16 and att.wo.scales.is_contiguous() and att.wo.scales.numel() == x.shape[-1] and ops.int8_partial_slices(rows, att.wo) in (1, 2))
+
+    def _forward_folded(self, x: Tensor, delta, input_pos: Tensor):
+        att, ff, a, f = self.attention, self.feed_forward, self.attention_norm, self.ffn_norm
+        bsz = x.shape[0]
+        x, q = ops.int8_norm_mm_rope_kv(x, delta, a.weight, a.eps, att.wqkv.weight, att.wqkv.scales, att.freqs_table, att.kv_cache.k_cache, att.kv_cache.v_cache,
+                                        input_pos, att.n_head, att.n_local_heads, att.head_dim)
+        y = ops.decode_attention(q, att.kv_cache.k_cache, att.kv_cache.v_cache, input_pos, att.left_pad_mask_pos).view(bsz, att.dim)
+        term = ops.int8_mm_partials(y, att.wo.weight, att.wo.scales, ops.int8_partial_slices(bsz, att.wo))
+        h, g = ops.int8_norm_mm_silu_gate(x, term, f.weight, f.eps, ff.w1.weight, ff.w1.scales, ff.w3.weight, ff.w3.scales)
+        return h, _project_deferred(ff.w2, g, x.shape[:-1])
 
 
 def _staged_block_supported(blk: "TransformerBlock", rows: int) -> bool:
@@ -512,6 +539,10 @@ class Transformer(nn.Module):
             delta = None
             for layer in self.layers:
                 x, delta = layer.forward_deferred(x, delta, input_pos, freqs_cis, mask, fully_causal)
+            out = self.output
+            if (fused_step and x.shape[0] == 1 and type(out) is WeightOnlyInt8Linear and type(self.norm) is RMSNorm and unwatched(out) and unwatched(self.norm)
+                    and ops.int8_norm_fits(x, self.norm.weight, delta, out)):
+                return ops.int8_norm_mm(x, delta, self.norm.weight, self.norm.eps, out.weight, out.scales)[1].view(x.shape[0], 1, -1)
             _, normed = ops.add_rmsnorm(x, delta, self.norm.weight, self.norm.eps)
             return self.output(normed)
         for layer in self.layers:

@@ -735,6 +735,72 @@ def int8_mm_rope_kv(x, q_weight, scales, freqs_cis, k_cache, v_cache, input_pos,
     return q
 
 
+def int8_norm_fits(x, weight, delta, *mods):
+    """True where the products of `mods` (WeightOnlyInt8Linear) can take the residual add and RMSNorm of their input x into their own launch: x one row of
+    bfloat16, delta None or the ScaledPartials of the linear before."""
+    k = x.shape[-1]
+    if not (x.is_contiguous() and _int8_fusable(x, *mods) and weight.dtype == torch.bfloat16 and weight.is_contiguous() and weight.numel() == k):
+        return False
+    if delta is not None and not (isinstance(delta, ScaledPartials) and delta.partials.dtype == torch.float32 and delta.partials.is_contiguous()
+                                  and delta.partials.shape[0] <= 2 and tuple(delta.partials.shape[1:]) == (x.numel() // k, k)
+                                  and delta.scales.dtype == torch.bfloat16 and delta.scales.is_contiguous() and delta.scales.numel() == k):
+        return False
+    return all(m.weight.is_contiguous() and m.scales.is_contiguous() and _lib.load().e2h_int8_norm_mm_supported(x.numel() // k, m.weight.shape[0], k) for m in mods)
+
+
+def _row_norm(x, delta, weight, eps):
+    """-> (the norm's arguments, h): h is x itself where nothing is added."""
+    if delta is None:
+        return _lib.RowNorm(_ptr(x), None, None, _ptr(weight), None, 0, float(eps)), x
+    h = torch.empty_like(x)
+    return _lib.RowNorm(_ptr(x), _ptr(delta.partials), _ptr(delta.scales), _ptr(weight), _ptr(h), delta.partials.shape[0], float(eps)), h
+
+
+def int8_norm_mm(x, delta, weight, eps, q, scales):
+    """add_rmsnorm (rmsnorm where delta is None) and int8_mm of its rows in one launch (int8_norm_fits) -> (h, y [rows, N])."""
+    _need_gpu(x, weight, q, scales)
+    n, k = q.shape
+    rows = x.numel() // k
+    norm, h = _row_norm(x, delta, weight, eps)
+    y = torch.empty((rows, n), dtype=torch.bfloat16, device=x.device)
+    _lib.check(_lib_for(x).e2h_int8_norm_mm(norm, _ptr(q), _ptr(scales), _ptr(y), rows, n, k, _stream(x)), "e2h_int8_norm_mm")
+    return h, y
+
+
+def int8_norm_mm_silu_gate(x, delta, weight, eps, q_gate, scales_gate, q_up, scales_up):
+    """add_rmsnorm and int8_mm_silu_gate of its rows in one launch (int8_norm_fits) -> (h, y [rows, N])."""
+    _need_gpu(x, weight, q_gate, scales_gate, q_up, scales_up)
+    n, k = q_gate.shape
+    if q_up.shape != q_gate.shape or scales_gate.numel() != n or scales_up.numel() != n:
+        raise RuntimeError("int8_norm_mm_silu_gate: shapes of the two linears do not match")
+    rows = x.numel() // k
+    norm, h = _row_norm(x, delta, weight, eps)
+    y = torch.empty((rows, n), dtype=torch.bfloat16, device=x.device)
+    _lib.check(_lib_for(x).e2h_int8_norm_mm_silu_gate(norm, _ptr(q_gate), _ptr(scales_gate), _ptr(q_up), _ptr(scales_up), _ptr(y), rows, n, k, _stream(x)),
+               "e2h_int8_norm_mm_silu_gate")
+    return h, y
+
+
+def int8_norm_mm_rope_kv(x, delta, weight, eps, q_weight, scales, freqs_cis, k_cache, v_cache, input_pos, n_head, n_kv_head, head_dim):
+    """add_rmsnorm and int8_mm_rope_kv of its rows in one launch (int8_norm_fits) -> (h, q [rows, H, D])."""
+    _need_gpu(x, weight, q_weight, scales, freqs_cis, k_cache, v_cache, input_pos)
+    assert input_pos.dtype == torch.int64 and input_pos.numel() >= 1 and freqs_cis.dtype == torch.bfloat16 and k_cache.dtype == torch.bfloat16 and v_cache.dtype == torch.bfloat16
+    assert k_cache.is_contiguous() and v_cache.is_contiguous() and freqs_cis.is_contiguous()
+    n, k = q_weight.shape
+    rows = x.numel() // k
+    if n != (n_head + 2 * n_kv_head) * head_dim or scales.numel() != n:
+        raise RuntimeError(f"int8_norm_mm_rope_kv: weight is [{n}, {k}], expected {(n_head + 2 * n_kv_head) * head_dim} rows")
+    if k_cache.shape[0] < rows or k_cache.shape[1] != n_kv_head or k_cache.shape[3] != head_dim or v_cache.shape != k_cache.shape:
+        raise RuntimeError("int8_norm_mm_rope_kv: caches must be [>= B, Hkv, S, D]")
+    if freqs_cis.shape[0] < k_cache.shape[2] or tuple(freqs_cis.shape[1:]) != (head_dim // 2, 2):
+        raise RuntimeError("int8_norm_mm_rope_kv: freqs_cis must be [>= S, D/2, 2]")
+    norm, h = _row_norm(x, delta, weight, eps)
+    q = torch.empty((rows, n_head, head_dim), dtype=torch.bfloat16, device=x.device)
+    _lib.check(_lib_for(x).e2h_int8_norm_mm_rope_kv(norm, _ptr(q_weight), _ptr(scales), _ptr(freqs_cis), _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(input_pos), rows,
+                                                    n_head, n_kv_head, head_dim, k_cache.shape[2], k, _stream(x)), "e2h_int8_norm_mm_rope_kv")
+    return h, q
+
+
 def sample_top_k(logits, q, temperature=1.0, top_k=None):
     """logits bf16 [B, V] (rows may be strided), q float32 [B, V] of Exp(1) draws -> (idx int32 [B, 1], probs float32 [B, V]):
     softmax(top-k-masked logits / max(temperature, 1e-5)) and argmax(probs / q), in one launch."""

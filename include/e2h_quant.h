@@ -277,6 +277,26 @@ int e2h_add_rmsnorm_partials(const uint16_t *x, const float *partials, int slice
                              const uint16_t *weight, uint16_t *h_out, uint16_t *y, int64_t rows, int64_t dim, float eps,
                              void *stream);
 
+/* The int8 products of a decode step of one row with the residual add and RMSNorm in front of them in the same launch: what e2h_add_rmsnorm_partials (partials
+ * float32 [slices, 1, k], slices 1 or 2, col_scales as there) or e2h_rmsnorm (partials NULL, h_out unused) followed by e2h_int8_mm, e2h_int8_mm_silu_gate or
+ * e2h_int8_mm_rope_kv give.  h_out must not overlap x.  Shapes for which the first function returns 1: m = 1, k % 128 == 0, k <= 8192. */
+typedef struct {
+  const uint16_t *x;
+  const float *partials;
+  const uint16_t *col_scales;
+  const uint16_t *weight;
+  uint16_t *h_out;
+  int slices;
+  float eps;
+} e2h_row_norm;
+int e2h_int8_norm_mm_supported(int64_t m, int64_t n, int64_t k);
+int e2h_int8_norm_mm(const e2h_row_norm *norm, const int8_t *q, const uint16_t *scales, uint16_t *y, int64_t m, int64_t n, int64_t k, void *stream);
+int e2h_int8_norm_mm_silu_gate(const e2h_row_norm *norm, const int8_t *q_gate, const uint16_t *scales_gate, const int8_t *q_up, const uint16_t *scales_up, uint16_t *y,
+                               int64_t m, int64_t n, int64_t k, void *stream);
+int e2h_int8_norm_mm_rope_kv(const e2h_row_norm *norm, const int8_t *q, const uint16_t *scales, const uint16_t *freqs_cis, uint16_t *q_out, uint16_t *k_cache,
+                             uint16_t *v_cache, const int64_t *input_pos, int64_t batch, int64_t n_head, int64_t n_kv_head, int64_t head_dim, int64_t cache_len, int64_t k,
+                             void *stream);
+
 /* ------------------------------------------------------------------------------------------------
  * Decode batches on staged activations.  The single-token steps of the decode loop (reference
  * inference_generate.py:123-157, decode_one_token :110-120) give every quantized linear at most a few dozen rows;

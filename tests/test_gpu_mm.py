@@ -731,3 +731,65 @@ def test_int8_rope_kv_matches_two_kernel_path(bsz, n_head, n_kv, d, k):
     kc3, vc3 = kc0.clone(), vc0.clone()
     ops.int8_mm_rope_kv(x, q_d, s_d, freqs, kc3, vc3, torch.tensor([s_max], device=DEV), n_head, n_kv, d)
     assert torch.equal(kc3, kc0) and torch.equal(vc3, vc0)
+
+
+@pytest.mark.parametrize("term", ["none", "one slice", "two slices"])
+@pytest.mark.parametrize("n,k", [(40, 128), (304, 2048), (2056, 3072), (4096, 4096), (1000, 5120), (96, 8192)])
+def test_int8_products_form_their_row_of_a_norm_as_the_norm_does(n, k, term):
+    """One row, pieces of the row from a part of one to two: bit for bit the norm's launch and the product's, where both add a row's squares by the same pieces (3072: one thread adds two of
+    them there, so the reciprocal root may differ in its last places, and a bfloat16 of the row by one step: 2^-8 of it, half the bound beside the outputs' own rounding)."""
+    q, s, q_d, s_d = _int8_case(n, k, seed=n + k)
+    _, _, q2_d, s2_d = _int8_case(n, k, seed=n + k + 1)
+    x = randn_bf16((1, k), seed=3).to(DEV)
+    w = (1.0 + randn_bf16((k,), std=0.1, seed=4).float()).to(torch.bfloat16).to(DEV)
+    delta = None
+    if term != "none":
+        gen = torch.Generator().manual_seed(k)
+        sums = torch.randn((1 + (term == "two slices"), 1, k), generator=gen) * 40
+        delta = ops.ScaledPartials(sums.to(DEV), randn_bf16((k,), std=0.02, seed=5).to(DEV))
+    h, normed = (x, ops.rmsnorm(x, w, 1e-5)) if delta is None else ops.add_rmsnorm(x, delta, w, 1e-5)
+
+    class Linear:
+        def __init__(self, weight, scales):
+            self.weight, self.scales = weight, scales
+
+    assert ops.int8_norm_fits(x, w, delta, Linear(q_d, s_d)) and not ops.int8_norm_fits(x.expand(2, k).contiguous(), w, None, Linear(q_d, s_d))
+    h1, y = ops.int8_norm_mm(x, delta, w, 1e-5, q_d, s_d)
+    h2, g = ops.int8_norm_mm_silu_gate(x, delta, w, 1e-5, q_d, s_d, q2_d, s2_d)
+    assert torch.equal(h1, h) and torch.equal(h2, h)
+    y_ref, g_ref = ops.int8_mm_direct(normed, q_d, s_d), ops.int8_mm_silu_gate(normed, q_d, s_d, q2_d, s2_d)
+    if k != 3072:
+        assert torch.equal(y, y_ref) and torch.equal(g, g_ref)
+    for got, ref in ((y, y_ref), (g, g_ref)):
+        assert qo.normwise_rel_err(bf16_to_np(got), bf16_to_np(ref)) <= 2.0 ** -7
+    err = qo.normwise_rel_err(bf16_to_np(y), qo.int8_linear_fp32(bf16_to_np(normed), q, s))
+    assert err <= TOL, err
+
+
+def test_int8_step_of_one_sequence_is_that_of_separate_norms():
+    """The folded step against the one that a watched module takes, bit for bit, and its caches."""
+    from easy_to_hard_amd.model import ModelArgs, random_quantized_transformer
+
+    cfg = ModelArgs(block_size=64, vocab_size=512, n_layer=3, n_head=4, n_local_heads=2, dim=256, intermediate_size=512)
+    model = random_quantized_transformer(cfg, "int8", device=DEV)
+    model.setup_caches(1, 64)
+    ids, pos = torch.tensor([[17]], device=DEV), torch.tensor([5], device=DEV)
+
+    def caches():
+        return [c.clone() for b in model.layers for c in (b.attention.kv_cache.k_cache, b.attention.kv_cache.v_cache)]
+
+    def step():
+        for b in model.layers:
+            b.attention.kv_cache.k_cache.normal_(generator=torch.Generator(device=DEV).manual_seed(1))
+            b.attention.kv_cache.v_cache.normal_(generator=torch.Generator(device=DEV).manual_seed(2))
+        with torch.no_grad():
+            return model(ids, pos), caches()
+
+    calls = []
+    folded, kept = step()
+    hooks = [m.register_forward_hook(lambda *_: calls.append(1)) for b in model.layers for m in (b.attention, b.feed_forward)] + [model.output.register_forward_hook(lambda *_: calls.append(1))]
+    apart, kept_apart = step()
+    for h in hooks:
+        h.remove()
+    assert len(calls) == 7  # a watched module is called
+    assert torch.equal(folded, apart) and all(torch.equal(a, b) for a, b in zip(kept, kept_apart))
