@@ -27,7 +27,6 @@ namespace e2h {
 namespace gemm256 {
 
 constexpr int kSide = 256, kLeastK = 192;
-constexpr int kStores = 32;  // vector stores of a wave per tile, exactly (see below)
 constexpr uint32_t kUnit = 256 * 128, kRing = 5 * kUnit;
 constexpr uint32_t kNowhere = 0xFFFFFFF0u;  // an offset past every buffer: the store is dropped
 
@@ -48,6 +47,7 @@ __device__ __forceinline__ void mma(f32x4_t &d, u32x4_t a, u32x4_t b) {
 // P names the tiles and what surrounds them.  P::Tile holds uniform values.
 //   static constexpr bool kHalves             whether tiles may have 128 rows and fewer, bool half(Tile): whether this one does; only the products of those are
 //                                             formed then, and the rows 32 j + 16 wm + r of a tile are wave wm's instead of 128 wm + 16 j + r
+//   static constexpr bool kPairs              whether the upper 64 columns of a wave's 128 belong to the lower ones, as up to gate
 //   bool first(Tile &), bool next(Tile &)     the workgroup's tiles, false: no more
 //   int chunks()                              K / 64
 //   rsrc x_rsrc(Tile), w_rsrc(Tile)           the operands
@@ -55,12 +55,14 @@ __device__ __forceinline__ void mma(f32x4_t &d, u32x4_t a, u32x4_t b) {
 //   uint32_t x_at(Tile, Fetch, i, row), w_at(Tile, col)   byte offset of row (0 .. 255, the i-th of this lane) and column of the tile, inside the buffer
 //   Dest, dest(Tile, row of the lane's first output, col, Dest &)   what store needs from memory
 //   store(Tile, Dest, j, p, row, col, v)      stores the eight outputs (row, col .. col + 7), one vector store in every case
+//   store(Tile, Dest, j, p, row, col, v, u)   with kPairs: v, and u of the columns 64 further on
 template <bool F16, class P>
 __device__ __forceinline__ void walk(P &p, uint8_t *lds) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave & 1, wn = wave >> 1, chunks = p.chunks();
   // a wave's 16-row blocks: neighbours, or every second one where tiles may be half empty
   constexpr int kXWave = P::kHalves ? 16 : 128, kXStep = P::kHalves ? 32 : 16;
+  constexpr int kStores = P::kPairs ? 16 : 32;  // vector stores of a wave per tile, exactly (see below)
   typename P::Tile cur, nxt;
   if (!p.first(cur)) return;  // uniform, before any barrier
 
@@ -77,7 +79,7 @@ __device__ __forceinline__ void walk(P &p, uint8_t *lds) {
   auto aim_w = [&](const typename P::Tile &t) {
     wr = p.w_rsrc(t);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) wsrc[i] = p.w_at(t, 8 * (wave + 4 * i) + (lane >> 3)) + wpiece;
+    for (int i = 0; i < 8; ++i) wsrc[i] = p.w_at(t, P::kPairs ? 32 * i + ((8 * wave + (lane >> 3)) & 31) : 8 * (wave + 4 * i) + (lane >> 3)) + wpiece;  // (the same: pairs want bit 6 a constant)
   };
   auto load_x = [&](int chunk, uint32_t unit, int i) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void_t *)(lds + unit + (wave + 4 * i) * 1024), 16, xsrc[i], static_cast<uint32_t>(chunk) * 128, 0, 0);
@@ -178,14 +180,22 @@ __device__ __forceinline__ void walk(P &p, uint8_t *lds) {
 #pragma unroll
       for (int j = 0; j < 8; ++j)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < (P::kPairs ? 2 : 4); ++q) {
           float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // rows that are not there: stored nowhere, but counted
           if (j < decltype(blocks)::value) {
             asm volatile("" : "+a"(acc[2 * q][j]), "+a"(acc[2 * q + 1][j]));  // read here: all 256 at once would not fit
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = acc[2 * q + (e >> 2)][j][e & 3];
           }
-          p.store(cur, dest, j, q, row + kXStep * j, col + 32 * q, v);
+          if constexpr (P::kPairs) {
+            float u[8];
+            asm volatile("" : "+a"(acc[2 * q + 4][j]), "+a"(acc[2 * q + 5][j]));
+#pragma unroll
+            for (int e = 0; e < 8; ++e) u[e] = acc[2 * q + 4 + (e >> 2)][j][e & 3];
+            p.store(cur, dest, j, q, row + kXStep * j, col + 32 * q, v, u);
+          } else {
+            p.store(cur, dest, j, q, row + kXStep * j, col + 32 * q, v);
+          }
           __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -208,6 +218,66 @@ __device__ __forceinline__ void walk(P &p, uint8_t *lds) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // loads past the last tile must land before the workgroup gives its LDS away
 }
 #endif
+
+// The tiles of one plain product, dealt to the XCDs in contiguous runs of equal length: panels of eight column blocks, all row
+// blocks of a panel after each other, so that the 32 tiles at work on an XCD share four row blocks and eight column blocks.
+// kCols: columns of y per tile, 256, or 128 of a pair of products (two rows of w each).
+template <int kCols = kSide>
+struct PlainWalk {
+  static constexpr bool kHalves = false, kPairs = kCols != kSide;
+  static constexpr int kPanel = 8;
+  struct Tile {
+    int rb, cb;
+  };
+  const uint16_t *x, *w;
+  uint16_t *y;
+  int M, N, K, t, end, stride;
+
+  __device__ __forceinline__ PlainWalk(const uint16_t *x_, const uint16_t *w_, uint16_t *y_, int M_, int N_, int K_) : x(x_), w(w_), y(y_), M(M_), N(N_), K(K_) {
+    const int64_t total = static_cast<int64_t>((M + 255) / 256) * ((N + kCols - 1) / kCols);
+    const int xcd = blockIdx.x & 7;
+    stride = static_cast<int>(gridDim.x >> 3);
+    end = static_cast<int>(total * (xcd + 1) / 8);
+    t = static_cast<int>(total * xcd / 8) + static_cast<int>(blockIdx.x >> 3) - stride;
+  }
+  __device__ __forceinline__ bool next(Tile &tile) {
+    t += stride;
+    if (t >= end) return false;
+    const int R = (M + 255) / 256, C = (N + kCols - 1) / kCols, panel = t / (kPanel * R), at = t - panel * kPanel * R;
+    const int wide = C - panel * kPanel < kPanel ? C - panel * kPanel : kPanel;
+    tile.rb = at / wide;
+    tile.cb = panel * kPanel + at - tile.rb * wide;
+    return true;
+  }
+  __device__ __forceinline__ bool first(Tile &tile) { return next(tile); }
+  __device__ __forceinline__ int chunks() const { return K / 64; }
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t x_rsrc(const Tile &) const { return make_rsrc(x, static_cast<uint32_t>(static_cast<size_t>(M) * K * 2)); }
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t w_rsrc(const Tile &) const { return make_rsrc(w, static_cast<uint32_t>(static_cast<size_t>(N) * K * (kPairs ? 4 : 2))); }
+  // a tile's own rows of y: rows past M lie behind the buffer, where stores are dropped
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t y_rsrc(const Tile &tile) const {
+    const int rows = M - tile.rb * 256 < 256 ? M - tile.rb * 256 : 256;
+    return make_rsrc(y + static_cast<size_t>(tile.rb) * 256 * N, static_cast<uint32_t>(rows) * static_cast<uint32_t>(N) * 2);
+  }
+  struct Fetch {};
+  __device__ __forceinline__ void fetch(const Tile &, int, int, Fetch &) const {}
+  __device__ __forceinline__ uint32_t x_at(const Tile &tile, const Fetch &, int, int row) const {
+    const int m = tile.rb * 256 + row;
+    return static_cast<uint32_t>(m < M ? m : M - 1) * static_cast<uint32_t>(K) * 2;
+  }
+  // column of y that column `col` (0 .. 255) of the tile's product goes into; the second matrix' rows of a pair stand behind the first one's
+  __device__ __forceinline__ int out_col(const Tile &tile, int col) const { return tile.cb * kCols + (kPairs ? (col >> 7) * 64 + (col & 63) : col); }
+  __device__ __forceinline__ uint32_t w_at(const Tile &tile, int col) const {
+    const int n = out_col(tile, col);
+    return (static_cast<uint32_t>(n < N ? n : N - 1) + (kPairs && (col & 64) ? static_cast<uint32_t>(N) : 0u)) * static_cast<uint32_t>(K) * 2;
+  }
+  __device__ __forceinline__ uint32_t y_at(const Tile &tile, int row, int col) const {
+    const int n = out_col(tile, col);
+    return n < N ? (static_cast<uint32_t>(row) * static_cast<uint32_t>(N) + static_cast<uint32_t>(n)) * 2 : kNowhere;
+  }
+};
+
+// Workgroups of a walk over so many tiles: a CU each, an XCD's share alike.
+inline unsigned grid_of(int64_t tiles) { return static_cast<unsigned>(8 * (tiles < 256 ? (tiles + 7) / 8 : 32)); }
 
 }  // namespace gemm256
 }  // namespace e2h

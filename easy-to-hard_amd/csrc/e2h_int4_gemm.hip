@@ -643,11 +643,11 @@ int int4_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint
 }
 
 int int4_gemm_gate(const uint16_t *x, const int32_t *packed, const uint16_t *sz, const int32_t *packed2, const uint16_t *sz2, uint16_t *y, const float *xsum,
-                   int xsum_stride, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream) {
+                   int xsum_stride, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream, const int *run_if, const int *row_flag) {
   if (K % 128 != 0 || N % 8 != 0 || shape.slices != 1) return E2H_ERR_BAD_SHAPE;
   const int shared = groupsize == 256;
   const GemmArgs a = {x, reinterpret_cast<const uint32_t *>(packed), reinterpret_cast<const uint32_t *>(sz), reinterpret_cast<const uint32_t *>(packed2),
-                      reinterpret_cast<const uint32_t *>(sz2), y, nullptr, xsum, xsum_stride, M, N, K, 0, 0, shared, nullptr, nullptr};
+                      reinterpret_cast<const uint32_t *>(sz2), y, nullptr, xsum, xsum_stride, M, N, K, 0, 0, shared, run_if, row_flag};
   const int rc = launch_gemm<true>(a, shared ? 128 : groupsize, shape, stream);
   return rc != E2H_OK ? rc : launch_status();
 }
@@ -656,11 +656,13 @@ int int4_gemm_gate(const uint16_t *x, const int32_t *packed, const uint16_t *sz,
 
 namespace e2h {
 int64_t int4_unpacked_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int inner_k_tiles);
+int64_t int4_gate_unpacked_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int inner_k_tiles);
+int int4_unpacked_gate(const uint16_t *x, const int32_t *packed, const uint16_t *sz, const int32_t *packed2, const uint16_t *sz2, uint16_t *y, int M, int N, int K, int groupsize,
+                       void *scratch, hipStream_t stream);
 constexpr int kUnpackRows = 1024;  // from here on callers offer memory for unpacked operands
 
-// Group sums of x, the only scratch of a gated call, or 0 where two calls of the 32x32-tile kernel and a pass that multiplies are expected to be no slower or a form is asked for by an
-// option.  The launch of both matrices has twice the workgroups, spares one pass over x for its group sums, the two products' way to memory and back, and a launch.  Calls on unpacked
-// operands (e2h_unpacked_gemm.hip) stay with those.
+// Scratch of a gated call: for unpacked operands (int4_gate_unpacked_bytes) or the group sums of x; or 0 where two calls of the 32x32-tile kernel and a pass that multiplies are expected to be no slower or a form is asked for by an
+// option.  The launch of both matrices has twice the workgroups, spares one pass over x for its group sums, the two products' way to memory and back, and a launch.
 int64_t int4_gate_rows_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int inner_k_tiles) {
   if (inner_k_tiles != 8 || (groupsize != 32 && groupsize != 64 && groupsize != 128 && groupsize != 256)) return 0;
   if (M <= 64 || N < 8 || N % 8 != 0 || K < 128 || K % 128 != 0 || K % groupsize != 0 || M > INT32_MAX / 64 || N > INT32_MAX / 64 || K > INT32_MAX / 64) return 0;
@@ -671,6 +673,7 @@ int64_t int4_gate_rows_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int
   const Options &o = options();
   if (o.int4_no_gemm32 || o.int4_gemm_tile || o.int4_gemm32_min_rows || o.int4_no_xsum || o.int4_k_slices || o.int4_rows_per_wave || o.row_tiles) return 0;
   const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
+  if (const int64_t unpacked = int4_gate_unpacked_bytes(M, N, K, groupsize, inner_k_tiles)) return unpacked;
   if (M >= kUnpackRows && int4_unpacked_bytes(M, N, K, groupsize, inner_k_tiles) > 0) return 0;
   const double calls = 2 * int4_gemm_shape(m, n, k, G, int64_t{32} << 20).us + 3 + static_cast<double>(M) * static_cast<double>(N) * 6 / 5e6;  // the pass moves six bytes an output
   return 1.07 * int4_gemm_shape(m, 2 * n, k, G, 0).us < calls ? bytes : 0;
@@ -683,6 +686,7 @@ int64_t int4_gate_rows_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int
 // take up to 34 % more and none 2 % less.
 bool int4_gate_rows_pay(int64_t M, int64_t N, int64_t K, int groupsize, int inner_k_tiles) {
   if (int4_gate_rows_bytes(M, N, K, groupsize, inner_k_tiles) == 0) return false;
+  if (int4_gate_unpacked_bytes(M, N, K, groupsize, inner_k_tiles) > 0) return true;
   const int G = groupsize == 256 ? 128 : groupsize, m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
   double call = int4_gemm_shape(m, n, k, G, int64_t{32} << 20).us;
   if (groupsize == 256 || (M + 127) / 128 * ((N + 127) / 128) < 320) {  // as e2h_int4_mm chooses
@@ -715,6 +719,8 @@ extern "C" int e2h_int4_mm_silu_gate_rows(const uint16_t *x, const int32_t *pack
       (reinterpret_cast<uintptr_t>(y) & 1u))
     return E2H_ERR_MISALIGNED;
   const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k), G = groupsize == 256 ? 128 : groupsize, stride = (M + 63) / 64 * 64;
+  if (aligned16(y) && int4_gate_unpacked_bytes(m, n, k, groupsize, inner_k_tiles) > 0)
+    return int4_unpacked_gate(x, packed_gate, sz_gate, packed_up, sz_up, y, M, N, K, groupsize, scratch, static_cast<hipStream_t>(stream));
   float *xsum = static_cast<float *>(scratch);
   const int rc = launch_x_group_sums(x, xsum, M, K, stride, G, static_cast<hipStream_t>(stream));
   if (rc != E2H_OK) return rc;

@@ -119,7 +119,7 @@ double int4_rows_us(int M, int N, int K, int groupsize, int tiles);
 // y = silu(x w) * (x w2) of two matrices of one shape in one launch of that kernel, rounded as the two products and F.silu(a) * b would be; `shape` as
 // int4_gemm_shape gives it for the columns of both, with one slice.
 int int4_gemm_gate(const uint16_t *x, const int32_t *packed, const uint16_t *sz, const int32_t *packed2, const uint16_t *sz2, uint16_t *y, const float *xsum,
-                   int xsum_stride, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream);
+                   int xsum_stride, Int4GemmShape shape, int M, int N, int K, int groupsize, hipStream_t stream, const int *run_if = nullptr, const int *row_flag = nullptr);
 
 // Many-row int4 matmul, 256 x 256 outputs per workgroup, weights dequantized to bfloat16 on the way into the matrix
 // cores (e2h_int4_gemm128.hip); needs no scratch memory.

@@ -425,7 +425,7 @@ __global__ __launch_bounds__(256, 2) void expert_tiles_kernel(const Product p) {
 template <bool UP>
 struct ExpertWalk {
   typedef e2h::Tile Tile;
-  static constexpr bool kHalves = true;
+  static constexpr bool kHalves = true, kPairs = false;
   const Product &p;
   int t, end, stride;
   int begin, after;  // tiles before the present expert's first, and up to its last

@@ -52,60 +52,7 @@ __global__ __launch_bounds__(256) void unpack_int8_kernel(const int8_t *__restri
   reinterpret_cast<u32x4_t *>(w)[2 * i + 1] = out[1];
 }
 
-// The tiles of one plain product, dealt to the XCDs in contiguous runs of equal length: panels of eight column blocks, all row
-// blocks of a panel after each other, so that the 32 tiles at work on an XCD share four row blocks and eight column blocks.
-struct PlainWalk {
-  static constexpr bool kHalves = false;
-  static constexpr int kPanel = 8;
-  struct Tile {
-    int rb, cb;
-  };
-  const uint16_t *x, *w;
-  uint16_t *y;
-  int M, N, K, t, end, stride;
-
-  __device__ __forceinline__ PlainWalk(const uint16_t *x_, const uint16_t *w_, uint16_t *y_, int M_, int N_, int K_) : x(x_), w(w_), y(y_), M(M_), N(N_), K(K_) {
-    const int64_t total = static_cast<int64_t>((M + 255) / 256) * ((N + 255) / 256);
-    const int xcd = blockIdx.x & 7;
-    stride = static_cast<int>(gridDim.x >> 3);
-    end = static_cast<int>(total * (xcd + 1) / 8);
-    t = static_cast<int>(total * xcd / 8) + static_cast<int>(blockIdx.x >> 3) - stride;
-  }
-  __device__ __forceinline__ bool next(Tile &tile) {
-    t += stride;
-    if (t >= end) return false;
-    const int R = (M + 255) / 256, C = (N + 255) / 256, panel = t / (kPanel * R), at = t - panel * kPanel * R;
-    const int wide = C - panel * kPanel < kPanel ? C - panel * kPanel : kPanel;
-    tile.rb = at / wide;
-    tile.cb = panel * kPanel + at - tile.rb * wide;
-    return true;
-  }
-  __device__ __forceinline__ bool first(Tile &tile) { return next(tile); }
-  __device__ __forceinline__ int chunks() const { return K / 64; }
-  __device__ __forceinline__ __amdgpu_buffer_rsrc_t x_rsrc(const Tile &) const { return make_rsrc(x, static_cast<uint32_t>(static_cast<size_t>(M) * K * 2)); }
-  __device__ __forceinline__ __amdgpu_buffer_rsrc_t w_rsrc(const Tile &) const { return make_rsrc(w, static_cast<uint32_t>(static_cast<size_t>(N) * K * 2)); }
-  // a tile's own rows of y: rows past M lie behind the buffer, where stores are dropped
-  __device__ __forceinline__ __amdgpu_buffer_rsrc_t y_rsrc(const Tile &tile) const {
-    const int rows = M - tile.rb * 256 < 256 ? M - tile.rb * 256 : 256;
-    return make_rsrc(y + static_cast<size_t>(tile.rb) * 256 * N, static_cast<uint32_t>(rows) * static_cast<uint32_t>(N) * 2);
-  }
-  struct Fetch {};
-  __device__ __forceinline__ void fetch(const Tile &, int, int, Fetch &) const {}
-  __device__ __forceinline__ uint32_t x_at(const Tile &tile, const Fetch &, int, int row) const {
-    const int m = tile.rb * 256 + row;
-    return static_cast<uint32_t>(m < M ? m : M - 1) * static_cast<uint32_t>(K) * 2;
-  }
-  __device__ __forceinline__ uint32_t w_at(const Tile &tile, int col) const {
-    const int n = tile.cb * 256 + col;
-    return static_cast<uint32_t>(n < N ? n : N - 1) * static_cast<uint32_t>(K) * 2;
-  }
-  __device__ __forceinline__ uint32_t y_at(const Tile &tile, int row, int col) const {
-    const int n = tile.cb * 256 + col;
-    return n < N ? (static_cast<uint32_t>(row) * static_cast<uint32_t>(N) + static_cast<uint32_t>(n)) * 2 : gemm256::kNowhere;
-  }
-};
-
-struct Int8Walk : PlainWalk {
+struct Int8Walk : gemm256::PlainWalk<> {
   const uint16_t *scales;
   __device__ __forceinline__ Int8Walk(const uint16_t *x_, const uint16_t *w_, const uint16_t *scales_, uint16_t *y_, int M_, int N_, int K_)
       : PlainWalk(x_, w_, y_, M_, N_, K_), scales(scales_) {}
@@ -130,6 +77,46 @@ struct Int8Walk : PlainWalk {
     __builtin_amdgcn_raw_buffer_store_b128(out, y_rsrc(tile), y_at(tile, row, col), 0, 0);
   }
 };
+
+// Both matrices of silu(x w1) * (x w3): a lane ends up with the two products of its outputs.
+struct Int8GateWalk : gemm256::PlainWalk<128> {
+  const uint16_t *scales, *scales2;
+  __device__ __forceinline__ Int8GateWalk(const uint16_t *x_, const uint16_t *w_, const uint16_t *scales_, const uint16_t *scales2_, uint16_t *y_, int M_, int N_, int K_)
+      : PlainWalk(x_, w_, y_, M_, N_, K_), scales(scales_), scales2(scales2_) {}
+  struct Dest {
+    u32x4_t scale[2], scale2[2];
+  };
+  __device__ __forceinline__ void dest(const Tile &tile, int, int col, Dest &d) const {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int n = out_col(tile, col + 32 * q), at = n < N ? n : N - 8;
+      d.scale[q] = *reinterpret_cast<const u32x4_t *>(scales + at);
+      d.scale2[q] = *reinterpret_cast<const u32x4_t *>(scales2 + at);
+    }
+  }
+  __device__ __forceinline__ void store(const Tile &tile, const Dest &d, int, int q, int row, int col, float (&v)[8], float (&u)[8]) const {
+    const auto low = [](uint32_t b) { return __builtin_bit_cast(float, b << 16); };
+    const auto high = [](uint32_t b) { return __builtin_bit_cast(float, b & 0xFFFF0000u); };
+    u32x4_t out;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {  // the rounding points of the two linears, of F.silu and of the product
+      const uint32_t a = pack_bf16(v[2 * e], v[2 * e + 1]), b = pack_bf16(u[2 * e], u[2 * e + 1]), sa = d.scale[q][e], sb = d.scale2[q][e];
+      const uint32_t g = pack_bf16(low(a) * low(sa), high(a) * high(sa)), up = pack_bf16(low(b) * low(sb), high(b) * high(sb));
+      const uint32_t act = pack_bf16(silu(low(g)), silu(high(g)));
+      out[e] = pack_bf16(low(act) * low(up), high(act) * high(up));
+    }
+    __builtin_amdgcn_raw_buffer_store_b128(out, y_rsrc(tile), y_at(tile, row, col), 0, 0);
+  }
+};
+
+__global__ __launch_bounds__(256, 1) void int8_unpacked_gate_kernel(const uint16_t *x, const uint16_t *w, const uint16_t *scales, const uint16_t *scales2, uint16_t *y, int M,
+                                                                    int N, int K) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[gemm256::kRing];
+  Int8GateWalk tiles(x, w, scales, scales2, y, M, N, K);
+  gemm256::walk<false>(tiles, lds);
+#endif
+}
 
 __global__ __launch_bounds__(256, 1) void int8_unpacked_gemm_kernel(const uint16_t *x, const uint16_t *w, const uint16_t *scales, uint16_t *y, int M, int N, int K) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -362,7 +349,29 @@ __global__ __launch_bounds__(256) void int4_unpack_w_kernel(const uint32_t *__re
   }
 }
 
-struct Int4Walk : PlainWalk {
+// Eight sums of a row and the columns n .. n + 7 (rows n + first .. of w), back in the operands' units and with what the row's float16 values lack.  up: the row's row_exp.
+template <class Walk>
+__device__ __forceinline__ void finish_int4(const Walk &walk, const typename Walk::Tile &tile, int up, const f32x4_t (&unit)[2], int row, int n, int first, float (&v)[8]) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = __builtin_ldexpf(v[e] * unit[e >> 2][e & 3], -static_cast<int>(static_cast<int16_t>(up)));
+  if (__builtin_expect(up >= 1 << 16, 0)) {
+    const int m = tile.rb * 256 + row;
+    const Lacking *list = walk.lacking + static_cast<size_t>(m < walk.M ? m : walk.M - 1) * kMostLacking;
+    const __amdgpu_buffer_rsrc_t wr = walk.w_rsrc(tile);
+#pragma unroll 1
+    for (int i = 0; i < up >> 16; ++i) {
+      const Lacking l = list[i];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {  // (columns past N: of column 0, not stored)
+        const uint32_t at = (static_cast<uint32_t>(first + (n < walk.N ? n + e : 0)) * static_cast<uint32_t>(walk.K) + static_cast<uint32_t>(l.at)) * 2;
+        const float w = static_cast<float>(__builtin_bit_cast(_Float16, __builtin_amdgcn_raw_buffer_load_b16(wr, at, 0, 0)));
+        v[e] = __builtin_fmaf(l.by, w * unit[e >> 2][e & 3], v[e]);
+      }
+    }
+  }
+}
+
+struct Int4Walk : gemm256::PlainWalk<> {
   const float *col_unit;
   const int *row_exp, *skip;
   const Lacking *lacking;
@@ -394,25 +403,60 @@ struct Int4Walk : PlainWalk {
   }
   __device__ __forceinline__ void store(const Tile &tile, const Dest &d, int j, int q, int row, int col, float (&v)[8]) const {
     u32x4_t out;
+    finish_int4(*this, tile, d.up[j], d.unit[q], row, out_col(tile, col), 0, v);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = __builtin_ldexpf(v[e] * d.unit[q][e >> 2][e & 3], -static_cast<int>(static_cast<int16_t>(d.up[j])));
-    if (__builtin_expect(d.up[j] >= 1 << 16, 0)) {
-      const int m = tile.rb * 256 + row, n = tile.cb * 256 + col;
-      const Lacking *list = lacking + static_cast<size_t>(m < M ? m : M - 1) * kMostLacking;
-      const __amdgpu_buffer_rsrc_t wr = w_rsrc(tile);
-#pragma unroll 1
-      for (int i = 0; i < d.up[j] >> 16; ++i) {
-        const Lacking l = list[i];
+    for (int e = 0; e < 4; ++e) out[e] = pack_bf16(v[2 * e], v[2 * e + 1]);
+    __builtin_amdgcn_raw_buffer_store_b128(out, y_rsrc(tile), y_at(tile, row, col), 0, 0);
+  }
+};
+
+// Both matrices of silu(x w1) * (x w3), the second one's rows and units behind the first one's.
+struct Int4GateWalk : gemm256::PlainWalk<128> {
+  const float *col_unit;
+  const int *row_exp, *skip;
+  const Lacking *lacking;
+  __device__ __forceinline__ Int4GateWalk(const Int4Scratch &s, uint16_t *y_, int M_, int N_, int KE)
+      : PlainWalk(s.x, s.w, y_, M_, N_, KE), col_unit(s.col_unit), row_exp(s.row_exp), skip(s.skip), lacking(s.lacking) {}
+  __device__ __forceinline__ bool next(Tile &tile) {
+    while (PlainWalk::next(tile))
+      if (!skip[tile.rb]) return true;
+    return false;
+  }
+  __device__ __forceinline__ bool first(Tile &tile) { return next(tile); }
+  struct Dest {
+    f32x4_t unit[2][2][2];  // of the eight columns of each store of a row, in both matrices
+    int up[8];
+  };
+  __device__ __forceinline__ void dest(const Tile &tile, int row, int col, Dest &d) const {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {  // (columns past N: of column 0, not stored)
-          const uint32_t at = (static_cast<uint32_t>(n < N ? n + e : 0) * static_cast<uint32_t>(K) + static_cast<uint32_t>(l.at)) * 2;
-          const float w = static_cast<float>(__builtin_bit_cast(_Float16, __builtin_amdgcn_raw_buffer_load_b16(wr, at, 0, 0)));
-          v[e] = __builtin_fmaf(l.by, w * d.unit[q][e >> 2][e & 3], v[e]);
-        }
+    for (int q = 0; q < 2; ++q) {
+      const int n = out_col(tile, col + 32 * q), at = n < N ? n : N - 8;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const f32x4_t *u = reinterpret_cast<const f32x4_t *>(col_unit + h * N + at);
+        d.unit[q][h][0] = u[0];
+        d.unit[q][h][1] = u[1];
       }
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) out[e] = pack_bf16(v[2 * e], v[2 * e + 1]);
+    for (int j = 0; j < 8; ++j) {
+      const int m = tile.rb * 256 + row + 16 * j;
+      d.up[j] = row_exp[m < M ? m : M - 1];
+    }
+  }
+  __device__ __forceinline__ void store(const Tile &tile, const Dest &d, int j, int q, int row, int col, float (&v)[8], float (&u)[8]) const {
+    const auto low = [](uint32_t b) { return __builtin_bit_cast(float, b << 16); };
+    const auto high = [](uint32_t b) { return __builtin_bit_cast(float, b & 0xFFFF0000u); };
+    const int n = out_col(tile, col);
+    finish_int4(*this, tile, d.up[j], d.unit[q][0], row, n, 0, v);
+    finish_int4(*this, tile, d.up[j], d.unit[q][1], row, n, N, u);
+    u32x4_t out;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t g = pack_bf16(v[2 * e], v[2 * e + 1]), up = pack_bf16(u[2 * e], u[2 * e + 1]);
+      const uint32_t act = pack_bf16(silu(low(g)), silu(high(g)));
+      out[e] = pack_bf16(low(act) * low(up), high(act) * high(up));
+    }
     __builtin_amdgcn_raw_buffer_store_b128(out, y_rsrc(tile), y_at(tile, row, col), 0, 0);
   }
 };
@@ -426,17 +470,34 @@ __global__ __launch_bounds__(256, 1) void int4_unpacked_gemm_kernel(const Int4Sc
 #endif
 }
 
+__global__ __launch_bounds__(256, 1) void int4_unpacked_gate_kernel(const Int4Scratch s, uint16_t *y, int M, int N, int KE) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if (*s.flag & 1) return;  // the whole grid
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[gemm256::kRing];
+  Int4GateWalk tiles(s, y, M, N, KE);
+  gemm256::walk<true>(tiles, lds);
+#endif
+}
+
 template <int G>
 void launch_unpack(const uint16_t *x, const uint32_t *wp, const uint32_t *sz, const Int4Scratch &s, int twice, int M, int N, int K, int KE, hipStream_t stream) {
-  hipLaunchKernelGGL(int4_unpack_x_kernel<G>, dim3(static_cast<unsigned>((M + 3) / 4)), dim3(256), 0, stream, x, M, K, KE, s, sum_stride(M));
+  if (x) hipLaunchKernelGGL(int4_unpack_x_kernel<G>, dim3(static_cast<unsigned>((M + 3) / 4)), dim3(256), 0, stream, x, M, K, KE, s, sum_stride(M));
   const int cols = (N + 15) / 16, shares = std::max(1, std::min(K / 512, (4096 + cols - 1) / cols));  // at least four blocks of 128 k each
   hipLaunchKernelGGL(int4_unpack_w_kernel<G>, dim3(static_cast<unsigned>(cols), static_cast<unsigned>(shares)), dim3(256), 0, stream, wp, sz, twice, M, N, K, KE, s);
 }
 
-unsigned grid_of(int64_t M, int64_t N) {
-  const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
-  return static_cast<unsigned>(8 * std::min<int64_t>(32, (tiles + 7) / 8));
+// x null: it is unpacked already
+void unpack(const uint16_t *x, const int32_t *packed, const uint16_t *scales_and_zeros, const Int4Scratch &s, int groupsize, int M, int N, int K, hipStream_t stream) {
+  const int twice = groupsize == 256, G = twice ? 128 : groupsize, KE = extended(K, G);
+  const uint32_t *wp = reinterpret_cast<const uint32_t *>(packed), *sz = reinterpret_cast<const uint32_t *>(scales_and_zeros);
+  switch (G) {
+    case 32: launch_unpack<32>(x, wp, sz, s, twice, M, N, K, KE, stream); break;
+    case 64: launch_unpack<64>(x, wp, sz, s, twice, M, N, K, KE, stream); break;
+    default: launch_unpack<128>(x, wp, sz, s, twice, M, N, K, KE, stream); break;
+  }
 }
+
+unsigned grid_of(int64_t M, int64_t N, int64_t cols = gemm256::kSide) { return gemm256::grid_of((M + 255) / 256 * ((N + cols - 1) / cols)); }
 
 }  // namespace
 
@@ -480,12 +541,13 @@ int64_t int8_unpacked_bytes(int64_t M, int64_t N, int64_t K) {
   return unpacked_cost(M, N, K, static_cast<double>(N) * static_cast<double>(K) * 3 / 4.8e6) < int8_gemm32_cost(M, N, K) ? N * K * 2 : 0;
 }
 
+// rows in slices that a 32-bit offset reaches
+int64_t rows_at_once(int64_t K) { return ((int64_t{1} << 32) - 1) / (2 * K) / 256 * 256; }
+
 int int8_unpacked_gemm(const uint16_t *x, const int8_t *q, const uint16_t *scales, uint16_t *y, int M, int N, int K, uint16_t *w, hipStream_t stream) {
   const int64_t pieces = static_cast<int64_t>(N) * K / 16;
   hipLaunchKernelGGL(unpack_int8_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, stream, q, w, pieces);
-  // rows in slices that a 32-bit offset reaches
-  int64_t most = ((int64_t{1} << 32) - 1) / (2 * static_cast<int64_t>(K));
-  most -= most % 256;
+  const int64_t most = rows_at_once(K);
   for (int64_t m0 = 0; m0 < M; m0 += most) {
     const int rows = static_cast<int>(M - m0 < most ? M - m0 : most);
     hipLaunchKernelGGL(int8_unpacked_gemm_kernel, dim3(grid_of(rows, N)), dim3(256), 0, stream, x + m0 * K, w, scales, y + m0 * N, rows, N, K);
@@ -512,18 +574,85 @@ int64_t int4_unpacked_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int 
 int int4_unpacked_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *scales_and_zeros, uint16_t *y, int M, int N, int K, int groupsize, void *scratch,
                        hipStream_t stream) {
   const Int4Scratch s = int4_scratch(static_cast<uint8_t *>(scratch), M, N, K, groupsize);
-  const int twice = groupsize == 256, G = twice ? 128 : groupsize, KE = extended(K, G);
-  const uint32_t *wp = reinterpret_cast<const uint32_t *>(packed), *sz = reinterpret_cast<const uint32_t *>(scales_and_zeros);
-  switch (G) {
-    case 32: launch_unpack<32>(x, wp, sz, s, twice, M, N, K, KE, stream); break;
-    case 64: launch_unpack<64>(x, wp, sz, s, twice, M, N, K, KE, stream); break;
-    default: launch_unpack<128>(x, wp, sz, s, twice, M, N, K, KE, stream); break;
-  }
+  const int G = groupsize == 256 ? 128 : groupsize, KE = extended(K, G);
+  unpack(x, packed, scales_and_zeros, s, groupsize, M, N, K, stream);
   hipLaunchKernelGGL(int4_unpacked_gemm_kernel, dim3(grid_of(M, N)), dim3(256), 0, stream, s, y, M, N, KE);
   return int4_gemm(x, packed, scales_and_zeros, y, s.xsum, sum_stride(M), nullptr, int4_gemm_shape(M, N, K, G, 0), M, N, K, groupsize, stream, s.flag, s.row_flag);
 }
 
+// A pass over the results of two calls, which gates them: six bytes an output.
+double gate_pass_cost(int64_t M, int64_t N) { return 3 + static_cast<double>(M) * static_cast<double>(N) * 6 / 5e6; }
+
+// Scratch of a gated call on unpacked operands, or 0 where it is not taken: where it is not expected to be 3 % faster than two calls, whichever form those have, and that pass, or, int4, than
+// the gated launch on codes.  Measured, us, two calls and the pass / here: int8 2 x 11008 x 4096 1500 rows 385 / 303, 8192 rows 1166 / 1044, 2 x 22016 x 8192 3000 rows 1911 / 1770,
+// 1200 rows 774 / 870: not taken; int4 2 x 11008 x 4096 g128 8192 rows 1327 / 1159, g64 2048 rows 446 / 378, g32 1200 rows 319 / 304.
+int64_t int8_gate_unpacked_bytes(int64_t M, int64_t N, int64_t K) {
+  if (M < 1024 || N < 8 || N > INT32_MAX / 2 || N % 8 != 0) return 0;
+  const int64_t bytes = int8_unpacked_bytes(M, 2 * N, K);
+  if (bytes == 0) return 0;
+  const double unpack = static_cast<double>(N) * static_cast<double>(K) * 3 / 4.8e6;
+  const double call = std::min(unpacked_cost(M, N, K, unpack), int8_gemm32_cost(M, N, K));
+  return 1.03 * unpacked_cost(M, 2 * N, K, 2 * unpack) < 2 * call + gate_pass_cost(M, N) ? bytes : 0;
+}
+
+int64_t int4_gate_unpacked_bytes(int64_t M, int64_t N, int64_t K, int groupsize, int inner_k_tiles) {
+  if (M < 1024 || N < 8 || N > INT32_MAX / 2 || N % 8 != 0) return 0;
+  const int64_t bytes = int4_unpacked_bytes(M, 2 * N, K, groupsize, inner_k_tiles);
+  if (bytes == 0) return 0;
+  const int G = groupsize == 256 ? 128 : groupsize;
+  const int64_t KE = extended(static_cast<int>(K), G);
+  const double w = static_cast<double>(N) * static_cast<double>(K) * 2.5 / 4.8e6, rows = static_cast<double>(M) * static_cast<double>(K) * 4 / 4.8e6 + 8;
+  const double call = std::min(unpacked_cost(M, N, KE, w + rows), int4_codes_cost(M, N, K, G));
+  return 1.03 * unpacked_cost(M, 2 * N, KE, 2 * w + rows) < std::min(2 * call + gate_pass_cost(M, N), int4_codes_cost(M, 2 * N, K, G)) ? bytes : 0;
+}
+
+// y = bf16( bf16(silu(bf16(x w1))) * bf16(x w3) ), scratch of int4_unpacked_bytes for both matrices' columns: x is unpacked once, the tiles of both products fill the chip
+// together, and the gate costs a tile what its lanes compute.  8192 x 2 x 11008 x 4096, group size 128: 1327 us in two calls and a pass over their results, 1159.
+int int4_unpacked_gate(const uint16_t *x, const int32_t *packed, const uint16_t *sz, const int32_t *packed2, const uint16_t *sz2, uint16_t *y, int M, int N, int K, int groupsize,
+                       void *scratch, hipStream_t stream) {
+  const Int4Scratch s = int4_scratch(static_cast<uint8_t *>(scratch), M, 2 * static_cast<int64_t>(N), K, groupsize);
+  const int G = groupsize == 256 ? 128 : groupsize, KE = extended(K, G);
+  Int4Scratch second = s;
+  second.w += static_cast<int64_t>(N) * KE;
+  second.col_unit += N;
+  unpack(x, packed, sz, s, groupsize, M, N, K, stream);
+  unpack(nullptr, packed2, sz2, second, groupsize, M, N, K, stream);
+  hipLaunchKernelGGL(int4_unpacked_gate_kernel, dim3(grid_of(M, N, 128)), dim3(256), 0, stream, s, y, M, N, KE);
+  return int4_gemm_gate(x, packed, sz, packed2, sz2, y, s.xsum, sum_stride(M), int4_gemm_shape(M, 2 * N, K, G, 0), M, N, K, groupsize, stream, s.flag, s.row_flag);
+}
+
+// The same of int8 linears, scratch of int8_unpacked_bytes for both matrices' rows.  8192 x 2 x 11008 x 4096: 1166 us, 1044.
+int int8_unpacked_gate(const uint16_t *x, const int8_t *q, const uint16_t *scales, const int8_t *q2, const uint16_t *scales2, uint16_t *y, int M, int N, int K, uint16_t *w,
+                       hipStream_t stream) {
+  const int64_t pieces = static_cast<int64_t>(N) * K / 16;
+  const dim3 grid(static_cast<unsigned>((pieces + 255) / 256));
+  hipLaunchKernelGGL(unpack_int8_kernel, grid, dim3(256), 0, stream, q, w, pieces);
+  hipLaunchKernelGGL(unpack_int8_kernel, grid, dim3(256), 0, stream, q2, w + static_cast<int64_t>(N) * K, pieces);
+  const int64_t most = rows_at_once(K);
+  for (int64_t m0 = 0; m0 < M; m0 += most) {
+    const int rows = static_cast<int>(M - m0 < most ? M - m0 : most);
+    hipLaunchKernelGGL(int8_unpacked_gate_kernel, dim3(grid_of(rows, N, 128)), dim3(256), 0, stream, x + m0 * K, w, scales, scales2, y + m0 * N, rows, N, K);
+  }
+  return launch_status();
+}
+
 }  // namespace e2h
+
+extern "C" int64_t e2h_int8_mm_silu_gate_rows_scratch_bytes(int64_t m, int64_t n, int64_t k) {
+  return m <= INT32_MAX ? e2h::int8_gate_unpacked_bytes(m, n, k) : 0;
+}
+
+extern "C" int e2h_int8_mm_silu_gate_rows(const uint16_t *x, const int8_t *q_gate, const uint16_t *scales_gate, const int8_t *q_up, const uint16_t *scales_up, uint16_t *y, int64_t m,
+                                          int64_t n, int64_t k, void *scratch, int64_t scratch_bytes, void *stream) {
+  using namespace e2h;
+  if (!x || !q_gate || !scales_gate || !q_up || !scales_up || !y || !scratch) return E2H_ERR_NULL_POINTER;
+  const int64_t need = e2h_int8_mm_silu_gate_rows_scratch_bytes(m, n, k);
+  if (need == 0) return E2H_ERR_BAD_SHAPE;
+  if (scratch_bytes < need) return E2H_ERR_SCRATCH_TOO_SMALL;
+  if (!aligned16(x) || !aligned16(q_gate) || !aligned16(q_up) || !aligned16(scales_gate) || !aligned16(scales_up) || !aligned16(y) || !aligned16(scratch)) return E2H_ERR_MISALIGNED;
+  return int8_unpacked_gate(x, q_gate, scales_gate, q_up, scales_up, y, static_cast<int>(m), static_cast<int>(n), static_cast<int>(k), static_cast<uint16_t *>(scratch),
+                            static_cast<hipStream_t>(stream));
+}
 
 extern "C" int64_t e2h_int4_mm_scratch_bytes(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles) {
   return e2h::int4_unpacked_bytes(m, n, k, groupsize, inner_k_tiles);

@@ -280,7 +280,11 @@ class FeedForward(nn.Module):
         """silu(w1 x) * w3 x of a prompt with one launch for both products, or None where the modules are to be called: few rows, weights that differ in form or do not fit x,
         somebody who watches their calls, or no gain."""
         w1, w3 = self.w1, self.w3
-        if not (FUSE_GATE and _fusable(x) and type(w1) is WeightOnlyInt4Linear and type(w3) is WeightOnlyInt4Linear) or torch.compiler.is_compiling():
+        if not (FUSE_GATE and _fusable(x) and type(w1) is type(w3)) or torch.compiler.is_compiling():
+            return None
+        if type(w1) is WeightOnlyInt8Linear:
+            return self._gate_rows_int8(x)
+        if type(w1) is not WeightOnlyInt4Linear:
             return None
         k, n, group = w1.in_features, w1.out_features, w1.groupsize
         if x.shape[-1] != k or x.numel() <= 64 * k or w1.padding or w3.padding or w3.groupsize != group or not ops.int4_gate_rows_pay(x.numel() // k, n, k, group):
@@ -294,6 +298,21 @@ class FeedForward(nn.Module):
         if seq_ops.watched(x, w1.weight, w1.scales_and_zeros, w3.weight, w3.scales_and_zeros):
             return None
         y = ops.int4_mm_silu_gate_rows(x.reshape(-1, k), w1.weight, w1.scales_and_zeros, w3.weight, w3.scales_and_zeros, group)
+        return None if y is None else y.view(*x.shape[:-1], n)
+
+    def _gate_rows_int8(self, x: Tensor) -> Optional[Tensor]:
+        w1, w3 = self.w1, self.w3
+        k, n = w1.in_features, w1.out_features
+        if x.shape[-1] != k or x.numel() <= 64 * k:
+            return None
+        for w in (w1, w3):
+            q, scales = w.weight, w.scales
+            if not (q.dtype == torch.int8 and scales.dtype == torch.bfloat16 and q.device == x.device and scales.device == x.device and tuple(q.shape) == (n, k)
+                    and tuple(scales.shape) == (n,) and unwatched(w)):
+                return None
+        if seq_ops.watched(x, w1.weight, w1.scales, w3.weight, w3.scales):
+            return None
+        y = ops.int8_mm_silu_gate_rows(x.reshape(-1, k), w1.weight, w1.scales, w3.weight, w3.scales)
         return None if y is None else y.view(*x.shape[:-1], n)
 
     def forward(self, x: Tensor, defer_output: bool = False) -> Tensor:

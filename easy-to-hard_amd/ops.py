@@ -707,6 +707,27 @@ def int8_mm_silu_gate(x, q_gate, scales_gate, q_up, scales_up):
     return y
 
 
+def int8_mm_silu_gate_rows(x, q_gate, scales_gate, q_up, scales_up):
+    """bf16(bf16(silu(int8_mm(x, gate))) * int8_mm(x, up)) over 1024 rows and more in one product launch, or None where the sizes are not taken (or there is no memory for
+    the launch's scratch)."""
+    _need_gpu(x, q_gate, scales_gate, q_up, scales_up)
+    assert x.dtype == torch.bfloat16 and x.dim() == 2 and q_gate.dtype == torch.int8 and q_up.dtype == torch.int8
+    assert scales_gate.dtype == torch.bfloat16 and scales_up.dtype == torch.bfloat16
+    n, k = q_gate.shape
+    m = x.shape[0]
+    if q_up.shape != q_gate.shape or x.shape[1] != k or scales_gate.numel() != n or scales_up.numel() != n:
+        raise RuntimeError("int8_mm_silu_gate_rows: shapes of the two linears and x do not match")
+    lib = _lib_for(x)
+    scratch = _unpacked_weight(m, x.device, lib.e2h_int8_mm_silu_gate_rows_scratch_bytes, n, k)
+    x, q_gate, q_up, scales_gate, scales_up = x.contiguous(), q_gate.contiguous(), q_up.contiguous(), scales_gate.contiguous(), scales_up.contiguous()
+    if scratch is None or any(t.data_ptr() % 16 for t in (x, q_gate, q_up, scales_gate, scales_up)):
+        return None
+    y = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    rc = lib.e2h_int8_mm_silu_gate_rows(_ptr(x), _ptr(q_gate), _ptr(scales_gate), _ptr(q_up), _ptr(scales_up), _ptr(y), m, n, k, _ptr(scratch), scratch.numel(), _stream(x))
+    _lib.check(rc, "e2h_int8_mm_silu_gate_rows")
+    return y
+
+
 def int8_rope_kv_supported(x, wqkv, freqs_cis, k_cache):
     """True when the fused projection + RoPE + cache write covers (x [B, 1, K], a WeightOnlyInt8Linear)."""
     return _int8_fusable(x, wqkv) and freqs_cis.shape[0] >= k_cache.shape[2]

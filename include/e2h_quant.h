@@ -198,12 +198,18 @@ int e2h_int4_mm_rope_kv(const uint16_t *x, const int32_t *packed, const uint16_t
                         void *stream);
 
 /* The gated launch over many rows, y = bf16(bf16(silu(x @ gate^T)) * (x @ up^T)) with both products rounded to bfloat16 first: what two calls of
- * e2h_int4_mm and e2h_silu_mul give, with the same sums in float32 as e2h_int4_mm has over the 32 x 32 tiles of such calls with one K slice.
+ * e2h_int4_mm and e2h_silu_mul give, with the same sums in float32 as e2h_int4_mm has over the 32 x 32 tiles of such calls with one K slice,
+ * or, from 1024 rows on, as e2h_int4_mm_scratch has on unpacked operands.
  *   65 <= m, any group size of e2h_int4_mm, inner_k_tiles == 8, k % 128 == 0, n % 8 == 0; scratch 16-byte aligned, scratch_bytes >= what
  *   e2h_int4_mm_silu_gate_rows_scratch_bytes returns, which is 0 where the shape is not taken (or not faster than those calls: the entry point then returns
  *   E2H_ERR_BAD_SHAPE).  The launch neither allocates nor keeps anything. */
 int64_t e2h_int4_mm_silu_gate_rows_scratch_bytes(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles);
-/* 1 where that launch is expected to take less time than two calls of e2h_int4_mm and e2h_silu_mul, whichever kernels those run, else 0 (a subset of the shapes that are taken). */
+/* The same of int8 linears, 1024 <= m, n % 8 == 0, k % 128 == 0, all pointers 16-byte aligned: what two calls of e2h_int8_mm_scratch and e2h_silu_mul give.  The first function
+ * returns 0 where the shape is not taken. */
+int64_t e2h_int8_mm_silu_gate_rows_scratch_bytes(int64_t m, int64_t n, int64_t k);
+int e2h_int8_mm_silu_gate_rows(const uint16_t *x, const int8_t *q_gate, const uint16_t *scales_gate, const int8_t *q_up, const uint16_t *scales_up, uint16_t *y,
+                               int64_t m, int64_t n, int64_t k, void *scratch, int64_t scratch_bytes, void *stream);
+/* (int4) 1 where that launch is expected to take less time than two calls of e2h_int4_mm and e2h_silu_mul, whichever kernels those run, else 0 (a subset of the shapes that are taken). */
 int e2h_int4_mm_silu_gate_rows_pays(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles);
 int e2h_int4_mm_silu_gate_rows(const uint16_t *x, const int32_t *packed_gate, const uint16_t *sz_gate, const int32_t *packed_up,
                                const uint16_t *sz_up, uint16_t *y, int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles,

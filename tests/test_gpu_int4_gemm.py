@@ -438,3 +438,90 @@ def test_odd_scales_in_96_row_workgroups(many_row_kernel, g, m, n, k):
     finite = torch.ones(n, dtype=torch.bool)
     finite[300] = False
     assert torch.equal(got[:, finite], want[:, finite].to(torch.bfloat16)) and not torch.isfinite(got[:, 300]).any()
+
+
+# ---- the gated launch on unpacked operands ------------------------------------------------------------------------------------------------
+def _gate_of(a, b):
+    """silu(a) * b with the rounding points of stock ops on bfloat16 tensors, from products in float64"""
+    a, b = a.to(torch.bfloat16), b.to(torch.bfloat16)
+    return ((a.double() / (1 + torch.exp(-a.double()))).to(torch.bfloat16).double() * b.double()).to(torch.bfloat16)
+
+
+def _check_gate(got, want):
+    """A gate within three units in the last place of float32 rounds to another bfloat16 in about one value of 4000, by a unit of 2^-7 of it at most; the product's own
+    rounding makes that two units at most.  Below -88.7, where exp(-a) leaves float32, gates are zero for at most 2^-121 in size and their products (|b| < 2^30) for 2^-91."""
+    got, want = got.double(), want.double()
+    assert torch.isfinite(got).all()
+    assert ((got - want).abs() <= 2.0 ** -6 * want.abs() + 2.0 ** -91).all()
+    assert ((got != want) & (want.abs() > 2.0 ** -90)).double().mean() <= 2e-3
+
+
+@pytest.mark.parametrize("g", [32, 64, 128, 256])
+@pytest.mark.parametrize("m,n,k", [(70000, 8, 256), (66049, 264, 512), (66100, 1032, 512)])  # ragged columns of a tile's 128, a last tile of 112 rows, of one and of 52
+def test_gated_unpacked_rows_are_the_two_exact_products_gated(g, m, n, k):
+    halves = [_case(m, n, k, g, seed=seed) for seed in (5, 77)]
+    x = halves[0][3]
+    weights = []
+    for codes, scale, zero, _ in halves:
+        weights += [torch.from_numpy(qo.int4_tile_pack(codes.numpy(), 8)).to(DEV), torch.stack([scale, zero], dim=-1).to(torch.bfloat16).contiguous().to(DEV)]
+    lib = _lib.load()
+    assert lib.e2h_int4_mm_silu_gate_rows_scratch_bytes(m, n, k, g, 8) >= lib.e2h_int4_mm_scratch_bytes(m, 2 * n, k, g, 8) > 0
+    got = ops.int4_mm_silu_gate_rows(x, *weights, g)
+    rows = torch.cat([torch.arange(0, 300), torch.arange(m - 300, m)]).to(DEV)
+    _check_gate(got[rows], _gate_of(*(_double(c, s, z, x, g, rows) for c, s, z, _ in halves)))
+
+
+def test_gated_unpacked_rows_leave_what_float16_lacks_to_the_other_kernel():
+    """A row that is not finite, a row of small values beside a large one, and a scale that float16 does not hold in the second matrix: as two calls give them."""
+    m, n, k, g = 66049, 264, 512, 128
+    gen = torch.Generator().manual_seed(4)
+    x = torch.randn((m, k), generator=gen).to(torch.bfloat16)
+    x[7, 5], x[300, 9] = float("inf"), float("nan")
+    x[900, 1:40] *= 2.0 ** -40
+    x = x.to(DEV)
+    w = [ops.int4_quantize_pack((torch.randn((n, k), generator=gen) * 0.02).to(torch.bfloat16).to(DEV), g, 8) for _ in range(2)]
+    for plant in (False, True):
+        if plant:
+            w[1][1][0, 33, 0] = float("inf")
+        got = ops.int4_mm_silu_gate_rows(x, *w[0], *w[1], g)
+        a, b = (ops.int4_mm(x, p, g, sz) for p, sz in w)
+        want = torch.nn.functional.silu(a.double()).to(torch.bfloat16).double() * b.double()
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want.to(torch.bfloat16)))
+        fine = torch.isfinite(want)
+        # the calls' sums have another order where the other kernel forms them: a product may round to another bfloat16, its gate by 1.1 times that
+        assert (got[fine].double() - want[fine]).norm() <= 2.0 ** -7 * want[fine].norm()
+
+
+@pytest.mark.parametrize("m,n,k", [(1030, 8200, 256), (1500, 5504, 384), (4096, 2056, 512), (70000, 8, 256)])
+def test_gated_int8_rows_are_the_two_calls_gated(m, n, k):
+    """Whole numbers as operands, so that products are exact whatever the order of their sums."""
+    gen = torch.Generator().manual_seed(m + n)
+    x = torch.randint(-8, 9, (m, k), generator=gen).to(torch.bfloat16).to(DEV)
+    q = [torch.randint(-128, 128, (n, k), generator=gen, dtype=torch.int8).to(DEV) for _ in range(2)]
+    s = [(torch.rand((n,), generator=gen) * 0.002).to(torch.bfloat16).to(DEV) for _ in range(2)]
+    got = ops.int8_mm_silu_gate_rows(x, q[0], s[0], q[1], s[1])
+    assert got is not None
+    a, b = (((x.double() @ w.double().t()).to(torch.bfloat16).double() * t.double()).to(torch.bfloat16) for w, t in zip(q, s))
+    _check_gate(got, _gate_of(a.double(), b.double()))
+    assert ops.int8_mm_silu_gate_rows(x[:1000], q[0], s[0], q[1], s[1]) is None
+
+
+def test_gated_int8_rows_leave_watched_modules_to_the_modules():
+    from easy_to_hard_amd.model import FeedForward, ModelArgs
+    from easy_to_hard_amd.quantize import WeightOnlyInt8QuantHandler
+
+    ff = FeedForward(ModelArgs(dim=256, intermediate_size=8200, n_head=4, n_layer=1))
+    WeightOnlyInt8QuantHandler(ff).convert_for_runtime()
+    gen = torch.Generator().manual_seed(1)
+    for lin in (ff.w1, ff.w2, ff.w3):
+        lin.weight = torch.randint(-128, 128, (lin.out_features, lin.in_features), generator=gen, dtype=torch.int8).to(DEV)
+        lin.scales = torch.full((lin.out_features,), 2.0 ** -11, dtype=torch.bfloat16, device=DEV)
+    x = torch.randn((2, 515, 256), generator=gen).to(torch.bfloat16).to(DEV)
+    whole = ff(x)
+    assert ff._gate_rows(x).shape == (2, 515, 8200)
+    seen = []
+    handle = ff.w3.register_forward_hook(lambda *_: seen.append(1))
+    assert ff._gate_rows(x) is None and seen == []
+    assert (ff(x).double() - whole.double()).norm() <= 2.0 ** -7 * whole.double().norm() and seen == [1]
+    handle.remove()
+    assert ff._gate_rows(x.float()) is None and ff._gate_rows(x[:, :20]) is None
