@@ -3,6 +3,7 @@
 // Measured on one MI355X, graph replay over rotating weights (vendor matmul in brackets): 22528 x 4096 at 1 / 32 rows 31.7 / 33.3 us
 // (50.4 / 45.2), 16384 x 4096 24.7 / 25.1 (33.5 / 33.4), 4096 x 16384 29.2 / 30 (31.0 / 35.3), 4096 x 8192 12.9 / 18.6 (16.3 /
 // 19.1), 4096 x 4096 7.7 / 11.6 (15.3 / 13.8), 32000 x 4096 44.4 / 45.8 (59.7 / 55.1): 4.2 to 6 TB/s of weights.
+#include "e2h_gemm256.h"
 #include "e2h_seq_common.h"
 #include "e2h_stream.h"
 
@@ -79,10 +80,71 @@ int run_linear(const stream::Args &a, bf16_t *y, float cap, float *scratch, hipS
   return launch_status();
 }
 
+// ---- many rows: the activation behind a tile of products (e2h_gemm256.h) ---------------------------------------------------------------
+template <int ACT>
+struct RowsWalk : gemm256::PlainWalk<> {
+  using gemm256::PlainWalk<>::PlainWalk;
+  struct Dest {};
+  __device__ __forceinline__ void dest(const Tile &, int, int, Dest &) const {}
+  __device__ __forceinline__ void store(const Tile &tile, const Dest &, int, int, int row, int col, float (&v)[8]) const {
+    u32x4_t out;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      out[e] = pack_bf16(v[2 * e], v[2 * e + 1]);
+      if (ACT == kSquare) {
+        const float lo = fmaxf(__builtin_bit_cast(float, out[e] << 16), 0.f), hi = fmaxf(__builtin_bit_cast(float, out[e] & 0xFFFF0000u), 0.f);
+        out[e] = pack_bf16(lo * lo, hi * hi);
+      }
+    }
+    __builtin_amdgcn_raw_buffer_store_b128(out, y_rsrc(tile), y_at(tile, row, col), 0, 0);
+  }
+};
+
+template <int ACT>
+__global__ __launch_bounds__(256, 1) void linear_rows_kernel(const uint16_t *x, const uint16_t *w, uint16_t *y, int M, int N, int K) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[gemm256::kRing];
+  RowsWalk<ACT> tiles(x, w, y, M, N, K);
+  gemm256::walk<false>(tiles, lds);
+#endif
+}
+
+bool rows_fit(int64_t m, int64_t n, int64_t k) {
+  return m >= 1 && n >= 8 && n % 8 == 0 && k % 64 == 0 && k >= gemm256::kLeastK && m <= INT32_MAX / 2 && n <= INT32_MAX / 2 && k <= INT32_MAX / 2 &&
+         m * k * 2 < (int64_t{1} << 32) && n * k * 2 < (int64_t{1} << 32) && 256 * n * 2 < (int64_t{1} << 32);
+}
+
 }  // namespace
 }  // namespace e2h
 
 using namespace e2h;
+
+// 1 where the product with its activation is expected to be faster here than the library's product and a pass over its result.  Measured, us, that / here: 16384 x 4096 1000 rows 114 / 96,
+// 8192 rows 817 / 743; 8192 x 2048 2048 rows 68 / 51; 2048 x 4096 8192 rows 112 / 95; 16384 x 4096 512 rows 70 / 76: not taken.  Without an activation the library's product is
+// 2 % the faster one where it fills the chip (16384 x 4096 8192 rows 725 / 742).
+// us, as for the quantized linears on the same loop (a last round that is not full runs at a higher clock), against the library's product at what it reaches where it fills the chip, 1.5
+// PFLOP/s, and a pass over the result of its own.
+extern "C" int e2h_seq_linear_rows_pays(int64_t rows, int64_t n, int64_t k, int act) {
+  if (rows <= 64 || act != kSquare || !rows_fit(rows, n, k)) return 0;
+  const int64_t tiles = (rows + 255) / 256 * ((n + 255) / 256), full = tiles / 256, rest = tiles % 256;
+  const double rounds = static_cast<double>(full) + (rest == 0 ? 0. : full == 0 ? 1. : 0.6 + 0.4 * static_cast<double>(rest) / 256);
+  const double outputs = static_cast<double>(rows) * static_cast<double>(n);
+  return 4 + rounds * (static_cast<double>(k) / 64 * 1.36 + 5) < outputs * static_cast<double>(k) * 2 / 1.5e9 + outputs * 4 / 6e6 + 12 ? 1 : 0;
+}
+
+extern "C" int e2h_seq_linear_rows(const void *x, const void *w, void *y, int64_t rows, int64_t n, int64_t k, int act, void *stream) {
+  if (!x || !w || !y) return E2H_ERR_NULL_POINTER;
+  if (!rows_fit(rows, n, k) || (act != kNone && act != kSquare)) return E2H_ERR_BAD_SHAPE;
+  if (!aligned16(x) || !aligned16(w) || !aligned16(y)) return E2H_ERR_MISALIGNED;
+  const dim3 grid(gemm256::grid_of((rows + 255) / 256 * ((n + 255) / 256)));
+  const auto *xs = static_cast<const uint16_t *>(x), *ws = static_cast<const uint16_t *>(w);
+  auto *ys = static_cast<uint16_t *>(y);
+  const int M = static_cast<int>(rows), N = static_cast<int>(n), K = static_cast<int>(k);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (act == kSquare) hipLaunchKernelGGL(linear_rows_kernel<kSquare>, grid, dim3(256), 0, s, xs, ws, ys, M, N, K);
+  else hipLaunchKernelGGL(linear_rows_kernel<kNone>, grid, dim3(256), 0, s, xs, ws, ys, M, N, K);
+  return launch_status();
+}
 
 extern "C" int64_t e2h_seq_linear_scratch_bytes(int64_t rows, int64_t n, int64_t k) {
   if (!stream::takes(rows, n, k, 2)) return E2H_ERR_BAD_SHAPE;

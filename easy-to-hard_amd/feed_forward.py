@@ -19,6 +19,8 @@ class SquaredReluFF(nn.Module):
     def forward(self, h: Tensor) -> Tensor:
         if fusable(self.up, h):
             return self.down(seq_ops.linear(h, self.up.weight, seq_ops.ACT_SQUARE_RELU))
+        if type(self.up) is DecodeLinear and self.up.bias is None and unwatched(self.up) and seq_ops.linear_rows_pay(h, self.up.weight, seq_ops.ACT_SQUARE_RELU):
+            return self.down(seq_ops.linear_rows(h, self.up.weight, seq_ops.ACT_SQUARE_RELU))
         return self.down(seq_ops.square_relu_(self.up(h)))
 
 

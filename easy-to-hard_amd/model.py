@@ -376,7 +376,7 @@ class TransformerBlock(nn.Module):
     def _norms_fold(self, x: Tensor, delta) -> bool:
         """True for the single-token step of one sequence through an int8 model whose modules nobody watches: the products behind the norms form their row themselves."""
         att, ff = self.attention, self.feed_forward
-        if x.shape[0] != 1 or not (FUSE_ROPE_PROJECTION and FUSE_GATE and DEFER_SPLIT_K and type(att) is Attention and type(ff) is FeedForward
+        if x.shape[0] != 1 or torch.compiler.is_compiling() or not (FUSE_ROPE_PROJECTION and FUSE_GATE and DEFER_SPLIT_K and type(att) is Attention and type(ff) is FeedForward
                                   and type(self.attention_norm) is RMSNorm and type(self.ffn_norm) is RMSNorm and att.can_fuse_decode(x, False)):
             return False
         lins = (att.wqkv, att.wo, ff.w1, ff.w3, ff.w2)
@@ -559,7 +559,7 @@ class Transformer(nn.Module):
             for layer in self.layers:
                 x, delta = layer.forward_deferred(x, delta, input_pos, freqs_cis, mask, fully_causal)
             out = self.output
-            if (fused_step and x.shape[0] == 1 and type(out) is WeightOnlyInt8Linear and type(self.norm) is RMSNorm and unwatched(out) and unwatched(self.norm)
+            if (fused_step and x.shape[0] == 1 and not torch.compiler.is_compiling() and type(out) is WeightOnlyInt8Linear and type(self.norm) is RMSNorm and unwatched(out) and unwatched(self.norm)
                     and ops.int8_norm_fits(x, self.norm.weight, delta, out)):
                 return ops.int8_norm_mm(x, delta, self.norm.weight, self.norm.eps, out.weight, out.scales)[1].view(x.shape[0], 1, -1)
             _, normed = ops.add_rmsnorm(x, delta, self.norm.weight, self.norm.eps)

@@ -774,3 +774,40 @@ def test_scoring_with_a_reward_head(tmp_path):
     weights["head"] = head.numpy()
     linear = ro.forward({**cfg, "logit_softcap": 1e12}, weights, toks.numpy())[0]
     assert rel(got, linear.mean(-1)) < 1e-4
+
+
+# ---- many rows through a linear and its activation in one launch ----------------------------------------------------------------------
+
+@pytest.mark.parametrize("act", [seq_ops.ACT_NONE, seq_ops.ACT_SQUARE_RELU])
+@pytest.mark.parametrize("rows,n,k", [(1, 8, 192), (65, 264, 192), (256, 256, 256), (257, 520, 320), (1000, 8, 4096), (3000, 4104, 256)])
+def test_linear_rows_is_the_rounded_product_and_its_activation(rows, n, k, act):
+    """Whole numbers, so that products are exact: ragged rows and columns of a 256 x 256 tile, the shortest K, more tiles than CUs."""
+    gen = torch.Generator().manual_seed(rows + n)
+    x = torch.randint(-8, 9, (rows, k), generator=gen).to(torch.bfloat16).to(DEV)
+    w = torch.randint(-8, 9, (n, k), generator=gen).to(torch.bfloat16).to(DEV)
+    want = (x.double() @ w.double().t()).to(torch.bfloat16)
+    if act == seq_ops.ACT_SQUARE_RELU:
+        want = seq_ops.square_relu_(want)
+    assert torch.equal(seq_ops.linear_rows(x, w, act), want)
+
+
+def test_feed_forward_of_many_rows_takes_one_launch_for_up_and_its_activation():
+    from easy_to_hard_amd.feed_forward import SquaredReluFF
+
+    ff = SquaredReluFF(256, 16384).to(DEV).to(torch.bfloat16).requires_grad_(False)
+    h = randn(2, 520, 256, dtype=torch.bfloat16)
+    assert seq_ops.linear_rows_pay(h, ff.up.weight, seq_ops.ACT_SQUARE_RELU) and not seq_ops.linear_rows_pay(h[:, :30], ff.up.weight, seq_ops.ACT_SQUARE_RELU)
+    y, seen = ff(h), []
+    handle = ff.up.register_forward_hook(lambda *_: seen.append(1))
+    apart = ff(h)
+    handle.remove()
+    assert seen == [1] and rel(f64(y), f64(apart)) < 4e-3  # sums in another order: roundings of the hidden values
+    nan = h.clone()
+    nan[0, 0, 0], nan[1, 3, 4] = float("nan"), float("inf")
+    ff.up.weight[:, 4] = ff.up.weight[:, 4].abs() + 0.1
+    assert torch.equal(torch.isnan(seq_ops.linear_rows(nan, ff.up.weight, seq_ops.ACT_SQUARE_RELU)), torch.isnan(seq_ops.square_relu_(torch.nn.functional.linear(nan, ff.up.weight))))
+    assert not seq_ops.linear_rows_pay(h.float(), ff.up.weight, 1) and not seq_ops.linear_rows_pay(h.transpose(0, 1), ff.up.weight, 1)
+    up = ff.up.weight.clone().requires_grad_()
+    assert not seq_ops.linear_rows_pay(h, up, 1)
+    with torch.no_grad():
+        assert seq_ops.linear_rows_pay(h, up, 1)
