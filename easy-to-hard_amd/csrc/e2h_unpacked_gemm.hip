@@ -66,7 +66,7 @@ struct Int8Walk : gemm256::PlainWalk<> {
       d.scale[q] = *reinterpret_cast<const u32x4_t *>(scales + (n < N ? n : N - 8));
     }
   }
-  __device__ __forceinline__ void store(const Tile &tile, const Dest &d, int, int q, int row, int col, float (&v)[8]) const {
+  __device__ __forceinline__ u32x4_t outputs(const Dest &d, int q, const float (&v)[8]) const {
     u32x4_t out;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -74,7 +74,10 @@ struct Int8Walk : gemm256::PlainWalk<> {
       out[e] = pack_bf16(__builtin_bit_cast(float, t << 16) * __builtin_bit_cast(float, s << 16),
                          __builtin_bit_cast(float, t & 0xFFFF0000u) * __builtin_bit_cast(float, s & 0xFFFF0000u));
     }
-    __builtin_amdgcn_raw_buffer_store_b128(out, y_rsrc(tile), y_at(tile, row, col), 0, 0);
+    return out;
+  }
+  __device__ __forceinline__ void store(const Tile &tile, const Dest &d, int, int q, int row, int col, float (&v)[8]) const {
+    __builtin_amdgcn_raw_buffer_store_b128(outputs(d, q, v), y_rsrc(tile), y_at(tile, row, col), 0, 0);
   }
 };
 
@@ -122,6 +125,113 @@ __global__ __launch_bounds__(256, 1) void int8_unpacked_gemm_kernel(const uint16
 #if defined(__HIP_DEVICE_COMPILE__)
   __shared__ __attribute__((aligned(1024))) uint8_t lds[gemm256::kRing];
   Int8Walk tiles(x, w, scales, y, M, N, K);
+  gemm256::walk<false>(tiles, lds);
+#endif
+}
+
+// What a fused q | k | v product of B sequences of T tokens (row b T + t) leaves behind: q [B][H][T][D] and k, v [B][Hkv][S][D], q and k rotated by the angles of the tokens'
+// positions.
+struct RopeRows {
+  const uint16_t *freqs;  // [freq_rows][D / 2][2]
+  uint16_t *q, *k, *v;
+  const int64_t *pos;     // [T]
+  int B, T, H, Hkv, S, D, freq_rows, by_token;  // by_token: k and v of token t are row t, else row pos[t]
+};
+
+// Stores of a walk over such a product.  A wave's 128 columns belong to one of the three.  The angles of a row of its outputs (a 16-byte load beside each store) come
+// kAhead - 1 rows ahead of their use, in registers that hold fragments in the main loop.
+struct RopeStore {
+  static constexpr int kAhead = 3;
+  struct Dest {
+    int pos[8];                   // of the lane's rows
+    int b, t;                     // sequence and token of the row being stored
+    u32x4_t cos_sin[kAhead][4];
+  };
+  const RopeRows &r;
+  int row_base;  // of the walk's first row
+
+  __device__ __forceinline__ void place(int row, Dest &d) const {
+    const int m = row_base + row;
+    d.b = m / r.T;
+    d.t = m - d.b * r.T;
+  }
+  __device__ __forceinline__ void step(Dest &d) const {  // 16 rows on; T is no less
+    d.t += 16;
+    if (d.t >= r.T) {
+      d.t -= r.T;
+      ++d.b;
+    }
+  }
+  __device__ __forceinline__ void dest(int row, Dest &d) const {
+    place(row, d);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      d.pos[j] = static_cast<int>(reinterpret_cast<const uint32_t *>(r.pos)[2 * d.t]);
+      step(d);
+    }
+  }
+  __device__ __forceinline__ void request(Dest &d, int j, int col, bool rotated) const {
+    const __amdgpu_buffer_rsrc_t f = make_rsrc(r.freqs, static_cast<uint32_t>(r.freq_rows) * static_cast<uint32_t>(r.D) * 2);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t at = static_cast<uint32_t>(d.pos[j]) * static_cast<uint32_t>(r.D) * 2 + static_cast<uint32_t>((col + 32 * q) & (r.D - 1)) * 2;
+      d.cos_sin[j % kAhead][q] = __builtin_amdgcn_raw_buffer_load_b128(f, rotated && d.pos[j] >= 0 && d.pos[j] < r.freq_rows ? at : gemm256::kNowhere, 0, 0);
+    }
+  }
+  // own: the outputs (row, n .. n + 7) of the product
+  __device__ __forceinline__ void store(Dest &d, int j, int q, int row, int rows, int n, u32x4_t own) const {
+    const auto low = [](uint32_t b) { return __builtin_bit_cast(float, b << 16); };
+    const auto high = [](uint32_t b) { return __builtin_bit_cast(float, b & 0xFFFF0000u); };
+    const int HD = r.H * r.D, KD = r.Hkv * r.D, wave_n = __builtin_amdgcn_readfirstlane(n) & ~127;
+    const bool is_q = wave_n < HD, rotated = wave_n < HD + KD;
+    if (q == 0) {
+      if (j == 0) {
+        place(row, d);
+#pragma unroll
+        for (int a = 0; a + 1 < kAhead; ++a) request(d, a, n, rotated);
+      } else {
+        step(d);
+      }
+      if (j + kAhead - 1 < 8) request(d, j + kAhead - 1, n, rotated);
+    }
+    u32x4_t out;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t x = own[e], f = d.cos_sin[j % kAhead][q][e];
+      const float r0 = low(x) * low(f) - high(x) * high(f), r1 = high(x) * low(f) + low(x) * high(f);  // two rounded products, then their sum, as torch forms it
+      out[e] = rotated ? pack_bf16(r0, r1) : x;
+    }
+    const int pos = d.pos[j], slot = r.by_token ? d.t : pos, at = n - (is_q ? 0 : rotated ? HD : HD + KD);
+    const int heads = is_q ? r.H : r.Hkv, length = is_q ? r.T : r.S, log_d = r.D == 128 ? 7 : 6;
+    const uint32_t line = static_cast<uint32_t>(d.b * heads + (at >> log_d)) * static_cast<uint32_t>(length) + static_cast<uint32_t>(is_q ? d.t : slot);
+    const uint32_t to = ((line << log_d) + static_cast<uint32_t>(at & (r.D - 1))) * 2;
+    const bool there = row < rows && pos >= 0 && slot >= 0 && slot < r.S && wave_n < HD + 2 * KD;
+    const __amdgpu_buffer_rsrc_t y = make_rsrc(is_q ? r.q : rotated ? r.k : r.v, static_cast<uint32_t>(r.B * heads) * static_cast<uint32_t>(length) * static_cast<uint32_t>(r.D) * 2);
+    __builtin_amdgcn_raw_buffer_store_b128(out, y, there ? to : gemm256::kNowhere, 0, 0);
+  }
+};
+
+struct Int8RopeWalk : Int8Walk {
+  RopeStore rope;
+  __device__ __forceinline__ Int8RopeWalk(const uint16_t *x_, const uint16_t *w_, const uint16_t *scales_, const RopeRows &r, int row_base, int M_, int N_, int K_)
+      : Int8Walk(x_, w_, scales_, nullptr, M_, N_, K_), rope{r, row_base} {}
+  struct Dest {
+    Int8Walk::Dest product;
+    RopeStore::Dest rope;
+  };
+  __device__ __forceinline__ void dest(const Tile &tile, int row, int col, Dest &d) const {
+    Int8Walk::dest(tile, row, col, d.product);
+    rope.dest(tile.rb * 256 + row, d.rope);
+  }
+  __device__ __forceinline__ void store(const Tile &tile, Dest &d, int j, int q, int row, int col, float (&v)[8]) const {
+    rope.store(d.rope, j, q, tile.rb * 256 + row, M, out_col(tile, col), outputs(d.product, q, v));
+  }
+};
+
+__global__ __launch_bounds__(256, 1) void int8_unpacked_rope_kernel(const uint16_t *x, const uint16_t *w, const uint16_t *scales, const RopeRows r, int row_base, int M, int N, int K) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[gemm256::kRing];
+  Int8RopeWalk tiles(x, w, scales, r, row_base, M, N, K);
   gemm256::walk<false>(tiles, lds);
 #endif
 }
@@ -636,7 +746,50 @@ int int8_unpacked_gate(const uint16_t *x, const int8_t *q, const uint16_t *scale
   return launch_status();
 }
 
+// Scratch of a fused q | k | v product whose tiles rotate, transpose and write the caches themselves, or 0 where it is not taken.  Where the product alone runs on unpacked
+// weights this is it and no pass over its results behind it (four bytes an output at 5.9 TB/s), for 3 us a round of tiles: 49152 x 12288 x 4096 and the pass 3290 + 413 us, here 3420.
+int64_t int8_unpacked_rope_bytes(int64_t batch, int64_t seqlen, int64_t n_head, int64_t n_kv_head, int64_t cache_len, int64_t head_dim, int64_t K) {
+  constexpr int64_t kMost = (int64_t{1} << 32) - 512;  // bytes that a 32-bit offset reaches
+  if (batch < 1 || seqlen < 16 || n_head < 1 || n_kv_head < 1 || cache_len < 1 || (head_dim != 64 && head_dim != 128)) return 0;
+  if (batch > INT32_MAX / 2 / seqlen || n_head > INT32_MAX / 1024 || n_kv_head > INT32_MAX / 1024 || cache_len > INT32_MAX / 2 / head_dim) return 0;
+  const int64_t q = n_head * head_dim, kv = n_kv_head * head_dim;
+  if (q % 128 != 0 || kv % 128 != 0 || q > kMost / 2 / (batch * seqlen) || kv > kMost / 2 / batch / cache_len) return 0;
+  return int8_unpacked_bytes(batch * seqlen, q + 2 * kv, K);
+}
+
+int int8_unpacked_rope(const uint16_t *x, const int8_t *q, const uint16_t *scales, const RopeRows &r, int K, uint16_t *w, hipStream_t stream) {
+  const int N = (r.H + 2 * r.Hkv) * r.D, M = r.B * r.T;
+  const int64_t pieces = static_cast<int64_t>(N) * K / 16;
+  hipLaunchKernelGGL(unpack_int8_kernel, dim3(static_cast<unsigned>((pieces + 255) / 256)), dim3(256), 0, stream, q, w, pieces);
+  const int64_t most = rows_at_once(K);
+  for (int64_t m0 = 0; m0 < M; m0 += most) {
+    const int rows = static_cast<int>(M - m0 < most ? M - m0 : most);
+    hipLaunchKernelGGL(int8_unpacked_rope_kernel, dim3(grid_of(rows, N)), dim3(256), 0, stream, x + m0 * K, w, scales, r, static_cast<int>(m0), rows, N, K);
+  }
+  return launch_status();
+}
+
 }  // namespace e2h
+
+extern "C" int64_t e2h_int8_mm_rope_kv_rows_scratch_bytes(int64_t batch, int64_t seqlen, int64_t n_head, int64_t n_kv_head, int64_t cache_len, int64_t head_dim, int64_t k) {
+  return e2h::int8_unpacked_rope_bytes(batch, seqlen, n_head, n_kv_head, cache_len, head_dim, k);
+}
+
+extern "C" int e2h_int8_mm_rope_kv_rows(const uint16_t *x, const int8_t *q, const uint16_t *scales, const uint16_t *freqs_cis, int64_t freq_rows, uint16_t *q_out, uint16_t *k_cache,
+                                        uint16_t *v_cache, const int64_t *input_pos, int64_t batch, int64_t seqlen, int64_t n_head, int64_t n_kv_head, int64_t cache_len,
+                                        int64_t head_dim, int64_t k, int rows_by_token, void *scratch, int64_t scratch_bytes, void *stream) {
+  using namespace e2h;
+  if (!x || !q || !scales || !freqs_cis || !q_out || !k_cache || !v_cache || !input_pos || !scratch) return E2H_ERR_NULL_POINTER;
+  const int64_t need = int8_unpacked_rope_bytes(batch, seqlen, n_head, n_kv_head, cache_len, head_dim, k);
+  if (need == 0 || freq_rows < 1 || freq_rows > INT32_MAX / 2 / head_dim) return E2H_ERR_BAD_SHAPE;
+  if (scratch_bytes < need) return E2H_ERR_SCRATCH_TOO_SMALL;
+  if (!aligned16(x) || !aligned16(q) || !aligned16(scales) || !aligned16(freqs_cis) || !aligned16(q_out) || !aligned16(k_cache) || !aligned16(v_cache) || !aligned16(scratch) ||
+      (reinterpret_cast<uintptr_t>(input_pos) & 7u))
+    return E2H_ERR_MISALIGNED;
+  const RopeRows r = {freqs_cis, q_out, k_cache, v_cache, input_pos, static_cast<int>(batch), static_cast<int>(seqlen), static_cast<int>(n_head), static_cast<int>(n_kv_head),
+                      static_cast<int>(cache_len), static_cast<int>(head_dim), static_cast<int>(freq_rows), rows_by_token ? 1 : 0};
+  return int8_unpacked_rope(x, q, scales, r, static_cast<int>(k), static_cast<uint16_t *>(scratch), static_cast<hipStream_t>(stream));
+}
 
 extern "C" int64_t e2h_int8_mm_silu_gate_rows_scratch_bytes(int64_t m, int64_t n, int64_t k) {
   return m <= INT32_MAX ? e2h::int8_gate_unpacked_bytes(m, n, k) : 0;

@@ -193,6 +193,22 @@ class Attention(nn.Module):
             return True
         return self.kv_cache is not None and self.freqs_table.shape[0] >= self.kv_cache.k_cache.shape[2]
 
+    def _rope_rows(self, x: Tensor, k: Tensor, v: Tensor, input_pos: Tensor, rows_by_token: bool) -> Optional[Tensor]:
+        """The rotated q of a prompt, k and v written, with the projection in the same launch, or None where the module is to be called: few rows, weights of another form or that do not
+        fit x, or somebody who watches its calls."""
+        w = self.wqkv
+        if not FUSE_ROPE_PROJECTION or torch.compiler.is_compiling() or type(w) is not WeightOnlyInt8Linear:
+            return None
+        scales, n, f = w.scales, self.dim + 2 * self.n_local_heads * self.head_dim, self.freqs_table
+        if not (x.numel() > 64 * x.shape[-1] and w.weight.dtype == torch.int8 and scales.dtype == torch.bfloat16 and tuple(w.weight.shape) == (n, x.shape[-1]) and tuple(scales.shape) == (n,)
+                and self.n_head * self.head_dim == self.dim and tuple(f.shape[1:]) == (self.head_dim // 2, 2) and k.dtype == v.dtype == torch.bfloat16 and v.shape == k.shape
+                and k.shape[0] >= x.shape[0] and k.shape[1] == self.n_local_heads and k.shape[3] == self.head_dim
+                and all(t.device == x.device for t in (w.weight, scales, f, k, v, input_pos)) and all(t.is_contiguous() for t in (f, k, v)) and unwatched(w)):
+            return None
+        if seq_ops.watched(x, w.weight, scales, f, k, v, input_pos):
+            return None
+        return ops.int8_mm_rope_kv_rows(x, w.weight, scales, f, k, v, input_pos, self.n_head, self.n_local_heads, self.head_dim, rows_by_token)
+
     def forward(self, x: Tensor, freqs_cis: Optional[Tensor], mask: Optional[Tensor], input_pos: Optional[Tensor] = None,
                 fully_causal: bool = False, defer_output: bool = False) -> Tensor:
         """defer_output (fused decode step only): the output projection may come back as float32 partial sums over K
@@ -219,16 +235,17 @@ class Attention(nn.Module):
                 return _project_deferred(self.wo, y.view(bsz, self.dim), (bsz, 1))
             return self.wo(y.view(bsz, 1, self.dim))
         if self._can_fuse_prefill_rope(x, input_pos, fully_causal):
-            # many new tokens per sequence: rotation, head-major layout and cache write in one pass over qkv
-            qkv = self.wqkv(x)
+            # many new tokens per sequence: rotation, head-major layout and cache write in one pass over qkv, or in the projection's own launch
             if fully_causal:
                 # no cache: k and v of exactly this length, rows in token order; the angles are those of input_pos
                 k = torch.empty((bsz, self.n_local_heads, seqlen, self.head_dim), dtype=torch.bfloat16, device=x.device)
                 v = torch.empty_like(k)
             else:
                 k, v = self.kv_cache.k_cache, self.kv_cache.v_cache
-            q = ops.rope_kv_write_seq(qkv, self.freqs_table, k, v, input_pos, self.n_head, self.n_local_heads, self.head_dim,
-                                      rows_by_token=fully_causal)
+            q = self._rope_rows(x, k, v, input_pos, fully_causal)
+            if q is None:
+                q = ops.rope_kv_write_seq(self.wqkv(x), self.freqs_table, k, v, input_pos, self.n_head, self.n_local_heads, self.head_dim,
+                                          rows_by_token=fully_causal)
             if ((fully_causal or isinstance(mask, _MaskByPosition)) and not torch.compiler.is_compiling()
                     and ops.prefill_attention_fits(bsz, seqlen, self.n_head, k, v, not fully_causal) and not seq_ops.watched(q, k, v) and not _stock_attention_wanted()):
                 y = ops.prefill_attention(q, k, v, None if fully_causal else input_pos, None if fully_causal else mask.left_pad)

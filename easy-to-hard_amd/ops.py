@@ -728,6 +728,32 @@ def int8_mm_silu_gate_rows(x, q_gate, scales_gate, q_up, scales_up):
     return y
 
 
+def int8_mm_rope_kv_rows(x, q_weight, scales, freqs_cis, k_cache, v_cache, input_pos, n_head, n_kv_head, head_dim, rows_by_token=False):
+    """rope_kv_write_seq(int8_mm(x, q_weight, scales), ..), x bf16 [B, T, K], in one product launch: the rotated q [B, H, T, D], or None where the sizes are not taken (or there
+    is no memory for the launch's scratch)."""
+    _need_gpu(x, q_weight, scales, freqs_cis, k_cache, v_cache, input_pos)
+    assert x.dtype == torch.bfloat16 and x.dim() == 3 and q_weight.dtype == torch.int8 and scales.dtype == torch.bfloat16 and freqs_cis.dtype == torch.bfloat16
+    assert input_pos.dtype == torch.int64 and k_cache.dtype == torch.bfloat16 and v_cache.dtype == torch.bfloat16
+    assert k_cache.is_contiguous() and v_cache.is_contiguous() and freqs_cis.is_contiguous()
+    bsz, t, k = x.shape
+    assert input_pos.numel() == t and tuple(q_weight.shape) == ((n_head + 2 * n_kv_head) * head_dim, k) and scales.numel() == q_weight.shape[0]
+    assert k_cache.shape[0] >= bsz and k_cache.shape[1] == n_kv_head and k_cache.shape[3] == head_dim and v_cache.shape == k_cache.shape
+    assert tuple(freqs_cis.shape[1:]) == (head_dim // 2, 2) and (rows_by_token or freqs_cis.shape[0] >= k_cache.shape[2])
+    lib = _lib_for(x)
+    sizes = (t, n_head, n_kv_head, k_cache.shape[2], head_dim, k)
+    scratch = _unpacked_weight(bsz * t, x.device, lambda rows, *rest: lib.e2h_int8_mm_rope_kv_rows_scratch_bytes(bsz, *rest), *sizes)
+    if scratch is None:
+        return None
+    x, q_weight, scales, input_pos = x.contiguous(), q_weight.contiguous(), scales.contiguous(), input_pos.contiguous()
+    if any(a.data_ptr() % 16 for a in (x, q_weight, scales, freqs_cis, k_cache, v_cache)):
+        return None
+    q = torch.empty((bsz, n_head, t, head_dim), dtype=torch.bfloat16, device=x.device)
+    rc = lib.e2h_int8_mm_rope_kv_rows(_ptr(x), _ptr(q_weight), _ptr(scales), _ptr(freqs_cis), freqs_cis.shape[0], _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(input_pos), bsz, *sizes,
+                                      1 if rows_by_token else 0, _ptr(scratch), scratch.numel(), _stream(x))
+    _lib.check(rc, "e2h_int8_mm_rope_kv_rows")
+    return q
+
+
 def int8_rope_kv_supported(x, wqkv, freqs_cis, k_cache):
     """True when the fused projection + RoPE + cache write covers (x [B, 1, K], a WeightOnlyInt8Linear)."""
     return _int8_fusable(x, wqkv) and freqs_cis.shape[0] >= k_cache.shape[2]

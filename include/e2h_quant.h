@@ -209,6 +209,13 @@ int64_t e2h_int4_mm_silu_gate_rows_scratch_bytes(int64_t m, int64_t n, int64_t k
 int64_t e2h_int8_mm_silu_gate_rows_scratch_bytes(int64_t m, int64_t n, int64_t k);
 int e2h_int8_mm_silu_gate_rows(const uint16_t *x, const int8_t *q_gate, const uint16_t *scales_gate, const int8_t *q_up, const uint16_t *scales_up, uint16_t *y,
                                int64_t m, int64_t n, int64_t k, void *scratch, int64_t scratch_bytes, void *stream);
+/* The fused int8 q | k | v projection of many rows with e2h_rope_kv_write_seq behind it in the same launch, bit for bit what e2h_int8_mm_scratch and that call give: x [batch * seqlen, k],
+ * q [(n_head + 2 n_kv_head) * head_dim, k], freqs_cis [freq_rows, head_dim / 2, 2], the rest as there.  head_dim 64 or 128, n_head * head_dim and n_kv_head * head_dim multiples of 128,
+ * 16 <= seqlen, k % 128 == 0; every pointer but input_pos 16-byte aligned.  The first function returns 0 where the shape is not taken. */
+int64_t e2h_int8_mm_rope_kv_rows_scratch_bytes(int64_t batch, int64_t seqlen, int64_t n_head, int64_t n_kv_head, int64_t cache_len, int64_t head_dim, int64_t k);
+int e2h_int8_mm_rope_kv_rows(const uint16_t *x, const int8_t *q, const uint16_t *scales, const uint16_t *freqs_cis, int64_t freq_rows, uint16_t *q_out, uint16_t *k_cache, uint16_t *v_cache,
+                             const int64_t *input_pos, int64_t batch, int64_t seqlen, int64_t n_head, int64_t n_kv_head, int64_t cache_len, int64_t head_dim, int64_t k, int rows_by_token,
+                             void *scratch, int64_t scratch_bytes, void *stream);
 /* (int4) 1 where that launch is expected to take less time than two calls of e2h_int4_mm and e2h_silu_mul, whichever kernels those run, else 0 (a subset of the shapes that are taken). */
 int e2h_int4_mm_silu_gate_rows_pays(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles);
 int e2h_int4_mm_silu_gate_rows(const uint16_t *x, const int32_t *packed_gate, const uint16_t *sz_gate, const int32_t *packed_up,

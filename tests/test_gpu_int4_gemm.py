@@ -525,3 +525,56 @@ def test_gated_int8_rows_leave_watched_modules_to_the_modules():
     assert (ff(x).double() - whole.double()).norm() <= 2.0 ** -7 * whole.double().norm() and seen == [1]
     handle.remove()
     assert ff._gate_rows(x.float()) is None and ff._gate_rows(x[:, :20]) is None
+
+
+@pytest.mark.parametrize("by_token", [False, True])
+@pytest.mark.parametrize("bsz,t,heads,kv_heads,length,d,k", [
+    (4141, 17, 2, 2, 40, 64, 256),          # a lane's rows 16 apart lie in as many sequences; two heads per 128 columns, a last tile of 128 columns
+    (70, 1003, 4, 2, 1100, 128, 256),       # fewer heads of k and v
+    (3, 1000, 32, 32, 1000, 128, 384),      # a last tile of 184 rows
+    (41, 1601, 1, 1, 1700, 128, 32768),     # x of more than 4 GB, in two slices of rows
+])
+def test_int8_projection_that_rotates_and_writes_the_caches(bsz, t, heads, kv_heads, length, d, k, by_token):
+    """Whole numbers as operands, so that products are exact whatever the order of their sums and the two ways agree bit for bit; tokens without a place in the cache write nothing."""
+    gen = torch.Generator(device=DEV).manual_seed(t + k)
+    n = (heads + 2 * kv_heads) * d
+    x = torch.empty((bsz, t, k), dtype=torch.bfloat16, device=DEV)
+    for row in x:
+        row.copy_(torch.randint(-8, 9, (t, k), generator=gen, device=DEV, dtype=torch.int8))
+    q = torch.randint(-128, 128, (n, k), generator=gen, device=DEV, dtype=torch.int8)
+    s = (torch.rand((n,), generator=gen, device=DEV) * 0.002).to(torch.bfloat16)
+    freqs = torch.randn((2000, d // 2, 2), generator=gen, device=DEV).to(torch.bfloat16)
+    pos = torch.randperm(t, generator=gen, device=DEV) + (300 if by_token else length - t)
+    rows, there = t if by_token else length, torch.ones(t, dtype=torch.bool, device=DEV)
+    if not by_token:
+        pos[t // 2], pos[t // 3] = length, -1
+        there[t // 2] = there[t // 3] = False
+    before = [torch.randn((bsz, kv_heads, rows, d), generator=gen, device=DEV).to(torch.bfloat16) for _ in range(2)]
+    got, want = [c.clone() for c in before], before
+    q_got = ops.int8_mm_rope_kv_rows(x, q, s, freqs, *got, pos, heads, kv_heads, d, by_token)
+    assert q_got is not None
+    q_want = ops.rope_kv_write_seq(ops.int8_mm(x.view(-1, k), q, s).view(bsz, t, n), freqs, *want, pos, heads, kv_heads, d, by_token)
+    assert torch.equal(q_got[:, :, there], q_want[:, :, there]) and torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+def test_int8_prompts_leave_watched_projections_to_the_modules():
+    from easy_to_hard_amd.model import Attention, ModelArgs, precompute_freqs_cis
+    from easy_to_hard_amd.quantize import WeightOnlyInt8QuantHandler
+
+    att = Attention(ModelArgs(dim=4096, n_head=32, n_local_heads=32, n_layer=1, intermediate_size=64))
+    WeightOnlyInt8QuantHandler(att).convert_for_runtime()
+    gen = torch.Generator().manual_seed(1)
+    for lin in (att.wqkv, att.wo):
+        lin.weight = torch.randint(-128, 128, (lin.out_features, lin.in_features), generator=gen, dtype=torch.int8).to(DEV)
+        lin.scales = torch.full((lin.out_features,), 2.0 ** -13, dtype=torch.bfloat16, device=DEV)
+    att.freqs_table = precompute_freqs_cis(1024, 128, 10000, device=DEV)
+    x, pos = torch.randn((3, 1000, 4096), generator=gen).to(torch.bfloat16).to(DEV), torch.arange(1000, device=DEV)
+    k, v = torch.empty((2, 3, 32, 1000, 128), dtype=torch.bfloat16, device=DEV)
+    with torch.no_grad():
+        assert att._rope_rows(x, k, v, pos, True).shape == (3, 32, 1000, 128)
+        whole, seen = att(x, None, None, pos, True), []
+        handle = att.wqkv.register_forward_hook(lambda *_: seen.append(1))
+        assert att._rope_rows(x, k, v, pos, True) is None and seen == []
+        assert torch.equal(att(x, None, None, pos, True), whole) and seen == [1]
+        handle.remove()
+        assert att._rope_rows(x[:, :20], k, v, pos[:20], True) is None and att._rope_rows(x, k.transpose(0, 1), v.transpose(0, 1), pos, True) is None
