@@ -65,6 +65,8 @@ _SIGNATURES = {
     "e2h_int8_mm_silu_gate_rows": (c_int, [_P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, _P, c_int64, _P]),
     "e2h_int8_mm_rope_kv_rows_scratch_bytes": (c_int64, [c_int64] * 7),
     "e2h_int8_mm_rope_kv_rows": (c_int, [_P, _P, _P, _P, c_int64, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, _P, c_int64, _P]),
+    "e2h_int4_mm_rope_kv_rows_scratch_bytes": (c_int64, [c_int64] * 7 + [c_int, c_int]),
+    "e2h_int4_mm_rope_kv_rows": (c_int, [_P, _P, _P, _P, c_int64, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_int, c_int, _P, c_int64, _P]),
     "e2h_int8_norm_mm_supported": (c_int, [c_int64, c_int64, c_int64]),
     "e2h_int8_norm_mm": (c_int, [ctypes.POINTER(RowNorm), _P, _P, _P, c_int64, c_int64, c_int64, _P]),
     "e2h_int8_norm_mm_silu_gate": (c_int, [ctypes.POINTER(RowNorm), _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, _P]),

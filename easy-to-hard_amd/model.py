@@ -197,17 +197,26 @@ class Attention(nn.Module):
         """The rotated q of a prompt, k and v written, with the projection in the same launch, or None where the module is to be called: few rows, weights of another form or that do not
         fit x, or somebody who watches its calls."""
         w = self.wqkv
-        if not FUSE_ROPE_PROJECTION or torch.compiler.is_compiling() or type(w) is not WeightOnlyInt8Linear:
+        if not FUSE_ROPE_PROJECTION or torch.compiler.is_compiling() or type(w) not in (WeightOnlyInt4Linear, WeightOnlyInt8Linear) or x.shape[0] * x.shape[1] < ops._UNPACK_ROWS:
             return None
-        scales, n, f = w.scales, self.dim + 2 * self.n_local_heads * self.head_dim, self.freqs_table
-        if not (x.numel() > 64 * x.shape[-1] and w.weight.dtype == torch.int8 and scales.dtype == torch.bfloat16 and tuple(w.weight.shape) == (n, x.shape[-1]) and tuple(scales.shape) == (n,)
-                and self.n_head * self.head_dim == self.dim and tuple(f.shape[1:]) == (self.head_dim // 2, 2) and k.dtype == v.dtype == torch.bfloat16 and v.shape == k.shape
-                and k.shape[0] >= x.shape[0] and k.shape[1] == self.n_local_heads and k.shape[3] == self.head_dim
-                and all(t.device == x.device for t in (w.weight, scales, f, k, v, input_pos)) and all(t.is_contiguous() for t in (f, k, v)) and unwatched(w)):
+        width, n, f = x.shape[-1], self.dim + 2 * self.n_local_heads * self.head_dim, self.freqs_table
+        if type(w) is WeightOnlyInt8Linear:
+            weights = w.weight, w.scales
+            fits = w.weight.dtype == torch.int8 and tuple(w.weight.shape) == (n, width) and tuple(w.scales.shape) == (n,)
+        else:
+            weights, p = (w.weight, w.scales_and_zeros), w.weight
+            fits = (not w.padding and w.in_features == width and w.out_features == n and p.dtype == torch.int32 and p.dim() == 4 and p.shape[3] == 4 and p.shape[2] == 32
+                    and p.shape[0] * 8 == n and p.shape[1] * 128 == width and tuple(w.scales_and_zeros.shape) == (width // w.groupsize, n, 2))
+        if not (fits and weights[1].dtype == torch.bfloat16 and self.n_head * self.head_dim == self.dim and tuple(f.shape[1:]) == (self.head_dim // 2, 2)
+                and k.dtype == v.dtype == torch.bfloat16 and v.shape == k.shape and k.shape[0] >= x.shape[0] and k.shape[1] == self.n_local_heads and k.shape[3] == self.head_dim
+                and all(t.device == x.device for t in (*weights, f, k, v, input_pos)) and all(t.is_contiguous() for t in (f, k, v)) and unwatched(w)):
             return None
-        if seq_ops.watched(x, w.weight, scales, f, k, v, input_pos):
+        if seq_ops.watched(x, *weights, f, k, v, input_pos):
             return None
-        return ops.int8_mm_rope_kv_rows(x, w.weight, scales, f, k, v, input_pos, self.n_head, self.n_local_heads, self.head_dim, rows_by_token)
+        heads = self.n_head, self.n_local_heads, self.head_dim, rows_by_token
+        if type(w) is WeightOnlyInt8Linear:
+            return ops.int8_mm_rope_kv_rows(x, *weights, f, k, v, input_pos, *heads)
+        return ops.int4_mm_rope_kv_rows(x, *weights, w.groupsize, f, k, v, input_pos, *heads)
 
     def forward(self, x: Tensor, freqs_cis: Optional[Tensor], mask: Optional[Tensor], input_pos: Optional[Tensor] = None,
                 fully_causal: bool = False, defer_output: bool = False) -> Tensor:

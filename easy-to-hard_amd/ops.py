@@ -728,30 +728,46 @@ def int8_mm_silu_gate_rows(x, q_gate, scales_gate, q_up, scales_up):
     return y
 
 
-def int8_mm_rope_kv_rows(x, q_weight, scales, freqs_cis, k_cache, v_cache, input_pos, n_head, n_kv_head, head_dim, rows_by_token=False):
-    """rope_kv_write_seq(int8_mm(x, q_weight, scales), ..), x bf16 [B, T, K], in one product launch: the rotated q [B, H, T, D], or None where the sizes are not taken (or there
-    is no memory for the launch's scratch)."""
-    _need_gpu(x, q_weight, scales, freqs_cis, k_cache, v_cache, input_pos)
-    assert x.dtype == torch.bfloat16 and x.dim() == 3 and q_weight.dtype == torch.int8 and scales.dtype == torch.bfloat16 and freqs_cis.dtype == torch.bfloat16
+def _rope_rows(x, weights, name, options, freqs_cis, k_cache, v_cache, input_pos, n_head, n_kv_head, head_dim, rows_by_token):
+    """The launches of the two functions below."""
+    _need_gpu(x, *weights, freqs_cis, k_cache, v_cache, input_pos)
+    assert x.dtype == torch.bfloat16 and x.dim() == 3 and freqs_cis.dtype == torch.bfloat16
     assert input_pos.dtype == torch.int64 and k_cache.dtype == torch.bfloat16 and v_cache.dtype == torch.bfloat16
     assert k_cache.is_contiguous() and v_cache.is_contiguous() and freqs_cis.is_contiguous()
     bsz, t, k = x.shape
-    assert input_pos.numel() == t and tuple(q_weight.shape) == ((n_head + 2 * n_kv_head) * head_dim, k) and scales.numel() == q_weight.shape[0]
-    assert k_cache.shape[0] >= bsz and k_cache.shape[1] == n_kv_head and k_cache.shape[3] == head_dim and v_cache.shape == k_cache.shape
+    assert input_pos.numel() == t and k_cache.shape[0] >= bsz and k_cache.shape[1] == n_kv_head and k_cache.shape[3] == head_dim and v_cache.shape == k_cache.shape
     assert tuple(freqs_cis.shape[1:]) == (head_dim // 2, 2) and (rows_by_token or freqs_cis.shape[0] >= k_cache.shape[2])
     lib = _lib_for(x)
-    sizes = (t, n_head, n_kv_head, k_cache.shape[2], head_dim, k)
-    scratch = _unpacked_weight(bsz * t, x.device, lambda rows, *rest: lib.e2h_int8_mm_rope_kv_rows_scratch_bytes(bsz, *rest), *sizes)
+    sizes = (t, n_head, n_kv_head, k_cache.shape[2], head_dim, k, *options)
+    scratch = _unpacked_weight(bsz * t, x.device, lambda rows, *rest: getattr(lib, name + "_scratch_bytes")(bsz, *rest), *sizes)
     if scratch is None:
         return None
-    x, q_weight, scales, input_pos = x.contiguous(), q_weight.contiguous(), scales.contiguous(), input_pos.contiguous()
-    if any(a.data_ptr() % 16 for a in (x, q_weight, scales, freqs_cis, k_cache, v_cache)):
+    x, input_pos, weights = x.contiguous(), input_pos.contiguous(), [w.contiguous() for w in weights]
+    if any(a.data_ptr() % 16 for a in (x, *weights, freqs_cis, k_cache, v_cache)):
         return None
     q = torch.empty((bsz, n_head, t, head_dim), dtype=torch.bfloat16, device=x.device)
-    rc = lib.e2h_int8_mm_rope_kv_rows(_ptr(x), _ptr(q_weight), _ptr(scales), _ptr(freqs_cis), freqs_cis.shape[0], _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(input_pos), bsz, *sizes,
-                                      1 if rows_by_token else 0, _ptr(scratch), scratch.numel(), _stream(x))
-    _lib.check(rc, "e2h_int8_mm_rope_kv_rows")
+    rc = getattr(lib, name)(_ptr(x), *map(_ptr, weights), _ptr(freqs_cis), freqs_cis.shape[0], _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(input_pos), bsz, *sizes,
+                            1 if rows_by_token else 0, _ptr(scratch), scratch.numel(), _stream(x))
+    _lib.check(rc, name)
     return q
+
+
+def int8_mm_rope_kv_rows(x, q_weight, scales, freqs_cis, k_cache, v_cache, input_pos, n_head, n_kv_head, head_dim, rows_by_token=False):
+    """rope_kv_write_seq(int8_mm(x, q_weight, scales), ..), x bf16 [B, T, K], in one product launch: the rotated q [B, H, T, D], or None where the sizes are not taken (or there
+    is no memory for the launch's scratch)."""
+    assert q_weight.dtype == torch.int8 and scales.dtype == torch.bfloat16
+    assert tuple(q_weight.shape) == ((n_head + 2 * n_kv_head) * head_dim, x.shape[-1]) and scales.numel() == q_weight.shape[0]
+    return _rope_rows(x, (q_weight, scales), "e2h_int8_mm_rope_kv_rows", (), freqs_cis, k_cache, v_cache, input_pos, n_head, n_kv_head, head_dim, rows_by_token)
+
+
+def int4_mm_rope_kv_rows(x, packed, scales_and_zeros, groupsize, freqs_cis, k_cache, v_cache, input_pos, n_head, n_kv_head, head_dim, rows_by_token=False):
+    """The same of int4_mm(x, packed, groupsize, scales_and_zeros)."""
+    assert packed.dtype == torch.int32 and packed.dim() == 4 and scales_and_zeros.dtype == torch.bfloat16
+    inner_k_tiles, k = packed.shape[3] * 2, x.shape[-1]
+    n = (n_head + 2 * n_kv_head) * head_dim
+    assert packed.shape[0] * 8 == n and packed.shape[1] * 16 * inner_k_tiles == k and packed.shape[2] == 32 and tuple(scales_and_zeros.shape) == (k // groupsize, n, 2)
+    return _rope_rows(x, (packed, scales_and_zeros), "e2h_int4_mm_rope_kv_rows", (groupsize, inner_k_tiles), freqs_cis, k_cache, v_cache, input_pos, n_head, n_kv_head, head_dim,
+                      rows_by_token)
 
 
 def int8_rope_kv_supported(x, wqkv, freqs_cis, k_cache):

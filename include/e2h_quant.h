@@ -216,6 +216,13 @@ int64_t e2h_int8_mm_rope_kv_rows_scratch_bytes(int64_t batch, int64_t seqlen, in
 int e2h_int8_mm_rope_kv_rows(const uint16_t *x, const int8_t *q, const uint16_t *scales, const uint16_t *freqs_cis, int64_t freq_rows, uint16_t *q_out, uint16_t *k_cache, uint16_t *v_cache,
                              const int64_t *input_pos, int64_t batch, int64_t seqlen, int64_t n_head, int64_t n_kv_head, int64_t cache_len, int64_t head_dim, int64_t k, int rows_by_token,
                              void *scratch, int64_t scratch_bytes, void *stream);
+/* The same of an int4 projection (packed, scales_and_zeros, groupsize, inner_k_tiles as for e2h_int4_mm; from 1024 rows on), bit for bit what e2h_int4_mm_scratch and
+ * e2h_rope_kv_write_seq give. */
+int64_t e2h_int4_mm_rope_kv_rows_scratch_bytes(int64_t batch, int64_t seqlen, int64_t n_head, int64_t n_kv_head, int64_t cache_len, int64_t head_dim, int64_t k, int groupsize,
+                                               int inner_k_tiles);
+int e2h_int4_mm_rope_kv_rows(const uint16_t *x, const int32_t *packed, const uint16_t *scales_and_zeros, const uint16_t *freqs_cis, int64_t freq_rows, uint16_t *q_out, uint16_t *k_cache,
+                             uint16_t *v_cache, const int64_t *input_pos, int64_t batch, int64_t seqlen, int64_t n_head, int64_t n_kv_head, int64_t cache_len, int64_t head_dim, int64_t k,
+                             int groupsize, int inner_k_tiles, int rows_by_token, void *scratch, int64_t scratch_bytes, void *stream);
 /* (int4) 1 where that launch is expected to take less time than two calls of e2h_int4_mm and e2h_silu_mul, whichever kernels those run, else 0 (a subset of the shapes that are taken). */
 int e2h_int4_mm_silu_gate_rows_pays(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles);
 int e2h_int4_mm_silu_gate_rows(const uint16_t *x, const int32_t *packed_gate, const uint16_t *sz_gate, const int32_t *packed_up,

@@ -557,6 +557,40 @@ def test_int8_projection_that_rotates_and_writes_the_caches(bsz, t, heads, kv_he
     assert torch.equal(q_got[:, :, there], q_want[:, :, there]) and torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
+@pytest.mark.parametrize("by_token", [False, True])
+@pytest.mark.parametrize("g,bsz,t,heads,kv_heads,length,d,k", [
+    (32, 70, 1003, 4, 2, 1100, 128, 256),
+    (64, 70, 1003, 4, 2, 1100, 128, 512),
+    (128, 4141, 17, 2, 2, 40, 64, 256),
+    (256, 32, 256, 32, 32, 300, 128, 4096),
+])
+def test_int4_projection_that_rotates_and_writes_the_caches(g, bsz, t, heads, kv_heads, length, d, k, by_token):
+    """Bit for bit the product and the pass behind it, also with rows and (then) a scale that the other kernel takes."""
+    gen = torch.Generator(device=DEV).manual_seed(t + k)
+    n, m = (heads + 2 * kv_heads) * d, bsz * t
+    x = torch.randn((m, k), generator=gen, device=DEV).to(torch.bfloat16)
+    x[7, 5], x[1300, 9] = float("inf"), float("nan")
+    x[900, 1:40] *= 2.0 ** -40
+    packed, sz = ops.int4_quantize_pack((torch.randn((n, k), generator=gen, device=DEV) * 0.02).to(torch.bfloat16), g, 8)
+    freqs = torch.randn((2000, d // 2, 2), generator=gen, device=DEV).to(torch.bfloat16)
+    pos = torch.randperm(t, generator=gen, device=DEV) + (300 if by_token else length - t)
+    rows, there = t if by_token else length, torch.ones(t, dtype=torch.bool, device=DEV)
+    if not by_token:
+        pos[t // 2 - 2], pos[3] = length, -1  # (not the planted rows' tokens: what those give is compared, too)
+        there[t // 2 - 2] = there[3] = False
+    for plant in (False, True):
+        if plant:
+            sz[0, 33, 0] = float("inf")
+        got = torch.randn((2, bsz, kv_heads, rows, d), generator=gen, device=DEV).to(torch.bfloat16)
+        want = got.clone()
+        q_got = ops.int4_mm_rope_kv_rows(x.view(bsz, t, k), packed, sz, g, freqs, *got, pos, heads, kv_heads, d, by_token)
+        assert q_got is not None
+        q_want = ops.rope_kv_write_seq(ops.int4_mm(x, packed, g, sz).view(bsz, t, n), freqs, *want, pos, heads, kv_heads, d, by_token)
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got.nan_to_num(), want.nan_to_num()) and torch.isnan(want).any()
+        a, b = q_got[:, :, there], q_want[:, :, there]
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(a.nan_to_num(), b.nan_to_num())
+
+
 def test_int8_prompts_leave_watched_projections_to_the_modules():
     from easy_to_hard_amd.model import Attention, ModelArgs, precompute_freqs_cis
     from easy_to_hard_amd.quantize import WeightOnlyInt8QuantHandler
