@@ -13,24 +13,54 @@ SeqOptions &seq_options() {
 
 namespace {
 
-// One workgroup per run of `run` consecutive tokens of one sequence, NB tokens at a time so that the loads of NB rows are in
-// flight together and one barrier serves NB row sums.  A thread owns NP pieces of four channels, so the convolution's previous
-// inputs stay in its registers from token to token; the taps - 1 tokens ahead of the run are normalised again by the
+#if defined(__HIP_DEVICE_COMPILE__)
+constexpr int kStreamed = 2;  // cache policy of a buffer store whose line nobody reads soon
+
+// four values of a row from piece `at` (four channels each) on
+template <typename T>
+__device__ __forceinline__ Quad<T> buffer_quad(__amdgpu_buffer_rsrc_t row, int at) {
+  Quad<T> q;
+  if constexpr (sizeof(T) == 4) q.raw = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(row, at * 16, 0, 0));
+  else q.raw = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(row, at * 8, 0, 0));
+  return q;
+}
+template <int POLICY>
+__device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t row, int at, f32x4_t v, float) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), row, at * 16, 0, POLICY);
+}
+template <int POLICY>
+__device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t row, int at, f32x4_t v, bf16_t) {
+  __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])}, row, at * 8, 0, POLICY);
+}
+#endif
+
+// One row per workgroup, or with a convolution (which needs its previous inputs) a run of `run` consecutive tokens of one sequence.  A thread owns NP pieces of four channels, so the
+// convolution's previous inputs stay in its registers from token to token; the taps - 1 tokens ahead of the run are normalised again by the
 // workgroup (inside the call) or come from the ring of kept inputs (before the call).  TAPS is the compiled depth of the
 // convolution (0 = none); shallower ones pad their weights with zeros in front.  LAYER: layer norms; the waves' means and squared
 // deviations are merged by their counts, so a row still costs one barrier per norm and no sum of squares cancels.
-template <typename T, int BLOCK, int NP, int TAPS, int NB, bool LAYER>
-__global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_args a, int runs, int run) {
+//
+// What bounds it: memory, once enough rows are on their way.  A run's workgroup asks for its next row before it waits for anything of this one (AHEAD): loads and stores have no branch
+// between them, or a wait for one row's loads would be one for all.  Without a convolution rows next to each other are at work at the same time, which beats runs with the next row on its
+// way (8192 x 4096, sum and norm 72 us, 80 in runs of 8), and large residual rows, which are not read again soon, are stored past the caches (58).
+// us at 4096 channels, in brackets runs of 8 (convolution: 1024 threads, two rows together) that waited for every row: 8192 rows with residual 58 (94), layer norm 63 (91), eight experts'
+// terms 161 (187), convolution 73 (101); 8000 rows 56 (85), 62 (106), 159 (214), 66 (167: one workgroup too many for a round); 2048 rows 17 (18), 20 (21), 39 (38), 25 (33).
+template <typename T, int BLOCK, int NP, int TAPS, bool LAYER, bool TERMS, bool AHEAD>
+__global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_args a, int runs, int run, int streamed) {
+#if defined(__HIP_DEVICE_COMPILE__)
   constexpr int kWaves = BLOCK / 64;
   constexpr int RING = TAPS > 1 ? TAPS - 1 : 1;
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
   const int W = static_cast<int>(a.width), seqlen = static_cast<int>(a.seqlen), taps = a.taps;
-  const int b = blockIdx.x / runs, t_begin = (blockIdx.x % runs) * run;
-  const int t_end = t_begin + run < seqlen ? t_begin + run : seqlen;
+  // without a convolution rows know nothing of their sequence
+  const int b = TAPS ? blockIdx.x / runs : 0, t_begin = TAPS ? (blockIdx.x % runs) * run : blockIdx.x;
+  const int64_t t_end = TAPS ? t_begin + run < seqlen ? t_begin + run : seqlen : a.batch * a.seqlen;
+  const int step = TAPS ? 1 : static_cast<int>(gridDim.x);
   const int pos0 = TAPS ? static_cast<int>(a.input_pos[0]) : 0;
   const int first = TAPS && a.first ? static_cast<int>(a.first[b]) : 0;
   const size_t row0 = static_cast<size_t>(b) * seqlen;
-  __shared__ float part[2][kWaves][NB * (LAYER ? 2 : 1)];
+  const uint32_t row_f32 = static_cast<uint32_t>(W) * 4, row_t = static_cast<uint32_t>(W) * sizeof(T);
+  __shared__ __attribute__((aligned(16))) float part[2][kWaves][LAYER ? 2 : 1];
   int phase = 0;
 
   auto wave_count = [&](int w) {  // channels of the row that wave w holds
@@ -42,83 +72,69 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
     }
     return static_cast<float>(n);
   };
-  // z -> (z - mean) / sqrt(variance + eps) * weight + bias for NB rows
-  auto layer_norm = [&](f32x4_t (&z)[NB][NP], const f32x4_t (&weight)[NP], const float *bias) {
+  auto piece = [&](int p) { return p * BLOCK + static_cast<int>(threadIdx.x); };
+  // z -> (z - mean) / sqrt(variance + eps) * weight + bias
+  auto layer_norm = [&](f32x4_t (&z)[NP], const f32x4_t (&weight)[NP], const f32x4_t (&bias)[NP]) {
     const float own = wave_count(threadIdx.x >> 6);
-    float mean[NB], dev[NB];
+    float s = 0.f;  // pieces beyond the width are zero
 #pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      float s = 0.f;  // pieces beyond the width are zero
+    for (int p = 0; p < NP; ++p) s += z[p][0] + z[p][1] + z[p][2] + z[p][3];
+    const float mean = own > 0.f ? wave_add(s) / own : 0.f;
+    float q = 0.f;
 #pragma unroll
-      for (int p = 0; p < NP; ++p) s += z[k][p][0] + z[k][p][1] + z[k][p][2] + z[k][p][3];
-      mean[k] = own > 0.f ? wave_add(s) / own : 0.f;
-      float q = 0.f;
+    for (int p = 0; p < NP; ++p)
+      if (piece(p) * 4 < W) {
+        const f32x4_t c = z[p] - mean;
 #pragma unroll
-      for (int p = 0; p < NP; ++p)
-        if ((p * BLOCK + static_cast<int>(threadIdx.x)) * 4 < W) {
-          const f32x4_t c = z[k][p] - mean[k];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) q = __builtin_fmaf(c[e], c[e], q);
-        }
-      dev[k] = wave_add(q);
-    }
-    if ((threadIdx.x & 63) == 0) {
-#pragma unroll
-      for (int k = 0; k < NB; ++k) {
-        part[phase][threadIdx.x >> 6][k] = mean[k];
-        part[phase][threadIdx.x >> 6][(LAYER ? NB : 0) + k] = dev[k];
+        for (int e = 0; e < 4; ++e) q = __builtin_fmaf(c[e], c[e], q);
       }
+    q = wave_add(q);
+    if ((threadIdx.x & 63) == 0) {
+      part[phase][threadIdx.x >> 6][0] = mean;
+      part[phase][threadIdx.x >> 6][LAYER ? 1 : 0] = q;
     }
     __syncthreads();
+    float m = 0.f, v = 0.f;
 #pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      float m = 0.f, v = 0.f;
+    for (int w = 0; w < kWaves; ++w) m = __builtin_fmaf(wave_count(w), part[phase][w][0], m);
+    m /= static_cast<float>(W);
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) m = __builtin_fmaf(wave_count(w), part[phase][w][k], m);
-      m /= static_cast<float>(W);
-#pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
-        const float c = part[phase][w][k] - m;
-        v += __builtin_fmaf(wave_count(w) * c, c, part[phase][w][(LAYER ? NB : 0) + k]);
-      }
-      const float r = 1.0f / sqrtf(v / static_cast<float>(W) + a.eps);
-#pragma unroll
-      for (int p = 0; p < NP; ++p) {
-        const int i = (p * BLOCK + threadIdx.x) * 4;
-        f32x4_t b = zero;
-        if (bias && i < W) b = load4(bias + i);
-        z[k][p] = (z[k][p] - m) * r * weight[p] + b;
-      }
+    for (int w = 0; w < kWaves; ++w) {
+      const float c = part[phase][w][0] - m;
+      v += __builtin_fmaf(wave_count(w) * c, c, part[phase][w][LAYER ? 1 : 0]);
     }
+    const float r = 1.0f / sqrtf(v / static_cast<float>(W) + a.eps);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) z[p] = (z[p] - m) * r * weight[p] + bias[p];
     phase ^= 1;
   };
 
-  auto block_sum = [&](float (&v)[NB]) {
+  auto inverse_rms = [&](const f32x4_t (&z)[NP]) {
+    float v = 0.f;
 #pragma unroll
-    for (int k = 0; k < NB; ++k) v[k] = wave_add(v[k]);
-    if ((threadIdx.x & 63) == 0) {
+    for (int p = 0; p < NP; ++p)
 #pragma unroll
-      for (int k = 0; k < NB; ++k) part[phase][threadIdx.x >> 6][k] = v[k];
-    }
+      for (int e = 0; e < 4; ++e) v = __builtin_fmaf(z[p][e], z[p][e], v);
+    v = wave_add(v);
+    if ((threadIdx.x & 63) == 0) part[phase][threadIdx.x >> 6][0] = v;
     __syncthreads();
+    v = 0.f;
 #pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      v[k] = 0.f;
-#pragma unroll
-      for (int w = 0; w < kWaves; ++w) v[k] += part[phase][w][k];
-      v[k] = 1.0f / sqrtf(v[k] / static_cast<float>(W) + a.eps);
-    }
+    for (int w = 0; w < kWaves; ++w) v += part[phase][w][0];
     phase ^= 1;  // the next sums go to the other half, so one barrier per sum is enough
+    return 1.0f / sqrtf(v / static_cast<float>(W) + a.eps);
   };
 
   // everything that does not depend on the rows; zero weights and rows beyond the width contribute nothing
-  f32x4_t wconv[TAPS > 0 ? TAPS : 1][NP], wd[NP], wn[NP], ring[RING][NP];
+  f32x4_t wconv[TAPS > 0 ? TAPS : 1][NP], wd[NP], wn[NP], bd[NP], bn[NP], ring[RING][NP];
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
-    const int i = (p * BLOCK + threadIdx.x) * 4;
-    wd[p] = wn[p] = zero;
+    const int i = piece(p) * 4;
+    wd[p] = wn[p] = bd[p] = bn[p] = zero;
     if (a.delta_weight && i < W) wd[p] = load4(a.delta_weight + i) + a.delta_offset;
     if (a.norm_weight && i < W) wn[p] = load4(a.norm_weight + i) + a.norm_offset;
+    if (LAYER && a.delta_bias && i < W) bd[p] = load4(a.delta_bias + i);
+    if (LAYER && a.norm_bias && i < W) bn[p] = load4(a.norm_bias + i);
     if (TAPS) {
 #pragma unroll
       for (int j = 0; j < TAPS; ++j) {
@@ -136,114 +152,95 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
     const float *src = a.tail_in + (static_cast<size_t>(b) * taps + (live ? static_cast<uint32_t>(pos) % static_cast<uint32_t>(taps) : 0u)) * W;
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-      const int i = (p * BLOCK + threadIdx.x) * 4;
+      const int i = piece(p) * 4;
       h[p] = zero;
       if (live && i < W) h[p] = load4(src + i);
     }
   };
 
-  // h (the convolution's inputs) of the tokens t .. t + NB - 1; emit: also store the updated residual rows
-  auto norm_rows = [&](int t, bool emit, f32x4_t (&h)[NB][NP]) {
-    f32x4_t d[NB][NP];
+  // What row t needs from memory, by loads that return zero past the width and for what the call does not have: no branch stands
+  // between them, so what waits for one knows how many were asked for behind it.
+  struct Raw {
+    f32x4_t h[NP];
+    Quad<T> d[NP];
+  };
+  auto request = [&](int64_t t, Raw &raw) {
+    const size_t base = (row0 + (t < 0 ? 0 : t < t_end ? t : t_end - 1)) * W;
+    const __amdgpu_buffer_rsrc_t x = make_rsrc(a.x + base, row_f32), d = make_rsrc(static_cast<const T *>(a.delta) + (a.delta ? base : 0), a.delta ? row_t : 0);
 #pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      const int tc = t + k < 0 ? 0 : t + k < seqlen ? t + k : seqlen - 1;
-      const size_t base = (row0 + tc) * W;
+    for (int p = 0; p < NP; ++p) raw.h[p] = buffer_quad<float>(x, piece(p)).raw;
 #pragma unroll
-      for (int p = 0; p < NP; ++p) {
-        const int i = (p * BLOCK + threadIdx.x) * 4;
-        h[k][p] = d[k][p] = zero;
-        if (i < W) {
-          h[k][p] = load4(a.x + base + i);
-          if (a.delta) d[k][p] = load4(static_cast<const T *>(a.delta) + base + i);
-        }
-      }
-      if (TAPS == 0 && a.terms) {
-        const float *tw = a.term_weights + (row0 + tc) * a.n_terms;
-        const T *term = static_cast<const T *>(a.terms) + (row0 + tc) * a.n_terms * W;
-        constexpr int kAhead = 4;  // terms whose loads are in flight together
-        for (int j0 = 0; j0 < static_cast<int>(a.n_terms); j0 += kAhead, term += kAhead * W) {
-          Quad<T> y[kAhead][NP];
-          float c[kAhead];
+    for (int p = 0; p < NP; ++p) raw.d[p] = buffer_quad<T>(d, piece(p));
+  };
+
+  // h (the convolution's input) of row t; emit: also store the updated residual row.  ahead: asked for in front of everything that waits
+  auto norm_row = [&](int64_t t, bool emit, const Raw &raw, auto ahead, f32x4_t (&h)[NP]) {
+    f32x4_t d[NP];
+    ahead();
 #pragma unroll
-          for (int j = 0; j < kAhead; ++j) {
-            const bool live = j0 + j < a.n_terms;
-            c[j] = live ? tw[j0 + j] : 0.f;
-#pragma unroll
-            for (int p = 0; p < NP; ++p) {
-              const int i = (p * BLOCK + threadIdx.x) * 4;
-              y[j][p].raw = {};
-              if (live && i < W) y[j][p] = load_quad(term + j * W + i);
-            }
-          }
-#pragma unroll
-          for (int j = 0; j < kAhead; ++j)
-#pragma unroll
-            for (int p = 0; p < NP; ++p) {
-              const f32x4_t v = y[j][p].f32();
-#pragma unroll
-              for (int e = 0; e < 4; ++e) d[k][p][e] = __builtin_fmaf(c[j], v[e], d[k][p][e]);
-            }
-        }
-      }
+    for (int p = 0; p < NP; ++p) {
+      h[p] = raw.h[p];
+      d[p] = raw.d[p].f32();
     }
-    if (LAYER && (a.delta || a.terms)) {
-      layer_norm(d, wd, a.delta_bias);
+    if constexpr (TERMS) {
+      const int n = static_cast<int>(a.n_terms);
+      const float *tw = a.term_weights + (row0 + t) * n;
+      const T *term = static_cast<const T *>(a.terms) + (row0 + t) * n * W;
+      constexpr int kAhead = 4;  // terms whose loads are in flight together
+      for (int j0 = 0; j0 < n; j0 += kAhead) {
+        Quad<T> y[kAhead][NP];
 #pragma unroll
-      for (int k = 0; k < NB; ++k)
+        for (int j = 0; j < kAhead; ++j) {
+          const bool live = j0 + j < n;
+          const __amdgpu_buffer_rsrc_t r = make_rsrc(term + static_cast<size_t>(live ? j0 + j : 0) * W, live ? row_t : 0);
 #pragma unroll
-        for (int p = 0; p < NP; ++p) {
-          const int i = (p * BLOCK + threadIdx.x) * 4;
-          if (i < W) {
-            h[k][p] += d[k][p];
-            if (emit && a.x_out && t + k < t_end) store4(a.x_out + (row0 + t + k) * W + i, h[k][p]);
+          for (int p = 0; p < NP; ++p) y[j][p] = buffer_quad<T>(r, piece(p));
+        }
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) {
+          const float c = j0 + j < n ? tw[j0 + j] : 0.f;
+#pragma unroll
+          for (int p = 0; p < NP; ++p) {
+            const f32x4_t v = y[j][p].f32();
+#pragma unroll
+            for (int e = 0; e < 4; ++e) d[p][e] = __builtin_fmaf(c, v[e], d[p][e]);
           }
         }
+      }
     }
-    if (!LAYER && (a.delta || a.terms)) {
-      float ss[NB];
-#pragma unroll
-      for (int k = 0; k < NB; ++k) {
-        ss[k] = 0.f;
+    if (a.delta || TERMS) {
+      if constexpr (LAYER) {
+        layer_norm(d, wd, bd);
 #pragma unroll
         for (int p = 0; p < NP; ++p)
+          if (piece(p) * 4 < W) h[p] += d[p];
+      } else {
+        const float r = inverse_rms(d);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) ss[k] = __builtin_fmaf(d[k][p][e], d[k][p][e], ss[k]);
+        for (int p = 0; p < NP; ++p) h[p] += d[p] * r * wd[p];
       }
-      block_sum(ss);
+      const bool there = emit && a.x_out;
+      const __amdgpu_buffer_rsrc_t to = make_rsrc(a.x_out + (there ? (row0 + t) * W : 0), there ? row_f32 : 0);
+      if (streamed) {
 #pragma unroll
-      for (int k = 0; k < NB; ++k)
+        for (int p = 0; p < NP; ++p) buffer_store<kStreamed>(to, piece(p), h[p], float{});
+      } else {
 #pragma unroll
-        for (int p = 0; p < NP; ++p) {
-          const int i = (p * BLOCK + threadIdx.x) * 4;
-          h[k][p] += d[k][p] * ss[k] * wd[p];
-          if (emit && a.x_out && i < W && t + k < t_end) store4(a.x_out + (row0 + t + k) * W + i, h[k][p]);
-        }
-    }
-    if (LAYER && a.norm_weight) layer_norm(h, wn, a.norm_bias);
-    if (!LAYER && a.norm_weight) {
-      float ss[NB];
-#pragma unroll
-      for (int k = 0; k < NB; ++k) {
-        ss[k] = 0.f;
-#pragma unroll
-        for (int p = 0; p < NP; ++p)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) ss[k] = __builtin_fmaf(h[k][p][e], h[k][p][e], ss[k]);
+        for (int p = 0; p < NP; ++p) buffer_store<0>(to, piece(p), h[p], float{});
       }
-      block_sum(ss);
-#pragma unroll
-      for (int k = 0; k < NB; ++k)
-#pragma unroll
-        for (int p = 0; p < NP; ++p) h[k][p] = h[k][p] * ss[k] * wn[p];
     }
-    if (TAPS) {
+    if (a.norm_weight) {
+      if constexpr (LAYER) {
+        layer_norm(h, wn, bn);
+      } else {
+        const float r = inverse_rms(h);
 #pragma unroll
-      for (int k = 0; k < NB; ++k)
-        if (pos0 + t + k < first) {  // padding: the convolution must not see it
+        for (int p = 0; p < NP; ++p) h[p] = h[p] * r * wn[p];
+      }
+    }
+    if (TAPS && pos0 + t < first) {  // padding: the convolution must not see it
 #pragma unroll
-          for (int p = 0; p < NP; ++p) h[k][p] = zero;
-        }
+      for (int p = 0; p < NP; ++p) h[p] = zero;
     }
   };
   auto push = [&](const f32x4_t (&h)[NP]) {
@@ -255,49 +252,48 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
     }
   };
 
+  Raw cur, next;
+  if (AHEAD) request(TAPS > 1 && t_begin > 0 ? t_begin - RING : t_begin, cur);
+  // the row that is asked for in front of row t's work is the one behind it (behind the last one that again, for nothing)
+  auto take = [&](int64_t t, bool emit, f32x4_t (&h)[NP]) {
+    if (!AHEAD) request(t, cur);
+    norm_row(t, emit, cur, [&] { if (AHEAD) request(t + 1, next); }, h);
+    if (AHEAD) cur = next;
+  };
   if (TAPS > 1) {
     if (t_begin == 0) {
 #pragma unroll
       for (int j = 0; j < RING; ++j) kept(j - RING, ring[j]);
     } else {
 #pragma unroll
-      for (int s = -((RING + NB - 1) / NB * NB); s < 0; s += NB) {
-        f32x4_t h[NB][NP];
-        norm_rows(t_begin + s, false, h);
-#pragma unroll
-        for (int k = 0; k < NB; ++k) {
-          if (t_begin + s + k < 0) kept(t_begin + s + k, h[k]);
-          push(h[k]);
-        }
+      for (int s = -RING; s < 0; ++s) {
+        f32x4_t h[NP];
+        take(t_begin + s, false, h);
+        if (t_begin + s < 0) kept(t_begin + s, h);
+        push(h);
       }
     }
   }
-  for (int t = t_begin; t < t_end; t += NB) {
-    f32x4_t h[NB][NP];
-    norm_rows(t, true, h);
+  for (int64_t t = t_begin; t < t_end; t += step) {
+    f32x4_t h[NP];
+    take(t, true, h);
+    const __amdgpu_buffer_rsrc_t out = make_rsrc(static_cast<const T *>(a.out) + (a.out ? (row0 + t) * W : 0), a.out ? row_t : 0);
 #pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      if (t + k < t_end) {
-        const size_t base = (row0 + t + k) * W;
+    for (int p = 0; p < NP; ++p) {
+      f32x4_t y = h[p];
+      if (TAPS) {
+        f32x4_t c = y * wconv[TAPS > 0 ? TAPS - 1 : 0][p];
+        if (TAPS > 1) {
 #pragma unroll
-        for (int p = 0; p < NP; ++p) {
-          const int i = (p * BLOCK + threadIdx.x) * 4;
-          f32x4_t y = h[k][p];
-          if (TAPS) {
-            f32x4_t c = y * wconv[TAPS > 0 ? TAPS - 1 : 0][p];
-            if (TAPS > 1) {
+          for (int j = 0; j < RING; ++j)
 #pragma unroll
-              for (int j = 0; j < RING; ++j)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) c[e] = __builtin_fmaf(ring[j][p][e], wconv[j][p][e], c[e]);
-            }
-            y += c;
-          }
-          if (a.out && i < W) store4(static_cast<T *>(a.out) + base + i, y);
+            for (int e = 0; e < 4; ++e) c[e] = __builtin_fmaf(ring[j][p][e], wconv[j][p][e], c[e]);
         }
-        if (TAPS > 1) push(h[k]);
+        y += c;
       }
+      buffer_store<0>(out, piece(p), y, T{});
     }
+    if (TAPS > 1) push(h);
   }
   if (TAPS > 1 && t_end == seqlen) {  // the last inputs of the call, oldest first in the ring registers; one token replaces one slot
 #pragma unroll
@@ -307,37 +303,49 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
         float *dst = a.tail_out + (static_cast<size_t>(b) * taps + static_cast<uint32_t>(pos) % static_cast<uint32_t>(taps)) * W;
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-          const int i = (p * BLOCK + threadIdx.x) * 4;
+          const int i = piece(p) * 4;
           if (i < W) store4(dst + i, ring[j][p]);
         }
       }
     }
   }
+#endif
 }
 
-template <typename T, int BLOCK, int NP, int TAPS, bool LAYER>
+template <typename T, int BLOCK, int NP, int TAPS, bool LAYER, bool TERMS>
 void launch_norm_conv_rows(const e2h_norm_conv_args &a, int runs, int run, hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>(a.batch * runs)), block(BLOCK);
-  constexpr int NB = NP > 1 || TAPS > 4 ? 1 : TAPS || LAYER ? 2 : 4;  // rows that fit the registers
-  if (run == 1) hipLaunchKernelGGL((norm_conv_kernel<T, BLOCK, NP, TAPS, 1, LAYER>), grid, block, 0, s, a, runs, run);
-  else hipLaunchKernelGGL((norm_conv_kernel<T, BLOCK, NP, TAPS, NB, LAYER>), grid, block, 0, s, a, runs, run);
+  const int64_t workgroups = TAPS ? a.batch * runs : a.batch * a.seqlen < (1 << 20) ? a.batch * a.seqlen : 1 << 20;
+  const dim3 grid(static_cast<unsigned>(workgroups)), block(BLOCK);
+  // from 21 million values on (x, the new x and two 16-bit operands are 12 bytes each) they do not stay in 256 MB of cache anyway; 4096 x 4096 takes as long with either store
+  const int streamed = a.batch * a.seqlen * a.width >= (int64_t{1} << 28) / 12;
+  if constexpr (TAPS > 0) {
+    if (run > 1) {
+      hipLaunchKernelGGL((norm_conv_kernel<T, BLOCK, NP, TAPS, LAYER, TERMS, true>), grid, block, 0, s, a, runs, run, streamed);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((norm_conv_kernel<T, BLOCK, NP, TAPS, LAYER, TERMS, false>), grid, block, 0, s, a, runs, run, streamed);
 }
 
 template <typename T, int BLOCK, int NP>
 void launch_norm_conv_taps(const e2h_norm_conv_args &a, int runs, int run, hipStream_t s) {
-  if constexpr (BLOCK != 1024 || NP != 1) {  // (that geometry is for convolutions only)
-    if (a.norm_kind == E2H_SEQ_LAYER_NORM) return launch_norm_conv_rows<T, BLOCK, NP, 0, true>(a, runs, run, s);
-    if (!a.conv) return launch_norm_conv_rows<T, BLOCK, NP, 0, false>(a, runs, run, s);
+  if (a.norm_kind == E2H_SEQ_LAYER_NORM) {
+    if (a.terms) return launch_norm_conv_rows<T, BLOCK, NP, 0, true, true>(a, runs, run, s);
+    return launch_norm_conv_rows<T, BLOCK, NP, 0, true, false>(a, runs, run, s);
   }
-  if (a.taps <= 4) launch_norm_conv_rows<T, BLOCK, NP, 4, false>(a, runs, run, s);
-  else launch_norm_conv_rows<T, BLOCK, NP, 8, false>(a, runs, run, s);
+  if (a.terms) return launch_norm_conv_rows<T, BLOCK, NP, 0, false, true>(a, runs, run, s);
+  if (!a.conv) return launch_norm_conv_rows<T, BLOCK, NP, 0, false, false>(a, runs, run, s);
+  if (a.taps <= 4) launch_norm_conv_rows<T, BLOCK, NP, 4, false, false>(a, runs, run, s);
+  else launch_norm_conv_rows<T, BLOCK, NP, 8, false, false>(a, runs, run, s);
 }
 
 template <typename T>
 void launch_norm_conv(const e2h_norm_conv_args &a, int runs, int run, hipStream_t s) {
   if (a.width <= 1024) launch_norm_conv_taps<T, 256, 1>(a, runs, run, s);
+  // eight values per thread where many rows are waiting: half the waves, which repeat a row's sums each (8192 x 2048, layer norm 31 us, 38 with four values; final norm 24, 31)
+  else if (a.width <= 2048 && !a.conv && a.batch * a.seqlen > 256) launch_norm_conv_taps<T, 256, 2>(a, runs, run, s);
   else if (a.width <= 2048) launch_norm_conv_taps<T, 512, 1>(a, runs, run, s);
-  else if (a.width <= 4096 && a.conv) launch_norm_conv_taps<T, 1024, 1>(a, runs, run, s);
+  else if (a.width <= 4096 && a.conv && run == 1) launch_norm_conv_taps<T, 1024, 1>(a, runs, run, s);
   else if (a.width <= 4096) launch_norm_conv_taps<T, 512, 2>(a, runs, run, s);
   else if (a.width <= 8192) launch_norm_conv_taps<T, 512, 4>(a, runs, run, s);
   else launch_norm_conv_taps<T, 1024, 4>(a, runs, run, s);
@@ -446,11 +454,14 @@ extern "C" int e2h_seq_norm_conv(const e2h_norm_conv_args *a, void *stream) {
       !aligned16(a->conv) || !aligned16(a->tail_in) || !aligned16(a->tail_out) || !aligned16(a->out) ||
       !aligned16(a->delta_bias) || !aligned16(a->norm_bias) || !aligned16(a->terms))
     return E2H_ERR_MISALIGNED;
-  // enough workgroups to fill the chip first, then longer runs so that fewer tokens are normalised twice
-  int run = seq_options().norm_run;
-  if (!run) {
-    run = static_cast<int>(a->batch * a->seqlen / (a->conv ? 256 : 1024));
-    run = run < 1 ? 1 : run > 32 ? 32 : run;
+  // The fewest tokens per workgroup with which the convolution's workgroups are a whole number of rounds, up to 32: longer runs normalise fewer tokens twice, and one workgroup beyond a round
+  // costs a round.  A round is a workgroup per CU, of narrower rows two or four (8192 x 2048: 512 workgroups 42 us, 256 54; 8192 x 1024: 1024 24, 256 49).
+  int run = a->conv ? seq_options().norm_run : 1;
+  const int64_t round = a->width <= 1024 ? 1024 : a->width <= 2048 ? 512 : 256;
+  for (int64_t most = round; !run; most += round) {
+    const int64_t per_sequence = most / a->batch;
+    if (per_sequence > 0 && (a->seqlen + per_sequence - 1) / per_sequence <= 32) run = static_cast<int>((a->seqlen + per_sequence - 1) / per_sequence);
+    if (a->seqlen <= 32 && per_sequence == 0) run = static_cast<int>(a->seqlen);
   }
   const int64_t runs = (a->seqlen + run - 1) / run;
   if (a->batch * runs > INT32_MAX) return E2H_ERR_BAD_SHAPE;

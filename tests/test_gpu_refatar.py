@@ -75,6 +75,32 @@ def test_norm_conv_over_portions(dtype, width, taps, run):
 
 
 @BOTH
+@pytest.mark.parametrize("b,t,width,taps", [(1, 33, 4096, 4), (3, 700, 4096, 4), (1, 8001, 64, 3), (2, 515, 2048, 2), (300, 5, 1028, 4), (2, 70, 8192, 6), (1, 5500, 4096, 0), (1, 257, 2048, 0),
+                                            (2, 150, 2052, 0), (3, 100, 1000, 0)])
+def test_norm_conv_of_many_rows(dtype, b, t, width, taps):
+    """runs of the convolution and their first tokens, rows without one, large rows that are streamed (5500 x 4096)"""
+    eps, rows = 1e-4, b * t
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x, d = torch.randn((rows, width), generator=g, device=DEV), torch.randn((rows, width), generator=g, device=DEV).to(dtype)
+    wd, wn = (0.3 * torch.randn((2, width), generator=g, device=DEV)).unbind(0)
+    kw = {}
+    if taps:
+        wc, first = 0.5 * torch.randn((taps, width), generator=g, device=DEV), torch.arange(b, device=DEV) % min(t, 4)
+        kw = dict(conv=wc, tails=(torch.full((b, taps, width), 7.0, device=DEV), torch.empty((b, taps, width), device=DEV)), input_pos=positions(0, t), first=first)
+    xo, y = seq_ops.norm_conv(x, b, t, eps, dtype, delta=d, delta_weight=wd, delta_offset=1.0, norm_weight=wn, norm_offset=1.0, **kw)
+    norm = lambda z, w: z / torch.sqrt((z * z).mean(-1, keepdim=True) + eps) * (1.0 + w.double())
+    want_x = x.double() + norm(d.double(), wd)
+    want = norm(want_x, wn).view(b, t, width)
+    if taps:
+        want = want * (torch.arange(t, device=DEV)[None, :, None] >= first[:, None, None])  # padding: the convolution does not see it
+        padded = torch.nn.functional.pad(want, (0, 0, taps - 1, 0))
+        want = want + sum(padded[:, j: j + t] * wc[j].double() for j in range(taps))
+    err = lambda got, ref: ((got.double() - ref).abs().max() / ref.abs().max()).item()
+    assert err(xo, want_x) < 2e-6
+    assert err(y.view(b, t, width), want) < (3e-6 if dtype == torch.float32 else 2.0 ** -8)  # a bfloat16 rounding of the largest value
+
+
+@BOTH
 def test_norm_conv_parts_and_padding(dtype):
     b, t, width, taps, eps = 3, 9, 72, 3, 1e-5
     x, d = randn(b * t, width, seed=1), randn(b * t, width, seed=2, dtype=dtype)
