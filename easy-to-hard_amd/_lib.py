@@ -148,8 +148,8 @@ _SEQ_SIGNATURES = {
     "e2h_seq_gelu_gate_rows": (c_int, [c_int, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, _P]),
     "e2h_seq_linear_scratch_bytes": (c_int64, [c_int64, c_int64, c_int64]),
     "e2h_seq_linear": (c_int, [_P, _P, _P, c_int64, c_int64, c_int64, c_int, c_float, _P, c_int64, _P]),
-    "e2h_seq_linear_rows_pays": (c_int, [c_int64, c_int64, c_int64, c_int]),
-    "e2h_seq_linear_rows": (c_int, [_P, _P, _P, c_int64, c_int64, c_int64, c_int, _P]),
+    "e2h_seq_linear_rows_pays": (c_int, [c_int64, c_int64, c_int64, c_int, c_float]),
+    "e2h_seq_linear_rows": (c_int, [_P, _P, _P, c_int64, c_int64, c_int64, c_int, c_float, _P]),
     "e2h_seq_rotary_table": (c_int, [_P, _P, _P, _P, c_int64, c_int64, c_int64, _P]),
     "e2h_seq_window_attention": (c_int, [_A(WindowAttentionArgs), _P]),
     "e2h_seq_window_attention_scratch_bytes": (c_int64, [_A(WindowAttentionArgs)]),

@@ -81,30 +81,77 @@ int run_linear(const stream::Args &a, bf16_t *y, float cap, float *scratch, hipS
 }
 
 // ---- many rows: the activation behind a tile of products (e2h_gemm256.h) ---------------------------------------------------------------
+// cap tanh(y / cap): with z = y y it is y + y z Q(z) up to |y| = 0.75 cap, Q by the Remez algorithm (3.3e-8 of tanh, half a unit in the last place of float32) in powers of 1 / cap^2, else
+// cap (1 - 2 / (1 + exp(2 y / cap))).  A tile's store forms the first for all of its values, and the second too where a wave's 512 values have one that needs it: six instructions a value
+// where tanhf and the division take 45, which would take as long as the pass over memory that is saved (128 values per lane and wave with nothing beside them).
+struct Cap {
+  float cap, limit, q[5], twice;  // limit: 0.75 cap; twice: 2 / cap in units of log 2
+};
+Cap cap_of(float cap) {
+  const double u = 1.0 / (static_cast<double>(cap) * cap);
+  const double q[5] = {-0.3333306838118954, 0.1332652117591573, -0.05339025879171665, 0.01966491390244702, -0.004769490464846426};
+  Cap c = {cap, 0.75f * cap, {}, static_cast<float>(2 * 1.4426950408889634 / cap)};
+  double power = u;
+  for (int j = 0; j < 5; ++j, power *= u) c.q[j] = static_cast<float>(q[j] * power);
+  return c;
+}
+// where cap^-10 and the squares of what lies below cap are far from the ends of float32
+bool cap_fits(float cap) { return cap >= 0x1p-6f && cap <= 0x1p10f; }
+
 template <int ACT>
 struct RowsWalk : gemm256::PlainWalk<> {
-  using gemm256::PlainWalk<>::PlainWalk;
+  Cap c;
+  __device__ __forceinline__ RowsWalk(const uint16_t *x_, const uint16_t *w_, uint16_t *y_, const Cap &c_, int M_, int N_, int K_) : PlainWalk(x_, w_, y_, M_, N_, K_), c(c_) {}
   struct Dest {};
   __device__ __forceinline__ void dest(const Tile &, int, int, Dest &) const {}
+  __device__ __forceinline__ float capped(float y) const {
+    const float z = y * y;
+    float q = c.q[4];
+#pragma unroll
+    for (int j = 3; j >= 0; --j) q = __builtin_fmaf(q, z, c.q[j]);
+    return __builtin_fmaf(y * z, q, y);
+  }
+  __device__ __forceinline__ float capped_far(float y, float near) const {
+    const float far = c.cap * __builtin_fmaf(-2.0f, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(y * c.twice)), 1.0f);
+    return __builtin_fabsf(y) > c.limit ? far : near;  // (what is no number stays none)
+  }
   __device__ __forceinline__ void store(const Tile &tile, const Dest &, int, int, int row, int col, float (&v)[8]) const {
+    const auto low = [](uint32_t b) { return __builtin_bit_cast(float, b << 16); };
+    const auto high = [](uint32_t b) { return __builtin_bit_cast(float, b & 0xFFFF0000u); };
     u32x4_t out;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      out[e] = pack_bf16(v[2 * e], v[2 * e + 1]);
-      if (ACT == kSquare) {
-        const float lo = fmaxf(__builtin_bit_cast(float, out[e] << 16), 0.f), hi = fmaxf(__builtin_bit_cast(float, out[e] & 0xFFFF0000u), 0.f);
+    for (int e = 0; e < 4; ++e) out[e] = pack_bf16(v[2 * e], v[2 * e + 1]);  // the linear's own output is rounded first
+    if (ACT == kSquare) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float lo = fmaxf(low(out[e]), 0.f), hi = fmaxf(high(out[e]), 0.f);
         out[e] = pack_bf16(lo * lo, hi * hi);
       }
+    }
+    if (ACT == kCap) {
+      float y[8], near[8], top = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        y[e] = e & 1 ? high(out[e >> 1]) : low(out[e >> 1]);
+        near[e] = capped(y[e]);
+        top = __builtin_fmaxf(top, __builtin_fabsf(y[e]));
+      }
+      if (__builtin_amdgcn_ballot_w64(top > c.limit)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) near[e] = capped_far(y[e], near[e]);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) out[e] = pack_bf16(near[2 * e], near[2 * e + 1]);
     }
     __builtin_amdgcn_raw_buffer_store_b128(out, y_rsrc(tile), y_at(tile, row, col), 0, 0);
   }
 };
 
 template <int ACT>
-__global__ __launch_bounds__(256, 1) void linear_rows_kernel(const uint16_t *x, const uint16_t *w, uint16_t *y, int M, int N, int K) {
+__global__ __launch_bounds__(256, 1) void linear_rows_kernel(const uint16_t *x, const uint16_t *w, uint16_t *y, const Cap cap, int M, int N, int K) {
 #if defined(__HIP_DEVICE_COMPILE__)
   __shared__ __attribute__((aligned(1024))) uint8_t lds[gemm256::kRing];
-  RowsWalk<ACT> tiles(x, w, y, M, N, K);
+  RowsWalk<ACT> tiles(x, w, y, cap, M, N, K);
   gemm256::walk<false>(tiles, lds);
 #endif
 }
@@ -121,28 +168,30 @@ using namespace e2h;
 
 // 1 where the product with its activation is expected to be faster here than the library's product and a pass over its result.  Measured, us, that / here: 16384 x 4096 1000 rows 114 / 96,
 // 8192 rows 817 / 743; 8192 x 2048 2048 rows 68 / 51; 2048 x 4096 8192 rows 112 / 95; 16384 x 4096 512 rows 70 / 76: not taken.  Without an activation the library's product is
-// 2 % the faster one where it fills the chip (16384 x 4096 8192 rows 725 / 742).
+// 2 % the faster one where it fills the chip (16384 x 4096 8192 rows 725 / 742).  With a soft cap 32000 x 4096 8192 rows: 217 us less of a prompt's pass than the library's 1425 and 229.
 // us, as for the quantized linears on the same loop (a last round that is not full runs at a higher clock), against the library's product at what it reaches where it fills the chip, 1.5
 // PFLOP/s, and a pass over the result of its own.
-extern "C" int e2h_seq_linear_rows_pays(int64_t rows, int64_t n, int64_t k, int act) {
-  if (rows <= 64 || act != kSquare || !rows_fit(rows, n, k)) return 0;
+extern "C" int e2h_seq_linear_rows_pays(int64_t rows, int64_t n, int64_t k, int act, float cap) {
+  if (rows <= 64 || (act != kSquare && (act != kCap || !cap_fits(cap))) || !rows_fit(rows, n, k)) return 0;
   const int64_t tiles = (rows + 255) / 256 * ((n + 255) / 256), full = tiles / 256, rest = tiles % 256;
   const double rounds = static_cast<double>(full) + (rest == 0 ? 0. : full == 0 ? 1. : 0.6 + 0.4 * static_cast<double>(rest) / 256);
   const double outputs = static_cast<double>(rows) * static_cast<double>(n);
-  return 4 + rounds * (static_cast<double>(k) / 64 * 1.36 + 5) < outputs * static_cast<double>(k) * 2 / 1.5e9 + outputs * 4 / 6e6 + 12 ? 1 : 0;
+  return 4 + rounds * (static_cast<double>(k) / 64 * 1.36 + (act == kCap ? 9 : 5)) < outputs * static_cast<double>(k) * 2 / 1.5e9 + outputs * 4 / 6e6 + 12 ? 1 : 0;
 }
 
-extern "C" int e2h_seq_linear_rows(const void *x, const void *w, void *y, int64_t rows, int64_t n, int64_t k, int act, void *stream) {
+extern "C" int e2h_seq_linear_rows(const void *x, const void *w, void *y, int64_t rows, int64_t n, int64_t k, int act, float cap, void *stream) {
   if (!x || !w || !y) return E2H_ERR_NULL_POINTER;
-  if (!rows_fit(rows, n, k) || (act != kNone && act != kSquare)) return E2H_ERR_BAD_SHAPE;
+  if (!rows_fit(rows, n, k) || act < kNone || act > kCap || (act == kCap && !cap_fits(cap))) return E2H_ERR_BAD_SHAPE;
   if (!aligned16(x) || !aligned16(w) || !aligned16(y)) return E2H_ERR_MISALIGNED;
   const dim3 grid(gemm256::grid_of((rows + 255) / 256 * ((n + 255) / 256)));
   const auto *xs = static_cast<const uint16_t *>(x), *ws = static_cast<const uint16_t *>(w);
   auto *ys = static_cast<uint16_t *>(y);
   const int M = static_cast<int>(rows), N = static_cast<int>(n), K = static_cast<int>(k);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (act == kSquare) hipLaunchKernelGGL(linear_rows_kernel<kSquare>, grid, dim3(256), 0, s, xs, ws, ys, M, N, K);
-  else hipLaunchKernelGGL(linear_rows_kernel<kNone>, grid, dim3(256), 0, s, xs, ws, ys, M, N, K);
+  const Cap c = act == kCap ? cap_of(cap) : Cap{};
+  if (act == kSquare) hipLaunchKernelGGL(linear_rows_kernel<kSquare>, grid, dim3(256), 0, s, xs, ws, ys, c, M, N, K);
+  else if (act == kCap) hipLaunchKernelGGL(linear_rows_kernel<kCap>, grid, dim3(256), 0, s, xs, ws, ys, c, M, N, K);
+  else hipLaunchKernelGGL(linear_rows_kernel<kNone>, grid, dim3(256), 0, s, xs, ws, ys, c, M, N, K);
   return launch_status();
 }
 

@@ -11,7 +11,7 @@ import torch.nn as nn
 from torch import Tensor
 
 from . import ops, seq_ops
-from .linear import fusable
+from .linear import DecodeLinear, fusable, unwatched
 from .state import SequenceState, StatePlan, rotary_turns
 
 
@@ -76,6 +76,9 @@ class StatefulDecoder(nn.Module):
         h = h[:, -1:] if greedy_token else h
         if self.logit_softcap is not None and fusable(self.output, h):
             logits = seq_ops.linear(h, self.output.weight, seq_ops.ACT_SOFTCAP, self.logit_softcap)
+        elif (self.logit_softcap is not None and type(self.output) is DecodeLinear and self.output.bias is None and unwatched(self.output)
+              and seq_ops.linear_rows_pay(h, self.output.weight, seq_ops.ACT_SOFTCAP, self.logit_softcap)):
+            logits = seq_ops.linear_rows(h, self.output.weight, seq_ops.ACT_SOFTCAP, self.logit_softcap)
         else:
             logits = self.output(h)
             if self.logit_softcap is not None:

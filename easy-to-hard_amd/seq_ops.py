@@ -174,7 +174,7 @@ def linear(x, weight, act=ACT_NONE, cap=0.0):
     return y
 
 
-def linear_rows_pay(x, weight, act):
+def linear_rows_pay(x, weight, act, cap=0.0):
     """True where linear_rows takes x [.., k] and weight [n, k], more rows than a decode step has, and is expected to be faster than the library's product and a pass over its
     result: bfloat16 on the GPU, 16-byte aligned, no gradients, nobody watching."""
     if torch.compiler.is_compiling():
@@ -187,15 +187,15 @@ def linear_rows_pay(x, weight, act):
         return False
     if not (x.is_contiguous() and weight.is_contiguous()) or x.data_ptr() % 16 or weight.data_ptr() % 16 or torch.is_autocast_enabled():
         return False
-    return bool(_lib.load_seq().e2h_seq_linear_rows_pays(rows, n, k, act)) and not watched(x, weight)
+    return bool(_lib.load_seq().e2h_seq_linear_rows_pays(rows, n, k, act, cap)) and not watched(x, weight)
 
 
-def linear_rows(x, weight, act):
+def linear_rows(x, weight, act, cap=0.0):
     """act(x weight^T) over many rows in one launch, see e2h_seq_linear_rows (linear_rows_pay)."""
     _need_gpu(x, weight)
     n, k = weight.shape
     y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
-    _lib.check_seq(_lib_for(x).e2h_seq_linear_rows(_p(x), _p(weight), _p(y), x.numel() // k, n, k, act, _stream(x)), "e2h_seq_linear_rows")
+    _lib.check_seq(_lib_for(x).e2h_seq_linear_rows(_p(x), _p(weight), _p(y), x.numel() // k, n, k, act, cap, _stream(x)), "e2h_seq_linear_rows")
     return y
 
 

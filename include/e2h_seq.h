@@ -84,10 +84,10 @@ int64_t e2h_seq_linear_scratch_bytes(int64_t rows, int64_t n, int64_t k);
 int e2h_seq_linear(const void *x, const void *w, void *y, int64_t rows, int64_t n, int64_t k, int act, float cap, void *scratch,
                    int64_t scratch_bytes, void *stream);
 
-/* The same over many rows, for act E2H_SEQ_ACT_NONE and E2H_SEQ_ACT_SQUARE_RELU: n a multiple of 8, k of 64 and at least 192, x, w and 256 rows of y below 4 GB, all three 16-byte
- * aligned; no scratch.  e2h_seq_linear_rows_pays: 1 where that is expected to take less time than a library product followed by e2h_seq_square_relu, else 0. */
-int e2h_seq_linear_rows_pays(int64_t rows, int64_t n, int64_t k, int act);
-int e2h_seq_linear_rows(const void *x, const void *w, void *y, int64_t rows, int64_t n, int64_t k, int act, void *stream);
+/* The same over many rows (a soft cap between 2^-6 and 2^10): n a multiple of 8, k of 64 and at least 192, x, w and 256 rows of y below 4 GB, all three 16-byte
+ * aligned; no scratch.  e2h_seq_linear_rows_pays: 1 where that is expected to take less time than a library product followed by e2h_seq_square_relu or e2h_seq_softcap, else 0. */
+int e2h_seq_linear_rows_pays(int64_t rows, int64_t n, int64_t k, int act, float cap);
+int e2h_seq_linear_rows(const void *x, const void *w, void *y, int64_t rows, int64_t n, int64_t k, int act, float cap, void *stream);
 
 /* Elementwise steps.  square_relu: y = max(x, 0)^2.  softcap: y = cap tanh(x / cap).  x and y may be the same memory.
  * gelu_gate_rows: y[r, i] = gelu_tanh(gate[r, i]) * table[tokens[r], column + i], i < dim; table rows are ld values long. */

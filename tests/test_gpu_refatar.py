@@ -817,6 +817,29 @@ def test_linear_rows_is_the_rounded_product_and_its_activation(rows, n, k, act):
     assert torch.equal(seq_ops.linear_rows(x, w, act), want)
 
 
+@pytest.mark.parametrize("cap", [2.0 ** -6, 0.5, 30.0, 1024.0])
+@pytest.mark.parametrize("rows,n,k", [(65, 264, 192), (257, 520, 320), (600, 8, 256)])
+def test_linear_rows_with_a_soft_cap(rows, n, k, cap):
+    """Logits from far below the cap to far beyond it, both signs in every tile; what is no number and infinities as tanh has them."""
+    gen = torch.Generator().manual_seed(rows + n)
+    x = torch.randint(-3, 4, (rows, k), generator=gen).to(torch.bfloat16)
+    x = (x * 2.0 ** torch.randint(-12, 5, (rows, 1), generator=gen) * (cap / k)).to(torch.bfloat16).to(DEV)
+    w = torch.randint(-3, 4, (n, k), generator=gen).to(torch.bfloat16).to(DEV)
+    x[3], x[4, 0] = 0.0, float("nan")
+    w[0], x[5] = 3.0, float("inf")
+    w[1], w[2], w[3] = -3.0, 0.0, 0.0
+    y = seq_ops.linear_rows(x, w, seq_ops.ACT_NONE).double()
+    want = (cap * torch.tanh(y / cap)).to(torch.bfloat16)
+    got = seq_ops.linear_rows(x, w, seq_ops.ACT_SOFTCAP, cap)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and got[5, 0].item() == cap and got[5, 1].item() == -cap and (got[3] == 0).all()
+    ok = ~torch.isnan(want)
+    steps = (got.view(torch.int16).int() - want.view(torch.int16).int()).abs()[ok]
+    # float32 values within a few units of the true ones: the bfloat16 next to it where one of them lies in a thousandth of a rounding boundary
+    assert steps.max() <= 1 and (steps != 0).float().mean() < 1e-3
+    assert not seq_ops.linear_rows_pay(x, w, seq_ops.ACT_SOFTCAP, 2.0 ** 11) and not seq_ops.linear_rows_pay(x, w, seq_ops.ACT_SOFTCAP, 2.0 ** -7)
+
+
+
 def test_feed_forward_of_many_rows_takes_one_launch_for_up_and_its_activation():
     from easy_to_hard_amd.feed_forward import SquaredReluFF
 
