@@ -85,6 +85,10 @@ _SIGNATURES = {
     "e2h_int4_mm_staged_partials": (c_int, [_P, _P, _P, _P, c_int64, c_int64, c_int64, c_int, c_int, _P]),
     "e2h_int4_mm_staged_silu_gate": (c_int, [_P, _P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int, _P]),
     "e2h_int4_mm_staged_rope_kv": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, _P]),
+    "e2h_add_rmsnorm_sums": (c_int, [_P, _P, _P, c_int, _P, _P, _P, _P, c_int64, c_int64, c_int, c_float, _P]),
+    "e2h_int4_mm_rows_slices": (c_int, [c_int64, c_int64, c_int64, c_int, c_int]),
+    "e2h_int4_mm_rows": (c_int, [_P, _P, _P, _P, c_int, _P, _P, c_int64, c_int64, c_int64, c_int, c_int, _P]),
+    "e2h_int4_mm_silu_gate_rows_sums": (c_int, [_P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int, c_int, _P, c_int64, _P]),
     "e2h_add_rmsnorm_staged": (c_int, [_P, _P, _P, c_int, _P, _P, _P, _P, _P, c_int64, c_int64, c_float, _P]),
     "e2h_stream_read_probe": (c_int, [_P, c_int64, _P, c_int64, _P, _P]),
     "e2h_decode_attention_staged": (c_int, [_P, _P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, c_float, _P]),
@@ -218,7 +222,7 @@ class _PythonCalls:
     def int4_linear(*_):
         return None
 
-    int8_linear = int4_linear
+    int8_linear = int4_rows = int4_linear
 
 
 def _load_calls(lib):
@@ -235,6 +239,7 @@ def _load_calls(lib):
     if module.torch_version != torch.__version__:  # it reads tensors' structures as that torch laid them out
         return f"was built for torch {module.torch_version}, this is {torch.__version__}"
     module.bind(*(ctypes.cast(f, c_void_p).value for f in (lib.e2h_int4_mm, lib.e2h_int8_mm, lib.e2h_stream_capturing)), ops._workspaces, check)
+    module.bind_rows(*(ctypes.cast(f, c_void_p).value for f in (lib.e2h_int4_mm_rows, lib.e2h_int4_mm_rows_slices)))
     return module
 
 

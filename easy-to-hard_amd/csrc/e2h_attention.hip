@@ -373,12 +373,19 @@ __global__ __launch_bounds__(64 * NW) void decode_attention_gqa_kernel(const uin
 // cost 64 rows of 2048 4.2 us instead of 3.5 (4096: 4.3 and 4.0), always four cost two slices 0.2.
 enum NormTerm { kNothing = 0, kDelta = 1, kSums = 2 };  // what is added to x first
 
+// Where the sums of a normalised row's quantization groups go, [dim / group][stride] as the many-row int4 matmul reads them, or null.  Lanes that hold a group's pieces of 8 values are
+// neighbours.  (A pass of its own over 471 x 4096 takes 3.5 - 4.8 us, the launch; here the values are in registers.)
+struct GroupSums {
+  float *out;
+  int stride, lanes;
+};
+
 template <int BLOCK, int kPieces, NormTerm SRC, int kMaxSlices>
 __global__ __launch_bounds__(BLOCK) void rmsnorm_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ delta,
                                                         const float *__restrict__ psum, int slices,
                                                         const uint16_t *__restrict__ col_scales,
                                                         const uint16_t *__restrict__ w, uint16_t *__restrict__ h_out,
-                                                        uint16_t *__restrict__ y, StagedOut staged, int dim, float eps) {
+                                                        uint16_t *__restrict__ y, StagedOut staged, GroupSums sums, int dim, float eps) {
   constexpr int kStride = BLOCK * 8, kWaves = BLOCK / 64;
   const size_t row = blockIdx.x;
   const uint16_t *xr = x + row * dim;
@@ -447,6 +454,13 @@ __global__ __launch_bounds__(BLOCK) void rmsnorm_kernel(const uint16_t *__restri
     }
     if (y) *reinterpret_cast<u32x4_t *>(y + row * dim + i) = o;
     if (staged.frag) staged_store_piece(staged, static_cast<int>(row), i >> 3, o);
+    if (sums.out) {  // (in the order of x_group_sums_kernel)
+      float s = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s += __builtin_bit_cast(float, o[j] << 16) + __builtin_bit_cast(float, o[j] & 0xFFFF0000u);
+      for (int off = 1; off < sums.lanes; off <<= 1) s += __shfl_xor(s, off);
+      if (((i >> 3) & (sums.lanes - 1)) == 0) sums.out[static_cast<size_t>((i >> 3) / sums.lanes) * sums.stride + row] = s;
+    }
   };
 
   u32x4_t keep[kPieces], keepd[kPieces], keepw[kPieces], keepc[kPieces];
@@ -596,9 +610,9 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t *__restric
 
 template <int BLOCK, int PIECES>
 void launch_rmsnorm_block(const uint16_t *x, const uint16_t *delta, const float *psum, int slices, const uint16_t *col_scales, const uint16_t *w,
-                          uint16_t *h_out, uint16_t *y, StagedOut staged, int64_t rows, int64_t dim, float eps, hipStream_t stream) {
+                          uint16_t *h_out, uint16_t *y, StagedOut staged, GroupSums sums, int64_t rows, int64_t dim, float eps, hipStream_t stream) {
   const auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(rows)), dim3(BLOCK), 0, stream, x, delta, psum, slices, col_scales, w, h_out, y, staged, static_cast<int>(dim), eps);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(rows)), dim3(BLOCK), 0, stream, x, delta, psum, slices, col_scales, w, h_out, y, staged, sums, static_cast<int>(dim), eps);
   };
   if (delta) launch(rmsnorm_kernel<BLOCK, PIECES, kDelta, 1>);
   else if (!psum) launch(rmsnorm_kernel<BLOCK, PIECES, kNothing, 1>);
@@ -610,13 +624,13 @@ void launch_rmsnorm_block(const uint16_t *x, const uint16_t *delta, const float 
 // 1024 threads leave a CU one row at a time (512 rows of 8192, two slices: 14.4 us, with two pieces 13.2; 320 of 5120 8.2 and 7.3; without sums 5.5 and 5.9: left).
 // More rows: workgroups of 256.  Rows of 2048 and fewer are one piece of those (64 rows, four slices 3.5 us; with a second, empty piece 4.2).
 void launch_rmsnorm(const uint16_t *x, const uint16_t *delta, const float *psum, int slices, const uint16_t *col_scales, const uint16_t *w,
-                    uint16_t *h_out, uint16_t *y, StagedOut staged, int64_t rows, int64_t dim, float eps, hipStream_t stream) {
+                    uint16_t *h_out, uint16_t *y, StagedOut staged, int64_t rows, int64_t dim, float eps, hipStream_t stream, GroupSums sums = {}) {
   const bool few = rows <= 512;
   const auto launch = dim <= 2048 ? launch_rmsnorm_block<256, 1>
                       : !few || dim < 4096 ? launch_rmsnorm_block<256, 2>
                       : dim == 4096 ? launch_rmsnorm_block<512, 1>
                       : (psum || delta) && rows > 256 ? launch_rmsnorm_block<512, 2> : launch_rmsnorm_block<1024, 1>;
-  launch(x, delta, psum, slices, col_scales, w, h_out, y, staged, rows, dim, eps, stream);
+  launch(x, delta, psum, slices, col_scales, w, h_out, y, staged, sums, rows, dim, eps, stream);
 }
 
 template <int D, int NW>
@@ -809,6 +823,18 @@ extern "C" int e2h_add_rmsnorm_staged(const uint16_t *x, const uint16_t *delta, 
     return E2H_ERR_MISALIGNED;
   launch_rmsnorm(x, delta, partials, partials ? slices : 0, partials ? col_scales : nullptr, weight, h_out, y, staged_out(staged, rows, dim), rows, dim,
                  eps, static_cast<hipStream_t>(stream));
+  return launch_status();
+}
+
+extern "C" int e2h_add_rmsnorm_sums(const uint16_t *x, const uint16_t *delta, const float *partials, int slices, const uint16_t *weight, uint16_t *h_out, uint16_t *y, float *sums,
+                                    int64_t rows, int64_t dim, int groupsize, float eps, void *stream) {
+  if (!x || !weight || !y || !sums || ((delta || partials) && !h_out)) return E2H_ERR_NULL_POINTER;
+  if (groupsize != 32 && groupsize != 64 && groupsize != 128 && groupsize != 256) return E2H_ERR_BAD_GROUPSIZE;
+  if ((delta && partials) || (partials && (slices < 1 || slices > 64)) || rows < 1 || rows > INT32_MAX / 2 || dim < 128 || dim % 128 != 0 || dim % groupsize != 0 || dim > INT32_MAX)
+    return E2H_ERR_BAD_SHAPE;
+  if (!aligned16(x) || !aligned16(delta) || !aligned16(partials) || !aligned16(weight) || !aligned16(h_out) || !aligned16(y) || !aligned16(sums)) return E2H_ERR_MISALIGNED;
+  const GroupSums to = {sums, static_cast<int>((rows + 63) / 64 * 64), (groupsize == 256 ? 128 : groupsize) / 8};
+  launch_rmsnorm(x, delta, partials, partials ? slices : 0, nullptr, weight, h_out, y, StagedOut{}, rows, dim, eps, static_cast<hipStream_t>(stream), to);
   return launch_status();
 }
 

@@ -6,7 +6,7 @@
 // raises its error, and so it does where an entry point refuses its arguments.  A launch that failed is reported from here: asked once more, the
 // runtime may take it, over whatever of a call of several launches has begun.
 //
-// Both functions take (x, weight, scales, .., out_features) and return a new tensor or None.
+// The functions take (x, weight, scales, .., out_features, ..) and return a new tensor or None.
 #include <Python.h>
 
 #include <ATen/core/Tensor.h>
@@ -25,10 +25,14 @@ namespace {
 
 typedef int (*Int4Mm)(const void *, const void *, const void *, void *, int64_t, int64_t, int64_t, int, int, void *, int64_t, void *);
 typedef int (*Int8Mm)(const void *, const void *, const void *, void *, int64_t, int64_t, int64_t, void *, int64_t, void *);
+typedef int (*Int4Rows)(const void *, const void *, const void *, void *, int, void *, void *, int64_t, int64_t, int64_t, int, int, void *);
+typedef int (*Int4RowsSlices)(int64_t, int64_t, int64_t, int, int);
 typedef int (*Capturing)(void *);
 
 Int4Mm int4_mm_entry = nullptr;
 Int8Mm int8_mm_entry = nullptr;
+Int4Rows int4_rows_entry = nullptr;
+Int4RowsSlices int4_rows_slices_entry = nullptr;
 Capturing capturing_entry = nullptr;
 PyObject *workspaces = nullptr;  // ops._workspaces: (device index, stream) -> tensor
 PyObject *check = nullptr;       // _lib.check: raises what a status stands for
@@ -95,6 +99,22 @@ PyObject *run(const char *entry, const at::Tensor &x, int64_t n, c10::DeviceInde
   return THPVariable_Wrap(std::move(y));
 }
 
+struct Int4Call {
+  c10::DeviceIndex device;
+  int64_t m, n, k, g;
+};
+
+// the sizes of x beside packed weights with inner_k_tiles 8; false: not for here
+bool int4_call(const at::Tensor &x, const at::Tensor &w, const at::Tensor &sz, int64_t g, int64_t out, Int4Call *c) {
+  if (!x.defined() || !x.is_cuda()) return false;
+  c->device = x.get_device();
+  if (c->device != c10::hip::current_device() || !plain(x, c->device, at::kBFloat16) || !plain(w, c->device, at::kInt) || !plain(sz, c->device, at::kBFloat16)) return false;
+  if (x.dim() < 1 || w.dim() != 4 || sz.dim() != 3 || w.size(2) != 32 || w.size(3) != 4) return false;
+  c->n = w.size(0) * 8, c->k = w.size(1) * 128, c->m = c->k > 0 ? x.numel() / c->k : 0, c->g = g;
+  if (x.size(-1) != c->k || c->n != out || c->m < 1 || c->m > kMostRows || (g != 32 && g != 64 && g != 128 && g != 256) || c->k % g != 0) return false;
+  return sz.size(0) == c->k / g && sz.size(1) == c->n && sz.size(2) == 2;
+}
+
 // (x, packed, scales_and_zeros, groupsize, out_features); inner_k_tiles 8
 PyObject *int4_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
@@ -105,16 +125,50 @@ PyObject *int4_linear(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   }
   const at::Tensor &x = THPVariable_Unpack(args[0]), &w = THPVariable_Unpack(args[1]), &sz = THPVariable_Unpack(args[2]);
-  if (!x.defined() || !x.is_cuda()) Py_RETURN_NONE;
-  const c10::DeviceIndex device = x.get_device();
-  if (device != c10::hip::current_device() || !plain(x, device, at::kBFloat16) || !plain(w, device, at::kInt) || !plain(sz, device, at::kBFloat16)) Py_RETURN_NONE;
-  if (x.dim() < 1 || w.dim() != 4 || sz.dim() != 3 || w.size(2) != 32 || w.size(3) != 4) Py_RETURN_NONE;
-  const int64_t n = w.size(0) * 8, k = w.size(1) * 128, m = k > 0 ? x.numel() / k : 0;
-  if (x.size(-1) != k || n != out || m < 1 || m > kMostRows || (g != 32 && g != 64 && g != 128 && g != 256) || k % g != 0) Py_RETURN_NONE;
-  if (sz.size(0) != k / g || sz.size(1) != n || sz.size(2) != 2) Py_RETURN_NONE;
-  return run("e2h_int4_mm", x, n, device, [&](void *y, void *ws, int64_t ws_bytes, void *stream) {
-    return int4_mm_entry(x.data_ptr(), w.data_ptr(), sz.data_ptr(), y, m, n, k, static_cast<int>(g), 8, ws, ws_bytes, stream);
+  Int4Call c;
+  if (!int4_call(x, w, sz, g, out, &c)) Py_RETURN_NONE;
+  return run("e2h_int4_mm", x, c.n, c.device, [&](void *y, void *ws, int64_t ws_bytes, void *stream) {
+    return int4_mm_entry(x.data_ptr(), w.data_ptr(), sz.data_ptr(), y, c.m, c.n, c.k, static_cast<int>(g), 8, ws, ws_bytes, stream);
   });
+  END_HANDLE_TH_ERRORS
+}
+
+// (x, packed, scales_and_zeros, groupsize, out_features, sums or None, defer): e2h_int4_mm_rows, where it takes the call.  sums: e2h_add_rmsnorm_sums' of x.  defer: where K is shared, the slices'
+// sums [slices, m, n] in the result's place.
+PyObject *int4_rows(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 7 || !int4_rows_entry || !THPVariable_CheckExact(args[0]) || !THPVariable_CheckExact(args[1]) || !THPVariable_CheckExact(args[2]) ||
+      (args[5] != Py_None && !THPVariable_CheckExact(args[5])) || watched())
+    Py_RETURN_NONE;
+  const int64_t g = PyLong_AsLongLong(args[3]), out = PyLong_AsLongLong(args[4]);
+  const bool defer = args[6] == Py_True, there = args[5] != Py_None;
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  const at::Tensor &x = THPVariable_Unpack(args[0]), &w = THPVariable_Unpack(args[1]), &sz = THPVariable_Unpack(args[2]);
+  Int4Call c;
+  if (!int4_call(x, w, sz, g, out, &c)) Py_RETURN_NONE;
+  const int slices = int4_rows_slices_entry(c.m, c.n, c.k, static_cast<int>(g), 8);
+  void *const stream = c10::hip::getCurrentHIPStream(c.device).stream();
+  if (slices < 1 || capturing_entry(stream) != 0) Py_RETURN_NONE;
+  const int64_t groups = c.k / (g < 128 ? g : 128), stride = (c.m + 63) / 64 * 64;
+  const auto floats = x.options().dtype(at::kFloat);
+  at::Tensor sums = there ? THPVariable_Unpack(args[5]) : at::empty({groups, stride}, floats), partials, y;
+  if (there && (!plain(sums, c.device, at::kFloat) || sums.dim() != 2 || sums.size(0) != groups || sums.size(1) != stride)) Py_RETURN_NONE;
+  if (slices > 1) partials = at::empty({slices, c.m, c.n}, floats);
+  if (slices == 1 || !defer) y = result_for(x, c.n);
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = int4_rows_entry(x.data_ptr(), w.data_ptr(), sz.data_ptr(), sums.data_ptr(), there, y.defined() ? y.data_ptr() : nullptr, partials.defined() ? partials.data_ptr() : nullptr, c.m, c.n,
+                       c.k, static_cast<int>(g), 8, stream);
+  Py_END_ALLOW_THREADS
+  if (failed(rc)) {
+    Py_XDECREF(PyObject_CallFunction(check, "is", rc, "e2h_int4_mm_rows"));
+    return nullptr;
+  }
+  if (rc != 0) Py_RETURN_NONE;
+  return THPVariable_Wrap(std::move(y.defined() ? y : partials));
   END_HANDLE_TH_ERRORS
 }
 
@@ -157,9 +211,20 @@ PyObject *bind(PyObject *, PyObject *args) {
   Py_RETURN_NONE;
 }
 
+// bind_rows(address of e2h_int4_mm_rows, of e2h_int4_mm_rows_slices)
+PyObject *bind_rows(PyObject *, PyObject *args) {
+  unsigned long long rows = 0, slices = 0;
+  if (!PyArg_ParseTuple(args, "KK", &rows, &slices)) return nullptr;
+  int4_rows_entry = reinterpret_cast<Int4Rows>(static_cast<uintptr_t>(rows));
+  int4_rows_slices_entry = reinterpret_cast<Int4RowsSlices>(static_cast<uintptr_t>(slices));
+  Py_RETURN_NONE;
+}
+
 PyMethodDef methods[] = {{"int4_linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(int4_linear)), METH_FASTCALL, nullptr},
                          {"int8_linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(int8_linear)), METH_FASTCALL, nullptr},
+                         {"int4_rows", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(int4_rows)), METH_FASTCALL, nullptr},
                          {"bind", bind, METH_VARARGS, nullptr},
+                         {"bind_rows", bind_rows, METH_VARARGS, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_calls", nullptr, -1, methods};
 

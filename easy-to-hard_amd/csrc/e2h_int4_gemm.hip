@@ -634,7 +634,7 @@ int int4_gemm(const uint16_t *x, const int32_t *packed, const uint16_t *sz, uint
                       xsum, xsum_stride, M, N, K, 0, 0, shared, run_if, row_flag};
   const int rc = launch_gemm<false>(a, groupsize, shape, stream);
   if (rc != E2H_OK) return rc;
-  if (shape.slices > 1) {
+  if (shape.slices > 1 && y) {
     const int64_t quads = static_cast<int64_t>(M) * N / 4;
     hipLaunchKernelGGL(add_slices_kernel, dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, stream, partials, y, quads,
                        static_cast<int64_t>(M) * N, shape.slices);
@@ -695,7 +695,45 @@ bool int4_gate_rows_pay(int64_t M, int64_t N, int64_t K, int groupsize, int inne
   }
   return 1.03 * int4_gemm_shape(m, 2 * n, k, G, 0).us + 6 < 2 * call + 3 + static_cast<double>(M) * static_cast<double>(N) * 6 / 5e6;
 }
+
+// The K slices of e2h_int4_mm_rows, 0 where it takes no such call: 65 to 1023 rows that e2h_int4_mm, given a workspace of the usual size, would run on this file's kernel, with the same
+// rows per workgroup and slices.
+Int4GemmShape int4_rows_shape(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles) {
+  const Int4GemmShape none = {0, 0, 0.};
+  if (inner_k_tiles != 8 || (groupsize != 32 && groupsize != 64 && groupsize != 128 && groupsize != 256)) return none;
+  if (m <= 64 || m >= kUnpackRows || n < 8 || n % 8 != 0 || k < 128 || k % 128 != 0 || k % groupsize != 0 || n > INT32_MAX / 64 || k > INT32_MAX / 64) return none;
+  if (m * k * 2 >= (int64_t{1} << 32) || n * k / 2 >= (int64_t{1} << 32) || k / groupsize * n * 4 >= (int64_t{1} << 32)) return none;
+  const Options &o = options();
+  if (o.int4_no_gemm32 || o.int4_gemm_tile || o.int4_gemm32_min_rows || o.int4_no_xsum || o.int4_k_slices || o.int4_rows_per_wave || o.int4_k_groups || o.int4_col_waves || o.row_tiles)
+    return none;
+  const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k), G = groupsize == 256 ? 128 : groupsize;
+  const Int4GemmShape shape = int4_gemm_shape(M, N, K, G, (int64_t{32} << 20) - k / G * ((m + 63) / 64 * 64) * 4);
+  if (groupsize != 256 && (m + 127) / 128 * ((n + 127) / 128) >= 320) return shape;
+  const int tiles = groupsize != 256 && (N + 127) / 128 * ((M + 63) / 64) >= 256 ? 2 : 1;
+  return shape.us < int4_rows_us(M, N, K, groupsize, tiles) ? shape : none;
+}
 }  // namespace e2h
+
+extern "C" int e2h_int4_mm_rows_slices(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles) {
+  return e2h::int4_rows_shape(m, n, k, groupsize, inner_k_tiles).slices;
+}
+
+extern "C" int e2h_int4_mm_rows(const uint16_t *x, const int32_t *packed, const uint16_t *scales_and_zeros, float *sums, int sums_there, uint16_t *y, float *partials, int64_t m, int64_t n,
+                                int64_t k, int groupsize, int inner_k_tiles, void *stream) {
+  using namespace e2h;
+  if (!x || !packed || !scales_and_zeros || !sums) return E2H_ERR_NULL_POINTER;
+  const Int4GemmShape shape = int4_rows_shape(m, n, k, groupsize, inner_k_tiles);
+  if (shape.slices == 0) return E2H_ERR_BAD_SHAPE;
+  if (shape.slices > 1 ? !partials : !y) return E2H_ERR_NULL_POINTER;
+  if (!aligned16(x) || !aligned16(packed) || !aligned16(scales_and_zeros) || !aligned16(sums) || !aligned16(partials) || (reinterpret_cast<uintptr_t>(y) & 7u)) return E2H_ERR_MISALIGNED;
+  const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k), stride = (M + 63) / 64 * 64;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (!sums_there) {
+    const int rc = launch_x_group_sums(x, sums, M, K, stride, groupsize == 256 ? 128 : groupsize, s);
+    if (rc != E2H_OK) return rc;
+  }
+  return int4_gemm(x, packed, scales_and_zeros, y, sums, stride, partials, shape, M, N, K, groupsize, s);
+}
 
 extern "C" int64_t e2h_int4_mm_silu_gate_rows_scratch_bytes(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles) {
   return e2h::int4_gate_rows_bytes(m, n, k, groupsize, inner_k_tiles);
@@ -705,10 +743,10 @@ extern "C" int e2h_int4_mm_silu_gate_rows_pays(int64_t m, int64_t n, int64_t k, 
   return e2h::int4_gate_rows_pay(m, n, k, groupsize, inner_k_tiles);
 }
 
-extern "C" int e2h_int4_mm_silu_gate_rows(const uint16_t *x, const int32_t *packed_gate, const uint16_t *sz_gate, const int32_t *packed_up, const uint16_t *sz_up,
-                                          uint16_t *y, int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles, void *scratch, int64_t scratch_bytes,
-                                          void *stream) {
-  using namespace e2h;
+namespace e2h {
+namespace {
+int gate_rows(const uint16_t *x, const int32_t *packed_gate, const uint16_t *sz_gate, const int32_t *packed_up, const uint16_t *sz_up, uint16_t *y, int64_t m, int64_t n, int64_t k,
+              int groupsize, int inner_k_tiles, void *scratch, int64_t scratch_bytes, bool sums_there, void *stream) {
   if (!x || !packed_gate || !sz_gate || !packed_up || !sz_up || !y || !scratch) return E2H_ERR_NULL_POINTER;
   if (groupsize != 32 && groupsize != 64 && groupsize != 128 && groupsize != 256) return E2H_ERR_BAD_GROUPSIZE;
   if (inner_k_tiles != 8) return E2H_ERR_BAD_INNER_K_TILES;
@@ -720,10 +758,25 @@ extern "C" int e2h_int4_mm_silu_gate_rows(const uint16_t *x, const int32_t *pack
     return E2H_ERR_MISALIGNED;
   const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k), G = groupsize == 256 ? 128 : groupsize, stride = (M + 63) / 64 * 64;
   if (aligned16(y) && int4_gate_unpacked_bytes(m, n, k, groupsize, inner_k_tiles) > 0)
-    return int4_unpacked_gate(x, packed_gate, sz_gate, packed_up, sz_up, y, M, N, K, groupsize, scratch, static_cast<hipStream_t>(stream));
+    return sums_there ? E2H_ERR_BAD_SHAPE
+                      : int4_unpacked_gate(x, packed_gate, sz_gate, packed_up, sz_up, y, M, N, K, groupsize, scratch, static_cast<hipStream_t>(stream));
   float *xsum = static_cast<float *>(scratch);
-  const int rc = launch_x_group_sums(x, xsum, M, K, stride, G, static_cast<hipStream_t>(stream));
+  const int rc = sums_there ? E2H_OK : launch_x_group_sums(x, xsum, M, K, stride, G, static_cast<hipStream_t>(stream));
   if (rc != E2H_OK) return rc;
   return int4_gemm_gate(x, packed_gate, sz_gate, packed_up, sz_up, y, xsum, stride, int4_gemm_shape(M, 2 * N, K, G, 0), M, N, K, groupsize,
                         static_cast<hipStream_t>(stream));
+}
+}  // namespace
+}  // namespace e2h
+
+extern "C" int e2h_int4_mm_silu_gate_rows(const uint16_t *x, const int32_t *packed_gate, const uint16_t *sz_gate, const int32_t *packed_up, const uint16_t *sz_up,
+                                          uint16_t *y, int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles, void *scratch, int64_t scratch_bytes,
+                                          void *stream) {
+  return e2h::gate_rows(x, packed_gate, sz_gate, packed_up, sz_up, y, m, n, k, groupsize, inner_k_tiles, scratch, scratch_bytes, false, stream);
+}
+
+extern "C" int e2h_int4_mm_silu_gate_rows_sums(const uint16_t *x, const int32_t *packed_gate, const uint16_t *sz_gate, const int32_t *packed_up, const uint16_t *sz_up,
+                                               uint16_t *y, int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles, void *sums, int64_t sums_bytes, void *stream) {
+  return m >= e2h::kUnpackRows ? E2H_ERR_BAD_SHAPE
+                               : e2h::gate_rows(x, packed_gate, sz_gate, packed_up, sz_up, y, m, n, k, groupsize, inner_k_tiles, sums, sums_bytes, true, stream);
 }

@@ -18,7 +18,7 @@ import torch.nn.functional as F
 from torch import Tensor
 from torch.utils._device import DeviceContext
 
-from . import ops, seq_ops
+from . import _lib, ops, seq_ops
 from .linear import unwatched
 from .quantize import WeightOnlyInt4Linear, WeightOnlyInt8Linear, find_multiple
 from .state import KVCache
@@ -139,6 +139,23 @@ def _project_deferred(lin, y2d: Tensor, lead_shape) -> Tensor:
     return lin(y2d.view(*lead_shape, -1))
 
 
+def _product_rows(lin, x: Tensor, sums: Optional[Tensor], defer: bool = False) -> Tensor:
+    """lin(x) of a prompt.  sums: those of x's quantization groups, from the norm in front (None: there are none).  defer: where the library shares K, the float32 sums of its
+    slices [slices, rows, N] may come back, for the next norm to add."""
+    if type(lin) is WeightOnlyInt4Linear and not lin.padding and unwatched(lin):
+        y = _lib.calls().int4_rows(x, lin.weight, lin.scales_and_zeros, lin.groupsize, lin.out_features, sums, defer)
+        if y is not None:
+            return y
+    return lin(x)
+
+
+def _sums_serve(lin, x: Tensor) -> bool:
+    """True where the products of a prompt's rows through `lin` read sums of quantization groups that a norm of x can leave."""
+    k = x.shape[-1]
+    return (type(lin) is WeightOnlyInt4Linear and not lin.padding and lin.in_features == k and k % 128 == 0 and k % lin.groupsize == 0
+            and ops.int4_rows_slices(x.numel() // k, lin.out_features, k, lin.groupsize, lin.inner_k_tiles) > 0)
+
+
 def _stock_attention_wanted() -> bool:
     """True where somebody intercepts torch functions (a default device does so too, but looks at no attention), or has switched off the backend whose place the
     package's attention of prompts takes."""
@@ -219,8 +236,9 @@ class Attention(nn.Module):
         return ops.int4_mm_rope_kv_rows(x, *weights, w.groupsize, f, k, v, input_pos, *heads)
 
     def forward(self, x: Tensor, freqs_cis: Optional[Tensor], mask: Optional[Tensor], input_pos: Optional[Tensor] = None,
-                fully_causal: bool = False, defer_output: bool = False) -> Tensor:
-        """defer_output (fused decode step only): the output projection may come back as float32 partial sums over K
+                fully_causal: bool = False, defer_output: bool = False, sums: Optional[Tensor] = None) -> Tensor:
+        """sums (TransformerBlock._forward_rows): those of x's quantization groups.
+        defer_output (fused decode step, or sums): the output projection may come back as float32 partial sums over K
         slices, to be added by the residual add + RMSNorm that follows (ops.add_rmsnorm takes either form)."""
         bsz, seqlen, _ = x.shape
         kv_size = self.n_local_heads * self.head_dim
@@ -253,12 +271,12 @@ class Attention(nn.Module):
                 k, v = self.kv_cache.k_cache, self.kv_cache.v_cache
             q = self._rope_rows(x, k, v, input_pos, fully_causal)
             if q is None:
-                q = ops.rope_kv_write_seq(self.wqkv(x), self.freqs_table, k, v, input_pos, self.n_head, self.n_local_heads, self.head_dim,
+                q = ops.rope_kv_write_seq(self.wqkv(x) if sums is None else _product_rows(self.wqkv, x, sums), self.freqs_table, k, v, input_pos, self.n_head, self.n_local_heads, self.head_dim,
                                           rows_by_token=fully_causal)
             if ((fully_causal or isinstance(mask, _MaskByPosition)) and not torch.compiler.is_compiling()
                     and ops.prefill_attention_fits(bsz, seqlen, self.n_head, k, v, not fully_causal) and not seq_ops.watched(q, k, v) and not _stock_attention_wanted()):
                 y = ops.prefill_attention(q, k, v, None if fully_causal else input_pos, None if fully_causal else mask.left_pad)
-                return self.wo(y)
+                return self.wo(y) if sums is None else _product_rows(self.wo, y, None, defer_output)
             k, v = k[:bsz], v[:bsz]
         else:
             q, k, v = self.wqkv(x).split([self.dim, kv_size, kv_size], dim=-1)
@@ -302,7 +320,7 @@ class FeedForward(nn.Module):
             return False
         return ops.int8_gate_supported(x, w1, w3)
 
-    def _gate_rows(self, x: Tensor) -> Optional[Tensor]:
+    def _gate_rows(self, x: Tensor, sums: Optional[Tensor] = None) -> Optional[Tensor]:
         """silu(w1 x) * w3 x of a prompt with one launch for both products, or None where the modules are to be called: few rows, weights that differ in form or do not fit x,
         somebody who watches their calls, or no gain."""
         w1, w3 = self.w1, self.w3
@@ -323,7 +341,7 @@ class FeedForward(nn.Module):
                 return None
         if seq_ops.watched(x, w1.weight, w1.scales_and_zeros, w3.weight, w3.scales_and_zeros):
             return None
-        y = ops.int4_mm_silu_gate_rows(x.reshape(-1, k), w1.weight, w1.scales_and_zeros, w3.weight, w3.scales_and_zeros, group)
+        y = ops.int4_mm_silu_gate_rows(x.reshape(-1, k), w1.weight, w1.scales_and_zeros, w3.weight, w3.scales_and_zeros, group, sums)
         return None if y is None else y.view(*x.shape[:-1], n)
 
     def _gate_rows_int8(self, x: Tensor) -> Optional[Tensor]:
@@ -341,7 +359,11 @@ class FeedForward(nn.Module):
         y = ops.int8_mm_silu_gate_rows(x.reshape(-1, k), w1.weight, w1.scales, w3.weight, w3.scales)
         return None if y is None else y.view(*x.shape[:-1], n)
 
-    def forward(self, x: Tensor, defer_output: bool = False) -> Tensor:
+    def forward(self, x: Tensor, defer_output: bool = False, sums: Optional[Tensor] = None) -> Tensor:
+        if sums is not None:  # TransformerBlock._forward_rows
+            y = self._gate_rows(x, sums)
+            if y is not None:
+                return _product_rows(self.w2, y, None, defer_output)
         if defer_output and self._gate_fusable_int8(x):
             y = ops.int8_mm_silu_gate(x.reshape(-1, x.shape[-1]), self.w1.weight, self.w1.scales, self.w3.weight, self.w3.scales)
             return _project_deferred(self.w2, y, x.shape[:-1])
@@ -390,6 +412,8 @@ class TransformerBlock(nn.Module):
         residual stream yet; the add is folded into this block's first norm.  Returns (h, this block's pending delta)."""
         if not fully_causal and x.shape[1] == 1 and self._norms_fold(x, delta):
             return self._forward_folded(x, delta, input_pos)
+        if self._rows_alone(x, input_pos, fully_causal):
+            return self._forward_rows(x, delta, input_pos, freqs_cis, mask, fully_causal)
         if delta is None:
             normed = ops.rmsnorm(x, self.attention_norm.weight, self.attention_norm.eps)
         else:
@@ -398,6 +422,25 @@ class TransformerBlock(nn.Module):
         h, normed2 = ops.add_rmsnorm(x, attn, self.ffn_norm.weight, self.ffn_norm.eps)
         return h, self.feed_forward(normed2, defer_output=DEFER_SPLIT_K)
 
+
+    def _rows_alone(self, x: Tensor, input_pos, fully_causal: bool) -> bool:
+        """True for a prompt of 65 to 1023 rows through an int4 block whose modules nobody watches: the norms leave the sums of quantization groups for the products behind them, and
+        add the slices of those in front of them."""
+        rows = x.shape[0] * x.shape[1]
+        if rows <= 64 or rows >= ops._UNPACK_ROWS or torch.compiler.is_compiling() or not (FUSE_GATE and DEFER_SPLIT_K):
+            return False
+        att, ff, norms = self.attention, self.feed_forward, (self.attention_norm, self.ffn_norm)
+        if not (type(att) is Attention and type(ff) is FeedForward and all(type(m) is RMSNorm and m.weight.dtype == torch.bfloat16 and m.weight.is_contiguous() for m in norms)
+                and all(unwatched(m) for m in (*norms, att, ff))):
+            return False
+        return _sums_serve(att.wqkv, x) and _sums_serve(ff.w1, x) and att._can_fuse_prefill_rope(x, input_pos, fully_causal) and not seq_ops.watched(x)
+
+    def _forward_rows(self, x: Tensor, delta, input_pos, freqs_cis, mask, fully_causal: bool):
+        att, ff, a, f = self.attention, self.feed_forward, self.attention_norm, self.ffn_norm
+        x, normed, sums = ops.add_rmsnorm_sums(x, delta, a.weight, a.eps, att.wqkv.groupsize)
+        attn = att(normed, freqs_cis, mask, input_pos, fully_causal, defer_output=True, sums=sums)
+        h, normed, sums = ops.add_rmsnorm_sums(x, attn, f.weight, f.eps, ff.w1.groupsize)
+        return h, ff(normed, defer_output=True, sums=sums)
 
     def _norms_fold(self, x: Tensor, delta) -> bool:
         """True for the single-token step of one sequence through an int8 model whose modules nobody watches: the products behind the norms form their row themselves."""
@@ -588,6 +631,11 @@ class Transformer(nn.Module):
             if (fused_step and x.shape[0] == 1 and not torch.compiler.is_compiling() and type(out) is WeightOnlyInt8Linear and type(self.norm) is RMSNorm and unwatched(out) and unwatched(self.norm)
                     and ops.int8_norm_fits(x, self.norm.weight, delta, out)):
                 return ops.int8_norm_mm(x, delta, self.norm.weight, self.norm.eps, out.weight, out.scales)[1].view(x.shape[0], 1, -1)
+            rows = x.shape[0] * x.shape[1]
+            if (64 < rows < ops._UNPACK_ROWS and not torch.compiler.is_compiling() and DEFER_SPLIT_K and type(self.norm) is RMSNorm and unwatched(self.norm)
+                    and _sums_serve(out, x) and not seq_ops.watched(x)):
+                _, normed, sums = ops.add_rmsnorm_sums(x, delta, self.norm.weight, self.norm.eps, out.groupsize)
+                return _product_rows(out, normed, sums)
             _, normed = ops.add_rmsnorm(x, delta, self.norm.weight, self.norm.eps)
             return self.output(normed)
         for layer in self.layers:

@@ -383,9 +383,9 @@ def int4_gate_rows_pay(m, n, k, groupsize, inner_k_tiles=8) -> bool:
     return bool(_lib.load().e2h_int4_mm_silu_gate_rows_pays(m, n, k, groupsize, inner_k_tiles))
 
 
-def int4_mm_silu_gate_rows(x, packed_gate, sz_gate, packed_up, sz_up, groupsize):
+def int4_mm_silu_gate_rows(x, packed_gate, sz_gate, packed_up, sz_up, groupsize, sums=None):
     """bf16(bf16(silu(int4_mm(x, gate))) * int4_mm(x, up)) over more than 64 rows in one product launch, or None where the sizes are not taken
-    (or there is no memory for the launch's scratch)."""
+    (or there is no memory for the launch's scratch).  sums: add_rmsnorm_sums' of x, under 1024 rows."""
     _need_gpu(x, packed_gate, sz_gate, packed_up, sz_up)
     if x.dtype != torch.bfloat16 or sz_gate.dtype != torch.bfloat16 or sz_up.dtype != torch.bfloat16:
         raise TypeError("int4_mm_silu_gate_rows: bfloat16 activations and scales_and_zeros expected")
@@ -399,16 +399,57 @@ def int4_mm_silu_gate_rows(x, packed_gate, sz_gate, packed_up, sz_up, groupsize)
     for sz in (sz_gate, sz_up):
         if groupsize not in _VALID_GROUPS or k % groupsize != 0 or tuple(sz.shape) != (k // groupsize, n, 2):
             raise RuntimeError(f"int4_mm_silu_gate_rows: groupsize={groupsize} does not fit scales_and_zeros {tuple(sz.shape)} and K={k}")
-    scratch = int4_gate_rows_scratch(m, n, k, groupsize, ikt, x.device)
+    if sums is not None:
+        _group_sums_fit(sums, m, k, groupsize, x.device)
+        name, scratch = "e2h_int4_mm_silu_gate_rows_sums", sums.view(torch.uint8).view(-1)
+    else:
+        name, scratch = "e2h_int4_mm_silu_gate_rows", int4_gate_rows_scratch(m, n, k, groupsize, ikt, x.device)
     if scratch is None:
         return None
     x, packed_gate, sz_gate = x.contiguous(), packed_gate.contiguous(), sz_gate.contiguous()
     packed_up, sz_up = packed_up.contiguous(), sz_up.contiguous()
     y = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
-    rc = _lib_for(x).e2h_int4_mm_silu_gate_rows(_ptr(x), _ptr(packed_gate), _ptr(sz_gate), _ptr(packed_up), _ptr(sz_up), _ptr(y), m, n, k, groupsize, ikt,
+    rc = getattr(_lib_for(x), name)(_ptr(x), _ptr(packed_gate), _ptr(sz_gate), _ptr(packed_up), _ptr(sz_up), _ptr(y), m, n, k, groupsize, ikt,
                                                 _ptr(scratch), scratch.numel(), _stream(x))
-    _lib.check(rc, "e2h_int4_mm_silu_gate_rows")
+    _lib.check(rc, name)
     return y
+
+
+def _group_sums_empty(rows, k, groupsize, device):
+    return torch.empty((k // min(groupsize, 128), (rows + 63) // 64 * 64), dtype=torch.float32, device=device)
+
+
+def _group_sums_fit(sums, rows, k, groupsize, device):
+    assert sums.dtype == torch.float32 and sums.is_contiguous() and sums.device == device and tuple(sums.shape) == (k // min(groupsize, 128), (rows + 63) // 64 * 64)
+
+
+def add_rmsnorm_sums(x, delta, weight, eps, groupsize):
+    """RMSNorm of h = x (delta None) or h = bf16(x + delta) (delta as add_rmsnorm takes it, of int4 linears), and the normalised rows' sums over quantization groups, which
+    int4_mm and int4_mm_silu_gate_rows otherwise form in a launch of their own -> (h, y, sums)."""
+    _need_gpu(x, weight)
+    assert x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
+    x = x.contiguous()
+    dim = x.shape[-1]
+    rows = x.numel() // dim
+    h, y, sums = x, torch.empty_like(x), _group_sums_empty(rows, dim, groupsize, x.device)
+    d16 = part = None
+    if delta is not None:
+        h = torch.empty_like(x)
+        if delta.dtype == torch.float32:
+            assert delta.dim() == 3 and delta.is_contiguous() and tuple(delta.shape[1:]) == (rows, dim)
+            part = delta
+        else:
+            assert delta.dtype == torch.bfloat16 and delta.shape == x.shape
+            d16 = delta.contiguous()
+    rc = _lib_for(x).e2h_add_rmsnorm_sums(_ptr(x), _ptr(d16) if d16 is not None else None, _ptr(part) if part is not None else None, part.shape[0] if part is not None else 0, _ptr(weight),
+                                          _ptr(h) if delta is not None else None, _ptr(y), _ptr(sums), rows, dim, groupsize, float(eps), _stream(x))
+    _lib.check(rc, "e2h_add_rmsnorm_sums")
+    return h, y, sums
+
+
+def int4_rows_slices(rows, n, k, groupsize, inner_k_tiles) -> int:
+    """K slices of e2h_int4_mm_rows, 0 where it does not take such a call."""
+    return _lib.load().e2h_int4_mm_rows_slices(rows, n, k, groupsize, inner_k_tiles)
 
 
 # ---------------------------------------------------------------------------------------------

@@ -229,6 +229,21 @@ int e2h_int4_mm_silu_gate_rows(const uint16_t *x, const int32_t *packed_gate, co
                                const uint16_t *sz_up, uint16_t *y, int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles,
                                void *scratch, int64_t scratch_bytes, void *stream);
 
+/* The products of a prompt of 65 to 1023 rows with what surrounds them in fewer launches.  `sums`: float32 [k / g][m rounded up to 64], the sums of every row of x over the weights'
+ * quantization groups (g = groupsize, 128 for groupsize 256), 16-byte aligned, which the matmul needs for its zero points.
+ *   e2h_add_rmsnorm_sums: e2h_rmsnorm, e2h_add_rmsnorm or (slices in order) e2h_add_rmsnorm_partials that writes those of y beside y; dim % 128 == 0, dim % groupsize == 0.
+ *   e2h_int4_mm_rows: e2h_int4_mm over such rows, bit for bit; sums_there == 0: it forms the sums itself, in `sums`.  With K in e2h_int4_mm_rows_slices > 1 slices `partials`
+ *   (float32 [slices, m, n]) is needed and holds the slices' sums, and y may be NULL: whoever reads the sums adds them (e2h_add_rmsnorm_sums).  e2h_int4_mm_rows_slices is 0 where such
+ *   calls run on another kernel; e2h_int4_mm_rows returns E2H_ERR_BAD_SHAPE then.
+ *   e2h_int4_mm_silu_gate_rows_sums: e2h_int4_mm_silu_gate_rows with sums that are there in the place of scratch, fewer than 1024 rows. */
+int e2h_add_rmsnorm_sums(const uint16_t *x, const uint16_t *delta, const float *partials, int slices, const uint16_t *weight, uint16_t *h_out, uint16_t *y, float *sums,
+                         int64_t rows, int64_t dim, int groupsize, float eps, void *stream);
+int e2h_int4_mm_rows_slices(int64_t m, int64_t n, int64_t k, int groupsize, int inner_k_tiles);
+int e2h_int4_mm_rows(const uint16_t *x, const int32_t *packed, const uint16_t *scales_and_zeros, float *sums, int sums_there, uint16_t *y, float *partials, int64_t m, int64_t n,
+                     int64_t k, int groupsize, int inner_k_tiles, void *stream);
+int e2h_int4_mm_silu_gate_rows_sums(const uint16_t *x, const int32_t *packed_gate, const uint16_t *sz_gate, const int32_t *packed_up, const uint16_t *sz_up, uint16_t *y, int64_t m,
+                                    int64_t n, int64_t k, int groupsize, int inner_k_tiles, void *sums, int64_t sums_bytes, void *stream);
+
 /* int8 forms of the two fused decode-step launches above (WeightOnlyInt8Linear modules, reference
  * models/quantize.py:405-429, in FeedForward.forward models/model.py:343-344 and Attention.forward :283-296).
  * Each linear's output is formed with the reference's two roundings, bf16(bf16(x @ q^T) * scales), before the SiLU-gate

@@ -612,3 +612,69 @@ def test_int8_prompts_leave_watched_projections_to_the_modules():
         assert torch.equal(att(x, None, None, pos, True), whole) and seen == [1]
         handle.remove()
         assert att._rope_rows(x[:, :20], k, v, pos[:20], True) is None and att._rope_rows(x, k.transpose(0, 1), v.transpose(0, 1), pos, True) is None
+
+
+# ---- prompts whose norms leave the group sums and add the slices -----------------------------------------------------------------------
+
+@pytest.mark.parametrize("g,m,n,k", [(128, 471, 4096, 4096), (32, 65, 12288, 1024), (64, 129, 12296, 1152), (256, 1023, 3080, 2304), (128, 471, 2048, 5632)])
+def test_group_sums_of_a_norm_serve_the_products_behind_it(g, m, n, k):
+    gen = torch.Generator(device=DEV).manual_seed(m + n)
+    randn = lambda *shape: torch.randn(shape, generator=gen, device=DEV).to(torch.bfloat16)
+    x, delta, w = randn(m, k), randn(m, k), randn(k)
+    lins = [ops.int4_quantize_pack(randn(n, k) * 0.02, g, 8) for _ in range(2)]
+    part = torch.randn((2, m, k), generator=gen, device=DEV)
+    for term, (h, want) in ((None, (x, ops.rmsnorm(x, w, 1e-5))), (delta, ops.add_rmsnorm(x, delta, w, 1e-5)), (part, ops.add_rmsnorm(x, part, w, 1e-5))):
+        h2, y, sums = ops.add_rmsnorm_sums(x, term, w, 1e-5, g)
+        assert torch.equal(h2, h) and torch.equal(y, want)
+    own = y.double().view(m, -1, min(g, 128)).sum(-1).t()
+    assert (sums[:, :m].double() - own).abs().max() <= min(g, 128) * 2.0 ** -24 * y.double().abs().view(m, -1, min(g, 128)).sum(-1).max()  # float32 sums in any order
+    packed, sz = lins[0]
+    slices = ops.int4_rows_slices(m, n, k, g, 8)
+    assert slices > 0
+    want = ops.int4_mm(y, packed, g, sz)
+    rows = lambda *rest: _lib.calls().int4_rows(y, packed, sz, g, n, *rest)
+    assert torch.equal(rows(sums, False), want) and torch.equal(rows(None, False), want)
+    left = rows(sums, True)
+    assert rows(sums[:, 64:], True) is None and rows(sums.double(), True) is None and _lib.calls().int4_rows(y[:64], packed, sz, g, n, None, False) is None
+    if slices == 1:
+        assert torch.equal(left, want)
+    else:
+        assert tuple(left.shape) == (slices, m, n) and left.dtype == torch.float32
+        assert (left.double().sum(0) - want.double()).abs().max() <= 2.0 ** -8 * want.double().abs().max()
+    if ops.int4_gate_rows_pay(m, n, k, g):
+        assert torch.equal(ops.int4_mm_silu_gate_rows(y, *lins[0], *lins[1], g, sums), ops.int4_mm_silu_gate_rows(y, *lins[0], *lins[1], g))
+    assert slices == (4 if n == 2048 else 2 if n == 4096 else 1)
+    assert ops.int4_rows_slices(64, n, k, g, 8) == 0 and ops.int4_rows_slices(1024, n, k, g, 8) == 0
+
+
+def test_a_prompt_with_group_sums_from_its_norms_equals_the_modules(monkeypatch):
+    from easy_to_hard_amd import generate
+    from easy_to_hard_amd.model import ModelArgs, Transformer
+    from easy_to_hard_amd.quantize import WeightOnlyInt4QuantHandler
+
+    torch.manual_seed(0)
+    model = Transformer(ModelArgs(block_size=512, vocab_size=8192, n_layer=2, n_head=16, n_local_heads=16, dim=2048, intermediate_size=5632)).to(torch.bfloat16)
+    for p in model.parameters():
+        if p.dim() == 2:
+            p.data.normal_(0.0, 0.02)
+    handler = WeightOnlyInt4QuantHandler(model.to(DEV), groupsize=64)
+    state = handler.create_quantized_state_dict()
+    model = handler.convert_for_runtime()
+    model.load_state_dict(state, assign=True)
+    model = model.to(DEV).eval().requires_grad_(False)
+    model.setup_caches(3, 200)
+    ids, pads = torch.randint(0, 8192, (3, 157), device=DEV), torch.tensor([0, 40, 7], device=DEV)
+    calls, real = [], ops.add_rmsnorm_sums
+    monkeypatch.setattr(ops, "add_rmsnorm_sums", lambda *a: calls.append(1) or real(*a))
+    caches = lambda: [t.clone() for b in model.layers for t in (b.attention.kv_cache.k_cache, b.attention.kv_cache.v_cache)]
+    with torch.no_grad():
+        got, kept = generate.extend(model, ids, 0, pads), caches()
+        assert len(calls) == 5
+        watched = [b.attention.wo.register_forward_hook(lambda *a: None) for b in model.layers] + [model.norm.register_forward_hook(lambda *a: None)]
+        attended = [b.attention.register_forward_hook(lambda *a: None) for b in model.layers]
+        want = generate.extend(model, ids, 0, pads)
+        assert len(calls) == 5
+    for hook in watched + attended:
+        hook.remove()
+    rel = lambda a, b: ((a.double() - b.double()).norm() / b.double().norm()).item()
+    assert rel(got, want) < 1e-2 and all(rel(a, b) < 1e-2 for a, b in zip(kept, caches()))  # slices in another order: single bfloat16 roundings, which travel on
