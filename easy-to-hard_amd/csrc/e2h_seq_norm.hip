@@ -404,6 +404,28 @@ __global__ __launch_bounds__(256) void gelu_gate_rows_kernel(const T *__restrict
   y[i] = from_f32<T>(g * e);
 }
 
+// Rows of a 16-bit embedding as float32 values, where the residual stream starts, and (h not null) as they are; eight values per thread.  Bound by memory: 8192 x 4096 (201 MB, 268 with
+// h), or in a decode step by the launch, one where a gather and a conversion were two.  A token that the table does not have becomes a row that is no number.
+__global__ __launch_bounds__(256) void embed_rows_kernel(const bf16_t *__restrict__ table, const int64_t *__restrict__ tokens, float *__restrict__ x, bf16_t *__restrict__ h, int64_t pieces,
+                                                         int per_row, int64_t vocab) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= pieces) return;
+  const int64_t row = i / per_row, token = tokens[row];
+  u32x4_t v = {0x7FC07FC0u, 0x7FC07FC0u, 0x7FC07FC0u, 0x7FC07FC0u};
+  if (token >= 0 && token < vocab) v = reinterpret_cast<const u32x4_t *>(table)[token * per_row + (i - row * per_row)];
+  f32x4_t lo, hi;
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    lo[2 * e] = __builtin_bit_cast(float, v[e] << 16);
+    lo[2 * e + 1] = __builtin_bit_cast(float, v[e] & 0xFFFF0000u);
+    hi[2 * e] = __builtin_bit_cast(float, v[2 + e] << 16);
+    hi[2 * e + 1] = __builtin_bit_cast(float, v[2 + e] & 0xFFFF0000u);
+  }
+  store4(x + 8 * i, lo);
+  store4(x + 8 * i + 4, hi);
+  if (h) reinterpret_cast<u32x4_t *>(h)[i] = v;
+}
+
 }  // namespace
 }  // namespace e2h
 
@@ -495,5 +517,16 @@ extern "C" int e2h_seq_gelu_gate_rows(int dtype, const void *gate, const void *t
   else
     hipLaunchKernelGGL(gelu_gate_rows_kernel<float>, grid, block, 0, s, static_cast<const float *>(gate), static_cast<const float *>(table), tokens,
                        static_cast<float *>(y), n, static_cast<int>(dim), ld, column, table_rows);
+  return launch_status();
+}
+
+extern "C" int e2h_seq_embed_rows(const void *table, const int64_t *tokens, float *x, void *h, int64_t rows, int64_t width, int64_t table_rows, void *stream) {
+  if (!table || !tokens || !x) return E2H_ERR_NULL_POINTER;
+  if (rows < 1 || width < 8 || width % 8 != 0 || width > INT32_MAX || table_rows < 1) return E2H_ERR_BAD_SHAPE;
+  const int64_t pieces = rows * (width / 8), blocks = (pieces + 255) / 256;
+  if (blocks > INT32_MAX / 256) return E2H_ERR_BAD_SHAPE;
+  if (!aligned16(table) || !aligned16(x) || !aligned16(h) || (reinterpret_cast<uintptr_t>(tokens) & 7u)) return E2H_ERR_MISALIGNED;
+  hipLaunchKernelGGL(embed_rows_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<const bf16_t *>(table), tokens, x,
+                     static_cast<bf16_t *>(h), pieces, static_cast<int>(width / 8), table_rows);
   return launch_status();
 }

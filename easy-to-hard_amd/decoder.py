@@ -15,6 +15,17 @@ from .linear import DecodeLinear, fusable, unwatched
 from .state import SequenceState, StatePlan, rotary_turns
 
 
+def embedded(emb: nn.Module, tokens: Tensor, want_rows: bool = True):
+    """emb(tokens) in float32, where the residual stream starts, and (want_rows) as it is; tokens int64 [rows]."""
+    w = emb.weight
+    if (not torch.compiler.is_compiling() and type(emb) is nn.Embedding and emb.max_norm is None and w.dtype == torch.bfloat16 and w.is_cuda and w.device == tokens.device and tokens.numel() > 0 and w.is_contiguous()
+            and tokens.is_contiguous() and w.shape[1] % 8 == 0 and w.data_ptr() % 16 == 0 and not (w.requires_grad and torch.is_grad_enabled())
+            and unwatched(emb) and not seq_ops.watched(w, tokens)):
+        return seq_ops.embed_rows(w, tokens, want_rows)
+    h = emb(tokens)
+    return h.float(), h
+
+
 class StatefulDecoder(nn.Module):
     returns_greedy_token = True  # forward(..., greedy_token=True) yields the token itself
     logit_softcap: Optional[float] = None

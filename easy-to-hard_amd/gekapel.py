@@ -16,7 +16,7 @@ import torch
 import torch.nn as nn
 
 from . import seq_ops
-from .decoder import StatefulDecoder
+from .decoder import StatefulDecoder, embedded
 from .feed_forward import ExpertMixture
 from .linear import DecodeLinear
 from .mixers import TokenMixer, WindowAttention
@@ -122,8 +122,7 @@ class Gekapel(StatefulDecoder):
 
     def _hidden(self, idx, bsz, seqlen, state, input_pos, first):
         dtype, eps = self.dtype, self.config.norm_eps
-        h = self.tok_embeddings(idx.view(-1))
-        x = h.float()
+        x, h = embedded(self.tok_embeddings, idx.view(-1))
         rotary = self.rotary_tables(bsz, seqlen, input_pos, first)
         pending = {}  # the sublayer output that has not been added to x yet, with its norm
 

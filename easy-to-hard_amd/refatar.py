@@ -16,7 +16,7 @@ import torch
 import torch.nn as nn
 
 from . import seq_ops
-from .decoder import StatefulDecoder
+from .decoder import StatefulDecoder, embedded
 from .feed_forward import SquaredReluFF
 from .linear import DecodeLinear
 from .mixers import GatedDelta, HGRN2, TokenMixer, WindowAttention
@@ -157,7 +157,7 @@ class Refatar(StatefulDecoder):
         """Normalised output of the last layer, [B, S, dim] in the model's dtype."""
         dtype, eps = self.dtype, self.config.norm_eps
         tokens = idx.view(-1)
-        x = self.tok_embeddings(tokens).float()
+        x, _ = embedded(self.tok_embeddings, tokens, want_rows=False)
         delta = None  # the sublayer output that has not been added to x yet, with its norm's weight and offset
 
         def norm(x, delta, weight=None, conv=None, ring=None, want_out=True):

@@ -199,6 +199,18 @@ def linear_rows(x, weight, act, cap=0.0):
     return y
 
 
+def embed_rows(table, tokens, want_rows=True):
+    """table[tokens] as float32 and (want_rows) as it is, in one launch; table bfloat16 [vocab, width], tokens int64 [rows] -> (x [rows, width], h or None)."""
+    _need_gpu(table, tokens)
+    if table.dtype != torch.bfloat16 or tokens.dtype != torch.int64 or not (table.is_contiguous() and tokens.is_contiguous()):
+        raise TypeError("embed_rows: a contiguous bfloat16 table and int64 tokens expected")
+    rows, width = tokens.numel(), table.shape[1]
+    x = torch.empty((rows, width), dtype=torch.float32, device=table.device)
+    h = torch.empty((rows, width), dtype=table.dtype, device=table.device) if want_rows else None
+    _lib.check_seq(_lib_for(table).e2h_seq_embed_rows(_p(table), _p(tokens), _p(x), _p(h), rows, width, table.shape[0], _stream(table)), "e2h_seq_embed_rows")
+    return x, h
+
+
 def gelu_gate_rows(gate, table, tokens, column):
     """gelu_tanh(gate) * table[tokens, column : column + dim]; gate [rows, dim], tokens int64 [rows]."""
     _need_gpu(gate, table, tokens)

@@ -95,6 +95,9 @@ int e2h_seq_square_relu(int dtype, const void *x, void *y, int64_t n, void *stre
 int e2h_seq_softcap(int dtype, const void *x, void *y, int64_t n, float cap, void *stream);
 int e2h_seq_gelu_gate_rows(int dtype, const void *gate, const void *table, const int64_t *tokens, void *y, int64_t rows, int64_t dim,
                            int64_t ld, int64_t column, int64_t table_rows, void *stream);
+/* embed_rows: x[r, i] = table[tokens[r], i] as float32 and, unless h is NULL, h[r, i] as it is; bfloat16 table [table_rows, width], width % 8 == 0, everything but tokens 16-byte
+ * aligned.  Rows of tokens outside the table are no numbers. */
+int e2h_seq_embed_rows(const void *table, const int64_t *tokens, float *x, void *h, int64_t rows, int64_t width, int64_t table_rows, void *stream);
 
 /* table[row, i] = (cos, sin) of the turn fraction of position * turns[i], i < pairs: turns[i] is the rotation per position in whole
  * turns (angle / 2 pi), positions count from the sequence's first one.  table is float32 [batch * seqlen, pairs, 2]. */

@@ -622,3 +622,26 @@ def test_scoring_with_a_reward_head(tmp_path):
     got = generate.model_score(model, toks[None].to(DEV))[0].cpu().numpy()
     weights = {**{n: t.float().numpy() for n, t in w.items()}, "head": head.numpy()}
     assert rel(got, go.forward(cfg, weights, toks.numpy())[0].mean(-1)) < 1e-4
+
+
+# ---- the start of the residual stream ------------------------------------------------------------------------------------------------
+
+@pytest.mark.parametrize("rows,width", [(1, 8), (3, 264), (700, 4096), (33, 2056)])
+def test_embedded_rows_are_the_embedding_and_its_float32_values(rows, width):
+    from easy_to_hard_amd.decoder import embedded
+
+    gen = torch.Generator().manual_seed(rows)
+    emb = torch.nn.Embedding(50, width, dtype=torch.bfloat16, device=DEV).requires_grad_(False)
+    tokens = torch.randint(0, 50, (rows,), generator=gen).to(DEV)
+    want = emb.weight[tokens]
+    x, h = embedded(emb, tokens)
+    assert x.dtype == torch.float32 and torch.equal(x, want.float()) and torch.equal(h, want)
+    x, h = embedded(emb, tokens, want_rows=False)
+    assert torch.equal(x, want.float()) and h is None
+    seen = []
+    handle = emb.register_forward_hook(lambda *_: seen.append(1))
+    x, h = embedded(emb, tokens, want_rows=False)  # somebody watches the module: its own call
+    handle.remove()
+    assert seen == [1] and torch.equal(x, want.float()) and torch.equal(h, want)
+    x, h = seq_ops.embed_rows(emb.weight, torch.tensor([0, 50, -1], device=DEV))
+    assert torch.equal(h[0], emb.weight[0]) and x[1:].isnan().all() and h[1:].isnan().all()
