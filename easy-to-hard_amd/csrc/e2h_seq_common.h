@@ -80,9 +80,10 @@ __device__ __forceinline__ float decayed(Decay d, float s) { return __builtin_fm
 __device__ __forceinline__ float sigmoid_f32(float z) { return 1.0f / (1.0f + expf(-z)); }
 __device__ __forceinline__ float silu_f32(float z) { return z / (1.0f + expf(-z)); }
 __device__ __forceinline__ float softplus_f32(float z) { return fmaxf(z, 0.0f) + log1pf(expf(-fabsf(z))); }
+// gelu of z by tanh
+__device__ __forceinline__ float gelu_tanh_f32(float z) { return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))); }
 
-
-// The same on the hardware's exponential and reciprocal (a few units in the last place), for kernels that evaluate them per
+// Sigmoid and silu on the hardware's exponential and reciprocal (a few units in the last place), for kernels that evaluate them per
 // token and channel of a prompt
 __device__ __forceinline__ float fast_sigmoid(float z) { return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-z * kLog2e)); }
 __device__ __forceinline__ float fast_silu(float z) { return z * fast_sigmoid(z); }

@@ -39,6 +39,34 @@ struct Linear {
   }
 };
 
+// gelu(bf16(acc)) * table[tokens[row], column + n], as e2h_seq_gelu_gate_rows forms it from the linear's output.  In a step of two layers at 32 rows the two launches of that cost
+// 2.7 us; with the rows asked for in `finish`, tokens first, half of it was lost again.
+struct GeluGate {
+  static constexpr bool kGate = false, kHalves = false;
+  struct Args {
+    bf16_t *y;
+    const bf16_t *table;
+    const int64_t *tokens;
+    int64_t ld, column, table_rows;
+  };
+  bf16_t row[4];  // of the table: on their way under the product
+  bool there[4];
+  __device__ __forceinline__ void load(const Args &, int, int) {}
+  __device__ __forceinline__ void load_rows(const Args &a, int m0, int M, int n, int N) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t token = a.tokens[m0 + r < M ? m0 + r : M - 1];
+      there[r] = token >= 0 && token < a.table_rows && n < N;
+      row[r] = a.table[there[r] ? token * a.ld + a.column + n : a.column];
+    }
+  }
+  __device__ __forceinline__ void finish(const Args &a, f32x4_t acc, f32x4_t, int m0, int M, int n, int N) const {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (n < N && m0 + r < M) a.y[static_cast<size_t>(m0 + r) * N + n] = from_f32<bf16_t>(gelu_tanh_f32(to_f32(from_f32<bf16_t>(acc[r]))) * (there[r] ? to_f32(row[r]) : 0.f));
+  }
+};
+
 // float32 sums of a K slice, [slices][M][N]
 struct Slice {
   static constexpr bool kGate = false, kHalves = false;
@@ -213,4 +241,13 @@ extern "C" int e2h_seq_linear(const void *x, const void *w, void *y, int64_t row
   if (act == kSquare) return run_linear<kSquare>(a, out, 0.f, f, s);
   if (act == kCap) return run_linear<kCap>(a, out, cap, f, s);
   return run_linear<kNone>(a, out, 0.f, f, s);
+}
+
+extern "C" int e2h_seq_linear_gelu_gate(const void *x, const void *w, const void *table, const int64_t *tokens, void *y, int64_t rows, int64_t n, int64_t k, int64_t ld, int64_t column,
+                                        int64_t table_rows, void *stream) {
+  if (!x || !w || !table || !tokens || !y) return E2H_ERR_NULL_POINTER;
+  if (!stream::takes(rows, n, k, 2) || sliced(rows, n, k) || column < 0 || column + n > ld || table_rows < 1) return E2H_ERR_BAD_SHAPE;
+  if (!aligned16(x) || !aligned16(w) || (reinterpret_cast<uintptr_t>(y) & 1u) || (reinterpret_cast<uintptr_t>(table) & 1u) || (reinterpret_cast<uintptr_t>(tokens) & 7u)) return E2H_ERR_MISALIGNED;
+  const stream::Args a{static_cast<const uint16_t *>(x), w, w, static_cast<int>(rows), static_cast<int>(n), static_cast<int>(k)};
+  return stream::run<stream::Bf16Weights, GeluGate>(a, {static_cast<bf16_t *>(y), static_cast<const bf16_t *>(table), tokens, ld, column, table_rows}, static_cast<hipStream_t>(stream));
 }

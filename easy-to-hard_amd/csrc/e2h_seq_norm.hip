@@ -400,8 +400,7 @@ __global__ __launch_bounds__(256) void gelu_gate_rows_kernel(const T *__restrict
   const int64_t tok = tokens[r];
   const float z = to_f32(gate[i]);
   const float e = tok >= 0 && tok < table_rows ? to_f32(table[tok * ld + column + c]) : 0.f;
-  const float g = 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-  y[i] = from_f32<T>(g * e);
+  y[i] = from_f32<T>(gelu_tanh_f32(z) * e);
 }
 
 // Rows of a 16-bit embedding as float32 values, where the residual stream starts, and (h not null) as they are; eight values per thread.  Bound by memory: 8192 x 4096 (201 MB, 268 with

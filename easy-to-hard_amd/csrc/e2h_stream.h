@@ -169,6 +169,12 @@ struct NormLoads {
   }
 };
 
+// whether an epilogue asks for something by its rows, too: load_rows(args, first row, M, column, N)
+template <typename Epi, typename = void>
+struct WantsRows : std::false_type {};
+template <typename Epi>
+struct WantsRows<Epi, std::void_t<decltype(&Epi::load_rows)>> : std::true_type {};
+
 // Epi: struct with kGate (two matrices, T / 2 tiles of each), kHalves (acc and acc2 are the sums over the two halves of K), Args, and per
 // unit a state: load(args, n, N) issues what it needs early, finish(args, acc, acc2, m0, M, n, N) stores rows m0 .. m0 + 3 of column n.
 // XR: rows of x in a tile that can be present (8: M <= 8, one load per unit of x instead of two).
@@ -294,6 +300,9 @@ __global__ __launch_bounds__(64 * kWaves) void stream_mm_kernel(const Args a, co
   for (int i = 0; i < kPerWave; ++i) {
     const int u = wave + kWaves * i;
     if (u < kUnits) epi[i].load(ea, n0 + 16 * (u / MT) + c, a.N);
+    if constexpr (WantsRows<Epi>::value) {
+      if (u < kUnits) epi[i].load_rows(ea, 16 * (u % MT) + 4 * b, a.M, n0 + 16 * (u / MT) + c, a.N);
+    }
   }
   __builtin_amdgcn_sched_barrier(0);
   uint32_t at = 0;

@@ -18,7 +18,7 @@ import torch.nn as nn
 from . import seq_ops
 from .decoder import StatefulDecoder, embedded
 from .feed_forward import SquaredReluFF
-from .linear import DecodeLinear
+from .linear import DecodeLinear, fusable
 from .mixers import GatedDelta, HGRN2, TokenMixer, WindowAttention
 from .state import StatePlan
 
@@ -173,8 +173,11 @@ class Refatar(StatefulDecoder):
                 x, h = norm(x, delta, layer.norm2, layer.canon2, layer.ring2)
                 delta = (layer.feed_forward(h), layer.norm2b, 1.0)
             x, h = norm(x, delta, want_out=dtype != torch.float32)
-            gate = layer.side_gate(x if h is None else h)
-            gate = seq_ops.gelu_gate_rows(gate, self.side_embeddings.weight, tokens, layer.side_column)
+            h, table = x if h is None else h, self.side_embeddings.weight
+            if not torch.compiler.is_compiling() and fusable(layer.side_gate, h) and not seq_ops.watched(table, tokens):
+                gate = seq_ops.linear_gelu_gate(h, layer.side_gate.weight, table, tokens, layer.side_column)
+            else:
+                gate = seq_ops.gelu_gate_rows(layer.side_gate(h), table, tokens, layer.side_column)
             delta = (layer.side_proj(gate), layer.side_norm, 0.0)
         state.commit(bsz, seqlen)
         d, dw, off = delta

@@ -225,6 +225,21 @@ def gelu_gate_rows(gate, table, tokens, column):
     return y
 
 
+def linear_gelu_gate(x, weight, table, tokens, column):
+    """gelu_gate_rows(linear(x, weight), table, tokens, column) of a decode batch, in one launch where there is one for the sizes."""
+    _need_gpu(x, weight, table, tokens)
+    n, k = weight.shape
+    rows = x.numel() // k
+    fits = (weight.is_contiguous() and x.is_contiguous() and not (weight.data_ptr() | x.data_ptr()) % 16 and x.dtype == weight.dtype == table.dtype == torch.bfloat16 and table.dim() == 2
+            and table.is_contiguous() and tokens.dtype == torch.int64 and tokens.numel() == rows and tokens.is_contiguous() and column + n <= table.shape[1])
+    if not fits or _lib.load_seq().e2h_seq_linear_scratch_bytes(rows, n, k) != 0:
+        return gelu_gate_rows(linear(x, weight), table, tokens, column)
+    y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
+    _lib.check_seq(_lib_for(x).e2h_seq_linear_gelu_gate(_p(x), _p(weight), _p(table), _p(tokens), _p(y), rows, n, k, table.shape[1], column, table.shape[0], _stream(x)),
+                   "e2h_seq_linear_gelu_gate")
+    return y
+
+
 def rotary_table(turns, input_pos, first, batch, seqlen):
     """(cos, sin) of position * turns for every row and rotated pair, float32 [batch * seqlen, pairs, 2]; turns float64 [pairs]
     in whole turns per position."""

@@ -84,6 +84,10 @@ int64_t e2h_seq_linear_scratch_bytes(int64_t rows, int64_t n, int64_t k);
 int e2h_seq_linear(const void *x, const void *w, void *y, int64_t rows, int64_t n, int64_t k, int act, float cap, void *scratch,
                    int64_t scratch_bytes, void *stream);
 
+/* e2h_seq_linear and e2h_seq_gelu_gate_rows (below) on its result in one launch, bit for bit; E2H_ERR_BAD_SHAPE where e2h_seq_linear_scratch_bytes is not 0. */
+int e2h_seq_linear_gelu_gate(const void *x, const void *w, const void *table, const int64_t *tokens, void *y, int64_t rows, int64_t n, int64_t k, int64_t ld, int64_t column,
+                             int64_t table_rows, void *stream);
+
 /* The same over many rows (a soft cap between 2^-6 and 2^10): n a multiple of 8, k of 64 and at least 192, x, w and 256 rows of y below 4 GB, all three 16-byte
  * aligned; no scratch.  e2h_seq_linear_rows_pays: 1 where that is expected to take less time than a library product followed by e2h_seq_square_relu or e2h_seq_softcap, else 0. */
 int e2h_seq_linear_rows_pays(int64_t rows, int64_t n, int64_t k, int act, float cap);

@@ -860,3 +860,19 @@ def test_feed_forward_of_many_rows_takes_one_launch_for_up_and_its_activation():
     assert not seq_ops.linear_rows_pay(h, up, 1)
     with torch.no_grad():
         assert seq_ops.linear_rows_pay(h, up, 1)
+
+
+# ---- the token side's gate in the launch of its product --------------------------------------------------------------------------------
+
+@pytest.mark.parametrize("rows,n,k,column", [(1, 256, 4096, 256), (17, 64, 2048, 0), (64, 40, 128, 24), (33, 8, 4096, 3)])
+def test_linear_with_the_token_gate_is_the_two_calls(rows, n, k, column):
+    gen = torch.Generator().manual_seed(rows)
+    x, w = (torch.randn(shape, generator=gen).to(torch.bfloat16).to(DEV) for shape in ((rows, k), (n, k)))
+    w *= k ** -0.5
+    table, tokens = torch.randn((50, column + n + 5), generator=gen).to(torch.bfloat16).to(DEV), torch.randint(-1, 51, (rows,), generator=gen).to(DEV)
+    want = seq_ops.gelu_gate_rows(seq_ops.linear(x, w), table, tokens, column)
+    assert torch.equal(seq_ops.linear_gelu_gate(x, w, table, tokens, column), want)
+    wide = torch.randn((32, 8192), generator=gen).to(torch.bfloat16).to(DEV)  # a product in slices of K
+    narrow = (torch.randn((n, 8192), generator=gen) / 90).to(torch.bfloat16).to(DEV)
+    some = torch.randint(0, 50, (32,), generator=gen).to(DEV)
+    assert torch.equal(seq_ops.linear_gelu_gate(wide, narrow, table, some, column), seq_ops.gelu_gate_rows(seq_ops.linear(wide, narrow), table, some, column))
