@@ -152,6 +152,8 @@ _SEQ_SIGNATURES = {
     "e2h_seq_gelu_gate_rows": (c_int, [c_int, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, _P]),
     "e2h_seq_embed_rows": (c_int, [_P, _P, _P, _P, c_int64, c_int64, c_int64, _P]),
     "e2h_seq_linear_gelu_gate": (c_int, [_P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, _P]),
+    "e2h_seq_norm_conv_sums": (c_int, [_A(NormConvArgs), _P, c_int, _P]),
+    "e2h_seq_linear_sums": (c_int, [_P, _P, _P, c_int64, c_int64, c_int64, _P]),
     "e2h_seq_linear_scratch_bytes": (c_int64, [c_int64, c_int64, c_int64]),
     "e2h_seq_linear": (c_int, [_P, _P, _P, c_int64, c_int64, c_int64, c_int, c_float, _P, c_int64, _P]),
     "e2h_seq_linear_rows_pays": (c_int, [c_int64, c_int64, c_int64, c_int, c_float]),

@@ -251,3 +251,11 @@ extern "C" int e2h_seq_linear_gelu_gate(const void *x, const void *w, const void
   const stream::Args a{static_cast<const uint16_t *>(x), w, w, static_cast<int>(rows), static_cast<int>(n), static_cast<int>(k)};
   return stream::run<stream::Bf16Weights, GeluGate>(a, {static_cast<bf16_t *>(y), static_cast<const bf16_t *>(table), tokens, ld, column, table_rows}, static_cast<hipStream_t>(stream));
 }
+
+extern "C" int e2h_seq_linear_sums(const void *x, const void *w, float *sums, int64_t rows, int64_t n, int64_t k, void *stream) {
+  if (!x || !w || !sums) return E2H_ERR_NULL_POINTER;
+  if (!stream::takes(rows, n, k, 2) || !sliced(rows, n, k)) return E2H_ERR_BAD_SHAPE;
+  if (!aligned16(x) || !aligned16(w) || !aligned16(sums)) return E2H_ERR_MISALIGNED;
+  const stream::Args a{static_cast<const uint16_t *>(x), w, w, static_cast<int>(rows), static_cast<int>(n), static_cast<int>(k)};
+  return stream::run<stream::Bf16Weights, Slice>(a, {sums}, static_cast<hipStream_t>(stream), kSlices);
+}

@@ -34,6 +34,13 @@ __device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t row, int at,
 }
 #endif
 
+// delta as the float32 sums of K slices [slices][rows][width] that its linear left (e2h_seq_linear_sums): rounded as the linear's own output.  The launch that adds them costs a step of 32
+// rows more than the norm, which waits for its row anyway, takes longer for reading four times as much.  Not with runs, whose rows are asked for ahead.
+struct DeltaSums {
+  const float *from;
+  int slices;
+};
+
 // One row per workgroup, or with a convolution (which needs its previous inputs) a run of `run` consecutive tokens of one sequence.  A thread owns NP pieces of four channels, so the
 // convolution's previous inputs stay in its registers from token to token; the taps - 1 tokens ahead of the run are normalised again by the
 // workgroup (inside the call) or come from the ring of kept inputs (before the call).  TAPS is the compiled depth of the
@@ -46,7 +53,7 @@ __device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t row, int at,
 // us at 4096 channels, in brackets runs of 8 (convolution: 1024 threads, two rows together) that waited for every row: 8192 rows with residual 58 (94), layer norm 63 (91), eight experts'
 // terms 161 (187), convolution 73 (101); 8000 rows 56 (85), 62 (106), 159 (214), 66 (167: one workgroup too many for a round); 2048 rows 17 (18), 20 (21), 39 (38), 25 (33).
 template <typename T, int BLOCK, int NP, int TAPS, bool LAYER, bool TERMS, bool AHEAD>
-__global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_args a, int runs, int run, int streamed) {
+__global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_args a, const DeltaSums sums, int runs, int run, int streamed) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int kWaves = BLOCK / 64;
   constexpr int RING = TAPS > 1 ? TAPS - 1 : 1;
@@ -182,6 +189,25 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
       h[p] = raw.h[p];
       d[p] = raw.d[p].f32();
     }
+    const bool summed = !AHEAD && !TERMS && !LAYER && sums.from;
+    if (summed) {
+      constexpr int kMost = 4;
+      f32x4_t part[kMost][NP];
+      const size_t slice = static_cast<size_t>(a.batch) * seqlen * W;
+#pragma unroll
+      for (int k = 0; k < kMost; ++k) {
+        const __amdgpu_buffer_rsrc_t r = make_rsrc(sums.from + (k < sums.slices ? k : 0) * slice + (row0 + t) * W, k < sums.slices ? row_f32 : 0);
+#pragma unroll
+        for (int p = 0; p < NP; ++p) part[k][p] = buffer_quad<float>(r, piece(p)).raw;
+      }
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+#pragma unroll
+        for (int k = 1; k < kMost; ++k) part[0][p] += part[k][p];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d[p][e] = to_f32(from_f32<T>(part[0][p][e]));
+      }
+    }
     if constexpr (TERMS) {
       const int n = static_cast<int>(a.n_terms);
       const float *tw = a.term_weights + (row0 + t) * n;
@@ -208,7 +234,7 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
         }
       }
     }
-    if (a.delta || TERMS) {
+    if (a.delta || TERMS || summed) {
       if constexpr (LAYER) {
         layer_norm(d, wd, bd);
 #pragma unroll
@@ -313,42 +339,42 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
 }
 
 template <typename T, int BLOCK, int NP, int TAPS, bool LAYER, bool TERMS>
-void launch_norm_conv_rows(const e2h_norm_conv_args &a, int runs, int run, hipStream_t s) {
+void launch_norm_conv_rows(const e2h_norm_conv_args &a, const DeltaSums &sums, int runs, int run, hipStream_t s) {
   const int64_t workgroups = TAPS ? a.batch * runs : a.batch * a.seqlen < (1 << 20) ? a.batch * a.seqlen : 1 << 20;
   const dim3 grid(static_cast<unsigned>(workgroups)), block(BLOCK);
   // from 21 million values on (x, the new x and two 16-bit operands are 12 bytes each) they do not stay in 256 MB of cache anyway; 4096 x 4096 takes as long with either store
   const int streamed = a.batch * a.seqlen * a.width >= (int64_t{1} << 28) / 12;
   if constexpr (TAPS > 0) {
     if (run > 1) {
-      hipLaunchKernelGGL((norm_conv_kernel<T, BLOCK, NP, TAPS, LAYER, TERMS, true>), grid, block, 0, s, a, runs, run, streamed);
+      hipLaunchKernelGGL((norm_conv_kernel<T, BLOCK, NP, TAPS, LAYER, TERMS, true>), grid, block, 0, s, a, sums, runs, run, streamed);
       return;
     }
   }
-  hipLaunchKernelGGL((norm_conv_kernel<T, BLOCK, NP, TAPS, LAYER, TERMS, false>), grid, block, 0, s, a, runs, run, streamed);
+  hipLaunchKernelGGL((norm_conv_kernel<T, BLOCK, NP, TAPS, LAYER, TERMS, false>), grid, block, 0, s, a, sums, runs, run, streamed);
 }
 
 template <typename T, int BLOCK, int NP>
-void launch_norm_conv_taps(const e2h_norm_conv_args &a, int runs, int run, hipStream_t s) {
+void launch_norm_conv_taps(const e2h_norm_conv_args &a, const DeltaSums &sums, int runs, int run, hipStream_t s) {
   if (a.norm_kind == E2H_SEQ_LAYER_NORM) {
-    if (a.terms) return launch_norm_conv_rows<T, BLOCK, NP, 0, true, true>(a, runs, run, s);
-    return launch_norm_conv_rows<T, BLOCK, NP, 0, true, false>(a, runs, run, s);
+    if (a.terms) return launch_norm_conv_rows<T, BLOCK, NP, 0, true, true>(a, sums, runs, run, s);
+    return launch_norm_conv_rows<T, BLOCK, NP, 0, true, false>(a, sums, runs, run, s);
   }
-  if (a.terms) return launch_norm_conv_rows<T, BLOCK, NP, 0, false, true>(a, runs, run, s);
-  if (!a.conv) return launch_norm_conv_rows<T, BLOCK, NP, 0, false, false>(a, runs, run, s);
-  if (a.taps <= 4) launch_norm_conv_rows<T, BLOCK, NP, 4, false, false>(a, runs, run, s);
-  else launch_norm_conv_rows<T, BLOCK, NP, 8, false, false>(a, runs, run, s);
+  if (a.terms) return launch_norm_conv_rows<T, BLOCK, NP, 0, false, true>(a, sums, runs, run, s);
+  if (!a.conv) return launch_norm_conv_rows<T, BLOCK, NP, 0, false, false>(a, sums, runs, run, s);
+  if (a.taps <= 4) launch_norm_conv_rows<T, BLOCK, NP, 4, false, false>(a, sums, runs, run, s);
+  else launch_norm_conv_rows<T, BLOCK, NP, 8, false, false>(a, sums, runs, run, s);
 }
 
 template <typename T>
-void launch_norm_conv(const e2h_norm_conv_args &a, int runs, int run, hipStream_t s) {
-  if (a.width <= 1024) launch_norm_conv_taps<T, 256, 1>(a, runs, run, s);
+void launch_norm_conv(const e2h_norm_conv_args &a, const DeltaSums &sums, int runs, int run, hipStream_t s) {
+  if (a.width <= 1024) launch_norm_conv_taps<T, 256, 1>(a, sums, runs, run, s);
   // eight values per thread where many rows are waiting: half the waves, which repeat a row's sums each (8192 x 2048, layer norm 31 us, 38 with four values; final norm 24, 31)
-  else if (a.width <= 2048 && !a.conv && a.batch * a.seqlen > 256) launch_norm_conv_taps<T, 256, 2>(a, runs, run, s);
-  else if (a.width <= 2048) launch_norm_conv_taps<T, 512, 1>(a, runs, run, s);
-  else if (a.width <= 4096 && a.conv && run == 1) launch_norm_conv_taps<T, 1024, 1>(a, runs, run, s);
-  else if (a.width <= 4096) launch_norm_conv_taps<T, 512, 2>(a, runs, run, s);
-  else if (a.width <= 8192) launch_norm_conv_taps<T, 512, 4>(a, runs, run, s);
-  else launch_norm_conv_taps<T, 1024, 4>(a, runs, run, s);
+  else if (a.width <= 2048 && !a.conv && a.batch * a.seqlen > 256) launch_norm_conv_taps<T, 256, 2>(a, sums, runs, run, s);
+  else if (a.width <= 2048) launch_norm_conv_taps<T, 512, 1>(a, sums, runs, run, s);
+  else if (a.width <= 4096 && a.conv && run == 1) launch_norm_conv_taps<T, 1024, 1>(a, sums, runs, run, s);
+  else if (a.width <= 4096) launch_norm_conv_taps<T, 512, 2>(a, sums, runs, run, s);
+  else if (a.width <= 8192) launch_norm_conv_taps<T, 512, 4>(a, sums, runs, run, s);
+  else launch_norm_conv_taps<T, 1024, 4>(a, sums, runs, run, s);
 }
 
 // ---- elementwise -----------------------------------------------------------------------------------------------------
@@ -459,8 +485,9 @@ extern "C" int e2h_seq_set_option(const char *name, int value) {
   return E2H_OK;
 }
 
-extern "C" int e2h_seq_norm_conv(const e2h_norm_conv_args *a, void *stream) {
-  if (!a || !a->x || ((a->delta || a->terms) && !a->delta_weight) || (a->terms && !a->term_weights)) return E2H_ERR_NULL_POINTER;
+namespace {
+int norm_conv(const e2h_norm_conv_args *a, const DeltaSums &sums, void *stream) {
+  if (!a || !a->x || ((a->delta || a->terms || sums.from) && !a->delta_weight) || (a->terms && !a->term_weights)) return E2H_ERR_NULL_POINTER;
   if (!a->out && !a->x_out) return E2H_ERR_NULL_POINTER;
   if (a->conv && (!a->input_pos || (a->taps > 1 && (!a->tail_in || !a->tail_out)))) return E2H_ERR_NULL_POINTER;
   if (a->batch < 1 || a->seqlen < 1 || a->width < 4 || a->width % 4 != 0 || a->width > 16384 || a->seqlen > INT32_MAX / 4)
@@ -487,9 +514,19 @@ extern "C" int e2h_seq_norm_conv(const e2h_norm_conv_args *a, void *stream) {
   const int64_t runs = (a->seqlen + run - 1) / run;
   if (a->batch * runs > INT32_MAX) return E2H_ERR_BAD_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (a->dtype == E2H_SEQ_BF16) launch_norm_conv<bf16_t>(*a, static_cast<int>(runs), run, s);
-  else launch_norm_conv<float>(*a, static_cast<int>(runs), run, s);
+  if (a->dtype == E2H_SEQ_BF16) launch_norm_conv<bf16_t>(*a, sums, static_cast<int>(runs), run, s);
+  else launch_norm_conv<float>(*a, sums, static_cast<int>(runs), run, s);
   return launch_status();
+}
+}  // namespace
+
+extern "C" int e2h_seq_norm_conv(const e2h_norm_conv_args *a, void *stream) { return norm_conv(a, DeltaSums{}, stream); }
+
+extern "C" int e2h_seq_norm_conv_sums(const e2h_norm_conv_args *a, const float *sums, int slices, void *stream) {
+  if (!a || !sums) return E2H_ERR_NULL_POINTER;
+  if (slices < 1 || slices > 4 || a->seqlen != 1 || a->delta || a->terms || a->norm_kind != E2H_SEQ_RMS_NORM) return E2H_ERR_BAD_SHAPE;
+  if (!aligned16(sums)) return E2H_ERR_MISALIGNED;
+  return norm_conv(a, DeltaSums{sums, slices}, stream);
 }
 
 extern "C" int e2h_seq_square_relu(int dtype, const void *x, void *y, int64_t n, void *stream) {

@@ -16,9 +16,12 @@ class SquaredReluFF(nn.Module):
         self.up = DecodeLinear(width, hidden, bias=False)
         self.down = DecodeLinear(hidden, width, bias=False)
 
-    def forward(self, h: Tensor) -> Tensor:
+    def forward(self, h: Tensor, defer: bool = False) -> Tensor:
+        """defer (a step whose next norm is seq_ops.norm_conv's): the result may come as float32 sums over slices of K, for that to add."""
         if fusable(self.up, h):
-            return self.down(seq_ops.linear(h, self.up.weight, seq_ops.ACT_SQUARE_RELU))
+            y = seq_ops.linear(h, self.up.weight, seq_ops.ACT_SQUARE_RELU)
+            sums = seq_ops.linear_sums(y, self.down.weight) if defer and fusable(self.down, y) else None
+            return self.down(y) if sums is None else sums
         if type(self.up) is DecodeLinear and self.up.bias is None and unwatched(self.up) and seq_ops.linear_rows_pay(h, self.up.weight, seq_ops.ACT_SQUARE_RELU):
             return self.down(seq_ops.linear_rows(h, self.up.weight, seq_ops.ACT_SQUARE_RELU))
         return self.down(seq_ops.square_relu_(self.up(h)))

@@ -18,7 +18,7 @@ import torch.nn as nn
 from . import seq_ops
 from .decoder import StatefulDecoder, embedded
 from .feed_forward import SquaredReluFF
-from .linear import DecodeLinear, fusable
+from .linear import DecodeLinear, fusable, unwatched
 from .mixers import GatedDelta, HGRN2, TokenMixer, WindowAttention
 from .state import StatePlan
 
@@ -171,7 +171,9 @@ class Refatar(StatefulDecoder):
             delta = (layer.mixer(h, bsz, seqlen, state, input_pos, first), layer.norm1b, 1.0)
             if layer.feed_forward is not None:
                 x, h = norm(x, delta, layer.norm2, layer.canon2, layer.ring2)
-                delta = (layer.feed_forward(h), layer.norm2b, 1.0)
+                ff = layer.feed_forward
+                defer = seqlen == 1 and dtype == torch.bfloat16 and not torch.compiler.is_compiling() and type(ff) is SquaredReluFF and unwatched(ff)
+                delta = (ff(h, defer=True) if defer else ff(h), layer.norm2b, 1.0)
             x, h = norm(x, delta, want_out=dtype != torch.float32)
             h, table = x if h is None else h, self.side_embeddings.weight
             if not torch.compiler.is_compiling() and fusable(layer.side_gate, h) and not seq_ops.watched(table, tokens):

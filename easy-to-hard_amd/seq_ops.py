@@ -64,7 +64,7 @@ def norm_conv(x, batch, seqlen, eps, dtype, delta=None, delta_weight=None, delta
               term_weights=None):
     """x + norm(delta), its norm and the norm's convolution over time (each optional) in one pass; x float32 [rows, width],
     conv float32 [taps, width].  The norms are RMS norms, or with layer_norm layer norms with optional biases.  terms
-    [rows * n, width] with term_weights float32 [rows, n] add a weighted sum to delta (or stand for it).  Returns (x_out float32 or x itself when there is no delta, out in `dtype` or None)."""
+    [rows * n, width] with term_weights float32 [rows, n] add a weighted sum to delta (or stand for it).  For one token per sequence delta may be linear_sums' float32 [slices, rows, width].  Returns (x_out float32 or x itself when there is no delta, out in `dtype` or None)."""
     _need_gpu(x)
     width = x.shape[-1]
     if x.dtype != torch.float32:
@@ -72,8 +72,13 @@ def norm_conv(x, batch, seqlen, eps, dtype, delta=None, delta_weight=None, delta
     _rows(x, batch, seqlen, "norm_conv", width)
     a = _lib.NormConvArgs(dtype=_DTYPES[dtype], batch=batch, seqlen=seqlen, width=width, eps=eps, delta_offset=delta_offset, norm_offset=norm_offset,
                           x=_p(x), norm_kind=int(layer_norm))
-    x_out = x
-    if delta is not None:
+    x_out, sums = x, None
+    if delta is not None and delta.dim() == 3:
+        _need_gpu(delta)
+        if delta.dtype != torch.float32 or not delta.is_contiguous() or tuple(delta.shape[1:]) != (batch * seqlen, width):
+            raise TypeError(f"norm_conv: sums must be float32 [slices, {batch * seqlen}, {width}], got {delta.dtype} {tuple(delta.shape)}")
+        sums = delta
+    elif delta is not None:
         _need_gpu(delta)
         _rows(delta, batch, seqlen, "norm_conv delta", width)
         if delta.dtype != dtype:
@@ -102,7 +107,10 @@ def norm_conv(x, batch, seqlen, eps, dtype, delta=None, delta_weight=None, delta
             a.tail_in, a.tail_out = _p(tails[0]), _p(tails[1])
     out = torch.empty((batch * seqlen, width), dtype=dtype, device=x.device) if want_out else None
     a.out = _p(out)
-    _lib.check_seq(_lib_for(x).e2h_seq_norm_conv(ctypes.byref(a), _stream(x)), "e2h_seq_norm_conv")
+    if sums is not None:
+        _lib.check_seq(_lib_for(x).e2h_seq_norm_conv_sums(ctypes.byref(a), _p(sums), sums.shape[0], _stream(x)), "e2h_seq_norm_conv_sums")
+    else:
+        _lib.check_seq(_lib_for(x).e2h_seq_norm_conv(ctypes.byref(a), _stream(x)), "e2h_seq_norm_conv")
     return x_out, out
 
 
@@ -172,6 +180,18 @@ def linear(x, weight, act=ACT_NONE, cap=0.0):
     scratch = torch.empty((need,), dtype=torch.uint8, device=x.device) if need > 0 else None
     _lib.check_seq(lib.e2h_seq_linear(_p(x2d), _p(weight), _p(y), rows, n, k, act, cap, _p(scratch), need, _stream(x)), "e2h_seq_linear")
     return y
+
+
+def linear_sums(x, weight):
+    """linear(x, weight) as the float32 sums of its slices of K [slices, rows, n], which norm_conv adds, or None where it has none."""
+    _need_gpu(x, weight)
+    n, k = weight.shape
+    rows = x.numel() // k
+    if _lib.load_seq().e2h_seq_linear_scratch_bytes(rows, n, k) <= 0 or not (x.is_contiguous() and weight.is_contiguous()) or (x.data_ptr() | weight.data_ptr()) % 16:
+        return None
+    sums = torch.empty((4, rows, n), dtype=torch.float32, device=x.device)
+    _lib.check_seq(_lib_for(x).e2h_seq_linear_sums(_p(x), _p(weight), _p(sums), rows, n, k, _stream(x)), "e2h_seq_linear_sums")
+    return sums
 
 
 def linear_rows_pay(x, weight, act, cap=0.0):

@@ -72,6 +72,8 @@ typedef struct {
   int64_t n_terms;
 } e2h_norm_conv_args;
 int e2h_seq_norm_conv(const e2h_norm_conv_args *a, void *stream);
+/* The same for one token per sequence, RMS norms and no terms, with delta (NULL in a) the sum in order of `slices` (1 to 4) float32 parts [slices, rows, width], rounded to dtype. */
+int e2h_seq_norm_conv_sums(const e2h_norm_conv_args *a, const float *sums, int slices, void *stream);
 
 /* y = act(x w^T) for the few rows of a decode step: x [rows, k], w [n, k] (nn.Linear.weight), y [rows, n], all bfloat16 and contiguous,
  * x and w 16-byte aligned; 1 <= rows <= 64, k a multiple of 8.  Sums are float32; the sum is rounded to bfloat16 before the activation
@@ -83,6 +85,9 @@ int e2h_seq_norm_conv(const e2h_norm_conv_args *a, void *stream);
 int64_t e2h_seq_linear_scratch_bytes(int64_t rows, int64_t n, int64_t k);
 int e2h_seq_linear(const void *x, const void *w, void *y, int64_t rows, int64_t n, int64_t k, int act, float cap, void *scratch,
                    int64_t scratch_bytes, void *stream);
+
+/* The float32 sums of e2h_seq_linear's four slices of K, sums [4, rows, n], for e2h_seq_norm_conv_sums to add; E2H_ERR_BAD_SHAPE where e2h_seq_linear_scratch_bytes is 0. */
+int e2h_seq_linear_sums(const void *x, const void *w, float *sums, int64_t rows, int64_t n, int64_t k, void *stream);
 
 /* e2h_seq_linear and e2h_seq_gelu_gate_rows (below) on its result in one launch, bit for bit; E2H_ERR_BAD_SHAPE where e2h_seq_linear_scratch_bytes is not 0. */
 int e2h_seq_linear_gelu_gate(const void *x, const void *w, const void *table, const int64_t *tokens, void *y, int64_t rows, int64_t n, int64_t k, int64_t ld, int64_t column,

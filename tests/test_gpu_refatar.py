@@ -876,3 +876,22 @@ def test_linear_with_the_token_gate_is_the_two_calls(rows, n, k, column):
     narrow = (torch.randn((n, 8192), generator=gen) / 90).to(torch.bfloat16).to(DEV)
     some = torch.randint(0, 50, (32,), generator=gen).to(DEV)
     assert torch.equal(seq_ops.linear_gelu_gate(wide, narrow, table, some, column), seq_ops.gelu_gate_rows(seq_ops.linear(wide, narrow), table, some, column))
+
+
+@pytest.mark.parametrize("rows,n,k,taps", [(17, 4096, 8192, 4), (32, 2048, 16384, 0), (64, 1028, 8192, 3), (33, 8, 8192, 0)])
+def test_norm_that_adds_the_slices_of_a_product_equals_the_product_and_the_norm(rows, n, k, taps):
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x, y, w = torch.randn((rows, n), generator=g, device=DEV), torch.randn((rows, k), generator=g, device=DEV).bfloat16(), (torch.randn((n, k), generator=g, device=DEV) / 90).bfloat16()
+    wd, wn = (0.3 * torch.randn((2, n), generator=g, device=DEV)).unbind(0)
+    sums = seq_ops.linear_sums(y, w)
+    assert tuple(sums.shape) == (4, rows, n)
+    for second in (wn, None):
+        tails = [torch.ones((rows, taps, n), device=DEV) for _ in range(2)] if taps else [None, None]
+        run = lambda delta, tail: seq_ops.norm_conv(x, rows, 1, 1e-4, torch.bfloat16, delta=delta, delta_weight=wd, delta_offset=1.0, norm_weight=second, norm_offset=1.0,
+                                                    **(dict(conv=wd.repeat(taps, 1), tails=(tail, tail), input_pos=positions(5, 1)) if taps else {}))
+        for got, want in zip(run(sums, tails[0]), run(seq_ops.linear(y, w), tails[1])):
+            assert torch.equal(got, want)
+        assert not taps or torch.equal(tails[0], tails[1])
+    assert seq_ops.linear_sums(y[:16], w) is None
+    with pytest.raises(RuntimeError):
+        seq_ops.norm_conv(x, 1, rows, 1e-4, torch.bfloat16, delta=sums, delta_weight=wd)  # several tokens of a sequence
