@@ -397,15 +397,25 @@ __global__ __launch_bounds__(BLOCK) void rmsnorm_kernel(const uint16_t *__restri
   const float *pr = SRC == kSums ? psum + row * dim : nullptr;
   auto sum_slices = [&](const f32x4_t (&lo)[kMaxSlices], const f32x4_t (&hi)[kMaxSlices], u32x4_t cs, int i) {
     f32x4_t a = lo[0], b = hi[0];
-#pragma unroll
-    for (int u = 1; u < kMaxSlices; ++u)
-      if (u < slices) {
-        a += lo[u];
-        b += hi[u];
+    if (kMaxSlices == 4 && sums.out) {  // (4 or 8 slices of the many-row int4 matmul: in pairs, as the launch that adds them without a norm)
+      a = (lo[0] + lo[1]) + (lo[kMaxSlices - 2] + lo[kMaxSlices - 1]);
+      b = (hi[0] + hi[1]) + (hi[kMaxSlices - 2] + hi[kMaxSlices - 1]);
+      if (slices == 8 && i < dim) {
+        const auto at = [&](int s2, int half) { return *reinterpret_cast<const f32x4_t *>(pr + s2 * slice_floats + i + half); };
+        a += (at(4, 0) + at(5, 0)) + (at(6, 0) + at(7, 0));
+        b += (at(4, 4) + at(5, 4)) + (at(6, 4) + at(7, 4));
       }
-    for (int s2 = kMaxSlices; s2 < slices && i < dim; ++s2) {
-      a += *reinterpret_cast<const f32x4_t *>(pr + s2 * slice_floats + i);
-      b += *reinterpret_cast<const f32x4_t *>(pr + s2 * slice_floats + i + 4);
+    } else {
+#pragma unroll
+      for (int u = 1; u < kMaxSlices; ++u)
+        if (u < slices) {
+          a += lo[u];
+          b += hi[u];
+        }
+      for (int s2 = kMaxSlices; s2 < slices && i < dim; ++s2) {
+        a += *reinterpret_cast<const f32x4_t *>(pr + s2 * slice_floats + i);
+        b += *reinterpret_cast<const f32x4_t *>(pr + s2 * slice_floats + i + 4);
+      }
     }
     if (col_scales) {
 #pragma unroll
@@ -830,7 +840,7 @@ extern "C" int e2h_add_rmsnorm_sums(const uint16_t *x, const uint16_t *delta, co
                                     int64_t rows, int64_t dim, int groupsize, float eps, void *stream) {
   if (!x || !weight || !y || !sums || ((delta || partials) && !h_out)) return E2H_ERR_NULL_POINTER;
   if (groupsize != 32 && groupsize != 64 && groupsize != 128 && groupsize != 256) return E2H_ERR_BAD_GROUPSIZE;
-  if ((delta && partials) || (partials && (slices < 1 || slices > 64)) || rows < 1 || rows > INT32_MAX / 2 || dim < 128 || dim % 128 != 0 || dim % groupsize != 0 || dim > INT32_MAX)
+  if ((delta && partials) || (partials && slices != 1 && slices != 2 && slices != 4 && slices != 8) || rows < 1 || rows > INT32_MAX / 2 || dim < 128 || dim % 128 != 0 || dim % groupsize != 0 || dim > INT32_MAX)
     return E2H_ERR_BAD_SHAPE;
   if (!aligned16(x) || !aligned16(delta) || !aligned16(partials) || !aligned16(weight) || !aligned16(h_out) || !aligned16(y) || !aligned16(sums)) return E2H_ERR_MISALIGNED;
   const GroupSums to = {sums, static_cast<int>((rows + 63) / 64 * 64), (groupsize == 256 ? 128 : groupsize) / 8};

@@ -231,7 +231,8 @@ int e2h_int4_mm_silu_gate_rows(const uint16_t *x, const int32_t *packed_gate, co
 
 /* The products of a prompt of 65 to 1023 rows with what surrounds them in fewer launches.  `sums`: float32 [k / g][m rounded up to 64], the sums of every row of x over the weights'
  * quantization groups (g = groupsize, 128 for groupsize 256), 16-byte aligned, which the matmul needs for its zero points.
- *   e2h_add_rmsnorm_sums: e2h_rmsnorm, e2h_add_rmsnorm or (slices in order) e2h_add_rmsnorm_partials that writes those of y beside y; dim % 128 == 0, dim % groupsize == 0.
+ *   e2h_add_rmsnorm_sums: e2h_rmsnorm, e2h_add_rmsnorm or e2h_add_rmsnorm_partials that writes those of y beside y; dim % 128 == 0, dim % groupsize == 0; 1, 2, 4 or 8 slices, which
+ *   it adds in pairs, then pairs of pairs, as e2h_int4_mm over many rows does: bit for bit that and e2h_add_rmsnorm.
  *   e2h_int4_mm_rows: e2h_int4_mm over such rows, bit for bit; sums_there == 0: it forms the sums itself, in `sums`.  With K in e2h_int4_mm_rows_slices > 1 slices `partials`
  *   (float32 [slices, m, n]) is needed and holds the slices' sums, and y may be NULL: whoever reads the sums adds them (e2h_add_rmsnorm_sums).  e2h_int4_mm_rows_slices is 0 where such
  *   calls run on another kernel; e2h_int4_mm_rows returns E2H_ERR_BAD_SHAPE then.
