@@ -426,7 +426,7 @@ __global__ __launch_bounds__(256) void int4_quantize_pack_kernel(const uint16_t 
     }
     group_minmax<LPG>(mn, mx);
     uint32_t c[8], pair;
-    if (mx - mn < 1e37f) {
+    if (__builtin_expect(mx - mn < 1e37f, 1)) {
       // qparams_from_minmax and requant_min, the division by 15 as quantize_two divides; scale * 8 is exact
       const float range = fmaxf(to_bf16(mx - mn), bf16_to_f32(0x3586));
       const float over = range * (1.0f / 15.0f);
