@@ -9,7 +9,7 @@ namespace e2h {
 struct SeqOptions {
   int recurrence_form;         // 0 = by token count, 1 = token by token, 2 = chunked
   int recurrence_chunk;        // 0 = heuristic, else tokens per workgroup of the chunked HGRN2 form (multiple of 16)
-  int norm_run;                // 0 = heuristic, else tokens per workgroup of the norm kernel
+  int norm_run;                // 0 = heuristic, else tokens per workgroup of the norm kernel with a convolution
   int attention_decode_waves;  // 0 = by window, else 4 or 8
   int attention_prompt_queries;  // 0 = by size, else 64 or 128 per workgroup (128: heads of 64 and 128 dimensions only)
   int expert_form;             // 0 = by size, 1 = plain kernel, 2 = lists made inside the matmul, 3 = sorted rows in large tiles

@@ -35,7 +35,7 @@ extern "C" {
 
 int e2h_seq_abi_version(void);
 /* Experiment switches (0 = built-in choice): "recurrence_form" 1 = token by token, 2 = chunked; "recurrence_chunk" = tokens a
- * workgroup of the chunked HGRN2 form covers; "norm_run" = tokens a workgroup of the norm kernel covers;
+ * workgroup of the chunked HGRN2 form covers; "norm_run" = tokens a workgroup of the norm kernel covers where it convolves;
  * "attention_decode_waves" = 4 or 8; "attention_prompt_queries" = 64 or 128 a workgroup of the prompt kernels takes; "expert_form" 1 = the plain kernel for all sizes, 2 = expert lists made inside the matmul
  * (few rows), 3 = sorted rows in large tiles. */
 int e2h_seq_set_option(const char *name, int value);
