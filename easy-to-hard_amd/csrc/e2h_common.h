@@ -76,17 +76,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, ui
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, bytes, 0x00020000);
 }
 
-// g / (1 + exp(-g)), within three units in the last place of float32: a power of two whose exponent -g log2(e) is carried in two parts, and a reciprocal; the denominator in units
-// of 2^24, so that it has a normal reciprocal wherever exp(-g) is finite.  Ten instructions; expf and a division take 35, which is what counts where a lane gates 128 values
-// behind a tile of products (as a pass over memory of its own a gate waits for that).
-__device__ __forceinline__ float silu(float g) {
-  const float x = __builtin_amdgcn_fmed3f(g, -1e4f, 1e4f);
-  const float t = x * -1.44269502f;
-  const float r = __builtin_fmaf(x, -1.92596303e-8f, __builtin_fmaf(x, -1.44269502f, -t));
-  const float d = __builtin_fmaf(__builtin_amdgcn_exp2f(t), __builtin_fmaf(r, 0x1p-24f * 0.693147181f, 0x1p-24f), 0x1p-24f);
-  return g * (__builtin_amdgcn_rcpf(d) * 0x1p-24f);
-}
-
 // Workgroup barrier that orders LDS traffic only.  __syncthreads() would also drain every outstanding
 // global load (loads and stores share one counter on this architecture), which would empty a register
 // prefetch pipeline once per use.

@@ -219,6 +219,74 @@ __device__ __forceinline__ void walk(P &p, uint8_t *lds) {
 }
 #endif
 
+#if defined(__HIPCC__)
+// ---- activations behind a tile ------------------------------------------------------------------------------------------------------------
+// A lane activates 128 values behind its tile with nothing beside it (35 instructions each, what expf and a division take, are 9 us a tile).  So they are formed by a few instructions that end
+// within kNear units in the last place of the form that a pass over memory has, and where a value lies that close to a boundary of its rounding to bfloat16 that form decides: all results
+// are bit for bit those of the pass.  Of 512 values of a wave's store one in eight has such a value; they are taken one per lane and round.
+constexpr uint32_t kNear = 8;
+typedef float f32x8_t __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ bool undecided(uint32_t bits) { return ((bits + 0x8000u + kNear) & 0xFFFFu) < 2 * kNear; }
+
+// v: close to form(the eight bfloat16 values of `of`); those near a boundary become that.  (Vectors: of arrays the compiler makes memory, whose waits would be counted as a tile's loads.)
+template <class Form>
+__device__ __forceinline__ f32x8_t settled(f32x8_t v, u32x4_t of, Form form) {
+  typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+  typedef uint32_t u32x8_t __attribute__((ext_vector_type(8)));
+  const u32x8_t bits = __builtin_bit_cast(u32x8_t, v);
+  u16x2_t least = {0xFFFF, 0xFFFF};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {  // the lower halves of two values at a time
+    const uint32_t low = __builtin_amdgcn_perm(bits[2 * i + 1], bits[2 * i], 0x05040100u);
+    const u16x2_t at = __builtin_bit_cast(u16x2_t, low) + static_cast<uint16_t>(0x8000u + kNear);
+    least = __builtin_elementwise_min(least, at);
+  }
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(least[0] < 2 * kNear || least[1] < 2 * kNear) == 0, 1)) return v;
+  uint32_t todo = 0;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) todo |= undecided(bits[e]) ? 1u << e : 0u;
+  while (todo) {
+    const int next = __builtin_ctz(todo), pair = next >> 1;
+    uint32_t two = pair == 1 ? of[1] : of[0];
+    two = pair == 2 ? of[2] : two;
+    two = pair == 3 ? of[3] : two;
+    const float y = form(__builtin_bit_cast(float, next & 1 ? two & 0xFFFF0000u : two << 16));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = next == e ? y : v[e];
+    todo &= todo - 1;
+  }
+  return v;
+}
+
+// g / (1 + exp(-g)) of a bfloat16 g, within three units in the last place of float32: a power of two whose exponent -g log2(e) is carried in two parts, and a reciprocal.  The denominator is in
+// units of 2^16, so that it has a normal reciprocal wherever exp(-g) is finite, and so is g, of which no bit is lost and no product leaves float32.
+__device__ __forceinline__ float near_silu(float g) {
+  const float x = __builtin_amdgcn_fmed3f(g, -1e4f, 1e4f);
+  const float t = x * -1.44269502f;
+  const float r = __builtin_fmaf(x, -1.92596303e-8f, __builtin_fmaf(x, -1.44269502f, -t));
+  const float d = __builtin_fmaf(__builtin_amdgcn_exp2f(t), __builtin_fmaf(r, 0x1p-16f * 0.693147181f, 0x1p-16f), 0x1p-16f);
+  return g * 0x1p-16f * __builtin_amdgcn_rcpf(d);
+}
+
+// bf16( bf16(silu(g)) * u ) of eight bfloat16 values each, as e2h_silu_mul forms it
+__device__ __forceinline__ u32x4_t gated(u32x4_t g, u32x4_t u) {
+  const auto low = [](uint32_t b) { return __builtin_bit_cast(float, b << 16); };
+  const auto high = [](uint32_t b) { return __builtin_bit_cast(float, b & 0xFFFF0000u); };
+  f32x8_t v;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) v[e] = near_silu(e & 1 ? high(g[e >> 1]) : low(g[e >> 1]));
+  v = settled(v, g, [](float z) { return z / (1.0f + expf(-z)); });
+  u32x4_t out;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t act = f32x2_to_bf16_rne(v[2 * e], v[2 * e + 1]);
+    out[e] = f32x2_to_bf16_rne(low(act) * low(u[e]), high(act) * high(u[e]));
+  }
+  return out;
+}
+#endif
+
 // The tiles of one plain product, dealt to the XCDs in contiguous runs of equal length: panels of eight column blocks, all row
 // blocks of a panel after each other, so that the 32 tiles at work on an XCD share four row blocks and eight column blocks.
 // kCols: columns of y per tile, 256, or 128 of a pair of products (two rows of w each).

@@ -100,15 +100,14 @@ struct Int8GateWalk : gemm256::PlainWalk<128> {
   __device__ __forceinline__ void store(const Tile &tile, const Dest &d, int, int q, int row, int col, float (&v)[8], float (&u)[8]) const {
     const auto low = [](uint32_t b) { return __builtin_bit_cast(float, b << 16); };
     const auto high = [](uint32_t b) { return __builtin_bit_cast(float, b & 0xFFFF0000u); };
-    u32x4_t out;
+    u32x4_t g, up;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {  // the rounding points of the two linears, of F.silu and of the product
+    for (int e = 0; e < 4; ++e) {  // the rounding points of the two linears
       const uint32_t a = pack_bf16(v[2 * e], v[2 * e + 1]), b = pack_bf16(u[2 * e], u[2 * e + 1]), sa = d.scale[q][e], sb = d.scale2[q][e];
-      const uint32_t g = pack_bf16(low(a) * low(sa), high(a) * high(sa)), up = pack_bf16(low(b) * low(sb), high(b) * high(sb));
-      const uint32_t act = pack_bf16(silu(low(g)), silu(high(g)));
-      out[e] = pack_bf16(low(act) * low(up), high(act) * high(up));
+      g[e] = pack_bf16(low(a) * low(sa), high(a) * high(sa));
+      up[e] = pack_bf16(low(b) * low(sb), high(b) * high(sb));
     }
-    __builtin_amdgcn_raw_buffer_store_b128(out, y_rsrc(tile), y_at(tile, row, col), 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(gemm256::gated(g, up), y_rsrc(tile), y_at(tile, row, col), 0, 0);
   }
 };
 
@@ -574,19 +573,13 @@ struct Int4GateWalk : gemm256::PlainWalk<128> {
     }
   }
   __device__ __forceinline__ void store(const Tile &tile, const Dest &d, int j, int q, int row, int col, float (&v)[8], float (&u)[8]) const {
-    const auto low = [](uint32_t b) { return __builtin_bit_cast(float, b << 16); };
-    const auto high = [](uint32_t b) { return __builtin_bit_cast(float, b & 0xFFFF0000u); };
     const int n = out_col(tile, col);
     finish_int4(*this, tile, d.up[j], d.unit[q][0], row, n, 0, v);
     finish_int4(*this, tile, d.up[j], d.unit[q][1], row, n, N, u);
-    u32x4_t out;
+    u32x4_t g, up;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const uint32_t g = pack_bf16(v[2 * e], v[2 * e + 1]), up = pack_bf16(u[2 * e], u[2 * e + 1]);
-      const uint32_t act = pack_bf16(silu(low(g)), silu(high(g)));
-      out[e] = pack_bf16(low(act) * low(up), high(act) * high(up));
-    }
-    __builtin_amdgcn_raw_buffer_store_b128(out, y_rsrc(tile), y_at(tile, row, col), 0, 0);
+    for (int e = 0; e < 4; ++e) g[e] = pack_bf16(v[2 * e], v[2 * e + 1]), up[e] = pack_bf16(u[2 * e], u[2 * e + 1]);
+    __builtin_amdgcn_raw_buffer_store_b128(gemm256::gated(g, up), y_rsrc(tile), y_at(tile, row, col), 0, 0);
   }
 };
 

@@ -471,6 +471,36 @@ def test_gated_unpacked_rows_are_the_two_exact_products_gated(g, m, n, k):
     _check_gate(got[rows], _gate_of(*(_double(c, s, z, x, g, rows) for c, s, z, _ in halves)))
 
 
+def test_gates_of_a_tile_round_as_the_pass_does_for_every_bfloat16():
+    """All 65536 gates as they are and times column scales up to where they overflow, beside ups of both signs: bit for bit two calls and silu_mul, NaN and infinities included."""
+    k = 256
+    x = torch.zeros((65536, k), dtype=torch.bfloat16)
+    x[:, 0] = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    x[:, 1] = 1.0
+    x = x.to(DEV)
+    q = torch.zeros((2, 8, k), dtype=torch.int8, device=DEV)
+    q[0, :, 0] = torch.tensor([1, -1, 3, 7, 1, 1, 101, 1])
+    q[1, :, 1] = torch.tensor([1, 3, -1, 1, 1, 5, 1, -7])
+    s = torch.tensor([[1, 1, 0.37, 2.0 ** -20, 2.0 ** 100, 2.0 ** -100, 0.0113, 1.7], [1, 0.3, 1, 2.0 ** 60, 1, 1, 2.0 ** -60, 1]], dtype=torch.bfloat16, device=DEV)
+    got = ops.int8_mm_silu_gate_rows(x, q[0], s[0], q[1], s[1])
+    a, b = (ops.int8_mm(x, w, t) for w, t in zip(q, s))
+    want = ops.silu_mul(a, b)
+    assert torch.isinf(a).any() and torch.isinf(want).any() and torch.isnan(want).any()
+    nan = torch.isnan(want)
+    assert torch.equal(torch.isnan(got), nan) and torch.equal(got[~nan].view(torch.int16), want[~nan].view(torch.int16))
+
+
+@pytest.mark.parametrize("g,m,n,k", [(32, 66049, 1032, 512), (128, 8190, 11000, 4096)])
+def test_gated_unpacked_rows_are_the_two_calls_on_unpacked_operands_bit_for_bit(g, m, n, k):
+    gen = torch.Generator(device=DEV).manual_seed(g)
+    x = torch.randn((m, k), generator=gen, device=DEV).to(torch.bfloat16)
+    w = [ops.int4_quantize_pack((torch.randn((n, k), generator=gen, device=DEV) * 0.05).to(torch.bfloat16), g, 8) for _ in range(2)]
+    lib = _lib.load()
+    assert lib.e2h_int4_mm_silu_gate_rows_scratch_bytes(m, n, k, g, 8) > 0 and lib.e2h_int4_mm_scratch_bytes(m, n, k, g, 8) > 0
+    want = ops.silu_mul(*(ops.int4_mm(x, p, g, sz) for p, sz in w))
+    assert torch.equal(ops.int4_mm_silu_gate_rows(x, *w[0], *w[1], g), want)
+
+
 def test_gated_unpacked_rows_leave_what_float16_lacks_to_the_other_kernel():
     """A row that is not finite, a row of small values beside a large one, and a scale that float16 does not hold in the second matrix: as two calls give them."""
     m, n, k, g = 66049, 264, 512, 128
