@@ -109,9 +109,10 @@ int run_linear(const stream::Args &a, bf16_t *y, float cap, float *scratch, hipS
 }
 
 // ---- many rows: the activation behind a tile of products (e2h_gemm256.h) ---------------------------------------------------------------
-// cap tanh(y / cap): with z = y y it is y + y z Q(z) up to |y| = 0.75 cap, Q by the Remez algorithm (3.3e-8 of tanh, half a unit in the last place of float32) in powers of 1 / cap^2, else
-// cap (1 - 2 / (1 + exp(2 y / cap))).  A tile's store forms the first for all of its values, and the second too where a wave's 512 values have one that needs it: six instructions a value
-// where tanhf and the division take 45, which would take as long as the pass over memory that is saved (128 values per lane and wave with nothing beside them).
+// cap tanh(y / cap): with z = y y it is y (1 + z Q(z)) up to |y| = 0.75 cap, Q by the Remez algorithm (3.3e-8 of tanh, half a unit in the last place of float32) in powers of 1 / cap^2, else
+// cap (1 - 2 / (1 + exp(2 y / cap))); what either could round otherwise to bfloat16 than e2h_seq_softcap does is formed as there (gemm256::settled).  A tile's store forms the first for all of
+// its values, and the second too where a wave's 512 values have one that needs it: ten instructions a value with the look at its rounding, where tanhf and the division take 45, which would
+// take as long as the pass over memory that is saved (128 values per lane and wave with nothing beside them).
 struct Cap {
   float cap, limit, q[5], twice;  // limit: 0.75 cap; twice: 2 / cap in units of log 2
 };
@@ -137,7 +138,7 @@ struct RowsWalk : gemm256::PlainWalk<> {
     float q = c.q[4];
 #pragma unroll
     for (int j = 3; j >= 0; --j) q = __builtin_fmaf(q, z, c.q[j]);
-    return __builtin_fmaf(y * z, q, y);
+    return y * __builtin_fmaf(z, q, 1.0f);  // (-0 stays that)
   }
   __device__ __forceinline__ float capped_far(float y, float near) const {
     const float far = c.cap * __builtin_fmaf(-2.0f, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(y * c.twice)), 1.0f);
@@ -157,7 +158,8 @@ struct RowsWalk : gemm256::PlainWalk<> {
       }
     }
     if (ACT == kCap) {
-      float y[8], near[8], top = 0.f;
+      gemm256::f32x8_t near;
+      float y[8], top = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         y[e] = e & 1 ? high(out[e >> 1]) : low(out[e >> 1]);
@@ -168,6 +170,8 @@ struct RowsWalk : gemm256::PlainWalk<> {
 #pragma unroll
         for (int e = 0; e < 8; ++e) near[e] = capped_far(y[e], near[e]);
       }
+      const float cap = c.cap;
+      near = gemm256::settled(near, out, [cap](float z) { return cap * tanhf(z / cap); });
 #pragma unroll
       for (int e = 0; e < 4; ++e) out[e] = pack_bf16(near[2 * e], near[2 * e + 1]);
     }

@@ -839,6 +839,21 @@ def test_linear_rows_with_a_soft_cap(rows, n, k, cap):
     assert not seq_ops.linear_rows_pay(x, w, seq_ops.ACT_SOFTCAP, 2.0 ** 11) and not seq_ops.linear_rows_pay(x, w, seq_ops.ACT_SOFTCAP, 2.0 ** -7)
 
 
+@pytest.mark.parametrize("cap", [2.0 ** -6, 0.3, 1.0, 15.0, 30.0, 50.0, 333.3, 1024.0])
+def test_soft_cap_of_a_tile_rounds_as_the_pass_does_for_every_bfloat16(cap):
+    """All 65536 logits, NaN and infinities included, each beside others of its tile below and beyond the cap: bit for bit the product and softcap_."""
+    x = torch.zeros((65536, 192), dtype=torch.bfloat16)
+    x[:, 0] = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    w = torch.zeros((264, 192), dtype=torch.bfloat16)
+    w[:, 0] = torch.linspace(-1.0, 1.0, 264).to(torch.bfloat16)
+    w[0], w[100, 0] = 1.0, 1.0
+    x, w = x.to(DEV), w.to(DEV)
+    want = seq_ops.softcap_(seq_ops.linear_rows(x, w, seq_ops.ACT_NONE), cap)
+    got = seq_ops.linear_rows(x, w, seq_ops.ACT_SOFTCAP, cap)
+    nan = torch.isnan(want)
+    assert torch.equal(torch.isnan(got), nan) and torch.equal(got[~nan].view(torch.int16), want[~nan].view(torch.int16))
+
+
 
 def test_feed_forward_of_many_rows_takes_one_launch_for_up_and_its_activation():
     from easy_to_hard_amd.feed_forward import SquaredReluFF
