@@ -52,10 +52,11 @@ struct DeltaSums {
 // way (8192 x 4096, sum and norm 72 us, 80 in runs of 8), and large residual rows, which are not read again soon, are stored past the caches (58).
 // us at 4096 channels, in brackets runs of 8 (convolution: 1024 threads, two rows together) that waited for every row: 8192 rows with residual 58 (94), layer norm 63 (91), eight experts'
 // terms 161 (187), convolution 73 (101); 8000 rows 56 (85), 62 (106), 159 (214), 66 (167: one workgroup too many for a round); 2048 rows 17 (18), 20 (21), 39 (38), 25 (33).
-template <typename T, int BLOCK, int NP, int TAPS, bool LAYER, bool TERMS, bool AHEAD>
+template <typename T, int BLOCK, int NP, int TAPS, bool LAYER, bool TERMS, bool AHEAD, int SPLIT>
 __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_args a, const DeltaSums sums, int runs, int run, int streamed) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  constexpr int kWaves = BLOCK / 64;
+  static_assert(SPLIT == 1 || SPLIT == NP, "a thread's pieces are summed together or each for itself");
+  constexpr int kWaves = BLOCK / 64, kSums = SPLIT * kWaves, kEach = NP / SPLIT;  // a row's partial sums, and the pieces that a thread adds to each
   constexpr int RING = TAPS > 1 ? TAPS - 1 : 1;
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
   const int W = static_cast<int>(a.width), seqlen = static_cast<int>(a.seqlen), taps = a.taps;
@@ -67,48 +68,52 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
   const int first = TAPS && a.first ? static_cast<int>(a.first[b]) : 0;
   const size_t row0 = static_cast<size_t>(b) * seqlen;
   const uint32_t row_f32 = static_cast<uint32_t>(W) * 4, row_t = static_cast<uint32_t>(W) * sizeof(T);
-  __shared__ __attribute__((aligned(16))) float part[2][kWaves][LAYER ? 2 : 1];
+  __shared__ __attribute__((aligned(16))) float part[2][kSums][LAYER ? 2 : 1];
   int phase = 0;
 
-  auto wave_count = [&](int w) {  // channels of the row that wave w holds
+  auto sum_count = [&](int u) {  // channels of the row in partial sum u, of wave u % kWaves
     int n = 0;
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int left = W - (p * BLOCK + w * 64) * 4;
+    for (int p = 0; p < kEach; ++p) {
+      const int left = W - ((u / kWaves * kEach + p) * BLOCK + u % kWaves * 64) * 4;
       n += left < 0 ? 0 : left > 256 ? 256 : left;
     }
     return static_cast<float>(n);
   };
+  const int wave = threadIdx.x >> 6;
   auto piece = [&](int p) { return p * BLOCK + static_cast<int>(threadIdx.x); };
   // z -> (z - mean) / sqrt(variance + eps) * weight + bias
   auto layer_norm = [&](f32x4_t (&z)[NP], const f32x4_t (&weight)[NP], const f32x4_t (&bias)[NP]) {
-    const float own = wave_count(threadIdx.x >> 6);
-    float s = 0.f;  // pieces beyond the width are zero
 #pragma unroll
-    for (int p = 0; p < NP; ++p) s += z[p][0] + z[p][1] + z[p][2] + z[p][3];
-    const float mean = own > 0.f ? wave_add(s) / own : 0.f;
-    float q = 0.f;
+    for (int u = 0; u < SPLIT; ++u) {
+      const float own = sum_count(u * kWaves + wave);
+      float s = 0.f;  // pieces beyond the width are zero
 #pragma unroll
-    for (int p = 0; p < NP; ++p)
-      if (piece(p) * 4 < W) {
-        const f32x4_t c = z[p] - mean;
+      for (int p = u * kEach; p < (u + 1) * kEach; ++p) s += z[p][0] + z[p][1] + z[p][2] + z[p][3];
+      const float mean = own > 0.f ? wave_add(s) / own : 0.f;
+      float q = 0.f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) q = __builtin_fmaf(c[e], c[e], q);
+      for (int p = u * kEach; p < (u + 1) * kEach; ++p)
+        if (piece(p) * 4 < W) {
+          const f32x4_t c = z[p] - mean;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) q = __builtin_fmaf(c[e], c[e], q);
+        }
+      q = wave_add(q);
+      if ((threadIdx.x & 63) == 0) {
+        part[phase][u * kWaves + wave][0] = mean;
+        part[phase][u * kWaves + wave][LAYER ? 1 : 0] = q;
       }
-    q = wave_add(q);
-    if ((threadIdx.x & 63) == 0) {
-      part[phase][threadIdx.x >> 6][0] = mean;
-      part[phase][threadIdx.x >> 6][LAYER ? 1 : 0] = q;
     }
     __syncthreads();
     float m = 0.f, v = 0.f;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) m = __builtin_fmaf(wave_count(w), part[phase][w][0], m);
+    for (int w = 0; w < kSums; ++w) m = __builtin_fmaf(sum_count(w), part[phase][w][0], m);
     m /= static_cast<float>(W);
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
+    for (int w = 0; w < kSums; ++w) {
       const float c = part[phase][w][0] - m;
-      v += __builtin_fmaf(wave_count(w) * c, c, part[phase][w][LAYER ? 1 : 0]);
+      v += __builtin_fmaf(sum_count(w) * c, c, part[phase][w][LAYER ? 1 : 0]);
     }
     const float r = 1.0f / sqrtf(v / static_cast<float>(W) + a.eps);
 #pragma unroll
@@ -117,19 +122,26 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
   };
 
   auto inverse_rms = [&](const f32x4_t (&z)[NP]) {
-    float v = 0.f;
+    float v[SPLIT];
 #pragma unroll
-    for (int p = 0; p < NP; ++p)
+    for (int u = 0; u < SPLIT; ++u) {
+      v[u] = 0.f;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v = __builtin_fmaf(z[p][e], z[p][e], v);
-    v = wave_add(v);
-    if ((threadIdx.x & 63) == 0) part[phase][threadIdx.x >> 6][0] = v;
+      for (int p = u * kEach; p < (u + 1) * kEach; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[u] = __builtin_fmaf(z[p][e], z[p][e], v[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < SPLIT; ++u) {
+      v[u] = wave_add(v[u]);
+      if ((threadIdx.x & 63) == 0) part[phase][u * kWaves + wave][0] = v[u];
+    }
     __syncthreads();
-    v = 0.f;
+    float sum = 0.f;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) v += part[phase][w][0];
+    for (int w = 0; w < kSums; ++w) sum += part[phase][w][0];
     phase ^= 1;  // the next sums go to the other half, so one barrier per sum is enough
-    return 1.0f / sqrtf(v / static_cast<float>(W) + a.eps);
+    return 1.0f / sqrtf(sum / static_cast<float>(W) + a.eps);
   };
 
   // everything that does not depend on the rows; zero weights and rows beyond the width contribute nothing
@@ -338,7 +350,7 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
 #endif
 }
 
-template <typename T, int BLOCK, int NP, int TAPS, bool LAYER, bool TERMS>
+template <typename T, int BLOCK, int NP, int TAPS, bool LAYER, bool TERMS, int SPLIT>
 void launch_norm_conv_rows(const e2h_norm_conv_args &a, const DeltaSums &sums, int runs, int run, hipStream_t s) {
   const int64_t workgroups = TAPS ? a.batch * runs : a.batch * a.seqlen < (1 << 20) ? a.batch * a.seqlen : 1 << 20;
   const dim3 grid(static_cast<unsigned>(workgroups)), block(BLOCK);
@@ -346,35 +358,48 @@ void launch_norm_conv_rows(const e2h_norm_conv_args &a, const DeltaSums &sums, i
   const int streamed = a.batch * a.seqlen * a.width >= (int64_t{1} << 28) / 12;
   if constexpr (TAPS > 0) {
     if (run > 1) {
-      hipLaunchKernelGGL((norm_conv_kernel<T, BLOCK, NP, TAPS, LAYER, TERMS, true>), grid, block, 0, s, a, sums, runs, run, streamed);
+      hipLaunchKernelGGL((norm_conv_kernel<T, BLOCK, NP, TAPS, LAYER, TERMS, true, SPLIT>), grid, block, 0, s, a, sums, runs, run, streamed);
       return;
     }
   }
-  hipLaunchKernelGGL((norm_conv_kernel<T, BLOCK, NP, TAPS, LAYER, TERMS, false>), grid, block, 0, s, a, sums, runs, run, streamed);
+  hipLaunchKernelGGL((norm_conv_kernel<T, BLOCK, NP, TAPS, LAYER, TERMS, false, SPLIT>), grid, block, 0, s, a, sums, runs, run, streamed);
 }
 
-template <typename T, int BLOCK, int NP>
+// CONV: with a convolution or not
+template <typename T, int BLOCK, int NP, bool CONV, int SPLIT = 1>
 void launch_norm_conv_taps(const e2h_norm_conv_args &a, const DeltaSums &sums, int runs, int run, hipStream_t s) {
-  if (a.norm_kind == E2H_SEQ_LAYER_NORM) {
-    if (a.terms) return launch_norm_conv_rows<T, BLOCK, NP, 0, true, true>(a, sums, runs, run, s);
-    return launch_norm_conv_rows<T, BLOCK, NP, 0, true, false>(a, sums, runs, run, s);
+  if constexpr (CONV) {
+    if (a.taps <= 4) launch_norm_conv_rows<T, BLOCK, NP, 4, false, false, SPLIT>(a, sums, runs, run, s);
+    else launch_norm_conv_rows<T, BLOCK, NP, 8, false, false, SPLIT>(a, sums, runs, run, s);
+  } else if (a.norm_kind == E2H_SEQ_LAYER_NORM) {
+    if (a.terms) launch_norm_conv_rows<T, BLOCK, NP, 0, true, true, SPLIT>(a, sums, runs, run, s);
+    else launch_norm_conv_rows<T, BLOCK, NP, 0, true, false, SPLIT>(a, sums, runs, run, s);
+  } else {
+    if (a.terms) launch_norm_conv_rows<T, BLOCK, NP, 0, false, true, SPLIT>(a, sums, runs, run, s);
+    else launch_norm_conv_rows<T, BLOCK, NP, 0, false, false, SPLIT>(a, sums, runs, run, s);
   }
-  if (a.terms) return launch_norm_conv_rows<T, BLOCK, NP, 0, false, true>(a, sums, runs, run, s);
-  if (!a.conv) return launch_norm_conv_rows<T, BLOCK, NP, 0, false, false>(a, sums, runs, run, s);
-  if (a.taps <= 4) launch_norm_conv_rows<T, BLOCK, NP, 4, false, false>(a, sums, runs, run, s);
-  else launch_norm_conv_rows<T, BLOCK, NP, 8, false, false>(a, sums, runs, run, s);
 }
 
+// A row's sums have one order (one with a convolution, one without) whatever the number of rows beside it and the length of runs: forms of half the threads keep a thread's two pieces apart
+// (SPLIT), as two threads of the other form have them.  8192 x 4096 with convolution 84 us, 78 with them added first; 8192 x 2048 31.7, 31.1, layer norm 34.6, 32.9.
 template <typename T>
 void launch_norm_conv(const e2h_norm_conv_args &a, const DeltaSums &sums, int runs, int run, hipStream_t s) {
-  if (a.width <= 1024) launch_norm_conv_taps<T, 256, 1>(a, sums, runs, run, s);
-  // eight values per thread where many rows are waiting: half the waves, which repeat a row's sums each (8192 x 2048, layer norm 31 us, 38 with four values; final norm 24, 31)
-  else if (a.width <= 2048 && !a.conv && a.batch * a.seqlen > 256) launch_norm_conv_taps<T, 256, 2>(a, sums, runs, run, s);
-  else if (a.width <= 2048) launch_norm_conv_taps<T, 512, 1>(a, sums, runs, run, s);
-  else if (a.width <= 4096 && a.conv && run == 1) launch_norm_conv_taps<T, 1024, 1>(a, sums, runs, run, s);
-  else if (a.width <= 4096) launch_norm_conv_taps<T, 512, 2>(a, sums, runs, run, s);
-  else if (a.width <= 8192) launch_norm_conv_taps<T, 512, 4>(a, sums, runs, run, s);
-  else launch_norm_conv_taps<T, 1024, 4>(a, sums, runs, run, s);
+  if (a.conv) {
+    if (a.width <= 1024) launch_norm_conv_taps<T, 256, 1, true>(a, sums, runs, run, s);
+    else if (a.width <= 2048) launch_norm_conv_taps<T, 512, 1, true>(a, sums, runs, run, s);
+    else if (a.width <= 4096 && run == 1) launch_norm_conv_taps<T, 1024, 1, true>(a, sums, runs, run, s);
+    else if (a.width <= 4096) launch_norm_conv_taps<T, 512, 2, true, 2>(a, sums, runs, run, s);
+    else if (a.width <= 8192) launch_norm_conv_taps<T, 512, 4, true>(a, sums, runs, run, s);
+    else launch_norm_conv_taps<T, 1024, 4, true>(a, sums, runs, run, s);
+    return;
+  }
+  if (a.width <= 1024) launch_norm_conv_taps<T, 256, 1, false>(a, sums, runs, run, s);
+  // eight values per thread where many rows are waiting: half the waves, which repeat a row's sums each (8192 x 2048, layer norm 35 us, 38 with four values; final norm 30, 31)
+  else if (a.width <= 2048 && a.batch * a.seqlen > 256) launch_norm_conv_taps<T, 256, 2, false, 2>(a, sums, runs, run, s);
+  else if (a.width <= 2048) launch_norm_conv_taps<T, 512, 1, false>(a, sums, runs, run, s);
+  else if (a.width <= 4096) launch_norm_conv_taps<T, 512, 2, false>(a, sums, runs, run, s);
+  else if (a.width <= 8192) launch_norm_conv_taps<T, 512, 4, false>(a, sums, runs, run, s);
+  else launch_norm_conv_taps<T, 1024, 4, false>(a, sums, runs, run, s);
 }
 
 // ---- elementwise -----------------------------------------------------------------------------------------------------

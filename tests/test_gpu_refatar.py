@@ -101,6 +101,31 @@ def test_norm_conv_of_many_rows(dtype, b, t, width, taps):
 
 
 @BOTH
+@pytest.mark.parametrize("width,taps,layer", [(4096, 4, False), (4096, 7, False), (3076, 3, False), (1500, 0, False), (2048, 0, True), (1028, 0, True), (2048, 0, False), (4096, 0, True)])
+def test_a_row_of_norm_conv_does_not_depend_on_the_rows_beside_it(dtype, width, taps, layer):
+    """Workgroups of fewer threads, which many rows and runs take, add a row's squares in the order of the others: bit for bit."""
+    g = torch.Generator(device=DEV).manual_seed(width)
+    rows, few = 1000, 60
+    x, d = 3 * torch.randn((rows, width), generator=g, device=DEV), torch.randn((rows, width), generator=g, device=DEV).to(dtype)
+    wd, wn, bd, bn = (0.3 * torch.randn((4, width), generator=g, device=DEV)).unbind(0)
+    wc = 0.5 * torch.randn((taps, width), generator=g, device=DEV)
+
+    def run(n):
+        kw = dict(layer_norm=True, delta_bias=bd, norm_bias=bn) if layer else {}
+        if taps:
+            kw = dict(conv=wc, tails=(torch.full((1, taps, width), 7.0, device=DEV), torch.empty((1, taps, width), device=DEV)), input_pos=positions(0, n))
+        return seq_ops.norm_conv(x[:n], 1, n, 1e-4, dtype, delta=d[:n], delta_weight=wd, delta_offset=1.0, norm_weight=wn, norm_offset=1.0, **kw)
+
+    many = run(rows)
+    for got, want in zip(run(few), many):
+        assert torch.equal(got, want[:few])
+    for length in (1, 3, 32) if taps else ():
+        _lib.set_seq_option("norm_run", length)
+        for got, want in zip(run(rows), many):
+            assert torch.equal(got, want)
+
+
+@BOTH
 def test_norm_conv_parts_and_padding(dtype):
     b, t, width, taps, eps = 3, 9, 72, 3, 1e-5
     x, d = randn(b * t, width, seed=1), randn(b * t, width, seed=2, dtype=dtype)
