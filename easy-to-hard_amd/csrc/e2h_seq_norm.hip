@@ -82,8 +82,15 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
   };
   const int wave = threadIdx.x >> 6;
   auto piece = [&](int p) { return p * BLOCK + static_cast<int>(threadIdx.x); };
+  // Rows beyond 8192 leave no registers for weights and biases in front of the row (kLate): read where they are used.  (2048 x 12288, two layer norms: 169 us, 1590 with 655 values of every thread spilled.)
+  constexpr bool kLate = TAPS == 0 && BLOCK * NP > 2048;
+  auto channel = [&](const float *from, int p, float offset) {
+    f32x4_t v = zero;
+    if (from && piece(p) * 4 < W) v = load4(from + piece(p) * 4) + offset;
+    return v;
+  };
   // z -> (z - mean) / sqrt(variance + eps) * weight + bias
-  auto layer_norm = [&](f32x4_t (&z)[NP], const f32x4_t (&weight)[NP], const f32x4_t (&bias)[NP]) {
+  auto layer_norm = [&](f32x4_t (&z)[NP], f32x4_t (&weight)[NP], f32x4_t (&bias)[NP], const float *late_weight, float offset, const float *late_bias) {
 #pragma unroll
     for (int u = 0; u < SPLIT; ++u) {
       const float own = sum_count(u * kWaves + wave);
@@ -117,7 +124,10 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
     }
     const float r = 1.0f / sqrtf(v / static_cast<float>(W) + a.eps);
 #pragma unroll
-    for (int p = 0; p < NP; ++p) z[p] = (z[p] - m) * r * weight[p] + bias[p];
+    for (int p = 0; p < NP; ++p) {
+      if (kLate) weight[p] = channel(late_weight, p, offset), bias[p] = channel(late_bias, p, 0.f);
+      z[p] = (z[p] - m) * r * weight[p] + bias[p];
+    }
     phase ^= 1;
   };
 
@@ -150,10 +160,10 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
   for (int p = 0; p < NP; ++p) {
     const int i = piece(p) * 4;
     wd[p] = wn[p] = bd[p] = bn[p] = zero;
-    if (a.delta_weight && i < W) wd[p] = load4(a.delta_weight + i) + a.delta_offset;
-    if (a.norm_weight && i < W) wn[p] = load4(a.norm_weight + i) + a.norm_offset;
-    if (LAYER && a.delta_bias && i < W) bd[p] = load4(a.delta_bias + i);
-    if (LAYER && a.norm_bias && i < W) bn[p] = load4(a.norm_bias + i);
+    if (!kLate && a.delta_weight && i < W) wd[p] = load4(a.delta_weight + i) + a.delta_offset;
+    if (!kLate && a.norm_weight && i < W) wn[p] = load4(a.norm_weight + i) + a.norm_offset;
+    if (!kLate && LAYER && a.delta_bias && i < W) bd[p] = load4(a.delta_bias + i);
+    if (!kLate && LAYER && a.norm_bias && i < W) bn[p] = load4(a.norm_bias + i);
     if (TAPS) {
 #pragma unroll
       for (int j = 0; j < TAPS; ++j) {
@@ -248,14 +258,17 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
     }
     if (a.delta || TERMS || summed) {
       if constexpr (LAYER) {
-        layer_norm(d, wd, bd);
+        layer_norm(d, wd, bd, a.delta_weight, a.delta_offset, a.delta_bias);
 #pragma unroll
         for (int p = 0; p < NP; ++p)
           if (piece(p) * 4 < W) h[p] += d[p];
       } else {
         const float r = inverse_rms(d);
 #pragma unroll
-        for (int p = 0; p < NP; ++p) h[p] += d[p] * r * wd[p];
+        for (int p = 0; p < NP; ++p) {
+          if (kLate) wd[p] = channel(a.delta_weight, p, a.delta_offset);
+          h[p] += d[p] * r * wd[p];
+        }
       }
       const bool there = emit && a.x_out;
       const __amdgpu_buffer_rsrc_t to = make_rsrc(a.x_out + (there ? (row0 + t) * W : 0), there ? row_f32 : 0);
@@ -269,11 +282,14 @@ __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_ar
     }
     if (a.norm_weight) {
       if constexpr (LAYER) {
-        layer_norm(h, wn, bn);
+        layer_norm(h, wn, bn, a.norm_weight, a.norm_offset, a.norm_bias);
       } else {
         const float r = inverse_rms(h);
 #pragma unroll
-        for (int p = 0; p < NP; ++p) h[p] = h[p] * r * wn[p];
+        for (int p = 0; p < NP; ++p) {
+          if (kLate) wn[p] = channel(a.norm_weight, p, a.norm_offset);
+          h[p] = h[p] * r * wn[p];
+        }
       }
     }
     if (TAPS && pos0 + t < first) {  // padding: the convolution must not see it

@@ -101,7 +101,7 @@ def test_norm_conv_of_many_rows(dtype, b, t, width, taps):
 
 
 @BOTH
-@pytest.mark.parametrize("width,taps,layer", [(4096, 4, False), (4096, 7, False), (3076, 3, False), (1500, 0, False), (2048, 0, True), (1028, 0, True), (2048, 0, False), (4096, 0, True)])
+@pytest.mark.parametrize("width,taps,layer", [(4096, 4, False), (4096, 7, False), (3076, 3, False), (1500, 0, False), (2048, 0, True), (1028, 0, True), (2048, 0, False), (4096, 0, True), (12292, 0, True), (16384, 0, False)])
 def test_a_row_of_norm_conv_does_not_depend_on_the_rows_beside_it(dtype, width, taps, layer):
     """Workgroups of fewer threads, which many rows and runs take, add a row's squares in the order of the others: bit for bit."""
     g = torch.Generator(device=DEV).manual_seed(width)
