@@ -2,6 +2,8 @@
 // its input convolution over time in one pass over the float32 residual stream, and the elementwise steps.
 #include <string.h>
 
+#include <algorithm>
+
 #include "e2h_seq_common.h"
 
 namespace e2h {
@@ -545,7 +547,7 @@ int norm_conv(const e2h_norm_conv_args *a, const DeltaSums &sums, void *stream) 
     return E2H_ERR_MISALIGNED;
   // The fewest tokens per workgroup with which the convolution's workgroups are a whole number of rounds, up to 32: longer runs normalise fewer tokens twice, and one workgroup beyond a round
   // costs a round.  A round is a workgroup per CU, of narrower rows two or four (8192 x 2048: 512 workgroups 42 us, 256 54; 8192 x 1024: 1024 24, 256 49).
-  int run = a->conv ? seq_options().norm_run : 1;
+  int run = a->conv ? std::min<int64_t>(seq_options().norm_run, a->seqlen) : 1;  // (single tokens: the form that adds slices)
   const int64_t round = a->width <= 1024 ? 1024 : a->width <= 2048 ? 512 : 256;
   for (int64_t most = round; !run; most += round) {
     const int64_t per_sequence = most / a->batch;

@@ -935,3 +935,26 @@ def test_norm_that_adds_the_slices_of_a_product_equals_the_product_and_the_norm(
     assert seq_ops.linear_sums(y[:16], w) is None
     with pytest.raises(RuntimeError):
         seq_ops.norm_conv(x, 1, rows, 1e-4, torch.bfloat16, delta=sums, delta_weight=wd)  # several tokens of a sequence
+
+
+@pytest.mark.parametrize("run", [0, 1, 8])
+@pytest.mark.parametrize("slices", [1, 2, 3, 4])
+@pytest.mark.parametrize("rows,n,taps", [(17, 4096, 4), (5, 1028, 3), (33, 8192, 8), (40, 2048, 0), (3, 12292, 0)])
+@BOTH
+def test_norm_adds_one_to_four_slices_whatever_the_runs(dtype, rows, n, taps, slices, run):
+    """The sum in order, rounded: bit for bit what a delta of that gives, also where runs of several tokens are asked for."""
+    g = torch.Generator(device=DEV).manual_seed(rows + slices)
+    x, sums = torch.randn((rows, n), generator=g, device=DEV), torch.randn((slices, rows, n), generator=g, device=DEV)
+    wd, wn = (0.3 * torch.randn((2, n), generator=g, device=DEV)).unbind(0)
+    delta = sums[0].clone()
+    for s in sums[1:]:
+        delta += s
+    _lib.set_seq_option("norm_run", run)
+    tails = [torch.ones((rows, taps, n), device=DEV) for _ in range(2)] if taps else [None, None]
+    norm = lambda d, tail: seq_ops.norm_conv(x, rows, 1, 1e-4, dtype, delta=d, delta_weight=wd, delta_offset=1.0, norm_weight=wn, norm_offset=1.0,
+                                             **(dict(conv=wd.repeat(taps, 1), tails=(tail, tail), input_pos=positions(5, 1)) if taps else {}))
+    for got, want in zip(norm(sums, tails[0]), norm(delta.to(dtype), tails[1])):
+        assert torch.equal(got, want)
+    assert not taps or torch.equal(tails[0], tails[1])
+    with pytest.raises(RuntimeError):
+        norm(torch.zeros((5, rows, n), device=DEV), tails[0])
