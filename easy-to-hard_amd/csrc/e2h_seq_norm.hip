@@ -533,7 +533,7 @@ int norm_conv(const e2h_norm_conv_args *a, const DeltaSums &sums, void *stream) 
   if (!a || !a->x || ((a->delta || a->terms || sums.from) && !a->delta_weight) || (a->terms && !a->term_weights)) return E2H_ERR_NULL_POINTER;
   if (!a->out && !a->x_out) return E2H_ERR_NULL_POINTER;
   if (a->conv && (!a->input_pos || (a->taps > 1 && (!a->tail_in || !a->tail_out)))) return E2H_ERR_NULL_POINTER;
-  if (a->batch < 1 || a->seqlen < 1 || a->width < 4 || a->width % 4 != 0 || a->width > 16384 || a->seqlen > INT32_MAX / 4)
+  if (a->batch < 1 || a->batch > INT32_MAX || a->seqlen < 1 || a->width < 4 || a->width % 4 != 0 || a->width > 16384 || a->seqlen > INT32_MAX / 4)
     return E2H_ERR_BAD_SHAPE;
   if (a->dtype != E2H_SEQ_BF16 && a->dtype != E2H_SEQ_F32) return E2H_ERR_BAD_SHAPE;
   if (a->conv && (a->taps < 1 || a->taps > 8)) return E2H_ERR_BAD_SHAPE;
@@ -555,7 +555,8 @@ int norm_conv(const e2h_norm_conv_args *a, const DeltaSums &sums, void *stream) 
     if (a->seqlen <= 32 && per_sequence == 0) run = static_cast<int>(a->seqlen);
   }
   const int64_t runs = (a->seqlen + run - 1) / run;
-  if (a->batch * runs > INT32_MAX) return E2H_ERR_BAD_SHAPE;
+  // without a convolution the kernel walks over rows, as many as runs of 32 would be workgroups
+  if (a->batch * (a->conv ? runs : (a->seqlen + 31) / 32) > INT32_MAX) return E2H_ERR_BAD_SHAPE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (a->dtype == E2H_SEQ_BF16) launch_norm_conv<bf16_t>(*a, sums, static_cast<int>(runs), run, s);
   else launch_norm_conv<float>(*a, sums, static_cast<int>(runs), run, s);

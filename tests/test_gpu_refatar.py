@@ -937,6 +937,20 @@ def test_norm_that_adds_the_slices_of_a_product_equals_the_product_and_the_norm(
         seq_ops.norm_conv(x, 1, rows, 1e-4, torch.bfloat16, delta=sums, delta_weight=wd)  # several tokens of a sequence
 
 
+def test_norm_of_more_rows_than_31_bits_count():
+    """Without a convolution rows are walked, so their number has no limit of a launch (51 GB of narrow rows)."""
+    batch, seqlen, width = 8, (1 << 28) + 125, 4
+    rows, last = batch * seqlen, 1000
+    x = torch.empty((rows, width), dtype=torch.float32, device=DEV)
+    x[-last:] = torch.randn((last, width), generator=torch.Generator(device=DEV).manual_seed(0), device=DEV)
+    w = torch.ones((width,), device=DEV)
+    _, got = seq_ops.norm_conv(x, batch, seqlen, 1e-4, torch.bfloat16, norm_weight=w)
+    _, want = seq_ops.norm_conv(x[-last:].clone(), 1, last, 1e-4, torch.bfloat16, norm_weight=w)
+    assert rows > 2 ** 31 and torch.equal(got[-last:], want)
+    del x, got
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("run", [0, 1, 8])
 @pytest.mark.parametrize("slices", [1, 2, 3, 4])
 @pytest.mark.parametrize("rows,n,taps", [(17, 4096, 4), (5, 1028, 3), (33, 8192, 8), (40, 2048, 0), (3, 12292, 0)])
