@@ -20,7 +20,7 @@ def embedded(emb: nn.Module, tokens: Tensor, want_rows: bool = True):
     w = emb.weight
     if (not torch.compiler.is_compiling() and type(emb) is nn.Embedding and emb.max_norm is None and w.dtype == torch.bfloat16 and w.is_cuda and w.device == tokens.device and tokens.numel() > 0 and w.is_contiguous()
             and tokens.is_contiguous() and w.shape[1] % 8 == 0 and w.data_ptr() % 16 == 0 and not (w.requires_grad and torch.is_grad_enabled())
-            and unwatched(emb) and not seq_ops.watched(w, tokens)):
+            and unwatched(emb) and not seq_ops.intercepted(w, tokens)):
         return seq_ops.embed_rows(w, tokens, want_rows)
     h = emb(tokens)
     return h.float(), h

@@ -16,7 +16,6 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 from torch import Tensor
-from torch.utils._device import DeviceContext
 
 from . import _lib, ops, seq_ops
 from .linear import unwatched
@@ -157,11 +156,9 @@ def _sums_serve(lin, x: Tensor) -> bool:
 
 
 def _stock_attention_wanted() -> bool:
-    """True where somebody intercepts torch functions (a default device does so too, but looks at no attention), or has switched off the backend whose place the
+    """True where somebody intercepts torch functions, or has switched off the backend whose place the
     package's attention of prompts takes."""
-    if torch._C._len_torch_function_stack() and any(type(m) is not DeviceContext for m in torch.overrides._get_current_function_mode_stack()):
-        return True
-    return not torch.backends.cuda.flash_sdp_enabled()
+    return seq_ops.function_modes() or not torch.backends.cuda.flash_sdp_enabled()
 
 
 class _MaskByPosition:

@@ -9,6 +9,7 @@ import ctypes
 
 import torch
 from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 from . import _lib
 from .ops import _current_device, _need_gpu, _OnDevice, _stream
@@ -148,6 +149,16 @@ def watched(*tensors):
     return not torch.compiler.is_compiling() and (torch._C._len_torch_dispatch_stack() > 0 or torch._C._get_tracing_state() is not None)
 
 
+def function_modes():
+    """True where somebody intercepts torch functions (a default device does so too, but only looks at factories)."""
+    return bool(torch._C._len_torch_function_stack()) and any(type(m) is not DeviceContext for m in torch.overrides._get_current_function_mode_stack())
+
+
+def intercepted(*tensors):
+    """watched(*tensors) or function_modes(): for launches in the place of torch's own functions."""
+    return function_modes() or watched(*tensors)
+
+
 def linear_streams(x, weight):
     """True where `linear` takes x [.., k] and weight [n, k]: bfloat16 on the GPU, up to 64 rows, no gradients, nobody watching."""
     k = weight.shape[1]
@@ -207,7 +218,7 @@ def linear_rows_pay(x, weight, act, cap=0.0):
         return False
     if not (x.is_contiguous() and weight.is_contiguous()) or x.data_ptr() % 16 or weight.data_ptr() % 16 or torch.is_autocast_enabled():
         return False
-    return bool(_lib.load_seq().e2h_seq_linear_rows_pays(rows, n, k, act, cap)) and not watched(x, weight)
+    return bool(_lib.load_seq().e2h_seq_linear_rows_pays(rows, n, k, act, cap)) and not intercepted(x, weight)
 
 
 def linear_rows(x, weight, act, cap=0.0):

@@ -972,3 +972,32 @@ def test_norm_adds_one_to_four_slices_whatever_the_runs(dtype, rows, n, taps, sl
     assert not taps or torch.equal(tails[0], tails[1])
     with pytest.raises(RuntimeError):
         norm(torch.zeros((5, rows, n), device=DEV), tails[0])
+
+
+# ---- launches in the place of torch functions ------------------------------------------------------------------------------------------
+
+class _Functions(torch.overrides.TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.names.append(getattr(func, "__name__", str(func)))
+        return func(*args, **(kwargs or {}))
+
+
+def test_who_intercepts_torch_functions_sees_the_products_of_a_prompt_and_its_embedding():
+    from easy_to_hard_amd.decoder import embedded
+    from easy_to_hard_amd.feed_forward import SquaredReluFF
+
+    ff = SquaredReluFF(256, 16384).to(DEV).to(torch.bfloat16).requires_grad_(False)
+    h, tokens = randn(2, 520, 256, dtype=torch.bfloat16), torch.arange(40, device=DEV)
+    emb = torch.nn.Embedding(50, 64, dtype=torch.bfloat16, device=DEV).requires_grad_(False)
+    assert seq_ops.linear_rows_pay(h, ff.up.weight, seq_ops.ACT_SQUARE_RELU) and seq_ops.linear_rows_pay(h, ff.up.weight, seq_ops.ACT_SOFTCAP, 30.0)
+    whole, rows = ff(h), embedded(emb, tokens)
+    with _Functions() as seen:
+        assert torch.equal(ff(h), whole) and seen.names.count("linear") == 2
+        assert not seq_ops.linear_rows_pay(h, ff.up.weight, seq_ops.ACT_SOFTCAP, 30.0)
+        assert all(torch.equal(a, b) for a, b in zip(embedded(emb, tokens), rows)) and "embedding" in seen.names
+    with torch.device(DEV):  # looks at factories only
+        assert seq_ops.linear_rows_pay(h, ff.up.weight, seq_ops.ACT_SQUARE_RELU)
