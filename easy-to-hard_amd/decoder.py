@@ -15,11 +15,15 @@ from .linear import DecodeLinear, fusable, unwatched
 from .state import SequenceState, StatePlan, rotary_turns
 
 
+# torch's embedding stops at a token outside the table where its kernels were built with assertions; where they were not it reads past the table, and the launch here makes a row of NaN instead
+EMBEDDING_UNCHECKED = "USE_ROCM_KERNEL_ASSERT=OFF" in torch.__config__.show()
+
+
 def embedded(emb: nn.Module, tokens: Tensor, want_rows: bool = True):
-    """emb(tokens) in float32, where the residual stream starts, and (want_rows) as it is; tokens int64 [rows]."""
+    """emb(tokens) in float32, where the residual stream starts, and (want_rows) as it is; tokens [rows]."""
     w = emb.weight
-    if (not torch.compiler.is_compiling() and type(emb) is nn.Embedding and emb.max_norm is None and w.dtype == torch.bfloat16 and w.is_cuda and w.device == tokens.device and tokens.numel() > 0 and w.is_contiguous()
-            and tokens.is_contiguous() and w.shape[1] % 8 == 0 and w.data_ptr() % 16 == 0 and not (w.requires_grad and torch.is_grad_enabled())
+    if (EMBEDDING_UNCHECKED and not torch.compiler.is_compiling() and type(emb) is nn.Embedding and emb.max_norm is None and w.dtype == torch.bfloat16 and w.is_cuda and w.device == tokens.device
+            and tokens.numel() > 0 and tokens.dtype == torch.int64 and w.is_contiguous() and tokens.is_contiguous() and w.shape[1] % 8 == 0 and w.data_ptr() % 16 == 0 and not (w.requires_grad and torch.is_grad_enabled())
             and unwatched(emb) and not seq_ops.intercepted(w, tokens)):
         return seq_ops.embed_rows(w, tokens, want_rows)
     h = emb(tokens)

@@ -645,3 +645,16 @@ def test_embedded_rows_are_the_embedding_and_its_float32_values(rows, width):
     assert seen == [1] and torch.equal(x, want.float()) and torch.equal(h, want)
     x, h = seq_ops.embed_rows(emb.weight, torch.tensor([0, 50, -1], device=DEV))
     assert torch.equal(h[0], emb.weight[0]) and x[1:].isnan().all() and h[1:].isnan().all()
+
+
+def test_embedding_of_other_tokens_and_of_a_torch_that_checks_them(monkeypatch):
+    from easy_to_hard_amd import decoder
+
+    emb = torch.nn.Embedding(50, 64, dtype=torch.bfloat16, device=DEV).requires_grad_(False)
+    tokens, calls, real = torch.arange(49, -1, -1, device=DEV), [], seq_ops.embed_rows
+    monkeypatch.setattr(seq_ops, "embed_rows", lambda *a: calls.append(1) or real(*a))
+    want = emb(tokens)
+    for unchecked, ids, count in ((True, tokens, 1), (True, tokens.int(), 1), (False, tokens, 1), (True, tokens[:0], 1), (True, tokens, 2)):
+        monkeypatch.setattr(decoder, "EMBEDDING_UNCHECKED", unchecked)
+        x, h = decoder.embedded(emb, ids)
+        assert torch.equal(h, want[:len(ids)]) and torch.equal(x, want[:len(ids)].float()) and len(calls) == count
