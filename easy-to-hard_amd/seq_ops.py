@@ -193,9 +193,15 @@ def linear(x, weight, act=ACT_NONE, cap=0.0):
     return y
 
 
+def _product(x, weight, what):
+    if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.dim() != 2 or x.dim() < 1 or x.shape[-1] != weight.shape[1]:
+        raise TypeError(f"{what}: bfloat16 [.., k] and [n, k] expected, got {x.dtype} {tuple(x.shape)} and {weight.dtype} {tuple(weight.shape)}")
+
+
 def linear_sums(x, weight):
     """linear(x, weight) as the float32 sums of its slices of K [slices, rows, n], which norm_conv adds, or None where it has none."""
     _need_gpu(x, weight)
+    _product(x, weight, "linear_sums")
     n, k = weight.shape
     rows = x.numel() // k
     if _lib.load_seq().e2h_seq_linear_scratch_bytes(rows, n, k) <= 0 or not (x.is_contiguous() and weight.is_contiguous()) or (x.data_ptr() | weight.data_ptr()) % 16:
@@ -224,6 +230,9 @@ def linear_rows_pay(x, weight, act, cap=0.0):
 def linear_rows(x, weight, act, cap=0.0):
     """act(x weight^T) over many rows in one launch, see e2h_seq_linear_rows (linear_rows_pay)."""
     _need_gpu(x, weight)
+    _product(x, weight, "linear_rows")
+    if not (x.is_contiguous() and weight.is_contiguous()):
+        raise RuntimeError("linear_rows: contiguous x and weight expected")
     n, k = weight.shape
     y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
     _lib.check_seq(_lib_for(x).e2h_seq_linear_rows(_p(x), _p(weight), _p(y), x.numel() // k, n, k, act, cap, _stream(x)), "e2h_seq_linear_rows")

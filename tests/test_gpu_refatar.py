@@ -902,6 +902,17 @@ def test_feed_forward_of_many_rows_takes_one_launch_for_up_and_its_activation():
         assert seq_ops.linear_rows_pay(h, up, 1)
 
 
+def test_products_of_many_rows_and_slices_refuse_other_types_and_layouts():
+    x, w = randn(300, 256, dtype=torch.bfloat16), randn(256, 256, dtype=torch.bfloat16)
+    for a, b in ((x.half(), w), (x, w.half()), (x, w.float()), (x[:, :192], w), (x, w[None])):
+        for call in (seq_ops.linear_sums, lambda a, b: seq_ops.linear_rows(a, b, seq_ops.ACT_NONE)):
+            with pytest.raises(TypeError):
+                call(a, b)
+    for a, b in ((x, w.t()), (x.t().contiguous().t(), w)):
+        with pytest.raises(RuntimeError):
+            seq_ops.linear_rows(a, b, seq_ops.ACT_NONE)
+
+
 # ---- the token side's gate in the launch of its product --------------------------------------------------------------------------------
 
 @pytest.mark.parametrize("rows,n,k,column", [(1, 256, 4096, 256), (17, 64, 2048, 0), (64, 40, 128, 24), (33, 8, 4096, 3)])
