@@ -852,8 +852,20 @@ def int8_norm_fits(x, weight, delta, *mods):
     return all(m.weight.is_contiguous() and m.scales.is_contiguous() and _lib.load().e2h_int8_norm_mm_supported(x.numel() // k, m.weight.shape[0], k) for m in mods)
 
 
-def _row_norm(x, delta, weight, eps):
-    """-> (the norm's arguments, h): h is x itself where nothing is added."""
+def _row_norm(x, delta, weight, eps, *products):
+    """-> (the norm's arguments, h): h is x itself where nothing is added.  products: weights and scales of those that take the row."""
+    k = x.shape[-1]
+    if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or not (x.is_contiguous() and weight.is_contiguous()) or weight.numel() != k:
+        raise TypeError(f"int8_norm_mm: contiguous bfloat16 x [.., {k}] and weight [{k}] expected, got {x.dtype} and {weight.dtype} {tuple(weight.shape)}")
+    for q, scales in products:
+        if q.dtype != torch.int8 or scales.dtype != torch.bfloat16 or q.dim() != 2 or q.shape[1] != k or scales.numel() != q.shape[0] or not (q.is_contiguous() and scales.is_contiguous()):
+            raise TypeError(f"int8_norm_mm: contiguous int8 [n, {k}] and bfloat16 [n] expected, got {q.dtype} {tuple(q.shape)} and {scales.dtype} {tuple(scales.shape)}")
+    if delta is not None:
+        part, cs = delta.partials, delta.scales
+        _need_gpu(part, cs)
+        if (part.dtype != torch.float32 or part.dim() != 3 or tuple(part.shape[1:]) != (x.numel() // k, k) or cs.dtype != torch.bfloat16 or cs.numel() != k
+                or not (part.is_contiguous() and cs.is_contiguous())):
+            raise TypeError(f"int8_norm_mm: partial sums float32 [slices, {x.numel() // k}, {k}] with bfloat16 scales [{k}] expected, got {part.dtype} {tuple(part.shape)}, {cs.dtype} {tuple(cs.shape)}")
     if delta is None:
         return _lib.RowNorm(_ptr(x), None, None, _ptr(weight), None, 0, float(eps)), x
     h = torch.empty_like(x)
@@ -865,7 +877,7 @@ def int8_norm_mm(x, delta, weight, eps, q, scales):
     _need_gpu(x, weight, q, scales)
     n, k = q.shape
     rows = x.numel() // k
-    norm, h = _row_norm(x, delta, weight, eps)
+    norm, h = _row_norm(x, delta, weight, eps, (q, scales))
     y = torch.empty((rows, n), dtype=torch.bfloat16, device=x.device)
     _lib.check(_lib_for(x).e2h_int8_norm_mm(norm, _ptr(q), _ptr(scales), _ptr(y), rows, n, k, _stream(x)), "e2h_int8_norm_mm")
     return h, y
@@ -878,7 +890,7 @@ def int8_norm_mm_silu_gate(x, delta, weight, eps, q_gate, scales_gate, q_up, sca
     if q_up.shape != q_gate.shape or scales_gate.numel() != n or scales_up.numel() != n:
         raise RuntimeError("int8_norm_mm_silu_gate: shapes of the two linears do not match")
     rows = x.numel() // k
-    norm, h = _row_norm(x, delta, weight, eps)
+    norm, h = _row_norm(x, delta, weight, eps, (q_gate, scales_gate), (q_up, scales_up))
     y = torch.empty((rows, n), dtype=torch.bfloat16, device=x.device)
     _lib.check(_lib_for(x).e2h_int8_norm_mm_silu_gate(norm, _ptr(q_gate), _ptr(scales_gate), _ptr(q_up), _ptr(scales_up), _ptr(y), rows, n, k, _stream(x)),
                "e2h_int8_norm_mm_silu_gate")
@@ -898,7 +910,7 @@ def int8_norm_mm_rope_kv(x, delta, weight, eps, q_weight, scales, freqs_cis, k_c
         raise RuntimeError("int8_norm_mm_rope_kv: caches must be [>= B, Hkv, S, D]")
     if freqs_cis.shape[0] < k_cache.shape[2] or tuple(freqs_cis.shape[1:]) != (head_dim // 2, 2):
         raise RuntimeError("int8_norm_mm_rope_kv: freqs_cis must be [>= S, D/2, 2]")
-    norm, h = _row_norm(x, delta, weight, eps)
+    norm, h = _row_norm(x, delta, weight, eps, (q_weight, scales))
     q = torch.empty((rows, n_head, head_dim), dtype=torch.bfloat16, device=x.device)
     _lib.check(_lib_for(x).e2h_int8_norm_mm_rope_kv(norm, _ptr(q_weight), _ptr(scales), _ptr(freqs_cis), _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(input_pos), rows,
                                                     n_head, n_kv_head, head_dim, k_cache.shape[2], k, _stream(x)), "e2h_int8_norm_mm_rope_kv")

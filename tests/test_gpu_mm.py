@@ -766,6 +766,29 @@ def test_int8_products_form_their_row_of_a_norm_as_the_norm_does(n, k, term):
     assert err <= TOL, err
 
 
+def test_int8_products_behind_a_norm_refuse_other_types_and_shapes():
+    k, n, d = 256, 384, 128
+    _, _, q, s = _int8_case(n, k, seed=1)
+    x, w = randn_bf16((1, k), seed=2).to(DEV), randn_bf16((k,), seed=3).to(DEV)
+    part, cs = torch.randn((2, 1, k), device=DEV), randn_bf16((k,), seed=4).to(DEV)
+    freqs, pos = randn_bf16((16, d // 2, 2), seed=5).to(DEV), torch.tensor([3], device=DEV)
+    caches = torch.zeros((2, 1, 1, 16, d), dtype=torch.bfloat16, device=DEV)
+    good = dict(x=x, delta=ops.ScaledPartials(part, cs), weight=w, q=q, scales=s)
+    calls = (lambda x, delta, weight, q, scales: ops.int8_norm_mm(x, delta, weight, 1e-5, q, scales),
+             lambda x, delta, weight, q, scales: ops.int8_norm_mm_silu_gate(x, delta, weight, 1e-5, q, scales, q, scales),
+             lambda x, delta, weight, q, scales: ops.int8_norm_mm_rope_kv(x, delta, weight, 1e-5, q, scales, freqs, *caches, pos, 1, 1, d))
+    bad = [dict(x=x.half()), dict(weight=w.float()), dict(weight=w.repeat(2)[::2]), dict(q=q.to(torch.uint8)), dict(q=q.t().contiguous().t()), dict(scales=s.float()), dict(scales=s.repeat(2)[::2]),
+           dict(delta=ops.ScaledPartials(part.half(), cs)), dict(delta=ops.ScaledPartials(part[:, :, :128], cs)), dict(delta=ops.ScaledPartials(part, cs.float())),
+           dict(delta=ops.ScaledPartials(part.transpose(0, 2).contiguous().transpose(0, 2), cs))]
+    for call in calls:
+        call(**good)
+        for change in bad:
+            with pytest.raises(TypeError):
+                call(**{**good, **change})
+        with pytest.raises(RuntimeError):
+            call(**{**good, "delta": ops.ScaledPartials(torch.zeros((3, 1, k), device=DEV), cs)})
+
+
 def test_int8_step_of_one_sequence_is_that_of_separate_norms():
     """The folded step against the one that a watched module takes, bit for bit, and its caches."""
     from easy_to_hard_amd.model import ModelArgs, random_quantized_transformer
