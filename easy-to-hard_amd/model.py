@@ -140,11 +140,11 @@ def _project_deferred(lin, y2d: Tensor, lead_shape) -> Tensor:
 
 def _product_rows(lin, x: Tensor, sums: Optional[Tensor], defer: bool = False) -> Tensor:
     """lin(x) of a prompt.  sums: those of x's quantization groups, from the norm in front (None: there are none).  defer: where the library shares K, the float32 sums of its
-    slices [slices, rows, N] may come back, for the next norm to add."""
+    slices may come back, for the next norm to add."""
     if type(lin) is WeightOnlyInt4Linear and not lin.padding and unwatched(lin):
         y = _lib.calls().int4_rows(x, lin.weight, lin.scales_and_zeros, lin.groupsize, lin.out_features, sums, defer)
         if y is not None:
-            return y
+            return ops.PairedPartials(y) if y.dtype == torch.float32 else y
     return lin(x)
 
 
@@ -236,7 +236,7 @@ class Attention(nn.Module):
                 fully_causal: bool = False, defer_output: bool = False, sums: Optional[Tensor] = None) -> Tensor:
         """sums (TransformerBlock._forward_rows): those of x's quantization groups.
         defer_output (fused decode step, or sums): the output projection may come back as float32 partial sums over K
-        slices, to be added by the residual add + RMSNorm that follows (ops.add_rmsnorm takes either form)."""
+        slices (ops.PairedPartials with sums), to be added by the residual add + RMSNorm that follows (ops.add_rmsnorm takes either form)."""
         bsz, seqlen, _ = x.shape
         kv_size = self.n_local_heads * self.head_dim
         if self.can_fuse_decode(x, fully_causal):

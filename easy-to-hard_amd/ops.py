@@ -433,6 +433,8 @@ def add_rmsnorm_sums(x, delta, weight, eps, groupsize):
     rows = x.numel() // dim
     h, y, sums = x, torch.empty_like(x), _group_sums_empty(rows, dim, groupsize, x.device)
     d16 = part = None
+    if isinstance(delta, PairedPartials):
+        delta = delta.partials
     if delta is not None:
         h = torch.empty_like(x)
         if delta.dtype == torch.float32:
@@ -552,6 +554,14 @@ def int8_partial_slices(rows: int, lin) -> int:
     return s if s > 0 else 0
 
 
+class PairedPartials:
+    """float32 K-slice sums [slices, rows, N] of an int4 matmul over more than 64 rows, which adds them in pairs, then pairs of pairs; add_rmsnorm and add_rmsnorm_sums take it in
+    place of `delta`."""
+
+    def __init__(self, partials):
+        self.partials = partials
+
+
 class ScaledPartials:
     """float32 K-slice sums [slices, rows, N] of an int8 matmul together with the column scales that turn them into the
     linear's output; add_rmsnorm takes it in place of `delta`."""
@@ -576,7 +586,9 @@ def int8_mm_partials(x, q, scales, slices):
 def add_rmsnorm(x, delta, weight, eps):
     """h = bf16(x + delta); returns (h, RMSNorm(h)) -- the residual add and the following norm in one kernel.  `delta` is
     either a bfloat16 tensor of x's shape, or float32 partial sums [slices, rows, dim] from int4_mm_partials, in which case
-    the term added is bf16(sum over slices, in order), or the ScaledPartials of int8_mm_partials."""
+    the term added is bf16(sum over slices, in order), or the ScaledPartials of int8_mm_partials or PairedPartials."""
+    if isinstance(delta, PairedPartials):
+        return add_rmsnorm_sums(x, delta, weight, eps, 128)[:2]
     col_scales = None
     if isinstance(delta, ScaledPartials):
         delta, col_scales = delta.partials, delta.scales

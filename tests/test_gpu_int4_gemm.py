@@ -713,3 +713,24 @@ def test_a_prompt_with_group_sums_from_its_norms_equals_the_modules(monkeypatch)
     for hook in watched:
         hook.remove()
     assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(kept, caches()))
+
+
+@pytest.mark.parametrize("watch", [None, "first", "second"])
+def test_slices_of_a_prompt_are_added_in_one_order_by_every_norm_behind_them(watch):
+    """A head that is no int4 linear, or small, and blocks that somebody watches take the plain norm, which has to add the slices of the block before as the matmul does: bit for bit the modules."""
+    from easy_to_hard_amd.model import ModelArgs, random_quantized_transformer
+
+    cfg = ModelArgs(block_size=256, vocab_size=2048, n_layer=2, n_head=16, n_local_heads=16, dim=2048, intermediate_size=5632)
+    model = random_quantized_transformer(cfg, "int4", groupsize=128, device=DEV).requires_grad_(False)
+    model.setup_caches(3, 200)
+    assert ops.int4_rows_slices(471, 2048, 5632, 128, 8) == 4 and ops.int4_rows_slices(471, 2048, 2048, 128, 8) == 0
+    gen = torch.Generator(device=DEV).manual_seed(4)
+    ids, pos = torch.randint(0, 2048, (3, 157), generator=gen, device=DEV), torch.arange(157, device=DEV)
+    watched = [] if watch is None else [model.layers[watch == "second"].ffn_norm.register_forward_hook(lambda *a: None)]
+    with torch.no_grad():
+        got = model(ids, pos)
+        watched += [m.register_forward_hook(lambda *a: None) for b in model.layers for m in (b.attention_norm, b.ffn_norm)]
+        want = model(ids, pos)
+    for hook in watched:
+        hook.remove()
+    assert torch.equal(got, want)
