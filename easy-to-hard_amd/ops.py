@@ -75,6 +75,12 @@ def _workspace(device):
     return ws
 
 
+def _capture_workspace(device):
+    """Makes the workspaces where a call stands for quantized linears that use none of their own: a first eager call is what a later capture relies on."""
+    if ("capture", device.index) not in _workspaces and not torch.cuda.is_current_stream_capturing():
+        _workspace(device)
+
+
 class _OnDevice:
     """The library's entry points launch on the current device: calls for tensors of another device run under a
     device guard (the caller's current device is left as it was)."""
@@ -428,6 +434,7 @@ def add_rmsnorm_sums(x, delta, weight, eps, groupsize):
     int4_mm and int4_mm_silu_gate_rows otherwise form in a launch of their own -> (h, y, sums)."""
     _need_gpu(x, weight)
     assert x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
+    _capture_workspace(x.device)
     x = x.contiguous()
     dim = x.shape[-1]
     rows = x.numel() // dim
@@ -867,6 +874,7 @@ def int8_norm_fits(x, weight, delta, *mods):
 def _row_norm(x, delta, weight, eps, *products):
     """-> (the norm's arguments, h): h is x itself where nothing is added.  products: weights and scales of those that take the row."""
     k = x.shape[-1]
+    _capture_workspace(x.device)
     if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or not (x.is_contiguous() and weight.is_contiguous()) or weight.numel() != k:
         raise TypeError(f"int8_norm_mm: contiguous bfloat16 x [.., {k}] and weight [{k}] expected, got {x.dtype} and {weight.dtype} {tuple(weight.shape)}")
     for q, scales in products:

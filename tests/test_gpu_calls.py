@@ -143,3 +143,32 @@ def test_a_failed_launch_is_reported_and_not_tried_again(mode):
     finally:
         bind(lib.e2h_int4_mm, lib.e2h_int8_mm)
     assert torch.equal(lin(x), want)
+
+
+@pytest.mark.parametrize("mode,eager,captured", [("int4", (3, 157), (3, 157)), ("int8", (1, 1), (1, 1)), ("int8", (1, 1), (1, 20))])
+def test_one_eager_pass_is_enough_for_a_capture(mode, eager, captured):
+    """Also where every quantized linear of the pass runs in a launch that has no workspace of its own."""
+    from easy_to_hard_amd.model import ModelArgs, random_quantized_transformer
+
+    cfg = ModelArgs(block_size=256, vocab_size=8192, n_layer=1, n_head=32, n_local_heads=32, dim=4096, intermediate_size=5632)
+    model = random_quantized_transformer(cfg, mode, device="cuda").requires_grad_(False)
+    model.setup_caches(3, 256)
+    at = lambda shape: (torch.randint(0, 8192, shape, device="cuda"), torch.arange(shape[1], device="cuda"))
+    before = dict(ops._workspaces)
+    ops._workspaces.clear()
+    try:
+        with torch.no_grad():
+            model(*at(eager))
+            torch.cuda.synchronize()
+            assert ("capture", 0) in ops._workspaces
+            ids, pos = at(captured)
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                logits = model(ids, pos)
+            for _ in range(3):
+                ids.copy_(at(captured)[0])
+                want = model(ids, pos)
+                graph.replay()
+                assert torch.equal(logits, want)
+    finally:
+        ops._workspaces.update(before)  # launches recorded earlier use them
