@@ -428,7 +428,7 @@ class TransformerBlock(nn.Module):
             return False
         att, ff, norms = self.attention, self.feed_forward, (self.attention_norm, self.ffn_norm)
         if not (type(att) is Attention and type(ff) is FeedForward and all(type(m) is RMSNorm and m.weight.dtype == torch.bfloat16 and m.weight.is_contiguous() for m in norms)
-                and all(unwatched(m) for m in (*norms, att, ff))):
+                and all(unwatched(m) for m in (*norms, att, ff))) or att.can_fuse_decode(x, fully_causal):  # (a step of many sequences: its attention reads no sums)
             return False
         return _sums_serve(att.wqkv, x) and _sums_serve(ff.w1, x) and att._can_fuse_prefill_rope(x, input_pos, fully_causal) and not seq_ops.watched(x)
 

@@ -734,3 +734,31 @@ def test_slices_of_a_prompt_are_added_in_one_order_by_every_norm_behind_them(wat
     for hook in watched:
         hook.remove()
     assert torch.equal(got, want)
+
+
+def test_steps_of_many_sequences_and_scoring_passes_of_some_hundred_rows(monkeypatch):
+    """A step of 80 sequences keeps the steps' own attention, whose products read no group sums: none are formed but the head's.  Without a cache (scoring) they serve as in a prompt."""
+    from easy_to_hard_amd.model import ModelArgs, random_quantized_transformer
+
+    cfg = ModelArgs(block_size=64, vocab_size=12288, n_layer=2, n_head=32, n_local_heads=32, dim=4096, intermediate_size=5632)
+    model = random_quantized_transformer(cfg, "int4", groupsize=128, device=DEV).requires_grad_(False)
+    model.setup_caches(80, 64)
+    assert all(ops.int4_rows_slices(m, 12288, 4096, 128, 8) > 0 for m in (80, 300))
+    calls, real = [], ops.add_rmsnorm_sums
+    monkeypatch.setattr(ops, "add_rmsnorm_sums", lambda *a: calls.append(1) or real(*a))
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    for shape, fully_causal, count in (((80, 1), False, 1), ((5, 60), True, 5)):
+        ids, pos = torch.randint(0, 12288, shape, generator=gen, device=DEV), torch.arange(shape[1], device=DEV) + (7 if shape[1] == 1 else 0)
+        for b in model.layers:
+            for cache in (b.attention.kv_cache.k_cache, b.attention.kv_cache.v_cache):
+                cache.normal_(generator=gen)
+        calls.clear()
+        with torch.no_grad():
+            got = model(ids, pos, fully_causal=fully_causal)
+            assert len(calls) == count
+            watched = [m.register_forward_hook(lambda *a: None) for m in (*(b.attention_norm for b in model.layers), model.norm)]
+            want = model(ids, pos, fully_causal=fully_causal)
+            assert len(calls) == count
+        for hook in watched:
+            hook.remove()
+        assert torch.equal(got, want)
