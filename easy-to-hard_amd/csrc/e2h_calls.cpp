@@ -154,9 +154,17 @@ PyObject *int4_rows(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   if (slices < 1 || capturing_entry(stream) != 0) Py_RETURN_NONE;
   const int64_t groups = c.k / (g < 128 ? g : 128), stride = (c.m + 63) / 64 * 64;
   const auto floats = x.options().dtype(at::kFloat);
-  at::Tensor sums = there ? THPVariable_Unpack(args[5]) : at::empty({groups, stride}, floats), partials, y;
-  if (there && (!plain(sums, c.device, at::kFloat) || sums.dim() != 2 || sums.size(0) != groups || sums.size(1) != stride)) Py_RETURN_NONE;
-  if (slices > 1) partials = at::empty({slices, c.m, c.n}, floats);
+  at::Tensor sums, partials, y;
+  if (there) {
+    sums = THPVariable_Unpack(args[5]);
+    if (!plain(sums, c.device, at::kFloat) || sums.dim() != 2 || sums.size(0) != groups || sums.size(1) != stride) Py_RETURN_NONE;
+  }
+  try {
+    if (!there) sums = at::empty({groups, stride}, floats);
+    if (slices > 1) partials = at::empty({slices, c.m, c.n}, floats);
+  } catch (const c10::OutOfMemoryError &) {
+    Py_RETURN_NONE;  // the calls without this have a workspace for both
+  }
   if (slices == 1 || !defer) y = result_for(x, c.n);
   int rc;
   Py_BEGIN_ALLOW_THREADS

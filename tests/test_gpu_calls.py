@@ -172,3 +172,22 @@ def test_one_eager_pass_is_enough_for_a_capture(mode, eager, captured):
                 assert torch.equal(logits, want)
     finally:
         ops._workspaces.update(before)  # launches recorded earlier use them
+
+
+def test_products_of_a_prompt_run_in_the_workspace_where_no_memory_is_left():
+    lin, x = _linear("int4", n=2048, k=5632, g=128), _x(1000, 5632)
+    rows = lambda defer: _lib.calls().int4_rows(x, lin.weight, lin.scales_and_zeros, 128, 2048, None, defer)
+    assert ops.int4_rows_slices(1000, 2048, 5632, 128, 8) > 1
+    want = lin(x)
+    assert torch.equal(rows(False), want) and rows(True).dtype == torch.float32
+    spare = lin(x)  # the result's place
+    torch.cuda.empty_cache()
+    del spare
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)
+    try:
+        assert rows(False) is None and rows(True) is None
+        assert torch.equal(lin(x), want)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(rows(False), want)
