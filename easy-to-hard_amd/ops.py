@@ -797,6 +797,8 @@ def _rope_rows(x, weights, name, options, freqs_cis, k_cache, v_cache, input_pos
     bsz, t, k = x.shape
     assert input_pos.numel() == t and k_cache.shape[0] >= bsz and k_cache.shape[1] == n_kv_head and k_cache.shape[3] == head_dim and v_cache.shape == k_cache.shape
     assert tuple(freqs_cis.shape[1:]) == (head_dim // 2, 2) and (rows_by_token or freqs_cis.shape[0] >= k_cache.shape[2])
+    if freqs_cis.shape[0] > (2 ** 31 - 1) // 2 // head_dim:  # an angle's place is counted in 32 bits there
+        return None
     lib = _lib_for(x)
     sizes = (t, n_head, n_kv_head, k_cache.shape[2], head_dim, k, *options)
     scratch = _unpacked_weight(bsz * t, x.device, lambda rows, *rest: getattr(lib, name + "_scratch_bytes")(bsz, *rest), *sizes)
