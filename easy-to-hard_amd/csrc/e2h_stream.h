@@ -38,7 +38,8 @@ struct RowNorm {
   float eps;
 };
 struct NoNorm {};
-constexpr int kNormPieces = 2, kNormPiece = 4096;  // pieces of the row, eight values per thread each
+constexpr int kNormPieces = 2, kNormPiece = 4096;  // pieces of the row, eight values per thread each; of rows between 2048 and 4096 pieces of 2048 for half of the threads, whose sums run over both,
+                                                   // as in the norm's own launch
 constexpr int kNormSums = 128, kNormBytes = kNormSums + kNormPieces * kNormPiece * 2;  // LDS: the waves' sums of squares, the row
 inline bool norm_fits(int64_t M, int64_t K) { return M == 1 && K >= 128 && K % 128 == 0 && K <= kNormPieces * kNormPiece; }
 
@@ -96,11 +97,19 @@ struct NormLoads {
   u32x4_t x[kNormPieces], w[kNormPieces], cs[kNormPieces];
   f32x4_t lo[kNormPieces][2], hi[kNormPieces][2];
 
+  static __device__ __forceinline__ bool halves(int K) { return K > kNormPiece / 2 && K < kNormPiece; }
+  static __device__ __forceinline__ int span(int K) { return halves(K) ? kNormPiece / 2 : kNormPiece; }
+  // this thread's place in piece p, K where it has none
+  static __device__ __forceinline__ int place(int K, int p) {
+    const int own = static_cast<int>(threadIdx.x) * 8, i = p * span(K) + own;
+    return own < span(K) && i < K ? i : K;
+  }
+
   __device__ __forceinline__ void request(const RowNorm &n, int K) {
 #pragma unroll
     for (int p = 0; p < kNormPieces; ++p) {
-      const int i = p * kNormPiece + static_cast<int>(threadIdx.x) * 8, at = i < K ? i : 0;  // past the row: its first piece, not used
-      if (K <= p * kNormPiece) break;
+      const int i = place(K, p), at = i < K ? i : 0;  // past the row: its first piece, not used
+      if (K <= p * span(K)) break;
       x[p] = *reinterpret_cast<const u32x4_t *>(n.x + at);
       if (n.partials) {
         const float *const from = n.partials + at, *const other = from + (n.slices > 1 ? K : 0);
@@ -119,11 +128,13 @@ struct NormLoads {
     float *const sums = reinterpret_cast<float *>(lds);
     const auto low = [](uint32_t v) { return __builtin_bit_cast(float, v << 16); };
     const auto high = [](uint32_t v) { return __builtin_bit_cast(float, v & 0xFFFF0000u); };
+    float ss = 0.f;
 #pragma unroll
     for (int p = 0; p < kNormPieces; ++p) {
-      const int i = p * kNormPiece + static_cast<int>(threadIdx.x) * 8;
-      float ss = 0.f;
-      if (K > p * kNormPiece) {
+      const int i = place(K, p);
+      float wave = 0.f;
+      if (!halves(K)) ss = 0.f;
+      if (K > p * span(K)) {
         if (n.partials) {
           f32x4_t a = lo[p][0], b = hi[p][0];
           if (n.slices > 1) a += lo[p][1], b += hi[p][1];
@@ -143,19 +154,20 @@ struct NormLoads {
             ss = __builtin_fmaf(h1, h1, ss);
           }
         }
+        wave = ss;
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
+        for (int off = 32; off > 0; off >>= 1) wave += __shfl_xor(wave, off);
       }
-      if ((threadIdx.x & 63) == 0) sums[p * kWaves + (threadIdx.x >> 6)] = ss;
+      if ((threadIdx.x & 63) == 0) sums[p * kWaves + (threadIdx.x >> 6)] = p == 0 && halves(K) ? 0.f : wave;
     }
     lds_barrier();
-    float ss = 0.f;
+    float sum = 0.f;
 #pragma unroll
-    for (int q = 0; q < kNormPieces * kWaves; ++q) ss += sums[q];
-    const float inv = rsqrtf(ss / static_cast<float>(K) + n.eps);
+    for (int q = 0; q < kNormPieces * kWaves; ++q) sum += sums[q];
+    const float inv = rsqrtf(sum / static_cast<float>(K) + n.eps);
 #pragma unroll
     for (int p = 0; p < kNormPieces; ++p) {
-      const int i = p * kNormPiece + static_cast<int>(threadIdx.x) * 8;
+      const int i = place(K, p);
       if (i >= K) break;
       u32x4_t o;
 #pragma unroll
