@@ -372,7 +372,7 @@ template <typename T, int BLOCK, int NP, int TAPS, bool LAYER, bool TERMS, int S
 void launch_norm_conv_rows(const e2h_norm_conv_args &a, const DeltaSums &sums, int runs, int run, hipStream_t s) {
   const int64_t workgroups = TAPS ? a.batch * runs : a.batch * a.seqlen < (1 << 20) ? a.batch * a.seqlen : 1 << 20;
   const dim3 grid(static_cast<unsigned>(workgroups)), block(BLOCK);
-  // from 21 million values on (x, the new x and two 16-bit operands are 12 bytes each) they do not stay in 256 MB of cache anyway; 4096 x 4096 takes as long with either store
+  // from 22.4 million values on (x, the new x and two 16-bit operands are 12 bytes each) they do not stay in 256 MB of cache anyway; 4096 x 4096 takes as long with either store
   const int streamed = a.batch * a.seqlen * a.width >= (int64_t{1} << 28) / 12;
   if constexpr (TAPS > 0) {
     if (run > 1) {

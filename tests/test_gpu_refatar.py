@@ -948,6 +948,42 @@ def test_norm_that_adds_the_slices_of_a_product_equals_the_product_and_the_norm(
         seq_ops.norm_conv(x, 1, rows, 1e-4, torch.bfloat16, delta=sums, delta_weight=wd)  # several tokens of a sequence
 
 
+@BOTH
+@pytest.mark.parametrize("rows,width,taps,layer,terms", [(700, 4096, 4, False, 0), (40, 72, 8, False, 0), (300, 2048, 0, True, 3), (9, 4100, 0, True, 0), (1500, 1000, 0, False, 2), (64, 8192, 0, False, 0)])
+def test_what_is_no_number_stays_in_its_row_and_in_the_convolution_s_reach(dtype, rows, width, taps, layer, terms):
+    """NaN and infinities in x, in delta and in a term: the rows that plain arithmetic gives them, all others as if they were not there."""
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x, d = torch.randn((rows, width), generator=g, device=DEV), torch.randn((rows, width), generator=g, device=DEV).to(dtype)
+    t = torch.randn((rows * max(terms, 1), width), generator=g, device=DEV).to(dtype)
+    tw = torch.rand((rows, max(terms, 1)), generator=g, device=DEV)
+    w, bias = 1.0 + 0.3 * torch.randn((width,), generator=g, device=DEV), torch.zeros((width,), device=DEV)
+    kw = dict(layer_norm=True, delta_bias=bias, norm_bias=bias) if layer else {}
+    if terms:
+        kw.update(terms=t, term_weights=tw)
+    if taps:
+        kw.update(conv=0.5 + torch.rand((taps, width), generator=g, device=DEV), input_pos=positions(0, rows))
+
+    def run():
+        tails = dict(tails=(torch.zeros((1, taps, width), device=DEV), torch.zeros((1, taps, width), device=DEV))) if taps else {}
+        return seq_ops.norm_conv(x, 1, rows, 1e-4, dtype, delta=d, delta_weight=w, norm_weight=w, **kw, **tails)
+
+    clean = [a.clone() for a in run()]
+    x[1, 3], d[rows // 2, width - 1] = float("inf"), float("nan")
+    bad = {1, rows // 2}
+    if terms:
+        t[(rows - 2) * terms + 1, 0] = float("-inf")
+        bad.add(rows - 2)
+    own, reach = (torch.zeros(rows, dtype=torch.bool, device=DEV) for _ in range(2))
+    for r in bad:
+        own[r] = True
+        reach[r: r + max(taps, 1)] = True
+    xo, y = run()
+    assert torch.equal(xo[~own], clean[0][~own]) and torch.equal(y[~reach], clean[1][~reach])
+    # a row's mean square is infinite or no number: so are all of its values, or (an infinite one's others) zero
+    assert not torch.isfinite(xo[own]).all(-1).any() and torch.isnan(y[reach]).any(-1).all()
+    assert torch.isnan(y[rows // 2]).all() and torch.isinf(xo[1, 3]) and torch.isnan(y[1, 3])
+
+
 def test_norm_of_more_rows_than_31_bits_count():
     """Without a convolution rows are walked, so their number has no limit of a launch (51 GB of narrow rows)."""
     batch, seqlen, width = 8, (1 << 28) + 125, 4
