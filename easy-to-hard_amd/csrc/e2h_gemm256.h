@@ -223,7 +223,8 @@ __device__ __forceinline__ void walk(P &p, uint8_t *lds) {
 // ---- activations behind a tile ------------------------------------------------------------------------------------------------------------
 // A lane activates 128 values behind its tile with nothing beside it (35 instructions each, what expf and a division take, are 9 us a tile).  So they are formed by a few instructions that end
 // within kNear units in the last place of the form that a pass over memory has, and where a value lies that close to a boundary of its rounding to bfloat16 that form decides: all results
-// are bit for bit those of the pass.  Of 512 values of a wave's store one in eight has such a value; they are taken one per lane and round.
+// are bit for bit those of the pass.  One in eight of a wave's stores of 512 has such a value; they are taken one per lane and round.  A scoring pass of 49152 rows through two int8 7B layers
+// takes 31.00 ms, without the look at the rounding (one gate of 65536 rounds otherwise) 30.82, with passes of their own 32.18.
 constexpr uint32_t kNear = 8;
 typedef float f32x8_t __attribute__((ext_vector_type(8)));
 

@@ -200,7 +200,7 @@ using namespace e2h;
 
 // 1 where the product with its activation is expected to be faster here than the library's product and a pass over its result.  Measured, us, that / here: 16384 x 4096 1000 rows 114 / 96,
 // 8192 rows 817 / 743; 8192 x 2048 2048 rows 68 / 51; 2048 x 4096 8192 rows 112 / 95; 16384 x 4096 512 rows 70 / 76: not taken.  Without an activation the library's product is
-// 2 % the faster one where it fills the chip (16384 x 4096 8192 rows 725 / 742).  With a soft cap 32000 x 4096 8192 rows 1425 + 229 / 1489.
+// 2 % the faster one where it fills the chip (16384 x 4096 8192 rows 725 / 742).  With a soft cap 32000 x 4096 8192 rows 1425 + 229 / 1504.
 // us, as for the quantized linears on the same loop (a last round that is not full runs at a higher clock), against the library's product at what it reaches where it fills the chip, 1.5
 // PFLOP/s, and a pass over the result of its own.
 extern "C" int e2h_seq_linear_rows_pays(int64_t rows, int64_t n, int64_t k, int act, float cap) {

@@ -52,8 +52,8 @@ struct DeltaSums {
 // What bounds it: memory, once enough rows are on their way.  A run's workgroup asks for its next row before it waits for anything of this one (AHEAD): loads and stores have no branch
 // between them, or a wait for one row's loads would be one for all.  Without a convolution rows next to each other are at work at the same time, which beats runs with the next row on its
 // way (8192 x 4096, sum and norm 72 us, 80 in runs of 8), and large residual rows, which are not read again soon, are stored past the caches (58).
-// us at 4096 channels, in brackets runs of 8 (convolution: 1024 threads, two rows together) that waited for every row: 8192 rows with residual 58 (94), layer norm 63 (91), eight experts'
-// terms 161 (187), convolution 73 (101); 8000 rows 56 (85), 62 (106), 159 (214), 66 (167: one workgroup too many for a round); 2048 rows 17 (18), 20 (21), 39 (38), 25 (33).
+// us at 4096 channels, in brackets runs of 8 (convolution: 1024 threads, two rows together) that waited for every row: 8192 rows with residual 60 (97), layer norm 66 (92), eight experts'
+// terms 166 (187), convolution 85 (112); 8000 rows 58 (86), 62 (106), 160 (214), 80 (167: one workgroup too many for a round); 2048 rows 18 (18), 21 (21), 40 (38), 28 (32).
 template <typename T, int BLOCK, int NP, int TAPS, bool LAYER, bool TERMS, bool AHEAD, int SPLIT>
 __global__ __launch_bounds__(BLOCK) void norm_conv_kernel(const e2h_norm_conv_args a, const DeltaSums sums, int runs, int run, int streamed) {
 #if defined(__HIP_DEVICE_COMPILE__)
