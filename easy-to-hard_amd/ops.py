@@ -870,6 +870,9 @@ def int8_norm_fits(x, weight, delta, *mods):
                                   and delta.partials.shape[0] <= 2 and tuple(delta.partials.shape[1:]) == (x.numel() // k, k)
                                   and delta.scales.dtype == torch.bfloat16 and delta.scales.is_contiguous() and delta.scales.numel() == k):
         return False
+    terms = (delta.partials, delta.scales) if delta is not None else ()
+    if any(t.data_ptr() % 16 for t in (x, weight, *terms, *(m.weight for m in mods))):  # the launches apart take an int8 weight anywhere
+        return False
     return all(m.weight.is_contiguous() and m.scales.is_contiguous() and _lib.load().e2h_int8_norm_mm_supported(x.numel() // k, m.weight.shape[0], k) for m in mods)
 
 

@@ -815,3 +815,20 @@ def test_int8_step_of_one_sequence_is_that_of_separate_norms():
         h.remove()
     assert len(calls) == 7  # a watched module is called
     assert torch.equal(folded, apart) and all(torch.equal(a, b) for a, b in zip(kept, kept_apart))
+
+
+def test_int8_step_of_one_sequence_takes_a_head_anywhere():
+    """A head that does not lie on 16 bytes runs in a launch of its own, behind the norm's."""
+    from easy_to_hard_amd.model import ModelArgs, random_quantized_transformer
+
+    cfg = ModelArgs(block_size=64, vocab_size=512, n_layer=2, n_head=4, n_local_heads=2, dim=256, intermediate_size=512)
+    model = random_quantized_transformer(cfg, "int8", device=DEV)
+    model.setup_caches(1, 64)
+    ids, pos = torch.tensor([[17]], device=DEV), torch.tensor([0], device=DEV)
+    flat = torch.empty((512 * 256 + 1,), dtype=torch.int8, device=DEV)
+    with torch.no_grad():
+        want = model(ids, pos)
+        flat[1:] = model.output.weight.view(-1)
+        model.output.weight = flat[1:].view(512, 256)
+        got = model(ids, pos)
+    assert (got.double() - want.double()).norm() <= 2.0 ** -7 * want.double().norm()  # sums in another order, rounded twice to bfloat16
